@@ -59,6 +59,23 @@ int viola_group_quantize_dual(const void* x, int x_dtype, int64_t rows, int64_t 
                               void* q, void* scale, void* qt, void* scale_t, int q_dtype, int gc,
                               float limit, float* column_partial, int scale_format, viola_stream_t stream);
 
+/* viola_group_quantize_dual with rows of q and qt q_pitch and qt_pitch codes apart (scales: ceil(pitch / 32) per row) and
+ * zero codes past the matrix, so that a GEMM may take the pitch as its k and load whole 16-byte pieces whatever the
+ * matrix's size (viola/nn/_grouped_kernels.py:127-158 lays the same codes out unpadded). Either layout may be absent
+ * (null); its pitch then is at least the matrix's own extent all the same. Groups of 32. */
+int viola_group_quantize_dual_pitched(const void* x, int x_dtype, int64_t rows, int64_t cols, void* q, int64_t q_pitch, void* scale,
+                                      void* qt, int64_t qt_pitch, void* scale_t, int q_dtype, float limit, float* column_partial,
+                                      int scale_format, viola_stream_t stream);
+/* Codes [batch][rows, cols] -> [batch][cols, out_pitch] with zeros past the matrix, and (scale != null) their grids of one
+ * scale per gr x gc block likewise; with column_partial, viola_column_reduce(column_partial, parts, sum_cols, column_sum)
+ * in the same launch. */
+int viola_codes_transpose_pitched(const void* x, void* out, int64_t batch, int64_t rows, int64_t cols, int64_t out_pitch,
+                                  const void* scale, void* scale_out, int gr, int gc, int scale_format,
+                                  const float* column_partial, int64_t parts, int64_t sum_cols, void* column_sum, int sum_dtype,
+                                  viola_stream_t stream);
+/* Codes [batch][rows, cols] -> [batch][rows, out_pitch] (out_pitch a multiple of 4), zeros past the matrix, scales likewise. */
+int viola_codes_repack(const void* x, void* out, int64_t batch, int64_t rows, int64_t cols, int64_t out_pitch, const void* scale,
+                       void* scale_out, int gr, int gc, int scale_format, viola_stream_t stream);
 /* viola_group_quantize_dual of h = act(g) * u [rows, cols], rounded to z_dtype, read from the stored projection
  * z = [g | u] [rows, 2 cols] (bf16 / fp16) instead of from a stored h: what the MXFP8 MLP hands from its gate/up
  * projection to its down projection (viola/nn/_mlp_kernels.py:195-230 encode h in the GEMM's epilogue; this is the
@@ -119,6 +136,16 @@ int viola_tensor_amax_scale(const void* x, int x_dtype, int64_t n, float* maxima
 int viola_tensor_quantize(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale, void* q, void* qt,
                           int q_dtype, float limit, viola_stream_t stream);
 
+/* amax, scale (with its history) and codes of one tensor in both layouts at pitched rows (see above): the calls
+ * viola_tensor_amax_scale and viola_tensor_quantize of viola/nn/linear.py:14-33 and _linear_kernels.py:231-260 as one, in
+ * fewer launches for small tensors. column_sum != null: x.sum(0) in sum_dtype from the same reads (columns whole 16-byte
+ * pieces, x 16-byte aligned; VIOLA_EUNSUPPORTED otherwise). workspace: 1024 floats, with column sums
+ * 1024 + viola_tensor_encode_slices(x_dtype, rows, cols) * cols, 16-byte aligned. */
+int viola_tensor_encode(const void* x, int x_dtype, int64_t rows, int64_t cols, float* workspace, int64_t workspace_floats,
+                        float* history, int history_len, int64_t index, int delayed, float limit, float* scale, void* q,
+                        int64_t q_pitch, void* qt, int64_t qt_pitch, int q_dtype, void* column_sum, int sum_dtype,
+                        viola_stream_t stream);
+int64_t viola_tensor_encode_slices(int x_dtype, int64_t rows, int64_t cols);
 /* ---------------------------------------------------------------- Hadamard-64 rotation (`rotation_size=64`)
  * H64 = H4 (x) H4 (x) H4, H4 = (ones(4, 4) - 2 flip(eye(4))) / 2, applied to each run of 64 consecutive columns of a
  * [rows, cols] matrix in FP32, in the operation order of viola/nn/_rotation_kernels.py:11-25 (_regular64); a last
@@ -376,6 +403,9 @@ int viola_comm_pack_table(const int64_t* table, int64_t buckets, int64_t max_uni
 int viola_comm_unpack_table(const int64_t* table, int64_t buckets, int64_t max_elements, int tile, int fp8_dtype,
                             int reduce, viola_stream_t stream);
 
+/* dst[0 .. count) on the device = host_words, carried in kernel arguments (no staging buffer; host_words may be reused at
+ * once). For tables of a few hundred words: offsets of variable groups. */
+int viola_store_words(int64_t* dst, const int64_t* host_words, int64_t count, viola_stream_t stream);
 /* ---------------------------------------------------------------- self checks (test support)
  * Compare the hardware FP8 conversion instructions with the software codecs over every fp32 bit
  * pattern of magnitude <= the format's clamp range (encode) and all 256 codes (decode); writes

@@ -1,4 +1,4 @@
-"""ctypes binding of libviola_hip.so (include/viola_hip.h) and tensor marshalling.
+"""ctypes binding of libviola_hip.so (include/viola_hip.h), tensor marshalling, and the loader of the native host path.
 
 PyTorch only supplies device memory and the current HIP stream here; every
 operator is one C-ABI call. There is no CPU or PyTorch fallback: if the library
@@ -6,6 +6,9 @@ is missing, or a tensor is not on the GPU, the call raises.
 """
 
 import ctypes
+import importlib
+import sys
+import types
 from pathlib import Path
 
 import torch
@@ -21,6 +24,10 @@ _i, _l, _f, _p = ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
 _SIGNATURES = {
     "viola_group_quantize": [_p, _i, _l, _l, _p, _i, _p, _i, _i, _f, _i, _p, _i, _i, _i, _p],
     "viola_group_quantize_dual": [_p, _i, _l, _l, _p, _p, _p, _p, _i, _i, _f, _p, _i, _p],
+    "viola_group_quantize_dual_pitched": [_p, _i, _l, _l, _p, _l, _p, _p, _l, _p, _i, _f, _p, _i, _p],
+    "viola_codes_transpose_pitched": [_p, _p, _l, _l, _l, _l, _p, _p, _i, _i, _i, _p, _l, _l, _p, _i, _p],
+    "viola_codes_repack": [_p, _p, _l, _l, _l, _l, _p, _p, _i, _i, _i, _p],
+    "viola_tensor_encode": [_p, _i, _l, _l, _p, _l, _p, _i, _l, _i, _f, _p, _p, _l, _p, _l, _i, _p, _i, _p],
     "viola_gated_quantize_dual": [_p, _i, _l, _l, _i, _p, _p, _p, _p, _i, _i, _f, _i, _p],
     "viola_column_reduce": [_p, _l, _l, _p, _i, _p],
     "viola_group_dequantize": [_p, _i, _p, _l, _l, _i, _i, _p, _p],
@@ -64,10 +71,11 @@ _SIGNATURES = {
     "viola_comm_unpack": [_p, _p, _l, _l, _l, _i, _i, _i, _p],
     "viola_comm_pack_table": [_p, _l, _l, _i, _i, _p],
     "viola_comm_unpack_table": [_p, _l, _l, _i, _i, _i, _p],
+    "viola_store_words": [_p, _p, _l, _p],
     "viola_selftest_fp8": [_p, _p],
     "viola_selftest_philox": [_p, _p, _l, _p],
 }
-EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan")
+EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan", "viola_tensor_encode_slices")
 
 _lib = None
 
@@ -85,10 +93,24 @@ def library():
             fn.argtypes, fn.restype = argtypes, ctypes.c_int
         lib.viola_abi_version.restype = ctypes.c_int
         lib.viola_error_string.argtypes, lib.viola_error_string.restype = [ctypes.c_int], ctypes.c_char_p
+        lib.viola_tensor_encode_slices.argtypes, lib.viola_tensor_encode_slices.restype = [_i, _l, _l], ctypes.c_int64
         lib.viola_ns_plan.argtypes, lib.viola_ns_plan.restype = [_l, _l, _l, _l, _i, _i, _i, ctypes.POINTER(ctypes.c_int)], ctypes.c_int
         assert lib.viola_abi_version() == 1
         _lib = lib
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host path (csrc/host.cpp): autograd nodes of the modules' standard recipes over the same entry points."""
+    global _host
+    if _host is None:
+        library()                                              # raises with build instructions when nothing is built
+        _host = importlib.import_module("viola_amd.csrc._host")
+        _host.set_timeline(_timeline)
+    return _host
 
 
 def ptr(tensor):
@@ -111,19 +133,38 @@ def stream():
     return torch.cuda.current_stream().cuda_stream
 
 
-timeline = None   # when a list, every call appends (name, start_event, end_event) recorded on the current stream
+_timeline = None
+
+
+class _Module(types.ModuleType):
+    """This module, with `timeline`: when set to a list, every call, from Python or from the native host path, appends
+    (name, start_event, end_event) recorded on the current stream."""
+
+    @property
+    def timeline(self):
+        return _timeline
+
+    @timeline.setter
+    def timeline(self, value):
+        global _timeline
+        _timeline = value
+        if _host is not None:
+            _host.set_timeline(value)
+
+
+sys.modules[__name__].__class__ = _Module
 
 
 def call(name, *args, unsupported_ok=False):
     """Invoke one entry point on the current stream; non-zero status raises (VIOLA_EUNSUPPORTED is returned instead
     when the caller has another route)."""
     lib = library()
-    if timeline is not None:
+    if _timeline is not None:
         start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         start.record()
         status = getattr(lib, name)(*args, stream())
         end.record()
-        timeline.append((name, start, end))
+        _timeline.append((name, start, end))
     else:
         status = getattr(lib, name)(*args, stream())
     if status == -2 and unsupported_ok:

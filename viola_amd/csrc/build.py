@@ -1,4 +1,5 @@
-"""Build libviola_hip.so for gfx950 with hipcc, in-tree next to the sources.
+"""Build libviola_hip.so for gfx950 with hipcc, and _host.so (the native host path) with the system compiler, in-tree next to
+the sources.
 
 python -m viola_amd.csrc.build        (or called by __graft_entry__.build())
 """
@@ -11,6 +12,7 @@ from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 LIBRARY = HERE / "libviola_hip.so"
+HOST_LIBRARY = HERE / "_host.so"                                          # Python extension: host.cpp over the C ABI
 ARCH = "gfx950"
 # -ffp-contract=off: the quantize / optimizer / codec kernels follow the reference's un-fused
 # fp32 operation order so FP8 codes and scales come out bit-exact. The GEMM files apply their
@@ -29,6 +31,28 @@ def hipcc():
 
 def _filter(text):
     return "\n".join(line for line in text.splitlines() if "is not a recognized feature for this target" not in line)
+
+
+def _host_command():
+    """host.cpp is host code only (autograd nodes, no kernels): the system compiler, torch's headers, the library above."""
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    torch_lib = Path(torch.__file__).parent / "lib"
+    includes = [f"-I{path}" for path in include_paths("cuda")] + [f"-I{sysconfig.get_paths()['include']}"]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-DTORCH_EXTENSION_NAME=_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, str(HERE / "host.cpp"),
+            "-o", str(HOST_LIBRARY), str(LIBRARY), f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+            "-Wl,-rpath,$ORIGIN"]
+
+
+def _build_host(incremental):
+    sources = [HERE / "host.cpp", HERE.parents[1] / "include" / "viola_hip.h"]
+    if incremental and HOST_LIBRARY.exists() and HOST_LIBRARY.stat().st_mtime > max(f.stat().st_mtime for f in sources):
+        return
+    result = subprocess.run(_host_command(), capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError("building the native host path failed:\n" + result.stdout + result.stderr)
 
 
 def build(verbose=True, incremental=False):
@@ -53,10 +77,11 @@ def build(verbose=True, incremental=False):
 
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
         objects = list(pool.map(compile_one, SOURCES))
-    link = [compiler, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(LIBRARY)]
+    link = [compiler, f"--offload-arch={ARCH}", "-shared", "-fPIC", f"-Wl,-soname,{LIBRARY.name}", *map(str, objects), "-o", str(LIBRARY)]
     result = subprocess.run(link, capture_output=True, text=True)
     if result.returncode != 0:
         raise RuntimeError("link failed:\n" + _filter(result.stdout + result.stderr))
+    _build_host(incremental)
     return LIBRARY
 
 

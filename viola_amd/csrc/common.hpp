@@ -348,4 +348,43 @@ __device__ __forceinline__ void gate_math(int activation, float g, float& act, f
     }
 }
 
+// out[c] = sum over p of partial[p][c] for the 32 columns of `block`, in a fixed order: 8 threads per column each add a
+// contiguous eighth of the parts in ascending order (loads issued 32 or eight at a time), then the eighths are added in
+// order. 256 threads; `piece` is 1 KB of LDS.
+template <typename TO>
+__device__ __forceinline__ void reduce_columns(const float* __restrict__ partial, int64_t parts, int64_t cols, TO* __restrict__ out,
+                                               int64_t block, float (*piece)[32]) {
+    const int c = threadIdx.x % 32, slice = threadIdx.x / 32;
+    const int64_t col = block * 32 + c;
+    const int64_t per = (parts + 7) / 8;
+    const int64_t begin = slice * per, end = begin + per < parts ? begin + per : parts;
+    float sum = 0.0f;
+    if (col < cols) {
+        int64_t part = begin;
+        for (; part + 32 <= end; part += 32) {                              // same order of additions, four times the loads in flight
+            float v[32];
+#pragma unroll
+            for (int u = 0; u < 32; ++u) v[u] = partial[(part + u) * cols + col];
+#pragma unroll
+            for (int u = 0; u < 32; ++u) sum += v[u];
+        }
+        for (; part + 8 <= end; part += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = partial[(part + u) * cols + col];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) sum += v[u];
+        }
+        for (; part < end; ++part) sum += partial[part * cols + col];
+    }
+    piece[slice][c] = sum;
+    __syncthreads();
+    if (slice == 0 && col < cols) {
+        float total = piece[0][c];
+#pragma unroll
+        for (int u = 1; u < 8; ++u) total += piece[u][c];
+        out[col] = from_f32<TO>(total);
+    }
+}
+
 }  // namespace viola

@@ -1,0 +1,902 @@
+// The Python operators' host path in native code: forward and backward of Linear, MLP and the variable-group linear for the
+// standard recipes, as autograd nodes that marshal tensors into libviola_hip's entry points.
+//
+// Why it is native: a forward + backward of a small layer is a dozen kernels of 3-6 us each, and the Python marshalling
+// around them (autograd.Function, one tensor per buffer, ctypes) took 130-200 us per step, three times the kernels. Here a
+// pass allocates one arena per lifetime (scratch of the call, what is kept for backward) and carves raw pointers out of it,
+// and backward runs on autograd's device thread without the interpreter.
+//
+// Row pitches: every GEMM operand made here has rows of a whole number of 128 k where its k axis is a token count (weight
+// gradient), and of 16 k (128 under E8M0 scales) otherwise, padded with zero codes, and the GEMM takes the pitch as its k.
+// The sums do not change; whatever the sizes, the kernels that load 16-byte pieces take the product.
+#include <torch/extension.h>
+
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include <atomic>
+#include <memory>
+#include <string>
+#include <vector>
+
+#include "../../include/viola_hip.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+namespace {
+
+// ---------------------------------------------------------------------------------------------------- calls
+// Instrumented mode (the `timeline` of viola_amd._lib): every call is bracketed by two timing events on the current stream.
+std::atomic<bool> recording{false};
+// the list and torch.cuda.Event; process-wide and never released (the interpreter may be gone before static destructors run)
+py::object* timeline_sink = nullptr;
+py::object* event_class = nullptr;
+
+void check(const char* name, int status) {
+    TORCH_CHECK(status == 0, name, " failed: ", viola_error_string(status), " (status ", status, ")");
+}
+
+template <typename F>
+int timed(const char* name, F&& f) {
+    if (__builtin_expect(!recording.load(std::memory_order_relaxed), 1)) return f();
+    py::gil_scoped_acquire gil;
+    if (!timeline_sink || timeline_sink->is_none()) return f();
+    py::object start = (*event_class)(py::arg("enable_timing") = true), end = (*event_class)(py::arg("enable_timing") = true);
+    start.attr("record")();
+    const int status = f();
+    end.attr("record")();
+    timeline_sink->attr("append")(py::make_tuple(name, start, end));
+    return status;
+}
+// VIOLA_CALL raises on a non-zero status, VIOLA_TRY hands VIOLA_EUNSUPPORTED back to a caller that has another route
+#define VIOLA_CALL(fn, ...) check(#fn, timed(#fn, [&] { return fn(__VA_ARGS__); }))
+#define VIOLA_TRY(fn, ...) timed(#fn, [&] { return fn(__VA_ARGS__); })
+
+int code_of(at::ScalarType t) {
+    switch (t) {
+        case at::kFloat: return VIOLA_F32;
+        case at::kBFloat16: return VIOLA_BF16;
+        case at::kHalf: return VIOLA_F16;
+        case at::kFloat8_e4m3fn: return VIOLA_E4M3;
+        case at::kFloat8_e5m2: return VIOLA_E5M2;
+        default: TORCH_CHECK(false, "viola_amd kernels do not take tensors of type ", t);
+    }
+}
+
+viola_stream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+const void* ptr(const Tensor& t) { return t.defined() && t.numel() ? t.const_data_ptr() : nullptr; }
+int64_t ceil_to(int64_t n, int64_t unit) { return (n + unit - 1) / unit * unit; }
+int64_t ceil_div(int64_t n, int64_t unit) { return (n + unit - 1) / unit; }
+
+// Several buffers of one lifetime as one allocation: take() reserves, make() allocates, at() hands out addresses.
+class Arena {
+public:
+    int64_t take(int64_t bytes) {
+        const int64_t begin = size_;
+        size_ += ceil_to(bytes, 256);
+        return begin;
+    }
+    void make(const at::Device& device) {
+        if (size_) buffer_ = at::empty({size_}, at::TensorOptions().dtype(at::kByte).device(device));
+    }
+    void* at(int64_t offset) const { return static_cast<char*>(buffer_.mutable_data_ptr()) + offset; }
+    template <typename T> T* as(int64_t offset) const { return static_cast<T*>(at(offset)); }
+    void release() { buffer_ = Tensor(); }
+
+private:
+    int64_t size_ = 0;
+    Tensor buffer_;
+};
+
+// ---------------------------------------------------------------------------------------------------- recipes
+// Calls of one per-tensor quantizer so far (its slot in the amax history); shared with nodes that advance it in backward.
+struct Counter {
+    int64_t value = 0;
+};
+
+// What a Linear's constructor fixed about its arithmetic. Standard recipes only: (1, 32) activation and gradient groups,
+// (32, 32) weight blocks, FP32 accumulation, no rotation, FP8-saved inputs.
+struct Recipe {
+    bool grouped = false, native = false, delayed = false;      // native: E8M0 scales; not grouped: one FP32 scale per tensor
+    bool fp8_weight = true, cache_transpose = false;
+    int fwd = VIOLA_E4M3, bwd = VIOLA_E4M3;
+    float fwd_limit = 448.0f, bwd_limit = 448.0f;
+    int64_t in = 0, out = 0;
+
+    explicit Recipe(const py::dict& d) {
+        grouped = d["grouped"].cast<bool>(); native = d["native"].cast<bool>(); delayed = d["delayed"].cast<bool>();
+        fp8_weight = d["fp8_weight"].cast<bool>(); cache_transpose = d["cache_transpose"].cast<bool>();
+        fwd = d["fwd"].cast<int>(); bwd = d["bwd"].cast<int>();
+        fwd_limit = d["fwd_limit"].cast<float>(); bwd_limit = d["bwd_limit"].cast<float>();
+        in = d["in"].cast<int64_t>(); out = d["out"].cast<int64_t>();
+    }
+    py::dict fields() const {                                    // for copies and pickles of a module
+        using namespace py::literals;
+        return py::dict("grouped"_a = grouped, "native"_a = native, "delayed"_a = delayed, "fp8_weight"_a = fp8_weight,
+                        "cache_transpose"_a = cache_transpose, "fwd"_a = fwd, "bwd"_a = bwd, "fwd_limit"_a = fwd_limit, "bwd_limit"_a = bwd_limit,
+                        "in"_a = in, "out"_a = out);
+    }
+    int scale_format() const { return native ? VIOLA_SCALE_E8M0 : VIOLA_SCALE_F32; }
+    int64_t scale_bytes() const { return native ? 1 : 4; }
+    int64_t pitch(int64_t k) const { return native ? ceil_to(k, 128) : k % 16 == 0 ? k : ceil_to(k, 128); }
+};
+
+// The tensors of one Linear, fetched from the module for this call.
+struct Layer {
+    std::shared_ptr<Recipe> recipe;
+    Tensor weight, bias, scale, transpose, transpose_scale;
+    // per-tensor recipes: history and counter of the weight, input and gradient quantizers
+    Tensor history[3];
+    std::shared_ptr<Counter> counter[3];
+};
+enum { WEIGHT = 0, INPUT = 1, GRAD = 2 };
+
+// Codes and scales of one operand; rows `pitch` codes apart.
+struct Codes {
+    const void* q = nullptr;
+    const void* s = nullptr;
+    int64_t pitch = 0;
+};
+
+
+// What a projection's backward needs, and where it lives.
+struct Kept {
+    Arena arena;                                                 // transposed codes of the input (+ its scale)
+    Codes input_t;
+    const float* input_scale = nullptr;                          // per-tensor recipes
+    SavedVariable weight;
+    Tensor weight_scale, weight_t, weight_t_scale;
+    int64_t rows = 0;
+    at::ScalarType x_dtype = at::kFloat, weight_grad = at::kFloat, bias_grad = at::kFloat;
+    bool has_input = false;
+
+    void release() {
+        arena.release();
+        weight.reset_data();
+        weight_scale = weight_t = weight_t_scale = Tensor();
+    }
+};
+
+// ---------------------------------------------------------------------------------------------------- products
+// out[m, n] = a b^T, k = the operands' common pitch. br: rows of b per scale row (32: weight blocks, 1: row-wise).
+void product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_fmt, int64_t m, int64_t n, int br, const Tensor& bias,
+             void* out, at::ScalarType out_dtype, const at::Device& device, viola_stream_t stream) {
+    const int64_t k = a.pitch;
+    TORCH_INTERNAL_ASSERT(b.pitch == k);
+    const void* bias_p = ptr(bias);
+    const int bias_code = bias_p ? code_of(bias.scalar_type()) : 0, out_code = code_of(out_dtype);
+    if (!r.grouped) {
+        VIOLA_CALL(viola_tensor_gemm, a.q, a_fmt, b.q, b_fmt, static_cast<const float*>(a.s), static_cast<const float*>(b.s), m, n, k, bias_p,
+                   bias_code, out, out_code, stream);
+        return;
+    }
+    const float *sa = static_cast<const float*>(a.s), *sb = static_cast<const float*>(b.s);
+    Tensor decoded[2];
+    if (r.native) {
+        const int status = VIOLA_TRY(viola_mx_gemm, a.q, a_fmt, b.q, b_fmt, static_cast<const uint8_t*>(a.s), static_cast<const uint8_t*>(b.s), m, n,
+                                     k, 1, br, bias_p, bias_code, out, out_code, stream);
+        if (status == 0) return;
+        if (status != VIOLA_EUNSUPPORTED) check("viola_mx_gemm", status);
+        // operands beyond 2 GiB, which the block-scaled kernel declines: the same product with the scales spelled out in FP32
+        const int64_t rows[2] = {m, ceil_div(n, br)};
+        const void* bytes[2] = {a.s, b.s};
+        for (int i = 0; i < 2; ++i) {
+            const Tensor view = at::from_blob(const_cast<void*>(bytes[i]), {rows[i], ceil_div(k, 32)}, at::TensorOptions().dtype(at::kByte).device(device));
+            decoded[i] = at::exp2(view.to(at::kFloat) - 127.0f);
+        }
+        sa = decoded[0].const_data_ptr<float>();
+        sb = decoded[1].const_data_ptr<float>();
+    }
+    VIOLA_CALL(viola_group_gemm, a.q, a_fmt, b.q, b_fmt, sa, sb, m, n, k, 1, 32, br, 32, bias_p, bias_code, out, out_code, stream);
+}
+
+// The gated projections: forward aux = [g | u], out = act(g) * u (aux may be null); backward aux read, out = [d u act'(g) | d act(g)].
+void gated_product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_fmt, int64_t m, int64_t h, const Tensor& bias, const Tensor& aux_or_empty,
+                   const Tensor& out, int activation, bool backward, viola_stream_t stream) {
+    const int64_t k = a.pitch;
+    TORCH_INTERNAL_ASSERT(b.pitch == k);
+    const void* bias_p = ptr(bias);
+    const int bias_code = bias_p ? code_of(bias.scalar_type()) : 0, dtype = code_of(out.scalar_type());
+    void* aux = const_cast<void*>(ptr(aux_or_empty));
+    void* to = const_cast<void*>(ptr(out));
+    if (!r.grouped) {
+        VIOLA_CALL(viola_tensor_gated_gemm, a.q, a_fmt, b.q, b_fmt, static_cast<const float*>(a.s), static_cast<const float*>(b.s), m, h, k, bias_p,
+                   bias_code, aux, to, dtype, activation, backward, stream);
+        return;
+    }
+    if (!r.native) {
+        VIOLA_CALL(viola_gated_gemm, a.q, a_fmt, b.q, b_fmt, static_cast<const float*>(a.s), static_cast<const float*>(b.s), m, h, k, 1, 32, 32, 32,
+                   bias_p, bias_code, aux, to, dtype, activation, backward, stream);
+        return;
+    }
+    const int status = VIOLA_TRY(viola_mx_gated_gemm, a.q, a_fmt, b.q, b_fmt, static_cast<const uint8_t*>(a.s), static_cast<const uint8_t*>(b.s), m, h, k, 1,
+                                 32, bias_p, bias_code, aux, to, dtype, activation, backward, stream);
+    if (status == 0) return;
+    if (status != VIOLA_EUNSUPPORTED) check("viola_mx_gated_gemm", status);
+    // up rows off the scale grid (h not a multiple of 32): the same values from the plain product and the elementwise kernels
+    if (backward) {
+        const Tensor d = at::empty({m, h}, out.options());
+        product(r, a, a_fmt, b, b_fmt, m, h, 32, Tensor(), d.mutable_data_ptr(), out.scalar_type(), out.device(), stream);
+        VIOLA_CALL(viola_gated_backward, aux, ptr(d), to, m, h, dtype, activation, stream);
+    } else {
+        const Tensor z = aux ? aux_or_empty : at::empty({m, 2 * h}, out.options());
+        product(r, a, a_fmt, b, b_fmt, m, 2 * h, 32, bias, z.mutable_data_ptr(), out.scalar_type(), out.device(), stream);
+        VIOLA_CALL(viola_gated_forward, ptr(z), to, m, h, dtype, activation, stream);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------- quantizers
+// Row-wise and / or transposed codes of a grouped operand into reserved arena space.
+struct GroupSpace {
+    int64_t q = -1, s = -1, qt = -1, st = -1, pitch = 0, pitch_t = 0;
+    void reserve(const Recipe& r, Arena* rowwise, Arena* transposed, int64_t rows, int64_t cols) {
+        pitch = r.pitch(cols);
+        pitch_t = ceil_to(rows, 128);
+        if (rowwise) { q = rowwise->take(rows * pitch); s = rowwise->take(rows * ceil_div(pitch, 32) * r.scale_bytes()); }
+        if (transposed) { qt = transposed->take(cols * pitch_t); st = transposed->take(cols * (pitch_t / 32) * r.scale_bytes()); }
+    }
+};
+
+void quantize_groups(const Recipe& r, const Tensor& x, int fmt, float limit, const GroupSpace& g, const Arena* rowwise, const Arena* transposed,
+                     float* column_partial, Codes* out, Codes* out_t, viola_stream_t stream) {
+    const int64_t rows = x.size(0), cols = x.size(1);
+    void *q = nullptr, *s = nullptr, *qt = nullptr, *st = nullptr;
+    if (g.q >= 0) { q = rowwise->at(g.q); s = rowwise->at(g.s); *out = {q, s, g.pitch}; }
+    if (g.qt >= 0) { qt = transposed->at(g.qt); st = transposed->at(g.st); *out_t = {qt, st, g.pitch_t}; }
+    const int dtype = code_of(x.scalar_type());
+    if (!qt && g.pitch == cols)                                  // row-wise only: the streaming kernel
+        VIOLA_CALL(viola_group_quantize, ptr(x), dtype, rows, cols, q, fmt, s, 1, 32, limit, 0, nullptr, 1, 32, r.scale_format(), stream);
+    else
+        VIOLA_CALL(viola_group_quantize_dual_pitched, ptr(x), dtype, rows, cols, q, g.pitch, s, qt, qt ? g.pitch_t : rows, st, fmt, limit, column_partial,
+                   r.scale_format(), stream);
+}
+
+Tensor as_matrix(const Tensor& t, int64_t cols) {
+    const Tensor flat = t.dim() == 2 ? t : t.reshape({-1, cols});
+    TORCH_CHECK(flat.size(1) == cols, "expected ", cols, " features, got ", flat.size(1));
+    return flat.is_contiguous() ? flat : flat.contiguous();
+}
+
+// Codes of the weight as the forward GEMM reads them: the stored ones, or for 16-bit storage freshly made; repacked where
+// the rows are not whole pieces.
+struct WeightSpace {
+    int64_t q = -1, s = -1, p = -1, ps = -1, pitch = 0;
+};
+
+WeightSpace reserve_weight(const Layer& l, Arena& temp) {
+    const Recipe& r = *l.recipe;
+    WeightSpace w;
+    w.pitch = r.pitch(r.in);
+    const int64_t scale_rows = ceil_div(r.out, 32);
+    if (!r.fp8_weight) {
+        w.q = temp.take(r.out * r.in);
+        w.s = temp.take(r.grouped ? scale_rows * ceil_div(r.in, 32) * r.scale_bytes() : 4);
+    }
+    if (w.pitch != r.in) {
+        w.p = temp.take(r.out * w.pitch);
+        if (r.grouped) w.ps = temp.take(scale_rows * ceil_div(w.pitch, 32) * r.scale_bytes());
+    }
+    return w;
+}
+
+// `scale_out` (per-tensor recipes with 16-bit storage): where the weight's scale goes instead of the arena
+Codes stored_weight(const Layer& l, const Tensor& weight, const WeightSpace& w, const Arena& temp, float* scale_out, Codes* unpadded, viola_stream_t stream) {
+    const Recipe& r = *l.recipe;
+    Codes c{ptr(weight), ptr(l.scale), r.in};
+    if (!r.fp8_weight) {
+        const int dtype = code_of(weight.scalar_type());
+        if (r.grouped) {
+            c = {temp.at(w.q), temp.at(w.s), r.in};
+            VIOLA_CALL(viola_group_quantize, ptr(weight), dtype, r.out, r.in, temp.at(w.q), r.fwd, temp.at(w.s), 32, 32, r.fwd_limit, 0, nullptr, 1, 32,
+                       r.scale_format(), stream);
+        } else {
+            // a temporary workspace of block maxima
+            Arena maxima;
+            const int64_t at = maxima.take(1024 * 4);
+            maxima.make(weight.device());
+            c = {temp.at(w.q), scale_out, r.in};
+            const Tensor& history = l.history[WEIGHT];
+            VIOLA_CALL(viola_tensor_encode, ptr(weight), dtype, r.out, r.in, maxima.as<float>(at), 1024, static_cast<float*>(history.mutable_data_ptr()),
+                       (int)history.numel(), l.counter[WEIGHT]->value, r.delayed, r.fwd_limit, scale_out, temp.at(w.q), r.in, nullptr, 0, r.fwd, nullptr,
+                       VIOLA_F32, stream);
+            ++l.counter[WEIGHT]->value;
+        }
+    }
+    if (unpadded) *unpadded = c;
+    if (w.pitch != r.in) {
+        void* scale_to = r.grouped ? temp.at(w.ps) : nullptr;
+        VIOLA_CALL(viola_codes_repack, c.q, temp.at(w.p), 1, r.out, r.in, w.pitch, r.grouped ? c.s : nullptr, scale_to, 32, 32, r.scale_format(), stream);
+        c = {temp.at(w.p), r.grouped ? scale_to : c.s, w.pitch};
+    }
+    return c;
+}
+
+// ---------------------------------------------------------------------------------------------------- one projection
+// gated < 0: y = x W^T + b. gated >= 0 (an activation): y = act(g) * u of [g | u] = x W^T + b, and *aux = [g | u] when kept.
+// hidden_codes: (gated, E8M0) hand y over as codes instead of values; input_codes: x arrives that way.
+struct CodedHidden {
+    Arena temp;                                                  // row-wise codes, used by this forward only
+    Codes codes;
+    Codes codes_t;                                               // in the down projection's Kept arena
+};
+
+struct Forward {
+    Tensor y, aux;
+};
+
+Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool need_backward, bool needs_w, Kept& kept, int gated, bool keep_aux,
+                CodedHidden* hidden_out, Kept* hidden_kept, bool hidden_transposed, const CodedHidden* coded_input) {
+    const Recipe& r = *l.recipe;
+    const bool save = need_backward && needs_w;
+    const int64_t rows = coded_input ? kept.rows : x2.size(0);
+    const at::Device device = l.weight.device();
+    const viola_stream_t stream = stream_of(l.weight);
+    kept.rows = rows;
+    kept.x_dtype = dtype;
+    kept.has_input = save;
+    if (need_backward) {
+        kept.weight = SavedVariable(l.weight, false);
+        kept.weight_scale = l.scale;
+        kept.weight_t = l.transpose;
+        kept.weight_t_scale = l.transpose_scale;
+        kept.weight_grad = l.weight.grad_dtype().value_or(l.weight.scalar_type());
+        if (l.bias.defined()) kept.bias_grad = l.bias.grad_dtype().value_or(l.bias.scalar_type());
+    }
+    const auto options = at::TensorOptions().dtype(dtype).device(device);
+    const int64_t h = r.out / 2;
+    Forward f;
+    if (rows == 0) {
+        f.y = at::empty({0, gated < 0 ? r.out : h}, options);
+        if (gated >= 0 && keep_aux) f.aux = at::empty({0, r.out}, options);
+        return f;
+    }
+    Arena temp;
+    const WeightSpace wspace = reserve_weight(l, temp);
+    Codes a, w, w_unpadded;
+    const bool cache_here = !r.fp8_weight && need_backward && r.cache_transpose;   // 16-bit storage: W^T of this forward's codes
+    if (r.grouped) {
+        GroupSpace g;
+        if (!coded_input) g.reserve(r, &temp, save ? &kept.arena : nullptr, rows, r.in);
+        temp.make(device);
+        if (save && !coded_input) kept.arena.make(device);
+        if (coded_input) {
+            a = coded_input->codes;
+            kept.input_t = coded_input->codes_t;
+        } else {
+            quantize_groups(r, x2, r.fwd, r.fwd_limit, g, &temp, &kept.arena, nullptr, &a, &kept.input_t, stream);
+        }
+        w = stored_weight(l, l.weight, wspace, temp, nullptr, &w_unpadded, stream);
+    } else {
+        const int64_t pitch = r.pitch(r.in), pitch_t = ceil_to(rows, 128);
+        const int64_t q = temp.take(rows * pitch), maxima = temp.take(1024 * 4);
+        const int64_t qt = save ? kept.arena.take(r.in * pitch_t) : -1;
+        const int64_t scales = kept.arena.take(8);               // of x and of a 16-bit weight: backward uses these very values
+        temp.make(device);
+        kept.arena.make(device);
+        float* sx = kept.arena.as<float>(scales);
+        const Tensor& history = l.history[INPUT];
+        VIOLA_CALL(viola_tensor_encode, ptr(x2), code_of(x2.scalar_type()), rows, r.in, temp.as<float>(maxima), 1024,
+                   static_cast<float*>(history.mutable_data_ptr()), (int)history.numel(), l.counter[INPUT]->value, r.delayed, r.fwd_limit, sx, temp.at(q),
+                   pitch, save ? kept.arena.at(qt) : nullptr, save ? pitch_t : 0, r.fwd, nullptr, VIOLA_F32, stream);
+        ++l.counter[INPUT]->value;
+        a = {temp.at(q), sx, pitch};
+        kept.input_scale = sx;
+        if (save) kept.input_t = {kept.arena.at(qt), sx, pitch_t};
+        w = stored_weight(l, l.weight, wspace, temp, sx + 1, &w_unpadded, stream);
+    }
+    if (cache_here) {
+        kept.weight_t = at::empty({r.in, r.out}, at::TensorOptions().dtype(at::kByte).device(device));
+        const bool grid = r.grouped;
+        if (grid) kept.weight_t_scale = at::empty({ceil_div(r.in, 32), ceil_div(r.out, 32)}, at::TensorOptions().dtype(r.native ? at::kByte : at::kFloat).device(device));
+        VIOLA_CALL(viola_codes_transpose_pitched, w_unpadded.q, kept.weight_t.mutable_data_ptr(), 1, r.out, r.in, r.out, grid ? w_unpadded.s : nullptr,
+                   grid ? kept.weight_t_scale.mutable_data_ptr() : nullptr, 32, 32, r.scale_format(), nullptr, 0, 0, nullptr, 0, stream);
+    }
+    if (gated < 0) {
+        f.y = at::empty({rows, r.out}, options);
+        product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, l.bias, f.y.mutable_data_ptr(), dtype, device, stream);
+        return f;
+    }
+    if (keep_aux) f.aux = at::empty({rows, r.out}, options);
+    if (hidden_out) {
+        // h leaves the product as codes with E8M0 scales in the layouts the down projection reads (its k is h wide)
+        Arena& keep = hidden_kept->arena;
+        const int64_t q = hidden_out->temp.take(rows * h), s = hidden_out->temp.take(rows * (h / 32));
+        const int64_t qt = hidden_transposed ? keep.take(h * rows) : -1, st = hidden_transposed ? keep.take(h * (rows / 32)) : -1;
+        hidden_out->temp.make(device);
+        keep.make(device);
+        void* qt_p = hidden_transposed ? keep.at(qt) : nullptr;
+        uint8_t* st_p = hidden_transposed ? keep.as<uint8_t>(st) : nullptr;
+        const void* bias_p = ptr(l.bias);
+        const int status = VIOLA_TRY(viola_mx_gated_gemm_encode, a.q, r.fwd, w.q, r.fwd, static_cast<const uint8_t*>(a.s), static_cast<const uint8_t*>(w.s), rows, h,
+                                     a.pitch, 1, 32, bias_p, bias_p ? code_of(l.bias.scalar_type()) : 0, const_cast<void*>(ptr(f.aux)), code_of(dtype),
+                                     hidden_out->temp.at(q), hidden_out->temp.as<uint8_t>(s), qt_p, st_p, r.fwd, r.fwd_limit, gated, stream);
+        if (status != 0 && status != VIOLA_EUNSUPPORTED) check("viola_mx_gated_gemm_encode", status);
+        if (status == 0) {
+            hidden_out->codes = {hidden_out->temp.at(q), hidden_out->temp.at(s), h};
+            hidden_out->codes_t = {qt_p, st_p, rows};
+            hidden_kept->rows = rows;
+            return f;
+        }
+        keep.release();
+        hidden_kept->arena = Arena();
+    }
+    f.y = at::empty({rows, h}, options);
+    gated_product(r, a, r.fwd, w, r.fwd, rows, h, l.bias, f.aux, f.y, gated, false, stream);
+    return f;
+}
+
+struct Gradients {
+    Tensor dx, dw, db;
+};
+
+// gated >= 0: dx is dz = [d u act'(g) | d act(g)] from aux = [g | u]. (w: the unpacked weight of the layer.)
+Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& dy_, bool needs_x, bool needs_w, bool needs_b, int gated, const Tensor& aux) {
+    const Recipe& r = *l.recipe;
+    const int64_t rows = kept.rows;
+    const at::Device device = w.device();
+    const viola_stream_t stream = stream_of(w);
+    const auto dx_options = at::TensorOptions().dtype(kept.x_dtype).device(device);
+    const int64_t dx_cols = gated < 0 ? r.in : 2 * r.in;
+    Gradients out;
+    if (rows == 0) {
+        if (needs_x) out.dx = at::zeros({0, dx_cols}, dx_options);
+        if (needs_w) out.dw = at::zeros({r.out, r.in}, dx_options.dtype(kept.weight_grad));
+        if (needs_b) out.db = at::zeros({r.out}, dx_options.dtype(kept.bias_grad));
+        return out;
+    }
+    const Tensor dy = as_matrix(dy_, r.out);
+    Arena temp;
+    Codes g, gt, wt;
+    float* partial = nullptr;
+    const int64_t parts = ceil_div(rows, 32), pitch = r.pitch(r.out);
+    // ---- space for the transposed weight
+    const bool cached = kept.weight_t.defined() && kept.weight_t.numel();
+    const bool make_wt = needs_x && !(cached && pitch == r.out);
+    const int64_t wt_q = make_wt ? temp.take(r.in * pitch) : -1, wt_s = make_wt && r.grouped ? temp.take(ceil_div(r.in, 32) * ceil_div(pitch, 32) * r.scale_bytes()) : -1;
+    const bool requantize = make_wt && !cached && !r.fp8_weight; // memory mode with 16-bit storage: this forward's codes again
+    const int64_t w_q = requantize ? temp.take(r.out * r.in) : -1;
+    const int64_t w_s = requantize && r.grouped ? temp.take(ceil_div(r.out, 32) * ceil_div(r.in, 32) * r.scale_bytes()) : -1;
+    if (needs_b) out.db = at::empty({r.out}, dx_options.dtype(kept.bias_grad));
+    if (r.grouped) {
+        GroupSpace space;
+        space.reserve(r, needs_x ? &temp : nullptr, needs_w ? &temp : nullptr, rows, r.out);
+        const bool rides = needs_b && needs_w;                   // the bias gradient's 32-row sums come from the quantizer's read of dy
+        const int64_t partial_at = rides ? temp.take(parts * r.out * 4) : -1;
+        temp.make(device);
+        if (rides) partial = temp.as<float>(partial_at);
+        if (needs_x || needs_w) quantize_groups(r, dy, r.bwd, r.bwd_limit, space, &temp, &temp, partial, &g, &gt, stream);
+        if (needs_b && !rides) out.db = at::sum(dy, at::IntArrayRef{0}, false, kept.bias_grad);
+    } else {
+        const int64_t pitch_t = ceil_to(rows, 128);
+        const int64_t q = needs_x ? temp.take(rows * pitch) : -1, qt = needs_w ? temp.take(r.out * pitch_t) : -1, scale_at = temp.take(4);
+        const int dtype = code_of(dy.scalar_type());
+        bool rides = needs_b;
+        const int64_t floats = 1024 + (rides ? viola_tensor_encode_slices(dtype, rows, r.out) * r.out : 0), work_at = temp.take(floats * 4);
+        temp.make(device);
+        float* scale = temp.as<float>(scale_at);
+        const Tensor& history = l.history[GRAD];
+        auto encode = [&](bool with_sum) {
+            return VIOLA_TRY(viola_tensor_encode, ptr(dy), dtype, rows, r.out, temp.as<float>(work_at), floats, static_cast<float*>(history.mutable_data_ptr()),
+                             (int)history.numel(), l.counter[GRAD]->value, r.delayed, r.bwd_limit, scale, needs_x ? temp.at(q) : nullptr, pitch,
+                             needs_w ? temp.at(qt) : nullptr, pitch_t, r.bwd, with_sum ? out.db.mutable_data_ptr() : nullptr,
+                             with_sum ? code_of(kept.bias_grad) : VIOLA_F32, stream);
+        };
+        int status = encode(rides);
+        if (status == VIOLA_EUNSUPPORTED && rides) {             // columns that are not whole 16-byte pieces: the sum as a pass of its own
+            out.db = at::sum(dy, at::IntArrayRef{0}, false, kept.bias_grad);
+            status = encode(false);
+        }
+        check("viola_tensor_encode", status);
+        ++l.counter[GRAD]->value;
+        if (needs_x) g = {temp.at(q), scale, pitch};
+        if (needs_w) gt = {temp.at(qt), scale, pitch_t};
+    }
+    if (needs_x) {
+        const void* w_scale = r.grouped ? ptr(kept.weight_scale) : r.fp8_weight ? ptr(kept.weight_scale) : kept.input_scale + 1;
+        wt = {ptr(kept.weight_t), r.grouped ? ptr(kept.weight_t_scale) : w_scale, pitch};
+        if (make_wt && cached) {
+            VIOLA_CALL(viola_codes_repack, ptr(kept.weight_t), temp.at(wt_q), 1, r.in, r.out, pitch, r.grouped ? ptr(kept.weight_t_scale) : nullptr,
+                       r.grouped ? temp.at(wt_s) : nullptr, 32, 32, r.scale_format(), stream);
+        } else if (make_wt) {
+            const void* codes = ptr(w);
+            if (requantize) {
+                codes = temp.at(w_q);
+                if (r.grouped) {
+                    w_scale = temp.at(w_s);
+                    VIOLA_CALL(viola_group_quantize, ptr(w), code_of(w.scalar_type()), r.out, r.in, temp.at(w_q), r.fwd, temp.at(w_s), 32, 32, r.fwd_limit, 0,
+                               nullptr, 1, 32, r.scale_format(), stream);
+                } else {
+                    VIOLA_CALL(viola_tensor_quantize, ptr(w), code_of(w.scalar_type()), r.out, r.in, static_cast<const float*>(w_scale), temp.at(w_q), nullptr,
+                               r.fwd, r.fwd_limit, stream);
+                }
+            }
+            VIOLA_CALL(viola_codes_transpose_pitched, codes, temp.at(wt_q), 1, r.out, r.in, pitch, r.grouped ? w_scale : nullptr,
+                       r.grouped ? temp.at(wt_s) : nullptr, 32, 32, r.scale_format(), partial, parts, r.out, partial ? out.db.mutable_data_ptr() : nullptr,
+                       partial ? code_of(kept.bias_grad) : VIOLA_F32, stream);
+            partial = nullptr;                                   // reduced by the same launch
+        }
+        if (make_wt) wt = {temp.at(wt_q), r.grouped ? temp.at(wt_s) : w_scale, pitch};
+    }
+    if (partial) VIOLA_CALL(viola_column_reduce, partial, parts, r.out, out.db.mutable_data_ptr(), code_of(kept.bias_grad), stream);
+    if (needs_x) {
+        out.dx = at::empty({rows, dx_cols}, dx_options);
+        if (gated < 0) product(r, g, r.bwd, wt, r.fwd, rows, r.in, 32, Tensor(), out.dx.mutable_data_ptr(), kept.x_dtype, device, stream);
+        else gated_product(r, g, r.bwd, wt, r.fwd, rows, r.in, Tensor(), aux, out.dx, gated, true, stream);
+    }
+    if (needs_w) {
+        out.dw = at::empty({r.out, r.in}, dx_options.dtype(kept.weight_grad));
+        product(r, gt, r.bwd, kept.input_t, r.fwd, r.out, r.in, 1, Tensor(), out.dw.mutable_data_ptr(), kept.weight_grad, device, stream);
+    }
+    return out;
+}
+
+bool wants(const Tensor& t) { return t.defined() && t.requires_grad(); }
+
+// ---------------------------------------------------------------------------------------------------- Linear
+struct LinearBackward : public Node {
+    Layer layer;                                                 // without its tensors, but for the quantizers' histories
+    Kept kept;
+    std::vector<int64_t> x_shape;
+
+    variable_list apply(variable_list&& grads) override {
+        const Tensor& dy = grads[0];
+        variable_list result(3);
+        if (!dy.defined()) return result;
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor weight = kept.weight.unpack();
+        Gradients g = unproject(layer, kept, weight, dy, task_should_compute_output(0), task_should_compute_output(1) && kept.has_input,
+                                task_should_compute_output(2), -1, Tensor());
+        if (g.dx.defined()) result[0] = g.dx.dim() == (int64_t)x_shape.size() ? g.dx : g.dx.view(x_shape);
+        result[1] = g.dw;
+        result[2] = g.db;
+        return result;
+    }
+    std::string name() const override { return "ViolaLinearBackward"; }
+    void release_variables() override { kept.release(); }
+};
+
+std::vector<int64_t> output_shape(const Tensor& x, int64_t features) {
+    std::vector<int64_t> shape = x.sizes().vec();
+    shape.back() = features;
+    return shape;
+}
+
+// The histories are updated in place by raw pointers; nothing else of the layer's tensors is kept by a node.
+Layer without_tensors(const Layer& l) {
+    Layer kept;
+    kept.recipe = l.recipe;
+    for (int i = 0; i < 3; ++i) { kept.history[i] = l.history[i]; kept.counter[i] = l.counter[i]; }
+    return kept;
+}
+
+Tensor linear(const Tensor& x, Layer& l) {
+    const bool wx = x.requires_grad(), ww = l.weight.requires_grad(), wb = wants(l.bias);
+    const bool need = at::GradMode::is_enabled() && (wx || ww || wb);
+    auto node = need ? std::shared_ptr<LinearBackward>(new LinearBackward(), torch::autograd::deleteNode) : nullptr;
+    Kept scratch;
+    Kept& kept = need ? node->kept : scratch;
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor x2 = as_matrix(x, l.recipe->in);
+        if (l.bias.defined() && !l.bias.is_contiguous()) l.bias = l.bias.contiguous();
+        y = project(l, x2, x.scalar_type(), need, ww, kept, -1, false, nullptr, nullptr, false, nullptr).y;
+        if (x.dim() != 2) y = y.view(output_shape(x, l.recipe->out));
+    }
+    if (need) {
+        node->layer = without_tensors(l);
+        node->x_shape = x.sizes().vec();
+        node->set_next_edges(torch::autograd::collect_next_edges(x, l.weight, l.bias));
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+// ---------------------------------------------------------------------------------------------------- MLP
+// One node for the whole gated MLP: dz, the gradient of [g | u], goes from the down projection's data-gradient product
+// (activation derivative in its epilogue) straight into the stacked gate/up projection's backward.
+struct MlpBackward : public Node {
+    Layer up, down;
+    Kept up_kept, down_kept;
+    SavedVariable z;
+    std::vector<int64_t> x_shape;
+    int activation = 0;
+    bool first_half = false;
+
+    variable_list apply(variable_list&& grads) override {
+        const Tensor& dy = grads[0];
+        variable_list result(5);
+        if (!dy.defined()) return result;
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor down_weight = down_kept.weight.unpack();
+        const Tensor up_weight = first_half ? up_kept.weight.unpack() : Tensor();
+        const bool upper = first_half && (task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2));
+        Gradients d = unproject(down, down_kept, down_weight, dy, upper, task_should_compute_output(3) && down_kept.has_input, task_should_compute_output(4),
+                                activation, upper ? z.unpack() : Tensor());
+        result[3] = d.dw;
+        result[4] = d.db;
+        if (!upper) return result;
+        Gradients u = unproject(up, up_kept, up_weight, d.dx, task_should_compute_output(0), task_should_compute_output(1) && up_kept.has_input,
+                                task_should_compute_output(2), -1, Tensor());
+        if (u.dx.defined()) result[0] = u.dx.dim() == (int64_t)x_shape.size() ? u.dx : u.dx.view(x_shape);
+        result[1] = u.dw;
+        result[2] = u.db;
+        return result;
+    }
+    std::string name() const override { return "ViolaMLPBackward"; }
+    void release_variables() override {
+        up_kept.release();
+        down_kept.release();
+        z.reset_data();
+    }
+};
+
+Tensor mlp(const Tensor& x, Layer& up, Layer& down, int activation) {
+    const bool grad = at::GradMode::is_enabled();
+    const bool up_w = up.weight.requires_grad(), down_w = down.weight.requires_grad();
+    const bool first_half = grad && (x.requires_grad() || up_w || wants(up.bias));
+    const bool whole = grad && (first_half || down_w || wants(down.bias));
+    auto node = whole ? std::shared_ptr<MlpBackward>(new MlpBackward(), torch::autograd::deleteNode) : nullptr;
+    Kept scratch_up, scratch_down;
+    Kept& up_kept = whole ? node->up_kept : scratch_up;
+    Kept& down_kept = whole ? node->down_kept : scratch_down;
+    Tensor y, z;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor x2 = as_matrix(x, up.recipe->in);
+        for (Layer* l : {&up, &down})
+            if (l->bias.defined() && !l->bias.is_contiguous()) l->bias = l->bias.contiguous();
+        const int64_t rows = x2.size(0), h = down.recipe->in;
+        // whole 128 x 128 pieces in both directions: the codes need no padding on either k axis of the down projection
+        const bool as_codes = up.recipe->native && rows > 0 && rows % 128 == 0 && h % 128 == 0;
+        CodedHidden hidden;
+        Forward first = project(up, x2, x.scalar_type(), first_half, up_w, up_kept, activation, first_half, as_codes ? &hidden : nullptr,
+                                as_codes ? &down_kept : nullptr, whole && down_w, nullptr);
+        z = first.aux;
+        const bool coded = !first.y.defined();
+        y = project(down, first.y, x.scalar_type(), whole, down_w, down_kept, -1, false, nullptr, nullptr, false, coded ? &hidden : nullptr).y;
+        if (x.dim() != 2) y = y.view(output_shape(x, down.recipe->out));
+    }
+    if (whole) {
+        node->up = without_tensors(up);
+        node->down = without_tensors(down);
+        node->activation = activation;
+        node->first_half = first_half;
+        node->x_shape = x.sizes().vec();
+        if (first_half) node->z = SavedVariable(z, false);
+        node->set_next_edges(torch::autograd::collect_next_edges(x, up.weight, up.bias, down.weight, down.bias));
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+// ---------------------------------------------------------------------------------------------------- variable groups
+struct Groups {
+    int64_t count = 0, rows = 0, padded = 0;
+    Arena arena;                                                 // row offsets, then offsets on the padded token axis
+    const int64_t* offsets = nullptr;
+    const int64_t* padded_offsets = nullptr;
+};
+
+// The offset tables travel as kernel arguments: no staging buffer, no copy the host has to wait for.
+void make_groups(Groups& g, const std::vector<int64_t>& counts, const at::Device& device, viola_stream_t stream) {
+    g.count = (int64_t)counts.size();
+    std::vector<int64_t> words(2 * (g.count + 1), 0);
+    int64_t* padded = words.data() + g.count + 1;
+    for (int64_t i = 0; i < g.count; ++i) {
+        TORCH_CHECK(counts[i] >= 0, "rows per group cannot be negative");
+        words[i + 1] = words[i] + counts[i];
+        padded[i + 1] = padded[i] + ceil_to(counts[i], 32);
+    }
+    // The padded token axis is the row length of the transposed codes: rounded up to 128 (empty slots at the end of the last
+    // group, zero codes) so that every row starts on a cache line and the quantizer's 64-byte pieces never straddle one.
+    padded[g.count] = ceil_to(padded[g.count], 128);
+    g.rows = words[g.count];
+    g.padded = padded[g.count];
+    const int64_t at = g.arena.take((int64_t)words.size() * 8);
+    g.arena.make(device);
+    VIOLA_CALL(viola_store_words, g.arena.as<int64_t>(at), words.data(), (int64_t)words.size(), stream);
+    g.offsets = g.arena.as<int64_t>(at);
+    g.padded_offsets = g.offsets + g.count + 1;
+}
+
+struct ExpertsBackward : public Node {
+    std::shared_ptr<Recipe> recipe;
+    Groups groups;
+    Arena kept;
+    Codes input_t;
+    SavedVariable weight;
+    Tensor weight_scale;
+    at::ScalarType x_dtype = at::kFloat, weight_grad = at::kFloat;
+    bool has_input = false;
+
+    variable_list apply(variable_list&& grads) override;
+    std::string name() const override { return "ViolaExpertsBackward"; }
+    void release_variables() override {
+        kept.release();
+        groups.arena.release();
+        weight.reset_data();
+        weight_scale = Tensor();
+    }
+};
+
+// x's row-wise codes and, where asked for, its per-group transposed codes; one read of x where the kernel takes the shape
+void quantize_segments(const Recipe& r, const Tensor& x, int fmt, float limit, const Groups& g, const Arena* rowwise, const GroupSpace& space, void* qt,
+                       float* st, Codes* out, viola_stream_t stream) {
+    const int64_t rows = x.size(0), cols = x.size(1);
+    const int dtype = code_of(x.scalar_type());
+    const bool together = qt && rowwise && x.element_size() == 2 && cols % 8 == 0 && space.pitch == cols && reinterpret_cast<uintptr_t>(ptr(x)) % 16 == 0;
+    if (qt)
+        VIOLA_CALL(viola_varlen_quantize_transposed, ptr(x), dtype, rows, cols, g.offsets, g.padded_offsets, (int)g.count, g.padded, qt, st, fmt, limit,
+                   together ? rowwise->at(space.q) : nullptr, together ? rowwise->as<float>(space.s) : nullptr, stream);
+    if (!rowwise) return;
+    Codes unused;
+    if (together) *out = {rowwise->at(space.q), rowwise->at(space.s), space.pitch};
+    else quantize_groups(r, x, fmt, limit, space, rowwise, nullptr, nullptr, out, &unused, stream);
+}
+
+void segment_product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_fmt, const Groups& g, int64_t n, void* out, at::ScalarType dtype,
+                     viola_stream_t stream) {
+    const int64_t k = a.pitch;
+    VIOLA_CALL(viola_varlen_group_gemm, a.q, a_fmt, b.q, b_fmt, static_cast<const float*>(a.s), static_cast<const float*>(b.s), g.offsets, (int)g.count, g.rows,
+               n, k, 1, 32, 32, 32, n * k, ceil_div(n, 32) * ceil_div(k, 32), out, code_of(dtype), stream);
+}
+
+Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scale, const std::vector<int64_t>& counts, const std::shared_ptr<Recipe>& recipe,
+               at::ScalarType weight_grad) {
+    TORCH_CHECK(x_.is_cuda() && x_.dim() == 2 && weight.dim() == 3 && weight.size(0) == (int64_t)counts.size() && x_.size(1) == weight.size(2));
+    TORCH_CHECK(weight_scale.is_contiguous() && weight.is_contiguous() && weight.is_cuda());
+    const Recipe& r = *recipe;
+    const bool wx = x_.requires_grad(), ww = weight.requires_grad();
+    const bool need = at::GradMode::is_enabled() && (wx || ww);
+    auto node = need ? std::shared_ptr<ExpertsBackward>(new ExpertsBackward(), torch::autograd::deleteNode) : nullptr;
+    const int64_t n = weight.size(1), k = weight.size(2);
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor x = x_.contiguous();
+        const at::Device device = x.device();
+        const viola_stream_t stream = stream_of(x);
+        Groups scratch_groups;
+        Groups& groups = need ? node->groups : scratch_groups;
+        make_groups(groups, counts, device, stream);
+        TORCH_CHECK(groups.rows == x.size(0), "the group sizes add up to ", groups.rows, " rows, x has ", x.size(0));
+        const bool save = need && ww && groups.rows;
+        Arena temp;
+        GroupSpace space;
+        space.reserve(r, &temp, nullptr, groups.rows, k);
+        const bool repack = space.pitch != k;
+        const int64_t wp = repack ? temp.take(groups.count * n * space.pitch) : -1;
+        const int64_t wps = repack ? temp.take(groups.count * ceil_div(n, 32) * ceil_div(space.pitch, 32) * 4) : -1;
+        temp.make(device);
+        void* qt = nullptr;
+        float* st = nullptr;
+        if (save) {
+            const int64_t q_at = node->kept.take(k * groups.padded), s_at = node->kept.take(k * (groups.padded / 32) * 4);
+            node->kept.make(device);
+            qt = node->kept.at(q_at);
+            st = node->kept.as<float>(s_at);
+            node->input_t = {qt, st, groups.padded};
+        }
+        y = at::empty({groups.rows, n}, x.options());
+        if (groups.rows) {
+            Codes a, w{ptr(weight), ptr(weight_scale), k};
+            quantize_segments(r, x, r.fwd, r.fwd_limit, groups, &temp, space, qt, st, &a, stream);
+            if (repack) {
+                VIOLA_CALL(viola_codes_repack, w.q, temp.at(wp), groups.count, n, k, space.pitch, w.s, temp.at(wps), 32, 32, VIOLA_SCALE_F32, stream);
+                w = {temp.at(wp), temp.at(wps), space.pitch};
+            }
+            segment_product(r, a, r.fwd, w, r.fwd, groups, n, y.mutable_data_ptr(), x.scalar_type(), stream);
+        }
+        if (need) {
+            node->has_input = save;
+            node->x_dtype = x.scalar_type();
+        }
+    }
+    if (need) {
+        node->recipe = recipe;
+        node->weight = SavedVariable(weight, false);
+        node->weight_scale = weight_scale;
+        node->weight_grad = weight_grad;
+        node->set_next_edges(torch::autograd::collect_next_edges(x_, weight));
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+variable_list ExpertsBackward::apply(variable_list&& grads) {
+    variable_list result(2);
+    if (!grads[0].defined()) return result;
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Recipe& r = *recipe;
+    const Tensor w = weight.unpack();
+    const int64_t count = w.size(0), n = w.size(1), k = w.size(2);
+    const Tensor dy = as_matrix(grads[0], n);
+    const at::Device device = w.device();
+    const viola_stream_t stream = stream_of(w);
+    const bool needs_x = task_should_compute_output(0), needs_w = task_should_compute_output(1);
+    const auto options = at::TensorOptions().device(device);
+    if (needs_w && !groups.rows) result[1] = at::zeros({count, n, k}, options.dtype(weight_grad));
+    if (needs_x && !groups.rows) result[0] = at::empty({0, k}, options.dtype(x_dtype));
+    if (!groups.rows) return result;
+    const bool weight_too = needs_w && has_input;
+    Arena temp;
+    GroupSpace space;
+    space.reserve(r, needs_x ? &temp : nullptr, nullptr, groups.rows, n);
+    const int64_t scale_cols = ceil_div(space.pitch, 32);
+    const int64_t wt = needs_x ? temp.take(count * k * space.pitch) : -1, wts = needs_x ? temp.take(count * ceil_div(k, 32) * scale_cols * 4) : -1;
+    const int64_t qt = weight_too ? temp.take(n * groups.padded) : -1, st = weight_too ? temp.take(n * (groups.padded / 32) * 4) : -1;
+    temp.make(device);
+    Codes g;
+    quantize_segments(r, dy, r.bwd, r.bwd_limit, groups, needs_x ? &temp : nullptr, space, weight_too ? temp.at(qt) : nullptr,
+                      weight_too ? temp.as<float>(st) : nullptr, &g, stream);
+    if (needs_x) {
+        VIOLA_CALL(viola_codes_transpose_pitched, ptr(w), temp.at(wt), count, n, k, space.pitch, ptr(weight_scale), temp.at(wts), 32, 32, VIOLA_SCALE_F32, nullptr, 0,
+                   0, nullptr, 0, stream);
+        result[0] = at::empty({groups.rows, k}, options.dtype(x_dtype));
+        segment_product(r, g, r.bwd, Codes{temp.at(wt), temp.at(wts), space.pitch}, r.fwd, groups, k, result[0].mutable_data_ptr(), x_dtype, stream);
+    }
+    if (weight_too) {
+        result[1] = at::empty({count, n, k}, options.dtype(weight_grad));
+        VIOLA_CALL(viola_varlen_wgrad_gemm, temp.at(qt), r.bwd, input_t.q, r.fwd, temp.as<float>(st), static_cast<const float*>(input_t.s), groups.padded_offsets,
+                   (int)count, groups.padded, n, k, result[1].mutable_data_ptr(), code_of(weight_grad), stream);
+    }
+    return result;
+}
+
+// ---------------------------------------------------------------------------------------------------- Python
+// (recipe, weight, bias, scale, transpose, transpose scale[, three histories, three counters])
+Layer layer_from(const py::tuple& t) {
+    Layer l;
+    l.recipe = t[0].cast<std::shared_ptr<Recipe>>();
+    l.weight = t[1].cast<Tensor>();
+    if (!t[2].is_none()) l.bias = t[2].cast<Tensor>();
+    l.scale = t[3].cast<Tensor>();
+    l.transpose = t[4].cast<Tensor>();
+    l.transpose_scale = t[5].cast<Tensor>();
+    if (t.size() > 6)
+        for (int i = 0; i < 3; ++i) {
+            l.history[i] = t[6 + i].cast<Tensor>();
+            l.counter[i] = t[9 + i].cast<std::shared_ptr<Counter>>();
+        }
+    return l;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+    event_class = new py::object(py::module_::import("torch.cuda").attr("Event"));
+    py::class_<Counter, std::shared_ptr<Counter>>(m, "Counter")
+        .def(py::init([](int64_t value) { auto c = std::make_shared<Counter>(); c->value = value; return c; }), py::arg("value") = 0)
+        .def_readwrite("value", &Counter::value)
+        .def("__reduce__", [](py::object self) { return py::make_tuple(self.attr("__class__"), py::make_tuple(self.attr("value"))); });
+    py::class_<Recipe, std::shared_ptr<Recipe>>(m, "Recipe")
+        .def(py::init<const py::dict&>())
+        .def("__reduce__", [](py::object self) { return py::make_tuple(self.attr("__class__"), py::make_tuple(self.cast<Recipe&>().fields())); });
+    m.def("set_timeline", [](py::object list) {
+        if (!timeline_sink) timeline_sink = new py::object();
+        *timeline_sink = list;
+        recording.store(!list.is_none());
+    });
+    m.def("linear", [](const Tensor& x, const py::tuple& layer) {
+        Layer l = layer_from(layer);
+        py::gil_scoped_release release;
+        return linear(x, l);
+    });
+    m.def("mlp", [](const Tensor& x, const py::tuple& up, const py::tuple& down, int activation) {
+        Layer u = layer_from(up), d = layer_from(down);
+        py::gil_scoped_release release;
+        return mlp(x, u, d, activation);
+    });
+    m.def("experts", [](const Tensor& x, const Tensor& weight, const Tensor& scale, const std::vector<int64_t>& counts, const std::shared_ptr<Recipe>& recipe,
+                        py::object weight_grad) {
+        const at::ScalarType grad = torch::python::detail::py_object_to_dtype(weight_grad);
+        py::gil_scoped_release release;
+        return experts(x, weight, scale, counts, recipe, grad);
+    });
+}

@@ -152,6 +152,7 @@ template <typename TIn, typename TOut, bool ROWWISE, bool TRANSPOSED, bool VEC>
 __global__ __launch_bounds__(256) void quantize_tile(const TIn* __restrict__ x, uint8_t* __restrict__ q,
                                                       float* __restrict__ scale, uint8_t* __restrict__ qt,
                                                       float* __restrict__ scale_t, int64_t rows, int64_t cols,
+                                                      int64_t q_pitch, int64_t qt_pitch,
                                                       float limit, float* __restrict__ column_partial, int e8m0) {
     __shared__ float tile[TILE_R * TILE_LD];
     const int64_t r0 = (int64_t)blockIdx.y * TILE_R, c0 = (int64_t)blockIdx.x * TILE_C;
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(256) void quantize_tile(const TIn* __restrict__ x, 
     if constexpr (ROWWISE) {
         const int r = t % TILE_R, g = t / TILE_R;                       // 128 rows x 2 column groups
         const int64_t row = r0 + r, col = c0 + g * 32;
-        if (row < rows && col < cols) {
+        if (q && row < rows && col < q_pitch) {
             float v[32];
             float amax = 0.0f, poison = 0.0f;
 #pragma unroll
@@ -171,17 +172,17 @@ __global__ __launch_bounds__(256) void quantize_tile(const TIn* __restrict__ x, 
                 poison = poison_of(poison, v[i]);
             }
             const float s = group_scale(amax, limit, e8m0);
-            const int64_t nc = (cols + 31) / 32;
+            const int64_t nc = (q_pitch + 31) / 32;
             put_scale(scale, row * nc + col / 32, s, e8m0);
-            const int count = (int)(cols - col < 32 ? cols - col : 32);
-            uint8_t* dst = q + row * cols + col;
+            const int count = (int)(q_pitch - col < 32 ? q_pitch - col : 32);
+            uint8_t* dst = q + row * q_pitch + col;
             store_group32<TOut>(v, s, poison, limit, dst, count, (reinterpret_cast<uintptr_t>(dst) & 15) == 0);
         }
     }
     if constexpr (TRANSPOSED) {
         const int c = t % TILE_C, g = t / TILE_C;                       // 64 columns x 4 row groups
         const int64_t col = c0 + c, row = r0 + g * 32;
-        if (col < cols && row < rows) {
+        if (qt && col < cols && row < qt_pitch) {
             float v[32];
             float amax = 0.0f, poison = 0.0f;
 #pragma unroll
@@ -191,16 +192,16 @@ __global__ __launch_bounds__(256) void quantize_tile(const TIn* __restrict__ x, 
                 poison = poison_of(poison, v[i]);
             }
             const float s = group_scale(amax, limit, e8m0);
-            const int64_t nr = (rows + 31) / 32;
+            const int64_t nr = (qt_pitch + 31) / 32;
             put_scale(scale_t, col * nr + row / 32, s, e8m0);
-            if (column_partial) {
+            if (column_partial && row < rows) {
                 float sum = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 32; ++i) sum += v[i];
                 column_partial[(row / 32) * cols + col] = sum;
             }
-            const int count = (int)(rows - row < 32 ? rows - row : 32);
-            uint8_t* dst = qt + col * rows + row;
+            const int count = (int)(qt_pitch - row < 32 ? qt_pitch - row : 32);
+            uint8_t* dst = qt + col * qt_pitch + row;
             store_group32<TOut>(v, s, poison, limit, dst, count, (reinterpret_cast<uintptr_t>(dst) & 15) == 0);
         }
     }
@@ -533,11 +534,11 @@ __device__ __noinline__ Exact16 encode_words16_exact(uint32_t w0, uint32_t w1, u
 template <typename TIn, typename TOut, bool INTERIOR>
 __device__ __forceinline__ void dual16_tile64(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ scale,
                                               uint8_t* __restrict__ qt, float* __restrict__ scale_t, int64_t rows, int64_t cols,
-                                              float limit, float* __restrict__ column_partial, int e8m0, int64_t r0, int64_t c0,
+                                              int64_t q_pitch, int64_t qt_pitch, bool vec, float limit, float* __restrict__ column_partial, int e8m0, int64_t r0, int64_t c0,
                                               uint16_t* park, int* flags) {
     constexpr int LDV = 64 + 4;                                              // values per parked row (34 dwords)
     const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
-    const int64_t nc = (cols + 31) / 32, nr = (rows + 31) / 32;
+    const int64_t nc = (q_pitch + 31) / 32, nr = (qt_pitch + 31) / 32;
     const bool clamp_free = limit == fp8_traits<TOut>::max;
 
     // ---- row-wise
@@ -550,6 +551,12 @@ __device__ __forceinline__ void dual16_tile64(const TIn* __restrict__ x, uint8_t
             const TIn* tile = x + r0 * cols + c0;
             raw[0] = *reinterpret_cast<const uint4*>(tile + offset);
             raw[1] = *reinterpret_cast<const uint4*>(tile + offset + 8);
+        } else if (row < rows && !vec) {
+            uint32_t* halves = reinterpret_cast<uint32_t*>(raw);
+            const uint16_t* src = reinterpret_cast<const uint16_t*>(x) + row * cols + col;
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (col + i < cols) halves[i / 2] |= (uint32_t)src[i] << (16 * (i % 2));
         } else if (row < rows) {
             if (col < cols) raw[0] = *reinterpret_cast<const uint4*>(x + row * cols + col);      // cols % 8 == 0: whole pieces
             if (col + 8 < cols) raw[1] = *reinterpret_cast<const uint4*>(x + row * cols + col + 8);
@@ -567,22 +574,25 @@ __device__ __forceinline__ void dual16_tile64(const TIn* __restrict__ x, uint8_t
             const Exact16 r = encode_words16_exact<TIn, TOut>(words[0], words[1], words[2], words[3], words[4], words[5], words[6], words[7], limit, e8m0);
             codes[0] = r.c0; codes[1] = r.c1; codes[2] = r.c2; codes[3] = r.c3; s_row = r.s;
         }
-        if constexpr (INTERIOR) {
-            *reinterpret_cast<uint4*>(q + r0 * cols + c0 + offset) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
+        if (!q) {
+            // transposed layout only
+        } else if constexpr (INTERIOR) {
+            *reinterpret_cast<uint4*>(q + r0 * q_pitch + c0 + ((uint32_t)lr * (uint32_t)q_pitch + (uint32_t)lc)) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
             if (tid % 2 == 0) put_scale(scale, (r0 * nc + c0 / 32) + (int64_t)((uint32_t)lr * (uint32_t)nc + (uint32_t)(lc / 32)), s_row, e8m0);
-        } else if (row < rows && col < cols) {
-            uint8_t* dst = q + row * cols + col;
-            if (col + 16 <= cols && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+        } else if (row < rows && col < q_pitch) {                            // columns cols .. q_pitch - 1: zero codes
+            uint8_t* dst = q + row * q_pitch + col;
+            if (col + 16 <= q_pitch && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
                 *reinterpret_cast<uint4*>(dst) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
             } else {
-                *reinterpret_cast<uint2*>(dst) = make_uint2(codes[0], codes[1]);                     // q is 8-byte aligned, cols % 8 == 0
-                if (col + 8 < cols) *reinterpret_cast<uint2*>(dst + 8) = make_uint2(codes[2], codes[3]);
+                const int count = (int)(q_pitch - col < 16 ? q_pitch - col : 16);
+                for (int i = 0; i < count; ++i) dst[i] = (uint8_t)(codes[i >> 2] >> (8 * (i & 3)));
             }
             if (tid % 2 == 0) put_scale(scale, row * nc + col / 32, s_row, e8m0);
         }
         const bool any_nonfinite = __builtin_amdgcn_ballot_w64(nonfinite) != 0;   // over the whole wavefront: outside the branch
         if (lane == 0) flags[wave] = any_nonfinite;
     }
+    if (!qt) return;                                                         // row-wise layout only (uniform)
     __syncthreads();
     // no NaN and no Inf anywhere in the tile: the transposed phase may then take its maxima in floating point
     const bool plain = (flags[0] | flags[1] | flags[2] | flags[3]) == 0;
@@ -614,22 +624,22 @@ __device__ __forceinline__ void dual16_tile64(const TIn* __restrict__ x, uint8_t
             sum = chunk % 2 == 0 ? sum + other : other + sum;                 // rows 0 .. 15 first, then 16 .. 31
         }
         if constexpr (INTERIOR) {
-            *reinterpret_cast<uint4*>(qt + c0 * rows + r0 + ((uint32_t)tc * (uint32_t)rows + (uint32_t)(chunk * 16))) = make_uint4(tcodes[0], tcodes[1], tcodes[2], tcodes[3]);
+            *reinterpret_cast<uint4*>(qt + c0 * qt_pitch + r0 + ((uint32_t)tc * (uint32_t)qt_pitch + (uint32_t)(chunk * 16))) = make_uint4(tcodes[0], tcodes[1], tcodes[2], tcodes[3]);
             if (chunk % 2 == 0) {
                 put_scale(scale_t, (c0 * nr + r0 / 32) + (int64_t)((uint32_t)tc * (uint32_t)nr + (uint32_t)(chunk / 2)), s_col, e8m0);
                 if (column_partial) (column_partial + (r0 / 32) * cols + c0)[(uint32_t)(chunk / 2) * (uint32_t)cols + (uint32_t)tc] = sum;
             }
-        } else if (tcol < cols && trow < rows) {
-            uint8_t* dst = qt + tcol * rows + trow;
-            if (trow + 16 <= rows && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+        } else if (tcol < cols && trow < qt_pitch) {                         // rows rows .. qt_pitch - 1: zero codes
+            uint8_t* dst = qt + tcol * qt_pitch + trow;
+            if (trow + 16 <= qt_pitch && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
                 *reinterpret_cast<uint4*>(dst) = make_uint4(tcodes[0], tcodes[1], tcodes[2], tcodes[3]);
             } else {
-                const int count = (int)(rows - trow < 16 ? rows - trow : 16);
+                const int count = (int)(qt_pitch - trow < 16 ? qt_pitch - trow : 16);
                 for (int i = 0; i < count; ++i) dst[i] = (uint8_t)(tcodes[i >> 2] >> (8 * (i & 3)));
             }
             if (chunk % 2 == 0) {
                 put_scale(scale_t, tcol * nr + trow / 32, s_col, e8m0);
-                if (column_partial) column_partial[(trow / 32) * cols + tcol] = sum;
+                if (column_partial && trow < rows) column_partial[(trow / 32) * cols + tcol] = sum;
             }
         }
     }
@@ -639,15 +649,16 @@ template <typename TIn, typename TOut>
 __global__ __launch_bounds__(256, 8) void quantize_dual16_tile64(const TIn* __restrict__ x, uint8_t* __restrict__ q,
                                                                float* __restrict__ scale, uint8_t* __restrict__ qt,
                                                                float* __restrict__ scale_t, int64_t rows, int64_t cols,
+                                                               int64_t q_pitch, int64_t qt_pitch,
                                                                float limit, float* __restrict__ column_partial, int e8m0, int xcd_walk,
-                                                               int aligned) {
+                                                               int aligned, int vec) {
     __shared__ __attribute__((aligned(16))) uint16_t park[64 * (64 + 4)];
     __shared__ __attribute__((aligned(16))) int flags[4];                   // per wavefront: its rows hold a NaN or an Inf
     // blocks are dispatched in index order: those in flight together take 32 row tiles of one column tile, then the next
     // column tile, so the transposed output is written in 2 KB runs per row however wide the matrix is (the launcher
     // keeps the tile count below 2^31)
     constexpr uint32_t BAND = 32;
-    const uint32_t tiles_x = (uint32_t)((cols + 63) / 64), tiles_y = (uint32_t)((rows + 63) / 64), tiles = tiles_x * tiles_y;
+    const uint32_t tiles_x = (uint32_t)((q_pitch + 63) / 64), tiles_y = (uint32_t)((qt_pitch + 63) / 64), tiles = tiles_x * tiles_y;
     uint32_t id = blockIdx.x;
     if (xcd_walk) {
         // consecutive block indices go to the eight XCDs in turn: give each XCD one contiguous eighth of the walk, so the
@@ -658,48 +669,16 @@ __global__ __launch_bounds__(256, 8) void quantize_dual16_tile64(const TIn* __re
     const uint32_t patch = id / (BAND * tiles_x), within = id % (BAND * tiles_x);
     const uint32_t tall = tiles_y - patch * BAND < BAND ? tiles_y - patch * BAND : BAND;
     const int64_t r0 = (int64_t)(patch * BAND + within % tall) * 64, c0 = (int64_t)(within / tall) * 64;
-    if (aligned && r0 + 64 <= rows && c0 + 64 <= cols) dual16_tile64<TIn, TOut, true>(x, q, scale, qt, scale_t, rows, cols, limit, column_partial, e8m0, r0, c0, park, flags);
-    else dual16_tile64<TIn, TOut, false>(x, q, scale, qt, scale_t, rows, cols, limit, column_partial, e8m0, r0, c0, park, flags);
+    if (aligned && r0 + 64 <= rows && c0 + 64 <= cols) dual16_tile64<TIn, TOut, true>(x, q, scale, qt, scale_t, rows, cols, q_pitch, qt_pitch, true, limit, column_partial, e8m0, r0, c0, park, flags);
+    else dual16_tile64<TIn, TOut, false>(x, q, scale, qt, scale_t, rows, cols, q_pitch, qt_pitch, vec != 0, limit, column_partial, e8m0, r0, c0, park, flags);
 }
 
 // ------------------------------------------------------------------ column sums from 32-row partials
-// out[c] = sum over p of partial[p][c] in a fixed order: 8 threads per column each add a contiguous eighth of the
-// parts in ascending order (loads issued 32 or eight at a time), then the eighths are added in order.
 template <typename TO>
 __global__ __launch_bounds__(256) void column_reduce_kernel(const float* __restrict__ partial, int64_t parts, int64_t cols,
                                                              TO* __restrict__ out) {
     __shared__ float piece[8][32];
-    const int c = threadIdx.x % 32, slice = threadIdx.x / 32;
-    const int64_t col = (int64_t)blockIdx.x * 32 + c;
-    const int64_t per = (parts + 7) / 8;
-    const int64_t begin = slice * per, end = begin + per < parts ? begin + per : parts;
-    float sum = 0.0f;
-    if (col < cols) {
-        int64_t part = begin;
-        for (; part + 32 <= end; part += 32) {                              // same order of additions, four times the loads in flight
-            float v[32];
-#pragma unroll
-            for (int u = 0; u < 32; ++u) v[u] = partial[(part + u) * cols + col];
-#pragma unroll
-            for (int u = 0; u < 32; ++u) sum += v[u];
-        }
-        for (; part + 8 <= end; part += 8) {
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = partial[(part + u) * cols + col];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) sum += v[u];
-        }
-        for (; part < end; ++part) sum += partial[part * cols + col];
-    }
-    piece[slice][c] = sum;
-    __syncthreads();
-    if (slice == 0 && col < cols) {
-        float total = piece[0][c];
-#pragma unroll
-        for (int u = 1; u < 8; ++u) total += piece[u][c];
-        out[col] = from_f32<TO>(total);
-    }
+    reduce_columns<TO>(partial, parts, cols, out, blockIdx.x, piece);
 }
 
 // ------------------------------------------------------------------ (32, 32) blocks, not transposed
@@ -823,24 +802,43 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const TQ* __restrict__ 
 // 4-byte loads (16 lanes cover 64 contiguous bytes of a row), a 4 x 4 transpose with byte permutes, the four words
 // handed over through LDS so that the stores are again 64 contiguous bytes per 16 lanes.
 // With a scale grid (one entry of scale_bytes bytes per block of codes, [srows, scols]), the grid is transposed in the
-// same launch: the blocks share out its entries, thread 0 .. moving one each.
+// same launch: the blocks share out its entries, thread 0 .. moving one each. Rows of the output are out_pitch codes
+// (scale_pitch entries) apart; what lies past the matrix is zero codes and zero scales.
+// With column sums to finish (the bias gradient, whose 32-row partials the quantizer of dY has just written), one more plane
+// of blocks does that: both jobs are a few microseconds of a launch that does not fill the chip.
+struct ColumnSums { const float* partial; int64_t parts, cols; void* out; int dtype; };
+
 template <bool WORDS>
 __global__ __launch_bounds__(256) void transpose_bytes(const uint8_t* __restrict__ x, uint8_t* __restrict__ out,
-                                                        int64_t rows, int64_t cols, const uint8_t* __restrict__ scale = nullptr,
-                                                        uint8_t* __restrict__ scale_out = nullptr, int64_t srows = 0,
-                                                        int64_t scols = 0, int scale_bytes = 0) {
+                                                        int64_t rows, int64_t cols, int64_t out_pitch,
+                                                        const uint8_t* __restrict__ scale, uint8_t* __restrict__ scale_out,
+                                                        int64_t srows, int64_t scols, int64_t scale_pitch, int scale_bytes,
+                                                        ColumnSums sums) {
+    if (sums.partial && blockIdx.z == gridDim.z - 1) {
+        __shared__ float piece[8][32];
+        const int64_t stride = (int64_t)gridDim.x * gridDim.y;
+        for (int64_t b = (int64_t)blockIdx.y * gridDim.x + blockIdx.x; b * 32 < sums.cols; b += stride) {
+            if (sums.dtype == VIOLA_F32) reduce_columns<float>(sums.partial, sums.parts, sums.cols, static_cast<float*>(sums.out), b, piece);
+            else if (sums.dtype == VIOLA_BF16) reduce_columns<bf16_t>(sums.partial, sums.parts, sums.cols, static_cast<bf16_t*>(sums.out), b, piece);
+            else reduce_columns<f16_t>(sums.partial, sums.parts, sums.cols, static_cast<f16_t*>(sums.out), b, piece);
+            __syncthreads();                                            // piece is reused
+        }
+        return;
+    }
     const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
     if (scale) {
-        const int64_t entries = srows * scols, blocks = (int64_t)gridDim.x * gridDim.y;
+        const int64_t entries = scale_pitch * scols, blocks = (int64_t)gridDim.x * gridDim.y;
         const int64_t per = (entries + blocks - 1) / blocks, first = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * per;
+        const int64_t from = (int64_t)blockIdx.z * srows * scols, to = (int64_t)blockIdx.z * entries;
         for (int64_t e = first + threadIdx.x; e < first + per && e < entries; e += blockDim.x) {
             const int64_t sr = e / scols, sc = e % scols;
-            if (scale_bytes == 4) reinterpret_cast<float*>(scale_out)[sc * srows + sr] = reinterpret_cast<const float*>(scale)[e];
-            else scale_out[sc * srows + sr] = scale[e];
+            const bool inside = sr < srows;
+            if (scale_bytes == 4) reinterpret_cast<float*>(scale_out)[to + sc * scale_pitch + sr] = inside ? reinterpret_cast<const float*>(scale)[from + e] : 0.0f;
+            else scale_out[to + sc * scale_pitch + sr] = inside ? scale[from + e] : 0;
         }
     }
     x += (int64_t)blockIdx.z * rows * cols;
-    out += (int64_t)blockIdx.z * rows * cols;
+    out += (int64_t)blockIdx.z * out_pitch * cols;
     if constexpr (WORDS) {
         __shared__ uint32_t tile[64][17];
         const int b = threadIdx.x % 16, a = threadIdx.x / 16;               // block of rows 4a.., cols 4b..
@@ -861,7 +859,7 @@ __global__ __launch_bounds__(256) void transpose_bytes(const uint8_t* __restrict
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int c = threadIdx.x / 16 + 16 * i, ra = threadIdx.x % 16;
-            if (c0 + c < cols && r0 + 4 * ra < rows) *reinterpret_cast<uint32_t*>(out + (c0 + c) * rows + r0 + 4 * ra) = tile[c][ra];
+            if (c0 + c < cols && r0 + 4 * ra < out_pitch) *reinterpret_cast<uint32_t*>(out + (c0 + c) * out_pitch + r0 + 4 * ra) = tile[c][ra];
         }
     } else {
         __shared__ uint8_t tile[64][64 + 4];
@@ -872,8 +870,36 @@ __global__ __launch_bounds__(256) void transpose_bytes(const uint8_t* __restrict
         __syncthreads();
         for (int id = threadIdx.x; id < 64 * 64; id += 256) {
             const int c = id / 64, r = id % 64;
-            if (r0 + r < rows && c0 + c < cols) out[(c0 + c) * rows + r0 + r] = tile[r][c];
+            if (r0 + r < out_pitch && c0 + c < cols) out[(c0 + c) * out_pitch + r0 + r] = tile[r][c];
         }
+    }
+}
+
+// ------------------------------------------------------------------ codes at another row pitch
+// out [rows, pitch] = x [rows, cols] with zero codes in columns cols .. pitch - 1, and the same for the grid of scales:
+// how a weight whose rows are not whole 16-byte pieces (128-byte pieces under E8M0 scales) reaches the GEMM kernel that
+// loads such pieces. One word of four codes per thread; a copy of the weight's bytes costs a few microseconds where the
+// guarded byte loads it avoids ran at 40 TFLOP/s.
+__global__ __launch_bounds__(256) void repack_codes(const uint8_t* __restrict__ x, uint8_t* __restrict__ out, int64_t rows, int64_t cols,
+                                                     int64_t pitch, const uint8_t* __restrict__ scale, uint8_t* __restrict__ scale_out,
+                                                     int64_t srows, int64_t scols, int64_t spitch, int scale_bytes) {
+    const uint32_t per_row = (uint32_t)(pitch / 4), words = (uint32_t)rows * per_row, stride = gridDim.x * blockDim.x;
+    const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t id = first; id < words; id += stride) {
+        const uint32_t r = id / per_row, c = (id - r * per_row) * 4;
+        const uint8_t* src = x + (int64_t)r * cols + c;
+        uint32_t w = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (c + i < cols) w |= (uint32_t)src[i] << (8 * i);
+        reinterpret_cast<uint32_t*>(out)[id] = w;
+    }
+    const uint32_t entries = (uint32_t)(srows * spitch);
+    for (uint32_t e = first; e < entries; e += stride) {
+        const uint32_t sr = e / (uint32_t)spitch, sc = e % (uint32_t)spitch;
+        const bool inside = sc < scols;
+        if (scale_bytes == 4) reinterpret_cast<float*>(scale_out)[e] = inside ? reinterpret_cast<const float*>(scale)[sr * scols + sc] : 0.0f;
+        else scale_out[e] = inside ? scale[sr * scols + sc] : 0;
     }
 }
 
@@ -1099,8 +1125,8 @@ static int launch_quantize(const void* x, int64_t rows, int64_t cols, void* q, f
     }
     if (gr == 1 && gc == 32 && transposed) {
         const dim3 grid((unsigned)((cols + TILE_C - 1) / TILE_C), (unsigned)((rows + TILE_R - 1) / TILE_R));
-        if (vec) VIOLA_LAUNCH((quantize_tile<TIn, TOut, false, true, true>), grid, dim3(256), 0, stream, xp, nullptr, nullptr, qp, scale, rows, cols, limit, nullptr, e8m0);
-        else VIOLA_LAUNCH((quantize_tile<TIn, TOut, false, true, false>), grid, dim3(256), 0, stream, xp, nullptr, nullptr, qp, scale, rows, cols, limit, nullptr, e8m0);
+        if (vec) VIOLA_LAUNCH((quantize_tile<TIn, TOut, false, true, true>), grid, dim3(256), 0, stream, xp, nullptr, nullptr, qp, scale, rows, cols, cols, rows, limit, nullptr, e8m0);
+        else VIOLA_LAUNCH((quantize_tile<TIn, TOut, false, true, false>), grid, dim3(256), 0, stream, xp, nullptr, nullptr, qp, scale, rows, cols, cols, rows, limit, nullptr, e8m0);
         return viola_launch_status();
     }
     if (gr == 32 && gc == 32 && !transposed && cols % 4 == 0 && reinterpret_cast<uintptr_t>(x) % (4 * sizeof(TIn)) == 0 &&
@@ -1139,28 +1165,30 @@ static int launch_reencode(const void* x, const float* source_scale, int64_t row
     return viola_launch_status();
 }
 
+// q (row pitch q_pitch >= cols, scales of ceil(q_pitch / 32) groups per row) and qt (row pitch qt_pitch >= rows) are filled
+// with zero codes past the matrix, so that a GEMM may take the pitch as its k. Either output may be absent; the pitches
+// then still size the walk.
 template <typename TIn, typename TOut>
-static int launch_dual(const void* x, int64_t rows, int64_t cols, void* q, float* scale, void* qt, float* scale_t,
-                       float limit, float* column_partial, int e8m0, hipStream_t stream) {
+static int launch_dual(const void* x, int64_t rows, int64_t cols, void* q, int64_t q_pitch, float* scale, void* qt, int64_t qt_pitch,
+                       float* scale_t, float limit, float* column_partial, int e8m0, hipStream_t stream) {
     const bool vec = cols % 8 == 0 && reinterpret_cast<uintptr_t>(x) % (8 * sizeof(TIn)) == 0;
-    const dim3 grid((unsigned)((cols + TILE_C - 1) / TILE_C), (unsigned)((rows + TILE_R - 1) / TILE_R));
     const TIn* xp = static_cast<const TIn*>(x);
     if constexpr (sizeof(TIn) == 2) {
-        if (vec && reinterpret_cast<uintptr_t>(q) % 8 == 0) {
-            const int64_t tiles64 = ((cols + 63) / 64) * ((rows + 63) / 64);
-            if (tiles64 + 8 < (1ll << 31)) {
-                // one to four rounds of resident blocks (eight per compute unit): the XCD-contiguous walk measured faster
-                // (8192 x 4096: 29.7 -> 27.7 us); longer launches are faster with the eight XCDs streaming one region
-                // (16384 x 4096: 68 against 76 us), shorter ones leave XCDs uneven
-                const int xcd_walk = tiles64 >= 2048 && tiles64 <= 8192;
-                // whole tiles may skip their bounds checks and address a lane's pieces by 32-bit offsets from the tile
-                const int aligned = cols % 16 == 0 && rows % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
-                                    reinterpret_cast<uintptr_t>(qt) % 16 == 0 && cols < (1ll << 24) && rows < (1ll << 24);
-                VIOLA_LAUNCH((quantize_dual16_tile64<TIn, TOut>), dim3((unsigned)((tiles64 + 7) / 8 * 8)), dim3(256), 0, stream, xp,
-                             static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, rows, cols, limit, column_partial, e8m0, xcd_walk,
-                             aligned);
-                return viola_launch_status();
-            }
+        const int64_t tiles64 = ((q_pitch + 63) / 64) * ((qt_pitch + 63) / 64);
+        if (tiles64 + 8 < (1ll << 31)) {
+            // one to four rounds of resident blocks (eight per compute unit): the XCD-contiguous walk measured faster
+            // (8192 x 4096: 29.7 -> 27.7 us); longer launches are faster with the eight XCDs streaming one region
+            // (16384 x 4096: 68 against 76 us), shorter ones leave XCDs uneven
+            const int xcd_walk = tiles64 >= 2048 && tiles64 <= 8192;
+            // whole tiles may skip their bounds checks and address a lane's pieces by 32-bit offsets from the tile
+            const int aligned = vec && q_pitch % 16 == 0 && qt_pitch % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
+                                reinterpret_cast<uintptr_t>(qt) % 16 == 0 && q_pitch < (1ll << 24) && qt_pitch < (1ll << 24);
+            VIOLA_LAUNCH((quantize_dual16_tile64<TIn, TOut>), dim3((unsigned)((tiles64 + 7) / 8 * 8)), dim3(256), 0, stream, xp,
+                         static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, rows, cols, q_pitch, qt_pitch, limit, column_partial, e8m0,
+                         xcd_walk, aligned, (int)vec);
+            return viola_launch_status();
+        }
+        if (vec && q && reinterpret_cast<uintptr_t>(q) % 8 == 0 && q_pitch == cols && qt_pitch == rows) {
             const int64_t tiles16 = ((cols + 63) / 64) * ((rows + 127) / 128);
             const dim3 grid16((unsigned)(tiles16 < 256 * 6 ? tiles16 : 256 * 6));
             VIOLA_LAUNCH((quantize_dual16<TIn, TOut, true>), grid16, dim3(256), 0, stream, xp, static_cast<uint8_t*>(q), scale,
@@ -1168,8 +1196,10 @@ static int launch_dual(const void* x, int64_t rows, int64_t cols, void* q, float
             return viola_launch_status();
         }
     }
-    if (vec) VIOLA_LAUNCH((quantize_tile<TIn, TOut, true, true, true>), grid, dim3(256), 0, stream, xp, static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, rows, cols, limit, column_partial, e8m0);
-    else VIOLA_LAUNCH((quantize_tile<TIn, TOut, true, true, false>), grid, dim3(256), 0, stream, xp, static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, rows, cols, limit, column_partial, e8m0);
+    const dim3 grid((unsigned)((q_pitch + TILE_C - 1) / TILE_C), (unsigned)((qt_pitch + TILE_R - 1) / TILE_R));
+    if (grid.y > 65535) return VIOLA_ETOOLARGE;
+    if (vec) VIOLA_LAUNCH((quantize_tile<TIn, TOut, true, true, true>), grid, dim3(256), 0, stream, xp, static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, rows, cols, q_pitch, qt_pitch, limit, column_partial, e8m0);
+    else VIOLA_LAUNCH((quantize_tile<TIn, TOut, true, true, false>), grid, dim3(256), 0, stream, xp, static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, rows, cols, q_pitch, qt_pitch, limit, column_partial, e8m0);
     return viola_launch_status();
 }
 
@@ -1230,19 +1260,19 @@ extern "C" int viola_group_quantize(const void* x, int x_dtype, int64_t rows, in
     return dispatch_in<e5m2_t>(x_dtype, x, rows, cols, q, scale, gr, gc, limit, transposed, e8m0, stream);
 }
 
-extern "C" int viola_group_quantize_dual(const void* x, int x_dtype, int64_t rows, int64_t cols, void* q, void* scale_,
-                                         void* qt, void* scale_t_, int q_dtype, int gc, float limit,
-                                         float* column_partial, int scale_format, viola_stream_t stream_) {
+extern "C" int viola_group_quantize_dual_pitched(const void* x, int x_dtype, int64_t rows, int64_t cols, void* q, int64_t q_pitch,
+                                                 void* scale_, void* qt, int64_t qt_pitch, void* scale_t_, int q_dtype, float limit,
+                                                 float* column_partial, int scale_format, viola_stream_t stream_) {
     hipStream_t stream = viola_enter(stream_);
     float* scale = static_cast<float*>(scale_);
     float* scale_t = static_cast<float*>(scale_t_);
     VIOLA_CHECK_ARG(scale_format == VIOLA_SCALE_F32 || scale_format == VIOLA_SCALE_E8M0);
     const int e8m0 = scale_format == VIOLA_SCALE_E8M0;
     VIOLA_CHECK_ARG(viola_is_fp8(q_dtype) && viola_is_float(x_dtype) && rows >= 0 && cols >= 0 && limit > 0.0f);
-    if (gc != 32) return VIOLA_EUNSUPPORTED;
+    VIOLA_CHECK_ARG(q_pitch >= cols && qt_pitch >= rows && (!column_partial || qt));
     if (rows == 0 || cols == 0) return 0;
-    VIOLA_CHECK_ARG(x && q && scale && qt && scale_t);
-#define VIOLA_DUAL(TI, TO) return launch_dual<TI, TO>(x, rows, cols, q, scale, qt, scale_t, limit, column_partial, e8m0, stream)
+    VIOLA_CHECK_ARG(x && (q || qt) && (!q || scale) && (!qt || scale_t));
+#define VIOLA_DUAL(TI, TO) return launch_dual<TI, TO>(x, rows, cols, q, q_pitch, scale, qt, qt_pitch, scale_t, limit, column_partial, e8m0, stream)
     if (q_dtype == VIOLA_E4M3) {
         if (x_dtype == VIOLA_F32) VIOLA_DUAL(float, e4m3_t);
         if (x_dtype == VIOLA_BF16) VIOLA_DUAL(bf16_t, e4m3_t);
@@ -1252,6 +1282,15 @@ extern "C" int viola_group_quantize_dual(const void* x, int x_dtype, int64_t row
     if (x_dtype == VIOLA_BF16) VIOLA_DUAL(bf16_t, e5m2_t);
     VIOLA_DUAL(f16_t, e5m2_t);
 #undef VIOLA_DUAL
+}
+
+extern "C" int viola_group_quantize_dual(const void* x, int x_dtype, int64_t rows, int64_t cols, void* q, void* scale,
+                                         void* qt, void* scale_t, int q_dtype, int gc, float limit,
+                                         float* column_partial, int scale_format, viola_stream_t stream) {
+    if (gc != 32) return VIOLA_EUNSUPPORTED;
+    if (rows > 0 && cols > 0) VIOLA_CHECK_ARG(q && qt);
+    return viola_group_quantize_dual_pitched(x, x_dtype, rows, cols, q, cols, scale, qt, rows, scale_t, q_dtype, limit, column_partial,
+                                             scale_format, stream);
 }
 
 extern "C" int viola_gated_quantize_dual(const void* z, int z_dtype, int64_t rows, int64_t cols, int activation, void* q,
@@ -1333,30 +1372,65 @@ extern "C" int viola_group_dequantize(const void* q, int q_dtype, const float* s
     return viola_launch_status();
 }
 
+// batch matrices of codes with (for scale != null) their grids of one scale per gr x gc block
+static int transpose_codes(const void* x, void* out, int64_t batch, int64_t rows, int64_t cols, int64_t out_pitch, const void* scale,
+                           void* scale_out, int gr, int gc, int scale_format, const ColumnSums& sums, hipStream_t stream) {
+    VIOLA_CHECK_ARG(x && out && (out_pitch + 63) / 64 <= 65535 && batch < 65535);
+    const int scale_bytes = scale_format == VIOLA_SCALE_F32 ? 4 : 1;
+    VIOLA_CHECK_ARG(reinterpret_cast<uintptr_t>(scale) % scale_bytes == 0 && reinterpret_cast<uintptr_t>(scale_out) % scale_bytes == 0);
+    const int64_t srows = scale ? (rows + gr - 1) / gr : 0, scols = scale ? (cols + gc - 1) / gc : 0, spitch = scale ? (out_pitch + gr - 1) / gr : 0;
+    const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((out_pitch + 63) / 64), (unsigned)(batch + (sums.partial ? 1 : 0)));
+    const bool words = rows % 4 == 0 && cols % 4 == 0 && out_pitch % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0;
+    const uint8_t* sp = static_cast<const uint8_t*>(scale);
+    uint8_t* so = static_cast<uint8_t*>(scale_out);
+    if (words) VIOLA_LAUNCH(transpose_bytes<true>, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(x), static_cast<uint8_t*>(out), rows, cols, out_pitch, sp, so, srows, scols, spitch, scale_bytes, sums);
+    else VIOLA_LAUNCH(transpose_bytes<false>, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(x), static_cast<uint8_t*>(out), rows, cols, out_pitch, sp, so, srows, scols, spitch, scale_bytes, sums);
+    return viola_launch_status();
+}
+
+extern "C" int viola_codes_transpose_pitched(const void* x, void* out, int64_t batch, int64_t rows, int64_t cols, int64_t out_pitch,
+                                             const void* scale, void* scale_out, int gr, int gc, int scale_format,
+                                             const float* column_partial, int64_t parts, int64_t sum_cols, void* column_sum, int sum_dtype,
+                                             viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG(!column_partial || (parts > 0 && sum_cols > 0 && column_sum && viola_is_float(sum_dtype)));
+    VIOLA_CHECK_ARG(batch >= 0 && rows >= 0 && cols >= 0 && out_pitch >= rows && gr > 0 && gc > 0 && (!scale == !scale_out));
+    VIOLA_CHECK_ARG(scale_format == VIOLA_SCALE_F32 || scale_format == VIOLA_SCALE_E8M0);
+    if (batch == 0 || rows == 0 || cols == 0) return 0;
+    return transpose_codes(x, out, batch, rows, cols, out_pitch, scale, scale_out, gr, gc, scale_format,
+                           {column_partial, parts, sum_cols, column_sum, sum_dtype}, stream);
+}
+
 extern "C" int viola_block_transpose(const void* x, void* out, int64_t rows, int64_t cols, const void* scale, void* scale_out,
                                      int gr, int gc, int scale_format, viola_stream_t stream_) {
     hipStream_t stream = viola_enter(stream_);
     VIOLA_CHECK_ARG(rows >= 0 && cols >= 0 && gr > 0 && gc > 0 && (scale_format == VIOLA_SCALE_F32 || scale_format == VIOLA_SCALE_E8M0));
     if (rows == 0 || cols == 0) return 0;
-    VIOLA_CHECK_ARG(x && out && scale && scale_out && (rows + 63) / 64 <= 65535);
-    const int scale_bytes = scale_format == VIOLA_SCALE_F32 ? 4 : 1;
-    VIOLA_CHECK_ARG(reinterpret_cast<uintptr_t>(scale) % scale_bytes == 0 && reinterpret_cast<uintptr_t>(scale_out) % scale_bytes == 0);
-    const int64_t srows = (rows + gr - 1) / gr, scols = (cols + gc - 1) / gc;
-    const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((rows + 63) / 64), 1);
-    const bool words = rows % 4 == 0 && cols % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0;
-    if (words) VIOLA_LAUNCH(transpose_bytes<true>, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(x), static_cast<uint8_t*>(out), rows, cols, static_cast<const uint8_t*>(scale), static_cast<uint8_t*>(scale_out), srows, scols, scale_bytes);
-    else VIOLA_LAUNCH(transpose_bytes<false>, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(x), static_cast<uint8_t*>(out), rows, cols, static_cast<const uint8_t*>(scale), static_cast<uint8_t*>(scale_out), srows, scols, scale_bytes);
-    return viola_launch_status();
+    VIOLA_CHECK_ARG(scale && scale_out);
+    return transpose_codes(x, out, 1, rows, cols, rows, scale, scale_out, gr, gc, scale_format, {}, stream);
 }
 
 extern "C" int viola_fp8_transpose(const void* x, void* out, int64_t batch, int64_t rows, int64_t cols, viola_stream_t stream_) {
     hipStream_t stream = viola_enter(stream_);
     VIOLA_CHECK_ARG(batch >= 0 && rows >= 0 && cols >= 0);
     if (batch == 0 || rows == 0 || cols == 0) return 0;
-    VIOLA_CHECK_ARG(x && out && (rows + 63) / 64 <= 65535 && batch <= 65535);
-    const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((rows + 63) / 64), (unsigned)batch);
-    const bool words = rows % 4 == 0 && cols % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0;
-    if (words) VIOLA_LAUNCH(transpose_bytes<true>, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(x), static_cast<uint8_t*>(out), rows, cols, nullptr, nullptr, 0, 0, 0);
-    else VIOLA_LAUNCH(transpose_bytes<false>, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(x), static_cast<uint8_t*>(out), rows, cols, nullptr, nullptr, 0, 0, 0);
+    return transpose_codes(x, out, batch, rows, cols, rows, nullptr, nullptr, 1, 1, VIOLA_SCALE_F32, {}, stream);
+}
+
+extern "C" int viola_codes_repack(const void* x, void* out, int64_t batch, int64_t rows, int64_t cols, int64_t out_pitch, const void* scale,
+                                  void* scale_out, int gr, int gc, int scale_format, viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG(batch >= 0 && rows >= 0 && cols >= 0 && out_pitch >= cols && out_pitch % 4 == 0 && gr > 0 && gc > 0 && (!scale == !scale_out));
+    VIOLA_CHECK_ARG(scale_format == VIOLA_SCALE_F32 || scale_format == VIOLA_SCALE_E8M0);
+    if (batch == 0 || rows == 0 || cols == 0) return 0;
+    VIOLA_CHECK_ARG(x && out && reinterpret_cast<uintptr_t>(out) % 4 == 0);
+    const int scale_bytes = scale_format == VIOLA_SCALE_F32 ? 4 : 1;
+    VIOLA_CHECK_ARG(reinterpret_cast<uintptr_t>(scale) % scale_bytes == 0 && reinterpret_cast<uintptr_t>(scale_out) % scale_bytes == 0);
+    const int64_t srows = scale ? batch * ((rows + gr - 1) / gr) : 0, scols = scale ? (cols + gc - 1) / gc : 0, spitch = scale ? (out_pitch + gc - 1) / gc : 0;
+    const int64_t words = batch * rows * (out_pitch / 4), blocks = (words + 255) / 256;
+    VIOLA_CHECK_ARG(words < (1ll << 31) && srows * spitch < (1ll << 31));
+    VIOLA_LAUNCH(repack_codes, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0, stream, static_cast<const uint8_t*>(x),
+                 static_cast<uint8_t*>(out), batch * rows, cols, out_pitch, static_cast<const uint8_t*>(scale), static_cast<uint8_t*>(scale_out),
+                 srows, scols, spitch, scale_bytes);
     return viola_launch_status();
 }

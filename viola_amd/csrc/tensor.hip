@@ -5,6 +5,8 @@
 
 namespace viola {
 
+__host__ __device__ static inline int64_t max64(int64_t a, int64_t b) { return a > b ? a : b; }
+
 // ------------------------------------------------------------------ amax
 template <typename TIn> struct Vec16;                       // 16 bytes of TIn
 template <> struct Vec16<float> { static constexpr int N = 4; };
@@ -262,6 +264,15 @@ __global__ __launch_bounds__(256) void rotation_inplace_kernel(T* __restrict__ x
     }
 }
 
+// What the quantizer may do on the side, so that small tensors (a few microseconds per launch) need fewer launches:
+//   maxima != null: form the tensor's scale from the amax pass's block maxima itself (every block reduces the at most 512
+//     floats again, one block also writes scale and history) instead of reading it from a launch in between;
+//   column_partial != null: blocks past the tiles each reduce 32 columns of the amax pass's column sums (the bias gradient).
+struct TensorQuantizeSide {
+    const float* maxima; int parts; float* history; int history_len; int64_t index; float* scale;
+    const float* column_partial; int64_t slices; void* column_sum; int sum_dtype; int64_t sum_blocks;
+};
+
 // 64 x 64 tile per 256-thread block: thread t quantizes 16 consecutive elements of tile row t / 4, stores them
 // row-wise (16 bytes) and, for the transposed layout, parks them in LDS, from where thread t collects 16 consecutive
 // rows of tile column t / 4. q = fp8(isnan(v) ? v : clamp(v / scale, +-limit)) with the one scale of the tensor.
@@ -269,20 +280,49 @@ __global__ __launch_bounds__(256) void rotation_inplace_kernel(T* __restrict__ x
 template <typename TIn, typename TOut, bool ROTATE>
 __global__ __launch_bounds__(256) void tensor_quantize_kernel(const TIn* __restrict__ x, const float* __restrict__ scale,
                                                                uint8_t* __restrict__ q, uint8_t* __restrict__ qt, int64_t rows,
-                                                               int64_t cols, float limit, int vector_in, int vector_q,
-                                                               int vector_qt) {
+                                                               int64_t cols, int64_t q_pitch, int64_t qt_pitch, float limit,
+                                                               int vector_in, int vector_q, int vector_qt, TensorQuantizeSide side) {
     constexpr int LD = 64 + 16;                                         // padded row of the parking tile (bytes)
     __shared__ __attribute__((aligned(16))) uint8_t park[64 * LD];
     const int tid = threadIdx.x, lr = tid / 4, lc = (tid % 4) * 16;
+    // the walk covers the padded outputs: columns up to q_pitch, rows up to qt_pitch (a pitch of 0: that output is absent)
+    const int64_t tiles_x = (max64(cols, q_pitch) + 63) / 64, tiles_y = (max64(rows, qt_pitch) + 63) / 64, tiles = tiles_x * tiles_y;
+    int64_t id = blockIdx.x;
+    if (side.column_partial) {                                          // these blocks first: they are the longer chains
+        if (id < side.sum_blocks) {
+            float(*piece)[32] = reinterpret_cast<float(*)[32]>(park);
+            if (side.sum_dtype == VIOLA_F32) reduce_columns<float>(side.column_partial, side.slices, cols, static_cast<float*>(side.column_sum), id, piece);
+            else if (side.sum_dtype == VIOLA_BF16) reduce_columns<bf16_t>(side.column_partial, side.slices, cols, static_cast<bf16_t*>(side.column_sum), id, piece);
+            else reduce_columns<f16_t>(side.column_partial, side.slices, cols, static_cast<f16_t*>(side.column_sum), id, piece);
+            return;
+        }
+        id -= side.sum_blocks;
+    }
     // blocks are dispatched in index order: those in flight together take a patch of 32 row tiles per column tile, then
     // the next column tile, so the transposed output is written in 2 KB runs per row however wide the matrix is
     constexpr int64_t BAND = 32;
-    const int64_t tiles_x = gridDim.x, tiles_y = gridDim.y, id = (int64_t)blockIdx.y * tiles_x + blockIdx.x;
     const int64_t patch = id / (BAND * tiles_x), within = id % (BAND * tiles_x);
     const int64_t tall = tiles_y - patch * BAND < BAND ? tiles_y - patch * BAND : BAND;
     const int64_t r0 = (patch * BAND + within % tall) * 64, c0 = within / tall * 64;
+    float s;
+    if (side.maxima) {
+        float m = 0.0f;
+        for (int i = tid; i < side.parts; i += 256) m = fmaxf(m, side.maxima[i]);
+        float* part = reinterpret_cast<float*>(park);
+        m = wave_max(m);
+        if (tid % WAVE == 0) part[tid / WAVE] = m;
+        __syncthreads();
+        const float amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+        __syncthreads();                                                // park is reused below
+        s = scale_of(amax, limit);
+        if (id == 0 && tid == 0) {
+            side.scale[0] = s;
+            side.history[side.index % side.history_len] = amax;
+        }
+    } else {
+        s = scale[0];
+    }
     const int64_t row = r0 + lr, col = c0 + lc;
-    const float s = scale[0];
     float v[16];
     load16<TIn>(x + row * cols, col, cols, row < rows, vector_in != 0, v);
     if constexpr (ROTATE) rotate64(v);
@@ -304,12 +344,12 @@ __global__ __launch_bounds__(256) void tensor_quantize_kernel(const TIn* __restr
         }
     }
     if (q && row < rows) {
-        uint8_t* dst = q + row * cols + col;
-        if (vector_q && col + 16 <= cols) {
+        uint8_t* dst = q + row * q_pitch + col;
+        if (vector_q && col + 16 <= q_pitch) {
             *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
         } else {
             for (int i = 0; i < 16; ++i)
-                if (col + i < cols) dst[i] = (uint8_t)(w[i / 4] >> (8 * (i % 4)));
+                if (col + i < q_pitch) dst[i] = (uint8_t)(w[i / 4] >> (8 * (i % 4)));
         }
     }
     if (qt) {
@@ -321,26 +361,29 @@ __global__ __launch_bounds__(256) void tensor_quantize_kernel(const TIn* __restr
         for (int i = 0; i < 16; ++i) t[i / 4] |= (uint32_t)park[(lc + i) * LD + lr] << (8 * (i % 4));
         const int64_t orow = c0 + lr, ocol = r0 + lc;
         if (orow < cols) {
-            uint8_t* dst = qt + orow * rows + ocol;
-            if (vector_qt && ocol + 16 <= rows) {
+            uint8_t* dst = qt + orow * qt_pitch + ocol;
+            if (vector_qt && ocol + 16 <= qt_pitch) {
                 *reinterpret_cast<uint4*>(dst) = make_uint4(t[0], t[1], t[2], t[3]);
             } else {
                 for (int i = 0; i < 16; ++i)
-                    if (ocol + i < rows) dst[i] = (uint8_t)(t[i / 4] >> (8 * (i % 4)));
+                    if (ocol + i < qt_pitch) dst[i] = (uint8_t)(t[i / 4] >> (8 * (i % 4)));
             }
         }
     }
 }
 
 template <typename TIn, typename TOut, bool ROTATE>
-static int launch_tensor_quantize(const void* x, const float* scale, void* q, void* qt, int64_t rows, int64_t cols, float limit,
-                                  hipStream_t stream) {
+static int launch_tensor_quantize(const void* x, const float* scale, void* q, int64_t q_pitch, void* qt, int64_t qt_pitch, int64_t rows,
+                                  int64_t cols, float limit, const TensorQuantizeSide& side, hipStream_t stream) {
     const int vector_in = reinterpret_cast<uintptr_t>(x) % 16 == 0 && (cols * sizeof(TIn)) % 16 == 0;
-    const int vector_q = q && reinterpret_cast<uintptr_t>(q) % 16 == 0 && cols % 16 == 0;
-    const int vector_qt = qt && reinterpret_cast<uintptr_t>(qt) % 16 == 0 && rows % 16 == 0;
-    const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((rows + 63) / 64));
-    VIOLA_LAUNCH((tensor_quantize_kernel<TIn, TOut, ROTATE>), grid, dim3(256), 0, stream, static_cast<const TIn*>(x), scale,
-                       static_cast<uint8_t*>(q), static_cast<uint8_t*>(qt), rows, cols, limit, vector_in, vector_q, vector_qt);
+    const int vector_q = q && reinterpret_cast<uintptr_t>(q) % 16 == 0 && q_pitch % 16 == 0;
+    const int vector_qt = qt && reinterpret_cast<uintptr_t>(qt) % 16 == 0 && qt_pitch % 16 == 0;
+    q_pitch = q ? q_pitch : 0;
+    qt_pitch = qt ? qt_pitch : 0;
+    const int64_t tiles = ((cols > q_pitch ? cols : q_pitch) + 63) / 64 * (((rows > qt_pitch ? rows : qt_pitch) + 63) / 64);
+    if (tiles + side.sum_blocks >= (1ll << 31)) return VIOLA_ETOOLARGE;
+    VIOLA_LAUNCH((tensor_quantize_kernel<TIn, TOut, ROTATE>), dim3((unsigned)(tiles + side.sum_blocks)), dim3(256), 0, stream, static_cast<const TIn*>(x), scale,
+                       static_cast<uint8_t*>(q), static_cast<uint8_t*>(qt), rows, cols, q_pitch, qt_pitch, limit, vector_in, vector_q, vector_qt, side);
     return viola_launch_status();
 }
 
@@ -404,12 +447,13 @@ extern "C" int viola_tensor_amax_scale(const void* x, int x_dtype, int64_t n, fl
 }
 
 template <bool ROTATE>
-static int tensor_quantize_entry(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale, void* q,
-                                 void* qt, int q_dtype, float limit, hipStream_t stream) {
+static int tensor_quantize_entry(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale, void* q, int64_t q_pitch,
+                                 void* qt, int64_t qt_pitch, int q_dtype, float limit, const TensorQuantizeSide& side, hipStream_t stream) {
     VIOLA_CHECK_ARG(viola_is_float(x_dtype) && viola_is_fp8(q_dtype) && rows >= 0 && cols >= 0 && limit > 0.0f);
+    VIOLA_CHECK_ARG((!q || q_pitch >= cols) && (!qt || qt_pitch >= rows));
     if (rows == 0 || cols == 0 || (!q && !qt)) return 0;
-    VIOLA_CHECK_ARG(x && scale && (rows + 63) / 64 <= 65535);
-#define VIOLA_TQ(TI, TO) return launch_tensor_quantize<TI, TO, ROTATE>(x, scale, q, qt, rows, cols, limit, stream)
+    VIOLA_CHECK_ARG(x && (scale || side.maxima));
+#define VIOLA_TQ(TI, TO) return launch_tensor_quantize<TI, TO, ROTATE>(x, scale, q, q_pitch, qt, qt_pitch, rows, cols, limit, side, stream)
     if (q_dtype == VIOLA_E4M3) {
         if (x_dtype == VIOLA_F32) VIOLA_TQ(float, e4m3_t);
         if (x_dtype == VIOLA_BF16) VIOLA_TQ(bf16_t, e4m3_t);
@@ -423,12 +467,69 @@ static int tensor_quantize_entry(const void* x, int x_dtype, int64_t rows, int64
 
 extern "C" int viola_tensor_quantize(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale, void* q,
                                      void* qt, int q_dtype, float limit, viola_stream_t stream) {
-    return tensor_quantize_entry<false>(x, x_dtype, rows, cols, scale, q, qt, q_dtype, limit, static_cast<hipStream_t>(stream));
+    return tensor_quantize_entry<false>(x, x_dtype, rows, cols, scale, q, cols, qt, rows, q_dtype, limit, {}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int viola_rotation_quantize(const void* x, int x_dtype, int64_t rows, int64_t cols, const float* scale, void* q,
                                        void* qt, int q_dtype, float limit, viola_stream_t stream) {
-    return tensor_quantize_entry<true>(x, x_dtype, rows, cols, scale, q, qt, q_dtype, limit, static_cast<hipStream_t>(stream));
+    return tensor_quantize_entry<true>(x, x_dtype, rows, cols, scale, q, cols, qt, rows, q_dtype, limit, {}, static_cast<hipStream_t>(stream));
+}
+
+// amax -> scale -> codes of one tensor at pitched rows, optionally with its column sums (see the header). Two launches where
+// the block maxima are few enough for every quantizer block to reduce them itself, otherwise the scale is a launch of its own;
+// with a delayed scale it always is (the history must be read before it is written).
+extern "C" int viola_tensor_encode(const void* x, int x_dtype, int64_t rows, int64_t cols, float* workspace, int64_t workspace_floats,
+                                   float* history, int history_len, int64_t index, int delayed, float limit, float* scale, void* q,
+                                   int64_t q_pitch, void* qt, int64_t qt_pitch, int q_dtype, void* column_sum, int sum_dtype,
+                                   viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG(viola_is_float(x_dtype) && viola_is_fp8(q_dtype) && rows > 0 && cols > 0 && x && workspace && history && history_len > 0);
+    VIOLA_CHECK_ARG(index >= 0 && limit > 0.0f && scale && (!column_sum || viola_is_float(sum_dtype)));
+    constexpr int64_t FEW = 512;
+    TensorQuantizeSide side = {};
+    int64_t parts;
+    int status;
+    if (column_sum) {
+        const int piece = 16 / viola_dtype_size(x_dtype);
+        if (cols % piece != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0) return VIOLA_EUNSUPPORTED;
+        const int64_t slices = viola_tensor_encode_slices(x_dtype, rows, cols);
+        parts = ((cols / piece + 255) / 256) * slices;
+        const int64_t sums_at = (parts + 3) / 4 * 4;                        // the partial sums are stored in 16-byte pieces
+        VIOLA_CHECK_ARG(workspace_floats >= sums_at + slices * cols && reinterpret_cast<uintptr_t>(workspace) % 16 == 0);
+        status = viola_tensor_amax_columns(x, x_dtype, rows, cols, slices, workspace, workspace + sums_at, stream_);
+        side.column_partial = workspace + sums_at;
+        side.slices = slices;
+        side.column_sum = column_sum;
+        side.sum_dtype = sum_dtype;
+        side.sum_blocks = (cols + 31) / 32;
+    } else {
+        // enough blocks that a thread holds a few 16-byte loads, at most what a quantizer block reduces on the side; large
+        // tensors take 1024 blocks (four per CU) to keep the memory busy
+        const int64_t n = rows * cols, wanted = (n + 8191) / 8192;
+        parts = wanted <= 2048 ? (wanted < 256 ? wanted : 256) : 1024;
+        VIOLA_CHECK_ARG(workspace_floats >= parts);
+        status = viola_tensor_amax(x, x_dtype, n, workspace, parts, stream_);
+    }
+    if (status) return status;
+    if (parts <= FEW && !(delayed && index != 0)) {
+        side.maxima = workspace;
+        side.parts = (int)parts;
+        side.history = history;
+        side.history_len = history_len;
+        side.index = index;
+        side.scale = scale;
+    } else {
+        status = viola_tensor_scale(workspace, parts, history, history_len, index, delayed, limit, scale, stream_);
+        if (status) return status;
+    }
+    return tensor_quantize_entry<false>(x, x_dtype, rows, cols, scale, q, q_pitch, qt, qt_pitch, q_dtype, limit, side, stream);
+}
+
+// Row slices of the amax-and-column-sums pass over a [rows, cols] matrix: about 512 blocks, at least eight rows each.
+extern "C" int64_t viola_tensor_encode_slices(int x_dtype, int64_t rows, int64_t cols) {
+    const int64_t piece = 16 / viola_dtype_size(x_dtype), blocks_x = max64(((cols + piece - 1) / piece + 255) / 256, 1), most = blocks_x < 512 ? 512 / blocks_x : 1;
+    const int64_t wanted = (rows + 7) / 8;
+    return wanted < most ? wanted : most;
 }
 
 extern "C" int viola_rotation_amax(const void* x, int x_dtype, int64_t rows, int64_t cols, float* maxima, int64_t parts,

@@ -8,6 +8,7 @@ transposed (1, 32) quantization of that group's own rows (32-token tiles counted
 first row). One launch covers all groups; empty groups yield no rows and a zero dW.
 """
 
+import functools
 import math
 
 import torch
@@ -15,11 +16,19 @@ from torch import nn
 
 from .. import _lib
 from . import _grouped_kernels as kernels
-from ._linear_kernels import transpose as transpose_payload
 from ..precision import settings
 
 _FORMATS = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
 GX, GW = (1, 32), (32, 32)
+
+
+@functools.lru_cache(maxsize=None)
+def _recipe(forward_dtype, backward_dtype):
+    """The recipe of the native host path (csrc/host.cpp), which runs forward and backward."""
+    forward, backward = _FORMATS[forward_dtype], _FORMATS[backward_dtype]
+    return _lib.host().Recipe({"grouped": True, "native": False, "delayed": False, "fp8_weight": True, "cache_transpose": False,
+                               "fwd": _lib.code(forward), "bwd": _lib.code(backward), "fwd_limit": torch.finfo(forward).max,
+                               "bwd_limit": torch.finfo(backward).max, "in": 0, "out": 0})
 
 
 def _offsets(counts, device):
@@ -34,17 +43,6 @@ def _offsets(counts, device):
     padded[-1] = (padded[-1] + 127) // 128 * 128
     both = torch.tensor([offsets, padded], dtype=torch.int64).to(device, non_blocking=True)
     return offsets, padded, both[0], both[1]
-
-
-def varlen_gemm(a, b, sa, sb, offsets_dev, *, out_dtype):
-    """a [M, K] codes with (1, 32) scales; b [G, N, K] codes with (32, 32) scales [G, N/32, K/32]."""
-    m, k = a.shape
-    groups, n, _ = b.shape
-    out = torch.empty((m, n), device=a.device, dtype=out_dtype)
-    _lib.call("viola_varlen_group_gemm", _lib.ptr(a), _lib.code(a.dtype), _lib.ptr(b), _lib.code(b.dtype),
-              _lib.ptr(sa), _lib.ptr(sb), _lib.ptr(offsets_dev), groups, m, n, k, GX[0], GX[1], GW[0], GW[1],
-              n * k, sb.shape[1] * sb.shape[2], _lib.ptr(out), _lib.code(out_dtype))
-    return out
 
 
 def quantize_transposed_segmented(x, dtype, offsets_dev, padded_dev, groups, t_total, *, rowwise=False):
@@ -66,63 +64,15 @@ def quantize_transposed_segmented(x, dtype, offsets_dev, padded_dev, groups, t_t
     return qt, st, q, s
 
 
-def varlen_wgrad(gt, xt, sgt, sxt, padded_dev, groups, *, out_dtype):
-    n, t_total = gt.shape
-    kout = xt.shape[0]
-    out = torch.empty((groups, n, kout), device=gt.device, dtype=out_dtype)
-    _lib.call("viola_varlen_wgrad_gemm", _lib.ptr(gt), _lib.code(gt.dtype), _lib.ptr(xt), _lib.code(xt.dtype),
-              _lib.ptr(sgt), _lib.ptr(sxt), _lib.ptr(padded_dev), groups, t_total, n, kout, _lib.ptr(out), _lib.code(out_dtype))
-    return out
-
-
-class _VarlenLinear(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, weight, weight_scale, counts, fp8, bwd_fp8, grad_dtype):
-        assert x.is_cuda and x.dim() == 2
-        x = x.contiguous()
-        groups = weight.shape[0]
-        offsets, padded, offsets_dev, padded_dev = _offsets(counts, x.device)
-        assert offsets[-1] == x.shape[0] and len(offsets) == groups + 1
-        need_w = ctx.needs_input_grad[1]
-        if need_w and x.shape[0]:
-            xt, sxt, qx, sx = quantize_transposed_segmented(x, fp8, offsets_dev, padded_dev, groups, padded[-1], rowwise=True)
-        else:
-            qx, sx = kernels.quantize(x, fp8, GX)
-            xt = sxt = x.new_empty(0)
-        y = varlen_gemm(qx, weight, sx, weight_scale, offsets_dev, out_dtype=x.dtype)
-        ctx.save_for_backward(xt, sxt, weight, weight_scale, offsets_dev, padded_dev)
-        ctx.meta = (groups, padded[-1], bwd_fp8, grad_dtype, x.dtype)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        xt, sxt, weight, weight_scale, offsets_dev, padded_dev = ctx.saved_tensors
-        groups, t_total, bwd_fp8, grad_dtype, x_dtype = ctx.meta
-        dy = dy.contiguous()
-        dx = dw = None
-        gt = None
-        if ctx.needs_input_grad[0]:
-            if ctx.needs_input_grad[1] and dy.shape[0]:
-                gt, sgt, qg, sg = quantize_transposed_segmented(dy, bwd_fp8, offsets_dev, padded_dev, groups, t_total, rowwise=True)
-            else:
-                qg, sg = kernels.quantize(dy, bwd_fp8, GX)
-            wt = transpose_payload(weight)
-            st = weight_scale.transpose(1, 2).contiguous()
-            dx = varlen_gemm(qg, wt, sg, st, offsets_dev, out_dtype=x_dtype)
-        if ctx.needs_input_grad[1]:
-            if gt is None:
-                gt, sgt = quantize_transposed_segmented(dy, bwd_fp8, offsets_dev, padded_dev, groups, t_total)
-            dw = varlen_wgrad(gt, xt, sgt, sxt, padded_dev, groups, out_dtype=grad_dtype)
-        return dx, dw, None, None, None, None, None
-
-
 def grouped_linear(x, weight, weight_scale, counts, *, forward_dtype="e4m3", backward_dtype="e4m3", grad_dtype=None):
     """y[rows of group g] = x[rows of group g] @ dequant(weight[g]).T for every group, one launch.
 
     weight [G, N, K] FP8 codes, weight_scale [G, ceil(N/32), ceil(K/32)] fp32, counts: rows per group
     (host list or CPU tensor, sum == x.shape[0])."""
+    assert x.is_cuda and x.dim() == 2
     grad_dtype = grad_dtype or weight.grad_dtype or torch.float32
-    return _VarlenLinear.apply(x, weight, weight_scale, counts, _FORMATS[forward_dtype], _FORMATS[backward_dtype], grad_dtype)
+    counts = counts.tolist() if isinstance(counts, torch.Tensor) else counts
+    return _lib.host().experts(x, weight, weight_scale, [int(c) for c in counts], _recipe(forward_dtype, backward_dtype), grad_dtype)
 
 
 class GroupedExperts(nn.Module):

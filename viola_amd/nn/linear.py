@@ -13,7 +13,8 @@ FP32, so the model runs on the generic kernel with explicit roundings; with `acc
 change nothing. `rotation_size=64` (per-tensor recipes only) stores and multiplies Hadamard-rotated X and W.
 
 How the module is put together: `_Numerics` checks the recipe options once and answers every question about clamp
-limits and scale storage; `_WeightStore` turns a master weight into what the module stores (codes, scales, the cached
+limits and scale storage and names the recipe for the native host path (csrc/host.cpp: forward and backward of the standard
+recipes; the options beyond them run through `_grouped_linear` / `_tensor_linear`); `_WeightStore` turns a master weight into what the module stores (codes, scales, the cached
 transpose) on the GPU; `Linear` itself owns the parameters and buffers under the names a checkpoint of the reference
 carries, and keeps their dtypes through module-wide casts.
 """
@@ -23,6 +24,7 @@ import math
 import torch
 from torch import nn
 
+from .. import _lib
 from . import _grouped_kernels as grouped
 from . import _linear_kernels as kernels
 from . import _rotation_kernels as rotation
@@ -40,8 +42,26 @@ class _Quantizer(nn.Module):
 
     def __init__(self, scaling, history_len, device):
         super().__init__()
-        self.scaling, self.index = scaling, 0
+        self.scaling, self._calls, self._counter = scaling, 0, None
         self.register_buffer("history", torch.zeros(history_len, device=device, dtype=torch.float32))
+
+    @property
+    def index(self):
+        """Calls so far: the next call's slot in the history. Kept by the native host path once that has taken a call."""
+        return self._calls if self._counter is None else self._counter.value
+
+    @index.setter
+    def index(self, value):
+        if self._counter is None:
+            self._calls = value
+        else:
+            self._counter.value = value
+
+    def counter(self):
+        """The counter itself, shared with the native host path (backward advances it off this thread)."""
+        if self._counter is None:
+            self._counter = _lib.host().Counter(self._calls)
+        return self._counter
 
     def _options(self, fp8_dtype, quantization_limit):
         return dict(history=self.history, index=self.index, delayed=self.scaling == "delayed", fp8_dtype=fp8_dtype,
@@ -113,6 +133,20 @@ class _Numerics:
 
     def tensor_limit(self, reduction, dtype):
         return self._clamp(self.accum_block_size or reduction, dtype)                      # linear.py:232-242
+
+    def standard(self, saved_input_dtype):
+        """Whether the native host path takes this recipe: the default group shapes, FP32 accumulation, no rotation, inputs
+        saved as FP8."""
+        groups = (self.weight_group_shape, self.input_group_shape, self.grad_group_shape)
+        return (groups == ((32, 32), (1, 32), (1, 32)) and self.accum_dtype == "fp32" and not self.rotation_size and saved_input_dtype == "fp8")
+
+    def native_recipe(self, layer):
+        limit = lambda dtype: float(self._clamp(1, dtype) or torch.finfo(dtype).max)
+        return _lib.host().Recipe({
+            "grouped": self._grouped_scaling, "native": self._native_scaling, "delayed": layer.input_quantizer.scaling == "delayed",
+            "fp8_weight": layer.weight_dtype == "fp8", "cache_transpose": layer.cache_weight_transpose, "fwd": _lib.code(self.fp8_dtype),
+            "bwd": _lib.code(self.backward_fp8_dtype), "fwd_limit": limit(self.fp8_dtype), "bwd_limit": limit(self.backward_fp8_dtype),
+            "in": layer.in_features, "out": layer.out_features})
 
     def scale_storage(self, weight_shape, fp8_storage):
         """(shape, dtype, initial value) of `weight_scale`: FP32 scales start at 1, E8M0 bytes at 127 = 2^0
@@ -216,6 +250,7 @@ class Linear(nn.Module):
         self.mode, self.weight_dtype, self.saved_input_dtype, self.autotune = mode, weight_dtype, saved_input_dtype, autotune
         self.cache_weight_transpose = (mode == "fast") if cache_weight_transpose is None else cache_weight_transpose
         self._store = _WeightStore(self)
+        self._standard, self._recipe = numerics.standard(saved_input_dtype), None
         self._master_ref = None
         self._allocate(bias, device, dtype or torch.get_default_dtype(), settings())
         for operand in ("weight", "input", "grad"):
@@ -309,6 +344,18 @@ class Linear(nn.Module):
         return layer
 
     # ------------------------------------------------------------------ execution
+    def _operands(self):
+        """What the native host path needs of this layer (its `layer_from`), read without nn.Module's attribute search."""
+        recipe = self._recipe
+        if recipe is None:
+            recipe = self._recipe = self._numerics.native_recipe(self)
+        held, buffers = self._parameters, self._buffers
+        operands = (recipe, held["weight"], held.get("bias"), buffers["weight_scale"], buffers["weight_transpose"], buffers["weight_transpose_scale"])
+        if self._grouped_scaling:
+            return operands
+        quantizers = [self._modules[name] for name in ("weight_quantizer", "input_quantizer", "grad_quantizer")]
+        return operands + tuple(q._buffers["history"] for q in quantizers) + tuple(q._counter or q.counter() for q in quantizers)
+
     def forward(self, x):
         assert x.is_cuda, "viola.nn.Linear executes on CUDA."
         if torch.is_autocast_enabled("cuda"):
@@ -316,6 +363,8 @@ class Linear(nn.Module):
         if self._store.pending:
             self.refresh_weight(self._master())
             assert not self._store.pending, _HOST_MASTER
+        if self._standard:
+            return _lib.host().linear(x, self._operands())
         trainable = [t for t in (x, self.weight, self.bias) if t is not None and t.requires_grad]
         need_backward = torch.is_grad_enabled() and bool(trainable)
         if self._grouped_scaling:
