@@ -1,0 +1,54 @@
+"""The native Newton-Schulz chain against the same chain product by product, and the native optimizer step on parameters
+that do not fit the table kernels."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("steps", [1, 2, 5])
+@pytest.mark.parametrize("method", ["standard", "gram"])
+@pytest.mark.parametrize("shape", [(64, 64), (3, 96, 160), (2, 160, 96), (33, 70)])
+def test_native_chain_equals_the_products_one_by_one(shape, method, steps):
+    from viola_amd.optim import _orthogonalize_kernels as nk
+    from viola_amd.optim._orthogonalize import METHODS
+    torch.manual_seed(steps)
+    x = torch.randn(*shape, device="cuda")
+    got, want = METHODS[method](x, steps=steps), nk.run(x, steps, method)
+    assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("options", [dict(granularity="block", block_shape=(16, 16)), dict(tile_size=64), dict(tile_size=256, rounding="stochastic")])
+def test_native_step_equals_stepping_each_parameter_alone(options):
+    """Ragged tiles, small tiles and 2-D blocks go through the per-tensor kernels; a batched 3-D group keeps its matrices;
+    bf16 weights round on store. Three steps, bit for bit what one optimizer per parameter gives."""
+    import viola_amd
+    shapes = [(48, 80), (48, 80), (33, 70), (2, 48, 64), (7,), (7,), (129,)]
+
+    def build(one_each):
+        torch.manual_seed(3)
+        params = [torch.nn.Parameter((torch.randn(*s, device="cuda") * .05).to(torch.bfloat16 if i == 1 else torch.float32)) for i, s in enumerate(shapes)]
+        groups = [dict(params=[p], batched=p.dim() == 3) for p in params]
+        make = lambda gs: viola_amd.optim.FP8Muon(gs, lr=2e-3, weight_decay=.01, rounding_seed=9, **options)
+        if not one_each:
+            return params, [make(groups)]
+        optimizers = [make([g]) for g in groups]
+        for i, opt in enumerate(optimizers):
+            opt.param_groups[0]["viola_parameter_indices"] = [i]
+        return params, optimizers
+
+    (together, one), (apart, each) = build(False), build(True)
+    for step in range(3):
+        torch.manual_seed(50 + step)
+        grads = [torch.randn(*s, device="cuda") * 1e-2 for s in shapes]
+        for params, optimizers in ((together, one), (apart, each)):
+            for i, (p, g) in enumerate(zip(params, grads)):
+                p.grad = g.to(p.dtype)
+            for opt in optimizers:
+                opt.step()
+    for i, (a, b) in enumerate(zip(together, apart)):
+        assert torch.equal(a, b), i
+        for key, value in one[0].state[a].items():
+            other = each[i].state[b][key]
+            assert torch.equal(value, other) if isinstance(value, torch.Tensor) else value == other == 3

@@ -33,26 +33,33 @@ def _filter(text):
     return "\n".join(line for line in text.splitlines() if "is not a recognized feature for this target" not in line)
 
 
-def _host_command():
-    """host.cpp is host code only (autograd nodes, no kernels): the system compiler, torch's headers, the library above."""
+HOST_SOURCES = ["host.cpp", "host_optim.cpp"]
+
+
+def _host_flags():
+    """Host code only (autograd nodes, no kernels): the system compiler, torch's headers, the library above."""
     import sysconfig
     import torch
     from torch.utils.cpp_extension import include_paths
     torch_lib = Path(torch.__file__).parent / "lib"
     includes = [f"-I{path}" for path in include_paths("cuda")] + [f"-I{sysconfig.get_paths()['include']}"]
-    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-            "-DTORCH_EXTENSION_NAME=_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, str(HERE / "host.cpp"),
-            "-o", str(HOST_LIBRARY), str(LIBRARY), f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
-            "-Wl,-rpath,$ORIGIN"]
+    compile_flags = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_host",
+                     f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes]
+    link_flags = ["-shared", str(LIBRARY), f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    return compile_flags, link_flags
 
 
-def _build_host(incremental):
-    sources = [HERE / "host.cpp", HERE.parents[1] / "include" / "viola_hip.h"]
-    if incremental and HOST_LIBRARY.exists() and HOST_LIBRARY.stat().st_mtime > max(f.stat().st_mtime for f in sources):
-        return
-    result = subprocess.run(_host_command(), capture_output=True, text=True)
+def _run(command, what):
+    result = subprocess.run(command, capture_output=True, text=True)
     if result.returncode != 0:
-        raise RuntimeError("building the native host path failed:\n" + result.stdout + result.stderr)
+        raise RuntimeError(f"{what} failed:\n" + _filter(result.stdout + result.stderr))
+
+
+def _host_object(name, incremental):
+    obj, headers = HERE / (name.rsplit(".", 1)[0] + ".o"), [HERE / "host.hpp", HERE.parents[1] / "include" / "viola_hip.h"]
+    if not (incremental and obj.exists() and obj.stat().st_mtime > max(f.stat().st_mtime for f in [HERE / name, *headers])):
+        _run([os.environ.get("CXX", "g++"), *_host_flags()[0], "-c", str(HERE / name), "-o", str(obj)], f"compiling {name}")
+    return obj
 
 
 def build(verbose=True, incremental=False):
@@ -60,7 +67,7 @@ def build(verbose=True, incremental=False):
     are newer than their source and every header."""
     compiler = hipcc()
     objects = []
-    newest_header = max(h.stat().st_mtime for h in HERE.glob("*.hpp"))
+    newest_header = max(h.stat().st_mtime for h in HERE.glob("*.hpp") if h.name != "host.hpp")
 
     def compile_one(name):
         obj = HERE / (name.rsplit(".", 1)[0] + ".o")
@@ -75,13 +82,13 @@ def build(verbose=True, incremental=False):
             print(message, file=sys.stderr)
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=8) as pool:
+        host_objects = [pool.submit(_host_object, name, incremental) for name in HOST_SOURCES]     # the longest compilations first
         objects = list(pool.map(compile_one, SOURCES))
+        host_objects = [job.result() for job in host_objects]
     link = [compiler, f"--offload-arch={ARCH}", "-shared", "-fPIC", f"-Wl,-soname,{LIBRARY.name}", *map(str, objects), "-o", str(LIBRARY)]
-    result = subprocess.run(link, capture_output=True, text=True)
-    if result.returncode != 0:
-        raise RuntimeError("link failed:\n" + _filter(result.stdout + result.stderr))
-    _build_host(incremental)
+    _run(link, "linking the library")
+    _run([os.environ.get("CXX", "g++"), *map(str, host_objects), "-o", str(HOST_LIBRARY), *_host_flags()[1]], "linking the native host path")
     return LIBRARY
 
 

@@ -9,89 +9,17 @@
 // Row pitches: every GEMM operand made here has rows of a whole number of 128 k where its k axis is a token count (weight
 // gradient), and of 16 k (128 under E8M0 scales) otherwise, padded with zero codes, and the GEMM takes the pitch as its k.
 // The sums do not change; whatever the sizes, the kernels that load 16-byte pieces take the product.
-#include <torch/extension.h>
+#include "host.hpp"
 
-#include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 
-#include <atomic>
-#include <memory>
-#include <string>
-#include <vector>
-
-#include "../../include/viola_hip.h"
-
-namespace py = pybind11;
-using at::Tensor;
+using namespace viola_host;
 using torch::autograd::Node;
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
 namespace {
-
-// ---------------------------------------------------------------------------------------------------- calls
-// Instrumented mode (the `timeline` of viola_amd._lib): every call is bracketed by two timing events on the current stream.
-std::atomic<bool> recording{false};
-// the list and torch.cuda.Event; process-wide and never released (the interpreter may be gone before static destructors run)
-py::object* timeline_sink = nullptr;
-py::object* event_class = nullptr;
-
-void check(const char* name, int status) {
-    TORCH_CHECK(status == 0, name, " failed: ", viola_error_string(status), " (status ", status, ")");
-}
-
-template <typename F>
-int timed(const char* name, F&& f) {
-    if (__builtin_expect(!recording.load(std::memory_order_relaxed), 1)) return f();
-    py::gil_scoped_acquire gil;
-    if (!timeline_sink || timeline_sink->is_none()) return f();
-    py::object start = (*event_class)(py::arg("enable_timing") = true), end = (*event_class)(py::arg("enable_timing") = true);
-    start.attr("record")();
-    const int status = f();
-    end.attr("record")();
-    timeline_sink->attr("append")(py::make_tuple(name, start, end));
-    return status;
-}
-// VIOLA_CALL raises on a non-zero status, VIOLA_TRY hands VIOLA_EUNSUPPORTED back to a caller that has another route
-#define VIOLA_CALL(fn, ...) check(#fn, timed(#fn, [&] { return fn(__VA_ARGS__); }))
-#define VIOLA_TRY(fn, ...) timed(#fn, [&] { return fn(__VA_ARGS__); })
-
-int code_of(at::ScalarType t) {
-    switch (t) {
-        case at::kFloat: return VIOLA_F32;
-        case at::kBFloat16: return VIOLA_BF16;
-        case at::kHalf: return VIOLA_F16;
-        case at::kFloat8_e4m3fn: return VIOLA_E4M3;
-        case at::kFloat8_e5m2: return VIOLA_E5M2;
-        default: TORCH_CHECK(false, "viola_amd kernels do not take tensors of type ", t);
-    }
-}
-
-viola_stream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
-const void* ptr(const Tensor& t) { return t.defined() && t.numel() ? t.const_data_ptr() : nullptr; }
-int64_t ceil_to(int64_t n, int64_t unit) { return (n + unit - 1) / unit * unit; }
-int64_t ceil_div(int64_t n, int64_t unit) { return (n + unit - 1) / unit; }
-
-// Several buffers of one lifetime as one allocation: take() reserves, make() allocates, at() hands out addresses.
-class Arena {
-public:
-    int64_t take(int64_t bytes) {
-        const int64_t begin = size_;
-        size_ += ceil_to(bytes, 256);
-        return begin;
-    }
-    void make(const at::Device& device) {
-        if (size_) buffer_ = at::empty({size_}, at::TensorOptions().dtype(at::kByte).device(device));
-    }
-    void* at(int64_t offset) const { return static_cast<char*>(buffer_.mutable_data_ptr()) + offset; }
-    template <typename T> T* as(int64_t offset) const { return static_cast<T*>(at(offset)); }
-    void release() { buffer_ = Tensor(); }
-
-private:
-    int64_t size_ = 0;
-    Tensor buffer_;
-};
 
 // ---------------------------------------------------------------------------------------------------- recipes
 // Calls of one per-tensor quantizer so far (its slot in the amax history); shared with nodes that advance it in backward.
@@ -883,6 +811,7 @@ PYBIND11_MODULE(_host, m) {
         *timeline_sink = list;
         recording.store(!list.is_none());
     });
+    register_optimizer(m);
     m.def("linear", [](const Tensor& x, const py::tuple& layer) {
         Layer l = layer_from(layer);
         py::gil_scoped_release release;

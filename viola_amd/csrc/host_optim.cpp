@@ -1,0 +1,456 @@
+// Native host path of the optimizer and the wire codec: FP8Muon's step over all parameters (buckets of equal-shaped matrices:
+// momentum, Newton-Schulz chain, weight update; AdamW for vectors) and FP8Communication's round trip.
+//
+// Why it is native: the step of one 1024 x 1024 matrix is 20 kernels of 3-9 us (about 170 us) and took 300 us of Python to
+// enqueue; per parameter a step costs about 1 us here.
+#include "host.hpp"
+
+#include <c10/core/Event.h>
+#include <c10/core/StreamGuard.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
+
+#include <algorithm>
+#include <cmath>
+#include <map>
+#include <tuple>
+
+using namespace viola_host;
+
+namespace {
+
+// ---------------------------------------------------------------------------------------------------- Newton-Schulz
+constexpr float A_COEFFICIENT = 3.4445f;
+
+// orthogonalize [..., rows, cols] in `steps` steps; every product of the chain reads and writes one arena, the last one the result
+Tensor newton_schulz(const Tensor& matrix_, int64_t steps, bool gram) {
+    TORCH_CHECK(matrix_.is_cuda() && matrix_.dim() >= 2 && steps > 0, "viola_amd kernels run on the GPU only");
+    const Tensor matrix = matrix_.contiguous();
+    const int64_t rows = matrix.size(-2), cols = matrix.size(-1), m = std::min(rows, cols), n = std::max(rows, cols);
+    const int64_t batch = rows * cols ? matrix.numel() / (rows * cols) : 0;
+    const bool tall = rows > cols;
+    const at::ScalarType type = gram ? at::kHalf : at::kBFloat16;
+    const int dtype = code_of(type);
+    const viola_stream_t stream = stream_of(matrix);
+    const Tensor result = at::empty(matrix.sizes(), matrix.options().dtype(type));
+    if (matrix.numel() == 0) return result;
+    const bool quintic = !gram || m == n;                        // the plain iteration; else the recurrence on the Gram matrix
+    const int64_t wide = 2 * batch * m * n, square = 2 * batch * m * m;
+    Arena arena;
+    const int64_t sums = arena.take(batch * 256 * 4);
+    int64_t x_at[2], s_at[6];
+    const int squares = quintic ? 2 : 6;
+    for (int64_t& at : x_at) at = arena.take(wide);
+    for (int i = 0; i < squares; ++i) s_at[i] = arena.take(square);
+    arena.make(matrix.device());
+    void *x = arena.at(x_at[0]), *spare = arena.at(x_at[1]);
+    VIOLA_CALL(viola_ns_prepare, matrix.const_data_ptr(), code_of(matrix.scalar_type()), x, dtype, batch, rows, cols, arena.as<float>(sums), stream);
+    auto gemm = [&](const void* a, const void* b, bool transpose_b, const void* residual, int epilogue, int64_t out_cols, int64_t k, void* out,
+                    float add_diag, void* out_diag, bool transpose_out) {
+        VIOLA_CALL(viola_ns_gemm, a, b, residual, out, dtype, transpose_b, epilogue, batch, m, out_cols, k, add_diag, out_diag, transpose_out, stream);
+    };
+    if (quintic) {
+        void *r = arena.at(s_at[0]), *z = arena.at(s_at[1]);
+        for (int64_t step = 0; step < steps; ++step) {
+            const bool last = step == steps - 1;
+            void* out = last ? result.mutable_data_ptr() : spare;
+            gemm(x, x, true, nullptr, 0, m, n, r, 0, nullptr, false);
+            gemm(r, r, true, r, 1, m, m, z, 0, nullptr, false);  // r = x x^T is symmetric bit for bit: r r = r r^T
+            gemm(z, x, false, x, 2, n, m, out, 0, nullptr, tall && last);
+            spare = x;
+            x = out;
+        }
+        return result;
+    }
+    void *r = arena.at(s_at[0]), *z = arena.at(s_at[1]), *q = arena.at(s_at[2]), *q_next = arena.at(s_at[3]), *rz = arena.at(s_at[4]), *r_next = arena.at(s_at[5]);
+    std::vector<int64_t> segments;
+    for (const int64_t length : {std::min<int64_t>(steps, 2), std::max<int64_t>(steps - 2, 0)})
+        if (length) segments.push_back(length);
+    for (size_t index = 0; index < segments.size(); ++index) {
+        const bool last = index + 1 == segments.size();
+        gemm(x, x, true, nullptr, 0, m, n, r, 0, nullptr, false);
+        for (int64_t i = 0; i < segments[index]; ++i) {
+            if (i == 0) {                                        // z and q = z + 3.4445 I from the one product
+                gemm(r, r, true, r, 1, m, m, z, A_COEFFICIENT, q, false);
+            } else {                                             // r = 3.4445 rz + z rz is symmetric only up to rounding: r r as written
+                gemm(r, r, false, r, 1, m, m, z, 0, nullptr, false);
+                gemm(z, q, false, q, 2, m, m, q_next, 0, nullptr, false);
+                std::swap(q, q_next);
+            }
+            if (i + 1 < segments[index]) {
+                gemm(z, r, false, r, 2, m, m, rz, 0, nullptr, false);
+                gemm(z, rz, false, rz, 2, m, m, r_next, 0, nullptr, false);
+                std::swap(r, r_next);
+            }
+        }
+        void* out = last ? result.mutable_data_ptr() : spare;
+        gemm(q, x, false, nullptr, 0, n, m, out, 0, nullptr, tall && last);
+        spare = x;
+        x = out;
+    }
+    return result;
+}
+
+// ---------------------------------------------------------------------------------------------------- FP8Muon.step
+// One parameter group's settings, read once per step.
+struct Group {
+    double lr, weight_decay, momentum, b1, b2, eps;
+    bool nesterov, batched, gram, match_rms;
+    int use_muon;                                                // -1: by the parameter's dimensions
+    int granularity, rounding, master_rounding;
+    int64_t tile, block_rows, block_cols, seed, master_seed, ns_steps;
+    at::ScalarType adam_state;
+};
+
+struct Item {
+    Tensor param, grad;
+    py::dict state;
+    const Group* group;
+    int64_t index, step;
+    Tensor q, scale;                                             // matrices: FP8 momentum and its scales
+    Tensor first, second;                                        // vectors: the moments
+};
+
+constexpr uint64_t MASK63 = (1ull << 63) - 1;
+int64_t rounding_key(int64_t seed, int64_t index, uint64_t stride) { return (int64_t)(((uint64_t)seed + (uint64_t)index * stride) & MASK63); }
+int64_t momentum_key(const Item& it) { return rounding_key(it.group->seed, it.index, 0x9E3779B97F4A7C15ull); }
+int64_t master_key(const Item& it) { return rounding_key(it.group->master_seed, it.index, 0x517CC1B727220A95ull); }
+bool aligned(const Tensor& t, int64_t bytes) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % bytes == 0; }
+int rounding_code(const py::handle& h) { return h.cast<std::string>() == "stochastic" ? VIOLA_STOCHASTIC : VIOLA_NEAREST; }
+
+Group read_group(const py::dict& d) {
+    Group g;
+    auto number = [&](const char* name) { return py::float_(py::object(d[name])).cast<double>(); };
+    auto integer = [&](const char* name) { return d[name].cast<int64_t>(); };
+    g.lr = number("lr"); g.weight_decay = number("weight_decay"); g.momentum = number("momentum"); g.eps = number("eps");
+    const auto betas = py::sequence(py::object(d["betas"])), block = py::sequence(py::object(d["block_shape"]));
+    g.b1 = betas[0].cast<double>(); g.b2 = betas[1].cast<double>();
+    g.block_rows = block[0].cast<int64_t>(); g.block_cols = block[1].cast<int64_t>();
+    g.nesterov = py::bool_(py::object(d["nesterov"])); g.batched = py::bool_(py::object(d["batched"]));
+    g.gram = d["ns_method"].cast<std::string>() == "gram";
+    g.match_rms = d["adjust_lr_fn"].cast<std::string>() == "match_rms_adamw";
+    g.use_muon = d["use_muon"].is_none() ? -1 : (int)(bool)py::bool_(py::object(d["use_muon"]));
+    g.granularity = d["granularity"].cast<std::string>() == "tile" ? 0 : 1;
+    g.rounding = rounding_code(d["rounding"]);
+    g.master_rounding = rounding_code(d["master_rounding"]);
+    g.tile = integer("tile_size"); g.seed = integer("rounding_seed"); g.master_seed = integer("master_rounding_seed"); g.ns_steps = integer("ns_steps");
+    g.adam_state = torch::python::detail::py_object_to_dtype(d["adam_state_dtype"]);
+    return g;
+}
+
+// The matrix a parameter stands for: conv filters flatten to [out, -1], batched groups keep their leading dimensions.
+std::vector<int64_t> matrix_shape(const Tensor& p, const Group& g) {
+    if (g.batched) return p.sizes().vec();
+    return {p.size(0), p.size(0) ? p.numel() / p.size(0) : 0};
+}
+
+class MuonHost {
+public:
+    void step(const py::list& work, const py::list& group_list) {
+        std::vector<Group> groups;
+        std::vector<PyObject*> handles;
+        groups.reserve(group_list.size());
+        for (const auto& g : group_list) {
+            groups.push_back(read_group(g.cast<py::dict>()));
+            handles.push_back(g.ptr());
+        }
+        // buckets in the order their first matrix comes; a bucket that would exceed batch_elements is closed and a new one begins
+        std::vector<std::vector<Item>> ready, vectors;
+        std::map<std::tuple<std::vector<int64_t>, int, bool, int64_t>, size_t> open;
+        using VectorKey = std::tuple<int, int, int, int, double, double, double, double, double, int64_t, int>;
+        std::map<VectorKey, size_t> vector_of;
+        for (const auto& entry : work) {
+            const auto t = entry.cast<py::tuple>();
+            Item it{t[0].cast<Tensor>(), t[1].cast<Tensor>(), t[2].cast<py::dict>(), nullptr, t[4].cast<int64_t>(), 0};
+            for (size_t i = 0; i < handles.size(); ++i)
+                if (handles[i] == t[3].ptr()) it.group = &groups[i];
+            TORCH_INTERNAL_ASSERT(it.group);
+            TORCH_CHECK(it.param.is_cuda() && !it.grad.is_sparse(), "viola_amd kernels run on the GPU only, on dense gradients");
+            const at::ScalarType kind = it.param.scalar_type();
+            if (kind != at::kFloat && kind != at::kBFloat16 && kind != at::kHalf) {
+                PyErr_SetString(PyExc_AssertionError, "Bind FP8 modules with viola.optim.bind_optimizer before stepping.");
+                throw py::error_already_set();
+            }
+            if (!it.state.contains("step")) it.state["step"] = 0;
+            it.step = it.state["step"].cast<int64_t>();
+            const Group& g = *it.group;
+            const int device = it.param.device().index();
+            const bool matrix = g.use_muon < 0 ? it.param.dim() >= 2 : g.use_muon != 0;
+            if (!matrix) {
+                const VectorKey key{device, (int)kind, (int)it.grad.scalar_type(), (int)g.adam_state, g.lr, g.weight_decay, g.b1, g.b2, g.eps, it.step, g.master_rounding};
+                const auto [at, fresh] = vector_of.try_emplace(key, vectors.size());
+                if (fresh) vectors.emplace_back();
+                prepare_vector(it);
+                vectors[at->second].push_back(std::move(it));
+                continue;
+            }
+            prepare_matrix(it);
+            const int64_t count = it.param.numel();
+            const auto key = std::make_tuple(matrix_shape(it.param, g), device, g.gram, g.ns_steps);
+            const auto [at, fresh] = open.try_emplace(key, ready.size());
+            if (fresh) ready.emplace_back();
+            std::vector<Item>& bucket = ready[at->second];
+            bucket.push_back(std::move(it));
+            if (((int64_t)bucket.size() + 1) * count > batch_elements) open.erase(at);
+        }
+        {
+            py::gil_scoped_release release;
+            step_buckets(ready);
+            for (auto& bucket : vectors) step_vectors(bucket);
+        }
+        for (auto* lists : {&ready, &vectors})
+            for (auto& bucket : *lists)
+                for (Item& it : bucket) it.state["step"] = it.step + 1;
+    }
+
+    int64_t lanes = 4;
+    // Equal-shaped matrices of one step go through Newton-Schulz as ONE batched chain (of at most this many elements): every
+    // matrix of the batch sees exactly the arithmetic it would see alone, and the launches fill the GPU.
+    int64_t batch_elements = 1ll << 28;
+
+    int64_t streams(int device) const {
+        const auto at = lanes_.find(device);
+        return at == lanes_.end() ? 0 : (int64_t)at->second.size();
+    }
+
+private:
+
+    // Device-side pointer tables, kept while their rows stay the same. Keyed by the stream that fills and reads them.
+    struct Table {
+        std::vector<int64_t> rows;
+        Arena arena;
+        int64_t at = 0;
+    };
+    std::map<std::tuple<viola_stream_t, int, std::vector<int64_t>, int64_t, int64_t>, Table> tables_;
+    std::map<int, std::vector<c10::Stream>> lanes_;
+
+    const int64_t* table(int kind, const std::vector<int64_t>& shape, int64_t count, int64_t ordinal, std::vector<int64_t>&& rows, const at::Device& device,
+                         viola_stream_t stream) {
+        Table& t = tables_[std::make_tuple(stream, kind, shape, count, ordinal)];
+        if (t.rows != rows) {
+            t.rows = std::move(rows);
+            t.arena = Arena();                                   // launches in flight may still read the old one: a new place
+            t.at = t.arena.take((int64_t)t.rows.size() * 8);
+            t.arena.make(device);
+            VIOLA_CALL(viola_store_words, t.arena.as<int64_t>(t.at), t.rows.data(), (int64_t)t.rows.size(), stream);
+        }
+        return t.arena.as<int64_t>(t.at);
+    }
+
+    static void prepare_vector(Item& it) {
+        if (!it.state.contains("exp_avg")) {
+            const auto options = at::TensorOptions().dtype(it.group->adam_state);
+            it.state["exp_avg"] = py::cast(at::zeros_like(it.param, options));
+            it.state["exp_avg_sq"] = py::cast(at::zeros_like(it.param, options));
+        }
+        it.first = it.state["exp_avg"].cast<Tensor>();
+        it.second = it.state["exp_avg_sq"].cast<Tensor>();
+    }
+
+    static void prepare_matrix(Item& it) {
+        TORCH_CHECK(it.param.dim() >= 2, "Muon updates matrices: a vector in a use_muon=True group");
+        if (!it.state.contains("momentum_q")) {
+            // 1-D tiles pad the payload to whole tiles, 2-D blocks do not
+            const Group& g = *it.group;
+            const std::vector<int64_t> shape = matrix_shape(it.param, g);
+            const int64_t n = it.param.numel(), rows = shape[shape.size() - 2], cols = shape.back();
+            int64_t payload = n, scales = ceil_div(n, g.tile);
+            if (g.granularity == 0) payload = scales * g.tile;
+            else scales = rows * cols ? n / (rows * cols) * ceil_div(rows, g.block_rows) * ceil_div(cols, g.block_cols) : 0;
+            const auto options = at::TensorOptions().device(it.param.device());
+            it.state["momentum_q"] = py::cast(at::zeros({payload}, options.dtype(at::kByte)));
+            it.state["momentum_scale"] = py::cast(at::ones({scales}, options.dtype(at::kFloat)));
+        }
+        it.q = it.state["momentum_q"].cast<Tensor>();
+        it.scale = it.state["momentum_scale"].cast<Tensor>();
+    }
+
+    // The chains of different buckets are independent, and a single chain leaves the GPU partly idle at every launch boundary
+    // (a Newton-Schulz GEMM of 28 matrices is ~590 tiles for 512 tile slots: its second round is nearly empty). Buckets
+    // therefore go to up to `lanes` streams of default priority, so the blocks of one chain fill the tails of the others; the
+    // caller's stream waits for all of them at the end.
+    void step_buckets(std::vector<std::vector<Item>>& ready) {
+        // buckets of one shape and size (a shape split because it exceeds batch_elements) each keep their own pointer tables
+        std::map<std::pair<std::vector<int64_t>, size_t>, int64_t> seen;
+        std::vector<int64_t> ordinals;
+        bool one_device = true;
+        for (const auto& bucket : ready) {
+            ordinals.push_back(seen[{matrix_shape(bucket[0].param, *bucket[0].group), bucket.size()}]++);
+            one_device = one_device && bucket[0].param.device() == ready[0][0].param.device();
+        }
+        if (ready.size() < 2 || lanes < 2 || !one_device) {
+            for (size_t i = 0; i < ready.size(); ++i) step_bucket(ready[i], ordinals[i]);
+            return;
+        }
+        const at::Device device = ready[0][0].param.device();
+        const c10::impl::VirtualGuardImpl guard(device.type());
+        std::vector<c10::Stream>& streams = lanes_[device.index()];
+        const size_t used = std::min<size_t>(lanes, ready.size());
+        while (streams.size() < used) streams.push_back(guard.getStreamFromGlobalPool(device, false));
+        const c10::Stream main = guard.getStream(device);
+        c10::Event start(device.type());
+        start.record(main);
+        // largest chains first, one lane after the other: the long ones start together and the short ones pack behind
+        std::vector<size_t> order(ready.size());
+        for (size_t i = 0; i < order.size(); ++i) order[i] = i;
+        auto elements = [&](size_t i) { return (int64_t)ready[i].size() * ready[i][0].param.numel(); };
+        std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return elements(a) > elements(b); });
+        for (size_t slot = 0; slot < order.size(); ++slot) {
+            const c10::Stream lane = streams[slot % used];
+            if (slot < used) start.block(lane);
+            const c10::StreamGuard on(lane);
+            step_bucket(ready[order[slot]], ordinals[order[slot]]);
+        }
+        for (size_t i = 0; i < used; ++i) {
+            c10::Event done(device.type());
+            done.record(streams[i]);
+            done.block(main);
+        }
+    }
+
+    static double update_scale(const Group& g, int64_t rows, int64_t cols) {
+        return g.match_rms ? .2 * std::pow((double)std::max(rows, cols), .5) : std::pow(std::max(1., (double)rows / (double)cols), .5);
+    }
+
+    void step_bucket(std::vector<Item>& bucket, int64_t ordinal) {
+        const Item& head = bucket[0];
+        const Group& g = *head.group;
+        const std::vector<int64_t> shape = matrix_shape(head.param, g);
+        const int64_t size = (int64_t)bucket.size(), count = head.param.numel(), rows = shape[shape.size() - 2], cols = shape.back();
+        if (count == 0) return;
+        const at::Device device = head.param.device();
+        const viola_stream_t stream = stream_of(head.param);
+        const Tensor updates_in = at::empty({size, count / (rows * cols), rows, cols}, at::TensorOptions().dtype(at::kBFloat16).device(device));
+        char* out = static_cast<char*>(updates_in.mutable_data_ptr());
+        std::vector<Tensor> grads;
+        for (Item& it : bucket) grads.push_back(it.grad.contiguous());
+
+        // ---- momentum: one launch for the bucket when its members share the recipe and fit the table kernel, else one each
+        const at::ScalarType kind = grads[0].scalar_type();
+        bool together = g.granularity == 0 && g.tile >= 256 && count % g.tile == 0 && size <= 65535 && (2 * count) % 8 == 0;
+        for (size_t i = 0; together && i < bucket.size(); ++i) {
+            const Item& it = bucket[i];
+            const Group& h = *it.group;
+            together = it.step == head.step && h.granularity == g.granularity && h.tile == g.tile && h.momentum == g.momentum && h.nesterov == g.nesterov &&
+                       h.rounding == g.rounding && grads[i].scalar_type() == kind && grads[i].numel() == count &&
+                       aligned(grads[i], 4 * grads[i].element_size()) && aligned(it.q, 4);
+        }
+        if (together) {
+            std::vector<int64_t> words;
+            for (size_t i = 0; i < bucket.size(); ++i) {
+                const int64_t q = (int64_t)bucket[i].q.const_data_ptr(), s = (int64_t)bucket[i].scale.const_data_ptr();
+                const int64_t row[8] = {(int64_t)grads[i].const_data_ptr(), q, s, q, s, (int64_t)(out + 2 * count * i), momentum_key(bucket[i]), 0};
+                words.insert(words.end(), row, row + 8);
+            }
+            const int64_t* t = table(0, shape, size, ordinal, std::move(words), device, stream);
+            VIOLA_CALL(viola_momentum_update_table, t, size, count / g.tile, code_of(kind), (int)g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step,
+                       stream);
+        } else {
+            for (size_t i = 0; i < bucket.size(); ++i) {
+                const Item& it = bucket[i];
+                const Group& h = *it.group;
+                const bool blocks = h.granularity == 1;
+                void* q = it.q.mutable_data_ptr();
+                float* s = static_cast<float*>(it.scale.mutable_data_ptr());
+                VIOLA_CALL(viola_momentum_update, grads[i].const_data_ptr(), code_of(grads[i].scalar_type()), q, s, q, s, out + 2 * count * i, count, (float)h.momentum,
+                           1.0f, h.nesterov, h.granularity, blocks ? 0 : (int)h.tile, blocks ? count / (rows * cols) : 1, blocks ? rows : 1, blocks ? cols : 1,
+                           blocks ? (int)h.block_rows : 1, blocks ? (int)h.block_cols : 1, h.rounding, it.step, momentum_key(it), stream);
+            }
+        }
+
+        const Tensor updates = newton_schulz(updates_in, g.ns_steps, g.gram);
+        const char* from = static_cast<const char*>(updates.const_data_ptr());
+        const int update_code = code_of(updates.scalar_type());
+
+        // ---- weights
+        together = count % 4 == 0 && size <= 65535;
+        for (const Item& it : bucket) {
+            const Group& h = *it.group;
+            together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms && it.param.scalar_type() == at::kFloat &&
+                       it.param.is_contiguous() && aligned(it.param, 16);
+        }
+        if (together) {
+            std::vector<int64_t> words;
+            for (size_t i = 0; i < bucket.size(); ++i) {
+                words.push_back((int64_t)bucket[i].param.const_data_ptr());
+                words.push_back((int64_t)(from + 2 * count * i));
+            }
+            const int64_t* t = table(1, shape, size, ordinal, std::move(words), device, stream);
+            VIOLA_CALL(viola_weight_update_table, t, size, count, update_code, (float)g.lr, (float)g.weight_decay, (float)update_scale(g, rows, cols), stream);
+            return;
+        }
+        for (size_t i = 0; i < bucket.size(); ++i) {
+            const Item& it = bucket[i];
+            const Group& h = *it.group;
+            TORCH_CHECK(it.param.is_contiguous(), "FP8Muon updates contiguous parameters");
+            VIOLA_CALL(viola_weight_update, it.param.mutable_data_ptr(), code_of(it.param.scalar_type()), from + 2 * count * i, update_code, count, (float)h.lr,
+                       (float)h.weight_decay, (float)update_scale(h, rows, cols), h.master_rounding, it.step, master_key(it), 0, stream);
+        }
+    }
+
+    // Vectors (biases, norms, modulation tables) are a few thousand elements each: those that share dtypes, hyper-parameters
+    // and step count take AdamW in one launch over a table of their pointers.
+    void step_vectors(std::vector<Item>& bucket) {
+        const Item& head = bucket[0];
+        const Group& g = *head.group;
+        const viola_stream_t stream = stream_of(head.param);
+        const double step = (double)(head.step + 1);
+        const float inv_c1 = (float)(1. / (1. - std::pow(g.b1, step))), inv_c2 = (float)(1. / (1. - std::pow(g.b2, step)));
+        const int weight_code = code_of(head.param.scalar_type()), grad_code = code_of(head.grad.scalar_type()), state_code = code_of(head.first.scalar_type());
+        std::vector<int64_t> words;
+        int64_t most = 0;
+        std::vector<Tensor> grads;
+        bool together = bucket.size() > 1 && bucket.size() <= 65535;
+        for (const Item& it : bucket) {
+            TORCH_CHECK(it.param.is_contiguous() && it.first.scalar_type() == it.second.scalar_type() && it.grad.numel() == it.param.numel());
+            together = together && it.grad.is_contiguous() && it.first.is_contiguous() && it.second.is_contiguous() &&
+                       it.first.scalar_type() == head.first.scalar_type();
+            grads.push_back(it.grad.contiguous());
+            const int64_t row[7] = {(int64_t)it.param.const_data_ptr(), (int64_t)grads.back().const_data_ptr(), (int64_t)it.first.const_data_ptr(),
+                                    (int64_t)it.second.const_data_ptr(), it.param.numel(), master_key(it), 0};
+            words.insert(words.end(), row, row + 7);
+            most = std::max(most, it.param.numel());
+        }
+        if (together) {
+            // one table per bucket of equal settings, told apart by what the first row points at
+            const int64_t* t = table(2, {words[0]}, (int64_t)bucket.size(), 0, std::move(words), head.param.device(), stream);
+            VIOLA_CALL(viola_adam_update_table, t, (int64_t)bucket.size(), most, weight_code, grad_code, state_code, (float)g.lr, (float)g.weight_decay, (float)g.b1,
+                       (float)g.b2, inv_c1, inv_c2, (float)g.eps, g.master_rounding, head.step, 1, 0, stream);
+            return;
+        }
+        for (size_t i = 0; i < bucket.size(); ++i) {
+            const Item& it = bucket[i];
+            if (it.param.numel() == 0) continue;
+            VIOLA_CALL(viola_adam_update, it.param.mutable_data_ptr(), weight_code, grads[i].const_data_ptr(), grad_code, it.first.mutable_data_ptr(),
+                       it.second.mutable_data_ptr(), code_of(it.first.scalar_type()), it.param.numel(), (float)g.lr, (float)g.weight_decay, (float)g.b1, (float)g.b2,
+                       inv_c1, inv_c2, (float)g.eps, g.master_rounding, it.step, master_key(it), 0, 1, 0, stream);
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------------------------------- wire codec
+// value <- decode(encode(value)) through the packet buffer
+void roundtrip(const Tensor& value, const Tensor& send, int64_t tile, py::object format) {
+    const int code = code_of(torch::python::detail::py_object_to_dtype(format));
+    TORCH_CHECK(value.is_cuda() && value.scalar_type() == at::kFloat && value.is_contiguous() && send.is_cuda() && send.is_contiguous());
+    const int64_t groups = ceil_div(value.numel(), tile);
+    TORCH_CHECK(ceil_to(groups * (tile + 4), 16) <= send.numel(), "the bucket exceeds the codec's capacity");
+    if (value.numel() == 0) return;
+    const viola_stream_t stream = stream_of(value);
+    float* x = static_cast<float*>(value.mutable_data_ptr());
+    void* packet = send.mutable_data_ptr();
+    VIOLA_CALL(viola_comm_pack, x, value.numel(), packet, 1, groups, (int)tile, code, stream);
+    VIOLA_CALL(viola_comm_unpack, packet, x, value.numel(), 1, groups, (int)tile, code, 0, stream);
+}
+
+}  // namespace
+
+namespace viola_host {
+
+void register_optimizer(py::module_& m) {
+    m.def("newton_schulz", &newton_schulz, py::arg("matrix"), py::arg("steps"), py::arg("gram"), py::call_guard<py::gil_scoped_release>());
+    m.def("roundtrip", &roundtrip);
+    py::class_<MuonHost>(m, "MuonHost").def(py::init<>()).def("step", &MuonHost::step).def_readwrite("lanes", &MuonHost::lanes)
+        .def_readwrite("batch_elements", &MuonHost::batch_elements).def("streams", &MuonHost::streams);
+}
+
+}  // namespace viola_host

@@ -477,10 +477,10 @@ static int launch_pack(const float* x, int64_t n, uint8_t* packet, int64_t rows,
 }
 
 // ------------------------------------------------------------------ small tables by value
-// Up to 64 words travel as the kernel's own arguments, so a table of offsets reaches the device in stream order without a
+// Up to 256 words travel as the kernel's own arguments, so a table of offsets reaches the device in stream order without a
 // staging buffer or a copy the host waits for.
-struct Words64 { int64_t v[64]; };
-__global__ __launch_bounds__(64) void store_words_kernel(int64_t* __restrict__ dst, Words64 words, int count) {
+struct Words { int64_t v[256]; };
+__global__ __launch_bounds__(256) void store_words_kernel(int64_t* __restrict__ dst, Words words, int count) {
     if ((int)threadIdx.x < count) dst[threadIdx.x] = words.v[threadIdx.x];
 }
 
@@ -604,11 +604,11 @@ extern "C" const char* viola_error_string(int code) {
 extern "C" int viola_store_words(int64_t* dst, const int64_t* host_words, int64_t count, viola_stream_t stream_) {
     hipStream_t stream = viola_enter(stream_);
     VIOLA_CHECK_ARG(count >= 0 && (count == 0 || (dst && host_words)));
-    for (int64_t done = 0; done < count; done += 64) {
-        Words64 words = {};
-        const int n = (int)(count - done < 64 ? count - done : 64);
+    for (int64_t done = 0; done < count; done += 256) {
+        Words words = {};
+        const int n = (int)(count - done < 256 ? count - done : 256);
         for (int i = 0; i < n; ++i) words.v[i] = host_words[done + i];
-        VIOLA_LAUNCH(store_words_kernel, dim3(1), dim3(64), 0, stream, dst + done, words, n);
+        VIOLA_LAUNCH(store_words_kernel, dim3(1), dim3(256), 0, stream, dst + done, words, n);
     }
     return viola_launch_status();
 }
