@@ -306,3 +306,53 @@ def test_varlen_segmented_quantizer_rowwise_byproduct(counts, cols, dtype):
         assert qt[:, padded[group] + count:padded[group + 1]].view(torch.uint8).count_nonzero() == 0
     assert padded[-1] % 128 == 0 and qt.shape == (cols, padded[-1])
 
+
+
+@pytest.mark.parametrize("scaling", ["tensor", "mx"])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,formats", [(4000, 1030, 1088, (0, 0)), (4096, 520, 4224, (1, 0)), (2048, 1024, 128, (0, 1)), (8192, 2048, 192, (0, 0)),
+                                           (1100, 1900, 3200, (1, 1)), (4097, 4101, 512, (0, 0))])
+def test_large_tile_products_at_tile_edges(m, n, k, formats, out_dtype, scaling):
+    """Sizes that the tile chooser sends to the 256 x 256, 256 x 128 and 128 x 128 alternating-phase kernels, with rows and
+    columns past the last whole tile, k of one chunk up to many and with a chunk cut short, bias on: integer operands and
+    power-of-two scales, so the sums are exact and every element must equal the integer product."""
+    from viola_amd.nn import _grouped_kernels as g, _linear_kernels as lk
+    if scaling == "mx":
+        k = -(-k // 128) * 128
+    torch.manual_seed(m + n + k)
+    fmt = (torch.float8_e4m3fn, torch.float8_e5m2)
+    a, b = torch.randint(-2, 3, (m, k), device="cuda").float(), torch.randint(-2, 3, (n, k), device="cuda").float()
+    bias = torch.randint(-8, 9, (n,), device="cuda").float()
+    qa, qb = a.to(fmt[formats[0]]), b.to(fmt[formats[1]])
+    if scaling == "tensor":
+        sa, sb = torch.full((1,), 2.0, device="cuda"), torch.full((1,), .5, device="cuda")
+        out = lk.gemm(qa, qb, sa, sb, out_dtype=out_dtype, bias=bias)
+        want = a @ b.T + bias
+    else:
+        sa = torch.randint(126, 129, (m, k // 32), device="cuda", dtype=torch.uint8)
+        sb = torch.randint(126, 129, (n, k // 32), device="cuda", dtype=torch.uint8)
+        spell = lambda t, s: t * torch.exp2(s.float() - 127).repeat_interleave(32, 1)
+        out = g.gemm(qa, qb, sa, sb, (1, 32), (1, 32), out_dtype=out_dtype, bias=bias, native=True)
+        want = spell(a, sa) @ spell(b, sb).T + bias
+    assert torch.equal(out, want.to(out_dtype))
+
+
+@pytest.mark.parametrize("scaling", ["tensor", "mx"])
+@pytest.mark.parametrize("m,h,k", [(4100, 2050, 640), (8192, 1024, 256)])
+def test_large_tile_gated_forward_without_aux_equals_the_kept_form(m, h, k, scaling):
+    """act(g) * u from the large tile's own epilogue (nothing kept) against the product that keeps [g | u] and the pass over it."""
+    from types import SimpleNamespace
+    from viola_amd.nn import _mlp_kernels as mk
+    torch.manual_seed(m)
+    if scaling == "mx":
+        h = h // 32 * 32
+    a, b = torch.randn(m, k, device="cuda").to(torch.float8_e4m3fn), torch.randn(2 * h, k, device="cuda").to(torch.float8_e4m3fn)
+    bias = torch.randn(2 * h, device="cuda")
+    layer = SimpleNamespace(_grouped_scaling=scaling == "mx", _native_scaling=scaling == "mx", accum_dtype="fp32", input_group_shape=(1, 32), weight_group_shape=(32, 32))
+    if scaling == "mx":
+        sa = torch.randint(120, 124, (m, k // 32), device="cuda", dtype=torch.uint8)
+        sb = torch.randint(120, 124, (2 * h // 32, k // 32), device="cuda", dtype=torch.uint8)
+    else:
+        sa, sb = torch.full((1,), .1, device="cuda"), torch.full((1,), .1, device="cuda")
+    call = lambda save: mk.gemm(a, b, sa, sb, layer=layer, out_dtype=torch.bfloat16, activation="gelu", bias=bias, save=save)[0]
+    assert torch.equal(call(True), call(False))

@@ -8,10 +8,10 @@ template <int MODE, bool B_ROWSCALE, typename TO, int TN, bool KSPLIT = false>
 static void launch_formats(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, dim3 grid, hipStream_t stream) {
     const bool a5 = a_dtype == VIOLA_E5M2, b5 = b_dtype == VIOLA_E5M2;
     const dim3 block(KSPLIT ? 2 * FTHREADS : FTHREADS);
-    if (!a5 && !b5) VIOLA_LAUNCH((group_gemm_fast<MODE, false, false, B_ROWSCALE, TO, TN, false, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
-    else if (a5 && !b5) VIOLA_LAUNCH((group_gemm_fast<MODE, true, false, B_ROWSCALE, TO, TN, false, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
-    else if (!a5 && b5) VIOLA_LAUNCH((group_gemm_fast<MODE, false, true, B_ROWSCALE, TO, TN, false, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
-    else VIOLA_LAUNCH((group_gemm_fast<MODE, true, true, B_ROWSCALE, TO, TN, false, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
+    if (!a5 && !b5) VIOLA_LAUNCH((group_gemm_fast<MODE, false, false, B_ROWSCALE, TO, TN, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
+    else if (a5 && !b5) VIOLA_LAUNCH((group_gemm_fast<MODE, true, false, B_ROWSCALE, TO, TN, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
+    else if (!a5 && b5) VIOLA_LAUNCH((group_gemm_fast<MODE, false, true, B_ROWSCALE, TO, TN, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
+    else VIOLA_LAUNCH((group_gemm_fast<MODE, true, true, B_ROWSCALE, TO, TN, false, false, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
 }
 
 // plain mode, the k range of a tile split over two teams of waves

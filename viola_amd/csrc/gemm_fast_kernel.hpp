@@ -28,9 +28,6 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int FBK = 64, FKG = FBK / 32;                           // k bytes and K groups per LDS stage
 constexpr int FTHREADS = 256, FSTAGES = 3;
-#ifndef VIOLA_BIG_STAGES
-#define VIOLA_BIG_STAGES 3                                         // ring depth of the 256 x 256 tile kernels (4 measured the same)
-#endif
 constexpr int F_TILE = BM * FBK;                                  // bytes of one operand tile
 constexpr int F_STAGE = 2 * F_TILE;
 // Scales travel in blocks of 8 K groups (4 chunks): 32 bytes per row and operand, fetched as two 16-byte pieces
@@ -121,29 +118,22 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // group 1), so lane (row, half) hands over the scale byte of K group `half` of its row. Scales travel in blocks of 16
 // K groups (one 16-byte piece per tile row and operand), double-buffered behind the ring; k must be a multiple of 128.
 constexpr int MX_GROUPS = 16, MX_CHUNKS = MX_GROUPS / FKG, MX_BLOCK = 2 * BM * MX_GROUPS;   // bytes of one block, a then b
-// BIG (per-tensor and block-scaled recipes): a 256 x 256 tile per 512-thread block, 2 x 4 waves of 4 x 2
-// sub-tiles, one block per CU. Without the per-group fold these kernels are bound by the L2 -> LDS stream (taking the
-// global loads out of the 128 x 128 kernel brings it from 1.7 to 4.4 PFLOP/s on a 16384 x 22016 x 4096 product, taking
-// the LDS reads out changes nothing); the larger tile moves half the bytes per flop.
 // KSPLIT (plain mode): for products with fewer than 512 tiles of 128 x 128 and a long k, such as a weight gradient. A
 // block of 512 threads is two teams of 2 x 2 waves, each with a stage ring and scale buffers of its own, that compute
 // the same 128 x 128 tile over the two halves of the k range (cut at a multiple of 256 k, one scale block); at the end
 // team 1 hands its totals over in LDS and team 0 adds them to its own (always in that order) and stores the tile.
 // Against the 128 x 64 tiles such products would otherwise get, a wave has the 2 x 2 sub-tiles' better ratio of MFMAs to
 // global loads and LDS reads, and a CU still holds eight waves.
-template <int MODE, bool A_BF8, bool B_BF8, bool B_ROWSCALE, typename TO, int TN, bool TENSOR = false, bool MX = false, bool BIG = false,
-          bool KSPLIT = false>
-__global__ __launch_bounds__(BIG || KSPLIT ? 512 : FTHREADS, BIG || KSPLIT ? 1 : TENSOR ? 3 : 2) void group_gemm_fast(GemmArgs p, int bias_dtype) {
-    static_assert(!KSPLIT || (MODE == MODE_PLAIN && !BIG), "the split exists for plain products on the small tiles");
+template <int MODE, bool A_BF8, bool B_BF8, bool B_ROWSCALE, typename TO, int TN, bool TENSOR = false, bool MX = false, bool KSPLIT = false>
+__global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 2) void group_gemm_fast(GemmArgs p, int bias_dtype) {
+    static_assert(!KSPLIT || MODE == MODE_PLAIN, "the split exists for plain products");
     static_assert(!TENSOR || !B_ROWSCALE, "per-tensor scaling has no row scales");
     static_assert(!MX || !TENSOR, "one scaling recipe per kernel");
-    static_assert(!BIG || ((TENSOR || MX) && TN == 2), "the large tile exists for the fold-free kernels");
     constexpr bool NOFOLD = TENSOR || MX;                                   // the products of a chunk go straight into the totals
-    constexpr int WAVES_N = BIG ? 4 : 2, THREADS = BIG ? 512 : FTHREADS;     // waves as 2 (m) x WAVES_N (n)
-    constexpr int TBM = BIG ? 2 * BM : BM;                                   // rows of a per tile
-    constexpr int K_TILE_A = BIG ? 2 * F_TILE : F_TILE, K_STAGE = BIG ? 4 * F_TILE : F_STAGE;
-    constexpr int K_STAGES = BIG ? VIOLA_BIG_STAGES : FSTAGES, K_RAW = K_STAGES * K_STAGE;   // ring depth: loads run K_STAGES chunks ahead
-    constexpr int K_MX_BLOCK = BIG ? 2 * MX_BLOCK : MX_BLOCK;
+    constexpr int WAVES_N = 2, THREADS = FTHREADS;                           // waves as 2 (m) x WAVES_N (n)
+    constexpr int TBM = BM;                                                  // rows of a per tile
+    constexpr int K_TILE_A = F_TILE, K_STAGE = F_STAGE, K_STAGES = FSTAGES, K_RAW = K_STAGES * K_STAGE;   // ring depth: loads run K_STAGES chunks ahead
+    constexpr int K_MX_BLOCK = MX_BLOCK;
     // without scale blocks the ring plus the epilogue's bias row is all the LDS a block needs: three blocks share a CU
     constexpr int TEAM_LDS = TENSOR ? K_RAW + 1024 : MX ? K_RAW + 2 * K_MX_BLOCK : F_LDS;
     __shared__ __attribute__((aligned(1024))) uint8_t lds_all[(KSPLIT ? 2 : 1) * TEAM_LDS];
@@ -152,7 +142,7 @@ __global__ __launch_bounds__(BIG || KSPLIT ? 512 : FTHREADS, BIG || KSPLIT ? 1 :
     // 64 wn + 32 i. Gated forward: the tile's b rows are 64 gate rows then the 64 up rows of the same n, and
     // i = 0 / 1 is the gate / up sub-tile of columns 32 wn .. 32 wn + 31, so one lane holds g and u of the same n.
     constexpr bool GATED = MODE == MODE_GATED_FWD;
-    constexpr int TM = BIG ? 4 : 2;
+    constexpr int TM = 2;
     constexpr int PANEL = GATED ? 32 * WAVES_N : 32 * TN * WAVES_N;
     static_assert(!GATED || TN == 2, "gated forward pairs a gate and an up sub-tile");
     // KSPLIT: `team` is the half of the k range this wave works on; tid, wave and lds are the team's own

@@ -1,0 +1,310 @@
+// FP8 products without a per-group fold (per-tensor scales, E8M0 block scales) for gfx950: the kernel for shapes that
+// give every CU a tile of its own. Same operand layout, MFMA orientation and stage format as gemm_fast_kernel.hpp.
+//
+// Eight waves (two per SIMD) own one tile. Their memory work and their math alternate in phases a barrier apart, the two
+// halves of the block half a turn out of step: while waves 0-3 run the MFMAs of chunk c (at raised priority), waves 4-7 read
+// their operands of chunk c from LDS into registers and issue the global -> LDS loads of chunk c + STAGES - 1, then they swap.
+// So each SIMD always has one wave in either role, the LDS port serves four waves at a time instead of eight in a burst, and
+// one operand register set per wave is enough (the 128 x 128 kernel reads the next chunk's operands in a burst ahead of its
+// MFMAs, which then wait for that burst to issue).
+#pragma once
+#include "gemm_fast_kernel.hpp"
+
+namespace viola {
+
+// WM x WN waves of TM x TN sub-tiles of 32 x 32; STAGES chunks of 64 k in the ring
+template <int WM_, int WN_, int TM_, int TN_, int STAGES_>
+struct PingPongShape {
+    static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, STAGES = STAGES_;
+    static constexpr int ROWS = WM * TM * 32, COLS = WN * TN * 32;
+    static constexpr int A_BYTES = ROWS * FBK, B_BYTES = COLS * FBK, STAGE = A_BYTES + B_BYTES;
+    static constexpr int A_LOADS = ROWS / 128, B_LOADS = COLS / 128, LOADS = A_LOADS + B_LOADS;   // 512 threads x 16 bytes = 128 rows
+    static_assert(WM * WN == 8 && ROWS % 128 == 0 && COLS % 128 == 0);
+};
+
+// GATED: the tile's b rows are COLS / 2 gate rows, then the up rows of the same columns of h (sub-tiles 0 and 1 of a wave);
+// out = act(g) * u, [g | u] itself is not kept.
+template <bool A_BF8, bool B_BF8, bool MX, typename S, int WAVES_PER_SIMD, bool GATED = false>
+__global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p, int bias_dtype, int out_dtype) {
+    constexpr int TM = S::TM, TN = S::TN, STAGES = S::STAGES;
+    static_assert(!GATED || TN == 2, "a gate and an up sub-tile per wave");
+    constexpr int PANEL = GATED ? S::COLS / 2 : S::COLS;                     // columns of the output per tile
+    constexpr int RING = STAGES * S::STAGE;
+    constexpr int SCALE_BLOCK = (S::ROWS + S::COLS) * MX_GROUPS;             // scale bytes of 16 K groups, a rows then b rows
+    constexpr int TAIL = MX ? 2 * SCALE_BLOCK : S::COLS * 4;                 // behind the ring: scale blocks, later the bias row
+    static_assert(TAIL >= S::COLS * 4);
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[RING + TAIL];
+    const int tid = threadIdx.x, lane = tid % WAVE, l32 = lane % 32, lhi = lane / 32;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int wm = wave / S::WN, wn = wave % S::WN;
+
+    // ---- tile: contiguous ranges per XCD, walked in groups of 8 m tiles (see group_gemm_fast)
+    const int per_xcd = gridDim.x / 8;
+    const int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (t >= p.tiles_m * p.tiles_n) return;
+    const int group = 8 * p.tiles_n, first_m = t / group * 8;
+    const int rows_here = p.tiles_m - first_m < 8 ? p.tiles_m - first_m : 8;
+    const int64_t m_begin = (int64_t)(first_m + t % group % rows_here) * S::ROWS, n_begin = (int64_t)(t % group / rows_here) * PANEL;
+
+    // ---- load plan: instruction `it` brings rows 128 it .. of an operand, unit U = 4 row + slot holds piece slot ^ ((row >> 2) & 3)
+    const i32x4 res_a = raw_resource(p.a + m_begin * p.lda), res_b = raw_resource(p.b);
+    constexpr uint32_t OUTSIDE = 0x80000000u;
+    const int chunks = (int)((p.k + FBK - 1) / FBK), full_chunks = (int)(p.k / FBK), groups_total = (int)((p.k + 31) / 32);
+    const int piece = (tid & 3) ^ ((tid >> 4) & 3);
+    const bool inside_tail = (int64_t)full_chunks * FBK + piece * 16 < p.k;
+    auto row_in = [](int64_t row, int64_t rows) -> uint32_t { return (uint32_t)(row < rows ? row : rows - 1); };
+    auto b_row = [&](int r) -> uint32_t {                                    // tile-local b row -> row of b
+        if constexpr (GATED) return (uint32_t)(r / PANEL) * (uint32_t)p.n + row_in(n_begin + r % PANEL, p.n);
+        else return row_in(n_begin + r, p.n);
+    };
+    uint32_t cur[S::LOADS];
+#pragma unroll
+    for (int it = 0; it < S::LOADS; ++it) {
+        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * 128 + tid / 4;
+        if (it < S::A_LOADS) cur[it] = (uint32_t)(row_in(m_begin + r, p.m) - m_begin) * (uint32_t)p.lda + piece * 16;
+        else cur[it] = b_row(r) * (uint32_t)p.ldb + piece * 16;
+    }
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    auto issue = [&](int c, int stage) {
+        if (__builtin_expect(c >= full_chunks, 0)) {                         // the chunk that straddles the end of k, and those past it
+            asm volatile("; end of the k range");
+            const bool here = c == full_chunks && inside_tail;
+#pragma unroll
+            for (int it = 0; it < S::LOADS; ++it) {
+                const uint32_t at = here ? cur[it] : OUTSIDE;
+                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, at, (uint32_t)c * FBK);
+            }
+            return;
+        }
+#pragma unroll
+        for (int it = 0; it < S::LOADS; ++it)
+            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * FBK);
+    };
+    // E8M0 scales: one 16-byte piece (16 K groups) per tile row, block `b` in buffer b & 1
+    const i32x4 res_sa = raw_resource(p.sa, p.sa_bytes), res_sb = raw_resource(p.sb, p.sb_bytes);
+    uint32_t scale_at = 0;
+    if constexpr (MX) {
+        scale_at = tid < S::ROWS ? row_in(m_begin + tid, p.m) / (uint32_t)p.ar * (uint32_t)p.ldsa : b_row(tid - S::ROWS) / (uint32_t)p.br * (uint32_t)p.ldsb;
+    }
+    auto issue_scales = [&](int block) {
+        if (wave * 64 >= S::ROWS + S::COLS) return;
+        const uint32_t to = lds_base + RING + (uint32_t)(block & 1) * SCALE_BLOCK + (uint32_t)wave * 1024;
+        load16_to_lds(wave * 64 < S::ROWS ? res_sa : res_sb, to, block * MX_GROUPS < groups_total ? scale_at : OUTSIDE, (uint32_t)(block * MX_GROUPS));
+    };
+
+    // ---- operand reads
+    const int sw = (l32 >> 2) & 3;
+    const int rd_a = (wm * TM * 32 + l32) * FBK + ((lhi ^ sw) * 16), rd_b = S::A_BYTES + ((GATED ? wn : wn * TN) * 32 + l32) * FBK + ((lhi ^ sw) * 16);
+    constexpr int NEXT_B = GATED ? PANEL : 32;                               // b rows from one sub-tile of a wave to the next
+    f32x16 total[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) total[i][j][r] = 0.0f;
+    i32x8 oa[TM], ob[TN];
+    // scale words of the chunk pair at hand: byte 0 = this lane's K group of the even chunk, byte 2 = of the odd chunk
+    uint32_t wa[TM], wb[TN];
+#pragma unroll
+    for (int j = 0; j < TM; ++j) wa[j] = 0;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) wb[i] = 0;
+    auto read = [&](int stage, int c) {
+        const uint8_t* base = lds + stage * S::STAGE;
+        auto operand = [&](int offset) -> i32x8 {
+            const i32x4 lo = *reinterpret_cast<const i32x4*>(base + offset), hi = *reinterpret_cast<const i32x4*>(base + (offset ^ 32));
+            return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+#pragma unroll
+        for (int i = 0; i < TN; ++i) ob[i] = operand(rd_b + i * NEXT_B * FBK);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) oa[j] = operand(rd_a + j * 32 * FBK);
+        if constexpr (MX) {
+            if ((c & 1) == 0) {
+                const uint8_t* block = lds + RING + ((c / MX_CHUNKS) & 1) * SCALE_BLOCK + (c % MX_CHUNKS) * FKG;
+#pragma unroll
+                for (int j = 0; j < TM; ++j) wa[j] = *reinterpret_cast<const uint32_t*>(block + (wm * TM * 32 + j * 32 + l32) * MX_GROUPS) >> (8 * lhi);
+#pragma unroll
+                for (int i = 0; i < TN; ++i) wb[i] = *reinterpret_cast<const uint32_t*>(block + (S::ROWS + (GATED ? wn : wn * TN) * 32 + i * NEXT_B + l32) * MX_GROUPS) >> (8 * lhi);
+            }
+        }
+    };
+    auto math = [&](auto odd) {
+        constexpr int FB = B_BF8 ? 1 : 0, FA = A_BF8 ? 1 : 0, BYTE = MX && decltype(odd)::value ? 2 : 0;
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+                total[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ob[i], oa[j], total[i][j], FB, FA, BYTE, MX ? (int)wb[i] : 0, BYTE, MX ? (int)wa[j] : 0);
+        // (the compiler sinks MFMAs into the following read phase otherwise: intrinsics without side effects cross a barrier)
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(total[i][j]));
+        __builtin_amdgcn_s_setprio(0);
+    };
+    auto pin_operands = [&] {                                                // in registers before the barrier, scale bytes in place
+#pragma unroll
+        for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(oa[j]), "+v"(wa[j]));
+#pragma unroll
+        for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(ob[i]), "+v"(wb[i]));
+    };
+    auto barrier = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // Phases. Waves 0-3 read chunk c in phase 2c and multiply in phase 2c + 1, waves 4-7 one phase later. The loads of chunk
+    // c + STAGES - 1 go out in the read phase of chunk c, into the stage of chunk c - 1: its last readers (waves 4-7, phase
+    // 2c - 1) had their operands in registers before the barrier that ended that phase. Every wave ends its read phase of
+    // chunk c with its own loads of chunk c + 1 landed (at most those of the STAGES - 2 chunks after it in flight; a scale
+    // block among them only makes the wait stricter), and chunk c + 1 is first read two barriers later.
+    constexpr int AHEAD = (STAGES - 2) * S::LOADS;
+    static_assert((STAGES - 1) * S::LOADS < 16 && STAGES >= 3);
+    if constexpr (MX) issue_scales(0);
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);                              // chunk 0 and scale block 0
+    barrier();
+    const bool late = wave >= 4;
+    if (late) barrier();
+    int stage = 0, fill = STAGES - 1;
+    auto step = [&](int c, auto odd) {
+        read(stage, c);
+        if constexpr (MX) {
+            if (c % MX_CHUNKS == 0) issue_scales(c / MX_CHUNKS + 1);
+        }
+        issue(c + STAGES - 1, fill);
+        stage = stage == STAGES - 1 ? 0 : stage + 1;
+        fill = fill == STAGES - 1 ? 0 : fill + 1;
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
+        pin_operands();
+        barrier();
+        math(odd);
+        barrier();
+    };
+    int c = 0;
+    for (; c + 1 < chunks; c += 2) {
+        step(c, std::false_type{});
+        step(c + 1, std::true_type{});
+    }
+    if (c < chunks) step(c, std::false_type{});
+    if (!late) barrier();
+    __builtin_amdgcn_s_waitcnt(0x0F70);                                      // the trailing loads must not land in what follows
+
+    // ---- epilogue
+    if constexpr (!MX) {
+        const float sa = p.sa[0], sb = p.sb[0];
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { const float v = total[i][j][r] * sa; total[i][j][r] = v * sb; }
+    }
+    barrier();                                                               // every wave has left the ring
+    float* bias_lds = reinterpret_cast<float*>(lds + RING);
+    if (p.bias) {
+        if (tid < S::COLS) {
+            const int64_t col = n_begin + tid % PANEL;
+            bias_lds[tid] = col < p.n ? load_bias(p.bias, (GATED ? tid / PANEL * p.n : 0) + col, bias_dtype) : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 bq = *reinterpret_cast<const float4*>(&bias_lds[(GATED ? wn : wn * TN) * 32 + i * NEXT_B + q * 8 + lhi * 4]);
+#pragma unroll
+                for (int j = 0; j < TM; ++j) {
+                    total[i][j][4 * q] += bq.x; total[i][j][4 * q + 1] += bq.y; total[i][j][4 * q + 2] += bq.z; total[i][j][4 * q + 3] += bq.w;
+                }
+            }
+    }
+    // (one kernel for the three output types: they differ from here on only)
+    auto finish = [&](auto type) {
+        using TO = decltype(type);
+        TO* out = static_cast<TO*>(p.out);
+        if constexpr (GATED) {
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float act, derivative, h;
+                    gate_math(p.activation, rounded<TO>(total[0][j][r]), act, derivative);
+                    h = act * rounded<TO>(total[TN - 1][j][r]);
+                    asm volatile("" : "+v"(h));                                 // an FP32 value of its own (see group_gemm_fast)
+                    total[0][j][r] = h;
+                }
+        }
+        const bool pieces_out = (p.ldo * sizeof(TO)) % 16 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+        // a wave parks 32 rows at a time in its own part of the ring and stores them as 16-byte pieces along the rows
+        constexpr int SUBS = GATED ? 1 : TN, PER = 16 / (int)sizeof(TO), COLS_W = 32 * SUBS, PLD = COLS_W + PER, PIECES = COLS_W / PER;
+        static_assert(8 * 32 * PLD * (int)sizeof(TO) <= RING);
+        TO* park = reinterpret_cast<TO*>(lds) + wave * 32 * PLD;
+        const int64_t ncol0 = n_begin + wn * COLS_W;
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+            const int64_t row0 = m_begin + (wm * TM + j) * 32;
+#pragma unroll
+            for (int i = 0; i < SUBS; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float v[4] = {total[i][j][4 * q], total[i][j][4 * q + 1], total[i][j][4 * q + 2], total[i][j][4 * q + 3]};
+                    Quad<TO>::store(&park[l32 * PLD + i * 32 + q * 8 + lhi * 4], v);
+                }
+#pragma unroll
+            for (int it = 0; it < 32 * PIECES / WAVE; ++it) {
+                const int id = it * WAVE + lane, pr = id / PIECES, pc = id % PIECES;
+                const int64_t mrow = row0 + pr, ncol = ncol0 + pc * PER;
+                const uint4 value = *reinterpret_cast<const uint4*>(&park[pr * PLD + pc * PER]);
+                if (mrow >= p.m || ncol >= p.n) continue;
+                if (pieces_out && ncol + PER <= p.n) {
+                    store_streaming(out + mrow * p.ldo + ncol, value);
+                } else {
+                    const TO* values = reinterpret_cast<const TO*>(&value);
+                    for (int e = 0; e < PER; ++e)
+                        if (ncol + e < p.n) out[mrow * p.ldo + ncol + e] = values[e];
+                }
+            }
+        }
+    };
+    if (out_dtype == VIOLA_F32) finish(float{});
+    else if (out_dtype == VIOLA_BF16) finish(bf16_t{});
+    else finish(f16_t{});
+}
+
+// The three tiles: 256 x 256 and 256 x 128 with one block per CU, 128 x 128 with two.
+using PingPongL = PingPongShape<2, 4, 4, 2, 4>;
+using PingPongM = PingPongShape<4, 2, 2, 2, 4>;
+using PingPongS = PingPongShape<2, 4, 2, 1, 4>;
+
+template <bool MX, typename S, int WAVES_PER_SIMD, bool GATED = false>
+static int launch_pingpong(const GemmArgs& args, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+    GemmArgs p = args;
+    constexpr int PANEL = GATED ? S::COLS / 2 : S::COLS;
+    p.tiles_m = (int)((p.m + S::ROWS - 1) / S::ROWS);
+    p.tiles_n = (int)((p.n + PANEL - 1) / PANEL);
+    if (!viola_is_float(out_dtype)) return VIOLA_EINVAL;
+    const bool a5 = a_dtype == VIOLA_E5M2, b5 = b_dtype == VIOLA_E5M2;
+    const dim3 grid((unsigned)(((int64_t)p.tiles_m * p.tiles_n + 7) / 8 * 8)), block(512);
+    if (!a5 && !b5) VIOLA_LAUNCH((gemm_pingpong<false, false, MX, S, WAVES_PER_SIMD, GATED>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else if (a5 && !b5) VIOLA_LAUNCH((gemm_pingpong<true, false, MX, S, WAVES_PER_SIMD, GATED>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else if (!a5 && b5) VIOLA_LAUNCH((gemm_pingpong<false, true, MX, S, WAVES_PER_SIMD, GATED>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else VIOLA_LAUNCH((gemm_pingpong<true, true, MX, S, WAVES_PER_SIMD, GATED>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    return viola_launch_status();
+}
+
+template <bool MX>
+static int launch_pingpong_tile(const GemmArgs& p, ScaledTile tile, bool gated, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+    if (gated) return launch_pingpong<MX, PingPongL, 2, true>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    if (tile == SCALED_TILE_L) return launch_pingpong<MX, PingPongL, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    if (tile == SCALED_TILE_M) return launch_pingpong<MX, PingPongM, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    return launch_pingpong<MX, PingPongS, 4>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+}
+
+}  // namespace viola

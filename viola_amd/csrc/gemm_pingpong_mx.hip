@@ -1,0 +1,12 @@
+// E8M0 block-scale (MXFP8) instances of the large-tile FP8 GEMM kernel.
+#include <type_traits>
+
+#include "gemm_pingpong.hpp"
+
+namespace viola {
+
+int launch_mx_pingpong(const GemmArgs& p, ScaledTile tile, bool gated, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+    return launch_pingpong_tile<true>(p, tile, gated, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+}
+
+}  // namespace viola
