@@ -356,3 +356,19 @@ def test_large_tile_gated_forward_without_aux_equals_the_kept_form(m, h, k, scal
         sa, sb = torch.full((1,), .1, device="cuda"), torch.full((1,), .1, device="cuda")
     call = lambda save: mk.gemm(a, b, sa, sb, layer=layer, out_dtype=torch.bfloat16, activation="gelu", bias=bias, save=save)[0]
     assert torch.equal(call(True), call(False))
+
+
+@pytest.mark.parametrize("gb", [(32, 32), (1, 32)])
+@pytest.mark.parametrize("m,n,k", [(1024, 2048, 1024), (1025, 2048, 1536), (2048, 2048, 1520), (2048, 2040, 1536), (2049, 2048, 1536), (2049, 2047, 96), (4100, 2000, 2080)])
+def test_group_gemm_around_the_tile_counts_where_the_form_changes(m, n, k, gb):
+    """128, 129 .. 256 and 257 up tiles of 128 x 128, short and long k: narrow and split, narrow, split, whole tiles. Integer
+    operands and power-of-two scales, so every element must equal the integer product."""
+    from viola_amd.nn import _grouped_kernels as g
+    torch.manual_seed(m + n + k)
+    a, b = torch.randint(-2, 3, (m, k), device="cuda").float(), torch.randint(-2, 3, (n, k), device="cuda").float()
+    groups = -(-k // 32)
+    sa = torch.exp2(torch.randint(-1, 2, (m, groups), device="cuda").float())
+    sb = torch.exp2(torch.randint(-1, 2, (-(-n // gb[0]), groups), device="cuda").float())
+    spell = lambda t, s, rows: t * s.repeat_interleave(rows, 0)[:t.shape[0]].repeat_interleave(32, 1)[:, :k]
+    out = g.gemm(a.to(E4), b.to(E4), sa, sb, (1, 32), gb, out_dtype=torch.float32)
+    assert torch.equal(out, spell(a, sa, 1) @ spell(b, sb, gb[0]).T)

@@ -38,6 +38,12 @@ struct GemmArgs {
 };
 
 
+// Any alignment and size; the FP16-accumulator model (per_tensor: scales applied to the finished total). gemm_generic.hip.
+int launch_group_gemm_generic(const GemmArgs& p, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, dim3 grid,
+                              hipStream_t stream);
+int launch_group_gemm_half(const GemmArgs& p, bool per_tensor, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, dim3 grid,
+                           hipStream_t stream);
+
 // Fast path (16-byte aligned operands, k ranges multiples of 16). Defined in gemm_fast.hip.
 int launch_group_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype,
                            bool rowscale, dim3 grid, hipStream_t stream);

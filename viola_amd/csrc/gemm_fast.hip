@@ -58,13 +58,15 @@ int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dt
     const int64_t b_rows = mode == MODE_GATED_FWD ? 2 * p.n : p.n;
     p.sa_bytes = (p.m + p.ar - 1) / p.ar * p.ldsa * 4;
     p.sb_bytes = (b_rows + p.br - 1) / p.br * p.ldsb * 4;
-    // Two blocks fit a CU: with fewer than 512 tiles of 128 x 128, halve the tile in n so that all 256 CUs get two.
-    // Over a long k, and with enough tiles to give half the CUs one each, keep the tile instead and split its k range inside
-    // the block (one block of twice the waves per CU): 7-12 % faster from 256 tiles up at k >= 2048. With 128 tiles or fewer the
-    // narrow tiles stay (more CUs busy) and their k range is split: a CU then holds eight waves instead of four
-    // (1024 x 1024 x 16384: 98 -> 76 us, 512 x 512 x 4096: 27.5 -> 22.3 us).
+    // Two blocks of 128 x 128 fit a CU, so from 257 tiles up every CU has work and the full tile, which reads the least, is
+    // the fastest form (4096 x 1152 x 4608: 75.6 -> 59.7 us against the split one, 6000 x 1000 x 1024: 27.0 -> 19.6 us against
+    // tiles halved in n). From 129 to 256 tiles a CU gets one: over a long k keep the tile and split its k range over twice the
+    // waves inside the block (7-12 % faster at 256 tiles, k >= 2048), else halve the tile in n for a second block per CU. With
+    // 128 tiles or fewer the narrow tiles keep more CUs busy and their k range is split: a CU then holds eight waves instead of
+    // four (1024 x 1024 x 16384: 98 -> 76 us, 512 x 512 x 4096: 27.5 -> 22.3 us). Narrow split tiles are one per CU: past 256 of
+    // them the second round costs more than the split gives (600 x 4096 x 1024: 17.2 us, unsplit 12.5 us).
     const int64_t tiles = (int64_t)grid.x * grid.y * grid.z;
-    const bool few = mode == MODE_PLAIN && tiles < 512;
+    const bool few = mode == MODE_PLAIN && tiles <= 256;
     const bool fixed_k = !p.offsets && !p.koffsets;
     const bool split = few && tiles > 128 && fixed_k && p.k >= SPLIT_MIN_K;
     const bool narrow = few && !split && p.n > 64;
@@ -75,7 +77,7 @@ int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dt
         grid = dim3((grid.x * grid.y + 7) / 8 * 8, 1, grid.z);
     }
     if (split) return launch_split<2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
-    if (narrow && fixed_k && p.k >= NARROW_SPLIT_MIN_K) return launch_split<1>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
+    if (narrow && tiles <= 128 && fixed_k && p.k >= NARROW_SPLIT_MIN_K) return launch_split<1>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
     if (narrow) return launch_mode<MODE_PLAIN, 1>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
     if (mode == MODE_PLAIN) return launch_mode<MODE_PLAIN, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
     if (mode == MODE_GATED_FWD) return launch_mode<MODE_GATED_FWD, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
