@@ -83,6 +83,16 @@ int viola_codes_repack(const void* x, void* out, int64_t batch, int64_t rows, in
 int viola_gated_quantize_dual(const void* z, int z_dtype, int64_t rows, int64_t cols, int activation,
                               void* q, void* scale, void* qt, void* scale_t, int q_dtype, int gc,
                               float limit, int scale_format, viola_stream_t stream);
+/* The same with the rows of q and qt q_pitch and qt_pitch codes apart, zero codes past the matrix, either layout absent (null). */
+int viola_gated_quantize_dual_pitched(const void* z, int z_dtype, int64_t rows, int64_t cols, int activation, void* q, int64_t q_pitch,
+                                      void* scale, void* qt, int64_t qt_pitch, void* scale_t, int q_dtype, float limit, int scale_format,
+                                      viola_stream_t stream);
+/* viola_gated_backward followed by viola_group_quantize_dual_pitched of its dz [rows, 2 h] (q: row pitch 2 h), without dz: z and
+ * dh [rows, h] are read, codes, scales and (column_partial != null, [ceil(rows / 32), 2 h]) column sums written. Bit for bit the
+ * two calls. bf16 / fp16, h a multiple of 64, 16-byte aligned z and dh; VIOLA_EUNSUPPORTED otherwise. */
+int viola_gated_backward_quantize_dual(const void* z, const void* dh, int dtype, int64_t rows, int64_t h, int activation, void* q, void* scale,
+                                       void* qt, int64_t qt_pitch, void* scale_t, int q_dtype, float limit, float* column_partial,
+                                       int scale_format, viola_stream_t stream);
 
 /* column_partial (nullable) of viola_group_quantize_dual receives [ceil(rows/32), cols] fp32 sums of x over
  * each 32-row group, taken from the same read; viola_column_reduce adds the parts in a fixed order:

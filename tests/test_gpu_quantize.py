@@ -267,3 +267,36 @@ def test_gated_quantize_dual_equals_activation_then_quantize(dtype, activation, 
                 assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     assert g.gated_quantize_dual(torch.zeros(4, 2 * 12, device="cuda", dtype=dtype), activation, torch.float8_e4m3fn) is None
     assert g.gated_quantize_dual(torch.zeros(4, 64, device="cuda"), activation, torch.float8_e4m3fn) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("activation", ["silu", "gelu", "relu"])
+@pytest.mark.parametrize("rows,h,native", [(64, 64, False), (1, 128, True), (130, 192, False), (256, 64, True)])
+def test_gated_gradient_quantizer_equals_gradient_then_quantize(rows, h, native, activation, dtype):
+    """Codes, scales and column sums of dz straight from [g | u] and dh are the stored dz's, bit for bit, in padded rows of the
+    transposed codes too; one layout alone as well."""
+    from viola_amd import _lib
+    torch.manual_seed(rows + h)
+    z = torch.randn(rows, 2 * h, device="cuda").mul(3).to(dtype)
+    dh = torch.randn(rows, h, device="cuda").to(dtype)
+    if rows > 60:
+        z[5, 3], dh[40, 7] = float("inf"), float("nan")
+    pitch, parts, width = -(-rows // 128) * 128, -(-rows // 32), 1 if native else 4
+    def outputs():
+        return [torch.full(shape, 77, device="cuda", dtype=torch.uint8) for shape in
+                ((rows, 2 * h), (rows, 2 * h // 32 * width), (2 * h, pitch), (2 * h, pitch // 32 * width), (parts, 2 * h * 4))]
+    dz = torch.empty(rows, 2 * h, device="cuda", dtype=dtype)
+    _lib.call("viola_gated_backward", z.data_ptr(), dh.data_ptr(), dz.data_ptr(), rows, h, _lib.code(dtype), _lib.ACTIVATION[activation])
+    want, got, alone = outputs(), outputs(), outputs()
+    p = [t.data_ptr() for t in want]
+    _lib.call("viola_group_quantize_dual_pitched", dz.data_ptr(), _lib.code(dtype), rows, 2 * h, p[0], 2 * h, p[1], p[2], pitch, p[3],
+              _lib.code(torch.float8_e4m3fn), 448., p[4], int(native))
+    source = (z.data_ptr(), dh.data_ptr(), _lib.code(dtype), rows, h, _lib.ACTIVATION[activation])
+    p = [t.data_ptr() for t in got]
+    _lib.call("viola_gated_backward_quantize_dual", *source, p[0], p[1], p[2], pitch, p[3], _lib.code(torch.float8_e4m3fn), 448., p[4], int(native))
+    for a, b in zip(got[:4], want[:4]):
+        assert torch.equal(a, b)
+    assert torch.equal(got[4].view(torch.float32).nan_to_num(), want[4].view(torch.float32).nan_to_num())
+    p = [t.data_ptr() for t in alone]
+    _lib.call("viola_gated_backward_quantize_dual", *source, p[0], p[1], None, rows, None, _lib.code(torch.float8_e4m3fn), 448., None, int(native))
+    assert torch.equal(alone[0], want[0]) and torch.equal(alone[1], want[1]) and (alone[2] == 77).all()

@@ -199,9 +199,14 @@ template <> __device__ __forceinline__ uint32_t hw_encode4<e5m2_t>(float a, floa
     int w = __builtin_amdgcn_cvt_pk_bf8_f32(a, b, 0, false);
     return (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(c, d, w, true);
 }
+// The quotients by an E8M0 scale: its reciprocal is a power of two as well, so one product is exact.
+struct PowerDivisor {
+    float r;
+    __device__ __forceinline__ float quotient(float v) const { return v * r; }
+};
 // clamp(v / s, +-limit) -> code, four at a time, for a group whose divisor took the fast path
-template <typename T>
-__device__ __forceinline__ uint32_t fast_encode4(const SharedDivisor& d, float limit, float a, float b, float c, float e) {
+template <typename T, typename D>
+__device__ __forceinline__ uint32_t fast_encode4(const D& d, float limit, float a, float b, float c, float e) {
     return hw_encode4<T>(__builtin_amdgcn_fmed3f(d.quotient(a), -limit, limit), __builtin_amdgcn_fmed3f(d.quotient(b), -limit, limit),
                          __builtin_amdgcn_fmed3f(d.quotient(c), -limit, limit), __builtin_amdgcn_fmed3f(d.quotient(e), -limit, limit));
 }
@@ -209,8 +214,8 @@ __device__ __forceinline__ uint32_t fast_encode4(const SharedDivisor& d, float l
 // The same without the clamp, for groups whose scale is max |v| / limit with limit the format's largest finite value:
 // a quotient is then at most limit in all but its last place, and everything below the first value that rounds past
 // the largest code (464 for e4m3, 61440 for e5m2) converts to that code, which is what the clamp would give.
-template <typename T>
-__device__ __forceinline__ uint32_t fast_encode4_unclamped(const SharedDivisor& d, float a, float b, float c, float e) {
+template <typename T, typename D>
+__device__ __forceinline__ uint32_t fast_encode4_unclamped(const D& d, float a, float b, float c, float e) {
     return hw_encode4<T>(d.quotient(a), d.quotient(b), d.quotient(c), d.quotient(e));
 }
 
@@ -330,18 +335,31 @@ __device__ __forceinline__ T round_store(float v, uint64_t element, uint64_t ste
     return from_f32<T>(v);
 }
 
+// 1 / (1 + exp(-x)) within 2 ulp, in a third of the instructions of the library's exp and division: exp2 of the product's two
+// halves (the low one multiplied in afterwards), one Newton step on the hardware reciprocal. Past +-150 it is 1 or 0 exactly.
+__device__ __forceinline__ float sigmoid(float x) {
+    const float c = __builtin_amdgcn_fmed3f(-x, -150.0f, 150.0f);
+    const float t = c * 1.44269502f;                                         // log2(e) = 1.44269502 + 1.92596e-8
+    const float low = fmaf(c, 1.92596299e-8f, fmaf(c, 1.44269502f, -t));
+    const float d = fmaf(__builtin_amdgcn_exp2f(t), fmaf(low, 0.693147182f, 1.0f), 1.0f);
+    const float r = __builtin_amdgcn_rcpf(d);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, r, 1.0f), r, r), d, 1.0f);   // 0 for an infinite d
+}
+
 // act(g) and act'(g) of a gated MLP as the gated GEMM epilogues write them (viola/nn/_mlp_kernels.py:158-194), shared by
 // the epilogues and by the passes that stand in for them, so both give the same bits. (The stand-alone forward operator
-// writes silu as g / (1 + exp(-g)), viola/nn/_gated_kernels.py:29-35, which differs in the last place.)
+// writes silu as g / (1 + exp(-g)), viola/nn/_gated_kernels.py:29-35, which differs in the last place.) gelu's
+// (1 + tanh(y)) / 2 is sigmoid(2 y): no cancellation where tanh is near -1.
 __device__ __forceinline__ void gate_math(int activation, float g, float& act, float& derivative) {
     if (activation == VIOLA_SILU) {
-        const float s = 1.0f / (1.0f + expf(-g));
+        const float s = sigmoid(g);
         act = g * s;
-        derivative = s * (1.0f + g * (1.0f - s));
+        derivative = fmaf(act, 1.0f - s, s);
     } else if (activation == VIOLA_GELU) {
-        const float t = tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g));
-        act = 0.5f * g * (1.0f + t);
-        derivative = 0.5f * (1.0f + t) + 0.5f * g * (1.0f - t * t) * 0.7978845608028654f * (1.0f + 0.134145f * g * g);
+        const float g2 = g * g;                                              // 2 y = g (c + 0.044715 c g^2), c = 2 sqrt(2 / pi)
+        const float s = sigmoid(g * fmaf(g2, 0.0713548162726f, 1.5957691216057308f));
+        act = g * s;
+        derivative = fmaf(act * (1.0f - s), fmaf(g2, 0.2140644488178f, 1.5957691216057308f), s);
     } else {
         act = fmaxf(g, 0.0f);
         derivative = g > 0.0f ? 1.0f : 0.0f;

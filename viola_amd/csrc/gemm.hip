@@ -98,15 +98,18 @@ extern "C" int viola_tensor_gemm_half(const void* a, int a_dtype, const void* b,
     return launch_group_gemm_half(p, true, a_dtype, b_dtype, bias_dtype, out_dtype, false, dim3((unsigned)gx, (unsigned)gy), stream);
 }
 
-// Large gated products run as the plain GEMM on large tiles plus one elementwise pass over its output: with one block per CU
-// nothing covers a block's gated epilogue, and the pass costs less than that (MLP step at 16384 x 4096 -> 11008: 7.55 ms
-// against 7.90 ms under per-tensor scales, 8.41 ms against 9.06 ms under MXFP8). No extra memory: forward the plain product is
-// the [g | u] the caller keeps anyway, backward it lands in the up half of dz and is replaced there.
-static bool gated_in_two_passes(int64_t m, int64_t n_plain, int64_t k, int64_t h, const void* aux, const void* out, int out_dtype) {
+// Large gated products run as the plain GEMM on the tile that suits it plus one elementwise pass over its output: with one block
+// per CU nothing covers a block's gated epilogue, and the pass costs less than that (MLP step at 16384 x 4096 -> 11008: 7.55 ms
+// against 7.90 ms under per-tensor scales, 8.41 ms against 9.06 ms under MXFP8). Backward the epilogue also reads [g | u] in
+// place, so the pass wins on every tile (4096 x 4608 x 1152 106 -> 78 us, 1024 x 1024 x 1024 19.2 -> 10.3 us) down to where a
+// second launch is what counts. No extra memory: forward the plain product is the [g | u] the caller keeps anyway, backward it
+// lands in the up half of dz and is replaced there.
+static bool gated_in_two_passes(int64_t m, int64_t k, int64_t h, const void* aux, const void* out, int out_dtype, bool backward) {
     const int64_t piece = out_dtype == VIOLA_F32 ? 4 : 8;
-    const ScaledTile tile = choose_scaled_tile(m, n_plain, k);
-    return aux && (tile == SCALED_TILE_L || tile == SCALED_TILE_M) && h % piece == 0 && aligned16(aux) && aligned16(out) &&
-           m * (h / piece) / 256 < 0x7fffffff;                               // the pass is one launch of 256-thread blocks
+    if (!aux || h % piece != 0 || !aligned16(aux) || !aligned16(out) || m * (h / piece) / 256 >= 0x7fffffff) return false;   // the pass is one launch of 256-thread blocks
+    if (backward) return m * h >= (1 << 17);
+    const ScaledTile tile = choose_scaled_tile(m, 2 * h, k);
+    return tile == SCALED_TILE_L || tile == SCALED_TILE_M;
 }
 
 static int tensor_gemm(const void* a, int a_dtype, const void* b, int b_dtype, const float* sa, const float* sb, int64_t m,
@@ -205,7 +208,7 @@ extern "C" int viola_tensor_gated_gemm(const void* a, int a_dtype, const void* b
     const dim3 grid((unsigned)((h + width - 1) / width), (unsigned)gy);
     const bool vec = k % 16 == 0 && k > 0 && aligned16(a) && aligned16(b);
     if (vec && 2 * h * k < (1ll << 31) && (int64_t)BM * k < (1ll << 31)) {
-        if (gated_in_two_passes(m, backward ? h : 2 * h, k, h, aux, out, out_dtype)) {
+        if (gated_in_two_passes(m, k, h, aux, out, out_dtype, backward)) {
             auto plain = [&](int64_t n, const void* n_bias, void* to, int64_t ldo) {
                 return tensor_gemm(a, a_dtype, b, b_dtype, sa, sb, m, n, k, n_bias, bias_dtype, to, ldo, out_dtype, stream);
             };
@@ -234,7 +237,7 @@ extern "C" int viola_mx_gated_gemm(const void* a, int a_dtype, const void* b, in
         reinterpret_cast<uintptr_t>(sb) % 4 != 0 || 2 * h * k >= (1ll << 31) || (int64_t)BM * k >= (1ll << 31) ||
         (br != 1 && br % 32 != 0) || (!backward && h % br != 0))
         return VIOLA_EUNSUPPORTED;
-    if (gated_in_two_passes(m, backward ? h : 2 * h, k, h, aux, out, out_dtype)) {
+    if (gated_in_two_passes(m, k, h, aux, out, out_dtype, backward)) {
         auto plain = [&](int64_t n, const void* n_bias, void* to, int64_t ldo) {
             return mx_gemm(a, a_dtype, b, b_dtype, sa, sb, m, n, k, ar, br, n_bias, bias_dtype, to, ldo, out_dtype, stream);
         };
@@ -298,10 +301,9 @@ extern "C" int viola_mx_gated_gemm_encode(const void* a, int a_dtype, const void
         (br != 1 && br % 32 != 0) || h % br != 0 || h % 32 != 0 || m % 32 != 0 || !aligned16(aux) || !aligned16(enc) ||
         !aligned16(enc_t))
         return VIOLA_EUNSUPPORTED;
-    if (aux && enc_t && aux_dtype != VIOLA_F32 && choose_scaled_tile(m, 2 * h, k) == SCALED_TILE_L && 128 * h < (1ll << 31)) {
-        // large products: the plain GEMM on 256 x 256 tiles writes [g | u], one pass over it writes the codes of h
-        // in both layouts (the encoding epilogue does not fit the large tile's registers; 2.0 ms against 2.5 ms at
-        // 16384 x 4096 -> 11008)
+    if (aux && enc_t && aux_dtype != VIOLA_F32 && choose_scaled_tile(m, 2 * h, k) != SCALED_TILE_FAST) {
+        // the plain GEMM on the tile that suits it writes [g | u], one pass over it writes the codes of h in both layouts
+        // (the encoding epilogue does not fit the large tiles' registers; 2.0 ms against 2.5 ms at 16384 x 4096 -> 11008)
         const int status = mx_gemm(a, a_dtype, b, b_dtype, sa, sb, m, 2 * h, k, ar, br, bias, bias_dtype, aux, 2 * h, aux_dtype, stream);
         if (status) return status;
         return viola_gated_quantize_dual(aux, aux_dtype, m, h, activation, enc, enc_scale, enc_t, enc_t_scale, enc_dtype, 32, limit,

@@ -38,21 +38,6 @@ __device__ __forceinline__ float load_dtype(const void* p, int64_t i, int dtype)
     return (float)static_cast<const _Float16*>(p)[i];
 }
 
-__device__ __forceinline__ void activation_pair(int activation, float g, float& act, float& derivative) {
-    if (activation == VIOLA_SILU) {
-        const float s = 1.0f / (1.0f + expf(-g));
-        act = g * s;
-        derivative = s * (1.0f + g * (1.0f - s));
-    } else if (activation == VIOLA_GELU) {
-        const float t = tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g));
-        act = 0.5f * g * (1.0f + t);
-        derivative = 0.5f * (1.0f + t) + 0.5f * g * (1.0f - t * t) * 0.7978845608028654f * (1.0f + 0.134145f * g * g);
-    } else {
-        act = fmaxf(g, 0.0f);
-        derivative = g > 0.0f ? 1.0f : 0.0f;
-    }
-}
-
 template <typename TO> __device__ __forceinline__ float round_through(float v) { return to_f32(from_f32<TO>(v)); }
 
 // A_BF8/B_BF8: operand formats (false = e4m3, true = e5m2). B_ROWSCALE: b scales vary inside a 32-row block.
@@ -310,7 +295,7 @@ __global__ __launch_bounds__(256, 2) void group_gemm_kernel(GemmArgs p, int bias
                     aux[mrow * 2 * p.n + p.n + ncol] = uq;
                 }
                 float act, derivative;
-                activation_pair(p.activation, to_f32(gq), act, derivative);
+                gate_math(p.activation, to_f32(gq), act, derivative);
                 out[mrow * p.ldo + ncol] = from_f32<TO>(act * to_f32(uq));
             }
         } else {
@@ -334,7 +319,7 @@ __global__ __launch_bounds__(256, 2) void group_gemm_kernel(GemmArgs p, int bias
                         const float g = to_f32(aux[mrow * 2 * p.n + ncol]);
                         const float u = to_f32(aux[mrow * 2 * p.n + p.n + ncol]);
                         float act, derivative;
-                        activation_pair(p.activation, g, act, derivative);
+                        gate_math(p.activation, g, act, derivative);
                         out[mrow * p.ldo + ncol] = from_f32<TO>(d * u * derivative);
                         out[mrow * p.ldo + p.n + ncol] = from_f32<TO>(d * act);
                     }

@@ -246,8 +246,10 @@ Codes stored_weight(const Layer& l, const Tensor& weight, const WeightSpace& w, 
 
 // ---------------------------------------------------------------------------------------------------- one projection
 // gated < 0: y = x W^T + b. gated >= 0 (an activation): y = act(g) * u of [g | u] = x W^T + b, and *aux = [g | u] when kept.
-// hidden_codes: (gated, E8M0) hand y over as codes instead of values; input_codes: x arrives that way.
+// hidden_out: (gated, grouped recipes) hand y over as codes instead of values where a kernel does; coded_input: x arrives that way.
 struct CodedHidden {
+    const Recipe* reader = nullptr;                              // the down projection's
+    bool transposed = false;                                     // its weight gradient wants the other layout too
     Arena temp;                                                  // row-wise codes, used by this forward only
     Codes codes;
     Codes codes_t;                                               // in the down projection's Kept arena
@@ -258,7 +260,7 @@ struct Forward {
 };
 
 Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool need_backward, bool needs_w, Kept& kept, int gated, bool keep_aux,
-                CodedHidden* hidden_out, Kept* hidden_kept, bool hidden_transposed, const CodedHidden* coded_input) {
+                CodedHidden* hidden_out, Kept* hidden_kept, const CodedHidden* coded_input) {
     const Recipe& r = *l.recipe;
     const bool save = need_backward && needs_w;
     const int64_t rows = coded_input ? kept.rows : x2.size(0);
@@ -330,15 +332,34 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         return f;
     }
     if (keep_aux) f.aux = at::empty({rows, r.out}, options);
-    if (hidden_out) {
+    if (hidden_out && keep_aux && dtype != at::kFloat && h % 8 == 0) {
+        // [g | u] is kept for backward anyway: the plain product on the tile that suits it best, then one pass over [g | u] that
+        // makes h's codes; h itself is never stored
+        const Recipe& to = *hidden_out->reader;
+        GroupSpace space;
+        space.reserve(to, &hidden_out->temp, hidden_out->transposed ? &hidden_kept->arena : nullptr, rows, h);
+        hidden_out->temp.make(device);
+        hidden_kept->arena.make(device);
+        product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, l.bias, f.aux.mutable_data_ptr(), dtype, device, stream);
+        hidden_out->codes = {hidden_out->temp.at(space.q), hidden_out->temp.at(space.s), space.pitch};
+        if (hidden_out->transposed) hidden_out->codes_t = {hidden_kept->arena.at(space.qt), hidden_kept->arena.at(space.st), space.pitch_t};
+        VIOLA_CALL(viola_gated_quantize_dual_pitched, ptr(f.aux), code_of(dtype), rows, h, gated, const_cast<void*>(hidden_out->codes.q), space.pitch,
+                   const_cast<void*>(hidden_out->codes.s), const_cast<void*>(hidden_out->codes_t.q), hidden_out->transposed ? space.pitch_t : rows,
+                   const_cast<void*>(hidden_out->codes_t.s), to.fwd, to.fwd_limit, to.scale_format(), stream);
+        hidden_kept->rows = rows;
+        return f;
+    }
+    // whole 128 x 128 pieces in both directions: the codes need no padding on either k axis of the down projection
+    if (hidden_out && r.native && rows % 128 == 0 && h % 128 == 0) {
         // h leaves the product as codes with E8M0 scales in the layouts the down projection reads (its k is h wide)
+        const bool transposed = hidden_out->transposed;
         Arena& keep = hidden_kept->arena;
         const int64_t q = hidden_out->temp.take(rows * h), s = hidden_out->temp.take(rows * (h / 32));
-        const int64_t qt = hidden_transposed ? keep.take(h * rows) : -1, st = hidden_transposed ? keep.take(h * (rows / 32)) : -1;
+        const int64_t qt = transposed ? keep.take(h * rows) : -1, st = transposed ? keep.take(h * (rows / 32)) : -1;
         hidden_out->temp.make(device);
         keep.make(device);
-        void* qt_p = hidden_transposed ? keep.at(qt) : nullptr;
-        uint8_t* st_p = hidden_transposed ? keep.as<uint8_t>(st) : nullptr;
+        void* qt_p = transposed ? keep.at(qt) : nullptr;
+        uint8_t* st_p = transposed ? keep.as<uint8_t>(st) : nullptr;
         const void* bias_p = ptr(l.bias);
         const int status = VIOLA_TRY(viola_mx_gated_gemm_encode, a.q, r.fwd, w.q, r.fwd, static_cast<const uint8_t*>(a.s), static_cast<const uint8_t*>(w.s), rows, h,
                                      a.pitch, 1, 32, bias_p, bias_p ? code_of(l.bias.scalar_type()) : 0, const_cast<void*>(ptr(f.aux)), code_of(dtype),
@@ -362,8 +383,15 @@ struct Gradients {
     Tensor dx, dw, db;
 };
 
+// The up projection's dy is dz of this [g | u] and of the dh handed over as dy.
+struct GatedGradient {
+    Tensor z;
+    int activation = 0;
+};
+
 // gated >= 0: dx is dz = [d u act'(g) | d act(g)] from aux = [g | u]. (w: the unpacked weight of the layer.)
-Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& dy_, bool needs_x, bool needs_w, bool needs_b, int gated, const Tensor& aux) {
+Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& dy_, bool needs_x, bool needs_w, bool needs_b, int gated, const Tensor& aux,
+                    const GatedGradient* gate = nullptr) {
     const Recipe& r = *l.recipe;
     const int64_t rows = kept.rows;
     const at::Device device = w.device();
@@ -377,7 +405,7 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
         if (needs_b) out.db = at::zeros({r.out}, dx_options.dtype(kept.bias_grad));
         return out;
     }
-    const Tensor dy = as_matrix(dy_, r.out);
+    const Tensor dy = as_matrix(dy_, gate ? r.out / 2 : r.out);
     Arena temp;
     Codes g, gt, wt;
     float* partial = nullptr;
@@ -397,7 +425,13 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
         const int64_t partial_at = rides ? temp.take(parts * r.out * 4) : -1;
         temp.make(device);
         if (rides) partial = temp.as<float>(partial_at);
-        if (needs_x || needs_w) quantize_groups(r, dy, r.bwd, r.bwd_limit, space, &temp, &temp, partial, &g, &gt, stream);
+        if (gate) {
+            void *q = nullptr, *s = nullptr, *qt = nullptr, *st = nullptr;
+            if (needs_x) { q = temp.at(space.q); s = temp.at(space.s); g = {q, s, space.pitch}; }
+            if (needs_w) { qt = temp.at(space.qt); st = temp.at(space.st); gt = {qt, st, space.pitch_t}; }
+            VIOLA_CALL(viola_gated_backward_quantize_dual, ptr(gate->z), ptr(dy), code_of(dy.scalar_type()), rows, r.out / 2, gate->activation, q, s, qt,
+                       needs_w ? space.pitch_t : rows, st, r.bwd, r.bwd_limit, partial, r.scale_format(), stream);
+        } else if (needs_x || needs_w) quantize_groups(r, dy, r.bwd, r.bwd_limit, space, &temp, &temp, partial, &g, &gt, stream);
         if (needs_b && !rides) out.db = at::sum(dy, at::IntArrayRef{0}, false, kept.bias_grad);
     } else {
         const int64_t pitch_t = ceil_to(rows, 128);
@@ -513,7 +547,7 @@ Tensor linear(const Tensor& x, Layer& l) {
         at::AutoDispatchBelowADInplaceOrView below;
         const Tensor x2 = as_matrix(x, l.recipe->in);
         if (l.bias.defined() && !l.bias.is_contiguous()) l.bias = l.bias.contiguous();
-        y = project(l, x2, x.scalar_type(), need, ww, kept, -1, false, nullptr, nullptr, false, nullptr).y;
+        y = project(l, x2, x.scalar_type(), need, ww, kept, -1, false, nullptr, nullptr, nullptr).y;
         if (x.dim() != 2) y = y.view(output_shape(x, l.recipe->out));
     }
     if (need) {
@@ -544,13 +578,16 @@ struct MlpBackward : public Node {
         const Tensor down_weight = down_kept.weight.unpack();
         const Tensor up_weight = first_half ? up_kept.weight.unpack() : Tensor();
         const bool upper = first_half && (task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2));
+        const bool up_x = task_should_compute_output(0), up_w = task_should_compute_output(1) && up_kept.has_input, up_b = task_should_compute_output(2);
+        // grouped recipes: the plain product writes dh, and the quantizer of dz makes dz as it reads dh and [g | u]
+        const bool direct = upper && up.recipe->grouped && up_kept.rows && up_kept.x_dtype != at::kFloat && down.recipe->in % 64 == 0 && (up_w || (up_x && !up_b));
+        GatedGradient gate{upper ? z.unpack() : Tensor(), activation};
         Gradients d = unproject(down, down_kept, down_weight, dy, upper, task_should_compute_output(3) && down_kept.has_input, task_should_compute_output(4),
-                                activation, upper ? z.unpack() : Tensor());
+                                direct ? -1 : activation, gate.z);
         result[3] = d.dw;
         result[4] = d.db;
         if (!upper) return result;
-        Gradients u = unproject(up, up_kept, up_weight, d.dx, task_should_compute_output(0), task_should_compute_output(1) && up_kept.has_input,
-                                task_should_compute_output(2), -1, Tensor());
+        Gradients u = unproject(up, up_kept, up_weight, d.dx, up_x, up_w, up_b, -1, Tensor(), direct ? &gate : nullptr);
         if (u.dx.defined()) result[0] = u.dx.dim() == (int64_t)x_shape.size() ? u.dx : u.dx.view(x_shape);
         result[1] = u.dw;
         result[2] = u.db;
@@ -579,15 +616,16 @@ Tensor mlp(const Tensor& x, Layer& up, Layer& down, int activation) {
         const Tensor x2 = as_matrix(x, up.recipe->in);
         for (Layer* l : {&up, &down})
             if (l->bias.defined() && !l->bias.is_contiguous()) l->bias = l->bias.contiguous();
-        const int64_t rows = x2.size(0), h = down.recipe->in;
-        // whole 128 x 128 pieces in both directions: the codes need no padding on either k axis of the down projection
-        const bool as_codes = up.recipe->native && rows > 0 && rows % 128 == 0 && h % 128 == 0;
+        const int64_t rows = x2.size(0);
         CodedHidden hidden;
+        hidden.reader = down.recipe.get();
+        hidden.transposed = whole && down_w;
+        const bool as_codes = up.recipe->grouped && rows > 0;
         Forward first = project(up, x2, x.scalar_type(), first_half, up_w, up_kept, activation, first_half, as_codes ? &hidden : nullptr,
-                                as_codes ? &down_kept : nullptr, whole && down_w, nullptr);
+                                as_codes ? &down_kept : nullptr, nullptr);
         z = first.aux;
         const bool coded = !first.y.defined();
-        y = project(down, first.y, x.scalar_type(), whole, down_w, down_kept, -1, false, nullptr, nullptr, false, coded ? &hidden : nullptr).y;
+        y = project(down, first.y, x.scalar_type(), whole, down_w, down_kept, -1, false, nullptr, nullptr, coded ? &hidden : nullptr).y;
         if (x.dim() != 2) y = y.view(output_shape(x, down.recipe->out));
     }
     if (whole) {

@@ -292,18 +292,7 @@ __global__ __launch_bounds__(256) void gated_backward_kernel(const void* __restr
         const float g = load_half(z, r * 2 * h + c, dtype), u = load_half(z, r * 2 * h + h + c, dtype);
         const float d = load_half(dy, idx, dtype);
         float a, derivative;
-        if (activation == VIOLA_SILU) {
-            const float s = 1.0f / (1.0f + expf(-g));
-            a = g * s;
-            derivative = s * (1.0f + g * (1.0f - s));
-        } else if (activation == VIOLA_GELU) {
-            const float t = tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g));
-            a = 0.5f * g * (1.0f + t);
-            derivative = 0.5f * (1.0f + t) + 0.5f * g * (1.0f - t * t) * 0.7978845608028654f * (1.0f + 0.134145f * g * g);
-        } else {
-            a = fmaxf(g, 0.0f);
-            derivative = g > 0.0f ? 1.0f : 0.0f;
-        }
+        gate_math(activation, g, a, derivative);
         store_half(dz, r * 2 * h + c, dtype, d * u * derivative);
         store_half(dz, r * 2 * h + h + c, dtype, d * a);
     }

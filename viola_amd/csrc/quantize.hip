@@ -207,13 +207,7 @@ __global__ __launch_bounds__(256) void quantize_tile(const TIn* __restrict__ x, 
     }
 }
 
-// ------------------------------------------------------------------ 16-bit inputs: both layouts per wavefront
-// A wavefront owns 32 rows x 64 columns. Lane l loads 16 bytes (8 elements) of rows l/8 + 8i, quantizes them for
-// the row-wise layout straight from registers (a 32-column group is four neighbouring lanes), and parks the raw
-// 16 bytes in a wave-private LDS tile. ds_read_b64_tr_b16 then hands every lane the 32 rows of ONE column, four at
-// a time, which is exactly a group of the transposed layout. The LDS tile holds 2-byte values (rows of 64 + 32
-// elements: four consecutive rows start 64 bytes apart in bank space), so LDS moves 12 instructions per 32
-// elements instead of one per element and layout. No block-level synchronisation.
+// ------------------------------------------------------------------ 16-bit values as words of two
 template <typename TIn> __device__ __forceinline__ float widen16(uint32_t bits);
 template <> __device__ __forceinline__ float widen16<bf16_t>(uint32_t bits) { return __uint_as_float(bits << 16); }
 template <> __device__ __forceinline__ float widen16<f16_t>(uint32_t bits) {
@@ -225,224 +219,9 @@ template <typename TIn> __device__ __forceinline__ uint32_t narrow16(float v);
 template <> __device__ __forceinline__ uint32_t narrow16<bf16_t>(float v) { return f32_to_bf16_bits(v); }
 template <> __device__ __forceinline__ uint32_t narrow16<f16_t>(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
 
-// GATED: x is [rows, 2 cols] = [gate | up] and the tile quantized is act(gate) * up [rows, cols]
-// (viola/nn/_mlp_kernels.py:195-230 hands h over as codes; here from the stored projection instead of the accumulators).
-template <typename TIn, typename TOut, bool ROWWISE, bool GATED = false>
-__global__ __launch_bounds__(256) void quantize_dual16(const TIn* __restrict__ x, uint8_t* __restrict__ q,
-                                                        float* __restrict__ scale, uint8_t* __restrict__ qt,
-                                                        float* __restrict__ scale_t, int64_t rows, int64_t cols,
-                                                        float limit, float* __restrict__ column_partial, int e8m0,
-                                                        int activation = 0) {
-    constexpr int LD = 64 + 32;
-    typedef short s16x4 __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    __shared__ __attribute__((aligned(16))) uint16_t park[4][32 * LD];
-    // Transposed codes leave as whole 128-byte lines: the block's four wavefronts hold rows 32 w .. 32 w + 31 of the same
-    // 64 columns, so each has a 32-byte run of every column's line; the runs meet here ([column][128 + 16 bytes]) and
-    // go out as 16-byte pieces, eight lanes to a line, instead of 64 lines touched per store instruction.
-    constexpr int XLD = 128 + 16;
-    __shared__ __attribute__((aligned(16))) uint8_t lines[64 * XLD];
-    const bool by_lines = rows % 16 == 0 && (reinterpret_cast<uintptr_t>(qt) & 15) == 0;   // pieces are whole and aligned
-    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);   // uniform: so is the buffer descriptor
-    uint16_t* mine = park[wave];
-    const int lr = lane / 8, ch = lane % 8;
-    const int64_t nc = (cols + 31) / 32;
-    // a block walks tiles of 128 rows x 64 columns (column tiles fastest) with the grid's stride: the wavefronts stay
-    // resident, so the SIMDs keep several of them in flight instead of waiting for new workgroups to be dispatched
-    const int64_t tiles_x = (cols + 63) / 64, tiles_y = (rows + 127) / 128, tiles = tiles_x * tiles_y;
-    for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    // tiles in flight together (consecutive indices) should form a compact patch: 16 row tiles of one column tile, then
-    // the next column tile, so that a row of x is read in long runs and a row of the transposed output (2 KB per 16
-    // row tiles) is written in long runs too, however wide the matrix is
-    constexpr int64_t BAND = 16;                                            // 8 .. 32 measure the same, 64 slower
-    const int64_t patch = tile / (BAND * tiles_x), within = tile % (BAND * tiles_x);
-    const int64_t tall = tiles_y - patch * BAND < BAND ? tiles_y - patch * BAND : BAND;
-    const int64_t block_r0 = (patch * BAND + within % tall) * 128;
-    const int64_t r0 = block_r0 + wave * 32, c0 = within / tall * 64;
-    const bool active = r0 < rows;                                           // a wavefront past the last row reads zeros and stores nothing
-    const int64_t col8 = c0 + ch * 8;
-
-    // all four loads first, without control flow: a raw buffer over the wavefront's 32 rows returns zero past its end
-    constexpr int WIDTH = GATED ? 2 : 1;                                     // x rows are [gate | up] when GATED
-    const int64_t span = active ? (rows - r0 < 32 ? rows - r0 : 32) * cols * 2 * WIDTH : 0;
-    const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc(const_cast<TIn*>(x + r0 * cols * WIDTH), 0, (int)span, 0x00020000);
-    u32x4 raw[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        raw[i] = __builtin_amdgcn_raw_buffer_load_b128(res, col8 < cols ? (int)(((lr + 8 * i) * cols * WIDTH + col8) * 2) : (int)0x80000000u, 0, 0);
-    if constexpr (GATED) {
-        // the tile quantized is h = act(gate) * up, rounded to TIn as the activation kernels store it
-        u32x4 up[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            up[i] = __builtin_amdgcn_raw_buffer_load_b128(res, col8 < cols ? (int)(((lr + 8 * i) * cols * 2 + cols + col8) * 2) : (int)0x80000000u, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                uint32_t packed = 0;
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const float g = widen16<TIn>(e ? raw[i][w] >> 16 : raw[i][w] & 0xffffu);
-                    const float u = widen16<TIn>(e ? up[i][w] >> 16 : up[i][w] & 0xffffu);
-                    float a, derivative;
-                    gate_math(activation, g, a, derivative);
-                    float hv = a * u;
-                    // keep the product an FP32 value of its own: folded into the narrowing conversion (a mixed-precision
-                    // FMA with a +0 addend) it rounds once instead of twice and turns -0 into +0
-                    asm volatile("" : "+v"(hv));
-                    packed |= narrow16<TIn>(hv) << (16 * e);
-                }
-                raw[i][w] = packed;
-            }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(&mine[(lr + 8 * i) * LD + ch * 8]) = raw[i];
-
-    // row-wise groups: four lanes x 8 values
-    float vr[4][8], s_row[4];
-    bool fast = true;
-    SharedDivisor d_row[4] = {SharedDivisor(1.0f, 0.0f), SharedDivisor(1.0f, 0.0f), SharedDivisor(1.0f, 0.0f), SharedDivisor(1.0f, 0.0f)};
-    // The largest magnitude of a group is found on the raw 16-bit patterns, two to an instruction: with the sign bit
-    // masked off, bf16 and fp16 order as unsigned integers like their values, and anything at or above the pattern of
-    // infinity is an Inf or a NaN, which sends the wavefront down the exact path below (where the maximum is taken
-    // again the way the reference's kernel takes it, ignoring NaN).
-    constexpr uint32_t MAGNITUDE = 0x7fff7fffu, INF16 = sizeof(TIn) == 2 && std::is_same<TIn, bf16_t>::value ? 0x7f80u : 0x7c00u;
-    auto top16 = [](uint32_t pairs) -> uint32_t { const uint32_t lo = pairs & 0xffffu, hi = pairs >> 16; return lo > hi ? lo : hi; };
-    if constexpr (ROWWISE) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) vr[i][e] = widen16<TIn>(e % 2 ? raw[i][e / 2] >> 16 : raw[i][e / 2] & 0xffffu);
-            uint32_t top = top16(pk_max_u16(pk_max_u16(raw[i][0] & MAGNITUDE, raw[i][1] & MAGNITUDE), pk_max_u16(raw[i][2] & MAGNITUDE, raw[i][3] & MAGNITUDE)));
-            const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)top, 0x4E, 0xf, 0xf, true);      // lanes 2 3 0 1 of the quad
-            top = top > other ? top : other;
-            const uint32_t next = (uint32_t)__builtin_amdgcn_mov_dpp((int)top, 0xB1, 0xf, 0xf, true);       // lanes 1 0 3 2
-            top = top > next ? top : next;
-            s_row[i] = group_scale(widen16<TIn>(top), limit, e8m0);
-            d_row[i] = SharedDivisor(s_row[i], top >= INF16 ? __uint_as_float(0x7fc00000u) : 0.0f);
-            fast = fast && d_row[i].fast;
-        }
-    }
-    // transposed groups: column lane % 16 of the 16-column strip lane / 16, rows 4t .. 4t+3 per read
-    const int64_t col = c0 + lane;
-    const int strip = (lane / 16) * 16, sub = lane & 15;
-    const uint16_t* at = &mine[(sub >> 2) * LD + strip + 4 * (sub & 3)];
-    float vc[32];
-    uint32_t top_col = 0;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const uint2 four = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * t * LD)));
-        vc[4 * t] = widen16<TIn>(four.x & 0xffffu); vc[4 * t + 1] = widen16<TIn>(four.x >> 16);
-        vc[4 * t + 2] = widen16<TIn>(four.y & 0xffffu); vc[4 * t + 3] = widen16<TIn>(four.y >> 16);
-        top_col = pk_max_u16(top_col, pk_max_u16(four.x & MAGNITUDE, four.y & MAGNITUDE));
-    }
-    top_col = top16(top_col);
-    float s_col = group_scale(widen16<TIn>(top_col), limit, e8m0);
-    const SharedDivisor d_col(s_col, top_col >= INF16 ? __uint_as_float(0x7fc00000u) : 0.0f);
-    fast = fast && d_col.fast;
-
-    // one decision per wavefront: the common case runs without a single divergent branch
-    uint2 row_codes[4];
-    uint32_t col_codes[8];
-    if (__builtin_amdgcn_ballot_w64(!fast) == 0 && limit == fp8_traits<TOut>::max) {
-        // the scale is max |v| / (the format's largest value): no quotient can round past the largest code
-        if constexpr (ROWWISE) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                row_codes[i] = make_uint2(fast_encode4_unclamped<TOut>(d_row[i], vr[i][0], vr[i][1], vr[i][2], vr[i][3]),
-                                          fast_encode4_unclamped<TOut>(d_row[i], vr[i][4], vr[i][5], vr[i][6], vr[i][7]));
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) col_codes[k] = fast_encode4_unclamped<TOut>(d_col, vc[4 * k], vc[4 * k + 1], vc[4 * k + 2], vc[4 * k + 3]);
-    } else if (__builtin_amdgcn_ballot_w64(!fast) == 0) {
-        if constexpr (ROWWISE) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                row_codes[i] = make_uint2(fast_encode4<TOut>(d_row[i], limit, vr[i][0], vr[i][1], vr[i][2], vr[i][3]),
-                                          fast_encode4<TOut>(d_row[i], limit, vr[i][4], vr[i][5], vr[i][6], vr[i][7]));
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) col_codes[k] = fast_encode4<TOut>(d_col, limit, vc[4 * k], vc[4 * k + 1], vc[4 * k + 2], vc[4 * k + 3]);
-    } else {
-        // some group of the wavefront holds an Inf or a NaN, or a scale outside the quotient route's domain: the maxima
-        // again as the reference's kernel takes them (fmax ignores NaN), true division, software encoder
-        const SharedDivisor exact(1.0f, __uint_as_float(0x7fc00000u));
-        if constexpr (ROWWISE) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float amax = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(vr[i][e]));
-                s_row[i] = group_scale(group_max<4>(amax), limit, e8m0);
-                row_codes[i] = encode8<TOut>(vr[i], s_row[i], limit, exact);
-            }
-        }
-        float amax = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(vc[i]));
-        s_col = group_scale(amax, limit, e8m0);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            col_codes[k] = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) col_codes[k] |= (uint32_t)encode_clamped<TOut>(vc[4 * k + e], s_col, limit) << (8 * e);
-        }
-    }
-
-    if constexpr (ROWWISE) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t row = r0 + lr + 8 * i;
-            if (row < rows && col8 < cols) {
-                *reinterpret_cast<uint2*>(q + row * cols + col8) = row_codes[i];
-                if (ch % 4 == 0) put_scale(scale, row * nc + col8 / 32, s_row[i], e8m0);
-            }
-        }
-    }
-    if (active && col < cols) {
-        const int64_t nr = (rows + 31) / 32;
-        put_scale(scale_t, col * nr + r0 / 32, s_col, e8m0);
-        if (column_partial) {
-            float sum = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 32; ++i) sum += vc[i];
-            column_partial[(r0 / 32) * cols + col] = sum;
-        }
-        uint8_t* dst = qt + col * rows + r0;
-        if (by_lines) {
-            // stored below, by the whole block
-        } else if (rows - r0 >= 32 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-            reinterpret_cast<uint4*>(dst)[0] = make_uint4(col_codes[0], col_codes[1], col_codes[2], col_codes[3]);
-            reinterpret_cast<uint4*>(dst)[1] = make_uint4(col_codes[4], col_codes[5], col_codes[6], col_codes[7]);
-        } else {
-            const int count = (int)(rows - r0 < 32 ? rows - r0 : 32);
-            for (int i = 0; i < count; ++i) dst[i] = (uint8_t)(col_codes[i >> 2] >> (8 * (i & 3)));
-        }
-    }
-    if (by_lines) {
-        __syncthreads();                                                     // the pieces of the tile before have been read
-        if (active) {
-            uint4* run = reinterpret_cast<uint4*>(&lines[lane * XLD + wave * 32]);
-            run[0] = make_uint4(col_codes[0], col_codes[1], col_codes[2], col_codes[3]);
-            run[1] = make_uint4(col_codes[4], col_codes[5], col_codes[6], col_codes[7]);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int id = it * 256 + (int)threadIdx.x, c = id >> 3, piece = id & 7;
-            const int64_t row = block_r0 + piece * 16;                       // rows % 16 == 0: a piece is inside or outside as a whole
-            if (c0 + c < cols && row < rows)
-                *reinterpret_cast<uint4*>(qt + (c0 + c) * rows + row) = *reinterpret_cast<const uint4*>(&lines[c * XLD + piece * 16]);
-        }
-    }
-    }
-}
-
 // ------------------------------------------------------------------ 16-bit inputs: both layouts from a 64 x 64 tile
 // A block of 256 threads per tile, one tile per block: eight blocks are resident on a compute unit at 64 registers, and
-// the launch is timed 15 - 25 % below the persistent 128 x 64 kernel above on every shape tried (8192 x 4096 bf16:
+// the launch is timed 15 - 25 % below a persistent kernel on 128 x 64 tiles on every shape tried (8192 x 4096 bf16:
 // 27.7 against 36.2 us). Row-wise: thread (row tid / 4, 16 columns) loads 32 bytes, a 32-column group is a pair of
 // lanes; four neighbouring lanes store 64 consecutive bytes of codes. The raw 16-bit values are parked in LDS
 // ([row][64 + 4 values], the four 16-column blocks of a row permuted by row / 16 so that the transposed phase's four
@@ -471,12 +250,16 @@ __device__ __forceinline__ bool encode_words16(const uint32_t (&words)[8], float
     s = group_scale(widen16<TIn>(top), limit, e8m0);
     const SharedDivisor d(s, nonfinite ? __uint_as_float(0x7fc00000u) : 0.0f);
     if (__builtin_amdgcn_ballot_w64(!d.fast) != 0) return false;
+    auto encode = [&](const auto& divisor) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float a = widen16<TIn>(words[2 * k] & 0xffffu), b = widen16<TIn>(words[2 * k] >> 16);
-        const float c = widen16<TIn>(words[2 * k + 1] & 0xffffu), e = widen16<TIn>(words[2 * k + 1] >> 16);
-        codes[k] = clamp_free ? fast_encode4_unclamped<TOut>(d, a, b, c, e) : fast_encode4<TOut>(d, limit, a, b, c, e);
-    }
+        for (int k = 0; k < 4; ++k) {
+            const float a = widen16<TIn>(words[2 * k] & 0xffffu), b = widen16<TIn>(words[2 * k] >> 16);
+            const float c = widen16<TIn>(words[2 * k + 1] & 0xffffu), e = widen16<TIn>(words[2 * k + 1] >> 16);
+            codes[k] = clamp_free ? fast_encode4_unclamped<TOut>(divisor, a, b, c, e) : fast_encode4<TOut>(divisor, limit, a, b, c, e);
+        }
+    };
+    if (e8m0) encode(PowerDivisor{d.r});
+    else encode(d);
     return true;
 }
 // The same for 16 finite values already widened: the maximum is taken in floating point, three values per instruction.
@@ -497,10 +280,14 @@ __device__ __forceinline__ bool encode_finite16(const float (&v)[16], float limi
     s = group_scale(amax, limit, e8m0);
     const SharedDivisor d(s, 0.0f);
     if (__builtin_amdgcn_ballot_w64(!d.fast) != 0) return false;
+    auto encode = [&](const auto& divisor) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        codes[k] = clamp_free ? fast_encode4_unclamped<TOut>(d, v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3])
-                              : fast_encode4<TOut>(d, limit, v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+        for (int k = 0; k < 4; ++k)
+            codes[k] = clamp_free ? fast_encode4_unclamped<TOut>(divisor, v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3])
+                                  : fast_encode4<TOut>(divisor, limit, v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+    };
+    if (e8m0) encode(PowerDivisor{d.r});
+    else encode(d);
     return true;
 }
 // The exact route: an Inf or a NaN in some group of the wavefront, or a scale outside the quotient route's domain. The
@@ -531,146 +318,253 @@ __device__ __noinline__ Exact16 encode_words16_exact(uint32_t w0, uint32_t w1, u
     return out;
 }
 
-template <typename TIn, typename TOut, bool INTERIOR>
-__device__ __forceinline__ void dual16_tile64(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ scale,
-                                              uint8_t* __restrict__ qt, float* __restrict__ scale_t, int64_t rows, int64_t cols,
-                                              int64_t q_pitch, int64_t qt_pitch, bool vec, float limit, float* __restrict__ column_partial, int e8m0, int64_t r0, int64_t c0,
-                                              uint16_t* park, int* flags) {
-    constexpr int LDV = 64 + 4;                                              // values per parked row (34 dwords)
-    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
-    const int64_t nc = (q_pitch + 31) / 32, nr = (qt_pitch + 31) / 32;
-    const bool clamp_free = limit == fp8_traits<TOut>::max;
+// The tile's matrix and where its codes go.
+struct Dual16 {
+    uint8_t* q; float* scale; uint8_t* qt; float* scale_t; float* column_partial;
+    int64_t rows, cols, q_pitch, qt_pitch;
+    float limit; int e8m0;
+};
+constexpr int DUAL16_LDV = 64 + 4;                                           // values per parked row (34 dwords)
 
-    // ---- row-wise
-    {
-        const int lr = tid / 4, lc = (tid % 4) * 16;
-        const int64_t row = r0 + lr, col = c0 + lc;
-        const uint32_t offset = (uint32_t)lr * (uint32_t)cols + (uint32_t)lc;   // from the tile's first element (INTERIOR: < 2^31)
-        uint4 raw[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
-        if constexpr (INTERIOR) {
-            const TIn* tile = x + r0 * cols + c0;
-            raw[0] = *reinterpret_cast<const uint4*>(tile + offset);
-            raw[1] = *reinterpret_cast<const uint4*>(tile + offset + 8);
-        } else if (row < rows && !vec) {
-            uint32_t* halves = reinterpret_cast<uint32_t*>(raw);
-            const uint16_t* src = reinterpret_cast<const uint16_t*>(x) + row * cols + col;
+// The thread's 16 values (row tid / 4 of the tile, columns 16 (tid % 4) ..) of a matrix `cols` wide and `pitch` apart, as words of
+// two; zeros past the matrix.
+template <typename TIn, bool INTERIOR>
+__device__ __forceinline__ void dual16_load(const TIn* __restrict__ x, int64_t rows, int64_t cols, int64_t pitch, bool vec, int64_t r0, int64_t c0,
+                                            uint32_t (&words)[8]) {
+    const int lr = threadIdx.x / 4, lc = (threadIdx.x % 4) * 16;
+    const int64_t row = r0 + lr, col = c0 + lc;
+    uint4 raw[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
+    if constexpr (INTERIOR) {
+        const TIn* tile = x + r0 * pitch + c0;
+        const uint32_t offset = (uint32_t)lr * (uint32_t)pitch + (uint32_t)lc;   // from the tile's first element (INTERIOR: < 2^31)
+        raw[0] = *reinterpret_cast<const uint4*>(tile + offset);
+        raw[1] = *reinterpret_cast<const uint4*>(tile + offset + 8);
+    } else if (row < rows && !vec) {
+        uint32_t* halves = reinterpret_cast<uint32_t*>(raw);
+        const uint16_t* src = reinterpret_cast<const uint16_t*>(x) + row * pitch + col;
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if (col + i < cols) halves[i / 2] |= (uint32_t)src[i] << (16 * (i % 2));
-        } else if (row < rows) {
-            if (col < cols) raw[0] = *reinterpret_cast<const uint4*>(x + row * cols + col);      // cols % 8 == 0: whole pieces
-            if (col + 8 < cols) raw[1] = *reinterpret_cast<const uint4*>(x + row * cols + col + 8);
-        }
-        {
-            uint2* mine = reinterpret_cast<uint2*>(&park[lr * LDV + (lc ^ (((lr >> 4) & 3) << 4))]);   // 16-column blocks swapped by row chunk
-            mine[0] = make_uint2(raw[0].x, raw[0].y); mine[1] = make_uint2(raw[0].z, raw[0].w);
-            mine[2] = make_uint2(raw[1].x, raw[1].y); mine[3] = make_uint2(raw[1].z, raw[1].w);
-        }
-        const uint32_t words[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
-        float s_row;
-        uint32_t codes[4];
-        bool nonfinite;
-        if (!encode_words16<TIn, TOut>(words, limit, e8m0, clamp_free, s_row, codes, nonfinite)) {
-            const Exact16 r = encode_words16_exact<TIn, TOut>(words[0], words[1], words[2], words[3], words[4], words[5], words[6], words[7], limit, e8m0);
-            codes[0] = r.c0; codes[1] = r.c1; codes[2] = r.c2; codes[3] = r.c3; s_row = r.s;
-        }
-        if (!q) {
-            // transposed layout only
-        } else if constexpr (INTERIOR) {
-            *reinterpret_cast<uint4*>(q + r0 * q_pitch + c0 + ((uint32_t)lr * (uint32_t)q_pitch + (uint32_t)lc)) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
-            if (tid % 2 == 0) put_scale(scale, (r0 * nc + c0 / 32) + (int64_t)((uint32_t)lr * (uint32_t)nc + (uint32_t)(lc / 32)), s_row, e8m0);
-        } else if (row < rows && col < q_pitch) {                            // columns cols .. q_pitch - 1: zero codes
-            uint8_t* dst = q + row * q_pitch + col;
-            if (col + 16 <= q_pitch && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-                *reinterpret_cast<uint4*>(dst) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
-            } else {
-                const int count = (int)(q_pitch - col < 16 ? q_pitch - col : 16);
-                for (int i = 0; i < count; ++i) dst[i] = (uint8_t)(codes[i >> 2] >> (8 * (i & 3)));
-            }
-            if (tid % 2 == 0) put_scale(scale, row * nc + col / 32, s_row, e8m0);
-        }
-        const bool any_nonfinite = __builtin_amdgcn_ballot_w64(nonfinite) != 0;   // over the whole wavefront: outside the branch
-        if (lane == 0) flags[wave] = any_nonfinite;
+        for (int i = 0; i < 16; ++i)
+            if (col + i < cols) halves[i / 2] |= (uint32_t)src[i] << (16 * (i % 2));
+    } else if (row < rows) {
+        if (col < cols) raw[0] = *reinterpret_cast<const uint4*>(x + row * pitch + col);      // cols % 8 == 0: whole pieces
+        if (col + 8 < cols) raw[1] = *reinterpret_cast<const uint4*>(x + row * pitch + col + 8);
     }
-    if (!qt) return;                                                         // row-wise layout only (uniform)
-    __syncthreads();
-    // no NaN and no Inf anywhere in the tile: the transposed phase may then take its maxima in floating point
-    const bool plain = (flags[0] | flags[1] | flags[2] | flags[3]) == 0;
+    words[0] = raw[0].x; words[1] = raw[0].y; words[2] = raw[0].z; words[3] = raw[0].w;
+    words[4] = raw[1].x; words[5] = raw[1].y; words[6] = raw[1].z; words[7] = raw[1].w;
+}
 
-    // ---- transposed: wavefront w takes columns 16 w .. + 15 of the tile; lane = (column lane / 4, rows 16 (lane % 4) .. + 15), so four
-    // neighbouring lanes write 64 consecutive bytes of one transposed row and a 32-row group is a pair of lanes
+// Row-wise codes of the tile at (r0, c0), its values parked for dual16_columns; flags[wave]: they hold a NaN or an Inf.
+template <typename TIn, typename TOut, bool INTERIOR>
+__device__ __forceinline__ void dual16_rows(const Dual16& d, const uint32_t (&words)[8], int64_t r0, int64_t c0, uint16_t* park, int* flags) {
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const int64_t nc = (d.q_pitch + 31) / 32;
+    const int lr = tid / 4, lc = (tid % 4) * 16;
+    const int64_t row = r0 + lr, col = c0 + lc;
     {
-        const int tc = wave * 16 + lane / 4, chunk = lane % 4;
-        const int64_t tcol = c0 + tc, trow = r0 + chunk * 16;                // first of the lane's 16 rows
-        uint32_t bits[16];
+        uint2* mine = reinterpret_cast<uint2*>(&park[lr * DUAL16_LDV + (lc ^ (((lr >> 4) & 3) << 4))]);   // 16-column blocks swapped by row chunk
+        mine[0] = make_uint2(words[0], words[1]); mine[1] = make_uint2(words[2], words[3]);
+        mine[2] = make_uint2(words[4], words[5]); mine[3] = make_uint2(words[6], words[7]);
+    }
+    float s_row = 0.0f;
+    uint32_t codes[4] = {0, 0, 0, 0};
+    bool nonfinite;
+    if (!d.q) {                                                              // transposed layout only
+        constexpr uint32_t MAGNITUDE = 0x7fff7fffu, INF16 = std::is_same<TIn, bf16_t>::value ? 0x7f80u : 0x7c00u;
+        uint32_t top = 0;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) bits[i] = park[(chunk * 16 + i) * LDV + (tc ^ (chunk << 4))];
-        float w[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) w[i] = widen16<TIn>(bits[i]);
-        float s_col;
-        uint32_t tcodes[4];
-        if (!plain || !encode_finite16<TOut>(w, limit, e8m0, clamp_free, s_col, tcodes)) {
-            const Exact16 r = encode_words16_exact<TIn, TOut>(bits[0] | bits[1] << 16, bits[2] | bits[3] << 16, bits[4] | bits[5] << 16, bits[6] | bits[7] << 16,
-                                                              bits[8] | bits[9] << 16, bits[10] | bits[11] << 16, bits[12] | bits[13] << 16,
-                                                              bits[14] | bits[15] << 16, limit, e8m0);
-            tcodes[0] = r.c0; tcodes[1] = r.c1; tcodes[2] = r.c2; tcodes[3] = r.c3; s_col = r.s;
+        for (int e = 0; e < 8; ++e) top = pk_max_u16(top, words[e] & MAGNITUDE);
+        nonfinite = (top & 0xffffu) >= INF16 || (top >> 16) >= INF16;
+    } else if (!encode_words16<TIn, TOut>(words, d.limit, d.e8m0, d.limit == fp8_traits<TOut>::max, s_row, codes, nonfinite)) {
+        const Exact16 r = encode_words16_exact<TIn, TOut>(words[0], words[1], words[2], words[3], words[4], words[5], words[6], words[7], d.limit, d.e8m0);
+        codes[0] = r.c0; codes[1] = r.c1; codes[2] = r.c2; codes[3] = r.c3; s_row = r.s;
+    }
+    if (!d.q) {
+        // nothing to store
+    } else if constexpr (INTERIOR) {
+        *reinterpret_cast<uint4*>(d.q + r0 * d.q_pitch + c0 + ((uint32_t)lr * (uint32_t)d.q_pitch + (uint32_t)lc)) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
+        if (tid % 2 == 0) put_scale(d.scale, (r0 * nc + c0 / 32) + (int64_t)((uint32_t)lr * (uint32_t)nc + (uint32_t)(lc / 32)), s_row, d.e8m0);
+    } else if (row < d.rows && col < d.q_pitch) {                            // columns cols .. q_pitch - 1: zero codes
+        uint8_t* dst = d.q + row * d.q_pitch + col;
+        if (col + 16 <= d.q_pitch && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+            *reinterpret_cast<uint4*>(dst) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
+        } else {
+            const int count = (int)(d.q_pitch - col < 16 ? d.q_pitch - col : 16);
+            for (int i = 0; i < count; ++i) dst[i] = (uint8_t)(codes[i >> 2] >> (8 * (i & 3)));
         }
-        float sum = 0.0f;
-        if (column_partial) {
+        if (tid % 2 == 0) put_scale(d.scale, row * nc + col / 32, s_row, d.e8m0);
+    }
+    const bool any_nonfinite = __builtin_amdgcn_ballot_w64(nonfinite) != 0;   // over the whole wavefront: outside the branch
+    if (lane == 0) flags[wave] = any_nonfinite;
+}
+
+// Transposed codes of the parked tile (after a barrier): wavefront w takes columns 16 w .. + 15; lane = (column lane / 4, rows
+// 16 (lane % 4) .. + 15), so four neighbouring lanes write 64 consecutive bytes of one transposed row and a 32-row group is a
+// pair of lanes.
+template <typename TIn, typename TOut, bool INTERIOR>
+__device__ __forceinline__ void dual16_columns(const Dual16& d, int64_t r0, int64_t c0, const uint16_t* park, const int* flags) {
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    const int64_t nr = (d.qt_pitch + 31) / 32;
+    // no NaN and no Inf anywhere in the tile: the maxima may then be taken in floating point
+    const bool plain = (flags[0] | flags[1] | flags[2] | flags[3]) == 0;
+    const int tc = wave * 16 + lane / 4, chunk = lane % 4;
+    const int64_t tcol = c0 + tc, trow = r0 + chunk * 16;                    // first of the lane's 16 rows
+    uint32_t bits[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sum += w[i];
-            const float other = quad_xor<1>(sum);
-            sum = chunk % 2 == 0 ? sum + other : other + sum;                 // rows 0 .. 15 first, then 16 .. 31
+    for (int i = 0; i < 16; ++i) bits[i] = park[(chunk * 16 + i) * DUAL16_LDV + (tc ^ (chunk << 4))];
+    float w[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[i] = widen16<TIn>(bits[i]);
+    float s_col;
+    uint32_t tcodes[4];
+    if (!plain || !encode_finite16<TOut>(w, d.limit, d.e8m0, d.limit == fp8_traits<TOut>::max, s_col, tcodes)) {
+        const Exact16 r = encode_words16_exact<TIn, TOut>(bits[0] | bits[1] << 16, bits[2] | bits[3] << 16, bits[4] | bits[5] << 16, bits[6] | bits[7] << 16,
+                                                          bits[8] | bits[9] << 16, bits[10] | bits[11] << 16, bits[12] | bits[13] << 16,
+                                                          bits[14] | bits[15] << 16, d.limit, d.e8m0);
+        tcodes[0] = r.c0; tcodes[1] = r.c1; tcodes[2] = r.c2; tcodes[3] = r.c3; s_col = r.s;
+    }
+    float sum = 0.0f;
+    if (d.column_partial) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum += w[i];
+        const float other = quad_xor<1>(sum);
+        sum = chunk % 2 == 0 ? sum + other : other + sum;                     // rows 0 .. 15 first, then 16 .. 31
+    }
+    if constexpr (INTERIOR) {
+        *reinterpret_cast<uint4*>(d.qt + c0 * d.qt_pitch + r0 + ((uint32_t)tc * (uint32_t)d.qt_pitch + (uint32_t)(chunk * 16))) = make_uint4(tcodes[0], tcodes[1], tcodes[2], tcodes[3]);
+        if (chunk % 2 == 0) {
+            put_scale(d.scale_t, (c0 * nr + r0 / 32) + (int64_t)((uint32_t)tc * (uint32_t)nr + (uint32_t)(chunk / 2)), s_col, d.e8m0);
+            if (d.column_partial) (d.column_partial + (r0 / 32) * d.cols + c0)[(uint32_t)(chunk / 2) * (uint32_t)d.cols + (uint32_t)tc] = sum;
         }
-        if constexpr (INTERIOR) {
-            *reinterpret_cast<uint4*>(qt + c0 * qt_pitch + r0 + ((uint32_t)tc * (uint32_t)qt_pitch + (uint32_t)(chunk * 16))) = make_uint4(tcodes[0], tcodes[1], tcodes[2], tcodes[3]);
-            if (chunk % 2 == 0) {
-                put_scale(scale_t, (c0 * nr + r0 / 32) + (int64_t)((uint32_t)tc * (uint32_t)nr + (uint32_t)(chunk / 2)), s_col, e8m0);
-                if (column_partial) (column_partial + (r0 / 32) * cols + c0)[(uint32_t)(chunk / 2) * (uint32_t)cols + (uint32_t)tc] = sum;
-            }
-        } else if (tcol < cols && trow < qt_pitch) {                         // rows rows .. qt_pitch - 1: zero codes
-            uint8_t* dst = qt + tcol * qt_pitch + trow;
-            if (trow + 16 <= qt_pitch && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-                *reinterpret_cast<uint4*>(dst) = make_uint4(tcodes[0], tcodes[1], tcodes[2], tcodes[3]);
-            } else {
-                const int count = (int)(qt_pitch - trow < 16 ? qt_pitch - trow : 16);
-                for (int i = 0; i < count; ++i) dst[i] = (uint8_t)(tcodes[i >> 2] >> (8 * (i & 3)));
-            }
-            if (chunk % 2 == 0) {
-                put_scale(scale_t, tcol * nr + trow / 32, s_col, e8m0);
-                if (column_partial && trow < rows) column_partial[(trow / 32) * cols + tcol] = sum;
-            }
+    } else if (tcol < d.cols && trow < d.qt_pitch) {                         // rows rows .. qt_pitch - 1: zero codes
+        uint8_t* dst = d.qt + tcol * d.qt_pitch + trow;
+        if (trow + 16 <= d.qt_pitch && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+            *reinterpret_cast<uint4*>(dst) = make_uint4(tcodes[0], tcodes[1], tcodes[2], tcodes[3]);
+        } else {
+            const int count = (int)(d.qt_pitch - trow < 16 ? d.qt_pitch - trow : 16);
+            for (int i = 0; i < count; ++i) dst[i] = (uint8_t)(tcodes[i >> 2] >> (8 * (i & 3)));
+        }
+        if (chunk % 2 == 0) {
+            put_scale(d.scale_t, tcol * nr + trow / 32, s_col, d.e8m0);
+            if (d.column_partial && trow < d.rows) d.column_partial[(trow / 32) * d.cols + tcol] = sum;
         }
     }
 }
 
-template <typename TIn, typename TOut>
-__global__ __launch_bounds__(256, 8) void quantize_dual16_tile64(const TIn* __restrict__ x, uint8_t* __restrict__ q,
-                                                               float* __restrict__ scale, uint8_t* __restrict__ qt,
-                                                               float* __restrict__ scale_t, int64_t rows, int64_t cols,
-                                                               int64_t q_pitch, int64_t qt_pitch,
-                                                               float limit, float* __restrict__ column_partial, int e8m0, int xcd_walk,
-                                                               int aligned, int vec) {
-    __shared__ __attribute__((aligned(16))) uint16_t park[64 * (64 + 4)];
-    __shared__ __attribute__((aligned(16))) int flags[4];                   // per wavefront: its rows hold a NaN or an Inf
-    // blocks are dispatched in index order: those in flight together take 32 row tiles of one column tile, then the next
-    // column tile, so the transposed output is written in 2 KB runs per row however wide the matrix is (the launcher
-    // keeps the tile count below 2^31)
+// The walk of the 64 x 64 tiles. Blocks are dispatched in index order: those in flight together take 32 row tiles of one column
+// tile, then the next column tile, so the transposed output is written in 2 KB runs per row however wide the matrix is (the
+// launcher keeps the tile count below 2^31). False: past the last tile.
+__device__ __forceinline__ bool dual16_tile(uint32_t tiles_x, uint32_t tiles_y, int xcd_walk, int64_t& r0, int64_t& c0) {
     constexpr uint32_t BAND = 32;
-    const uint32_t tiles_x = (uint32_t)((q_pitch + 63) / 64), tiles_y = (uint32_t)((qt_pitch + 63) / 64), tiles = tiles_x * tiles_y;
+    const uint32_t tiles = tiles_x * tiles_y;
     uint32_t id = blockIdx.x;
     if (xcd_walk) {
         // consecutive block indices go to the eight XCDs in turn: give each XCD one contiguous eighth of the walk, so the
         // halves of a 128-byte line of the transposed output (two row tiles) meet in one L2
         id = (id % 8) * ((tiles + 7) / 8) + id / 8;
     }
-    if (id >= tiles) return;
+    if (id >= tiles) return false;
     const uint32_t patch = id / (BAND * tiles_x), within = id % (BAND * tiles_x);
     const uint32_t tall = tiles_y - patch * BAND < BAND ? tiles_y - patch * BAND : BAND;
-    const int64_t r0 = (int64_t)(patch * BAND + within % tall) * 64, c0 = (int64_t)(within / tall) * 64;
-    if (aligned && r0 + 64 <= rows && c0 + 64 <= cols) dual16_tile64<TIn, TOut, true>(x, q, scale, qt, scale_t, rows, cols, q_pitch, qt_pitch, true, limit, column_partial, e8m0, r0, c0, park, flags);
-    else dual16_tile64<TIn, TOut, false>(x, q, scale, qt, scale_t, rows, cols, q_pitch, qt_pitch, vec != 0, limit, column_partial, e8m0, r0, c0, park, flags);
+    r0 = (int64_t)(patch * BAND + within % tall) * 64;
+    c0 = (int64_t)(within / tall) * 64;
+    return true;
+}
+
+template <typename TIn, typename TOut>
+__global__ __launch_bounds__(256, 8) void quantize_dual16_tile64(const TIn* __restrict__ x, const Dual16 d, int xcd_walk, int aligned, int vec) {
+    __shared__ __attribute__((aligned(16))) uint16_t park[64 * DUAL16_LDV];
+    __shared__ __attribute__((aligned(16))) int flags[4];                   // per wavefront: its rows hold a NaN or an Inf
+    int64_t r0, c0;
+    if (!dual16_tile((uint32_t)((d.q_pitch + 63) / 64), (uint32_t)((d.qt_pitch + 63) / 64), xcd_walk, r0, c0)) return;
+    auto tile = [&](auto interior) __attribute__((always_inline)) {
+        constexpr bool INTERIOR = decltype(interior)::value;
+        uint32_t words[8];
+        dual16_load<TIn, INTERIOR>(x, d.rows, d.cols, d.cols, vec != 0, r0, c0, words);
+        dual16_rows<TIn, TOut, INTERIOR>(d, words, r0, c0, park, flags);
+        if (!d.qt) return;                                                   // row-wise layout only (uniform)
+        __syncthreads();
+        dual16_columns<TIn, TOut, INTERIOR>(d, r0, c0, park, flags);
+    };
+    if (aligned && r0 + 64 <= d.rows && c0 + 64 <= d.cols) tile(std::true_type{});
+    else tile(std::false_type{});
+}
+
+// The gated activation of a MLP in front of the quantizer, from the stored projection z = [g | u] [rows, 2 h]: h = act(g) * u
+// never leaves the registers as a 16-bit matrix, nor does dz (below). FP16: the products are kept FP32 values of their own: folded
+// into the narrowing conversion (a mixed-precision FMA with a +0 addend) they would round once instead of twice and turn -0
+// into +0.
+template <typename TIn>
+__device__ __forceinline__ uint32_t narrow_pair(float a, float b) {
+    if constexpr (std::is_same<TIn, bf16_t>::value) return f32_to_bf16x2_bits(a, b);
+    asm volatile("" : "+v"(a), "+v"(b));
+    return narrow16<TIn>(a) | narrow16<TIn>(b) << 16;
+}
+
+// Forward: one tile of h. What bounds it: bytes (6 per element of h: 4 read, 2 written) and, close behind, the arithmetic of the
+// activation and of both encoders. 4096 x 4608 gelu: 55 -> 30 us against a
+// persistent kernel on 128 x 64 tiles; 16384 x 11008 silu: 288 us, 3.8 TB/s.
+template <typename TIn, typename TOut, int ACT>
+__global__ __launch_bounds__(256, 8) void gated_quantize_dual16(const TIn* __restrict__ z, const Dual16 d, int xcd_walk, int aligned) {
+    __shared__ __attribute__((aligned(16))) uint16_t park[64 * DUAL16_LDV];
+    __shared__ __attribute__((aligned(16))) int flags[4];
+    int64_t r0, c0;
+    if (!dual16_tile((uint32_t)((d.q_pitch + 63) / 64), (uint32_t)((d.qt_pitch + 63) / 64), xcd_walk, r0, c0)) return;
+    auto tile = [&](auto interior) __attribute__((always_inline)) {
+        constexpr bool INTERIOR = decltype(interior)::value;
+        uint32_t g[8], u[8];
+        dual16_load<TIn, INTERIOR>(z, d.rows, d.cols, 2 * d.cols, true, r0, c0, g);
+        dual16_load<TIn, INTERIOR>(z + d.cols, d.rows, d.cols, 2 * d.cols, true, r0, c0, u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float lo, hi, derivative;
+            gate_math(ACT, widen16<TIn>(g[e] & 0xffffu), lo, derivative);
+            gate_math(ACT, widen16<TIn>(g[e] >> 16), hi, derivative);
+            g[e] = narrow_pair<TIn>(lo * widen16<TIn>(u[e] & 0xffffu), hi * widen16<TIn>(u[e] >> 16));
+        }
+        dual16_rows<TIn, TOut, INTERIOR>(d, g, r0, c0, park, flags);
+        if (!d.qt) return;
+        __syncthreads();
+        dual16_columns<TIn, TOut, INTERIOR>(d, r0, c0, park, flags);
+    };
+    if (aligned && r0 + 64 <= d.rows && c0 + 64 <= d.cols) tile(std::true_type{});
+    else tile(std::false_type{});
+}
+
+// Backward: dz = [dh u act'(g) | dh act(g)] [rows, 2 h], h a multiple of 64; the block of a tile of dh makes both tiles of dz, so z
+// and dh are read once (10 bytes per element of h, against 8 for making dz in the product's epilogue and 8 for reading it back
+// into the quantizer). 4096 x 4608 gelu behind a k of 1152: 106 + 30 -> 39 + 50 us; 16384 x 11008 silu: 541 us, 3.3 TB/s.
+// Four blocks per CU: with six the registers do not hold all of a lane's loads in flight (4096 x 4608 46 -> 41 us).
+template <typename TIn, typename TOut, int ACT>
+__global__ __launch_bounds__(256, 4) void gated_backward_quantize_dual16(const TIn* __restrict__ z, const TIn* __restrict__ dh, int64_t h, const Dual16 d,
+                                                                         int xcd_walk, int aligned) {
+    __shared__ __attribute__((aligned(16))) uint16_t park[2][64 * DUAL16_LDV];
+    __shared__ __attribute__((aligned(16))) int flags[2][4];
+    int64_t r0, c0;
+    if (!dual16_tile((uint32_t)(h / 64), (uint32_t)((d.qt_pitch + 63) / 64), xcd_walk, r0, c0)) return;
+    auto tile = [&](auto interior) __attribute__((always_inline)) {
+        constexpr bool INTERIOR = decltype(interior)::value;
+        uint32_t g[8], u[8], dy[8];
+        dual16_load<TIn, INTERIOR>(z, d.rows, h, 2 * h, true, r0, c0, g);
+        dual16_load<TIn, INTERIOR>(z + h, d.rows, h, 2 * h, true, r0, c0, u);
+        dual16_load<TIn, INTERIOR>(dh, d.rows, h, h, true, r0, c0, dy);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float act[2], derivative[2];
+            const float v[2] = {widen16<TIn>(dy[e] & 0xffffu), widen16<TIn>(dy[e] >> 16)};
+            gate_math(ACT, widen16<TIn>(g[e] & 0xffffu), act[0], derivative[0]);
+            gate_math(ACT, widen16<TIn>(g[e] >> 16), act[1], derivative[1]);
+            g[e] = narrow_pair<TIn>(v[0] * widen16<TIn>(u[e] & 0xffffu) * derivative[0], v[1] * widen16<TIn>(u[e] >> 16) * derivative[1]);
+            dy[e] = narrow_pair<TIn>(v[0] * act[0], v[1] * act[1]);
+        }
+        dual16_rows<TIn, TOut, INTERIOR>(d, g, r0, c0, park[0], flags[0]);
+        dual16_rows<TIn, TOut, INTERIOR>(d, dy, r0, h + c0, park[1], flags[1]);
+        if (!d.qt) return;
+        __syncthreads();
+        dual16_columns<TIn, TOut, INTERIOR>(d, r0, c0, park[0], flags[0]);
+        dual16_columns<TIn, TOut, INTERIOR>(d, r0, h + c0, park[1], flags[1]);
+    };
+    if (aligned && r0 + 64 <= d.rows) tile(std::true_type{});
+    else tile(std::false_type{});
 }
 
 // ------------------------------------------------------------------ column sums from 32-row partials
@@ -1097,6 +991,10 @@ __global__ __launch_bounds__(256, 8) void quantize_segmented16_tile64(const TIn*
 
 // ------------------------------------------------------------------ host dispatch
 template <typename TIn, typename TOut>
+static int launch_dual(const void* x, int64_t rows, int64_t cols, void* q, int64_t q_pitch, float* scale, void* qt, int64_t qt_pitch,
+                       float* scale_t, float limit, float* column_partial, int e8m0, hipStream_t stream);
+
+template <typename TIn, typename TOut>
 static int launch_quantize(const void* x, int64_t rows, int64_t cols, void* q, float* scale, int gr, int gc,
                            float limit, int transposed, int e8m0, hipStream_t stream) {
     const TIn* xp = static_cast<const TIn*>(x);
@@ -1116,12 +1014,7 @@ static int launch_quantize(const void* x, int64_t rows, int64_t cols, void* q, f
         return viola_launch_status();
     }
     if constexpr (sizeof(TIn) == 2) {
-        if (gr == 1 && gc == 32 && transposed && vec) {
-            const int64_t tiles16 = ((cols + 63) / 64) * ((rows + 127) / 128);
-            const dim3 grid16((unsigned)(tiles16 < 256 * 6 ? tiles16 : 256 * 6));
-            VIOLA_LAUNCH((quantize_dual16<TIn, TOut, false>), grid16, dim3(256), 0, stream, xp, nullptr, nullptr, qp, scale, rows, cols, limit, nullptr, e8m0, 0);
-            return viola_launch_status();
-        }
+        if (gr == 1 && gc == 32 && transposed) return launch_dual<TIn, TOut>(x, rows, cols, nullptr, cols, nullptr, q, rows, scale, limit, nullptr, e8m0, stream);
     }
     if (gr == 1 && gc == 32 && transposed) {
         const dim3 grid((unsigned)((cols + TILE_C - 1) / TILE_C), (unsigned)((rows + TILE_R - 1) / TILE_R));
@@ -1165,6 +1058,16 @@ static int launch_reencode(const void* x, const float* source_scale, int64_t row
     return viola_launch_status();
 }
 
+// One to four rounds of resident blocks (eight per compute unit): the XCD-contiguous walk measured faster (8192 x 4096: 29.7 ->
+// 27.7 us); longer launches are faster with the eight XCDs streaming one region (16384 x 4096: 68 against 76 us), shorter ones
+// leave XCDs uneven.
+static int dual16_xcd_walk(int64_t tiles) { return tiles >= 2048 && tiles <= 8192; }
+// whole tiles may skip their bounds checks and address a lane's pieces by 32-bit offsets from the tile
+static bool dual16_aligned(const Dual16& d) {
+    return d.q_pitch % 16 == 0 && d.qt_pitch % 16 == 0 && reinterpret_cast<uintptr_t>(d.q) % 16 == 0 && reinterpret_cast<uintptr_t>(d.qt) % 16 == 0 &&
+           d.q_pitch < (1ll << 24) && d.qt_pitch < (1ll << 24) && d.cols < (1ll << 24);
+}
+
 // q (row pitch q_pitch >= cols, scales of ceil(q_pitch / 32) groups per row) and qt (row pitch qt_pitch >= rows) are filled
 // with zero codes past the matrix, so that a GEMM may take the pitch as its k. Either output may be absent; the pitches
 // then still size the walk.
@@ -1175,26 +1078,11 @@ static int launch_dual(const void* x, int64_t rows, int64_t cols, void* q, int64
     const TIn* xp = static_cast<const TIn*>(x);
     if constexpr (sizeof(TIn) == 2) {
         const int64_t tiles64 = ((q_pitch + 63) / 64) * ((qt_pitch + 63) / 64);
-        if (tiles64 + 8 < (1ll << 31)) {
-            // one to four rounds of resident blocks (eight per compute unit): the XCD-contiguous walk measured faster
-            // (8192 x 4096: 29.7 -> 27.7 us); longer launches are faster with the eight XCDs streaming one region
-            // (16384 x 4096: 68 against 76 us), shorter ones leave XCDs uneven
-            const int xcd_walk = tiles64 >= 2048 && tiles64 <= 8192;
-            // whole tiles may skip their bounds checks and address a lane's pieces by 32-bit offsets from the tile
-            const int aligned = vec && q_pitch % 16 == 0 && qt_pitch % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
-                                reinterpret_cast<uintptr_t>(qt) % 16 == 0 && q_pitch < (1ll << 24) && qt_pitch < (1ll << 24);
-            VIOLA_LAUNCH((quantize_dual16_tile64<TIn, TOut>), dim3((unsigned)((tiles64 + 7) / 8 * 8)), dim3(256), 0, stream, xp,
-                         static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, rows, cols, q_pitch, qt_pitch, limit, column_partial, e8m0,
-                         xcd_walk, aligned, (int)vec);
-            return viola_launch_status();
-        }
-        if (vec && q && reinterpret_cast<uintptr_t>(q) % 8 == 0 && q_pitch == cols && qt_pitch == rows) {
-            const int64_t tiles16 = ((cols + 63) / 64) * ((rows + 127) / 128);
-            const dim3 grid16((unsigned)(tiles16 < 256 * 6 ? tiles16 : 256 * 6));
-            VIOLA_LAUNCH((quantize_dual16<TIn, TOut, true>), grid16, dim3(256), 0, stream, xp, static_cast<uint8_t*>(q), scale,
-                               static_cast<uint8_t*>(qt), scale_t, rows, cols, limit, column_partial, e8m0, 0);
-            return viola_launch_status();
-        }
+        if (tiles64 + 8 >= (1ll << 31)) return VIOLA_ETOOLARGE;
+        const Dual16 d = {static_cast<uint8_t*>(q), scale, static_cast<uint8_t*>(qt), scale_t, column_partial, rows, cols, q_pitch, qt_pitch, limit, e8m0};
+        VIOLA_LAUNCH((quantize_dual16_tile64<TIn, TOut>), dim3((unsigned)((tiles64 + 7) / 8 * 8)), dim3(256), 0, stream, xp, d, dual16_xcd_walk(tiles64),
+                     (int)(vec && dual16_aligned(d)), (int)vec);
+        return viola_launch_status();
     }
     const dim3 grid((unsigned)((q_pitch + TILE_C - 1) / TILE_C), (unsigned)((qt_pitch + TILE_R - 1) / TILE_R));
     if (grid.y > 65535) return VIOLA_ETOOLARGE;
@@ -1293,34 +1181,67 @@ extern "C" int viola_group_quantize_dual(const void* x, int x_dtype, int64_t row
                                              scale_format, stream);
 }
 
-extern "C" int viola_gated_quantize_dual(const void* z, int z_dtype, int64_t rows, int64_t cols, int activation, void* q,
-                                         void* scale, void* qt, void* scale_t, int q_dtype, int gc, float limit,
-                                         int scale_format, viola_stream_t stream_) {
+template <typename F>
+static int with_gate_types(int in_dtype, int q_dtype, int activation, F&& f) {
+    auto by_act = [&](auto in, auto out) {
+        if (activation == VIOLA_SILU) return f(in, out, std::integral_constant<int, VIOLA_SILU>{});
+        if (activation == VIOLA_GELU) return f(in, out, std::integral_constant<int, VIOLA_GELU>{});
+        return f(in, out, std::integral_constant<int, VIOLA_RELU>{});
+    };
+    auto by_out = [&](auto in) { return q_dtype == VIOLA_E4M3 ? by_act(in, e4m3_t{}) : by_act(in, e5m2_t{}); };
+    return in_dtype == VIOLA_BF16 ? by_out(bf16_t{}) : by_out(f16_t{});
+}
+
+extern "C" int viola_gated_quantize_dual_pitched(const void* z, int z_dtype, int64_t rows, int64_t cols, int activation, void* q, int64_t q_pitch,
+                                                 void* scale, void* qt, int64_t qt_pitch, void* scale_t, int q_dtype, float limit, int scale_format,
+                                                 viola_stream_t stream_) {
     hipStream_t stream = viola_enter(stream_);
     VIOLA_CHECK_ARG(scale_format == VIOLA_SCALE_F32 || scale_format == VIOLA_SCALE_E8M0);
     VIOLA_CHECK_ARG(activation == VIOLA_SILU || activation == VIOLA_GELU || activation == VIOLA_RELU);
-    VIOLA_CHECK_ARG(viola_is_fp8(q_dtype) && viola_is_float(z_dtype) && rows >= 0 && cols >= 0 && limit > 0.0f);
-    if (gc != 32 || z_dtype == VIOLA_F32 || cols % 8 != 0) return VIOLA_EUNSUPPORTED;
+    VIOLA_CHECK_ARG(viola_is_fp8(q_dtype) && viola_is_float(z_dtype) && rows >= 0 && cols >= 0 && limit > 0.0f && q_pitch >= cols && qt_pitch >= rows);
+    if (z_dtype == VIOLA_F32 || cols % 8 != 0) return VIOLA_EUNSUPPORTED;
     if (rows == 0 || cols == 0) return 0;
-    VIOLA_CHECK_ARG(z && q && scale && qt && scale_t);
-    if (reinterpret_cast<uintptr_t>(z) % 16 != 0 || reinterpret_cast<uintptr_t>(q) % 8 != 0) return VIOLA_EUNSUPPORTED;
-    if (64 * cols * 2 >= (1ll << 31)) return VIOLA_EUNSUPPORTED;            // a wavefront's 32 rows are one buffer
-    const int e8m0 = scale_format == VIOLA_SCALE_E8M0;
-    const int64_t tiles16 = ((cols + 63) / 64) * ((rows + 127) / 128);
-    const dim3 grid16((unsigned)(tiles16 < 256 * 6 ? tiles16 : 256 * 6));
-#define VIOLA_GATED_DUAL(TI, TO)                                                                                            \
-    VIOLA_LAUNCH((quantize_dual16<TI, TO, true, true>), grid16, dim3(256), 0, stream, static_cast<const TI*>(z),       \
-                       static_cast<uint8_t*>(q), static_cast<float*>(scale), static_cast<uint8_t*>(qt),                      \
-                       static_cast<float*>(scale_t), rows, cols, limit, (float*)nullptr, e8m0, activation)
-    if (q_dtype == VIOLA_E4M3) {
-        if (z_dtype == VIOLA_BF16) VIOLA_GATED_DUAL(bf16_t, e4m3_t);
-        else VIOLA_GATED_DUAL(f16_t, e4m3_t);
-    } else {
-        if (z_dtype == VIOLA_BF16) VIOLA_GATED_DUAL(bf16_t, e5m2_t);
-        else VIOLA_GATED_DUAL(f16_t, e5m2_t);
-    }
-#undef VIOLA_GATED_DUAL
-    return viola_launch_status();
+    VIOLA_CHECK_ARG(z && (q || qt) && (!q || scale) && (!qt || scale_t));
+    const int64_t tiles = ((q_pitch + 63) / 64) * ((qt_pitch + 63) / 64);
+    if (reinterpret_cast<uintptr_t>(z) % 16 != 0 || tiles + 8 >= (1ll << 31)) return VIOLA_EUNSUPPORTED;
+    const Dual16 d = {static_cast<uint8_t*>(q), static_cast<float*>(scale), static_cast<uint8_t*>(qt), static_cast<float*>(scale_t), nullptr, rows, cols,
+                      q_pitch, qt_pitch, limit, scale_format == VIOLA_SCALE_E8M0};
+    return with_gate_types(z_dtype, q_dtype, activation, [&](auto in, auto out, auto act) {
+        using TIn = decltype(in);
+        VIOLA_LAUNCH((gated_quantize_dual16<TIn, decltype(out), decltype(act)::value>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, stream,
+                     static_cast<const TIn*>(z), d, dual16_xcd_walk(tiles), (int)dual16_aligned(d));
+        return viola_launch_status();
+    });
+}
+
+extern "C" int viola_gated_quantize_dual(const void* z, int z_dtype, int64_t rows, int64_t cols, int activation, void* q,
+                                         void* scale, void* qt, void* scale_t, int q_dtype, int gc, float limit,
+                                         int scale_format, viola_stream_t stream) {
+    if (gc != 32) return VIOLA_EUNSUPPORTED;
+    if (rows > 0 && cols > 0) VIOLA_CHECK_ARG(q && qt);
+    return viola_gated_quantize_dual_pitched(z, z_dtype, rows, cols, activation, q, cols, scale, qt, rows, scale_t, q_dtype, limit, scale_format, stream);
+}
+
+extern "C" int viola_gated_backward_quantize_dual(const void* z, const void* dh, int dtype, int64_t rows, int64_t h, int activation, void* q, void* scale,
+                                                  void* qt, int64_t qt_pitch, void* scale_t, int q_dtype, float limit, float* column_partial,
+                                                  int scale_format, viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG(scale_format == VIOLA_SCALE_F32 || scale_format == VIOLA_SCALE_E8M0);
+    VIOLA_CHECK_ARG(activation == VIOLA_SILU || activation == VIOLA_GELU || activation == VIOLA_RELU);
+    VIOLA_CHECK_ARG(viola_is_fp8(q_dtype) && viola_is_float(dtype) && rows >= 0 && h >= 0 && limit > 0.0f && qt_pitch >= rows && (!column_partial || qt));
+    if (dtype == VIOLA_F32 || h % 64 != 0) return VIOLA_EUNSUPPORTED;
+    if (rows == 0 || h == 0) return 0;
+    VIOLA_CHECK_ARG(z && dh && (q || qt) && (!q || scale) && (!qt || scale_t));
+    const int64_t tiles = (h / 64) * ((qt_pitch + 63) / 64);
+    if (reinterpret_cast<uintptr_t>(z) % 16 != 0 || reinterpret_cast<uintptr_t>(dh) % 16 != 0 || tiles + 8 >= (1ll << 31)) return VIOLA_EUNSUPPORTED;
+    const Dual16 d = {static_cast<uint8_t*>(q), static_cast<float*>(scale), static_cast<uint8_t*>(qt), static_cast<float*>(scale_t), column_partial, rows, 2 * h,
+                      2 * h, qt_pitch, limit, scale_format == VIOLA_SCALE_E8M0};
+    return with_gate_types(dtype, q_dtype, activation, [&](auto in, auto out, auto act) {
+        using TIn = decltype(in);
+        VIOLA_LAUNCH((gated_backward_quantize_dual16<TIn, decltype(out), decltype(act)::value>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, stream,
+                     static_cast<const TIn*>(z), static_cast<const TIn*>(dh), h, d, dual16_xcd_walk(tiles), (int)dual16_aligned(d));
+        return viola_launch_status();
+    });
 }
 
 extern "C" int viola_column_reduce(const float* partial, int64_t parts, int64_t cols, void* out, int out_dtype,
