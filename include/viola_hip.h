@@ -115,6 +115,16 @@ int viola_fp8_transpose(const void* x, void* out, int64_t batch, int64_t rows, i
 int viola_block_transpose(const void* x, void* out, int64_t rows, int64_t cols, const void* scale, void* scale_out,
                           int gr, int gc, int scale_format, viola_stream_t stream);
 
+/* A Linear on at most 32 rows in one launch: out [m, n] = x W^T + bias, w [n, k] codes.
+ * x is bf16 / fp16, to be quantized to w's format in the kernel: grouped, with a scale per row and 32 k (viola_group_quantize),
+ * otherwise with one for the tensor, whose maximum goes to history[slot] and whose scale to scale[0] (nullable): viola_tensor_encode
+ * with delayed = 0. Or x is codes of either format with its scale(s) sx. sw: grouped, one scale per 32 x 32 block of w (both in
+ * scale_format), otherwise one. The product is viola_group_gemm's or viola_tensor_gemm's.
+ * VIOLA_EUNSUPPORTED for m > 32, k % 16 != 0, fp32 x or unaligned operands. */
+int viola_skinny_linear(const void* x, int x_dtype, const float* sx, int64_t m, int64_t k, const void* w, int w_dtype, const void* sw,
+                        int grouped, int64_t n, float limit, int scale_format, float* history, int64_t slot, float* scale,
+                        const void* bias, int bias_dtype, void* out, int out_dtype, viola_stream_t stream);
+
 /* ---------------------------------------------------------------- per-tensor scaling (`current` / `delayed`)
  * viola/nn/_linear_kernels.py:231-242 `tensor_scale` = _amax_kernel :33-46 + _scale_kernel :49-71.
  * viola_tensor_amax: maxima[i] = max |x| over part i of `parts` (NaN dropped); maxima is caller scratch of `parts`

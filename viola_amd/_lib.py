@@ -35,6 +35,7 @@ _SIGNATURES = {
     "viola_group_dequantize": [_p, _i, _p, _l, _l, _i, _i, _p, _p],
     "viola_fp8_transpose": [_p, _p, _l, _l, _l, _p],
     "viola_block_transpose": [_p, _p, _l, _l, _p, _p, _i, _i, _i, _p],
+    "viola_skinny_linear": [_p, _i, _p, _l, _l, _p, _i, _p, _i, _l, _f, _i, _p, _l, _p, _p, _i, _p, _i, _p],
     "viola_group_gemm": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _i, _i, _i, _i, _p, _i, _p, _i, _p],
     "viola_group_gemm_half": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _i, _i, _i, _i, _p, _i, _p, _i, _i, _i, _p],
     "viola_tensor_gemm_half": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _p, _i, _p, _i, _i, _i, _p],

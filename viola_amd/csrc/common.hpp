@@ -49,6 +49,8 @@ static inline int viola_dtype_size(int dtype) { return dtype == VIOLA_F32 ? 4 : 
 
 namespace viola {
 
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 constexpr int WAVE = 64;
 
 // ------------------------------------------------------------------ storage types
@@ -144,6 +146,29 @@ template <> __device__ __forceinline__ f16_t from_f32<f16_t>(float v) { return f
 template <> __device__ __forceinline__ e4m3_t from_f32<e4m3_t>(float v) { return e4m3_t{f32_to_e4m3(v)}; }
 template <> __device__ __forceinline__ e5m2_t from_f32<e5m2_t>(float v) { return e5m2_t{f32_to_e5m2(v)}; }
 
+// one element of a word of two 16-bit values
+template <typename TIn> __device__ __forceinline__ float widen16(uint32_t bits);
+template <> __device__ __forceinline__ float widen16<bf16_t>(uint32_t bits) { return __uint_as_float(bits << 16); }
+template <> __device__ __forceinline__ float widen16<f16_t>(uint32_t bits) {
+    const uint16_t b = (uint16_t)bits;
+    return (float)__builtin_bit_cast(_Float16, b);
+}
+
+template <typename TIn> __device__ __forceinline__ uint32_t narrow16(float v);
+template <> __device__ __forceinline__ uint32_t narrow16<bf16_t>(float v) { return f32_to_bf16_bits(v); }
+template <> __device__ __forceinline__ uint32_t narrow16<f16_t>(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
+
+__device__ __forceinline__ float load_float(const void* p, int64_t i, int dtype) {
+    if (dtype == VIOLA_F32) return static_cast<const float*>(p)[i];
+    if (dtype == VIOLA_BF16) return bf16_bits_to_f32(static_cast<const uint16_t*>(p)[i]);
+    return (float)static_cast<const _Float16*>(p)[i];
+}
+__device__ __forceinline__ void store_float(void* p, int64_t i, int dtype, float v) {
+    if (dtype == VIOLA_F32) static_cast<float*>(p)[i] = v;
+    else if (dtype == VIOLA_BF16) static_cast<uint16_t*>(p)[i] = f32_to_bf16_bits(v);
+    else static_cast<_Float16*>(p)[i] = (_Float16)v;
+}
+
 template <typename T> struct fp8_traits;
 template <> struct fp8_traits<e4m3_t> { static constexpr float max = 448.0f; };
 template <> struct fp8_traits<e5m2_t> { static constexpr float max = 57344.0f; };
@@ -231,6 +256,18 @@ __device__ __forceinline__ uint8_t encode_clamped(float v, float s, float limit)
     const float t = v / s;
     const float c = t != t ? t : fminf(fmaxf(t, -limit), limit);
     return from_f32<TOut>(c).bits;
+}
+
+template <typename TOut>
+__device__ __forceinline__ uint2 encode8(const float (&v)[8], float s, float limit, const SharedDivisor& d) {
+    if (d.fast) return make_uint2(fast_encode4<TOut>(d, limit, v[0], v[1], v[2], v[3]), fast_encode4<TOut>(d, limit, v[4], v[5], v[6], v[7]));
+    uint32_t lo = 0, hi = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        lo |= (uint32_t)encode_clamped<TOut>(v[i], s, limit) << (8 * i);
+        hi |= (uint32_t)encode_clamped<TOut>(v[4 + i], s, limit) << (8 * i);
+    }
+    return make_uint2(lo, hi);
 }
 
 // amax / limit, or for E8M0 scales the smallest power of two that is not below it (the reference's

@@ -61,12 +61,6 @@ __device__ __forceinline__ f32x16 mfma32(long x, long y, f32x16 c) {
     else return __builtin_amdgcn_mfma_f32_32x32x16_bf8_bf8(x, y, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float load_bias(const void* p, int64_t i, int dtype) {
-    if (dtype == VIOLA_F32) return static_cast<const float*>(p)[i];
-    if (dtype == VIOLA_BF16) return bf16_bits_to_f32(static_cast<const uint16_t*>(p)[i]);
-    return (float)static_cast<const _Float16*>(p)[i];
-}
-
 // Four consecutive outputs of one row.
 template <typename TO> struct Quad;
 template <> struct Quad<float> {
@@ -654,7 +648,7 @@ __global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 
             float4 bias_q[TN][4];
             if (p.bias) {
                 float* bias_lds = reinterpret_cast<float*>(lds + K_RAW);
-                if (tid < PANEL) bias_lds[tid] = n_begin + tid < p.n ? load_bias(p.bias, n_begin + tid, bias_dtype) : 0.0f;
+                if (tid < PANEL) bias_lds[tid] = n_begin + tid < p.n ? load_float(p.bias, n_begin + tid, bias_dtype) : 0.0f;
                 __syncthreads();
 #pragma unroll
                 for (int i = 0; i < TN; ++i)
@@ -751,8 +745,8 @@ __global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 
                 for (int r = 0; r < 16; ++r) {
                     const int64_t ncol = col0 + (r / 4) * 8 + lhi * 4 + r % 4;
                     const bool inside = p.bias && ncol < p.n;
-                    bias_g[r] = inside ? load_bias(p.bias, ncol, bias_dtype) : 0.0f;
-                    bias_u[r] = inside ? load_bias(p.bias, p.n + ncol, bias_dtype) : 0.0f;
+                    bias_g[r] = inside ? load_float(p.bias, ncol, bias_dtype) : 0.0f;
+                    bias_u[r] = inside ? load_float(p.bias, p.n + ncol, bias_dtype) : 0.0f;
                 }
 #pragma unroll
                 for (int j = 0; j < TM; ++j) {
@@ -899,8 +893,8 @@ __global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 
                 for (int e = 0; e < 4; ++e) {
                     float gv = total[0][j][r4 * 4 + e], uv = total[1][j][r4 * 4 + e];
                     if (p.bias && ncol + e < p.n) {
-                        gv += load_bias(p.bias, ncol + e, bias_dtype);
-                        uv += load_bias(p.bias, p.n + ncol + e, bias_dtype);
+                        gv += load_float(p.bias, ncol + e, bias_dtype);
+                        uv += load_float(p.bias, p.n + ncol + e, bias_dtype);
                     }
                     gq[e] = rounded<TO>(gv);
                     uq[e] = rounded<TO>(uv);
@@ -930,7 +924,7 @@ __global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 
                     if (p.bias) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            if (ncol + e < p.n) v[e] += load_bias(p.bias, ncol + e, bias_dtype);
+                            if (ncol + e < p.n) v[e] += load_float(p.bias, ncol + e, bias_dtype);
                     }
                     if (full && vec_out) Quad<TO>::store(out + mrow * p.ldo + ncol, v);
                     else for (int e = 0; e < 4; ++e) if (ncol + e < p.n) out[mrow * p.ldo + ncol + e] = from_f32<TO>(v[e]);

@@ -32,12 +32,6 @@ __device__ __forceinline__ f32x16 mfma32(long x, long y, f32x16 c) {
     else return __builtin_amdgcn_mfma_f32_32x32x16_bf8_bf8(x, y, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float load_dtype(const void* p, int64_t i, int dtype) {
-    if (dtype == VIOLA_F32) return static_cast<const float*>(p)[i];
-    if (dtype == VIOLA_BF16) return bf16_bits_to_f32(static_cast<const uint16_t*>(p)[i]);
-    return (float)static_cast<const _Float16*>(p)[i];
-}
-
 template <typename TO> __device__ __forceinline__ float round_through(float v) { return to_f32(from_f32<TO>(v)); }
 
 // A_BF8/B_BF8: operand formats (false = e4m3, true = e5m2). B_ROWSCALE: b scales vary inside a 32-row block.
@@ -286,8 +280,8 @@ __global__ __launch_bounds__(256, 2) void group_gemm_kernel(GemmArgs p, int bias
                 if (ncol >= p.n) continue;
                 float gv = total[0][j][r], uv = total[1][j][r];
                 if (p.bias) {
-                    gv += load_dtype(p.bias, ncol, bias_dtype);
-                    uv += load_dtype(p.bias, p.n + ncol, bias_dtype);
+                    gv += load_float(p.bias, ncol, bias_dtype);
+                    uv += load_float(p.bias, p.n + ncol, bias_dtype);
                 }
                 const TO gq = from_f32<TO>(gv), uq = from_f32<TO>(uv);
                 if (aux) {
@@ -311,7 +305,7 @@ __global__ __launch_bounds__(256, 2) void group_gemm_kernel(GemmArgs p, int bias
                         v = (v * p.sa[0]) * p.sb[0];
                     }
                     if constexpr (MODE == MODE_PLAIN) {
-                        if (p.bias) v += load_dtype(p.bias, ncol, bias_dtype);
+                        if (p.bias) v += load_float(p.bias, ncol, bias_dtype);
                         out[mrow * p.ldo + ncol] = from_f32<TO>(v);
                     } else {
                         const TO* aux = static_cast<const TO*>(p.aux);

@@ -211,7 +211,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     if (p.bias) {
         if (tid < S::COLS) {
             const int64_t col = n_begin + tid % PANEL;
-            bias_lds[tid] = col < p.n ? load_bias(p.bias, (GATED ? tid / PANEL * p.n : 0) + col, bias_dtype) : 0.0f;
+            bias_lds[tid] = col < p.n ? load_float(p.bias, (GATED ? tid / PANEL * p.n : 0) + col, bias_dtype) : 0.0f;
         }
         __syncthreads();
 #pragma unroll

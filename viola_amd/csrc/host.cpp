@@ -91,6 +91,11 @@ struct Kept {
 };
 
 // ---------------------------------------------------------------------------------------------------- products
+// Rows the kernel for a handful of them takes (viola_skinny_linear), and up to which k (times two past 16 rows) it quantizes x
+// itself: every block of it does so again, which beyond costs more than the quantizer's launch (measured, 4096 wide: k = 1024
+// 5.3 against 7.5 us, 4096 10.6 against 10.5, 8192 15.5 against 13.9).
+constexpr int64_t FEW_ROWS = 32, QUANTIZED_IN_PRODUCT = 3072;
+
 // out[m, n] = a b^T, k = the operands' common pitch. br: rows of b per scale row (32: weight blocks, 1: row-wise).
 void product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_fmt, int64_t m, int64_t n, int br, const Tensor& bias,
              void* out, at::ScalarType out_dtype, const at::Device& device, viola_stream_t stream) {
@@ -98,6 +103,12 @@ void product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_f
     TORCH_INTERNAL_ASSERT(b.pitch == k);
     const void* bias_p = ptr(bias);
     const int bias_code = bias_p ? code_of(bias.scalar_type()) : 0, out_code = code_of(out_dtype);
+    if (m <= FEW_ROWS && br == 32) {
+        const int status = VIOLA_TRY(viola_skinny_linear, a.q, a_fmt, static_cast<const float*>(a.s), m, k, b.q, b_fmt, b.s, r.grouped, n, r.fwd_limit,
+                                     r.scale_format(), nullptr, 0, nullptr, bias_p, bias_code, out, out_code, stream);
+        if (status == 0) return;
+        if (status != VIOLA_EUNSUPPORTED) check("viola_skinny_linear", status);
+    }
     if (!r.grouped) {
         VIOLA_CALL(viola_tensor_gemm, a.q, a_fmt, b.q, b_fmt, static_cast<const float*>(a.s), static_cast<const float*>(b.s), m, n, k, bias_p,
                    bias_code, out, out_code, stream);
@@ -286,9 +297,25 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         return f;
     }
     Arena temp;
+    const bool cache_here = !r.fp8_weight && need_backward && r.cache_transpose;   // 16-bit storage: W^T of this forward's codes
+    if (gated < 0 && rows <= FEW_ROWS && !need_backward && !coded_input && r.fp8_weight && x2.element_size() == 2 && (rows > 16 ? 2 : 1) * r.in <= QUANTIZED_IN_PRODUCT &&
+        (r.grouped || !(r.delayed && l.counter[INPUT]->value))) {
+        // a few rows, nothing kept for backward: x is quantized inside the product
+        f.y = at::empty({rows, r.out}, options);
+        const void* bias_p = ptr(l.bias);
+        float* history = r.grouped ? nullptr : static_cast<float*>(l.history[INPUT].mutable_data_ptr());
+        const int64_t slot = r.grouped ? 0 : l.counter[INPUT]->value % l.history[INPUT].numel();
+        const int status = VIOLA_TRY(viola_skinny_linear, ptr(x2), code_of(x2.scalar_type()), nullptr, rows, r.in, ptr(l.weight), r.fwd, ptr(l.scale), r.grouped,
+                                     r.out, r.fwd_limit, r.scale_format(), history, slot, nullptr, bias_p, bias_p ? code_of(l.bias.scalar_type()) : 0,
+                                     f.y.mutable_data_ptr(), code_of(dtype), stream);
+        if (status == 0) {
+            if (!r.grouped) ++l.counter[INPUT]->value;
+            return f;
+        }
+        if (status != VIOLA_EUNSUPPORTED) check("viola_skinny_linear", status);
+    }
     const WeightSpace wspace = reserve_weight(l, temp);
     Codes a, w, w_unpadded;
-    const bool cache_here = !r.fp8_weight && need_backward && r.cache_transpose;   // 16-bit storage: W^T of this forward's codes
     if (r.grouped) {
         GroupSpace g;
         if (!coded_input) g.reserve(r, &temp, save ? &kept.arena : nullptr, rows, r.in);
@@ -331,8 +358,9 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, l.bias, f.y.mutable_data_ptr(), dtype, device, stream);
         return f;
     }
-    if (keep_aux) f.aux = at::empty({rows, r.out}, options);
-    if (hidden_out && keep_aux && dtype != at::kFloat && h % 8 == 0) {
+    const bool through_z = keep_aux || (hidden_out && rows <= FEW_ROWS);     // (a few rows: the plain product has the kernel for them)
+    if (through_z) f.aux = at::empty({rows, r.out}, options);
+    if (hidden_out && through_z && dtype != at::kFloat && h % 8 == 0) {
         // [g | u] is kept for backward anyway: the plain product on the tile that suits it best, then one pass over [g | u] that
         // makes h's codes; h itself is never stored
         const Recipe& to = *hidden_out->reader;

@@ -258,28 +258,17 @@ __global__ __launch_bounds__(256) void comm_unpack_quads_table_kernel(const int6
 
 
 // ------------------------------------------------------------------ gated activations
-__device__ __forceinline__ float load_half(const void* p, int64_t i, int dtype) {
-    if (dtype == VIOLA_F32) return static_cast<const float*>(p)[i];
-    if (dtype == VIOLA_BF16) return bf16_bits_to_f32(static_cast<const uint16_t*>(p)[i]);
-    return (float)static_cast<const _Float16*>(p)[i];
-}
-__device__ __forceinline__ void store_half(void* p, int64_t i, int dtype, float v) {
-    if (dtype == VIOLA_F32) static_cast<float*>(p)[i] = v;
-    else if (dtype == VIOLA_BF16) static_cast<uint16_t*>(p)[i] = f32_to_bf16_bits(v);
-    else static_cast<_Float16*>(p)[i] = (_Float16)v;
-}
-
 __global__ __launch_bounds__(256) void gated_forward_kernel(const void* __restrict__ z, void* __restrict__ out, int64_t rows,
                                                              int64_t h, int dtype, int activation) {
     const int64_t total = rows * h;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
         const int64_t r = idx / h, c = idx % h;
-        const float g = load_half(z, r * 2 * h + c, dtype), u = load_half(z, r * 2 * h + h + c, dtype);
+        const float g = load_float(z, r * 2 * h + c, dtype), u = load_float(z, r * 2 * h + h + c, dtype);
         float a, derivative;
         // the stand-alone operator divides (viola/nn/_gated_kernels.py:29-35); the GEMM epilogues multiply by 1 / (1 + exp(-g))
         if (activation == VIOLA_SILU) a = g / (1.0f + expf(-g));
         else gate_math(activation, g, a, derivative);
-        store_half(out, idx, dtype, a * u);
+        store_float(out, idx, dtype, a * u);
     }
 }
 
@@ -289,12 +278,12 @@ __global__ __launch_bounds__(256) void gated_backward_kernel(const void* __restr
     const int64_t total = rows * h;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
         const int64_t r = idx / h, c = idx % h;
-        const float g = load_half(z, r * 2 * h + c, dtype), u = load_half(z, r * 2 * h + h + c, dtype);
-        const float d = load_half(dy, idx, dtype);
+        const float g = load_float(z, r * 2 * h + c, dtype), u = load_float(z, r * 2 * h + h + c, dtype);
+        const float d = load_float(dy, idx, dtype);
         float a, derivative;
         gate_math(activation, g, a, derivative);
-        store_half(dz, r * 2 * h + c, dtype, d * u * derivative);
-        store_half(dz, r * 2 * h + h + c, dtype, d * a);
+        store_float(dz, r * 2 * h + c, dtype, d * u * derivative);
+        store_float(dz, r * 2 * h + h + c, dtype, d * a);
     }
 }
 

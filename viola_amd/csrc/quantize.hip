@@ -45,17 +45,6 @@ template <> struct Chunk8<float> {
     }
 };
 
-template <typename TOut>
-__device__ __forceinline__ uint2 encode8(const float (&v)[8], float s, float limit, const SharedDivisor& d) {
-    if (d.fast) return make_uint2(fast_encode4<TOut>(d, limit, v[0], v[1], v[2], v[3]), fast_encode4<TOut>(d, limit, v[4], v[5], v[6], v[7]));
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        lo |= (uint32_t)encode_clamped<TOut>(v[i], s, limit) << (8 * i);
-        hi |= (uint32_t)encode_clamped<TOut>(v[4 + i], s, limit) << (8 * i);
-    }
-    return make_uint2(lo, hi);
-}
 
 // ------------------------------------------------------------------ row-wise (1, GC)
 // Requires cols % 8 == 0, x aligned to 8 elements, q aligned to 8 bytes.
@@ -206,18 +195,6 @@ __global__ __launch_bounds__(256) void quantize_tile(const TIn* __restrict__ x, 
         }
     }
 }
-
-// ------------------------------------------------------------------ 16-bit values as words of two
-template <typename TIn> __device__ __forceinline__ float widen16(uint32_t bits);
-template <> __device__ __forceinline__ float widen16<bf16_t>(uint32_t bits) { return __uint_as_float(bits << 16); }
-template <> __device__ __forceinline__ float widen16<f16_t>(uint32_t bits) {
-    const uint16_t b = (uint16_t)bits;
-    return (float)__builtin_bit_cast(_Float16, b);
-}
-
-template <typename TIn> __device__ __forceinline__ uint32_t narrow16(float v);
-template <> __device__ __forceinline__ uint32_t narrow16<bf16_t>(float v) { return f32_to_bf16_bits(v); }
-template <> __device__ __forceinline__ uint32_t narrow16<f16_t>(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
 
 // ------------------------------------------------------------------ 16-bit inputs: both layouts from a 64 x 64 tile
 // A block of 256 threads per tile, one tile per block: eight blocks are resident on a compute unit at 64 registers, and
