@@ -410,6 +410,10 @@ int viola_comm_pack(const float* x, int64_t n, void* packet, int64_t rows, int64
 int viola_comm_unpack(const void* packet, float* out, int64_t n, int64_t rows, int64_t groups, int tile, int fp8_dtype,
                       int reduce, viola_stream_t stream);
 
+/* viola_comm_pack of x[n] into one row of a packet and viola_comm_unpack of that back into x, one pass (n <= groups * tile).
+ * VIOLA_EUNSUPPORTED for x not 16-byte aligned or tiles other than 64 .. 512. */
+int viola_comm_roundtrip(float* x, int64_t n, void* packet, int64_t groups, int tile, int fp8_dtype, viola_stream_t stream);
+
 /* viola_comm_pack / viola_comm_unpack for many buckets in one launch: the reference drains its gradient buckets one
  * pack and one unpack launch at a time (viola/distributed/gradients.py:101-125 -> fp8.py:49-85), and a 25 MB bucket
  * is too short a launch to reach the memory system's streaming rate. table: device array of `buckets` rows of eight

@@ -4,6 +4,8 @@ that do not fit the table kernels."""
 import pytest
 import torch
 
+from viola_amd import _lib
+
 pytestmark = pytest.mark.gpu
 
 
@@ -52,3 +54,20 @@ def test_native_step_equals_stepping_each_parameter_alone(options):
         for key, value in one[0].state[a].items():
             other = each[i].state[b][key]
             assert torch.equal(value, other) if isinstance(value, torch.Tensor) else value == other == 3
+
+
+@pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
+@pytest.mark.parametrize("tile,n", [(64, 1), (128, 4095), (256, 70001), (512, 66048), (256, 1 << 20)])
+def test_wire_round_trip_in_one_pass_equals_pack_then_unpack(tile, n, fp8):
+    """Values and packet bytes, with a short last tile, an Inf and a NaN."""
+    torch.manual_seed(n)
+    x = torch.randn(n, device="cuda") * torch.exp2(torch.randint(-20, 20, (n,), device="cuda").float())
+    if n > 4000:
+        x[17], x[n - 1] = float("nan"), float("inf")
+    groups = -(-n // tile)
+    packets = [torch.zeros((groups * (tile + 4) + 15) // 16 * 16, device="cuda", dtype=torch.uint8) for _ in range(2)]
+    got, want = x.clone(), x.clone()
+    _lib.call("viola_comm_roundtrip", got.data_ptr(), n, packets[0].data_ptr(), groups, tile, _lib.code(fp8))
+    _lib.call("viola_comm_pack", x.data_ptr(), n, packets[1].data_ptr(), 1, groups, tile, _lib.code(fp8))
+    _lib.call("viola_comm_unpack", packets[1].data_ptr(), want.data_ptr(), n, 1, groups, tile, _lib.code(fp8), 0)
+    assert torch.equal(packets[0], packets[1]) and torch.equal(got.view(torch.int32), want.view(torch.int32))

@@ -438,6 +438,9 @@ void roundtrip(const Tensor& value, const Tensor& send, int64_t tile, py::object
     const viola_stream_t stream = stream_of(value);
     float* x = static_cast<float*>(value.mutable_data_ptr());
     void* packet = send.mutable_data_ptr();
+    const int status = VIOLA_TRY(viola_comm_roundtrip, x, value.numel(), packet, groups, (int)tile, code, stream);
+    if (status == 0) return;
+    if (status != VIOLA_EUNSUPPORTED) check("viola_comm_roundtrip", status);
     VIOLA_CALL(viola_comm_pack, x, value.numel(), packet, 1, groups, (int)tile, code, stream);
     VIOLA_CALL(viola_comm_unpack, packet, x, value.numel(), 1, groups, (int)tile, code, 0, stream);
 }
