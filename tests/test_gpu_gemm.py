@@ -372,3 +372,21 @@ def test_group_gemm_around_the_tile_counts_where_the_form_changes(m, n, k, gb):
     spell = lambda t, s, rows: t * s.repeat_interleave(rows, 0)[:t.shape[0]].repeat_interleave(32, 1)[:, :k]
     out = g.gemm(a.to(E4), b.to(E4), sa, sb, (1, 32), gb, out_dtype=torch.float32)
     assert torch.equal(out, spell(a, sa, 1) @ spell(b, sb, gb[0]).T)
+
+
+@pytest.mark.parametrize("counts", [[0] * 63 + [130, 0, 5], [1] * 65, [0, 129] * 40 + [0], [700, 0, 300]])
+def test_varlen_group_gemm_counts_its_tiles_over_more_groups_than_lanes(counts):
+    """Groups on both sides of the 64 one count covers, empty ones at every edge: integer operands, so each group's rows equal the
+    integer product with its own weight."""
+    groups, k, n, total = len(counts), 64, 300, sum(counts)
+    torch.manual_seed(groups)
+    a, b = torch.randint(-2, 3, (total, k), device="cuda").float(), torch.randint(-2, 3, (groups, n, k), device="cuda").float()
+    offsets = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], device="cuda")
+    sa, sb = torch.ones(total, k // 32, device="cuda"), torch.full((groups, -(-n // 32), k // 32), .5, device="cuda")
+    out, qa, qb = torch.full((total, n), 7.0, device="cuda"), a.to(E4), b.to(E4)
+    _lib.call("viola_varlen_group_gemm", qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E4), sa.data_ptr(), sb.data_ptr(), offsets.data_ptr(), groups,
+              total, n, k, 1, 32, 32, 32, n * k, sb[0].numel(), out.data_ptr(), 0)
+    row = 0
+    for g, c in enumerate(counts):
+        assert torch.equal(out[row:row + c], a[row:row + c] @ b[g].T * .5)
+        row += c

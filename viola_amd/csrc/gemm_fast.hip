@@ -71,7 +71,7 @@ int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dt
     const bool split = few && tiles > 128 && fixed_k && p.k >= SPLIT_MIN_K;
     const bool narrow = few && !split && p.n > 64;
     if (narrow) grid.x = (unsigned)((p.n + 63) / 64);
-    if (!p.offsets && (int64_t)grid.x * grid.y < (1 << 30)) {
+    if ((int64_t)grid.x * grid.y < (1 << 30)) {
         p.tiles_n = (int)grid.x;
         p.tiles_m = (int)grid.y;
         grid = dim3((grid.x * grid.y + 7) / 8 * 8, 1, grid.z);

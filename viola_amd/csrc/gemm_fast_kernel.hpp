@@ -89,6 +89,19 @@ template <> struct Quad<f16_t> {
     }
 };
 
+// Row tiles of group base + lane, and of all groups base .. base + lane together (groups past the last have none).
+__device__ __forceinline__ void group_scan(const GemmArgs& p, int base, int& tiles, int& end) {
+    const int lane = threadIdx.x % WAVE, g = base + lane;
+    tiles = 0;
+    if (g < p.groups) tiles = (int)((p.offsets[g + 1] - p.offsets[g] + BM - 1) / BM);
+    end = tiles;
+#pragma unroll
+    for (int step = 1; step < WAVE; step *= 2) {
+        const int below = __shfl_up(end, step, WAVE);
+        if (lane >= step) end += below;
+    }
+}
+
 // A finished 16-byte piece of the output, stored with the streaming hint: nothing in this launch reads it again, and
 // kept out of the way it does not push the operand panels that the tiles of an XCD share out of its L2 (8192 x 4096 x
 // 1024 with a 64 MB output: 85 -> 80 us).
@@ -151,14 +164,26 @@ __global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 
     // Workgroups are dealt round-robin to the 8 XCDs (block i -> XCD i % 8), each with its own L2. Give every XCD a
     // contiguous range of output tiles, walked in groups of 8 m tiles x all n tiles (n slowest inside a group), so the
     // blocks resident on one XCD at a time share a few rows of a and b.
-    int tile_m = blockIdx.y, tile_n = blockIdx.x;
+    // Variable groups: the launcher knows only a bound on the row tiles; every wavefront counts them from the offsets (a lane per
+    // group), so the walk covers the tiles there are and all XCDs get the same share of them.
+    int tile_m = blockIdx.y, tile_n = blockIdx.x, tiles_m = p.tiles_m;
+    int group_tiles = 0, group_end = 0;                                      // of the lane's group (the first 64)
+    if (p.offsets) {
+        tiles_m = 0;
+        for (int base = 0; base < p.groups; base += WAVE) {
+            int count, end;
+            group_scan(p, base, count, end);
+            if (base == 0) { group_tiles = count; group_end = end; }
+            tiles_m += __builtin_amdgcn_readlane(end, WAVE - 1);
+        }
+    }
     if (p.tiles_m) {
-        const int per_xcd = gridDim.x / 8;
-        const int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-        if (t >= p.tiles_m * p.tiles_n) return;
+        const int per_xcd = p.offsets ? (int)(((int64_t)tiles_m * p.tiles_n + 7) / 8) : (int)(gridDim.x / 8);
+        const int seq = blockIdx.x / 8, t = (blockIdx.x % 8) * per_xcd + seq;
+        if (seq >= per_xcd || t >= tiles_m * p.tiles_n) return;
         const int group = 8 * p.tiles_n;
         const int first_m = t / group * 8;
-        const int rows = p.tiles_m - first_m < 8 ? p.tiles_m - first_m : 8;
+        const int rows = tiles_m - first_m < 8 ? tiles_m - first_m : 8;
         tile_m = first_m + t % group % rows;
         tile_n = t % group / rows;
     }
@@ -168,16 +193,21 @@ __global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 
     const float* sbptr = p.sb;
     uint8_t* outptr = static_cast<uint8_t*>(p.out);
     if (p.offsets) {
-        int64_t tile = tile_m;
-        int g = 0;
-        bool found = false;
-        for (; g < p.groups; ++g) {
-            const int64_t lo = p.offsets[g], hi = p.offsets[g + 1];
-            const int64_t tiles = (hi - lo + BM - 1) / BM;
-            if (tile < tiles) { m_begin = lo + tile * BM; m_end = hi; found = true; break; }
-            tile -= tiles;
+        if (tile_m >= tiles_m) return;
+        int tile = tile_m, g = 0;
+        for (int base = 0;; base += WAVE) {                                  // ends: tile_m is one of the tiles counted above
+            if (base) group_scan(p, base, group_tiles, group_end);
+            const uint64_t past = __builtin_amdgcn_ballot_w64(tile < group_end);
+            if (past) {
+                const int at = __builtin_ctzll(past);
+                tile -= __builtin_amdgcn_readlane(group_end - group_tiles, at);
+                g = base + at;
+                break;
+            }
+            tile -= __builtin_amdgcn_readlane(group_end, WAVE - 1);
         }
-        if (!found) return;
+        m_begin = p.offsets[g] + (int64_t)tile * BM;
+        m_end = p.offsets[g + 1];
         bptr += (int64_t)g * p.b_group_stride;
         sbptr += (int64_t)g * p.sb_group_stride;
     }
