@@ -24,6 +24,8 @@
 //     LDS as 16-byte pieces.
 //   * work order: the 1-D grid is cut into eight contiguous ranges, one per XCD (blockIdx % 8), and
 //     inside a range tiles walk n fastest, so the tiles that share an a panel meet in one L2.
+#include <type_traits>
+
 #include "ns_args.hpp"
 
 namespace viola {
@@ -236,50 +238,92 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void ns_gemm_fast(NsArgs
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    auto compute = [&](const uint16_t* stage) {
+    // the operands of 16 k of a stage
+    auto fetch = [&](const uint16_t* stage, int ks, uint4 (&opa)[WM], uint4 (&opb)[WN]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int ks = 0; ks < SBK / 16; ++ks) {
-            uint4 opa[WM], opb[WN];
-#pragma unroll
-            for (int i = 0; i < WN; ++i) {
-                if constexpr (B_KN) {
-                    // i * 32 columns = 4 units further along the row: the swizzle only touches bits the
-                    // lane's own term already fixed modulo 8 units when 4 i stays below 8, so add it before
-                    // the XOR would be wrong; the unit index is rebuilt instead
-                    const int unit = ((wn * 4 * WN + i * 4 + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (BN % 128 == 0 ? (kn_row & 3) * 4 : ((kn_row >> 1) & 1) * 4));
-                    const uint16_t* at = stage + A_EL + (kn_row + ks * 16) * BN + unit * 8 + 4 * (lane & 1);
-                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
-                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * BN));
-                    const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-                    opb[i] = make_uint4(l2.x, l2.y, h2.x, h2.y);
-                } else {
-                    opb[i] = *reinterpret_cast<const uint4*>(stage + ((b_frag + i * 32 * SBK) ^ (ks * 16)));
-                }
+        for (int i = 0; i < WN; ++i) {
+            if constexpr (B_KN) {
+                // i * 32 columns = 4 units further along the row: the swizzle only touches bits the
+                // lane's own term already fixed modulo 8 units when 4 i stays below 8, so add it before
+                // the XOR would be wrong; the unit index is rebuilt instead
+                const int unit = ((wn * 4 * WN + i * 4 + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (BN % 128 == 0 ? (kn_row & 3) * 4 : ((kn_row >> 1) & 1) * 4));
+                const uint16_t* at = stage + A_EL + (kn_row + ks * 16) * BN + unit * 8 + 4 * (lane & 1);
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * BN));
+                const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+                opb[i] = make_uint4(l2.x, l2.y, h2.x, h2.y);
+            } else {
+                opb[i] = *reinterpret_cast<const uint4*>(stage + ((b_frag + i * 32 * SBK) ^ (ks * 16)));
             }
-#pragma unroll
-            for (int j = 0; j < WM; ++j) opa[j] = *reinterpret_cast<const uint4*>(stage + ((a_frag + j * 32 * SBK) ^ (ks * 16)));
-#pragma unroll
-            for (int i = 0; i < WN; ++i)
-#pragma unroll
-                for (int j = 0; j < WM; ++j) acc[i][j] = ns_mfma<IS_BF16>(opb[i], opa[j], acc[i][j]);
         }
+#pragma unroll
+        for (int j = 0; j < WM; ++j) opa[j] = *reinterpret_cast<const uint4*>(stage + ((a_frag + j * 32 * SBK) ^ (ks * 16)));
+    };
+    auto multiply = [&](const uint4 (&opa)[WM], const uint4 (&opb)[WN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < WN; ++i)
+#pragma unroll
+            for (int j = 0; j < WM; ++j) acc[i][j] = ns_mfma<IS_BF16>(opb[i], opa[j], acc[i][j]);
     };
 
     const int64_t chunks = (k + SBK - 1) / SBK;
     constexpr int AHEAD = STAGES - 1;                                   // chunks in flight beyond the one being multiplied
 #pragma unroll
     for (int c = 0; c < AHEAD; ++c) issue((int64_t)c * SBK, c);
-    int cur = 0, fill = AHEAD;
-    for (int64_t c = 0; c < chunks; ++c) {
-        // all loads but those of the newest AHEAD - 1 chunks have landed: chunk c is in LDS for this wave ...
-        constexpr int IN_FLIGHT = (AHEAD - 1) * (A_LOADS + B_LOADS);  // vmcnt: low four bits, two more in bits 14..15
+    auto landed = [](auto count) __attribute__((always_inline)) {            // all but the newest `count` loads; vmcnt: low four bits, two more in bits 14..15
+        constexpr int IN_FLIGHT = decltype(count)::value;
         static_assert(IN_FLIGHT < 64, "the count fits the wait instruction");
         __builtin_amdgcn_s_waitcnt(0x0F70 | (IN_FLIGHT & 15) | ((IN_FLIGHT >> 4) << 14));
-        __syncthreads();                    // ... and for every wave; stage `fill` was last read in chunk c-1
-        issue((c + AHEAD) * SBK, fill);     // past the end: zeros into a stage nobody reads
-        compute(lds + cur * STAGE_EL);
-        cur = cur == STAGES - 1 ? 0 : cur + 1;
-        fill = fill == STAGES - 1 ? 0 : fill + 1;
+    };
+    constexpr int LOADS = A_LOADS + B_LOADS;
+    if constexpr (WM * WN == 1 && !B_KN) {
+        // One accumulator per wave and one block per CU: nothing else hides the LDS reads, which take longer than the four dependent
+        // MFMAs of a chunk (a 64 x 64 tile reads 32 KB per chunk, 256 clocks). The next chunk's operands are read under this one's
+        // math: r = x x^T of a 1024 x 1024 matrix 7.4 -> 6.6 us, 1088 x 2432 12.8 -> 10.1, 256 x 2176 10.9 -> 8.8. (A [k, n] operand's
+        // transposing reads are shorter than its math; there it costs 0.1 us.)
+        static_assert(STAGES >= 4, "chunk c + AHEAD goes where chunk c - 1 was, whose reads were over a chunk ago");
+        constexpr int KS = SBK / 16;
+        uint4 opa[2][KS][WM], opb[2][KS][WN];
+        landed(std::integral_constant<int, (AHEAD - 1) * LOADS>{});
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) fetch(lds, ks, opa[0][ks], opb[0][ks]);
+        int next = 1, fill = AHEAD;
+        auto step = [&](int64_t c, auto parity) __attribute__((always_inline)) {
+            constexpr int P = decltype(parity)::value;
+            landed(std::integral_constant<int, (AHEAD - 2) * LOADS>{});      // chunk c + 1 is in LDS
+            __syncthreads();
+            issue((c + AHEAD) * SBK, fill);                                  // past the end: zeros into a stage whose content nobody uses
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) fetch(lds + next * STAGE_EL, ks, opa[1 - P][ks], opb[1 - P][ks]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) multiply(opa[P][ks], opb[P][ks]);
+            next = next == STAGES - 1 ? 0 : next + 1;
+            fill = fill == STAGES - 1 ? 0 : fill + 1;
+        };
+        int64_t c = 0;
+        for (; c + 1 < chunks; c += 2) {
+            step(c, std::integral_constant<int, 0>{});
+            step(c + 1, std::integral_constant<int, 1>{});
+        }
+        if (c < chunks) step(c, std::integral_constant<int, 0>{});
+    } else {
+        int cur = 0, fill = AHEAD;
+        for (int64_t c = 0; c < chunks; ++c) {
+            // all loads but those of the newest AHEAD - 1 chunks have landed: chunk c is in LDS for this wave ...
+            landed(std::integral_constant<int, (AHEAD - 1) * LOADS>{});
+            __syncthreads();                    // ... and for every wave; stage `fill` was last read in chunk c-1
+            issue((c + AHEAD) * SBK, fill);     // past the end: zeros into a stage nobody reads
+#pragma unroll
+            for (int ks = 0; ks < SBK / 16; ++ks) {
+                uint4 opa[WM], opb[WN];
+                fetch(lds + cur * STAGE_EL, ks, opa, opb);
+                multiply(opa, opb);
+            }
+            cur = cur == STAGES - 1 ? 0 : cur + 1;
+            fill = fill == STAGES - 1 ? 0 : fill + 1;
+        }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);     // drain the trailing loads before the LDS allocation is released
 
