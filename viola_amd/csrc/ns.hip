@@ -314,13 +314,16 @@ __global__ __launch_bounds__(256) void ns_scale16_kernel(const TIn* __restrict__
                                                           const float* __restrict__ workspace, int64_t count) {
     __shared__ float denom_s;
     const int64_t bz = blockIdx.y;
-    const float denom = ns_denominator(workspace, bz, IS_BF16, &denom_s);
-    const SharedDivisor divisor(denom, 0.0f);
     const uint4* src = reinterpret_cast<const uint4*>(in + bz * count);
     uint4* dst = reinterpret_cast<uint4*>(out + bz * count);
-    const int64_t octets = count / 8;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < octets; i += (int64_t)gridDim.x * 256) {
-        const uint4 raw = src[i];
+    const int64_t octets = count / 8, step = (int64_t)gridDim.x * 256;
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    uint4 next = i < octets ? src[i] : make_uint4(0, 0, 0, 0);               // under way while the denominator is formed
+    const float denom = ns_denominator(workspace, bz, IS_BF16, &denom_s);
+    const SharedDivisor divisor(denom, 0.0f);
+    for (; i < octets; i += step) {
+        const uint4 raw = next;
+        if (i + step < octets) next = src[i + step];
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
         uint32_t o[4];
 #pragma unroll
@@ -463,6 +466,13 @@ static int launch_ns(const void* a, const void* b, const void* residual, void* o
     return viola_launch_status();
 }
 
+// Blocks per matrix of the scaling pass: a piece per thread while that is a few rounds of blocks (a single matrix of a million
+// values: one round over all CUs, 6.8 -> 4.6 us), four per thread for the large batches.
+static unsigned ns_scale_blocks(int64_t octets, int64_t batch) {
+    const int64_t blocks = (octets + 255) / 256, wanted = blocks * batch <= 2048 ? blocks : octets / 256 / 4;
+    return (unsigned)(wanted < 1 ? 1 : wanted > 4096 ? 4096 : wanted);
+}
+
 template <typename TIn, bool IS_BF16>
 static int launch_prepare(const void* in, void* out, int64_t batch, int64_t rows, int64_t cols, float* workspace,
                           hipStream_t stream) {
@@ -476,7 +486,7 @@ static int launch_prepare(const void* in, void* out, int64_t batch, int64_t rows
                 VIOLA_LAUNCH((ns_scale16_transposed_kernel<TIn, IS_BF16>), tgrid, dim3(256), 0, stream, src, static_cast<uint16_t*>(out), workspace, rows, cols);
             } else {
                 const int64_t octets = rows * cols / 8;
-                const unsigned bx = (unsigned)(octets / 256 / 4 < 1 ? 1 : octets / 256 / 4 > 4096 ? 4096 : octets / 256 / 4);
+                const unsigned bx = ns_scale_blocks(octets, batch);
                 VIOLA_LAUNCH((ns_scale16_kernel<TIn, IS_BF16>), dim3(bx, (unsigned)batch), dim3(256), 0, stream, src, static_cast<uint16_t*>(out), workspace, rows * cols);
             }
             return viola_launch_status();
@@ -487,7 +497,7 @@ static int launch_prepare(const void* in, void* out, int64_t batch, int64_t rows
         if (aligned && (rows * cols) % 8 == 0 && rows <= cols) {
             VIOLA_LAUNCH((ns_sumsq32_kernel<IS_BF16>), dim3(PARTS, (unsigned)batch), dim3(256), 0, stream, src, workspace, rows * cols);
             const int64_t octets = rows * cols / 8;
-            const unsigned bx = (unsigned)(octets / 256 / 4 < 1 ? 1 : octets / 256 / 4 > 4096 ? 4096 : octets / 256 / 4);
+            const unsigned bx = ns_scale_blocks(octets, batch);
             VIOLA_LAUNCH((ns_scale32_kernel<IS_BF16>), dim3(bx, (unsigned)batch), dim3(256), 0, stream, src, static_cast<uint16_t*>(out), workspace, rows * cols);
             return viola_launch_status();
         }

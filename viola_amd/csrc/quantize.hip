@@ -1002,7 +1002,9 @@ static int launch_quantize(const void* x, int64_t rows, int64_t cols, void* q, f
     if (gr == 32 && gc == 32 && !transposed && cols % 4 == 0 && reinterpret_cast<uintptr_t>(x) % (4 * sizeof(TIn)) == 0 &&
         reinterpret_cast<uintptr_t>(q) % 4 == 0) {
         const int64_t units = (rows + 31) / 32 * ((cols + 127) / 128);
-        VIOLA_LAUNCH((quantize_block32<TIn, TOut>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, stream, xp, qp, scale,
+        // a wavefront per block while that is all the CUs get (1024 x 1024: 64 blocks of four -> 256 of one, 7.0 -> 5.8 us)
+        const int waves = units <= 1024 ? 1 : 4;
+        VIOLA_LAUNCH((quantize_block32<TIn, TOut>), dim3((unsigned)((units + waves - 1) / waves)), dim3(64 * waves), 0, stream, xp, qp, scale,
                            rows, cols, (cols + 31) / 32, limit, e8m0);
         return viola_launch_status();
     }

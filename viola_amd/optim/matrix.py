@@ -2,7 +2,12 @@
 (viola/optim/matrix.py:14-135, plain-tensor path). One GPU: DTensor parameters, owner
 gather/scatter and mesh all-reduces of the reference are not part of this build."""
 
+import functools
+from itertools import chain
+
 import torch
+from torch.autograd import profiler
+from torch.optim.optimizer import _global_optimizer_post_hooks, _global_optimizer_pre_hooks
 
 
 class MatrixOptimizer(torch.optim.Optimizer):
@@ -17,6 +22,39 @@ class MatrixOptimizer(torch.optim.Optimizer):
         super().__init__(params, defaults)
         self.register_load_state_dict_pre_hook(self._before_load)
         self.register_load_state_dict_post_hook(self._after_load)
+
+    @staticmethod
+    def profile_hook_step(func):
+        """The stock wrapper of `step` (hooks before and after, a profiler range around) without the range while no profiler
+        runs: entering and leaving one costs about 6 us of host time, which a small model's step waits for."""
+        recorded = torch.optim.Optimizer.profile_hook_step(func)
+
+        @functools.wraps(func)
+        def wrapper(self, *args, **kwargs):
+            if profiler._is_profiler_enabled:
+                return recorded(self, *args, **kwargs)
+            args = (self, *args)
+            for hook in chain(_global_optimizer_pre_hooks.values(), self._optimizer_step_pre_hooks.values()):
+                result = hook(self, args, kwargs)
+                if result is not None:
+                    if not (isinstance(result, tuple) and len(result) == 2):
+                        raise RuntimeError(f"{func} must return None or a tuple of (new_args, new_kwargs), but got {result}.")
+                    args, kwargs = result
+            out = func(*args, **kwargs)
+            self._optimizer_step_code()
+            for hook in chain(self._optimizer_step_post_hooks.values(), _global_optimizer_post_hooks.values()):
+                hook(self, args, kwargs)
+            return out
+
+        return wrapper
+
+    def zero_grad(self, set_to_none=True):
+        if not set_to_none or profiler._is_profiler_enabled:
+            return super().zero_grad(set_to_none)
+        for group in self.param_groups:
+            for param in group["params"]:
+                if param.grad is not None:
+                    param.grad = None
 
     def _step_local(self, parameter, gradient, state, group, index):
         raise NotImplementedError
