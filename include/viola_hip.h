@@ -115,12 +115,13 @@ int viola_fp8_transpose(const void* x, void* out, int64_t batch, int64_t rows, i
 int viola_block_transpose(const void* x, void* out, int64_t rows, int64_t cols, const void* scale, void* scale_out,
                           int gr, int gc, int scale_format, viola_stream_t stream);
 
-/* A Linear on at most 32 rows in one launch: out [m, n] = x W^T + bias, w [n, k] codes.
+/* A small Linear in one launch (at most 32 rows, or at most 256 tiles of 32 x 32 of output): out [m, n] = x W^T + bias, w [n, k] codes.
  * x is bf16 / fp16, to be quantized to w's format in the kernel: grouped, with a scale per row and 32 k (viola_group_quantize),
  * otherwise with one for the tensor, whose maximum goes to history[slot] and whose scale to scale[0] (nullable): viola_tensor_encode
  * with delayed = 0. Or x is codes of either format with its scale(s) sx. sw: grouped, one scale per 32 x 32 block of w (both in
  * scale_format), otherwise one. The product is viola_group_gemm's or viola_tensor_gemm's.
- * VIOLA_EUNSUPPORTED for m > 32, k % 16 != 0, fp32 x or unaligned operands. */
+ * VIOLA_EUNSUPPORTED for larger outputs (16-bit x: past 32 rows already from 256 tiles of 16 x 32), k % 16 != 0, fp32 x or unaligned
+ * operands. */
 int viola_skinny_linear(const void* x, int x_dtype, const float* sx, int64_t m, int64_t k, const void* w, int w_dtype, const void* sw,
                         int grouped, int64_t n, float limit, int scale_format, float* history, int64_t slot, float* scale,
                         const void* bias, int bias_dtype, void* out, int out_dtype, viola_stream_t stream);

@@ -1,9 +1,9 @@
-// A Linear applied to a handful of rows (decoding): out [m, n] = x W^T + bias with x quantized on the way in, one launch.
+// Linear products too small to fill the chip with tiles of 128 x 64 (decoding, short sequences, narrow layers): out [m, n] = x W^T +
+// bias on tiles of 16 or 32 a side whose k range all waves of a block share, x quantized on the way in where that pays.
 #include "common.hpp"
 
 namespace viola {
 
-constexpr int SKINNY_ROWS = 32;
 // Most waves of a block: with two tiles of either kind a lane needs more than a quarter of the registers.
 constexpr int skinny_waves(int mt, int nt) { return mt * nt == 1 ? 16 : 8; }
 
@@ -96,16 +96,18 @@ __device__ __forceinline__ void skinny_encode(const uint4 (&raw)[2], float s, fl
 }
 
 // What bounds it: one read of W, and below about 16 MB of W the latency of a launch that reads anything at all. So nothing is
-// staged: a block owns 16 NT rows of W, its waves a share of k each, and a lane loads its 16-byte pieces of W and its 16 values of
+// staged: a block owns a tile of 16 MT x 16 NT, its waves a share of k each, and a lane loads its 16-byte pieces of W and its 16 values of
 // x straight into registers, the next step's loads in flight under the arithmetic of this one. A step is 64 k: lane l has row
 // l % 16, k 16 (l / 16) .. + 15 of both operands, so one exchange between the half waves puts the first scale group into one
-// v_mfma_f32_16x16x32 and the second into another (k in the same new order on both sides). Every block quantizes all of x for
-// itself, m values per row of W read, which is why m stops at 32. A lane quantizes the row of x whose column of the result it
+// v_mfma_f32_16x16x32 and the second into another (k in the same new order on both sides). Every block quantizes its rows
+// of x for itself, which is why it has few of them. A lane quantizes the row of x whose column of the result it
 // accumulates, so scales stay in their lanes. The waves' sums meet in LDS.
 //   GROUPED: a scale per row and 32 k of x and per 32 x 32 block of W (FP32 or E8M0), applied as acc * (sx sw) per group.
 //   else one scale per tensor: acc runs through, (sum * sx) * sw at the end. CODED: x arrives as codes with its scale; otherwise
 //   every block takes the maximum of x (the launcher bounds its size) and block 0 records it.
-// 8 x 1024 -> 4096, grouped: 2.3 (quantizer) + 9.9 -> 5.3 us.
+// 8 x 1024 -> 4096, grouped: 2.3 (quantizer) + 9.9 -> 5.3 us. As codes, against 128 x 64 tiles with their k split in two:
+// 256 x 4096 -> 256 grouped 22.2 -> 8.9 us, per-tensor 11.9 -> 6.9; 64 x 1024 -> 1024 9.2 -> 4.4 and 6.2 -> 4.1; 128 x 4096 -> 2048 22.5 ->
+// 15.3 and 11.9 -> 10.5.
 // TIn: type of x's values (CODED: its format, TX); TX, TW: formats of the two operands.
 template <typename TIn, typename TX, typename TW, bool GROUPED, int MT, int NT>
 __global__ __launch_bounds__(64 * skinny_waves(MT, NT)) void skinny_linear(const SkinnyArgs p) {
@@ -118,6 +120,7 @@ __global__ __launch_bounds__(64 * skinny_waves(MT, NT)) void skinny_linear(const
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int l16 = lane & 15, quarter = lane >> 4;
     const int64_t n0 = (int64_t)blockIdx.x * 16 * NT;
+    const int m0 = (int)blockIdx.y * 16 * MT;
     const int64_t steps = (p.k + 63) / 64, begin = steps * wave / waves, end = steps * (wave + 1) / waves;
 
     const uint8_t* wrow[NT];
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(64 * skinny_waves(MT, NT)) void skinny_linear(const
     int64_t xscale[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-        const int64_t row = 16 * t + l16 < p.m ? 16 * t + l16 : p.m - 1;
+        const int64_t row = m0 + 16 * t + l16 < p.m ? m0 + 16 * t + l16 : p.m - 1;
         xrow[t] = static_cast<const uint8_t*>(p.x) + row * p.k * XB;
         xscale[t] = row;
     }
@@ -183,7 +186,7 @@ __global__ __launch_bounds__(64 * skinny_waves(MT, NT)) void skinny_linear(const
         __syncthreads();
         for (int i = 0; i < waves; ++i) amax = fmaxf(amax, part[i]);
         s_tensor = scale_of(amax, p.limit);
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (blockIdx.x + blockIdx.y == 0 && threadIdx.x == 0) {
             if (p.scale) p.scale[0] = s_tensor;
             p.history[p.slot] = amax;
         }
@@ -284,7 +287,7 @@ __global__ __launch_bounds__(64 * skinny_waves(MT, NT)) void skinny_linear(const
         f32x4_t v = {0, 0, 0, 0};
         for (int i = 0; i < waves; ++i) v += sums[(i * MT * NT + tile) * WAVE + lane];
         // lane l: row l % 16 of x, columns 4 (l / 16) .. + 3 of the tile
-        const int row = tile / NT * 16 + l16;
+        const int row = m0 + tile / NT * 16 + l16;
         const int64_t col = n0 + tile % NT * 16 + quarter * 4;
         if (row >= p.m || col >= p.n) continue;
         float f[4];
@@ -296,24 +299,35 @@ __global__ __launch_bounds__(64 * skinny_waves(MT, NT)) void skinny_linear(const
         }
         const int64_t at = (int64_t)row * p.n + col;
         if (p.n % 4 == 0 && p.out_dtype == VIOLA_BF16) *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + at) = make_uint2(f32_to_bf16x2_bits(f[0], f[1]), f32_to_bf16x2_bits(f[2], f[3]));
+        else if (p.n % 4 == 0 && p.out_dtype == VIOLA_F16) *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + at) = make_uint2(narrow16<f16_t>(f[0]) | narrow16<f16_t>(f[1]) << 16, narrow16<f16_t>(f[2]) | narrow16<f16_t>(f[3]) << 16);
         else for (int r = 0; r < 4 && col + r < p.n; ++r) store_float(p.out, at + r, p.out_dtype, f[r]);
     }
 }
 
+// The tile: the smallest that leaves one block per CU (256). Past that a second round of blocks reads W and x again and larger
+// tiles from LDS win (256 x 4096 -> 1024: 32 x 32 tiles 28 us per round pair, 128 x 64 tiles 22 us), except for up to 32 rows,
+// where those would be mostly padding. False: not this kernel.
+static bool skinny_tile(int64_t m, int64_t n, int& mt, int& nt) {
+    auto fits = [&](int rows, int cols) { return ((m + 16 * rows - 1) / (16 * rows)) * ((n + 16 * cols - 1) / (16 * cols)) <= 256; };
+    mt = nt = 1;
+    if (fits(1, 1)) return true;
+    nt = 2;
+    if (fits(1, 2)) return true;
+    mt = m > 16 ? 2 : 1;
+    return fits(2, 2) || m <= 32;
+}
+
 template <typename TIn, typename TX, typename TW, bool GROUPED>
-static int launch_skinny(const SkinnyArgs& p, hipStream_t stream) {
-    // Rows of W per block: 16 until that fills the CUs twice over, then 32, which halves the work of quantizing x. Waves: two
-    // steps of k for each (one while there are few blocks).
-    const int nt = p.n >= 8192 ? 2 : 1, mt = p.m > 16 ? 2 : 1;
-    const int64_t blocks = (p.n + 16 * nt - 1) / (16 * nt), steps = (p.k + 63) / 64;
+static int launch_skinny(const SkinnyArgs& p, int mt, int nt, hipStream_t stream) {
+    // waves: two steps of k for each (one while there are few blocks)
+    const int64_t blocks_n = (p.n + 16 * nt - 1) / (16 * nt), blocks_m = (p.m + 16 * mt - 1) / (16 * mt), steps = (p.k + 63) / 64;
     int waves = skinny_waves(mt, nt);
-    while (waves > 1 && steps < waves * (blocks < 128 ? 1 : 2)) waves /= 2;
-    const dim3 grid((unsigned)blocks), block((unsigned)(64 * waves));
+    while (waves > 1 && steps < waves * (blocks_n * blocks_m < 128 ? 1 : 2)) waves /= 2;
+    const dim3 grid((unsigned)blocks_n, (unsigned)blocks_m), block((unsigned)(64 * waves));
     const size_t lds = (size_t)waves * mt * nt * 1024;
 #define VIOLA_SKINNY(MT, NT) VIOLA_LAUNCH((skinny_linear<TIn, TX, TW, GROUPED, MT, NT>), grid, block, lds, stream, p)
     if (mt == 1 && nt == 1) VIOLA_SKINNY(1, 1);
     else if (mt == 1) VIOLA_SKINNY(1, 2);
-    else if (nt == 1) VIOLA_SKINNY(2, 1);
     else VIOLA_SKINNY(2, 2);
 #undef VIOLA_SKINNY
     return viola_launch_status();
@@ -332,7 +346,8 @@ extern "C" int viola_skinny_linear(const void* x, int x_dtype, const float* sx, 
     VIOLA_CHECK_ARG(m >= 0 && n >= 0 && k >= 0 && limit > 0.0f && (scale_format == VIOLA_SCALE_F32 || scale_format == VIOLA_SCALE_E8M0));
     if (m == 0 || n == 0) return 0;
     VIOLA_CHECK_ARG(out && sw && (k == 0 || (x && w)));
-    if (m > SKINNY_ROWS || k == 0 || k % 16 != 0 || k >= (1 << 30) || n >= (1ll << 31) || x_dtype == VIOLA_F32 ||
+    int mt, nt;
+    if (m > 4096 || !skinny_tile(m, n, mt, nt) || (!coded && m > 32 && mt > 1) || k == 0 || k % 16 != 0 || k >= (1 << 30) || n >= (1ll << 31) || x_dtype == VIOLA_F32 ||
         reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 8 != 0 ||
         (grouped && (reinterpret_cast<uintptr_t>(sw) % 8 != 0 || reinterpret_cast<uintptr_t>(sx) % 8 != 0)))
         return VIOLA_EUNSUPPORTED;
@@ -346,7 +361,7 @@ extern "C" int viola_skinny_linear(const void* x, int x_dtype, const float* sx, 
         using TIn = decltype(in);
         using TX = decltype(x_format);
         using TW = decltype(w_format);
-        return grouped ? launch_skinny<TIn, TX, TW, true>(p, stream) : launch_skinny<TIn, TX, TW, false>(p, stream);
+        return grouped ? launch_skinny<TIn, TX, TW, true>(p, mt, nt, stream) : launch_skinny<TIn, TX, TW, false>(p, mt, nt, stream);
     };
     auto by_weight = [&](auto x_format) { return w_dtype == VIOLA_E4M3 ? launch(x_format, x_format, e4m3_t{}) : launch(x_format, x_format, e5m2_t{}); };
     auto by_format = [&](auto in) { return w_dtype == VIOLA_E4M3 ? launch(in, e4m3_t{}, e4m3_t{}) : launch(in, e5m2_t{}, e5m2_t{}); };

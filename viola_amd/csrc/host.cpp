@@ -91,10 +91,12 @@ struct Kept {
 };
 
 // ---------------------------------------------------------------------------------------------------- products
-// Rows the kernel for a handful of them takes (viola_skinny_linear), and up to which k (times two past 16 rows) it quantizes x
-// itself: every block of it does so again, which beyond costs more than the quantizer's launch (measured, 4096 wide: k = 1024
-// 5.3 against 7.5 us, 4096 10.6 against 10.5, 8192 15.5 against 13.9).
-constexpr int64_t FEW_ROWS = 32, QUANTIZED_IN_PRODUCT = 3072;
+// Outputs the kernel for small products may take (viola_skinny_linear decides), and up to which k (times two where a block has 32
+// rows) it quantizes x itself: every block does so again, which beyond costs more than the quantizer's launch (measured, 8 rows,
+// 4096 wide: k = 1024 5.3 against 7.5 us, 4096 10.6 against 10.5, 8192 15.5 against 13.9). Per-tensor scales: every block reads
+// the whole of x for its maximum.
+constexpr int64_t FEW_ROWS = 32, SMALL_OUTPUT = 256 * 32 * 32, QUANTIZED_IN_PRODUCT = 3072, WHOLE_TENSOR = 1 << 16;
+bool small_product(int64_t m, int64_t n) { return m <= FEW_ROWS || m * n <= SMALL_OUTPUT; }
 
 // out[m, n] = a b^T, k = the operands' common pitch. br: rows of b per scale row (32: weight blocks, 1: row-wise).
 void product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_fmt, int64_t m, int64_t n, int br, const Tensor& bias,
@@ -103,7 +105,7 @@ void product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_f
     TORCH_INTERNAL_ASSERT(b.pitch == k);
     const void* bias_p = ptr(bias);
     const int bias_code = bias_p ? code_of(bias.scalar_type()) : 0, out_code = code_of(out_dtype);
-    if (m <= FEW_ROWS && br == 32) {
+    if (br == 32 && small_product(m, n)) {
         const int status = VIOLA_TRY(viola_skinny_linear, a.q, a_fmt, static_cast<const float*>(a.s), m, k, b.q, b_fmt, b.s, r.grouped, n, r.fwd_limit,
                                      r.scale_format(), nullptr, 0, nullptr, bias_p, bias_code, out, out_code, stream);
         if (status == 0) return;
@@ -298,9 +300,9 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
     }
     Arena temp;
     const bool cache_here = !r.fp8_weight && need_backward && r.cache_transpose;   // 16-bit storage: W^T of this forward's codes
-    if (gated < 0 && rows <= FEW_ROWS && !need_backward && !coded_input && r.fp8_weight && x2.element_size() == 2 && (rows > 16 ? 2 : 1) * r.in <= QUANTIZED_IN_PRODUCT &&
-        (r.grouped || !(r.delayed && l.counter[INPUT]->value))) {
-        // a few rows, nothing kept for backward: x is quantized inside the product
+    if (gated < 0 && small_product(rows, r.out) && !need_backward && !coded_input && r.fp8_weight && x2.element_size() == 2 && (rows > 16 && rows * r.out > 256 * 16 * 32 ? 2 : 1) * r.in <= QUANTIZED_IN_PRODUCT &&
+        (r.grouped || (rows * r.in <= WHOLE_TENSOR && !(r.delayed && l.counter[INPUT]->value)))) {
+        // nothing kept for backward: x is quantized inside the product
         f.y = at::empty({rows, r.out}, options);
         const void* bias_p = ptr(l.bias);
         float* history = r.grouped ? nullptr : static_cast<float*>(l.history[INPUT].mutable_data_ptr());
