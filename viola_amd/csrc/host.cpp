@@ -91,12 +91,14 @@ struct Kept {
 };
 
 // ---------------------------------------------------------------------------------------------------- products
-// Outputs the kernel for small products may take (viola_skinny_linear decides), and up to which k (times two where a block has 32
-// rows) it quantizes x itself: every block does so again, which beyond costs more than the quantizer's launch (measured, 8 rows,
-// 4096 wide: k = 1024 5.3 against 7.5 us, 4096 10.6 against 10.5, 8192 15.5 against 13.9). Per-tensor scales: every block reads
-// the whole of x for its maximum.
-constexpr int64_t FEW_ROWS = 32, SMALL_OUTPUT = 256 * 32 * 32, QUANTIZED_IN_PRODUCT = 3072, WHOLE_TENSOR = 1 << 16;
-bool small_product(int64_t m, int64_t n) { return m <= FEW_ROWS || m * n <= SMALL_OUTPUT; }
+// Outputs the kernel for small products takes (viola_skinny_linear: one tile of 32 x 32 or less per CU, any width up to 32 rows), and
+// up to which k (times two where a block has 32 rows) it quantizes x itself: every block does so again, which beyond costs more
+// than the quantizer's launch (measured, 8 rows, 4096 wide: k = 1024 5.3 against 7.5 us, 4096 10.6 against 10.5, 8192 15.5 against
+// 13.9). Per-tensor scales: every block reads the whole of x for its maximum.
+constexpr int64_t QUANTIZED_IN_PRODUCT = 3072, WHOLE_TENSOR = 1 << 16;
+bool small_product(int64_t m, int64_t n) { return m <= 32 || (m <= 4096 && ceil_div(m, 32) * ceil_div(n, 32) <= 256); }
+// Codes between the rows of a product's operands: that kernel takes any whole number of 16-byte pieces.
+int64_t product_pitch(const Recipe& r, int64_t m, int64_t n, int64_t k) { return k % 16 == 0 && small_product(m, n) ? k : r.pitch(k); }
 
 // out[m, n] = a b^T, k = the operands' common pitch. br: rows of b per scale row (32: weight blocks, 1: row-wise).
 void product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, int b_fmt, int64_t m, int64_t n, int br, const Tensor& bias,
@@ -175,8 +177,8 @@ void gated_product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b, i
 // Row-wise and / or transposed codes of a grouped operand into reserved arena space.
 struct GroupSpace {
     int64_t q = -1, s = -1, qt = -1, st = -1, pitch = 0, pitch_t = 0;
-    void reserve(const Recipe& r, Arena* rowwise, Arena* transposed, int64_t rows, int64_t cols) {
-        pitch = r.pitch(cols);
+    void reserve(const Recipe& r, Arena* rowwise, Arena* transposed, int64_t rows, int64_t cols, int64_t row_pitch) {
+        pitch = row_pitch;
         pitch_t = ceil_to(rows, 128);
         if (rowwise) { q = rowwise->take(rows * pitch); s = rowwise->take(rows * ceil_div(pitch, 32) * r.scale_bytes()); }
         if (transposed) { qt = transposed->take(cols * pitch_t); st = transposed->take(cols * (pitch_t / 32) * r.scale_bytes()); }
@@ -209,10 +211,10 @@ struct WeightSpace {
     int64_t q = -1, s = -1, p = -1, ps = -1, pitch = 0;
 };
 
-WeightSpace reserve_weight(const Layer& l, Arena& temp) {
+WeightSpace reserve_weight(const Layer& l, Arena& temp, int64_t pitch) {
     const Recipe& r = *l.recipe;
     WeightSpace w;
-    w.pitch = r.pitch(r.in);
+    w.pitch = pitch;
     const int64_t scale_rows = ceil_div(r.out, 32);
     if (!r.fp8_weight) {
         w.q = temp.take(r.out * r.in);
@@ -300,77 +302,80 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
     }
     Arena temp;
     const bool cache_here = !r.fp8_weight && need_backward && r.cache_transpose;   // 16-bit storage: W^T of this forward's codes
-    if (gated < 0 && small_product(rows, r.out) && !need_backward && !coded_input && r.fp8_weight && x2.element_size() == 2 && (rows > 16 && rows * r.out > 256 * 16 * 32 ? 2 : 1) * r.in <= QUANTIZED_IN_PRODUCT &&
-        (r.grouped || (rows * r.in <= WHOLE_TENSOR && !(r.delayed && l.counter[INPUT]->value)))) {
-        // nothing kept for backward: x is quantized inside the product
-        f.y = at::empty({rows, r.out}, options);
+    // gated: through [g | u] by the plain product, where it is kept for backward anyway or the product is a small one
+    const bool through_z = gated >= 0 && (keep_aux || (hidden_out && small_product(rows, r.out)));
+    const bool plain = gated < 0 || (hidden_out && through_z && dtype != at::kFloat && h % 8 == 0);
+    if (through_z) f.aux = at::empty({rows, r.out}, options);
+    if (gated < 0) f.y = at::empty({rows, r.out}, options);
+    Tensor& output = gated < 0 ? f.y : f.aux;
+    // Nothing kept for backward and a small product: x is quantized inside it.
+    auto quantized_inside = [&] {
+        if (!plain || need_backward || coded_input || !r.fp8_weight || x2.element_size() != 2 || !small_product(rows, r.out)) return false;
+        if ((rows > 16 && rows * r.out > 256 * 16 * 32 ? 2 : 1) * r.in > QUANTIZED_IN_PRODUCT) return false;
+        if (!r.grouped && (rows * r.in > WHOLE_TENSOR || (r.delayed && l.counter[INPUT]->value))) return false;
         const void* bias_p = ptr(l.bias);
         float* history = r.grouped ? nullptr : static_cast<float*>(l.history[INPUT].mutable_data_ptr());
         const int64_t slot = r.grouped ? 0 : l.counter[INPUT]->value % l.history[INPUT].numel();
         const int status = VIOLA_TRY(viola_skinny_linear, ptr(x2), code_of(x2.scalar_type()), nullptr, rows, r.in, ptr(l.weight), r.fwd, ptr(l.scale), r.grouped,
                                      r.out, r.fwd_limit, r.scale_format(), history, slot, nullptr, bias_p, bias_p ? code_of(l.bias.scalar_type()) : 0,
-                                     f.y.mutable_data_ptr(), code_of(dtype), stream);
-        if (status == 0) {
-            if (!r.grouped) ++l.counter[INPUT]->value;
-            return f;
-        }
-        if (status != VIOLA_EUNSUPPORTED) check("viola_skinny_linear", status);
-    }
-    const WeightSpace wspace = reserve_weight(l, temp);
+                                     output.mutable_data_ptr(), code_of(dtype), stream);
+        if (status != 0 && status != VIOLA_EUNSUPPORTED) check("viola_skinny_linear", status);
+        if (status == 0 && !r.grouped) ++l.counter[INPUT]->value;
+        return status == 0;
+    };
+    const bool done = quantized_inside();
+    if (done && gated < 0) return f;
+    const int64_t pitch = plain ? product_pitch(r, rows, r.out, r.in) : r.pitch(r.in);
     Codes a, w, w_unpadded;
-    if (r.grouped) {
-        GroupSpace g;
-        if (!coded_input) g.reserve(r, &temp, save ? &kept.arena : nullptr, rows, r.in);
-        temp.make(device);
-        if (save && !coded_input) kept.arena.make(device);
-        if (coded_input) {
-            a = coded_input->codes;
-            kept.input_t = coded_input->codes_t;
+    if (!done) {
+        const WeightSpace wspace = reserve_weight(l, temp, pitch);
+        if (r.grouped) {
+            GroupSpace g;
+            if (!coded_input) g.reserve(r, &temp, save ? &kept.arena : nullptr, rows, r.in, pitch);
+            temp.make(device);
+            if (save && !coded_input) kept.arena.make(device);
+            if (coded_input) {
+                a = coded_input->codes;
+                kept.input_t = coded_input->codes_t;
+            } else {
+                quantize_groups(r, x2, r.fwd, r.fwd_limit, g, &temp, &kept.arena, nullptr, &a, &kept.input_t, stream);
+            }
+            w = stored_weight(l, l.weight, wspace, temp, nullptr, &w_unpadded, stream);
         } else {
-            quantize_groups(r, x2, r.fwd, r.fwd_limit, g, &temp, &kept.arena, nullptr, &a, &kept.input_t, stream);
+            const int64_t pitch_t = ceil_to(rows, 128);
+            const int64_t q = temp.take(rows * pitch), maxima = temp.take(1024 * 4);
+            const int64_t qt = save ? kept.arena.take(r.in * pitch_t) : -1;
+            const int64_t scales = kept.arena.take(8);               // of x and of a 16-bit weight: backward uses these very values
+            temp.make(device);
+            kept.arena.make(device);
+            float* sx = kept.arena.as<float>(scales);
+            const Tensor& history = l.history[INPUT];
+            VIOLA_CALL(viola_tensor_encode, ptr(x2), code_of(x2.scalar_type()), rows, r.in, temp.as<float>(maxima), 1024,
+                       static_cast<float*>(history.mutable_data_ptr()), (int)history.numel(), l.counter[INPUT]->value, r.delayed, r.fwd_limit, sx, temp.at(q),
+                       pitch, save ? kept.arena.at(qt) : nullptr, save ? pitch_t : 0, r.fwd, nullptr, VIOLA_F32, stream);
+            ++l.counter[INPUT]->value;
+            a = {temp.at(q), sx, pitch};
+            kept.input_scale = sx;
+            if (save) kept.input_t = {kept.arena.at(qt), sx, pitch_t};
+            w = stored_weight(l, l.weight, wspace, temp, sx + 1, &w_unpadded, stream);
         }
-        w = stored_weight(l, l.weight, wspace, temp, nullptr, &w_unpadded, stream);
-    } else {
-        const int64_t pitch = r.pitch(r.in), pitch_t = ceil_to(rows, 128);
-        const int64_t q = temp.take(rows * pitch), maxima = temp.take(1024 * 4);
-        const int64_t qt = save ? kept.arena.take(r.in * pitch_t) : -1;
-        const int64_t scales = kept.arena.take(8);               // of x and of a 16-bit weight: backward uses these very values
-        temp.make(device);
-        kept.arena.make(device);
-        float* sx = kept.arena.as<float>(scales);
-        const Tensor& history = l.history[INPUT];
-        VIOLA_CALL(viola_tensor_encode, ptr(x2), code_of(x2.scalar_type()), rows, r.in, temp.as<float>(maxima), 1024,
-                   static_cast<float*>(history.mutable_data_ptr()), (int)history.numel(), l.counter[INPUT]->value, r.delayed, r.fwd_limit, sx, temp.at(q),
-                   pitch, save ? kept.arena.at(qt) : nullptr, save ? pitch_t : 0, r.fwd, nullptr, VIOLA_F32, stream);
-        ++l.counter[INPUT]->value;
-        a = {temp.at(q), sx, pitch};
-        kept.input_scale = sx;
-        if (save) kept.input_t = {kept.arena.at(qt), sx, pitch_t};
-        w = stored_weight(l, l.weight, wspace, temp, sx + 1, &w_unpadded, stream);
+        if (cache_here) {
+            kept.weight_t = at::empty({r.in, r.out}, at::TensorOptions().dtype(at::kByte).device(device));
+            const bool grid = r.grouped;
+            if (grid) kept.weight_t_scale = at::empty({ceil_div(r.in, 32), ceil_div(r.out, 32)}, at::TensorOptions().dtype(r.native ? at::kByte : at::kFloat).device(device));
+            VIOLA_CALL(viola_codes_transpose_pitched, w_unpadded.q, kept.weight_t.mutable_data_ptr(), 1, r.out, r.in, r.out, grid ? w_unpadded.s : nullptr,
+                       grid ? kept.weight_t_scale.mutable_data_ptr() : nullptr, 32, 32, r.scale_format(), nullptr, 0, 0, nullptr, 0, stream);
+        }
+        if (plain) product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, l.bias, output.mutable_data_ptr(), dtype, device, stream);
     }
-    if (cache_here) {
-        kept.weight_t = at::empty({r.in, r.out}, at::TensorOptions().dtype(at::kByte).device(device));
-        const bool grid = r.grouped;
-        if (grid) kept.weight_t_scale = at::empty({ceil_div(r.in, 32), ceil_div(r.out, 32)}, at::TensorOptions().dtype(r.native ? at::kByte : at::kFloat).device(device));
-        VIOLA_CALL(viola_codes_transpose_pitched, w_unpadded.q, kept.weight_t.mutable_data_ptr(), 1, r.out, r.in, r.out, grid ? w_unpadded.s : nullptr,
-                   grid ? kept.weight_t_scale.mutable_data_ptr() : nullptr, 32, 32, r.scale_format(), nullptr, 0, 0, nullptr, 0, stream);
-    }
-    if (gated < 0) {
-        f.y = at::empty({rows, r.out}, options);
-        product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, l.bias, f.y.mutable_data_ptr(), dtype, device, stream);
-        return f;
-    }
-    const bool through_z = keep_aux || (hidden_out && rows <= FEW_ROWS);     // (a few rows: the plain product has the kernel for them)
-    if (through_z) f.aux = at::empty({rows, r.out}, options);
-    if (hidden_out && through_z && dtype != at::kFloat && h % 8 == 0) {
-        // [g | u] is kept for backward anyway: the plain product on the tile that suits it best, then one pass over [g | u] that
-        // makes h's codes; h itself is never stored
+    if (gated < 0) return f;
+    if (plain) {
+        // one pass over [g | u] makes h's codes; h itself is never stored
         const Recipe& to = *hidden_out->reader;
         GroupSpace space;
-        space.reserve(to, &hidden_out->temp, hidden_out->transposed ? &hidden_kept->arena : nullptr, rows, h);
+        space.reserve(to, &hidden_out->temp, hidden_out->transposed ? &hidden_kept->arena : nullptr, rows, h, product_pitch(to, rows, to.out, h));
         hidden_out->temp.make(device);
         hidden_kept->arena.make(device);
-        product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, l.bias, f.aux.mutable_data_ptr(), dtype, device, stream);
         hidden_out->codes = {hidden_out->temp.at(space.q), hidden_out->temp.at(space.s), space.pitch};
         if (hidden_out->transposed) hidden_out->codes_t = {hidden_kept->arena.at(space.qt), hidden_kept->arena.at(space.st), space.pitch_t};
         VIOLA_CALL(viola_gated_quantize_dual_pitched, ptr(f.aux), code_of(dtype), rows, h, gated, const_cast<void*>(hidden_out->codes.q), space.pitch,
@@ -439,7 +444,7 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
     Arena temp;
     Codes g, gt, wt;
     float* partial = nullptr;
-    const int64_t parts = ceil_div(rows, 32), pitch = r.pitch(r.out);
+    const int64_t parts = ceil_div(rows, 32), pitch = gated < 0 ? product_pitch(r, rows, r.in, r.out) : r.pitch(r.out);
     // ---- space for the transposed weight
     const bool cached = kept.weight_t.defined() && kept.weight_t.numel();
     const bool make_wt = needs_x && !(cached && pitch == r.out);
@@ -450,7 +455,7 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
     if (needs_b) out.db = at::empty({r.out}, dx_options.dtype(kept.bias_grad));
     if (r.grouped) {
         GroupSpace space;
-        space.reserve(r, needs_x ? &temp : nullptr, needs_w ? &temp : nullptr, rows, r.out);
+        space.reserve(r, needs_x ? &temp : nullptr, needs_w ? &temp : nullptr, rows, r.out, pitch);
         const bool rides = needs_b && needs_w;                   // the bias gradient's 32-row sums come from the quantizer's read of dy
         const int64_t partial_at = rides ? temp.take(parts * r.out * 4) : -1;
         temp.make(device);
@@ -765,7 +770,7 @@ Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scal
         const bool save = need && ww && groups.rows;
         Arena temp;
         GroupSpace space;
-        space.reserve(r, &temp, nullptr, groups.rows, k);
+        space.reserve(r, &temp, nullptr, groups.rows, k, r.pitch(k));
         const bool repack = space.pitch != k;
         const int64_t wp = repack ? temp.take(groups.count * n * space.pitch) : -1;
         const int64_t wps = repack ? temp.take(groups.count * ceil_div(n, 32) * ceil_div(space.pitch, 32) * 4) : -1;
@@ -823,7 +828,7 @@ variable_list ExpertsBackward::apply(variable_list&& grads) {
     const bool weight_too = needs_w && has_input;
     Arena temp;
     GroupSpace space;
-    space.reserve(r, needs_x ? &temp : nullptr, nullptr, groups.rows, n);
+    space.reserve(r, needs_x ? &temp : nullptr, nullptr, groups.rows, n, r.pitch(n));
     const int64_t scale_cols = ceil_div(space.pitch, 32);
     const int64_t wt = needs_x ? temp.take(count * k * space.pitch) : -1, wts = needs_x ? temp.take(count * ceil_div(k, 32) * scale_cols * 4) : -1;
     const int64_t qt = weight_too ? temp.take(n * groups.padded) : -1, st = weight_too ? temp.take(n * (groups.padded / 32) * 4) : -1;
