@@ -159,7 +159,7 @@ int viola_tensor_quantize(const void* x, int x_dtype, int64_t rows, int64_t cols
 
 /* amax, scale (with its history) and codes of one tensor in both layouts at pitched rows (see above): the calls
  * viola_tensor_amax_scale and viola_tensor_quantize of viola/nn/linear.py:14-33 and _linear_kernels.py:231-260 as one, in
- * fewer launches for small tensors. column_sum != null: x.sum(0) in sum_dtype from the same reads (columns whole 16-byte
+ * fewer launches for small tensors. q or qt may be NULL, and both: then only the scale, the history and the sums. column_sum != null: x.sum(0) in sum_dtype from the same reads (columns whole 16-byte
  * pieces, x 16-byte aligned; VIOLA_EUNSUPPORTED otherwise). workspace: 1024 floats, with column sums
  * 1024 + viola_tensor_encode_slices(x_dtype, rows, cols) * cols, 16-byte aligned. */
 int viola_tensor_encode(const void* x, int x_dtype, int64_t rows, int64_t cols, float* workspace, int64_t workspace_floats,
@@ -167,6 +167,7 @@ int viola_tensor_encode(const void* x, int x_dtype, int64_t rows, int64_t cols, 
                         int64_t q_pitch, void* qt, int64_t qt_pitch, int q_dtype, void* column_sum, int sum_dtype,
                         viola_stream_t stream);
 int64_t viola_tensor_encode_slices(int x_dtype, int64_t rows, int64_t cols);
+
 /* ---------------------------------------------------------------- Hadamard-64 rotation (`rotation_size=64`)
  * H64 = H4 (x) H4 (x) H4, H4 = (ones(4, 4) - 2 flip(eye(4))) / 2, applied to each run of 64 consecutive columns of a
  * [rows, cols] matrix in FP32, in the operation order of viola/nn/_rotation_kernels.py:11-25 (_regular64); a last

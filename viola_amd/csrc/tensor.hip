@@ -511,6 +511,12 @@ extern "C" int viola_tensor_encode(const void* x, int x_dtype, int64_t rows, int
         status = viola_tensor_amax(x, x_dtype, n, workspace, parts, stream_);
     }
     if (status) return status;
+    if (!q && !qt) {
+        // no codes wanted (only the bias of a layer is trained): there is no quantizer whose blocks would form the scale and finish
+        // the sums on the side
+        status = viola_tensor_scale(workspace, parts, history, history_len, index, delayed, limit, scale, stream_);
+        return status || !column_sum ? status : viola_column_reduce(side.column_partial, side.slices, cols, column_sum, sum_dtype, stream_);
+    }
     if (parts <= FEW && !(delayed && index != 0)) {
         side.maxima = workspace;
         side.parts = (int)parts;
