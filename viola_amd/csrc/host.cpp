@@ -49,6 +49,8 @@ struct Recipe {
                         "cache_transpose"_a = cache_transpose, "fwd"_a = fwd, "bwd"_a = bwd, "fwd_limit"_a = fwd_limit, "bwd_limit"_a = bwd_limit,
                         "in"_a = in, "out"_a = out);
     }
+    at::ScalarType codes() const { return fwd == VIOLA_E4M3 ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
+    at::ScalarType scales() const { return native ? at::kByte : at::kFloat; }
     int scale_format() const { return native ? VIOLA_SCALE_E8M0 : VIOLA_SCALE_F32; }
     int64_t scale_bytes() const { return native ? 1 : 4; }
     int64_t pitch(int64_t k) const { return native ? ceil_to(k, 128) : k % 16 == 0 ? k : ceil_to(k, 128); }
@@ -63,6 +65,29 @@ struct Layer {
     std::shared_ptr<Counter> counter[3];
 };
 enum { WEIGHT = 0, INPUT = 1, GRAD = 2 };
+
+bool holds(const Tensor& t, const at::Device& device, at::ScalarType type, at::IntArrayRef sizes) {
+    return t.defined() && t.device() == device && t.scalar_type() == type && t.sizes() == sizes && t.is_contiguous();
+}
+
+// Whether a layer's tensors are what the kernels here read by raw pointer: the recipe's formats and shapes, contiguous, on x's
+// device. Any other call is the general path's (nn/_grouped_linear.py, nn/_tensor_linear.py), which copies a weight whose rows
+// are not contiguous, follows the weight's own FP8 format and refuses what no kernel takes.
+bool takes(const Layer& l, const at::Device& device) {
+    const Recipe& r = *l.recipe;
+    const int64_t rows = ceil_div(r.out, 32), cols = ceil_div(r.in, 32);
+    const at::ScalarType stored = l.weight.scalar_type();
+    if (r.fp8_weight ? stored != r.codes() : stored != at::kFloat && stored != at::kBFloat16 && stored != at::kHalf) return false;
+    if (r.in == 0 || r.out == 0 || !device.is_cuda() || !holds(l.weight, device, stored, {r.out, r.in})) return false;
+    if (r.fp8_weight && !(r.grouped ? holds(l.scale, device, r.scales(), {rows, cols}) : holds(l.scale, device, at::kFloat, {1}))) return false;
+    if (l.transpose.numel() && !(holds(l.transpose, device, r.codes(), {r.in, r.out}) && (!r.grouped || holds(l.transpose_scale, device, r.scales(), {cols, rows}))))
+        return false;
+    if (l.bias.defined() && (l.bias.device() != device || l.bias.numel() != r.out)) return false;
+    if (!r.grouped)
+        for (const Tensor& history : l.history)
+            if (history.device() != device || history.scalar_type() != at::kFloat || !history.is_contiguous() || history.numel() == 0) return false;
+    return true;
+}
 
 // Codes and scales of one operand; rows `pitch` codes apart.
 struct Codes {
@@ -532,6 +557,13 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
     return out;
 }
 
+// The weight as backward reads it. It is the caller's tensor, which may have been moved or replaced (`.data`) since the forward pass.
+Tensor weight_now(const Tensor& w, const Recipe& r, const Tensor& dy) {
+    TORCH_CHECK(w.device() == dy.device() && w.sizes() == at::IntArrayRef({r.out, r.in}) && (!r.fp8_weight || w.scalar_type() == r.codes()),
+                "the weight of a viola Linear was moved or replaced between forward and backward");
+    return w.contiguous();
+}
+
 bool wants(const Tensor& t) { return t.defined() && t.requires_grad(); }
 
 // ---------------------------------------------------------------------------------------------------- Linear
@@ -545,7 +577,7 @@ struct LinearBackward : public Node {
         variable_list result(3);
         if (!dy.defined()) return result;
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor weight = kept.weight.unpack();
+        const Tensor weight = weight_now(kept.weight.unpack(), *layer.recipe, dy);
         Gradients g = unproject(layer, kept, weight, dy, task_should_compute_output(0), task_should_compute_output(1) && kept.has_input,
                                 task_should_compute_output(2), -1, Tensor());
         if (g.dx.defined()) result[0] = g.dx.dim() == (int64_t)x_shape.size() ? g.dx : g.dx.view(x_shape);
@@ -610,8 +642,8 @@ struct MlpBackward : public Node {
         variable_list result(5);
         if (!dy.defined()) return result;
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor down_weight = down_kept.weight.unpack();
-        const Tensor up_weight = first_half ? up_kept.weight.unpack() : Tensor();
+        const Tensor down_weight = weight_now(down_kept.weight.unpack(), *down.recipe, dy);
+        const Tensor up_weight = first_half ? weight_now(up_kept.weight.unpack(), *up.recipe, dy) : Tensor();
         const bool upper = first_half && (task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2));
         const bool up_x = task_should_compute_output(0), up_w = task_should_compute_output(1) && up_kept.has_input, up_b = task_should_compute_output(2);
         // grouped recipes: the plain product writes dh, and the quantizer of dz makes dz as it reads dh and [g | u]
@@ -713,6 +745,8 @@ struct ExpertsBackward : public Node {
     Codes input_t;
     SavedVariable weight;
     Tensor weight_scale;
+    std::vector<int64_t> weight_shape;
+    int weight_fmt = VIOLA_E4M3;
     at::ScalarType x_dtype = at::kFloat, weight_grad = at::kFloat;
     bool has_input = false;
 
@@ -751,7 +785,10 @@ void segment_product(const Recipe& r, const Codes& a, int a_fmt, const Codes& b,
 Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scale, const std::vector<int64_t>& counts, const std::shared_ptr<Recipe>& recipe,
                at::ScalarType weight_grad) {
     TORCH_CHECK(x_.is_cuda() && x_.dim() == 2 && weight.dim() == 3 && weight.size(0) == (int64_t)counts.size() && x_.size(1) == weight.size(2));
-    TORCH_CHECK(weight_scale.is_contiguous() && weight.is_contiguous() && weight.is_cuda());
+    const int w_fmt = code_of(weight.scalar_type());             // the codes' own format, whatever the recipe encodes x in
+    TORCH_CHECK((w_fmt == VIOLA_E4M3 || w_fmt == VIOLA_E5M2) && weight.is_contiguous() && weight.device() == x_.device(), "weight: contiguous FP8 codes on x's device");
+    TORCH_CHECK(holds(weight_scale, x_.device(), at::kFloat, {weight.size(0), ceil_div(weight.size(1), 32), ceil_div(weight.size(2), 32)}),
+                "weight_scale: contiguous FP32 [groups, ceil(out / 32), ceil(in / 32)] on x's device");
     const Recipe& r = *recipe;
     const bool wx = x_.requires_grad(), ww = weight.requires_grad();
     const bool need = at::GradMode::is_enabled() && (wx || ww);
@@ -792,7 +829,7 @@ Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scal
                 VIOLA_CALL(viola_codes_repack, w.q, temp.at(wp), groups.count, n, k, space.pitch, w.s, temp.at(wps), 32, 32, VIOLA_SCALE_F32, stream);
                 w = {temp.at(wp), temp.at(wps), space.pitch};
             }
-            segment_product(r, a, r.fwd, w, r.fwd, groups, n, y.mutable_data_ptr(), x.scalar_type(), stream);
+            segment_product(r, a, r.fwd, w, w_fmt, groups, n, y.mutable_data_ptr(), x.scalar_type(), stream);
         }
         if (need) {
             node->has_input = save;
@@ -803,6 +840,8 @@ Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scal
         node->recipe = recipe;
         node->weight = SavedVariable(weight, false);
         node->weight_scale = weight_scale;
+        node->weight_shape = weight.sizes().vec();
+        node->weight_fmt = w_fmt;
         node->weight_grad = weight_grad;
         node->set_next_edges(torch::autograd::collect_next_edges(x_, weight));
         torch::autograd::set_history(y, node);
@@ -815,8 +854,11 @@ variable_list ExpertsBackward::apply(variable_list&& grads) {
     if (!grads[0].defined()) return result;
     at::AutoDispatchBelowADInplaceOrView below;
     const Recipe& r = *recipe;
-    const Tensor w = weight.unpack();
+    const Tensor w = weight.unpack().contiguous();
+    const int w_fmt = code_of(w.scalar_type());
     const int64_t count = w.size(0), n = w.size(1), k = w.size(2);
+    TORCH_CHECK(w.device() == grads[0].device() && w_fmt == weight_fmt && w.sizes() == at::IntArrayRef(weight_shape),
+                "the weight of a grouped linear was moved or replaced between forward and backward");
     const Tensor dy = as_matrix(grads[0], n);
     const at::Device device = w.device();
     const viola_stream_t stream = stream_of(w);
@@ -840,7 +882,7 @@ variable_list ExpertsBackward::apply(variable_list&& grads) {
         VIOLA_CALL(viola_codes_transpose_pitched, ptr(w), temp.at(wt), count, n, k, space.pitch, ptr(weight_scale), temp.at(wts), 32, 32, VIOLA_SCALE_F32, nullptr, 0,
                    0, nullptr, 0, stream);
         result[0] = at::empty({groups.rows, k}, options.dtype(x_dtype));
-        segment_product(r, g, r.bwd, Codes{temp.at(wt), temp.at(wts), space.pitch}, r.fwd, groups, k, result[0].mutable_data_ptr(), x_dtype, stream);
+        segment_product(r, g, r.bwd, Codes{temp.at(wt), temp.at(wts), space.pitch}, w_fmt, groups, k, result[0].mutable_data_ptr(), x_dtype, stream);
     }
     if (weight_too) {
         result[1] = at::empty({count, n, k}, options.dtype(weight_grad));
@@ -885,13 +927,16 @@ PYBIND11_MODULE(_host, m) {
         recording.store(!list.is_none());
     });
     register_optimizer(m);
-    m.def("linear", [](const Tensor& x, const py::tuple& layer) {
+    // None: a call for the general path
+    m.def("linear", [](const Tensor& x, const py::tuple& layer) -> std::optional<Tensor> {
         Layer l = layer_from(layer);
+        if (!takes(l, x.device())) return std::nullopt;
         py::gil_scoped_release release;
         return linear(x, l);
     });
-    m.def("mlp", [](const Tensor& x, const py::tuple& up, const py::tuple& down, int activation) {
+    m.def("mlp", [](const Tensor& x, const py::tuple& up, const py::tuple& down, int activation) -> std::optional<Tensor> {
         Layer u = layer_from(up), d = layer_from(down);
+        if (!takes(u, x.device()) || !takes(d, x.device()) || u.recipe->out != 2 * d.recipe->in) return std::nullopt;
         py::gil_scoped_release release;
         return mlp(x, u, d, activation);
     });

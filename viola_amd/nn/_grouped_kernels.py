@@ -135,6 +135,7 @@ def gemm(a, b, sa, sb, group_a, group_b, *, out_dtype, native=False, bias=None, 
     n = b.shape[0]
     assert tuple(sa.shape) == scale_shape((m, k), group_a) and tuple(sb.shape) == scale_shape((n, k), group_b)
     out = torch.empty((m, n), device=a.device, dtype=out_dtype)
+    assert bias is None or bias.numel() in (0, n)
     bias_c = bias.contiguous() if bias is not None else None
     if accum_dtype == "fp16":
         assert not native, "MXFP8 MMA uses FP32 accumulation."

@@ -82,6 +82,8 @@ def gemm(a, b, sa, sb, *, out_dtype, bias=None, autotune=False, accum_dtype="fp3
     assert a.is_cuda and a.is_contiguous() and b.is_contiguous() and a.shape[1] == b.shape[1]
     out = torch.empty((a.shape[0], b.shape[0]), device=a.device, dtype=out_dtype)
     has_bias = bias is not None and bias.numel() > 0
+    assert not has_bias or bias.numel() == b.shape[0]
+    bias = bias.contiguous() if has_bias else None
     if accum_dtype == "fp16":
         _lib.call("viola_tensor_gemm_half", _lib.ptr(a), _lib.code(a.dtype), _lib.ptr(b), _lib.code(b.dtype), _lib.ptr(sa), _lib.ptr(sb),
                   a.shape[0], b.shape[0], a.shape[1], _lib.ptr(bias) if has_bias else None, _lib.code(bias.dtype) if has_bias else 0,

@@ -50,6 +50,7 @@ def gemm(a, b, sa, sb, *, layer, out_dtype, activation, backward=False, aux=None
         aux = torch.empty((m, 2 * h) if save else (0, 0), device=a.device, dtype=out_dtype)
     else:
         assert aux.dtype == out_dtype and aux.is_contiguous() and tuple(aux.shape) == (m, 2 * h)
+    assert bias is None or bias.numel() in (0, b.shape[0])
     bias_c = bias.contiguous() if bias is not None else None
     bias_code = _lib.code(bias_c.dtype) if bias_c is not None else 0
     empty = torch.empty((0, 0), device=a.device, dtype=torch.uint8)
@@ -94,6 +95,7 @@ def _encoded_forward(a, b, sa, sb, *, layer, out_dtype, activation, bias, save, 
         scale = torch.empty((m, h // 32), device=a.device, dtype=torch.uint8)
         codes_t = torch.empty((h, m) if transpose else (0, 0), device=a.device, dtype=fp8)
         scale_t = torch.empty((h, m // 32) if transpose else (0, 0), device=a.device, dtype=torch.uint8)
+        assert bias is None or bias.numel() in (0, b.shape[0])
         bias_c = bias.contiguous() if bias is not None else None
         status = _lib.call("viola_mx_gated_gemm_encode", _lib.ptr(a), _lib.code(a.dtype), _lib.ptr(b), _lib.code(b.dtype),
                            _lib.ptr(sa), _lib.ptr(sb), m, h, k, ga[0], gb[0], _lib.ptr(bias_c),

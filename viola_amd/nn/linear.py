@@ -364,7 +364,9 @@ class Linear(nn.Module):
             self.refresh_weight(self._master())
             assert not self._store.pending, _HOST_MASTER
         if self._standard:
-            return _lib.host().linear(x, self._operands())
+            y = _lib.host().linear(x, self._operands())
+            if y is not None:                                                  # None: operands only the general path takes
+                return y
         trainable = [t for t in (x, self.weight, self.bias) if t is not None and t.requires_grad]
         need_backward = torch.is_grad_enabled() and bool(trainable)
         if self._grouped_scaling:
