@@ -97,23 +97,80 @@ struct Codes {
 };
 
 
-// What a projection's backward needs, and where it lives.
-struct Kept {
-    Arena arena;                                                 // transposed codes of the input (+ its scale)
-    Codes input_t;
-    const float* input_scale = nullptr;                          // per-tensor recipes
-    SavedVariable weight;
-    Tensor weight_scale, weight_t, weight_t_scale;
-    int64_t rows = 0;
-    at::ScalarType x_dtype = at::kFloat, weight_grad = at::kFloat, bias_grad = at::kFloat;
-    bool has_input = false;
-
-    void release() {
-        arena.release();
-        weight.reset_data();
-        weight_scale = weight_t = weight_t_scale = Tensor();
+// Where transposed codes and their scales lie in an arena; rows `pitch` codes apart.
+struct Place {
+    int64_t q = -1, s = -1, pitch = 0;
+    Codes in(const void* base) const {
+        const char* p = static_cast<const char*>(base);
+        return q < 0 ? Codes{} : Codes{p + q, p + s, pitch};
     }
 };
+
+// A tensor that was saved for backward, as it comes back: a saved-tensor hook may have moved it or made another of it.
+Tensor restored(const SavedVariable& saved, const at::Device& device, at::ScalarType type, at::IntArrayRef sizes) {
+    const Tensor t = saved.unpack();
+    TORCH_CHECK(t.defined() && t.device() == device && t.scalar_type() == type && t.sizes() == sizes, "a tensor saved by a viola module came back changed");
+    return t.contiguous();
+}
+
+// What a projection's backward needs. All of it is saved the way autograd saves tensors, so that saved-tensor hooks (save_on_cpu,
+// checkpointing) see it, in-place changes are noticed and it is freed with the graph; no address outlives the forward pass.
+struct Kept {
+    Arena arena;                                                 // forward only: transposed codes of the input, per-tensor scales
+    Tensor weight_t, weight_t_scale;                             // forward only: the cached W^T, or this forward's
+    Place input;                                                 // in the saved arena
+    int64_t scales = -1;                                         // per-tensor recipes: the scale of x, then that of a 16-bit weight
+    SavedVariable saved_arena, weight, weight_scale, saved_weight_t, saved_weight_t_scale;
+    int64_t rows = 0;
+    at::ScalarType x_dtype = at::kFloat, weight_grad = at::kFloat, bias_grad = at::kFloat;
+    bool has_input = false, has_weight_t = false;
+
+    // After the forward pass, where hooks run as they do for any operator: outside of its dispatch guard.
+    void save(const Layer& l) {
+        saved_arena = SavedVariable(arena.tensor(), false);
+        weight = SavedVariable(l.weight, false);
+        if (l.recipe->fp8_weight) weight_scale = SavedVariable(l.scale, false);
+        has_weight_t = weight_t.defined() && weight_t.numel();
+        if (has_weight_t) {
+            saved_weight_t = SavedVariable(weight_t, false);
+            if (l.recipe->grouped) saved_weight_t_scale = SavedVariable(weight_t_scale, false);
+        }
+        arena.release();
+        weight_t = weight_t_scale = Tensor();
+    }
+    void release() {
+        for (SavedVariable* v : {&saved_arena, &weight, &weight_scale, &saved_weight_t, &saved_weight_t_scale}) v->reset_data();
+    }
+};
+
+// The tensors of one layer as its backward reads them.
+struct Restored {
+    Tensor arena, weight, weight_scale, weight_t, weight_t_scale;
+    Codes input_t;
+    const float* scales = nullptr;
+};
+
+Restored restore(const Kept& kept, const Recipe& r, const Tensor& dy) {
+    const at::Device device = dy.device();
+    const int64_t rows = ceil_div(r.out, 32), cols = ceil_div(r.in, 32);
+    Restored t;
+    t.weight = kept.weight.unpack();
+    // the caller's tensor: it may have been moved or replaced (`.data`) since
+    TORCH_CHECK(t.weight.device() == device && t.weight.sizes() == at::IntArrayRef({r.out, r.in}) && (!r.fp8_weight || t.weight.scalar_type() == r.codes()),
+                "the weight of a viola Linear was moved or replaced between forward and backward");
+    t.weight = t.weight.contiguous();
+    if (kept.arena.size()) {
+        t.arena = restored(kept.saved_arena, device, at::kByte, {kept.arena.size()});
+        t.input_t = kept.input.in(t.arena.const_data_ptr());
+        if (kept.scales >= 0) t.scales = reinterpret_cast<const float*>(static_cast<const char*>(t.arena.const_data_ptr()) + kept.scales);
+    }
+    if (r.fp8_weight) t.weight_scale = r.grouped ? restored(kept.weight_scale, device, r.scales(), {rows, cols}) : restored(kept.weight_scale, device, at::kFloat, {1});
+    if (kept.has_weight_t) {
+        t.weight_t = restored(kept.saved_weight_t, device, r.codes(), {r.in, r.out});
+        if (r.grouped) t.weight_t_scale = restored(kept.saved_weight_t_scale, device, r.scales(), {cols, rows});
+    }
+    return t;
+}
 
 // ---------------------------------------------------------------------------------------------------- products
 // Outputs the kernel for small products takes (viola_skinny_linear: one tile of 32 x 32 or less per CU, any width up to 32 rows), and
@@ -291,8 +348,7 @@ struct CodedHidden {
     const Recipe* reader = nullptr;                              // the down projection's
     bool transposed = false;                                     // its weight gradient wants the other layout too
     Arena temp;                                                  // row-wise codes, used by this forward only
-    Codes codes;
-    Codes codes_t;                                               // in the down projection's Kept arena
+    Codes codes;                                                 // the other layout goes to the down projection's Kept arena
 };
 
 struct Forward {
@@ -310,8 +366,6 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
     kept.x_dtype = dtype;
     kept.has_input = save;
     if (need_backward) {
-        kept.weight = SavedVariable(l.weight, false);
-        kept.weight_scale = l.scale;
         kept.weight_t = l.transpose;
         kept.weight_t_scale = l.transpose_scale;
         kept.weight_grad = l.weight.grad_dtype().value_or(l.weight.scalar_type());
@@ -361,9 +415,10 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
             if (save && !coded_input) kept.arena.make(device);
             if (coded_input) {
                 a = coded_input->codes;
-                kept.input_t = coded_input->codes_t;
             } else {
-                quantize_groups(r, x2, r.fwd, r.fwd_limit, g, &temp, &kept.arena, nullptr, &a, &kept.input_t, stream);
+                Codes in_arena;
+                quantize_groups(r, x2, r.fwd, r.fwd_limit, g, &temp, &kept.arena, nullptr, &a, &in_arena, stream);
+                if (save) kept.input = {g.qt, g.st, g.pitch_t};
             }
             w = stored_weight(l, l.weight, wspace, temp, nullptr, &w_unpadded, stream);
         } else {
@@ -380,14 +435,14 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
                        pitch, save ? kept.arena.at(qt) : nullptr, save ? pitch_t : 0, r.fwd, nullptr, VIOLA_F32, stream);
             ++l.counter[INPUT]->value;
             a = {temp.at(q), sx, pitch};
-            kept.input_scale = sx;
-            if (save) kept.input_t = {kept.arena.at(qt), sx, pitch_t};
+            kept.scales = scales;
+            if (save) kept.input = {qt, scales, pitch_t};
             w = stored_weight(l, l.weight, wspace, temp, sx + 1, &w_unpadded, stream);
         }
         if (cache_here) {
-            kept.weight_t = at::empty({r.in, r.out}, at::TensorOptions().dtype(at::kByte).device(device));
+            kept.weight_t = at::empty({r.in, r.out}, at::TensorOptions().dtype(r.codes()).device(device));
             const bool grid = r.grouped;
-            if (grid) kept.weight_t_scale = at::empty({ceil_div(r.in, 32), ceil_div(r.out, 32)}, at::TensorOptions().dtype(r.native ? at::kByte : at::kFloat).device(device));
+            if (grid) kept.weight_t_scale = at::empty({ceil_div(r.in, 32), ceil_div(r.out, 32)}, at::TensorOptions().dtype(r.scales()).device(device));
             VIOLA_CALL(viola_codes_transpose_pitched, w_unpadded.q, kept.weight_t.mutable_data_ptr(), 1, r.out, r.in, r.out, grid ? w_unpadded.s : nullptr,
                        grid ? kept.weight_t_scale.mutable_data_ptr() : nullptr, 32, 32, r.scale_format(), nullptr, 0, 0, nullptr, 0, stream);
         }
@@ -402,10 +457,11 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         hidden_out->temp.make(device);
         hidden_kept->arena.make(device);
         hidden_out->codes = {hidden_out->temp.at(space.q), hidden_out->temp.at(space.s), space.pitch};
-        if (hidden_out->transposed) hidden_out->codes_t = {hidden_kept->arena.at(space.qt), hidden_kept->arena.at(space.st), space.pitch_t};
+        if (hidden_out->transposed) hidden_kept->input = {space.qt, space.st, space.pitch_t};
         VIOLA_CALL(viola_gated_quantize_dual_pitched, ptr(f.aux), code_of(dtype), rows, h, gated, const_cast<void*>(hidden_out->codes.q), space.pitch,
-                   const_cast<void*>(hidden_out->codes.s), const_cast<void*>(hidden_out->codes_t.q), hidden_out->transposed ? space.pitch_t : rows,
-                   const_cast<void*>(hidden_out->codes_t.s), to.fwd, to.fwd_limit, to.scale_format(), stream);
+                   const_cast<void*>(hidden_out->codes.s), hidden_out->transposed ? hidden_kept->arena.at(space.qt) : nullptr,
+                   hidden_out->transposed ? space.pitch_t : rows, hidden_out->transposed ? hidden_kept->arena.at(space.st) : nullptr, to.fwd, to.fwd_limit,
+                   to.scale_format(), stream);
         hidden_kept->rows = rows;
         return f;
     }
@@ -427,11 +483,10 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         if (status != 0 && status != VIOLA_EUNSUPPORTED) check("viola_mx_gated_gemm_encode", status);
         if (status == 0) {
             hidden_out->codes = {hidden_out->temp.at(q), hidden_out->temp.at(s), h};
-            hidden_out->codes_t = {qt_p, st_p, rows};
+            if (transposed) hidden_kept->input = {qt, st, rows};
             hidden_kept->rows = rows;
             return f;
         }
-        keep.release();
         hidden_kept->arena = Arena();
     }
     f.y = at::empty({rows, h}, options);
@@ -449,11 +504,12 @@ struct GatedGradient {
     int activation = 0;
 };
 
-// gated >= 0: dx is dz = [d u act'(g) | d act(g)] from aux = [g | u]. (w: the unpacked weight of the layer.)
-Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& dy_, bool needs_x, bool needs_w, bool needs_b, int gated, const Tensor& aux,
+// gated >= 0: dx is dz = [d u act'(g) | d act(g)] from aux = [g | u].
+Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const Tensor& dy_, bool needs_x, bool needs_w, bool needs_b, int gated, const Tensor& aux,
                     const GatedGradient* gate = nullptr) {
     const Recipe& r = *l.recipe;
     const int64_t rows = kept.rows;
+    const Tensor& w = t.weight;
     const at::Device device = w.device();
     const viola_stream_t stream = stream_of(w);
     const auto dx_options = at::TensorOptions().dtype(kept.x_dtype).device(device);
@@ -471,7 +527,7 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
     float* partial = nullptr;
     const int64_t parts = ceil_div(rows, 32), pitch = gated < 0 ? product_pitch(r, rows, r.in, r.out) : r.pitch(r.out);
     // ---- space for the transposed weight
-    const bool cached = kept.weight_t.defined() && kept.weight_t.numel();
+    const bool cached = kept.has_weight_t;
     const bool make_wt = needs_x && !(cached && pitch == r.out);
     const int64_t wt_q = make_wt ? temp.take(r.in * pitch) : -1, wt_s = make_wt && r.grouped ? temp.take(ceil_div(r.in, 32) * ceil_div(pitch, 32) * r.scale_bytes()) : -1;
     const bool requantize = make_wt && !cached && !r.fp8_weight; // memory mode with 16-bit storage: this forward's codes again
@@ -519,10 +575,10 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
         if (needs_w) gt = {temp.at(qt), scale, pitch_t};
     }
     if (needs_x) {
-        const void* w_scale = r.grouped ? ptr(kept.weight_scale) : r.fp8_weight ? ptr(kept.weight_scale) : kept.input_scale + 1;
-        wt = {ptr(kept.weight_t), r.grouped ? ptr(kept.weight_t_scale) : w_scale, pitch};
+        const void* w_scale = r.fp8_weight ? ptr(t.weight_scale) : r.grouped ? nullptr : t.scales + 1;
+        wt = {ptr(t.weight_t), r.grouped ? ptr(t.weight_t_scale) : w_scale, pitch};
         if (make_wt && cached) {
-            VIOLA_CALL(viola_codes_repack, ptr(kept.weight_t), temp.at(wt_q), 1, r.in, r.out, pitch, r.grouped ? ptr(kept.weight_t_scale) : nullptr,
+            VIOLA_CALL(viola_codes_repack, ptr(t.weight_t), temp.at(wt_q), 1, r.in, r.out, pitch, r.grouped ? ptr(t.weight_t_scale) : nullptr,
                        r.grouped ? temp.at(wt_s) : nullptr, 32, 32, r.scale_format(), stream);
         } else if (make_wt) {
             const void* codes = ptr(w);
@@ -552,16 +608,9 @@ Gradients unproject(const Layer& l, Kept& kept, const Tensor& w, const Tensor& d
     }
     if (needs_w) {
         out.dw = at::empty({r.out, r.in}, dx_options.dtype(kept.weight_grad));
-        product(r, gt, r.bwd, kept.input_t, r.fwd, r.out, r.in, 1, Tensor(), out.dw.mutable_data_ptr(), kept.weight_grad, device, stream);
+        product(r, gt, r.bwd, t.input_t, r.fwd, r.out, r.in, 1, Tensor(), out.dw.mutable_data_ptr(), kept.weight_grad, device, stream);
     }
     return out;
-}
-
-// The weight as backward reads it. It is the caller's tensor, which may have been moved or replaced (`.data`) since the forward pass.
-Tensor weight_now(const Tensor& w, const Recipe& r, const Tensor& dy) {
-    TORCH_CHECK(w.device() == dy.device() && w.sizes() == at::IntArrayRef({r.out, r.in}) && (!r.fp8_weight || w.scalar_type() == r.codes()),
-                "the weight of a viola Linear was moved or replaced between forward and backward");
-    return w.contiguous();
 }
 
 bool wants(const Tensor& t) { return t.defined() && t.requires_grad(); }
@@ -576,9 +625,9 @@ struct LinearBackward : public Node {
         const Tensor& dy = grads[0];
         variable_list result(3);
         if (!dy.defined()) return result;
+        const Restored tensors = restore(kept, *layer.recipe, dy);
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor weight = weight_now(kept.weight.unpack(), *layer.recipe, dy);
-        Gradients g = unproject(layer, kept, weight, dy, task_should_compute_output(0), task_should_compute_output(1) && kept.has_input,
+        Gradients g = unproject(layer, kept, tensors, dy, task_should_compute_output(0), task_should_compute_output(1) && kept.has_input,
                                 task_should_compute_output(2), -1, Tensor());
         if (g.dx.defined()) result[0] = g.dx.dim() == (int64_t)x_shape.size() ? g.dx : g.dx.view(x_shape);
         result[1] = g.dw;
@@ -619,6 +668,7 @@ Tensor linear(const Tensor& x, Layer& l) {
     }
     if (need) {
         node->layer = without_tensors(l);
+        node->kept.save(l);
         node->x_shape = x.sizes().vec();
         node->set_next_edges(torch::autograd::collect_next_edges(x, l.weight, l.bias));
         torch::autograd::set_history(y, node);
@@ -641,20 +691,20 @@ struct MlpBackward : public Node {
         const Tensor& dy = grads[0];
         variable_list result(5);
         if (!dy.defined()) return result;
-        at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor down_weight = weight_now(down_kept.weight.unpack(), *down.recipe, dy);
-        const Tensor up_weight = first_half ? weight_now(up_kept.weight.unpack(), *up.recipe, dy) : Tensor();
+        const Restored down_tensors = restore(down_kept, *down.recipe, dy);
         const bool upper = first_half && (task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2));
         const bool up_x = task_should_compute_output(0), up_w = task_should_compute_output(1) && up_kept.has_input, up_b = task_should_compute_output(2);
         // grouped recipes: the plain product writes dh, and the quantizer of dz makes dz as it reads dh and [g | u]
         const bool direct = upper && up.recipe->grouped && up_kept.rows && up_kept.x_dtype != at::kFloat && down.recipe->in % 64 == 0 && (up_w || (up_x && !up_b));
-        GatedGradient gate{upper ? z.unpack() : Tensor(), activation};
-        Gradients d = unproject(down, down_kept, down_weight, dy, upper, task_should_compute_output(3) && down_kept.has_input, task_should_compute_output(4),
+        const Restored up_tensors = upper ? restore(up_kept, *up.recipe, dy) : Restored();
+        GatedGradient gate{upper ? restored(z, dy.device(), up_kept.x_dtype, {up_kept.rows, up.recipe->out}) : Tensor(), activation};
+        at::AutoDispatchBelowADInplaceOrView below;
+        Gradients d = unproject(down, down_kept, down_tensors, dy, upper, task_should_compute_output(3) && down_kept.has_input, task_should_compute_output(4),
                                 direct ? -1 : activation, gate.z);
         result[3] = d.dw;
         result[4] = d.db;
         if (!upper) return result;
-        Gradients u = unproject(up, up_kept, up_weight, d.dx, up_x, up_w, up_b, -1, Tensor(), direct ? &gate : nullptr);
+        Gradients u = unproject(up, up_kept, up_tensors, d.dx, up_x, up_w, up_b, -1, Tensor(), direct ? &gate : nullptr);
         if (u.dx.defined()) result[0] = u.dx.dim() == (int64_t)x_shape.size() ? u.dx : u.dx.view(x_shape);
         result[1] = u.dw;
         result[2] = u.db;
@@ -701,7 +751,13 @@ Tensor mlp(const Tensor& x, Layer& up, Layer& down, int activation) {
         node->activation = activation;
         node->first_half = first_half;
         node->x_shape = x.sizes().vec();
-        if (first_half) node->z = SavedVariable(z, false);
+        if (first_half) {
+            node->up_kept.save(up);
+            node->z = SavedVariable(z, false);
+        } else {
+            node->up_kept.arena.release();
+        }
+        node->down_kept.save(down);
         node->set_next_edges(torch::autograd::collect_next_edges(x, up.weight, up.bias, down.weight, down.bias));
         torch::autograd::set_history(y, node);
     }
@@ -711,9 +767,13 @@ Tensor mlp(const Tensor& x, Layer& up, Layer& down, int activation) {
 // ---------------------------------------------------------------------------------------------------- variable groups
 struct Groups {
     int64_t count = 0, rows = 0, padded = 0;
-    Arena arena;                                                 // row offsets, then offsets on the padded token axis
+    Arena arena;                                                 // forward only: row offsets, then offsets on the padded token axis
     const int64_t* offsets = nullptr;
     const int64_t* padded_offsets = nullptr;
+    void at(const Tensor& table) {
+        offsets = static_cast<const int64_t*>(table.const_data_ptr());
+        padded_offsets = offsets + count + 1;
+    }
 };
 
 // The offset tables travel as kernel arguments: no staging buffer, no copy the host has to wait for.
@@ -734,17 +794,15 @@ void make_groups(Groups& g, const std::vector<int64_t>& counts, const at::Device
     const int64_t at = g.arena.take((int64_t)words.size() * 8);
     g.arena.make(device);
     VIOLA_CALL(viola_store_words, g.arena.as<int64_t>(at), words.data(), (int64_t)words.size(), stream);
-    g.offsets = g.arena.as<int64_t>(at);
-    g.padded_offsets = g.offsets + g.count + 1;
+    g.at(g.arena.tensor());
 }
 
 struct ExpertsBackward : public Node {
     std::shared_ptr<Recipe> recipe;
     Groups groups;
-    Arena kept;
-    Codes input_t;
-    SavedVariable weight;
-    Tensor weight_scale;
+    Arena kept;                                                  // forward only: transposed codes of x
+    Place input;                                                 // in the saved arena
+    SavedVariable tables, saved_arena, weight, weight_scale;     // see Kept
     std::vector<int64_t> weight_shape;
     int weight_fmt = VIOLA_E4M3;
     at::ScalarType x_dtype = at::kFloat, weight_grad = at::kFloat;
@@ -753,10 +811,7 @@ struct ExpertsBackward : public Node {
     variable_list apply(variable_list&& grads) override;
     std::string name() const override { return "ViolaExpertsBackward"; }
     void release_variables() override {
-        kept.release();
-        groups.arena.release();
-        weight.reset_data();
-        weight_scale = Tensor();
+        for (SavedVariable* v : {&tables, &saved_arena, &weight, &weight_scale}) v->reset_data();
     }
 };
 
@@ -819,7 +874,7 @@ Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scal
             node->kept.make(device);
             qt = node->kept.at(q_at);
             st = node->kept.as<float>(s_at);
-            node->input_t = {qt, st, groups.padded};
+            node->input = {q_at, s_at, groups.padded};
         }
         y = at::empty({groups.rows, n}, x.options());
         if (groups.rows) {
@@ -839,7 +894,11 @@ Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scal
     if (need) {
         node->recipe = recipe;
         node->weight = SavedVariable(weight, false);
-        node->weight_scale = weight_scale;
+        node->weight_scale = SavedVariable(weight_scale, false);
+        node->tables = SavedVariable(node->groups.arena.tensor(), false);
+        node->saved_arena = SavedVariable(node->kept.tensor(), false);
+        node->groups.arena.release();
+        node->kept.release();
         node->weight_shape = weight.sizes().vec();
         node->weight_fmt = w_fmt;
         node->weight_grad = weight_grad;
@@ -852,14 +911,19 @@ Tensor experts(const Tensor& x_, const Tensor& weight, const Tensor& weight_scal
 variable_list ExpertsBackward::apply(variable_list&& grads) {
     variable_list result(2);
     if (!grads[0].defined()) return result;
-    at::AutoDispatchBelowADInplaceOrView below;
     const Recipe& r = *recipe;
     const Tensor w = weight.unpack().contiguous();
-    const int w_fmt = code_of(w.scalar_type());
-    const int64_t count = w.size(0), n = w.size(1), k = w.size(2);
-    TORCH_CHECK(w.device() == grads[0].device() && w_fmt == weight_fmt && w.sizes() == at::IntArrayRef(weight_shape),
+    TORCH_CHECK(w.device() == grads[0].device() && w.sizes() == at::IntArrayRef(weight_shape) && code_of(w.scalar_type()) == weight_fmt,
                 "the weight of a grouped linear was moved or replaced between forward and backward");
+    const int w_fmt = weight_fmt;
+    const int64_t count = w.size(0), n = w.size(1), k = w.size(2);
+    const Tensor scale = restored(weight_scale, w.device(), at::kFloat, {count, ceil_div(n, 32), ceil_div(k, 32)});
+    const Tensor table = restored(tables, w.device(), at::kByte, {groups.arena.size()});
+    const Tensor codes = has_input ? restored(saved_arena, w.device(), at::kByte, {kept.size()}) : Tensor();
+    at::AutoDispatchBelowADInplaceOrView below;
     const Tensor dy = as_matrix(grads[0], n);
+    Groups groups = this->groups;                                // a second backward pass may run beside this one
+    groups.at(table);
     const at::Device device = w.device();
     const viola_stream_t stream = stream_of(w);
     const bool needs_x = task_should_compute_output(0), needs_w = task_should_compute_output(1);
@@ -879,13 +943,14 @@ variable_list ExpertsBackward::apply(variable_list&& grads) {
     quantize_segments(r, dy, r.bwd, r.bwd_limit, groups, needs_x ? &temp : nullptr, space, weight_too ? temp.at(qt) : nullptr,
                       weight_too ? temp.as<float>(st) : nullptr, &g, stream);
     if (needs_x) {
-        VIOLA_CALL(viola_codes_transpose_pitched, ptr(w), temp.at(wt), count, n, k, space.pitch, ptr(weight_scale), temp.at(wts), 32, 32, VIOLA_SCALE_F32, nullptr, 0,
+        VIOLA_CALL(viola_codes_transpose_pitched, ptr(w), temp.at(wt), count, n, k, space.pitch, ptr(scale), temp.at(wts), 32, 32, VIOLA_SCALE_F32, nullptr, 0,
                    0, nullptr, 0, stream);
         result[0] = at::empty({groups.rows, k}, options.dtype(x_dtype));
         segment_product(r, g, r.bwd, Codes{temp.at(wt), temp.at(wts), space.pitch}, w_fmt, groups, k, result[0].mutable_data_ptr(), x_dtype, stream);
     }
     if (weight_too) {
         result[1] = at::empty({count, n, k}, options.dtype(weight_grad));
+        const Codes input_t = input.in(codes.const_data_ptr());
         VIOLA_CALL(viola_varlen_wgrad_gemm, temp.at(qt), r.bwd, input_t.q, r.fwd, temp.as<float>(st), static_cast<const float*>(input_t.s), groups.padded_offsets,
                    (int)count, groups.padded, n, k, result[1].mutable_data_ptr(), code_of(weight_grad), stream);
     }
@@ -927,23 +992,24 @@ PYBIND11_MODULE(_host, m) {
         recording.store(!list.is_none());
     });
     register_optimizer(m);
+    // Each binding is wrapped so that what torch throws (out of memory, an error raised inside a hook) reaches Python as its own type.
     // None: a call for the general path
-    m.def("linear", [](const Tensor& x, const py::tuple& layer) -> std::optional<Tensor> {
+    m.def("linear", torch::wrap_pybind_function([](const Tensor& x, const py::tuple& layer) -> std::optional<Tensor> {
         Layer l = layer_from(layer);
         if (!takes(l, x.device())) return std::nullopt;
         py::gil_scoped_release release;
         return linear(x, l);
-    });
-    m.def("mlp", [](const Tensor& x, const py::tuple& up, const py::tuple& down, int activation) -> std::optional<Tensor> {
+    }));
+    m.def("mlp", torch::wrap_pybind_function([](const Tensor& x, const py::tuple& up, const py::tuple& down, int activation) -> std::optional<Tensor> {
         Layer u = layer_from(up), d = layer_from(down);
         if (!takes(u, x.device()) || !takes(d, x.device()) || u.recipe->out != 2 * d.recipe->in) return std::nullopt;
         py::gil_scoped_release release;
         return mlp(x, u, d, activation);
-    });
-    m.def("experts", [](const Tensor& x, const Tensor& weight, const Tensor& scale, const std::vector<int64_t>& counts, const std::shared_ptr<Recipe>& recipe,
-                        py::object weight_grad) {
+    }));
+    m.def("experts", torch::wrap_pybind_function([](const Tensor& x, const Tensor& weight, const Tensor& scale, const std::vector<int64_t>& counts,
+                                                    const std::shared_ptr<Recipe>& recipe, const py::object& weight_grad) {
         const at::ScalarType grad = torch::python::detail::py_object_to_dtype(weight_grad);
         py::gil_scoped_release release;
         return experts(x, weight, scale, counts, recipe, grad);
-    });
+    }));
 }

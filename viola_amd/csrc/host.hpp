@@ -74,6 +74,8 @@ public:
     void* at(int64_t offset) const { return static_cast<char*>(buffer_.mutable_data_ptr()) + offset; }
     template <typename T> T* as(int64_t offset) const { return static_cast<T*>(at(offset)); }
     void release() { buffer_ = Tensor(); }
+    const Tensor& tensor() const { return buffer_; }
+    int64_t size() const { return size_; }
 
 private:
     int64_t size_ = 0;

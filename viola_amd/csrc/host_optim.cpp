@@ -450,10 +450,11 @@ void roundtrip(const Tensor& value, const Tensor& send, int64_t tile, py::object
 namespace viola_host {
 
 void register_optimizer(py::module_& m) {
-    m.def("newton_schulz", &newton_schulz, py::arg("matrix"), py::arg("steps"), py::arg("gram"), py::call_guard<py::gil_scoped_release>());
-    m.def("roundtrip", &roundtrip);
-    py::class_<MuonHost>(m, "MuonHost").def(py::init<>()).def("step", &MuonHost::step).def_readwrite("lanes", &MuonHost::lanes)
-        .def_readwrite("batch_elements", &MuonHost::batch_elements).def("streams", &MuonHost::streams);
+    m.def("newton_schulz", torch::wrap_pybind_function_no_gil(newton_schulz), py::arg("matrix"), py::arg("steps"), py::arg("gram"));
+    m.def("roundtrip", torch::wrap_pybind_function(roundtrip));
+    py::class_<MuonHost>(m, "MuonHost").def(py::init<>())
+        .def("step", torch::wrap_pybind_function([](MuonHost& host, const py::list& work, const py::list& groups) { host.step(work, groups); }))
+        .def_readwrite("lanes", &MuonHost::lanes).def_readwrite("batch_elements", &MuonHost::batch_elements).def("streams", &MuonHost::streams);
 }
 
 }  // namespace viola_host
