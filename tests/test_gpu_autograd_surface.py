@@ -143,3 +143,35 @@ def test_a_graph_is_freed_by_its_first_backward_pass(kind, scaling):
     assert all(torch.equal(a, b) for a, b in zip(first, _gradients(module, x)))
     with pytest.raises(RuntimeError, match="second time"):
         y.backward(dy)
+
+
+SURFACES = [("linear", s) for s in RECIPES] + [("mlp", "grouped"), ("mlp", "current"), ("experts", "grouped")]
+
+
+@pytest.mark.parametrize("kind,scaling", SURFACES)
+def test_forward_mode_is_refused(kind, scaling):
+    """The modules have no forward-mode derivative: a dual input must raise, not lose its tangent."""
+    import torch.autograd.forward_ad as forward_ad
+    module, (x, _, extra) = _build(kind, scaling, {}), _inputs(kind)
+    with forward_ad.dual_level():
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            module(forward_ad.make_dual(x, torch.ones_like(x)), *extra)
+
+
+@pytest.mark.parametrize("kind,scaling", SURFACES)
+def test_functorch_transforms_are_refused(kind, scaling):
+    module, (x, _, extra) = _build(kind, scaling, {}), _inputs(kind)
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        torch.func.grad(lambda t: module(t, *extra).float().sum())(x)
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        torch.func.vmap(lambda t: module(x, *extra) + t)(torch.ones(2, 1, device="cuda"))
+
+
+@pytest.mark.parametrize("kind,scaling", SURFACES[:-1])
+def test_tracing_is_refused(kind, scaling):
+    """torch.jit has no FP8 types: a trace must fail, not record this input's output as a constant."""
+    module, (x, _, _) = _build(kind, scaling, {}), _inputs(kind)
+    for p in module.parameters():
+        p.requires_grad_(False)
+    with pytest.raises(RuntimeError):
+        torch.jit.trace(module, x, check_trace=False)

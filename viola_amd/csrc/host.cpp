@@ -70,14 +70,25 @@ bool holds(const Tensor& t, const at::Device& device, at::ScalarType type, at::I
     return t.defined() && t.device() == device && t.scalar_type() == type && t.sizes() == sizes && t.is_contiguous();
 }
 
+// Whether a framework transform is at work that sees operators and autograd functions, not these kernels: vmap, grad and the like
+// (functorch), tracing, a dispatch mode written in Python.
+bool transformed() {
+    static const c10::DispatchKeySet keys({c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::Tracer, c10::DispatchKey::Python});
+    return c10::impl::tls_local_dispatch_key_set().included_.has_any(keys);
+}
+
+// A tensor subclass with its own dispatch, or a dual number of forward-mode differentiation, whose tangent would be lost here.
+bool plain(const Tensor& t) { return !t.defined() || (!t.unsafeGetTensorImpl()->is_python_dispatch() && !t._fw_grad(0).defined()); }
+
 // Whether a layer's tensors are what the kernels here read by raw pointer: the recipe's formats and shapes, contiguous, on x's
-// device. Any other call is the general path's (nn/_grouped_linear.py, nn/_tensor_linear.py), which copies a weight whose rows
+// device, and plain. Any other call is the general path's (nn/_grouped_linear.py, nn/_tensor_linear.py), which copies a weight whose rows
 // are not contiguous, follows the weight's own FP8 format and refuses what no kernel takes.
 bool takes(const Layer& l, const at::Device& device) {
     const Recipe& r = *l.recipe;
     const int64_t rows = ceil_div(r.out, 32), cols = ceil_div(r.in, 32);
     const at::ScalarType stored = l.weight.scalar_type();
     if (r.fp8_weight ? stored != r.codes() : stored != at::kFloat && stored != at::kBFloat16 && stored != at::kHalf) return false;
+    if (!plain(l.weight) || !plain(l.bias)) return false;
     if (r.in == 0 || r.out == 0 || !device.is_cuda() || !holds(l.weight, device, stored, {r.out, r.in})) return false;
     if (r.fp8_weight && !(r.grouped ? holds(l.scale, device, r.scales(), {rows, cols}) : holds(l.scale, device, at::kFloat, {1}))) return false;
     if (l.transpose.numel() && !(holds(l.transpose, device, r.codes(), {r.in, r.out}) && (!r.grouped || holds(l.transpose_scale, device, r.scales(), {cols, rows}))))
@@ -996,18 +1007,20 @@ PYBIND11_MODULE(_host, m) {
     // None: a call for the general path
     m.def("linear", torch::wrap_pybind_function([](const Tensor& x, const py::tuple& layer) -> std::optional<Tensor> {
         Layer l = layer_from(layer);
-        if (!takes(l, x.device())) return std::nullopt;
+        if (transformed() || !plain(x) || !takes(l, x.device())) return std::nullopt;
         py::gil_scoped_release release;
         return linear(x, l);
     }));
     m.def("mlp", torch::wrap_pybind_function([](const Tensor& x, const py::tuple& up, const py::tuple& down, int activation) -> std::optional<Tensor> {
         Layer u = layer_from(up), d = layer_from(down);
-        if (!takes(u, x.device()) || !takes(d, x.device()) || u.recipe->out != 2 * d.recipe->in) return std::nullopt;
+        if (transformed() || !plain(x) || !takes(u, x.device()) || !takes(d, x.device()) || u.recipe->out != 2 * d.recipe->in) return std::nullopt;
         py::gil_scoped_release release;
         return mlp(x, u, d, activation);
     }));
     m.def("experts", torch::wrap_pybind_function([](const Tensor& x, const Tensor& weight, const Tensor& scale, const std::vector<int64_t>& counts,
                                                     const std::shared_ptr<Recipe>& recipe, const py::object& weight_grad) {
+        TORCH_CHECK_NOT_IMPLEMENTED(plain(x) && plain(weight) && plain(scale) && !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode),
+                                    "the grouped linear has neither forward-mode derivatives nor rules for functorch transforms");
         const at::ScalarType grad = torch::python::detail::py_object_to_dtype(weight_grad);
         py::gil_scoped_release release;
         return experts(x, weight, scale, counts, recipe, grad);
