@@ -131,3 +131,41 @@ def test_experts_follow_the_format_of_their_codes():
     assert rel_l2(y, want_y) < .04 and rel_l2(x.grad, want_dx) < .04
     with pytest.raises(RuntimeError, match="weight_scale"):
         viola_amd.nn.grouped_linear(x, weight, scale[:, :, :3].contiguous(), counts, grad_dtype=torch.float32)
+
+
+class _Double(torch.nn.Module):
+    def forward(self, t):
+        return 2 * t
+
+
+@pytest.mark.parametrize("scaling", ["grouped", "mxfp8", "current"])
+@pytest.mark.parametrize("native", [True, False])                                  # False: an option of the general path
+def test_parametrized_and_pruned_parameters(scaling, native):
+    """weight and bias that are attributes computed from other parameters: the products of the values they have (2 w is exact
+    in bf16), gradients to what they come from."""
+    import viola_amd
+    from torch.nn.utils import parametrize, prune
+    x, dy = _data(96, 128, 192)
+    options = dict(scaling=scaling, weight_dtype="bf16", **({} if native else dict(saved_input_dtype="bf16")))
+
+    def build():
+        torch.manual_seed(1)
+        return viola_amd.nn.Linear(128, 192, device="cuda", dtype=torch.bfloat16, **options)
+
+    module, plain = build(), build()
+    for name in ("weight", "bias"):
+        parametrize.register_parametrization(module, name, _Double())
+        getattr(plain, name).data.mul_(2)
+    y, dx, *grads = _step(module, x, dy)
+    want_y, want_dx, dw, db = _step(plain, x, dy)
+    assert torch.equal(y, want_y) and torch.equal(dx, want_dx)
+    got = {p.dim(): g for p, g in zip(module.parameters(), grads)}
+    assert rel_l2(got[2], 2 * dw) < BOUND and rel_l2(got[1], 2 * db) < BOUND          # in the parameter's own 16 bits
+
+    module, plain = build(), build()
+    prune.l1_unstructured(module, "weight", .5)
+    plain.weight.data.copy_(module.weight.data)
+    y, dx, *_ = _step(module, x, dy)
+    want = _step(plain, x, dy)
+    assert torch.equal(y, want[0]) and torch.equal(dx, want[1])
+    assert rel_l2(module.weight_orig.grad, want[2] * module.weight_mask) < BOUND

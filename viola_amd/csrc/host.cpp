@@ -366,6 +366,9 @@ struct Forward {
     Tensor y, aux;
 };
 
+// The type of a parameter's gradient. A tensor that was itself computed (a parametrized weight) has no gradient type of its own.
+at::ScalarType gradient_type(const Tensor& p) { return (p.is_leaf() ? p.grad_dtype() : std::nullopt).value_or(p.scalar_type()); }
+
 Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool need_backward, bool needs_w, Kept& kept, int gated, bool keep_aux,
                 CodedHidden* hidden_out, Kept* hidden_kept, const CodedHidden* coded_input) {
     const Recipe& r = *l.recipe;
@@ -379,8 +382,8 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
     if (need_backward) {
         kept.weight_t = l.transpose;
         kept.weight_t_scale = l.transpose_scale;
-        kept.weight_grad = l.weight.grad_dtype().value_or(l.weight.scalar_type());
-        if (l.bias.defined()) kept.bias_grad = l.bias.grad_dtype().value_or(l.bias.scalar_type());
+        kept.weight_grad = gradient_type(l.weight);
+        if (l.bias.defined()) kept.bias_grad = gradient_type(l.bias);
     }
     const auto options = at::TensorOptions().dtype(dtype).device(device);
     const int64_t h = r.out / 2;

@@ -20,6 +20,11 @@ def _scale_dtype(native):
     return torch.uint8 if native else torch.float32
 
 
+def gradient_dtype(parameter):
+    """The type of a parameter's gradient. A tensor that was itself computed (a parametrized weight) has none of its own."""
+    return (parameter.grad_dtype if parameter.is_leaf else None) or parameter.dtype
+
+
 def decode_scale(scale):
     """E8M0 bytes -> the FP32 scales they stand for (exact); FP32 scales pass through."""
     return torch.exp2(scale.float() - 127.) if scale.dtype == torch.uint8 else scale

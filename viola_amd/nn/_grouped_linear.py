@@ -74,8 +74,8 @@ def forward_core(x, weight, bias, layer, need_backward, needs, *, gated=None, en
             saved_x, saved_scale = x2.new_empty(0), x2.new_empty(0)
         record = SimpleNamespace(tensors=(saved_x, saved_scale, weight, sw, wt, st), layer=layer, shape=shape,
                                  x_dtype=x_dtype, save_fp8=save_fp8, input_limit=limit,
-                                 weight_grad_dtype=weight.grad_dtype or weight.dtype,
-                                 bias_grad_dtype=(bias.grad_dtype or bias.dtype) if bias is not None else None)
+                                 weight_grad_dtype=kernels.gradient_dtype(weight),
+                                 bias_grad_dtype=kernels.gradient_dtype(bias) if bias is not None else None)
     if encode[0]:
         return (y, *extra), aux, record
     return y.reshape(*shape[:-1], y.shape[-1]), aux, record

@@ -11,7 +11,7 @@ from types import SimpleNamespace
 
 import torch
 
-from . import _gated_kernels
+from . import _gated_kernels, _grouped_kernels
 from . import _linear_kernels as kernels
 from . import _mlp_kernels
 from . import _rotation_kernels as rotation
@@ -54,8 +54,8 @@ def forward_core(x, weight, bias, layer, need_backward, needs, *, gated=None):
         # the scales this very forward used, not the quantizers' mutable state
         record = SimpleNamespace(tensors=(saved_x, sx, weight, sw, wt), layer=layer, shape=shape, x_dtype=x2.dtype,
                                  save_fp8=save_fp8, input_limit=input_limit,
-                                 weight_grad_dtype=weight.grad_dtype or weight.dtype,
-                                 bias_grad_dtype=(bias.grad_dtype or bias.dtype) if bias is not None else None)
+                                 weight_grad_dtype=_grouped_kernels.gradient_dtype(weight),
+                                 bias_grad_dtype=_grouped_kernels.gradient_dtype(bias) if bias is not None else None)
     return y.reshape(*shape[:-1], y.shape[-1]), aux, record
 
 

@@ -345,12 +345,15 @@ class Linear(nn.Module):
 
     # ------------------------------------------------------------------ execution
     def _operands(self):
-        """What the native host path needs of this layer (its `layer_from`), read without nn.Module's attribute search."""
+        """What the native host path needs of this layer (its `layer_from`), read without nn.Module's attribute search where the
+        parameters are plain ones (a parametrization or pruning turns them into attributes)."""
         recipe = self._recipe
         if recipe is None:
             recipe = self._recipe = self._numerics.native_recipe(self)
         held, buffers = self._parameters, self._buffers
-        operands = (recipe, held["weight"], held.get("bias"), buffers["weight_scale"], buffers["weight_transpose"], buffers["weight_transpose_scale"])
+        weight = held["weight"] if "weight" in held else self.weight
+        bias = held["bias"] if "bias" in held else self.bias
+        operands = (recipe, weight, bias, buffers["weight_scale"], buffers["weight_transpose"], buffers["weight_transpose_scale"])
         if self._grouped_scaling:
             return operands
         quantizers = [self._modules[name] for name in ("weight_quantizer", "input_quantizer", "grad_quantizer")]
