@@ -71,3 +71,25 @@ def test_wire_round_trip_in_one_pass_equals_pack_then_unpack(tile, n, fp8):
     _lib.call("viola_comm_pack", x.data_ptr(), n, packets[1].data_ptr(), 1, groups, tile, _lib.code(fp8))
     _lib.call("viola_comm_unpack", packets[1].data_ptr(), want.data_ptr(), n, 1, groups, tile, _lib.code(fp8), 0)
     assert torch.equal(packets[0], packets[1]) and torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("shape,key", [((64, 128), "momentum_q"), ((64, 128), "momentum_scale"), ((96,), "exp_avg"), ((96,), "exp_avg_sq")])
+@pytest.mark.parametrize("how", ["host", "short"])
+def test_state_that_is_not_where_the_kernels_read_is_refused(shape, key, how):
+    """State offloaded to the host, or cut, must be refused before anything is launched: the kernels read it by address."""
+    import viola_amd
+    params = [torch.nn.Parameter(torch.randn(*shape, device="cuda")) for _ in range(3)]
+    opt = viola_amd.optim.FP8Muon(params, lr=1e-3)
+    for p in params:
+        p.grad = torch.randn_like(p)
+    opt.step()
+    state = opt.state[params[1]]
+    held = state[key]
+    state[key] = held.cpu() if how == "host" else held[:held.numel() // 2]
+    before = [p.detach().clone() for p in params]
+    with pytest.raises(RuntimeError, match="state of a parameter"):
+        opt.step()
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(before, params))
+    state[key] = held
+    opt.step()

@@ -236,6 +236,13 @@ private:
         return t.arena.as<int64_t>(t.at);
     }
 
+    // The state is the caller's: it may have been loaded, moved to the host or replaced, and the kernels read it by raw pointer.
+    static void check_state(const Item& it, const Tensor& state, int64_t elements, int64_t bytes_each) {
+        TORCH_CHECK(state.device() == it.param.device() && state.is_contiguous() && state.numel() >= elements && state.element_size() == bytes_each,
+                    "FP8Muon: the state of a parameter of ", it.param.numel(), " elements must be contiguous on ", it.param.device(), " with at least ", elements,
+                    " elements of ", bytes_each, " bytes, it has ", state.numel(), " of ", state.element_size(), " on ", state.device());
+    }
+
     static void prepare_vector(Item& it) {
         if (!it.state.contains("exp_avg")) {
             const auto options = at::TensorOptions().dtype(it.group->adam_state);
@@ -244,24 +251,28 @@ private:
         }
         it.first = it.state["exp_avg"].cast<Tensor>();
         it.second = it.state["exp_avg_sq"].cast<Tensor>();
+        check_state(it, it.first, it.param.numel(), it.first.element_size());
+        check_state(it, it.second, it.param.numel(), it.first.element_size());
     }
 
     static void prepare_matrix(Item& it) {
         TORCH_CHECK(it.param.dim() >= 2, "Muon updates matrices: a vector in a use_muon=True group");
+        // 1-D tiles pad the payload to whole tiles, 2-D blocks do not
+        const Group& g = *it.group;
+        const std::vector<int64_t> shape = matrix_shape(it.param, g);
+        const int64_t n = it.param.numel(), rows = shape[shape.size() - 2], cols = shape.back();
+        int64_t payload = n, scales = ceil_div(n, g.tile);
+        if (g.granularity == 0) payload = scales * g.tile;
+        else scales = rows * cols ? n / (rows * cols) * ceil_div(rows, g.block_rows) * ceil_div(cols, g.block_cols) : 0;
         if (!it.state.contains("momentum_q")) {
-            // 1-D tiles pad the payload to whole tiles, 2-D blocks do not
-            const Group& g = *it.group;
-            const std::vector<int64_t> shape = matrix_shape(it.param, g);
-            const int64_t n = it.param.numel(), rows = shape[shape.size() - 2], cols = shape.back();
-            int64_t payload = n, scales = ceil_div(n, g.tile);
-            if (g.granularity == 0) payload = scales * g.tile;
-            else scales = rows * cols ? n / (rows * cols) * ceil_div(rows, g.block_rows) * ceil_div(cols, g.block_cols) : 0;
             const auto options = at::TensorOptions().device(it.param.device());
             it.state["momentum_q"] = py::cast(at::zeros({payload}, options.dtype(at::kByte)));
             it.state["momentum_scale"] = py::cast(at::ones({scales}, options.dtype(at::kFloat)));
         }
         it.q = it.state["momentum_q"].cast<Tensor>();
         it.scale = it.state["momentum_scale"].cast<Tensor>();
+        check_state(it, it.q, payload, 1);
+        check_state(it, it.scale, scales, 4);
     }
 
     // The chains of different buckets are independent, and a single chain leaves the GPU partly idle at every launch boundary
@@ -431,7 +442,8 @@ private:
 // value <- decode(encode(value)) through the packet buffer
 void roundtrip(const Tensor& value, const Tensor& send, int64_t tile, py::object format) {
     const int code = code_of(torch::python::detail::py_object_to_dtype(format));
-    TORCH_CHECK(value.is_cuda() && value.scalar_type() == at::kFloat && value.is_contiguous() && send.is_cuda() && send.is_contiguous());
+    TORCH_CHECK(value.is_cuda() && value.scalar_type() == at::kFloat && value.is_contiguous(), "the codec takes contiguous FP32 values on the GPU");
+    TORCH_CHECK(send.device() == value.device() && send.scalar_type() == at::kByte && send.is_contiguous(), "the packet buffer is on ", send.device(), ", the values on ", value.device());
     const int64_t groups = ceil_div(value.numel(), tile);
     TORCH_CHECK(ceil_to(groups * (tile + 4), 16) <= send.numel(), "the bucket exceeds the codec's capacity");
     if (value.numel() == 0) return;
