@@ -22,22 +22,24 @@ using torch::autograd::variable_list;
 namespace {
 
 // ---------------------------------------------------------------------------------------------------- recipes
-// Calls of one per-tensor quantizer so far (its slot in the amax history); shared with nodes that advance it in backward.
+// State of one per-tensor quantizer, shared with its module and with nodes that advance it in backward: calls so far (its slot in
+// the amax history), and whether its scale is that of the history (a checkpoint brings this along, so it may change).
 struct Counter {
     int64_t value = 0;
+    bool delayed = false;
 };
 
 // What a Linear's constructor fixed about its arithmetic. Standard recipes only: (1, 32) activation and gradient groups,
 // (32, 32) weight blocks, FP32 accumulation, no rotation, FP8-saved inputs.
 struct Recipe {
-    bool grouped = false, native = false, delayed = false;      // native: E8M0 scales; not grouped: one FP32 scale per tensor
+    bool grouped = false, native = false;      // native: E8M0 scales; not grouped: one FP32 scale per tensor
     bool fp8_weight = true, cache_transpose = false;
     int fwd = VIOLA_E4M3, bwd = VIOLA_E4M3;
     float fwd_limit = 448.0f, bwd_limit = 448.0f;
     int64_t in = 0, out = 0;
 
     explicit Recipe(const py::dict& d) {
-        grouped = d["grouped"].cast<bool>(); native = d["native"].cast<bool>(); delayed = d["delayed"].cast<bool>();
+        grouped = d["grouped"].cast<bool>(); native = d["native"].cast<bool>();
         fp8_weight = d["fp8_weight"].cast<bool>(); cache_transpose = d["cache_transpose"].cast<bool>();
         fwd = d["fwd"].cast<int>(); bwd = d["bwd"].cast<int>();
         fwd_limit = d["fwd_limit"].cast<float>(); bwd_limit = d["bwd_limit"].cast<float>();
@@ -45,7 +47,7 @@ struct Recipe {
     }
     py::dict fields() const {                                    // for copies and pickles of a module
         using namespace py::literals;
-        return py::dict("grouped"_a = grouped, "native"_a = native, "delayed"_a = delayed, "fp8_weight"_a = fp8_weight,
+        return py::dict("grouped"_a = grouped, "native"_a = native, "fp8_weight"_a = fp8_weight,
                         "cache_transpose"_a = cache_transpose, "fwd"_a = fwd, "bwd"_a = bwd, "fwd_limit"_a = fwd_limit, "bwd_limit"_a = bwd_limit,
                         "in"_a = in, "out"_a = out);
     }
@@ -338,7 +340,7 @@ Codes stored_weight(const Layer& l, const Tensor& weight, const WeightSpace& w, 
             c = {temp.at(w.q), scale_out, r.in};
             const Tensor& history = l.history[WEIGHT];
             VIOLA_CALL(viola_tensor_encode, ptr(weight), dtype, r.out, r.in, maxima.as<float>(at), 1024, static_cast<float*>(history.mutable_data_ptr()),
-                       (int)history.numel(), l.counter[WEIGHT]->value, r.delayed, r.fwd_limit, scale_out, temp.at(w.q), r.in, nullptr, 0, r.fwd, nullptr,
+                       (int)history.numel(), l.counter[WEIGHT]->value, l.counter[WEIGHT]->delayed, r.fwd_limit, scale_out, temp.at(w.q), r.in, nullptr, 0, r.fwd, nullptr,
                        VIOLA_F32, stream);
             ++l.counter[WEIGHT]->value;
         }
@@ -405,7 +407,7 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
     auto quantized_inside = [&] {
         if (!plain || need_backward || coded_input || !r.fp8_weight || x2.element_size() != 2 || !small_product(rows, r.out)) return false;
         if ((rows > 16 && rows * r.out > 256 * 16 * 32 ? 2 : 1) * r.in > QUANTIZED_IN_PRODUCT) return false;
-        if (!r.grouped && (rows * r.in > WHOLE_TENSOR || (r.delayed && l.counter[INPUT]->value))) return false;
+        if (!r.grouped && (rows * r.in > WHOLE_TENSOR || (l.counter[INPUT]->delayed && l.counter[INPUT]->value))) return false;
         const void* bias_p = ptr(l.bias);
         float* history = r.grouped ? nullptr : static_cast<float*>(l.history[INPUT].mutable_data_ptr());
         const int64_t slot = r.grouped ? 0 : l.counter[INPUT]->value % l.history[INPUT].numel();
@@ -445,7 +447,7 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
             float* sx = kept.arena.as<float>(scales);
             const Tensor& history = l.history[INPUT];
             VIOLA_CALL(viola_tensor_encode, ptr(x2), code_of(x2.scalar_type()), rows, r.in, temp.as<float>(maxima), 1024,
-                       static_cast<float*>(history.mutable_data_ptr()), (int)history.numel(), l.counter[INPUT]->value, r.delayed, r.fwd_limit, sx, temp.at(q),
+                       static_cast<float*>(history.mutable_data_ptr()), (int)history.numel(), l.counter[INPUT]->value, l.counter[INPUT]->delayed, r.fwd_limit, sx, temp.at(q),
                        pitch, save ? kept.arena.at(qt) : nullptr, save ? pitch_t : 0, r.fwd, nullptr, VIOLA_F32, stream);
             ++l.counter[INPUT]->value;
             a = {temp.at(q), sx, pitch};
@@ -574,7 +576,7 @@ Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const T
         const Tensor& history = l.history[GRAD];
         auto encode = [&](bool with_sum) {
             return VIOLA_TRY(viola_tensor_encode, ptr(dy), dtype, rows, r.out, temp.as<float>(work_at), floats, static_cast<float*>(history.mutable_data_ptr()),
-                             (int)history.numel(), l.counter[GRAD]->value, r.delayed, r.bwd_limit, scale, needs_x ? temp.at(q) : nullptr, pitch,
+                             (int)history.numel(), l.counter[GRAD]->value, l.counter[GRAD]->delayed, r.bwd_limit, scale, needs_x ? temp.at(q) : nullptr, pitch,
                              needs_w ? temp.at(qt) : nullptr, pitch_t, r.bwd, with_sum ? out.db.mutable_data_ptr() : nullptr,
                              with_sum ? code_of(kept.bias_grad) : VIOLA_F32, stream);
         };
@@ -994,9 +996,10 @@ Layer layer_from(const py::tuple& t) {
 PYBIND11_MODULE(_host, m) {
     event_class = new py::object(py::module_::import("torch.cuda").attr("Event"));
     py::class_<Counter, std::shared_ptr<Counter>>(m, "Counter")
-        .def(py::init([](int64_t value) { auto c = std::make_shared<Counter>(); c->value = value; return c; }), py::arg("value") = 0)
+        .def(py::init([](int64_t value, bool delayed) { return std::make_shared<Counter>(Counter{value, delayed}); }), py::arg("value") = 0, py::arg("delayed") = false)
         .def_readwrite("value", &Counter::value)
-        .def("__reduce__", [](py::object self) { return py::make_tuple(self.attr("__class__"), py::make_tuple(self.attr("value"))); });
+        .def_readwrite("delayed", &Counter::delayed)
+        .def("__reduce__", [](py::object self) { return py::make_tuple(self.attr("__class__"), py::make_tuple(self.attr("value"), self.attr("delayed"))); });
     py::class_<Recipe, std::shared_ptr<Recipe>>(m, "Recipe")
         .def(py::init<const py::dict&>())
         .def("__reduce__", [](py::object self) { return py::make_tuple(self.attr("__class__"), py::make_tuple(self.cast<Recipe&>().fields())); });

@@ -26,7 +26,7 @@ GX, GW = (1, 32), (32, 32)
 def _recipe(forward_dtype, backward_dtype):
     """The recipe of the native host path (csrc/host.cpp), which runs forward and backward."""
     forward, backward = _FORMATS[forward_dtype], _FORMATS[backward_dtype]
-    return _lib.host().Recipe({"grouped": True, "native": False, "delayed": False, "fp8_weight": True, "cache_transpose": False,
+    return _lib.host().Recipe({"grouped": True, "native": False, "fp8_weight": True, "cache_transpose": False,
                                "fwd": _lib.code(forward), "bwd": _lib.code(backward), "fwd_limit": torch.finfo(forward).max,
                                "bwd_limit": torch.finfo(backward).max, "in": 0, "out": 0})
 

@@ -42,8 +42,19 @@ class _Quantizer(nn.Module):
 
     def __init__(self, scaling, history_len, device):
         super().__init__()
-        self.scaling, self._calls, self._counter = scaling, 0, None
+        self._calls, self._counter = 0, None
+        self.scaling = scaling
         self.register_buffer("history", torch.zeros(history_len, device=device, dtype=torch.float32))
+
+    @property
+    def scaling(self):
+        return self._scaling
+
+    @scaling.setter
+    def scaling(self, value):
+        self._scaling = value
+        if self._counter is not None:
+            self._counter.delayed = value == "delayed"
 
     @property
     def index(self):
@@ -60,7 +71,7 @@ class _Quantizer(nn.Module):
     def counter(self):
         """The counter itself, shared with the native host path (backward advances it off this thread)."""
         if self._counter is None:
-            self._counter = _lib.host().Counter(self._calls)
+            self._counter = _lib.host().Counter(self._calls, self._scaling == "delayed")
         return self._counter
 
     def _options(self, fp8_dtype, quantization_limit):
@@ -134,19 +145,17 @@ class _Numerics:
     def tensor_limit(self, reduction, dtype):
         return self._clamp(self.accum_block_size or reduction, dtype)                      # linear.py:232-242
 
-    def standard(self, saved_input_dtype):
-        """Whether the native host path takes this recipe: the default group shapes, FP32 accumulation, no rotation, inputs
-        saved as FP8."""
-        groups = (self.weight_group_shape, self.input_group_shape, self.grad_group_shape)
-        return (groups == ((32, 32), (1, 32), (1, 32)) and self.accum_dtype == "fp32" and not self.rotation_size and saved_input_dtype == "fp8")
-
     def native_recipe(self, layer):
+        """The layer's recipe for the native host path, or False where that does not take it: it runs the default group shapes,
+        FP32 accumulation, no rotation, inputs saved as FP8."""
+        groups = (layer.weight_group_shape, layer.input_group_shape, layer.grad_group_shape)
+        if groups != ((32, 32), (1, 32), (1, 32)) or layer.accum_dtype != "fp32" or layer.rotation_size or layer.saved_input_dtype != "fp8":
+            return False
         limit = lambda dtype: float(self._clamp(1, dtype) or torch.finfo(dtype).max)
         return _lib.host().Recipe({
-            "grouped": self._grouped_scaling, "native": self._native_scaling, "delayed": layer.input_quantizer.scaling == "delayed",
-            "fp8_weight": layer.weight_dtype == "fp8", "cache_transpose": layer.cache_weight_transpose, "fwd": _lib.code(self.fp8_dtype),
-            "bwd": _lib.code(self.backward_fp8_dtype), "fwd_limit": limit(self.fp8_dtype), "bwd_limit": limit(self.backward_fp8_dtype),
-            "in": layer.in_features, "out": layer.out_features})
+            "grouped": layer._grouped_scaling, "native": layer._native_scaling, "fp8_weight": layer.weight_dtype == "fp8",
+            "cache_transpose": layer.cache_weight_transpose, "fwd": _lib.code(layer.fp8_dtype), "bwd": _lib.code(layer.backward_fp8_dtype),
+            "fwd_limit": limit(layer.fp8_dtype), "bwd_limit": limit(layer.backward_fp8_dtype), "in": layer.in_features, "out": layer.out_features})
 
     def scale_storage(self, weight_shape, fp8_storage):
         """(shape, dtype, initial value) of `weight_scale`: FP32 scales start at 1, E8M0 bytes at 127 = 2^0
@@ -229,6 +238,10 @@ class Linear(nn.Module):
     weights as storage; dequantize_weight() returns real weights in the original coordinates.
     """
 
+    # Options that are read at every call: changing one drops the native host path's recipe, which was made from them.
+    _RECIPE_OPTIONS = frozenset(("in_features", "out_features", "fp8_dtype", "backward_fp8_dtype", "_grouped_scaling", "_native_scaling",
+                                 "weight_group_shape", "input_group_shape", "grad_group_shape", "weight_dtype", "saved_input_dtype",
+                                 "cache_weight_transpose", "rotation_size", "accum_dtype"))
     _KEPT_BUFFERS = ("weight_scale", "weight_transpose", "weight_transpose_scale")
 
     def __init__(self, in_features, out_features, bias=True, *, mode="memory", weight_dtype="fp8",
@@ -250,12 +263,16 @@ class Linear(nn.Module):
         self.mode, self.weight_dtype, self.saved_input_dtype, self.autotune = mode, weight_dtype, saved_input_dtype, autotune
         self.cache_weight_transpose = (mode == "fast") if cache_weight_transpose is None else cache_weight_transpose
         self._store = _WeightStore(self)
-        self._standard, self._recipe = numerics.standard(saved_input_dtype), None
         self._master_ref = None
         self._allocate(bias, device, dtype or torch.get_default_dtype(), settings())
         for operand in ("weight", "input", "grad"):
             setattr(self, f"{operand}_quantizer", _Quantizer(scaling, history_len, device))
         self.reset_parameters()
+
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        if name in self._RECIPE_OPTIONS:
+            self.__dict__["_recipe"] = None
 
     def _allocate(self, bias, device, dtype, policy):
         """Parameters and buffers under the reference's names (linear.py:203-226). With FP8 storage the initial
@@ -346,10 +363,12 @@ class Linear(nn.Module):
     # ------------------------------------------------------------------ execution
     def _operands(self):
         """What the native host path needs of this layer (its `layer_from`), read without nn.Module's attribute search where the
-        parameters are plain ones (a parametrization or pruning turns them into attributes)."""
+        parameters are plain ones (a parametrization or pruning turns them into attributes). None: an option it does not take."""
         recipe = self._recipe
         if recipe is None:
-            recipe = self._recipe = self._numerics.native_recipe(self)
+            recipe = self.__dict__["_recipe"] = self._numerics.native_recipe(self)
+        if recipe is False:
+            return None
         held, buffers = self._parameters, self._buffers
         weight = held["weight"] if "weight" in held else self.weight
         bias = held["bias"] if "bias" in held else self.bias
@@ -366,8 +385,9 @@ class Linear(nn.Module):
         if self._store.pending:
             self.refresh_weight(self._master())
             assert not self._store.pending, _HOST_MASTER
-        if self._standard:
-            y = _lib.host().linear(x, self._operands())
+        operands = self._operands()
+        if operands is not None:
+            y = _lib.host().linear(x, operands)
             if y is not None:                                                  # None: operands only the general path takes
                 return y
         trainable = [t for t in (x, self.weight, self.bias) if t is not None and t.requires_grad]
