@@ -139,8 +139,11 @@ class _Binding:
         self.slots = list(by_param.values())
         if self.matrix:
             optimizer._partition = None
-        optimizer.register_step_pre_hook(self._before_step)
-        optimizer.register_step_post_hook(self._after_step)
+        if self.matrix:
+            optimizer.bind_step(self._before_step, self._after_step)
+        else:
+            optimizer.register_step_pre_hook(self._before_step)
+            optimizer.register_step_post_hook(self._after_step)
         optimizer.register_state_dict_post_hook(self._on_save)
         optimizer.register_load_state_dict_pre_hook(self._on_load)
         optimizer.register_load_state_dict_post_hook(self._after_load)

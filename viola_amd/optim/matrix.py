@@ -3,11 +3,23 @@
 gather/scatter and mesh all-reduces of the reference are not part of this build."""
 
 import functools
-from itertools import chain
 
 import torch
 from torch.autograd import profiler
-from torch.optim.optimizer import _global_optimizer_post_hooks, _global_optimizer_pre_hooks
+from torch.optim import optimizer as stock
+
+# torch.optim puts a profiler range around `step` and `zero_grad`; entering and leaving one costs about 6 us of host time, which a
+# small model's step waits for. Whether anyone is looking is not public: the short way exists for the PyTorch version whose
+# names are these (2.10), everywhere else and whenever anybody is looking the stock methods run.
+_KNOWN = torch.__version__.startswith("2.10.") and hasattr(profiler, "_is_profiler_enabled")
+
+
+def _unobserved():
+    return _KNOWN and not profiler._is_profiler_enabled
+
+
+def _no_global_hooks():
+    return not stock._global_optimizer_pre_hooks and not stock._global_optimizer_post_hooks
 
 
 class MatrixOptimizer(torch.optim.Optimizer):
@@ -19,42 +31,53 @@ class MatrixOptimizer(torch.optim.Optimizer):
         self.skip_nonfinite = skip_nonfinite
         self.step_was_skipped = False
         self._partition = None
+        self._caller_hooks, self._bound = False, None
         super().__init__(params, defaults)
         self.register_load_state_dict_pre_hook(self._before_load)
         self.register_load_state_dict_post_hook(self._after_load)
 
+    def bind_step(self, before, after):
+        """Hooks of the master binding around every step. They are ordinary step hooks, which the stock `step` runs among the
+        others; the short way calls them itself."""
+        assert self._bound is None
+        super().register_step_pre_hook(before)
+        super().register_step_post_hook(after)
+        self._bound = (before, after)
+
+    def register_step_pre_hook(self, hook):
+        self._caller_hooks = True
+        return super().register_step_pre_hook(hook)
+
+    def register_step_post_hook(self, hook):
+        self._caller_hooks = True
+        return super().register_step_post_hook(hook)
+
     @staticmethod
     def profile_hook_step(func):
-        """The stock wrapper of `step` (hooks before and after, a profiler range around) without the range while no profiler
-        runs: entering and leaving one costs about 6 us of host time, which a small model's step waits for."""
-        recorded = torch.optim.Optimizer.profile_hook_step(func)
+        """What torch.optim makes of a subclass's `step`. A plain `step()` without anybody's hooks but the binding's goes straight
+        to `func`; any other runs the stock wrapper, which alone knows the order of hooks and what they may replace."""
+        wrapped = torch.optim.Optimizer.profile_hook_step(func)
 
         @functools.wraps(func)
-        def wrapper(self, *args, **kwargs):
-            if profiler._is_profiler_enabled:
-                return recorded(self, *args, **kwargs)
-            args = (self, *args)
-            for hook in chain(_global_optimizer_pre_hooks.values(), self._optimizer_step_pre_hooks.values()):
-                result = hook(self, args, kwargs)
-                if result is not None:
-                    if not (isinstance(result, tuple) and len(result) == 2):
-                        raise RuntimeError(f"{func} must return None or a tuple of (new_args, new_kwargs), but got {result}.")
-                    args, kwargs = result
-            out = func(*args, **kwargs)
-            self._optimizer_step_code()
-            for hook in chain(self._optimizer_step_post_hooks.values(), _global_optimizer_post_hooks.values()):
-                hook(self, args, kwargs)
-            return out
+        def step(self, *args, **kwargs):
+            # an optimizer that was unpickled has neither attribute (torch keeps its state and groups only): the stock way
+            if args or kwargs or self.__dict__.get("_caller_hooks", True) or not (_unobserved() and _no_global_hooks()):
+                return wrapped(self, *args, **kwargs)
+            if self._bound is None:
+                return func(self)
+            self._bound[0](self, (self,), {})
+            result = func(self)
+            self._bound[1](self, (self,), {})
+            return result
 
-        return wrapper
+        return step
 
     def zero_grad(self, set_to_none=True):
-        if not set_to_none or profiler._is_profiler_enabled:
+        if not set_to_none or not _unobserved():
             return super().zero_grad(set_to_none)
         for group in self.param_groups:
             for param in group["params"]:
-                if param.grad is not None:
-                    param.grad = None
+                param.grad = None
 
     def _step_local(self, parameter, gradient, state, group, index):
         raise NotImplementedError
