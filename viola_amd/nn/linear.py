@@ -42,8 +42,7 @@ class _Quantizer(nn.Module):
 
     def __init__(self, scaling, history_len, device):
         super().__init__()
-        self._calls, self._counter = 0, None
-        self.scaling = scaling
+        self.__dict__.update(_calls=0, _counter=None, _scaling=scaling)
         self.register_buffer("history", torch.zeros(history_len, device=device, dtype=torch.float32))
 
     @property
@@ -257,13 +256,12 @@ class Linear(nn.Module):
                              accum_reduce_dtype, quantization_limit, rotation_size, weight_group_shape,
                              input_group_shape, grad_group_shape)
         self._numerics = numerics
-        for field in _Numerics.FIELDS:                                         # the attributes the autograd functions read
-            setattr(self, field, getattr(numerics, field))
-        self.in_features, self.out_features = in_features, out_features
-        self.mode, self.weight_dtype, self.saved_input_dtype, self.autotune = mode, weight_dtype, saved_input_dtype, autotune
-        self.cache_weight_transpose = (mode == "fast") if cache_weight_transpose is None else cache_weight_transpose
+        # the attributes the autograd functions read (plain values, written without nn.Module's search for what they might be)
+        self.__dict__.update({field: getattr(numerics, field) for field in _Numerics.FIELDS})
+        self.__dict__.update(in_features=in_features, out_features=out_features, mode=mode, weight_dtype=weight_dtype,
+                             saved_input_dtype=saved_input_dtype, autotune=autotune, _recipe=None, _master_ref=None,
+                             cache_weight_transpose=(mode == "fast") if cache_weight_transpose is None else cache_weight_transpose)
         self._store = _WeightStore(self)
-        self._master_ref = None
         self._allocate(bias, device, dtype or torch.get_default_dtype(), settings())
         for operand in ("weight", "input", "grad"):
             setattr(self, f"{operand}_quantizer", _Quantizer(scaling, history_len, device))
