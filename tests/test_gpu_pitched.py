@@ -194,3 +194,45 @@ def test_variable_groups_on_sizes_that_are_multiples_of_nothing(bf16_gradients, 
         want = ol.linear(x[rows], w, torch.zeros(n_out), dy[rows])
         for got, key in ((y[rows], "y"), (xg.grad[rows], "dx"), (experts.weight.grad[g], "dw")):
             assert rel_l2(got, want[key]) < 4e-3, (g, key)
+
+
+@pytest.mark.parametrize("tokens,n_in,n_out", [(500, 512, 512), (1001, 1024, 1024), (3001, 1024, 1024), (2049, 512, 512), (1533, 256, 300)])
+def test_step_behind_a_ragged_token_count_differs_by_the_order_of_the_sums(bf16_gradients, tokens, n_in, n_out):
+    """A padded pitch takes the weight gradient off the guarded kernel, which adds the 32-k groups in ascending order, to kernels
+    that for few tiles and k >= 1024 add two halves of the k range separately. Below that nothing changes. Above it FP32 sums
+    differ by about sqrt(k / 32) 2^-24, a bf16 ulp is 2^-8 of the value: one gradient element in 10^4 rounds the other way
+    (measured 0.7 to 2.3e-4), one momentum code in 10^5 (at most 2e-5 over 768 x 3072), by one step in the first step. The
+    Newton-Schulz products spread that over the update: 1e-4 of the master's norm, and 0.2 to 0.5 % of the FP8 weights lie
+    so near a rounding edge that they take the neighbouring code. Bounds are four times what was measured."""
+    from viola_amd import nn, optim
+    from viola_amd.nn import _grouped_kernels as g
+
+    def build():
+        torch.manual_seed(0)
+        module = nn.Linear(n_in, n_out, device="cuda", dtype=torch.bfloat16, scaling="grouped", backward_dtype="e4m3")
+        optimizer = optim.bind_optimizer(module, optim.FP8Muon(module.parameters(), lr=1e-3, weight_decay=.01))
+        return module, optimizer, next(p for p in optimizer.param_groups[0]["params"] if p.dim() == 2)
+
+    torch.manual_seed(10)
+    x, dy = torch.randn(tokens, n_in, device="cuda").bfloat16(), (torch.randn(tokens, n_out, device="cuda") * 1e-2).bfloat16()
+    gt, sgt = g.quantize_dual(dy, E4, (1, 32))[2:]
+    xt, sxt = g.quantize_dual(x, E4, (1, 32))[2:]
+    ascending = g.gemm(gt, xt, sgt, sxt, (1, 32), (1, 32), out_dtype=torch.bfloat16)      # rows of `tokens` codes: the guarded kernel
+    (a, opt_a, master_a), (b, opt_b, master_b) = build(), build()
+    for module in (a, b):
+        module(x).backward(dy)
+    gradient = a.weight.grad.clone()
+    b.weight.grad = ascending.clone()
+    opt_a.step()
+    opt_b.step()
+    differ = lambda p, q: (p != q).float().mean().item()
+    codes = [opt.state[master]["momentum_q"] for opt, master in ((opt_a, master_a), (opt_b, master_b))]
+    weights = [m.weight.detach().float() for m in (a, b)]
+    real = [m.dequantize_weight() for m in (a, b)]
+    if -(-tokens // 128) * 128 < 1024:
+        assert torch.equal(gradient, ascending) and torch.equal(*codes) and torch.equal(*weights) and torch.equal(master_a, master_b)
+        return
+    assert rel_l2(gradient, ascending) < 1e-4 and 0 < differ(gradient, ascending) < 1e-3
+    assert differ(*codes) < 1e-4 and (codes[0].int() - codes[1].int()).abs().max().item() <= 1
+    assert rel_l2(master_a, master_b) < 5e-4
+    assert differ(*weights) < .02 and rel_l2(*real) < 5e-3                                # a code step is 1/8 of a value: sqrt(.005) / 16
