@@ -63,7 +63,7 @@ bool launch_gated_pieces(const void* z, const void* dy, int64_t dy_stride, void*
                          int activation, bool backward, bool epilogue_form, hipStream_t stream);
 
 // Which kernel a plain per-tensor or block-scaled product runs on: gemm_pingpong with tiles of 256 x 256 (L), 256 x 128 (M) or
-// 128 x 128 (S), or group_gemm_fast (128 x 128 with several blocks per CU; below 128 such tiles its narrow and split forms).
+// 128 x 128 (S), or group_gemm_fast (from 512 tiles of 128 x 128 up with several blocks per CU, below 128 with halved tiles).
 // The choice is the least of four estimates in microseconds, fitted to the measured times of 27 shapes (bf16 outputs; within
 // 15 % of each). A round of one tile per CU takes a fixed part (first loads, stores of the tile) and a time per chunk of 64 k
 // that grows with the share of CUs at work, because the clock falls as the matrix pipes fill (2.4 to 1.7 GHz):

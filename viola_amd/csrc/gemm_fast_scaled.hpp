@@ -7,7 +7,7 @@ namespace viola {
 
 // Per-tensor scales (TENSOR: args.sa / args.sb point at one float each) or E8M0 block scales (MX: they point at
 // bytes; ldsa / ldsb = bytes per scale row). grid: (n tiles, m tiles of 128); n tiles are 128 wide, 64 for gated forward.
-// KSPLIT: the k range of a 128 x 128 tile split over two teams of waves in a 512-thread block (plain mode)
+// KSPLIT: the k range of a 128 x 64 tile split over two teams of waves in a 512-thread block (plain mode)
 template <int MODE, typename TO, int TN, bool TENSOR, bool MX, bool KSPLIT = false>
 static void launch_scaled_formats(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, dim3 grid, hipStream_t stream) {
     const bool a5 = a_dtype == VIOLA_E5M2, b5 = b_dtype == VIOLA_E5M2;
@@ -18,9 +18,9 @@ static void launch_scaled_formats(const GemmArgs& p, int a_dtype, int b_dtype, i
     else VIOLA_LAUNCH((group_gemm_fast<MODE, true, true, false, TO, TN, TENSOR, MX, KSPLIT>), grid, block, 0, stream, p, bias_dtype);
 }
 
-#ifndef VIOLA_SCALED_SPLIT_MIN_K
-#define VIOLA_SCALED_SPLIT_MIN_K 2048
-#endif
+// shortest k range that the narrow tiles split
+constexpr int64_t SCALED_SPLIT_MIN_K = 2048;
+
 template <bool TENSOR, bool MX>
 static int launch_scaled_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, dim3 grid,
                                    hipStream_t stream) {
@@ -37,13 +37,10 @@ static int launch_scaled_gemm_fast(const GemmArgs& args, int mode, int a_dtype, 
                             : mode == MODE_GATED_FWD && !p.aux && !p.enc ? choose_scaled_tile(p.m, 2 * p.n, p.k) : SCALED_TILE_FAST;
     if (mode == MODE_PLAIN ? tile != SCALED_TILE_FAST : tile == SCALED_TILE_L)
         return (MX ? launch_mx_pingpong : launch_tensor_pingpong)(p, tile, mode != MODE_PLAIN, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
-    // fewer than 512 tiles of 128 x 128: halve the tile in n, or from 129 tiles up and over a long k keep the tile and
-    // split its k range inside the block; the narrow tiles split a long k range as well (the grouped recipe's rule)
-    const int64_t tiles = (int64_t)grid.x * grid.y;
-    const bool few = mode == MODE_PLAIN && tiles < 512;
-    const bool long_k = p.k >= VIOLA_SCALED_SPLIT_MIN_K;
-    const bool split = few && tiles > 128 && long_k;
-    const bool narrow = few && !split && p.n > 64;
+    // fewer than 128 tiles of 128 x 128 (from 128 up choose_scaled_tile finds an alternating-phase tile): halve the tile in n to
+    // keep more CUs busy, and over a long k split its k range inside the block (the grouped recipe's rule)
+    const bool narrow = mode == MODE_PLAIN && (int64_t)grid.x * grid.y < 128 && p.n > 64;
+    const bool split = narrow && p.k >= SCALED_SPLIT_MIN_K;
     if (narrow) grid.x = (unsigned)((p.n + 63) / 64);
     if ((int64_t)grid.x * grid.y < (1 << 30)) {
         p.tiles_n = (int)grid.x;
@@ -51,8 +48,7 @@ static int launch_scaled_gemm_fast(const GemmArgs& args, int mode, int a_dtype, 
         grid = dim3((grid.x * grid.y + 7) / 8 * 8, 1, 1);
     }
 #define VIOLA_SCALED(TO)                                                                                                        \
-    if (split) launch_scaled_formats<MODE_PLAIN, TO, 2, TENSOR, MX, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream);        \
-    else if (narrow && long_k) launch_scaled_formats<MODE_PLAIN, TO, 1, TENSOR, MX, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream); \
+    if (split) launch_scaled_formats<MODE_PLAIN, TO, 1, TENSOR, MX, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream);        \
     else if (narrow) launch_scaled_formats<MODE_PLAIN, TO, 1, TENSOR, MX>(p, a_dtype, b_dtype, bias_dtype, grid, stream);        \
     else if (mode == MODE_PLAIN) launch_scaled_formats<MODE_PLAIN, TO, 2, TENSOR, MX>(p, a_dtype, b_dtype, bias_dtype, grid, stream); \
     else if (mode == MODE_GATED_FWD) launch_scaled_formats<MODE_GATED_FWD, TO, 2, TENSOR, MX>(p, a_dtype, b_dtype, bias_dtype, grid, stream); \
