@@ -93,3 +93,44 @@ def test_state_that_is_not_where_the_kernels_read_is_refused(shape, key, how):
     assert all(torch.equal(a, b) for a, b in zip(before, params))
     state[key] = held
     opt.step()
+
+
+@pytest.mark.parametrize("odd", ["gradient off 16 bytes", "gradient of another type", "weight off 16 bytes", "strided gradient"])
+def test_buckets_with_a_member_that_does_not_fit_the_table_kernels(odd):
+    """Whole tiles of 256, so a bucket takes one launch over pointer tables; with one odd member each goes alone. Either way two
+    steps give what the per-tensor operators give, bit for bit."""
+    import viola_amd
+    from viola_amd.optim import _kernels as k
+    from viola_amd.optim._orthogonalize import METHODS
+    torch.manual_seed(8)
+    shape, count = (48, 64), 48 * 64
+
+    def shifted(t):
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+    weights = [torch.randn(*shape, device="cuda") * .05 for _ in range(3)]
+    if odd == "weight off 16 bytes":
+        weights[1] = shifted(weights[1])
+        assert weights[1].data_ptr() % 16
+    params = [torch.nn.Parameter(w) for w in weights]
+    opt = viola_amd.optim.FP8Muon(params, lr=2e-3, weight_decay=.01, rounding="stochastic", rounding_seed=5)
+    twins = [w.detach().clone() for w in weights]
+    state = [(torch.zeros(count, device="cuda", dtype=torch.uint8), torch.ones(count // 256, device="cuda")) for _ in params]
+    for step in range(2):
+        grads = [torch.randn(*shape, device="cuda") * 1e-2 for _ in params]
+        if odd == "gradient off 16 bytes":
+            grads[1] = shifted(grads[1])
+        elif odd == "gradient of another type":
+            grads[1] = grads[1].bfloat16()
+            params[1].grad_dtype = torch.bfloat16
+        elif odd == "strided gradient":
+            grads[1] = grads[1].t().contiguous().t()
+        for p, g in zip(params, grads):
+            p.grad = g
+        opt.step()
+        for i, (w, g, (q, s)) in enumerate(zip(twins, grads, state)):
+            out = torch.empty(count, device="cuda", dtype=torch.bfloat16)
+            k.momentum_update(g, q, s, q, s, out, beta=.95, rounding="stochastic", rounding_step=step, rounding_key=(5 + i * 0x9E3779B97F4A7C15) & ((1 << 63) - 1))
+            k.weight_update(w, METHODS["standard"](out.view(shape), steps=5), 2e-3, .01, update_scale=.2 * 64 ** .5)
+    for p, w, (q, s) in zip(params, twins, state):
+        assert torch.equal(opt.state[p]["momentum_q"], q) and torch.equal(opt.state[p]["momentum_scale"], s) and torch.equal(p, w)

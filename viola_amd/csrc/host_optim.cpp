@@ -90,6 +90,114 @@ Tensor newton_schulz(const Tensor& matrix_, int64_t steps, bool gram) {
     return result;
 }
 
+// ---------------------------------------------------------------------------------------------------- pointer tables
+bool aligned(const void* p, int64_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; }
+
+// Device-side pointer tables, kept while their rows stay the same. Keyed by the stream that fills and reads them.
+class Tables {
+public:
+    const int64_t* get(int kind, const std::vector<int64_t>& shape, int64_t count, int64_t ordinal, std::vector<int64_t>&& rows, const at::Device& device,
+                       viola_stream_t stream) {
+        Table& t = tables_[std::make_tuple(stream, kind, shape, count, ordinal)];
+        if (t.rows != rows) {
+            t.rows = std::move(rows);
+            t.arena = Arena();                                   // launches in flight may still read the old one: a new place
+            t.at = t.arena.take((int64_t)t.rows.size() * 8);
+            t.arena.make(device);
+            VIOLA_CALL(viola_store_words, t.arena.as<int64_t>(t.at), t.rows.data(), (int64_t)t.rows.size(), stream);
+        }
+        return t.arena.as<int64_t>(t.at);
+    }
+
+private:
+    struct Table {
+        std::vector<int64_t> rows;
+        Arena arena;
+        int64_t at = 0;
+    };
+    std::map<std::tuple<viola_stream_t, int, std::vector<int64_t>, int64_t, int64_t>, Table> tables_;
+};
+enum { MOMENTUM_TABLE = 0, WEIGHT_TABLE = 1, ADAM_TABLE = 2 };
+
+// One launch for a list of tensors of equal size (AdamW: of any size) over a table of their pointers. False, with nothing done:
+// they do not fit the table kernel, and each takes a launch of its own.
+struct MomentumRow {
+    Tensor grad, q, scale;
+    void* out;                                                   // bf16
+    int64_t key;
+};
+bool momentum_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<MomentumRow>& rows, int64_t count, int64_t tile,
+                       float beta, float inv_loss_scale, bool nesterov, int rounding, int64_t step, viola_stream_t stream) {
+    if (rows.empty() || rows.size() > 65535 || tile < 256 || count % tile != 0) return false;
+    const at::ScalarType kind = rows[0].grad.scalar_type();
+    std::vector<int64_t> words;
+    for (const MomentumRow& r : rows) {
+        const void *g = r.grad.const_data_ptr(), *q = r.q.const_data_ptr();
+        if (r.grad.scalar_type() != kind || r.grad.numel() != count || !r.grad.is_contiguous() || !aligned(g, 4 * r.grad.element_size()) || !aligned(q, 4) ||
+            !aligned(r.out, 8))
+            return false;
+        const int64_t s = (int64_t)r.scale.const_data_ptr(), row[8] = {(int64_t)g, (int64_t)q, s, (int64_t)q, s, (int64_t)r.out, r.key, 0};
+        words.insert(words.end(), row, row + 8);
+    }
+    const int64_t* t = tables.get(MOMENTUM_TABLE, shape, (int64_t)rows.size(), ordinal, std::move(words), rows[0].q.device(), stream);
+    VIOLA_CALL(viola_momentum_update_table, t, (int64_t)rows.size(), count / tile, code_of(kind), (int)tile, beta, inv_loss_scale, nesterov, rounding, step, stream);
+    return true;
+}
+
+struct WeightRow {
+    Tensor weight;
+    const void* update;
+};
+bool weights_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<WeightRow>& rows, int64_t count,
+                      at::ScalarType update_type, float lr, float weight_decay, float update_scale, viola_stream_t stream) {
+    if (rows.empty() || rows.size() > 65535 || count % 4 != 0) return false;
+    const int64_t update_bytes = 4 * (int64_t)at::elementSize(update_type);
+    std::vector<int64_t> words;
+    for (const WeightRow& r : rows) {
+        const void* w = r.weight.const_data_ptr();
+        if (r.weight.scalar_type() != at::kFloat || r.weight.numel() != count || !r.weight.is_contiguous() || !aligned(w, 16) || !aligned(r.update, update_bytes))
+            return false;
+        words.push_back((int64_t)w);
+        words.push_back((int64_t)r.update);
+    }
+    const int64_t* t = tables.get(WEIGHT_TABLE, shape, (int64_t)rows.size(), ordinal, std::move(words), rows[0].weight.device(), stream);
+    VIOLA_CALL(viola_weight_update_table, t, (int64_t)rows.size(), count, code_of(update_type), lr, weight_decay, update_scale, stream);
+    return true;
+}
+
+struct AdamRow {
+    Tensor weight, grad, first, second;
+    int64_t key, offset;
+};
+struct AdamSettings {
+    float lr, weight_decay, b1, b2, inv_c1, inv_c2, eps;
+    int rounding;
+    int64_t step;                                                // before this one
+    bool adamw, maximize;
+};
+bool adam_together(Tables& tables, const std::vector<AdamRow>& rows, const AdamSettings& a, viola_stream_t stream) {
+    if (rows.empty() || rows.size() > 65535) return false;
+    const AdamRow& head = rows[0];
+    std::vector<int64_t> words;
+    int64_t most = 0;
+    for (const AdamRow& r : rows) {
+        for (const Tensor* t : {&r.weight, &r.grad, &r.first, &r.second})
+            if (!t->is_contiguous() || t->numel() != r.weight.numel()) return false;
+        if (r.weight.scalar_type() != head.weight.scalar_type() || r.grad.scalar_type() != head.grad.scalar_type() ||
+            r.first.scalar_type() != head.first.scalar_type() || r.second.scalar_type() != head.first.scalar_type())
+            return false;
+        const int64_t row[7] = {(int64_t)r.weight.const_data_ptr(), (int64_t)r.grad.const_data_ptr(), (int64_t)r.first.const_data_ptr(),
+                                (int64_t)r.second.const_data_ptr(), r.weight.numel(), r.key, r.offset};
+        words.insert(words.end(), row, row + 7);
+        most = std::max(most, r.weight.numel());
+    }
+    // one table per list of equal settings, told apart by what the first row points at
+    const int64_t* t = tables.get(ADAM_TABLE, {words[0]}, (int64_t)rows.size(), 0, std::move(words), head.weight.device(), stream);
+    VIOLA_CALL(viola_adam_update_table, t, (int64_t)rows.size(), most, code_of(head.weight.scalar_type()), code_of(head.grad.scalar_type()),
+               code_of(head.first.scalar_type()), a.lr, a.weight_decay, a.b1, a.b2, a.inv_c1, a.inv_c2, a.eps, a.rounding, a.step, a.adamw, a.maximize, stream);
+    return true;
+}
+
 // ---------------------------------------------------------------------------------------------------- FP8Muon.step
 // One parameter group's settings, read once per step.
 struct Group {
@@ -114,7 +222,6 @@ constexpr uint64_t MASK63 = (1ull << 63) - 1;
 int64_t rounding_key(int64_t seed, int64_t index, uint64_t stride) { return (int64_t)(((uint64_t)seed + (uint64_t)index * stride) & MASK63); }
 int64_t momentum_key(const Item& it) { return rounding_key(it.group->seed, it.index, 0x9E3779B97F4A7C15ull); }
 int64_t master_key(const Item& it) { return rounding_key(it.group->master_seed, it.index, 0x517CC1B727220A95ull); }
-bool aligned(const Tensor& t, int64_t bytes) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % bytes == 0; }
 int rounding_code(const py::handle& h) { return h.cast<std::string>() == "stochastic" ? VIOLA_STOCHASTIC : VIOLA_NEAREST; }
 
 Group read_group(const py::dict& d) {
@@ -213,28 +320,8 @@ public:
     }
 
 private:
-
-    // Device-side pointer tables, kept while their rows stay the same. Keyed by the stream that fills and reads them.
-    struct Table {
-        std::vector<int64_t> rows;
-        Arena arena;
-        int64_t at = 0;
-    };
-    std::map<std::tuple<viola_stream_t, int, std::vector<int64_t>, int64_t, int64_t>, Table> tables_;
+    Tables tables_;
     std::map<int, std::vector<c10::Stream>> lanes_;
-
-    const int64_t* table(int kind, const std::vector<int64_t>& shape, int64_t count, int64_t ordinal, std::vector<int64_t>&& rows, const at::Device& device,
-                         viola_stream_t stream) {
-        Table& t = tables_[std::make_tuple(stream, kind, shape, count, ordinal)];
-        if (t.rows != rows) {
-            t.rows = std::move(rows);
-            t.arena = Arena();                                   // launches in flight may still read the old one: a new place
-            t.at = t.arena.take((int64_t)t.rows.size() * 8);
-            t.arena.make(device);
-            VIOLA_CALL(viola_store_words, t.arena.as<int64_t>(t.at), t.rows.data(), (int64_t)t.rows.size(), stream);
-        }
-        return t.arena.as<int64_t>(t.at);
-    }
 
     // The state is the caller's: it may have been loaded, moved to the host or replaced, and the kernels read it by raw pointer.
     static void check_state(const Item& it, const Tensor& state, int64_t elements, int64_t bytes_each) {
@@ -336,26 +423,16 @@ private:
         for (Item& it : bucket) grads.push_back(it.grad.contiguous());
 
         // ---- momentum: one launch for the bucket when its members share the recipe and fit the table kernel, else one each
-        const at::ScalarType kind = grads[0].scalar_type();
-        bool together = g.granularity == 0 && g.tile >= 256 && count % g.tile == 0 && size <= 65535 && (2 * count) % 8 == 0;
+        bool together = g.granularity == 0;
+        std::vector<MomentumRow> momentum_rows;
         for (size_t i = 0; together && i < bucket.size(); ++i) {
             const Item& it = bucket[i];
             const Group& h = *it.group;
             together = it.step == head.step && h.granularity == g.granularity && h.tile == g.tile && h.momentum == g.momentum && h.nesterov == g.nesterov &&
-                       h.rounding == g.rounding && grads[i].scalar_type() == kind && grads[i].numel() == count &&
-                       aligned(grads[i], 4 * grads[i].element_size()) && aligned(it.q, 4);
+                       h.rounding == g.rounding;
+            momentum_rows.push_back({grads[i], it.q, it.scale, out + 2 * count * i, momentum_key(it)});
         }
-        if (together) {
-            std::vector<int64_t> words;
-            for (size_t i = 0; i < bucket.size(); ++i) {
-                const int64_t q = (int64_t)bucket[i].q.const_data_ptr(), s = (int64_t)bucket[i].scale.const_data_ptr();
-                const int64_t row[8] = {(int64_t)grads[i].const_data_ptr(), q, s, q, s, (int64_t)(out + 2 * count * i), momentum_key(bucket[i]), 0};
-                words.insert(words.end(), row, row + 8);
-            }
-            const int64_t* t = table(0, shape, size, ordinal, std::move(words), device, stream);
-            VIOLA_CALL(viola_momentum_update_table, t, size, count / g.tile, code_of(kind), (int)g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step,
-                       stream);
-        } else {
+        if (!together || !momentum_together(tables_, shape, ordinal, momentum_rows, count, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step, stream)) {
             for (size_t i = 0; i < bucket.size(); ++i) {
                 const Item& it = bucket[i];
                 const Group& h = *it.group;
@@ -373,22 +450,16 @@ private:
         const int update_code = code_of(updates.scalar_type());
 
         // ---- weights
-        together = count % 4 == 0 && size <= 65535;
-        for (const Item& it : bucket) {
-            const Group& h = *it.group;
-            together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms && it.param.scalar_type() == at::kFloat &&
-                       it.param.is_contiguous() && aligned(it.param, 16);
+        together = true;
+        std::vector<WeightRow> weight_rows;
+        for (size_t i = 0; i < bucket.size(); ++i) {
+            const Group& h = *bucket[i].group;
+            together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms;
+            weight_rows.push_back({bucket[i].param, from + 2 * count * i});
         }
-        if (together) {
-            std::vector<int64_t> words;
-            for (size_t i = 0; i < bucket.size(); ++i) {
-                words.push_back((int64_t)bucket[i].param.const_data_ptr());
-                words.push_back((int64_t)(from + 2 * count * i));
-            }
-            const int64_t* t = table(1, shape, size, ordinal, std::move(words), device, stream);
-            VIOLA_CALL(viola_weight_update_table, t, size, count, update_code, (float)g.lr, (float)g.weight_decay, (float)update_scale(g, rows, cols), stream);
+        if (together && weights_together(tables_, shape, ordinal, weight_rows, count, updates.scalar_type(), (float)g.lr, (float)g.weight_decay,
+                                         (float)update_scale(g, rows, cols), stream))
             return;
-        }
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Item& it = bucket[i];
             const Group& h = *it.group;
@@ -406,28 +477,16 @@ private:
         const viola_stream_t stream = stream_of(head.param);
         const double step = (double)(head.step + 1);
         const float inv_c1 = (float)(1. / (1. - std::pow(g.b1, step))), inv_c2 = (float)(1. / (1. - std::pow(g.b2, step)));
-        const int weight_code = code_of(head.param.scalar_type()), grad_code = code_of(head.grad.scalar_type()), state_code = code_of(head.first.scalar_type());
-        std::vector<int64_t> words;
-        int64_t most = 0;
+        const int weight_code = code_of(head.param.scalar_type()), grad_code = code_of(head.grad.scalar_type());
+        std::vector<AdamRow> rows;
         std::vector<Tensor> grads;
-        bool together = bucket.size() > 1 && bucket.size() <= 65535;
         for (const Item& it : bucket) {
             TORCH_CHECK(it.param.is_contiguous() && it.first.scalar_type() == it.second.scalar_type() && it.grad.numel() == it.param.numel());
-            together = together && it.grad.is_contiguous() && it.first.is_contiguous() && it.second.is_contiguous() &&
-                       it.first.scalar_type() == head.first.scalar_type();
+            rows.push_back({it.param, it.grad, it.first, it.second, master_key(it), 0});
             grads.push_back(it.grad.contiguous());
-            const int64_t row[7] = {(int64_t)it.param.const_data_ptr(), (int64_t)grads.back().const_data_ptr(), (int64_t)it.first.const_data_ptr(),
-                                    (int64_t)it.second.const_data_ptr(), it.param.numel(), master_key(it), 0};
-            words.insert(words.end(), row, row + 7);
-            most = std::max(most, it.param.numel());
         }
-        if (together) {
-            // one table per bucket of equal settings, told apart by what the first row points at
-            const int64_t* t = table(2, {words[0]}, (int64_t)bucket.size(), 0, std::move(words), head.param.device(), stream);
-            VIOLA_CALL(viola_adam_update_table, t, (int64_t)bucket.size(), most, weight_code, grad_code, state_code, (float)g.lr, (float)g.weight_decay, (float)g.b1,
-                       (float)g.b2, inv_c1, inv_c2, (float)g.eps, g.master_rounding, head.step, 1, 0, stream);
-            return;
-        }
+        const AdamSettings settings{(float)g.lr, (float)g.weight_decay, (float)g.b1, (float)g.b2, inv_c1, inv_c2, (float)g.eps, g.master_rounding, head.step, true, false};
+        if (bucket.size() > 1 && adam_together(tables_, rows, settings, stream)) return;
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Item& it = bucket[i];
             if (it.param.numel() == 0) continue;
@@ -464,6 +523,43 @@ namespace viola_host {
 void register_optimizer(py::module_& m) {
     m.def("newton_schulz", torch::wrap_pybind_function_no_gil(newton_schulz), py::arg("matrix"), py::arg("steps"), py::arg("gram"));
     m.def("roundtrip", torch::wrap_pybind_function(roundtrip));
+    // The table launches of FP8Muon's step as operators of their own (optim/_kernels.py); the lists are one entry per tensor.
+    py::class_<Tables, std::shared_ptr<Tables>>(m, "Tables").def(py::init<>());
+    m.def("momentum_update_many", torch::wrap_pybind_function([](Tables& tables, const std::vector<Tensor>& grads, const std::vector<Tensor>& qs,
+                                                                 const std::vector<Tensor>& scales, const std::vector<Tensor>& outs, const std::vector<int64_t>& keys,
+                                                                 int64_t tile, double beta, double inv_loss_scale, bool nesterov, int rounding, int64_t step) {
+        std::vector<MomentumRow> rows;
+        for (size_t i = 0; i < grads.size(); ++i) {
+            TORCH_CHECK(grads[i].is_cuda() && qs[i].is_cuda() && scales[i].is_cuda() && outs[i].is_cuda(), "viola_amd kernels run on the GPU only");
+            if (outs[i].scalar_type() != at::kBFloat16 || outs[i].numel() < grads[i].numel()) return false;
+            rows.push_back({grads[i], qs[i], scales[i], outs[i].mutable_data_ptr(), keys[i]});
+        }
+        return momentum_together(tables, {}, 0, rows, grads[0].numel(), tile, (float)beta, (float)inv_loss_scale, nesterov, rounding, step, stream_of(grads[0]));
+    }));
+    m.def("weight_update_many", torch::wrap_pybind_function([](Tables& tables, const std::vector<Tensor>& weights, const std::vector<Tensor>& updates, double lr,
+                                                               double weight_decay, double update_scale) {
+        std::vector<WeightRow> rows;
+        for (size_t i = 0; i < weights.size(); ++i) {
+            TORCH_CHECK(weights[i].is_cuda() && updates[i].is_cuda(), "viola_amd kernels run on the GPU only");
+            if (updates[i].scalar_type() != updates[0].scalar_type() || updates[i].numel() != weights[i].numel() || !updates[i].is_contiguous()) return false;
+            rows.push_back({weights[i], updates[i].const_data_ptr()});
+        }
+        return weights_together(tables, {}, 0, rows, weights[0].numel(), updates[0].scalar_type(), (float)lr, (float)weight_decay, (float)update_scale,
+                                stream_of(weights[0]));
+    }));
+    m.def("adam_update_many", torch::wrap_pybind_function([](Tables& tables, const std::vector<Tensor>& weights, const std::vector<Tensor>& grads,
+                                                             const std::vector<Tensor>& firsts, const std::vector<Tensor>& seconds, const std::vector<int64_t>& keys,
+                                                             const std::vector<int64_t>& offsets, const std::vector<double>& hyper, int rounding, int64_t step,
+                                                             bool adamw, bool maximize) {
+        std::vector<AdamRow> rows;
+        for (size_t i = 0; i < weights.size(); ++i) {
+            TORCH_CHECK(weights[i].is_cuda() && grads[i].is_cuda() && firsts[i].is_cuda() && seconds[i].is_cuda(), "viola_amd kernels run on the GPU only");
+            rows.push_back({weights[i], grads[i], firsts[i], seconds[i], keys[i], offsets[i]});
+        }
+        const AdamSettings settings{(float)hyper[0], (float)hyper[1], (float)hyper[2], (float)hyper[3], (float)hyper[4], (float)hyper[5], (float)hyper[6], rounding, step,
+                                    adamw, maximize};
+        return adam_together(tables, rows, settings, stream_of(weights[0]));
+    }));
     py::class_<MuonHost>(m, "MuonHost").def(py::init<>())
         .def("step", torch::wrap_pybind_function([](MuonHost& host, const py::list& work, const py::list& groups) { host.step(work, groups); }))
         .def_readwrite("lanes", &MuonHost::lanes).def_readwrite("batch_elements", &MuonHost::batch_elements).def("streams", &MuonHost::streams);

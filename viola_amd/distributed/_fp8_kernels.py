@@ -37,8 +37,15 @@ def unpack(packet, out, tile_size, fp8_dtype, *, reduce=False):
 
 
 def _table(rows, device, cache):
-    from ..optim._kernels import _device_table
-    return _device_table(rows, device, cache)
+    """int64 rows as a device tensor; `cache` (a dict) keeps it between calls and it is rebuilt when any entry changes."""
+    held = cache.get("rows") if cache is not None else None
+    if held == rows:
+        return cache["table"]
+    staging = torch.tensor(rows, dtype=torch.int64).pin_memory()
+    table = staging.to(device, non_blocking=True)
+    if cache is not None:
+        cache.update(rows=rows, table=table, staging=staging)
+    return table
 
 
 def pack_many(sources, packets, tile_size, fp8_dtype, *, cache=None):
