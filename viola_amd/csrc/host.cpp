@@ -976,6 +976,31 @@ variable_list ExpertsBackward::apply(variable_list&& grads) {
     return result;
 }
 
+// quantize_segments as an operator of its own: (qt, st), with `rowwise` also the row-wise codes and scales (views of padded rows)
+std::vector<Tensor> segments(const Tensor& x, const Recipe& r, const Tensor& offsets, const Tensor& padded_offsets, int64_t count, int64_t padded, bool rowwise) {
+    TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous());
+    const int64_t rows = x.size(0), cols = x.size(1);
+    const at::Device device = x.device();
+    for (const Tensor* t : {&offsets, &padded_offsets})
+        TORCH_CHECK(holds(*t, device, at::kLong, {count + 1}), "offsets: contiguous int64 [groups + 1] on x's device");
+    Groups g;
+    g.count = count; g.rows = rows; g.padded = padded;
+    g.offsets = offsets.const_data_ptr<int64_t>(); g.padded_offsets = padded_offsets.const_data_ptr<int64_t>();
+    const auto options = at::TensorOptions().device(device);
+    const Tensor qt = at::empty({cols, padded}, options.dtype(r.codes())), st = at::empty({cols, padded / 32}, options.dtype(at::kFloat));
+    Arena temp;
+    GroupSpace space;
+    if (rowwise) space.reserve(r, &temp, nullptr, rows, cols, r.pitch(cols));
+    temp.make(device);
+    Codes out;
+    quantize_segments(r, x, r.fwd, r.fwd_limit, g, rowwise ? &temp : nullptr, space, qt.mutable_data_ptr(), st.mutable_data_ptr<float>(), &out, stream_of(x));
+    if (!rowwise) return {qt, st};
+    const int64_t scales = ceil_div(space.pitch, 32);
+    const Tensor q = temp.tensor().narrow(0, space.q, rows * space.pitch).view({rows, space.pitch}).view(r.codes());
+    const Tensor s = temp.tensor().narrow(0, space.s, rows * scales * 4).view({rows, scales * 4}).view(at::kFloat);
+    return {qt, st, q.narrow(1, 0, cols), s.narrow(1, 0, ceil_div(cols, 32))};
+}
+
 // ---------------------------------------------------------------------------------------------------- Python
 // (recipe, weight, bias, scale, transpose, transpose scale[, three histories, three counters])
 Layer layer_from(const py::tuple& t) {
@@ -1012,6 +1037,15 @@ PYBIND11_MODULE(_host, m) {
         recording.store(!list.is_none());
     });
     register_optimizer(m);
+    m.def("segment_offsets", torch::wrap_pybind_function([](const std::vector<int64_t>& counts, const at::Device& device) {
+        Groups g;
+        make_groups(g, counts, device, c10::hip::getCurrentHIPStream(device.index()).stream());
+        return g.arena.tensor();
+    }));
+    m.def("quantize_segments", torch::wrap_pybind_function([](const Tensor& x, const std::shared_ptr<Recipe>& recipe, const Tensor& offsets,
+                                                              const Tensor& padded_offsets, int64_t count, int64_t padded, bool rowwise) {
+        return segments(x, *recipe, offsets, padded_offsets, count, padded, rowwise);
+    }));
     // Each binding is wrapped so that what torch throws (out of memory, an error raised inside a hook) reaches Python as its own type.
     // None: a call for the general path
     m.def("linear", torch::wrap_pybind_function([](const Tensor& x, const py::tuple& layer) -> std::optional<Tensor> {

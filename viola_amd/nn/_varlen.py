@@ -19,7 +19,7 @@ from . import _grouped_kernels as kernels
 from ..precision import settings
 
 _FORMATS = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
-GX, GW = (1, 32), (32, 32)
+GW = (32, 32)
 
 
 @functools.lru_cache(maxsize=None)
@@ -32,36 +32,20 @@ def _recipe(forward_dtype, backward_dtype):
 
 
 def _offsets(counts, device):
+    """Row offsets of the groups and offsets on the padded token axis (whole tiles of 32 per group, 128 in all), on the host and
+    as the native host path puts them on the device."""
     counts = [int(c) for c in (counts.tolist() if isinstance(counts, torch.Tensor) else counts)]
-    assert all(c >= 0 for c in counts)
-    offsets, padded = [0], [0]
-    for c in counts:
-        offsets.append(offsets[-1] + c)
-        padded.append(padded[-1] + (c + 31) // 32 * 32)
-    # The padded token axis is the row length of the transposed codes: rounded up to 128 (empty slots at the end of the
-    # last group, zero codes) so that every row starts on a cache line and the quantizer's 64-byte pieces never straddle one.
-    padded[-1] = (padded[-1] + 127) // 128 * 128
-    both = torch.tensor([offsets, padded], dtype=torch.int64).to(device, non_blocking=True)
-    return offsets, padded, both[0], both[1]
+    table = _lib.host().segment_offsets(counts, torch.device(device)).view(torch.int64)[:2 * (len(counts) + 1)].view(2, -1)
+    offsets, padded = table.tolist()
+    return offsets, padded, table[0], table[1]
 
 
 def quantize_transposed_segmented(x, dtype, offsets_dev, padded_dev, groups, t_total, *, rowwise=False):
     """Per-group quantized transpose of x [M, C]: codes [C, t_total], scales [C, t_total/32]. With rowwise, also the
-    plain (1, 32) row-wise codes and scales of x from the same read: returns (qt, st, q, s)."""
-    rows, cols = x.shape
-    qt = torch.empty((cols, t_total), device=x.device, dtype=dtype)
-    st = torch.empty((cols, t_total // 32), device=x.device, dtype=torch.float32)
-    fused = rowwise and x.element_size() == 2 and cols % 8 == 0 and x.data_ptr() % 16 == 0
-    q = torch.empty((rows, cols), device=x.device, dtype=dtype) if fused else None
-    s = torch.empty((rows, -(-cols // 32)), device=x.device, dtype=torch.float32) if fused else None
-    _lib.call("viola_varlen_quantize_transposed", _lib.ptr(x), _lib.code(x.dtype), rows, cols, _lib.ptr(offsets_dev),
-              _lib.ptr(padded_dev), groups, t_total, _lib.ptr(qt), _lib.ptr(st), _lib.code(dtype),
-              float(torch.finfo(dtype).max), _lib.ptr(q), _lib.ptr(s))
-    if not rowwise:
-        return qt, st
-    if not fused:
-        q, s = kernels.quantize(x, dtype, GX)
-    return qt, st, q, s
+    plain (1, 32) row-wise codes and scales of x, from the same read where the kernel takes the shape: returns (qt, st, q, s).
+    The quantizer of the native host path's forward and backward, as an operator."""
+    name = {fp8: key for key, fp8 in _FORMATS.items()}[dtype]
+    return tuple(_lib.host().quantize_segments(x, _recipe(name, name), offsets_dev, padded_dev, int(groups), int(t_total), bool(rowwise)))
 
 
 def grouped_linear(x, weight, weight_scale, counts, *, forward_dtype="e4m3", backward_dtype="e4m3", grad_dtype=None):
