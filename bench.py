@@ -308,10 +308,10 @@ def main():
                     avg_launch_ms=gemm["avg_ms"], traffic=GEMM_TRAFFIC_BYTES,
                     traffic_source="stored calibration (two rocprofv3 --pmc runs, profiles/linear_step_8192x1024x4096_hbm_traffic.txt), not read in this run")
     quant = {}
-    if "viola_group_quantize_dual" in breakdown:
+    if "viola_group_quantize_dual_pitched" in breakdown:
         # X [M, K] and dY [M, N] each once per step: 4.25 B per element (bf16 in, two FP8 layouts + scales out)
         per_step = 4.25 * (M * K + M * N) / 2
-        q = breakdown["viola_group_quantize_dual"]
+        q = breakdown["viola_group_quantize_dual_pitched"]
         quant = dict(kernel="quantize_dual16_tile64 (row-wise + transposed + column partials, one read)", avg_ms=q["avg_ms"],
                      gbs=per_step / (q["avg_ms"] * 1e-3) / 1e9, frac_hbm=per_step / (q["avg_ms"] * 1e-3) / 1e9 / PEAK["hbm_gbs"])
 
