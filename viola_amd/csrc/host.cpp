@@ -696,8 +696,10 @@ Tensor linear(const Tensor& x, Layer& l) {
 }
 
 // ---------------------------------------------------------------------------------------------------- MLP
-// One node for the whole gated MLP: dz, the gradient of [g | u], goes from the down projection's data-gradient product
-// (activation derivative in its epilogue) straight into the stacked gate/up projection's backward.
+// One node for the whole gated MLP. Grouped and block-scaled recipes: the down projection's data-gradient product writes dh, and
+// the quantizer of the stacked gate/up projection's gradient makes dz, the gradient of [g | u], as it reads dh and [g | u]; dz is
+// never stored. Per-tensor recipes, whose scale needs dz before it is quantized, and shapes that quantizer does not take: the
+// product itself hands out dz (viola_*_gated_gemm: in its epilogue, or on large tiles in one pass over dh).
 struct MlpBackward : public Node {
     Layer up, down;
     Kept up_kept, down_kept;

@@ -478,8 +478,8 @@ __device__ __forceinline__ uint32_t narrow_pair(float a, float b) {
 }
 
 // Forward: one tile of h. What bounds it: bytes (6 per element of h: 4 read, 2 written) and, close behind, the arithmetic of the
-// activation and of both encoders. 4096 x 4608 gelu: 55 -> 30 us against a
-// persistent kernel on 128 x 64 tiles; 16384 x 11008 silu: 288 us, 3.8 TB/s.
+// activation and of both encoders. 4096 x 4608 gelu: 55 -> 28 us against a
+// persistent kernel on 128 x 64 tiles; 16384 x 11008 silu: 277 us, 3.9 TB/s.
 template <typename TIn, typename TOut, int ACT>
 __global__ __launch_bounds__(256, 8) void gated_quantize_dual16(const TIn* __restrict__ z, const Dual16 d, int xcd_walk, int aligned) {
     __shared__ __attribute__((aligned(16))) uint16_t park[64 * DUAL16_LDV];
@@ -509,8 +509,8 @@ __global__ __launch_bounds__(256, 8) void gated_quantize_dual16(const TIn* __res
 
 // Backward: dz = [dh u act'(g) | dh act(g)] [rows, 2 h], h a multiple of 64; the block of a tile of dh makes both tiles of dz, so z
 // and dh are read once (10 bytes per element of h, against 8 for making dz in the product's epilogue and 8 for reading it back
-// into the quantizer). 4096 x 4608 gelu behind a k of 1152: 106 + 30 -> 39 + 50 us; 16384 x 11008 silu: 541 us, 3.3 TB/s.
-// Four blocks per CU: with six the registers do not hold all of a lane's loads in flight (4096 x 4608 46 -> 41 us).
+// into the quantizer). 4096 x 4608 gelu behind a k of 1152: 106 + 30 -> 39 + 51 us; 16384 x 11008 silu: 501 us, 3.6 TB/s.
+// Four blocks per CU: with six the registers do not hold all of a lane's loads in flight (4096 x 4608 alone, back to back: 46 -> 41 us).
 template <typename TIn, typename TOut, int ACT>
 __global__ __launch_bounds__(256, 4) void gated_backward_quantize_dual16(const TIn* __restrict__ z, const TIn* __restrict__ dh, int64_t h, const Dual16 d,
                                                                          int xcd_walk, int aligned) {
