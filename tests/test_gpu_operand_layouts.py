@@ -169,3 +169,21 @@ def test_parametrized_and_pruned_parameters(scaling, native):
     want = _step(plain, x, dy)
     assert torch.equal(y, want[0]) and torch.equal(dx, want[1])
     assert rel_l2(module.weight_orig.grad, want[2] * module.weight_mask) < BOUND
+
+
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+@pytest.mark.parametrize("scaling", ["grouped", "current"])
+def test_a_strided_bias_keeps_its_gradient(scaling, kind):
+    import viola_amd
+    x, dy = _data(64, 128, 192 if kind == "linear" else 128)
+    results = []
+    for strided in (False, True):
+        torch.manual_seed(1)
+        cls = viola_amd.nn.Linear if kind == "linear" else viola_amd.nn.MLP
+        module = cls(128, 192, device="cuda", dtype=torch.bfloat16, scaling=scaling)
+        for name, p in module.named_parameters():
+            if strided and name.endswith("bias"):
+                p.data = torch.stack([p.data, p.data + 1], 1)[:, 0]
+        results.append(_step(module, x, dy))
+    for got, want in zip(*results):
+        assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(got, want)

@@ -390,6 +390,7 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         kept.weight_grad = gradient_type(l.weight);
         if (l.bias.defined()) kept.bias_grad = gradient_type(l.bias);
     }
+    const Tensor bias = l.bias.defined() ? l.bias.contiguous() : Tensor();      // the layer's own stays what the graph is connected to
     const auto options = at::TensorOptions().dtype(dtype).device(device);
     const int64_t h = r.out / 2;
     Forward f;
@@ -411,11 +412,11 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         if (!plain || need_backward || coded_input || !r.fp8_weight || x2.element_size() != 2 || !small_product(rows, r.out)) return false;
         if ((rows > 16 && rows * r.out > 256 * 16 * 32 ? 2 : 1) * r.in > QUANTIZED_IN_PRODUCT) return false;
         if (!r.grouped && (rows * r.in > WHOLE_TENSOR || (l.counter[INPUT]->delayed && l.counter[INPUT]->value))) return false;
-        const void* bias_p = ptr(l.bias);
+        const void* bias_p = ptr(bias);
         float* history = r.grouped ? nullptr : static_cast<float*>(l.history[INPUT].mutable_data_ptr());
         const int64_t slot = r.grouped ? 0 : l.counter[INPUT]->value % l.history[INPUT].numel();
         const int status = VIOLA_TRY(viola_skinny_linear, ptr(x2), code_of(x2.scalar_type()), nullptr, rows, r.in, ptr(l.weight), r.fwd, ptr(l.scale), r.grouped,
-                                     r.out, r.fwd_limit, r.scale_format(), history, slot, nullptr, bias_p, bias_p ? code_of(l.bias.scalar_type()) : 0,
+                                     r.out, r.fwd_limit, r.scale_format(), history, slot, nullptr, bias_p, bias_p ? code_of(bias.scalar_type()) : 0,
                                      output.mutable_data_ptr(), code_of(dtype), stream);
         if (status != 0 && status != VIOLA_EUNSUPPORTED) check("viola_skinny_linear", status);
         if (status == 0 && !r.grouped) ++l.counter[INPUT]->value;
@@ -465,7 +466,7 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
             VIOLA_CALL(viola_codes_transpose_pitched, w_unpadded.q, kept.weight_t.mutable_data_ptr(), 1, r.out, r.in, r.out, grid ? w_unpadded.s : nullptr,
                        grid ? kept.weight_t_scale.mutable_data_ptr() : nullptr, 32, 32, r.scale_format(), nullptr, 0, 0, nullptr, 0, stream);
         }
-        if (plain) product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, l.bias, output.mutable_data_ptr(), dtype, device, stream);
+        if (plain) product(r, a, r.fwd, w, r.fwd, rows, r.out, 32, bias, output.mutable_data_ptr(), dtype, device, stream);
     }
     if (gated < 0) return f;
     if (plain) {
@@ -495,9 +496,9 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         keep.make(device);
         void* qt_p = transposed ? keep.at(qt) : nullptr;
         uint8_t* st_p = transposed ? keep.as<uint8_t>(st) : nullptr;
-        const void* bias_p = ptr(l.bias);
+        const void* bias_p = ptr(bias);
         const int status = VIOLA_TRY(viola_mx_gated_gemm_encode, a.q, r.fwd, w.q, r.fwd, static_cast<const uint8_t*>(a.s), static_cast<const uint8_t*>(w.s), rows, h,
-                                     a.pitch, 1, 32, bias_p, bias_p ? code_of(l.bias.scalar_type()) : 0, const_cast<void*>(ptr(f.aux)), code_of(dtype),
+                                     a.pitch, 1, 32, bias_p, bias_p ? code_of(bias.scalar_type()) : 0, const_cast<void*>(ptr(f.aux)), code_of(dtype),
                                      hidden_out->temp.at(q), hidden_out->temp.as<uint8_t>(s), qt_p, st_p, r.fwd, r.fwd_limit, gated, stream);
         if (status != 0 && status != VIOLA_EUNSUPPORTED) check("viola_mx_gated_gemm_encode", status);
         if (status == 0) {
@@ -509,7 +510,7 @@ Forward project(const Layer& l, const Tensor& x2, at::ScalarType dtype, bool nee
         hidden_kept->arena = Arena();
     }
     f.y = at::empty({rows, h}, options);
-    gated_product(r, a, r.fwd, w, r.fwd, rows, h, l.bias, f.aux, f.y, gated, false, stream);
+    gated_product(r, a, r.fwd, w, r.fwd, rows, h, bias, f.aux, f.y, gated, false, stream);
     return f;
 }
 
@@ -681,7 +682,6 @@ Tensor linear(const Tensor& x, Layer& l) {
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const Tensor x2 = as_matrix(x, l.recipe->in);
-        if (l.bias.defined() && !l.bias.is_contiguous()) l.bias = l.bias.contiguous();
         y = project(l, x2, x.scalar_type(), need, ww, kept, -1, false, nullptr, nullptr, nullptr).y;
         if (x.dim() != 2) y = y.view(output_shape(x, l.recipe->out));
     }
@@ -752,8 +752,6 @@ Tensor mlp(const Tensor& x, Layer& up, Layer& down, int activation) {
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const Tensor x2 = as_matrix(x, up.recipe->in);
-        for (Layer* l : {&up, &down})
-            if (l->bias.defined() && !l->bias.is_contiguous()) l->bias = l->bias.contiguous();
         const int64_t rows = x2.size(0);
         CodedHidden hidden;
         hidden.reader = down.recipe.get();
