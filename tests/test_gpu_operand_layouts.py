@@ -187,3 +187,36 @@ def test_a_strided_bias_keeps_its_gradient(scaling, kind):
         results.append(_step(module, x, dy))
     for got, want in zip(*results):
         assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("up,down", [(dict(scaling="grouped"), dict(scaling="current")), (dict(scaling="current"), dict(scaling="grouped")),
+                                     (dict(scaling="mxfp8"), dict(scaling="current")), (dict(scaling="current"), dict(scaling="mxfp8")),
+                                     (dict(scaling="mxfp8"), dict(scaling="grouped")), (dict(scaling="mxfp8"), dict(scaling="mxfp8", forward_dtype="e5m2")),
+                                     (dict(scaling="mxfp8"), dict(scaling="mxfp8", quantization_limit=64.))])
+@pytest.mark.parametrize("rows,train", [(128, True), (128, False), (8, False), (2048, False)])
+def test_mlp_with_a_down_projection_of_another_recipe(up, down, rows, train):
+    """An MLP one of whose projections was replaced, against the same two Linears with the float activation between them."""
+    import viola_amd
+    F = torch.nn.functional
+    torch.manual_seed(rows)
+    mlp = viola_amd.nn.MLP(128, 256, device="cuda", dtype=torch.bfloat16, **up)
+    mlp.down = viola_amd.nn.Linear(256, 128, device="cuda", dtype=torch.bfloat16, **down)
+    x, dy = _data(rows, 128, 128)
+
+    def composed(t):
+        z = mlp.gate_up(t)
+        return mlp.down((F.silu(z[..., :256].float()) * z[..., 256:].float()).to(z.dtype))
+
+    if not train:
+        with torch.no_grad():
+            assert rel_l2(mlp(x), composed(x)) < .025                             # h may round to the neighbouring code
+        return
+    results = []
+    for call in (mlp, composed):
+        t = x.clone().requires_grad_()
+        mlp.zero_grad()
+        y = call(t)
+        y.backward(dy)
+        results.append([y.detach(), t.grad] + [p.grad for p in mlp.parameters()])
+    for got, want in zip(*results):
+        assert rel_l2(got, want) < .04                                            # another e5m2 rounding of dz (2^-3 / sqrt(12) of a few elements)

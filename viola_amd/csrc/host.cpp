@@ -633,6 +633,11 @@ Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const T
     return out;
 }
 
+// The two projections of an MLP hand h over in one form: one of them replaced by a Linear of another recipe is the general path's.
+bool pair(const Recipe& up, const Recipe& down) {
+    return up.out == 2 * down.in && up.grouped == down.grouped && up.native == down.native && up.fwd == down.fwd && up.fwd_limit == down.fwd_limit;
+}
+
 bool wants(const Tensor& t) { return t.defined() && t.requires_grad(); }
 
 // ---------------------------------------------------------------------------------------------------- Linear
@@ -1056,7 +1061,7 @@ PYBIND11_MODULE(_host, m) {
     }));
     m.def("mlp", torch::wrap_pybind_function([](const Tensor& x, const py::tuple& up, const py::tuple& down, int activation) -> std::optional<Tensor> {
         Layer u = layer_from(up), d = layer_from(down);
-        if (transformed() || !plain(x) || !takes(u, x.device()) || !takes(d, x.device()) || u.recipe->out != 2 * d.recipe->in) return std::nullopt;
+        if (transformed() || !plain(x) || !takes(u, x.device()) || !takes(d, x.device()) || !pair(*u.recipe, *d.recipe)) return std::nullopt;
         py::gil_scoped_release release;
         return mlp(x, u, d, activation);
     }));
