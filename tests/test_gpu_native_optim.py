@@ -9,7 +9,7 @@ from viola_amd import _lib
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("steps", [1, 2, 5])
+@pytest.mark.parametrize("steps", [0, 1, 2, 5])
 @pytest.mark.parametrize("method", ["standard", "gram"])
 @pytest.mark.parametrize("shape", [(64, 64), (3, 96, 160), (2, 160, 96), (33, 70)])
 def test_native_chain_equals_the_products_one_by_one(shape, method, steps):

@@ -23,7 +23,8 @@ constexpr float A_COEFFICIENT = 3.4445f;
 
 // orthogonalize [..., rows, cols] in `steps` steps; every product of the chain reads and writes one arena, the last one the result
 Tensor newton_schulz(const Tensor& matrix_, int64_t steps, bool gram) {
-    TORCH_CHECK(matrix_.is_cuda() && matrix_.dim() >= 2 && steps > 0, "viola_amd kernels run on the GPU only");
+    TORCH_CHECK(matrix_.is_cuda(), "viola_amd kernels run on the GPU only");
+    TORCH_CHECK(matrix_.dim() >= 2 && steps >= 0, "Newton-Schulz takes matrices and a number of steps, got ", matrix_.dim(), " dimensions and ", steps, " steps");
     const Tensor matrix = matrix_.contiguous();
     const int64_t rows = matrix.size(-2), cols = matrix.size(-1), m = std::min(rows, cols), n = std::max(rows, cols);
     const int64_t batch = rows * cols ? matrix.numel() / (rows * cols) : 0;
@@ -42,8 +43,9 @@ Tensor newton_schulz(const Tensor& matrix_, int64_t steps, bool gram) {
     for (int64_t& at : x_at) at = arena.take(wide);
     for (int i = 0; i < squares; ++i) s_at[i] = arena.take(square);
     arena.make(matrix.device());
-    void *x = arena.at(x_at[0]), *spare = arena.at(x_at[1]);
+    void *x = steps ? arena.at(x_at[0]) : result.mutable_data_ptr(), *spare = arena.at(x_at[1]);   // no steps: the scaled matrix
     VIOLA_CALL(viola_ns_prepare, matrix.const_data_ptr(), code_of(matrix.scalar_type()), x, dtype, batch, rows, cols, arena.as<float>(sums), stream);
+    if (steps == 0) return result;
     auto gemm = [&](const void* a, const void* b, bool transpose_b, const void* residual, int epilogue, int64_t out_cols, int64_t k, void* out,
                     float add_diag, void* out_diag, bool transpose_out) {
         VIOLA_CALL(viola_ns_gemm, a, b, residual, out, dtype, transpose_b, epilogue, batch, m, out_cols, k, add_diag, out_diag, transpose_out, stream);
