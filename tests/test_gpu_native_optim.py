@@ -134,3 +134,23 @@ def test_buckets_with_a_member_that_does_not_fit_the_table_kernels(odd):
             k.weight_update(w, METHODS["standard"](out.view(shape), steps=5), 2e-3, .01, update_scale=.2 * 64 ** .5)
     for p, w, (q, s) in zip(params, twins, state):
         assert torch.equal(opt.state[p]["momentum_q"], q) and torch.equal(opt.state[p]["momentum_scale"], s) and torch.equal(p, w)
+
+
+def test_operators_read_strided_gradients_in_order():
+    """A 1-D gradient with a stride: flattening it is no copy."""
+    from viola_amd.optim import _kernels as k
+    torch.manual_seed(6)
+    n = 512
+    grad = torch.randn(n, 2, device="cuda")[:, 0]
+    assert not grad.is_contiguous()
+    results = []
+    for g in (grad, grad.contiguous()):
+        w, m, v = torch.ones(n, device="cuda"), torch.zeros(n, device="cuda"), torch.zeros(n, device="cuda")
+        k.adam_update(w, g, m, v, lr=1e-2, weight_decay=.01, betas=(.9, .95), eps=1e-8, step=1)
+        q, s, out = torch.zeros(n, device="cuda", dtype=torch.uint8), torch.ones(n // 256, device="cuda"), torch.empty(n, device="cuda", dtype=torch.bfloat16)
+        k.momentum_update(g, q, s, q, s, out, beta=.95)
+        w2 = torch.ones(n, device="cuda")
+        k.weight_update(w2, g, 1e-2, .01)
+        results.append((w, m, v, q, s, out, w2))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

@@ -43,7 +43,7 @@ def momentum_update(grad, q, scales, next_q, next_scales, out, *, beta, tile_siz
     """m = beta*deq(q) + (1-beta)*grad/loss_scale; (next_q, next_scales) = e4m3 tiles of m;
     out = bf16 update (Nesterov or plain). q/next_q and scales/next_scales may alias."""
     assert grad.is_cuda and out.dtype == torch.bfloat16
-    flat = grad.reshape(-1)
+    flat = grad.reshape(-1).contiguous()
     n = flat.numel()
     geometry = _geometry(n, granularity, tile_size, block_shape, matrix_shape)
     _lib.call("viola_momentum_update", _lib.ptr(flat), _lib.code(flat.dtype), _lib.ptr(q), _lib.ptr(scales),
@@ -60,7 +60,7 @@ def copy_scaled(update, partition, src, dst, count, scale):
 def weight_update(weight, grad, lr, weight_decay, *, update_scale=1.0, rounding="nearest", step=0, key=0, offset=0):
     """weight = weight*(1 - lr*wd) - lr*update_scale*grad in fp32, stored in weight's dtype."""
     assert weight.is_cuda and weight.is_contiguous()
-    flat = grad.reshape(-1)
+    flat = grad.reshape(-1).contiguous()
     _lib.call("viola_weight_update", _lib.ptr(weight), _lib.code(weight.dtype), _lib.ptr(flat), _lib.code(flat.dtype),
               weight.numel(), float(lr), float(weight_decay), float(update_scale), _lib.ROUNDING[rounding],
               int(step), int(key), int(offset))
@@ -70,7 +70,7 @@ def adam_update(weight, grad, first, second, *, lr, weight_decay, betas, eps, st
                 offset=0, adamw=True, maximize=False, bias_correction=True):
     assert weight.is_cuda and weight.is_contiguous() and first.dtype == second.dtype
     b1, b2 = betas
-    flat = grad.reshape(-1)
+    flat = grad.reshape(-1).contiguous()
     _lib.call("viola_adam_update", _lib.ptr(weight), _lib.code(weight.dtype), _lib.ptr(flat), _lib.code(flat.dtype),
               _lib.ptr(first), _lib.ptr(second), _lib.code(first.dtype), weight.numel(), float(lr), float(weight_decay),
               float(b1), float(b2), 1. / (1. - b1 ** step) if bias_correction else 1.,
