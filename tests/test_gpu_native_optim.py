@@ -154,3 +154,33 @@ def test_operators_read_strided_gradients_in_order():
         results.append((w, m, v, q, s, out, w2))
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("refused", ["strided matrix", "strided vector", "FP8 parameter"])
+def test_a_refused_step_changes_nothing(refused):
+    """One parameter that FP8Muon does not update, behind others that it does: the step raises before its first launch."""
+    import viola_amd
+    torch.manual_seed(9)
+    shapes = [(64, 128), (64, 128), (128, 64), (96,)]
+    params = [torch.nn.Parameter(torch.randn(*s, device="cuda")) for s in shapes]
+    if refused == "strided matrix":
+        params.append(torch.nn.Parameter(torch.randn(80, 48, device="cuda").t()))
+    elif refused == "strided vector":
+        params.append(torch.nn.Parameter(torch.randn(96, 2, device="cuda")[:, 0]))
+    else:
+        params.append(torch.nn.Parameter(torch.randn(64, 64, device="cuda").to(torch.float8_e4m3fn)))
+        params[-1].grad_dtype = torch.float32
+    opt = viola_amd.optim.FP8Muon(params[:-1], lr=1e-2)
+    for p in params:
+        p.grad = torch.randn(p.shape, device="cuda")
+    opt.step()
+    opt.add_param_group(dict(params=[params[-1]]))
+    before = [p.detach().clone() for p in params]
+    state = [{key: value.clone() if isinstance(value, torch.Tensor) else value for key, value in opt.state[p].items()} for p in params[:-1]]
+    with pytest.raises((RuntimeError, AssertionError)):
+        opt.step()
+    torch.cuda.synchronize()
+    for p, old, kept in zip(params, before, state + [{}]):
+        assert torch.equal(p.detach().view(torch.uint8) if p.element_size() == 1 else p, old.view(torch.uint8) if p.element_size() == 1 else old)
+        for key, value in kept.items():
+            assert torch.equal(opt.state[p][key], value) if isinstance(value, torch.Tensor) else opt.state[p][key] == value

@@ -332,6 +332,7 @@ private:
                     " elements of ", bytes_each, " bytes, it has ", state.numel(), " of ", state.element_size(), " on ", state.device());
     }
 
+    // Whatever is refused is refused here, before the first launch: a step that raises has changed nothing.
     static void prepare_vector(Item& it) {
         if (!it.state.contains("exp_avg")) {
             const auto options = at::TensorOptions().dtype(it.group->adam_state);
@@ -342,10 +343,13 @@ private:
         it.second = it.state["exp_avg_sq"].cast<Tensor>();
         check_state(it, it.first, it.param.numel(), it.first.element_size());
         check_state(it, it.second, it.param.numel(), it.first.element_size());
+        TORCH_CHECK(it.param.is_contiguous() && it.first.scalar_type() == it.second.scalar_type() && it.grad.numel() == it.param.numel(),
+                    "FP8Muon updates contiguous parameters, with both moments in one type");
     }
 
     static void prepare_matrix(Item& it) {
         TORCH_CHECK(it.param.dim() >= 2, "Muon updates matrices: a vector in a use_muon=True group");
+        TORCH_CHECK(it.param.is_contiguous(), "FP8Muon updates contiguous parameters");
         // 1-D tiles pad the payload to whole tiles, 2-D blocks do not
         const Group& g = *it.group;
         const std::vector<int64_t> shape = matrix_shape(it.param, g);
@@ -389,6 +393,27 @@ private:
         const c10::Stream main = guard.getStream(device);
         c10::Event start(device.type());
         start.record(main);
+        // the caller's stream waits for the lanes however this ends (an allocation may fail on the way): what they read is freed there
+        struct Join {
+            std::vector<c10::Stream>& streams;
+            size_t used;
+            c10::Stream main;
+            bool done = false;
+            void now() {
+                done = true;
+                for (size_t i = 0; i < used; ++i) {
+                    c10::Event event(main.device_type());
+                    event.record(streams[i]);
+                    event.block(main);
+                }
+            }
+            ~Join() {
+                try {
+                    if (!done) now();
+                } catch (...) {                                  // already on the way out with an error
+                }
+            }
+        } join{streams, used, main};
         // largest chains first, one lane after the other: the long ones start together and the short ones pack behind
         std::vector<size_t> order(ready.size());
         for (size_t i = 0; i < order.size(); ++i) order[i] = i;
@@ -400,11 +425,7 @@ private:
             const c10::StreamGuard on(lane);
             step_bucket(ready[order[slot]], ordinals[order[slot]]);
         }
-        for (size_t i = 0; i < used; ++i) {
-            c10::Event done(device.type());
-            done.record(streams[i]);
-            done.block(main);
-        }
+        join.now();
     }
 
     static double update_scale(const Group& g, int64_t rows, int64_t cols) {
@@ -465,7 +486,6 @@ private:
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Item& it = bucket[i];
             const Group& h = *it.group;
-            TORCH_CHECK(it.param.is_contiguous(), "FP8Muon updates contiguous parameters");
             VIOLA_CALL(viola_weight_update, it.param.mutable_data_ptr(), code_of(it.param.scalar_type()), from + 2 * count * i, update_code, count, (float)h.lr,
                        (float)h.weight_decay, (float)update_scale(h, rows, cols), h.master_rounding, it.step, master_key(it), 0, stream);
         }
@@ -483,7 +503,6 @@ private:
         std::vector<AdamRow> rows;
         std::vector<Tensor> grads;
         for (const Item& it : bucket) {
-            TORCH_CHECK(it.param.is_contiguous() && it.first.scalar_type() == it.second.scalar_type() && it.grad.numel() == it.param.numel());
             rows.push_back({it.param, it.grad, it.first, it.second, master_key(it), 0});
             grads.push_back(it.grad.contiguous());
         }
