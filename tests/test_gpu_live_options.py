@@ -59,3 +59,17 @@ def test_an_option_changed_after_the_first_call(scaling, name, value):
         assert torch.equal(got, want)
     if name == "accum_dtype":                                                      # FP16 partial sums are another product
         assert not torch.equal(after[0], before[0]) and rel_l2(after[0], before[0]) < .05
+
+
+@pytest.mark.parametrize("scaling", ["current", "delayed"])
+def test_an_empty_batch_leaves_the_quantizers_alone(scaling):
+    """It has no maximum: neither the calls counted nor the history change, and the next batch computes what it would have."""
+    x, dy = _data()
+    used, fresh = _layer(scaling), _layer(scaling)
+    empty = torch.empty(0, 256, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    y = used(empty)
+    y.backward(torch.empty(0, 192, device="cuda", dtype=torch.bfloat16))
+    assert y.shape == (0, 192) and empty.grad.shape == (0, 256) and used.weight.grad.count_nonzero() == 0 and used.bias.grad.count_nonzero() == 0
+    assert [q.index for q in (used.input_quantizer, used.grad_quantizer)] == [0, 0]
+    for got, want in zip(_step(used, x, dy), _step(fresh, x, dy)):
+        assert torch.equal(got, want)

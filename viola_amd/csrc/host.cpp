@@ -26,10 +26,12 @@ namespace {
 
 // ---------------------------------------------------------------------------------------------------- recipes
 // State of one per-tensor quantizer, shared with its module and with nodes that advance it in backward: calls so far (its slot in
-// the amax history), and whether its scale is that of the history (a checkpoint brings this along, so it may change).
+// the amax history), and whether its scale is that of the history (a checkpoint brings this along, so it may change). Atomic:
+// backward counts on autograd's thread, without the interpreter's lock, while the program may read or set it.
 struct Counter {
-    int64_t value = 0;
-    bool delayed = false;
+    std::atomic<int64_t> value;
+    std::atomic<bool> delayed;
+    Counter(int64_t value, bool delayed) : value(value), delayed(delayed) {}
 };
 
 // What a Linear's constructor fixed about its arithmetic. Standard recipes only: (1, 32) activation and gradient groups,
@@ -1029,9 +1031,9 @@ Layer layer_from(const py::tuple& t) {
 PYBIND11_MODULE(_host, m) {
     event_class = new py::object(py::module_::import("torch.cuda").attr("Event"));
     py::class_<Counter, std::shared_ptr<Counter>>(m, "Counter")
-        .def(py::init([](int64_t value, bool delayed) { return std::make_shared<Counter>(Counter{value, delayed}); }), py::arg("value") = 0, py::arg("delayed") = false)
-        .def_readwrite("value", &Counter::value)
-        .def_readwrite("delayed", &Counter::delayed)
+        .def(py::init([](int64_t value, bool delayed) { return std::make_shared<Counter>(value, delayed); }), py::arg("value") = 0, py::arg("delayed") = false)
+        .def_property("value", [](const Counter& c) { return c.value.load(); }, [](Counter& c, int64_t value) { c.value = value; })
+        .def_property("delayed", [](const Counter& c) { return c.delayed.load(); }, [](Counter& c, bool delayed) { c.delayed = delayed; })
         .def("__reduce__", [](py::object self) { return py::make_tuple(self.attr("__class__"), py::make_tuple(self.attr("value"), self.attr("delayed"))); });
     py::class_<Recipe, std::shared_ptr<Recipe>>(m, "Recipe")
         .def(py::init<const py::dict&>())
