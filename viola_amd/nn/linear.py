@@ -45,6 +45,16 @@ class _Quantizer(nn.Module):
         self.__dict__.update(_calls=0, _counter=None, _scaling=scaling)
         self.register_buffer("history", torch.zeros(history_len, device=device, dtype=torch.float32))
 
+    def __setstate__(self, state):
+        """A module pickled whole, also one from when these were plain attributes."""
+        state = dict(state)
+        for public, held in (("scaling", "_scaling"), ("index", "_calls")):
+            if public in state:
+                state[held] = state.pop(public)
+        super().__setstate__(dict(dict(_counter=None), **state))
+        if self._counter is not None:
+            self._counter.delayed = self._scaling == "delayed"
+
     @property
     def scaling(self):
         return self._scaling
@@ -266,6 +276,9 @@ class Linear(nn.Module):
         for operand in ("weight", "input", "grad"):
             setattr(self, f"{operand}_quantizer", _Quantizer(scaling, history_len, device))
         self.reset_parameters()
+
+    def __setstate__(self, state):
+        super().__setstate__(dict(state, _recipe=None))                        # made again from the options
 
     def __setattr__(self, name, value):
         super().__setattr__(name, value)
