@@ -1,0 +1,98 @@
+"""GPU parity: the large-tile form of the grouped-scale products (256 x 256, row-wise b scales 256 x 128) at its edges.
+
+Integer operands and power-of-two scales throughout, so that the sums are exact in FP32 and every element must equal the integer
+product, rounded once where the output is narrower."""
+
+import pytest
+import torch
+
+from viola_amd import _lib
+
+pytestmark = pytest.mark.gpu
+E4, E5 = torch.float8_e4m3fn, torch.float8_e5m2
+
+
+def _integers(*shape):
+    return torch.randint(-2, 3, shape, device="cuda").float()
+
+
+def _scales(*shape):
+    return torch.exp2(torch.randint(-1, 2, shape, device="cuda").float())
+
+
+def _spell(t, s, rows):
+    return t * s.repeat_interleave(rows, 0)[:t.shape[0]].repeat_interleave(32, 1)[:, :t.shape[1]]
+
+
+# rows and columns short of the last tile, columns whose rows of the output are 16-byte aligned or not; k that ends inside a chunk
+# of 64, inside a piece of four scales and inside a block of eight
+@pytest.mark.parametrize("gb", [(32, 32), (1, 32)])
+@pytest.mark.parametrize("m,n,k,formats,out_dtype", [(4090, 4070, 2064, (E4, E4), torch.float32), (4096, 4096, 1536, (E5, E4), torch.bfloat16),
+                                                     (4001, 4072, 2272, (E4, E5), torch.float16), (8190, 8180, 2592, (E5, E5), torch.bfloat16)])
+def test_grouped_products_on_large_tiles(m, n, k, formats, out_dtype, gb):
+    from viola_amd.nn import _grouped_kernels as g
+    torch.manual_seed(m + n + k)
+    a, b, groups = _integers(m, k), _integers(n, k), -(-k // 32)
+    sa, sb = _scales(m, groups), _scales(-(-n // gb[0]), groups)
+    bias = torch.randint(-8, 9, (n,), device="cuda").float()
+    out = g.gemm(a.to(formats[0]), b.to(formats[1]), sa, sb, (1, 32), gb, out_dtype=out_dtype, bias=bias)
+    assert torch.equal(out, (_spell(a, sa, 1) @ _spell(b, sb, gb[0]).T + bias).to(out_dtype))
+
+
+@pytest.mark.parametrize("gb", [(32, 32), (1, 32)])
+@pytest.mark.parametrize("k", [1568, 1824])                                  # 49 and 57 groups: one scale in the last piece, and in the last block
+def test_scales_of_the_next_row_do_not_leak_on_large_tiles(gb, k):
+    """The piece that holds a row's last scales reaches into the next row's: a NaN or an Inf there stays in its own row."""
+    from viola_amd.nn import _grouped_kernels as g
+    torch.manual_seed(k)
+    m, n = 4096, 4096
+    a, b = _integers(m, k), _integers(n, k)
+    sa, sb = _scales(m, k // 32), _scales(n // gb[0], k // 32)
+    clean = g.gemm(a.to(E4), b.to(E4), sa, sb, (1, 32), gb, out_dtype=torch.float32)
+    bad = [7, 256, 4095]
+    sa[bad, 0] = torch.tensor([float("nan"), float("inf"), float("nan")], device="cuda")
+    out = g.gemm(a.to(E4), b.to(E4), sa, sb, (1, 32), gb, out_dtype=torch.float32)
+    keep = torch.ones(m, dtype=torch.bool, device="cuda")
+    keep[bad] = False
+    assert torch.equal(out[keep], clean[keep]) and not torch.isfinite(out[bad]).all()
+    sa[bad, 0] = 1.0
+    base = g.gemm(a.to(E4), b.to(E4), sa, sb, (1, 32), gb, out_dtype=torch.float32)
+    row = 65
+    sb[row, 0] = float("nan")
+    out = g.gemm(a.to(E4), b.to(E4), sa, sb, (1, 32), gb, out_dtype=torch.float32)
+    inside = torch.arange(n, device="cuda") // gb[0] == row
+    assert torch.equal(out[:, ~inside], base[:, ~inside]) and torch.isnan(out[:, inside]).all()
+
+
+@pytest.mark.parametrize("counts", [[7500, 0, 1, 7400, 256, 15843, 0], [1000] * 66])
+def test_varlen_products_on_large_tiles(counts):
+    """Row ranges per group (more groups than a count of 64 covers in the second case), empty ones among them."""
+    torch.manual_seed(len(counts))
+    groups, n, k, total = len(counts), 1000, 2048, sum(counts)
+    a, b = _integers(total, k), _integers(groups, n, k)
+    offsets = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], device="cuda")
+    sa, sb = _scales(total, k // 32), _scales(groups, -(-n // 32), k // 32)
+    out, qa, qb = torch.full((total, n), 7.0, device="cuda"), a.to(E4), b.to(E4)
+    _lib.call("viola_varlen_group_gemm", qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E4), sa.data_ptr(), sb.data_ptr(), offsets.data_ptr(),
+              groups, total, n, k, 1, 32, 32, 32, n * k, sb[0].numel(), out.data_ptr(), 0)
+    row = 0
+    for g, c in enumerate(counts):
+        assert torch.equal(out[row:row + c], _spell(a[row:row + c], sa[row:row + c], 1) @ _spell(b[g], sb[g], 32).T)
+        row += c
+
+
+def test_varlen_weight_gradient_on_large_tiles():
+    """k ranges per group: none, one slot of 32, ranges that end inside a chunk."""
+    torch.manual_seed(3)
+    slots, n, kout = [0, 2080, 32, 4096, 1952, 0, 2176], 1024, 4000
+    offsets = torch.tensor([0, *torch.tensor(slots).cumsum(0).tolist()], device="cuda")
+    total = -(-sum(slots) // 128) * 128
+    a, b = _integers(n, total), _integers(kout, total)
+    sa, sb = _scales(n, total // 32), _scales(kout, total // 32)
+    out, qa, qb = torch.full((len(slots), n, kout), 7.0, device="cuda"), a.to(E4), b.to(E5)
+    _lib.call("viola_varlen_wgrad_gemm", qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E5), sa.data_ptr(), sb.data_ptr(), offsets.data_ptr(),
+              len(slots), total, n, kout, out.data_ptr(), 0)
+    a, b, start = _spell(a, sa, 1), _spell(b, sb, 1), 0
+    for g, length in enumerate(slots):
+        assert torch.equal(out[g], a[:, start:start + length] @ b[:, start:start + length].T)
+        start += length

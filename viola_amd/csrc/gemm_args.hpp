@@ -48,6 +48,11 @@ int launch_group_gemm_half(const GemmArgs& p, bool per_tensor, int a_dtype, int 
 int launch_group_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype,
                            bool rowscale, dim3 grid, hipStream_t stream);
 
+// The grouped recipe on tiles of 256 x 256 (row-wise b scales: 256 x 128); row_tiles: tiles of 256 rows (variable groups: a bound on
+// them), groups: k ranges. gemm_pingpong_grouped.hip.
+int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, unsigned groups,
+                          hipStream_t stream);
+
 // Per-tensor scales on the same fast kernel (one v_mfma_f32_32x32x64_f8f6f4 per sub-tile and 64 k); mode = MODE_PLAIN or a
 // gated mode (grid.x then counts the gated tile width). Defined in gemm_fast.hip.
 int launch_tensor_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, dim3 grid,

@@ -1,5 +1,7 @@
 // Grouped FP32-scale instances of the fast FP8 GEMM kernel (plain, gated forward, gated backward; uniform or
 // row-wise b scales).
+#include <math.h>
+
 #include "gemm_fast_kernel.hpp"
 
 namespace viola {
@@ -52,12 +54,40 @@ static int launch_mode(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dty
 constexpr int64_t SPLIT_MIN_K = 1536, NARROW_SPLIT_MIN_K = 1024;
 
 
+// Whether a plain product runs on gemm_pingpong_grouped: the lesser of two estimates in microseconds, fitted to the measured times
+// of 42 shapes (bf16 outputs, within 8 % of nearly all). Two blocks of 128 x 128 of group_gemm_fast share a CU and cover each
+// other's first loads and stores, so a round of 512 costs little beside its chunks of 64 k, and a last one of up to 256 goes
+// faster; the large tiles take a CU each, whole rounds of 256, with nothing to cover their ends. So they win from about k = 1024
+// (8192 x 4096 x 1024 74 -> 68 us, 16384 x 4096 x 256 55 -> 56) where they fill the chip (4096 x 4096 x 2048, 256 of them, 68 -> 61;
+// 6000 x 4096 x 1024, 384, 55 -> 60; row-wise 4096 x 3072 x 8192, 384, 245 -> 251). At 256 tiles of 128 x 128 and fewer the split
+// forms have more of the chip at work (8192 x 4096 x 1024 transposed, 88 -> 115 us). Groups of rows fill half of their last tile
+// on average; groups of k have each the average length.
+static bool prefer_pingpong(const GemmArgs& p, bool rowscale, unsigned k_groups) {
+    constexpr double CUS = 256.0;
+    if (p.k < 256 || 256 * p.lda >= (1ll << 31)) return false;
+    auto tiles = [&](int64_t rows, int64_t cols) {
+        const double row_tiles = p.offsets ? (double)p.m / rows + 0.5 * p.groups : (double)((p.m + rows - 1) / rows);
+        return row_tiles * (double)((p.n + cols - 1) / cols) * k_groups;
+    };
+    const double chunks = (double)p.k / 64.0 / k_groups, small = tiles(128, 128), large = tiles(256, rowscale ? 128 : 256);
+    if (small <= CUS) return false;
+    const double pair = rowscale ? 1.2 : 0.97, idle = rowscale ? 0.82 : 1.2, busy = rowscale ? 1.04 : 1.61, ends = rowscale ? 6.0 : 7.5;
+    const double pairs = floor(small / (2 * CUS)), left = small - pairs * 2 * CUS;
+    const double now = pairs * (chunks * pair + 3.3) + (left > 0 ? chunks * pair * (left <= CUS ? 0.52 : 1.0) + 3.3 : 0.0);
+    const double rounds = floor(large / CUS), rest = large / CUS - rounds;
+    return rounds * (chunks * busy + ends) + (rest > 0 ? chunks * (idle + (busy - idle) * rest) + ends : 0.0) < now;
+}
+
 int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale,
                            dim3 grid, hipStream_t stream) {
     GemmArgs p = args;
     const int64_t b_rows = mode == MODE_GATED_FWD ? 2 * p.n : p.n;
     p.sa_bytes = (p.m + p.ar - 1) / p.ar * p.ldsa * 4;
     p.sb_bytes = (b_rows + p.br - 1) / p.br * p.ldsb * 4;
+    if (mode == MODE_PLAIN && prefer_pingpong(p, rowscale, grid.z)) {
+        const int64_t row_tiles = p.offsets ? p.m / 256 + p.groups : (p.m + 255) / 256;
+        return launch_group_pingpong(p, (int)row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid.z, stream);
+    }
     // Two blocks of 128 x 128 fit a CU, so from 257 tiles up every CU has work and the full tile, which reads the least, is
     // the fastest form (4096 x 1152 x 4608: 75.6 -> 59.7 us against the split one, 6000 x 1000 x 1024: 27.0 -> 19.6 us against
     // tiles halved in n). From 129 to 256 tiles a CU gets one: over a long k keep the tile and split its k range over twice the

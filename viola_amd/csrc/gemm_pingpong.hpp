@@ -8,6 +8,8 @@
 // one operand register set per wave is enough (the 128 x 128 kernel reads the next chunk's operands in a burst ahead of its
 // MFMAs, which then wait for that burst to issue).
 #pragma once
+#include <type_traits>
+
 #include "gemm_fast_kernel.hpp"
 
 namespace viola {
@@ -21,6 +23,62 @@ struct PingPongShape {
     static constexpr int A_LOADS = ROWS / 128, B_LOADS = COLS / 128, LOADS = A_LOADS + B_LOADS;   // 512 threads x 16 bytes = 128 rows
     static_assert(WM * WN == 8 && ROWS % 128 == 0 && COLS % 128 == 0);
 };
+
+// Epilogue. The tile's bias as fp32 in LDS (COLS floats), -0 where there is none: adding that changes nothing, not even a sign.
+template <typename S, bool GATED = false>
+__device__ __forceinline__ void stage_bias(const GemmArgs& p, int64_t n_begin, float* bias_lds, int bias_dtype) {
+    constexpr int PANEL = GATED ? S::COLS / 2 : S::COLS;
+    const int tid = threadIdx.x;
+    if (tid < S::COLS) {
+        const int64_t col = n_begin + tid % PANEL;
+        bias_lds[tid] = p.bias && col < p.n ? load_float(p.bias, (GATED ? tid / PANEL * p.n : 0) + col, bias_dtype) : -0.0f;
+    }
+    __syncthreads();
+}
+
+// A wave parks its first SUBS sub-tile columns, 32 rows at a time, in its own part of the ring (which every wave has left) and
+// stores them as 16-byte pieces along the rows. The bias (nullptr: added before) is added on the way: before it, on all totals
+// at once, the 256 x 256 tiles have no registers to spare (48 spilled; 70 instead of 68 us at 8192 x 4096 x 1024, grouped).
+template <typename S, int SUBS, bool BIAS, typename TO>
+__device__ __forceinline__ void store_tile(const f32x16 (&total)[S::TN][S::TM], const GemmArgs& p, TO* out, int64_t m_begin, int64_t m_end,
+                                           int64_t n_begin, uint8_t* ring, const float* bias_lds) {
+    const int lane = threadIdx.x % WAVE, l32 = lane % 32, lhi = lane / 32;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE), wm = wave / S::WN, wn = wave % S::WN;
+    const bool pieces_out = (p.ldo * sizeof(TO)) % 16 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    constexpr int PER = 16 / (int)sizeof(TO), COLS_W = 32 * SUBS, PLD = COLS_W + PER, PIECES = COLS_W / PER;
+    static_assert(8 * 32 * PLD * (int)sizeof(TO) <= S::STAGES * S::STAGE);
+    TO* park = reinterpret_cast<TO*>(ring) + wave * 32 * PLD;
+    const int64_t ncol0 = n_begin + wn * COLS_W;
+#pragma unroll
+    for (int j = 0; j < S::TM; ++j) {
+        const int64_t row0 = m_begin + (wm * S::TM + j) * 32;
+#pragma unroll
+        for (int i = 0; i < SUBS; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v[4] = {total[i][j][4 * q], total[i][j][4 * q + 1], total[i][j][4 * q + 2], total[i][j][4 * q + 3]};
+                if constexpr (BIAS) {
+                    const float4 bq = *reinterpret_cast<const float4*>(&bias_lds[(wn * SUBS + i) * 32 + q * 8 + lhi * 4]);
+                    v[0] += bq.x; v[1] += bq.y; v[2] += bq.z; v[3] += bq.w;
+                }
+                Quad<TO>::store(&park[l32 * PLD + i * 32 + q * 8 + lhi * 4], v);
+            }
+#pragma unroll
+        for (int it = 0; it < 32 * PIECES / WAVE; ++it) {
+            const int id = it * WAVE + lane, pr = id / PIECES, pc = id % PIECES;
+            const int64_t mrow = row0 + pr, ncol = ncol0 + pc * PER;
+            const uint4 value = *reinterpret_cast<const uint4*>(&park[pr * PLD + pc * PER]);
+            if (mrow >= m_end || ncol >= p.n) continue;
+            if (pieces_out && ncol + PER <= p.n) {
+                store_streaming(out + mrow * p.ldo + ncol, value);
+            } else {
+                const TO* values = reinterpret_cast<const TO*>(&value);
+                for (int e = 0; e < PER; ++e)
+                    if (ncol + e < p.n) out[mrow * p.ldo + ncol + e] = values[e];
+            }
+        }
+    }
+}
 
 // GATED: the tile's b rows are COLS / 2 gate rows, then the up rows of the same columns of h (sub-tiles 0 and 1 of a wave);
 // out = act(g) * u, [g | u] itself is not kept.
@@ -208,32 +266,23 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     }
     barrier();                                                               // every wave has left the ring
     float* bias_lds = reinterpret_cast<float*>(lds + RING);
-    if (p.bias) {
-        if (tid < S::COLS) {
-            const int64_t col = n_begin + tid % PANEL;
-            bias_lds[tid] = col < p.n ? load_float(p.bias, (GATED ? tid / PANEL * p.n : 0) + col, bias_dtype) : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < TN; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float4 bq = *reinterpret_cast<const float4*>(&bias_lds[(GATED ? wn : wn * TN) * 32 + i * NEXT_B + q * 8 + lhi * 4]);
-#pragma unroll
-                for (int j = 0; j < TM; ++j) {
-                    total[i][j][4 * q] += bq.x; total[i][j][4 * q + 1] += bq.y; total[i][j][4 * q + 2] += bq.z; total[i][j][4 * q + 3] += bq.w;
-                }
-            }
-    }
+    stage_bias<S, GATED>(p, n_begin, bias_lds, bias_dtype);
     // (one kernel for the three output types: they differ from here on only)
     auto finish = [&](auto type) {
         using TO = decltype(type);
-        TO* out = static_cast<TO*>(p.out);
         if constexpr (GATED) {
+            float4 bias_g[4], bias_u[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                bias_g[q] = *reinterpret_cast<const float4*>(&bias_lds[wn * 32 + q * 8 + lhi * 4]);
+                bias_u[q] = *reinterpret_cast<const float4*>(&bias_lds[PANEL + wn * 32 + q * 8 + lhi * 4]);
+            }
 #pragma unroll
             for (int j = 0; j < TM; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
+                    total[0][j][r] += (&bias_g[r / 4].x)[r % 4];
+                    total[TN - 1][j][r] += (&bias_u[r / 4].x)[r % 4];
                     float act, derivative, h;
                     gate_math(p.activation, rounded<TO>(total[0][j][r]), act, derivative);
                     h = act * rounded<TO>(total[TN - 1][j][r]);
@@ -241,37 +290,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
                     total[0][j][r] = h;
                 }
         }
-        const bool pieces_out = (p.ldo * sizeof(TO)) % 16 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-        // a wave parks 32 rows at a time in its own part of the ring and stores them as 16-byte pieces along the rows
-        constexpr int SUBS = GATED ? 1 : TN, PER = 16 / (int)sizeof(TO), COLS_W = 32 * SUBS, PLD = COLS_W + PER, PIECES = COLS_W / PER;
-        static_assert(8 * 32 * PLD * (int)sizeof(TO) <= RING);
-        TO* park = reinterpret_cast<TO*>(lds) + wave * 32 * PLD;
-        const int64_t ncol0 = n_begin + wn * COLS_W;
-#pragma unroll
-        for (int j = 0; j < TM; ++j) {
-            const int64_t row0 = m_begin + (wm * TM + j) * 32;
-#pragma unroll
-            for (int i = 0; i < SUBS; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float v[4] = {total[i][j][4 * q], total[i][j][4 * q + 1], total[i][j][4 * q + 2], total[i][j][4 * q + 3]};
-                    Quad<TO>::store(&park[l32 * PLD + i * 32 + q * 8 + lhi * 4], v);
-                }
-#pragma unroll
-            for (int it = 0; it < 32 * PIECES / WAVE; ++it) {
-                const int id = it * WAVE + lane, pr = id / PIECES, pc = id % PIECES;
-                const int64_t mrow = row0 + pr, ncol = ncol0 + pc * PER;
-                const uint4 value = *reinterpret_cast<const uint4*>(&park[pr * PLD + pc * PER]);
-                if (mrow >= p.m || ncol >= p.n) continue;
-                if (pieces_out && ncol + PER <= p.n) {
-                    store_streaming(out + mrow * p.ldo + ncol, value);
-                } else {
-                    const TO* values = reinterpret_cast<const TO*>(&value);
-                    for (int e = 0; e < PER; ++e)
-                        if (ncol + e < p.n) out[mrow * p.ldo + ncol + e] = values[e];
-                }
-            }
-        }
+        store_tile<S, GATED ? 1 : TN, !GATED>(total, p, static_cast<TO*>(p.out), m_begin, p.m, n_begin, lds, bias_lds);
     };
     if (out_dtype == VIOLA_F32) finish(float{});
     else if (out_dtype == VIOLA_BF16) finish(bf16_t{});

@@ -1,0 +1,368 @@
+// Plain products with FP32 scales per 32 k (the grouped recipe) on large tiles: the phases of gemm_pingpong.hpp with the fold of
+// gemm_fast_kernel.hpp. A block of eight waves owns one tile; waves 0-3 and 4-7 alternate between reading operands and multiplying.
+//
+// What bounds it. A unit (32 x 32 outputs, one K group) is two K = 16 MFMAs, 64 cycles of the matrix pipe, and 16 FMAs that fold
+// the group's sums into the totals under sa * sb. A wave issues an FMA every 4.3 cycles, an MFMA every 6 or so, 82 to 87 cycles
+// for the unit; and under that load on random data the card is at its power limit (1.8 - 1.9 GHz), so what counts next is the
+// energy spent beside the arithmetic. Hence the tiles: 256 x 256 with 64 x 128 outputs per wave reads 768 bytes of operands from
+// LDS per unit where 64 x 64 per wave read 1024, and fetches half of what two tiles of 128 x 128 fetch.
+//
+// Uniform b scales (forward, data gradient; ROWS false, 256 x 256). Three accumulators rotate: the FMAs among the MFMAs of unit u fold unit
+// u - 2, whose sums are there without a wait (two accumulators, folding unit u - 1, cost nine wait states a unit: 500 against
+// 432 us at 16384 x 4096 x 4096). The last two units of a chunk are folded in the wave's next read phase, under the other half's
+// MFMAs, so that the accumulators' numbering starts over with each chunk; all 256 registers are in use.
+//   16384 x 4096 x 4096   505 -> 445 us    16384 x 22016 x 4096   2700 -> 2400    8192 x 4096 x 1024   76 -> 67
+// Row-wise b scales (weight gradient; ROWS true, 256 x 128). The products sa * sb of a pair of units come from one
+// v_mfma_f32_32x32x1_2b (see group_gemm_fast), which occupies the FMA units for its 64 cycles as well; the pair of units before
+// is folded meanwhile, across chunks too, out of two sets of accumulators and products.
+//   22016 x 4096 x 16384  3450 -> 3070 us  4096 x 11008 x 16384   1660 -> 1545    4096 x 4096 x 4096   160 -> 142
+#pragma once
+#include "gemm_pingpong.hpp"
+
+namespace viola {
+
+using GroupedWide = PingPongShape<2, 4, 4, 2, 4>;                            // uniform b scales: 64 x 128 outputs (a x b) per wave, transposed
+using GroupedRows = PingPongShape<4, 2, 2, 2, 4>;                            // row-wise b scales: 64 x 64
+
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+// Row tiles (of ROWS rows) of group base + lane, and of all groups base .. base + lane together.
+template <int ROWS>
+__device__ __forceinline__ void group_row_tiles(const GemmArgs& p, int base, int& tiles, int& end) {
+    const int lane = threadIdx.x % WAVE, g = base + lane;
+    tiles = g < p.groups ? (int)((p.offsets[g + 1] - p.offsets[g] + ROWS - 1) / ROWS) : 0;
+    end = tiles;
+#pragma unroll
+    for (int step = 1; step < WAVE; step *= 2) {
+        const int below = __shfl_up(end, step, WAVE);
+        if (lane >= step) end += below;
+    }
+}
+
+template <bool A_BF8, bool B_BF8, bool ROWS>
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int bias_dtype, int out_dtype) {
+    using S = std::conditional_t<ROWS, GroupedRows, GroupedWide>;
+    constexpr int TM = S::TM, TN = S::TN, STAGES = S::STAGES, RING = STAGES * S::STAGE;
+    // A scale block is 8 K groups in 16-byte pieces of 4: [half][row of a], then [half][row of b], or with uniform b scales
+    // [half][sub-tile of b] (what 64 lanes of one load instruction bring)
+    constexpr int B_ENTRIES = ROWS ? S::COLS : S::COLS / 32;
+    constexpr int A_SCALES = 2 * S::ROWS * 16, B_SCALES = ROWS ? 2 * B_ENTRIES * 16 : 1024, SCALE_BLOCK = A_SCALES + B_SCALES;
+    static_assert(2 * S::ROWS == 512 && (ROWS || 2 * B_ENTRIES <= 64) && 2 * SCALE_BLOCK >= S::COLS * 4);
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[RING + 2 * SCALE_BLOCK];
+    const int tid = threadIdx.x, lane = tid % WAVE, l32 = lane % 32, lhi = lane / 32;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int wm = wave / S::WN, wn = wave % S::WN;
+
+    // ---- tile: contiguous ranges per XCD, walked in groups of 4 m tiles, so that the 32 tiles at work on an XCD are 4 x 8
+    // (8 x 4: 70 instead of 67 us at 8192 x 4096 x 1024). Variable groups: see group_gemm_fast.
+    constexpr int WALK = 4;
+    int tiles_m = p.tiles_m, group_tiles = 0, group_end = 0;
+    if (p.offsets) {
+        tiles_m = 0;
+        for (int base = 0; base < p.groups; base += WAVE) {
+            int count, end;
+            group_row_tiles<S::ROWS>(p, base, count, end);
+            if (base == 0) { group_tiles = count; group_end = end; }
+            tiles_m += __builtin_amdgcn_readlane(end, WAVE - 1);
+        }
+    }
+    const int per_xcd = p.offsets ? (int)(((int64_t)tiles_m * p.tiles_n + 7) / 8) : (int)(gridDim.x / 8);
+    const int seq = blockIdx.x / 8, t = (blockIdx.x % 8) * per_xcd + seq;
+    if (seq >= per_xcd || t >= tiles_m * p.tiles_n) return;
+    const int walk = WALK * p.tiles_n, first_m = t / walk * WALK;
+    const int rows_here = tiles_m - first_m < WALK ? tiles_m - first_m : WALK;
+    const int tile_m = first_m + t % walk % rows_here;
+    const int64_t n_begin = (int64_t)(t % walk / rows_here) * S::COLS;
+    int64_t m_begin = (int64_t)tile_m * S::ROWS, m_end = p.m, k_begin = 0, k_end = p.k;
+    const uint8_t* bptr = p.b;
+    const float* sbptr = p.sb;
+    int64_t out_shift = 0;
+    if (p.offsets) {
+        int tile = tile_m, g = 0;
+        for (int base = 0;; base += WAVE) {                                  // ends: tile_m is one of the tiles counted above
+            if (base) group_row_tiles<S::ROWS>(p, base, group_tiles, group_end);
+            const uint64_t past = __builtin_amdgcn_ballot_w64(tile < group_end);
+            if (past) {
+                const int at = __builtin_ctzll(past);
+                tile -= __builtin_amdgcn_readlane(group_end - group_tiles, at);
+                g = base + at;
+                break;
+            }
+            tile -= __builtin_amdgcn_readlane(group_end, WAVE - 1);
+        }
+        m_begin = p.offsets[g] + (int64_t)tile * S::ROWS;
+        m_end = p.offsets[g + 1];
+        bptr += (int64_t)g * p.b_group_stride;
+        sbptr += (int64_t)g * p.sb_group_stride;
+    }
+    if (p.koffsets) {
+        k_begin = p.koffsets[blockIdx.z];
+        k_end = p.koffsets[blockIdx.z + 1];
+        out_shift = (int64_t)blockIdx.z * p.out_group_stride;
+    }
+    const int64_t k_len = k_end - k_begin;
+
+    // ---- load plan: as in gemm_pingpong
+    const i32x4 res_a = raw_resource(p.a + m_begin * p.lda + k_begin), res_b = raw_resource(bptr + k_begin);
+    constexpr uint32_t OUTSIDE = 0x80000000u;
+    const int chunks = (int)((k_len + FBK - 1) / FBK), full_chunks = (int)(k_len / FBK), groups_total = (int)((k_len + 31) / 32);
+    const int piece = (tid & 3) ^ ((tid >> 4) & 3);
+    const bool inside_tail = (int64_t)full_chunks * FBK + piece * 16 < k_len;
+    auto row_in = [](int64_t row, int64_t rows) -> uint32_t { return (uint32_t)(row < rows ? row : rows - 1); };
+    uint32_t cur[S::LOADS];
+#pragma unroll
+    for (int it = 0; it < S::LOADS; ++it) {
+        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * 128 + tid / 4;
+        if (it < S::A_LOADS) cur[it] = (uint32_t)(row_in(m_begin + r, m_end) - m_begin) * (uint32_t)p.lda;
+        else cur[it] = row_in(n_begin + r, p.n) * (uint32_t)p.ldb;
+        asm volatile("" : "+v"(cur[it]));                                    // (as one 64-bit multiply-add it would hold a register pair all along)
+        cur[it] += piece * 16;
+    }
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    auto issue = [&](int c, int stage) {
+        if (__builtin_expect(c >= full_chunks, 0)) {                         // the chunk that straddles the end of k, and those past it
+            asm volatile("; end of the k range");
+            const bool here = c == full_chunks && inside_tail;
+#pragma unroll
+            for (int it = 0; it < S::LOADS; ++it) {
+                const uint32_t at = here ? cur[it] : OUTSIDE;
+                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, at, (uint32_t)c * FBK);
+            }
+            return;
+        }
+#pragma unroll
+        for (int it = 0; it < S::LOADS; ++it)
+            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * FBK);
+    };
+    // Scale block `block` -> buffer block & 1: every thread one piece of the a rows, the first waves one of b (lanes past b's last
+    // entry read zero). Entries past the end of the k range, which hold whatever follows in memory (see group_gemm_fast), are
+    // cleared once in LDS.
+    const i32x4 res_sa = raw_resource(p.sa, p.sa_bytes), res_sb = raw_resource(sbptr, p.sb_bytes);
+    const int a_half = wave * WAVE / S::ROWS, b_half = ROWS ? wave * WAVE / B_ENTRIES : lane / B_ENTRIES;
+    const uint32_t group0 = (uint32_t)(k_begin >> 5) * 4;
+    uint32_t sa_at = row_in(m_begin + tid % S::ROWS, m_end) / (uint32_t)p.ar * (uint32_t)p.ldsa * 4 + group0 + a_half * 16;
+    uint32_t sb_at = row_in(n_begin + tid % B_ENTRIES * (ROWS ? 1 : 32), p.n) / (uint32_t)p.br * (uint32_t)p.ldsb * 4 + group0 + b_half * 16;
+    if (b_half >= 2) sb_at = OUTSIDE;
+    asm volatile("" : "+v"(sa_at), "+v"(sb_at));
+    const int last_block = (groups_total - 1) / F_SGROUPS;
+    auto issue_scales = [&](int block) {                                     // (past the last block: that one again, to keep the load counts uniform)
+        const uint32_t to = lds_base + RING + (uint32_t)(block & 1) * SCALE_BLOCK + (uint32_t)wave * 1024;
+        const uint32_t first = (uint32_t)(block < last_block ? block : last_block) * F_SGROUPS * 4;
+        if (wave < B_SCALES / 1024) load16_to_lds(res_sb, to + A_SCALES, sb_at, first);
+        load16_to_lds(res_sa, to, sa_at, first);
+    };
+    const bool straddles = groups_total % F_SGROUPS != 0;
+    auto clear_past_the_end = [&] {
+        const int left_a = groups_total - (last_block * F_SGROUPS + a_half * 4), left_b = groups_total - (last_block * F_SGROUPS + b_half * 4);
+        float* mine = reinterpret_cast<float*>(lds + RING + (last_block & 1) * SCALE_BLOCK + tid * 16);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (q >= left_a) mine[q] = 0.0f;
+            if (q >= left_b && wave < B_SCALES / 1024) mine[A_SCALES / 4 + q] = 0.0f;
+        }
+    };
+
+    // ---- operands: a lane's 16 bytes of K group kg of its row in every sub-tile, and the scales
+    const int sw = (l32 >> 2) & 3;
+    const int rd_a = (wm * TM * 32 + l32) * FBK + ((lhi ^ sw) * 16), rd_b = S::A_BYTES + (wn * TN * 32 + l32) * FBK + ((lhi ^ sw) * 16);
+    f32x16 total[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) total[i][j][r] = 0.0f;
+    i32x4 oa[FKG][TM], ob[FKG][TN];
+    // sa[j]: of the lane's row in sub-tile j; ROWS: sa[0] of row `lane` of the wave's 64, the operand of the scale products
+    constexpr int SA = ROWS ? 1 : TM;
+    float sa[SA][FKG], sb[TN][FKG];
+    auto read = [&](int stage, int c) {
+        // (addresses of K group 1 made here from those of K group 0: kept over the loop they would take two registers too many)
+        int at_a = stage * S::STAGE + rd_a, at_b = stage * S::STAGE + rd_b;
+        asm volatile("" : "+v"(at_a), "+v"(at_b));
+#pragma unroll
+        for (int kg = 0; kg < FKG; ++kg) {
+#pragma unroll
+            for (int i = 0; i < TN; ++i) ob[kg][i] = *reinterpret_cast<const i32x4*>(lds + (at_b ^ (kg * 32)) + i * 32 * FBK);
+#pragma unroll
+            for (int j = 0; j < TM; ++j) oa[kg][j] = *reinterpret_cast<const i32x4*>(lds + (at_a ^ (kg * 32)) + j * 32 * FBK);
+        }
+        const int g8 = c % F_SCHUNKS * FKG;                                  // group of the block (even: both groups of the chunk in one read)
+        const float* block = reinterpret_cast<const float*>(lds + RING + ((c / F_SCHUNKS) & 1) * SCALE_BLOCK);
+#pragma unroll
+        for (int j = 0; j < SA; ++j) {
+            const float2 v = *reinterpret_cast<const float2*>(&block[((g8 >> 2) * S::ROWS + wm * TM * 32 + j * 32 + (ROWS ? lane : l32)) * 4 + (g8 & 3)]);
+            sa[j][0] = v.x; sa[j][1] = v.y;
+        }
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+            const int entry = ROWS ? (wn * TN + i) * 32 + l32 : wn * TN + i;
+            const float2 v = *reinterpret_cast<const float2*>(&block[A_SCALES / 4 + ((g8 >> 2) * B_ENTRIES + entry) * 4 + (g8 & 3)]);
+            // (uniform: into scalar registers)
+            sb[i][0] = ROWS ? v.x : __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v.x)));
+            sb[i][1] = ROWS ? v.y : __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v.y)));
+        }
+    };
+    auto pin_operands = [&] {                                                // in registers before the barrier
+#pragma unroll
+        for (int kg = 0; kg < FKG; ++kg) {
+#pragma unroll
+            for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(oa[kg][j]));
+#pragma unroll
+            for (int j = 0; j < SA; ++j) asm volatile("" : "+v"(sa[j][kg]));
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                asm volatile("" : "+v"(ob[kg][i]));
+                if constexpr (ROWS) asm volatile("" : "+v"(sb[i][kg]));
+                else asm volatile("" : "+s"(sb[i][kg]));
+            }
+        }
+    };
+
+    // ---- math
+    const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    auto product = [&](int kg, int i, int j, int half, const f32x16& onto) -> f32x16 {
+        auto codes = [&](const i32x4& v) -> long { return (long)(((uint64_t)(uint32_t)v[2 * half + 1] << 32) | (uint32_t)v[2 * half]); };
+        return mfma32<A_BF8, B_BF8>(codes(ob[kg][i]), codes(oa[kg][j]), onto);
+    };
+    constexpr int ACCS = ROWS ? 4 : 3;
+    f32x16 acc[ACCS];
+#pragma unroll
+    for (int x = 0; x < ACCS; ++x)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[x][r] = 0.0f;
+    // uniform b scales: units in the order (kg, i, j), unit u in accumulator u % 3
+    constexpr int UNITS = FKG * TN * TM, LAG = 2;
+    float scale[ACCS] = {};
+    auto fold_unit = [&](int u, int first, int count) {
+        const int i = u / TM % TN, j = u % TM, x = u % ACCS;
+#pragma unroll
+        for (int r = first; r < first + count; ++r) total[i][j][r] = fmaf(acc[x][r], scale[x], total[i][j][r]);
+    };
+    // row-wise: pairs of units (kg, i, j = 0 and 1), pair q in accumulators 2 (q & 1) + j, its scale products in prod[q & 1]
+    constexpr int PAIRS = FKG * TN;
+    f32x32 prod[ROWS ? 2 : 1];
+    if constexpr (ROWS) {
+#pragma unroll
+        for (int r = 0; r < 32; ++r) prod[0][r] = prod[1][r] = 0.0f;
+    }
+    auto fold_pair = [&](int q, int first, int count) {                      // elements first .. of the pair's 32
+        const int set = q & 1;
+#pragma unroll
+        for (int e = first; e < first + count; ++e) {
+            const int j = e / 16, r = e % 16;
+            total[q % TN][j][r] = fmaf(acc[2 * set + j][r], prod[set][e], total[q % TN][j][r]);
+        }
+    };
+    auto math = [&] {
+        __builtin_amdgcn_s_setprio(1);
+        if constexpr (!ROWS) {
+#pragma unroll
+            for (int u = 0; u < UNITS; ++u) {
+                const int kg = u / (TN * TM), i = u / TM % TN, j = u % TM, x = u % ACCS;
+                acc[x] = product(kg, i, j, 0, zero);
+                if (u >= LAG) fold_unit(u - LAG, 0, 8);
+                __builtin_amdgcn_sched_barrier(0);
+                acc[x] = product(kg, i, j, 1, acc[x]);
+                if (u >= LAG) fold_unit(u - LAG, 8, 8);
+                __builtin_amdgcn_sched_barrier(0);
+                scale[x] = sa[j][kg] * sb[i][kg];
+            }
+#pragma unroll
+            for (int u = UNITS - LAG; u < UNITS; ++u) asm volatile("" : "+v"(acc[u % ACCS]), "+v"(scale[u % ACCS]));
+        } else {
+            static_assert(!ROWS || (TM == 2 && PAIRS % 2 == 0));
+            const f32x32 zero32 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int q = 0; q < PAIRS; ++q) {
+                const int kg = q / TN, i = q % TN, set = q & 1, before = (q + PAIRS - 1) % PAIRS;
+                prod[set] = __builtin_amdgcn_mfma_f32_32x32x1f32(sb[i][kg], sa[0][kg], zero32, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                fold_pair(before, 0, 8);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const int j = x & 1;
+                    acc[2 * set + j] = product(kg, i, j, x / 2, x < 2 ? zero : acc[2 * set + j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fold_pair(before, 8 + x * 6, 6);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                asm volatile("" : "+v"(total[before % TN][0]), "+v"(total[before % TN][1]));
+            }
+            asm volatile("" : "+v"(acc[2]), "+v"(acc[3]), "+v"(prod[ROWS ? 1 : 0]));
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+    auto drain = [&] {                                                       // the units of the last chunk that are not folded yet
+        if constexpr (!ROWS) {
+#pragma unroll
+            for (int u = UNITS - LAG; u < UNITS; ++u) fold_unit(u, 0, 16);
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(total[i][j]));
+        } else {
+            fold_pair(PAIRS - 1, 0, 32);
+        }
+    };
+    auto barrier = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // ---- phases, stages and waits: as in gemm_pingpong. Scale block b + 1 is fetched in the read phase of chunk 4 b, into the
+    // buffer that block b - 1 left a chunk ago (its last readers, waves 4-7, had it in registers before the barrier that ended
+    // their read phase); it has landed when the read phase of chunk 4 b + 1 ends and is first read in chunk 4 b + 4, with the
+    // straddling piece cleared in chunk 4 b + 2.
+    constexpr int AHEAD = (STAGES - 2) * S::LOADS;
+    static_assert(AHEAD + 1 < 16 && STAGES >= 3);
+    issue_scales(0);
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);                              // chunk 0 and scale block 0
+    barrier();
+    if (last_block == 0 && straddles) {
+        clear_past_the_end();
+        __syncthreads();
+    }
+    const bool late = wave >= 4;
+    if (late) barrier();
+    int stage = 0, fill = STAGES - 1;
+    for (int c = 0; c < chunks; ++c) {
+        read(stage, c);
+        const bool scales_now = c % F_SCHUNKS == 0;
+        if (scales_now) issue_scales(c / F_SCHUNKS + 1);
+        if (c % F_SCHUNKS == 2 && c / F_SCHUNKS + 1 == last_block && straddles) clear_past_the_end();
+        issue(c + STAGES - 1, fill);
+        stage = stage == STAGES - 1 ? 0 : stage + 1;
+        fill = fill == STAGES - 1 ? 0 : fill + 1;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!ROWS) {
+            drain();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (scales_now) __builtin_amdgcn_s_waitcnt(0x0070 | (AHEAD + 1));   // (the scale block just issued is among the newest)
+        else __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
+        pin_operands();
+        barrier();
+        math();
+        barrier();
+    }
+    if (!late) barrier();
+    drain();
+    __builtin_amdgcn_s_waitcnt(0x0F70);                                      // the trailing loads must not land in what follows
+    barrier();
+    float* bias_lds = reinterpret_cast<float*>(lds + RING);
+    stage_bias<S>(p, n_begin, bias_lds, bias_dtype);
+    auto finish = [&](auto type) {
+        using TO = decltype(type);
+        store_tile<S, TN, true>(total, p, static_cast<TO*>(p.out) + out_shift, m_begin, m_end, n_begin, lds, bias_lds);
+    };
+    if (out_dtype == VIOLA_F32) finish(float{});
+    else if (out_dtype == VIOLA_BF16) finish(bf16_t{});
+    else finish(f16_t{});
+}
+
+}  // namespace viola

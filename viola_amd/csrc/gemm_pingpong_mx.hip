@@ -1,6 +1,4 @@
 // E8M0 block-scale (MXFP8) instances of the large-tile FP8 GEMM kernel.
-#include <type_traits>
-
 #include "gemm_pingpong.hpp"
 
 namespace viola {

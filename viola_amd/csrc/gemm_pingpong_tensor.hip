@@ -1,6 +1,4 @@
 // Per-tensor-scale instances of the large-tile FP8 GEMM kernel.
-#include <type_traits>
-
 #include "gemm_pingpong.hpp"
 
 namespace viola {
