@@ -216,6 +216,14 @@ int viola_group_gemm(const void* a, int a_dtype, const void* b, int b_dtype, con
                      int64_t m, int64_t n, int64_t k, int ar, int ak, int br, int bk,
                      const void* bias, int bias_dtype, void* out, int out_dtype, viola_stream_t stream);
 
+/* The same with a scale per row and 32 k on both sides (ar = br = 1, ak = bk = 32), no bias, the k range cut into `parts` (2 .. 64)
+ * that are computed side by side: their FP32 products go to workspace (parts * (m * n rounded up to 4) floats, 16-byte aligned) and
+ * are added in ascending order. viola_group_gemm_parts says how many are worth it (1: viola_group_gemm). VIOLA_EUNSUPPORTED, with
+ * nothing launched, where k % 16 != 0, the operands are not 16-byte aligned or beyond 2 GiB. */
+int viola_group_gemm_parts(int64_t m, int64_t n, int64_t k);
+int viola_group_gemm_in_parts(const void* a, int a_dtype, const void* b, int b_dtype, const float* sa, const float* sb, int64_t m, int64_t n,
+                              int64_t k, void* out, int out_dtype, int parts, float* workspace, int64_t workspace_floats, viola_stream_t stream);
+
 /* viola_group_gemm under accum_dtype="fp16" (viola/nn/_grouped_kernels.py:268-292, :310-318): the raw products of
  * gcd(ak, bk, accum_block) k (accum_block 0: gcd(ak, bk)) meet in an FP16 partial, fp16(partial + 32 products) per
  * 32 k, which is then scaled, (partial * sa) * sb, added to a total kept in reduce_dtype (VIOLA_F32 or VIOLA_BF16,

@@ -96,3 +96,40 @@ def test_varlen_weight_gradient_on_large_tiles():
     for g, length in enumerate(slots):
         assert torch.equal(out[g], a[:, start:start + length] @ b[:, start:start + length].T)
         start += length
+
+
+@pytest.mark.parametrize("m,n,k,parts,out_dtype", [(3072, 768, 9856, 3, torch.bfloat16), (512, 516, 2080, 8, torch.float32), (200, 100, 1040, 64, torch.float16),
+                                                   (257, 333, 4112, 5, torch.bfloat16), (1024, 1024, 192, 2, torch.float32), (64, 40, 16, 2, torch.float32)])
+def test_product_in_parts_of_k(m, n, k, parts, out_dtype):
+    """The k range cut into parts: parts that end inside a chunk and inside a block of scales, fewer chunks than parts, rows of the
+    partial products that are not whole pieces, tiles that do not divide over the XCDs."""
+    torch.manual_seed(m + n + k)
+    a, b, groups = _integers(m, k), _integers(n, k), -(-k // 32)
+    sa, sb = _scales(m, groups), _scales(n, groups)
+    out, qa, qb = torch.full((m, n), 7.0, device="cuda", dtype=out_dtype), a.to(E4), b.to(E5)
+    floats = parts * (-(-m * n // 4) * 4)
+    workspace = torch.full((floats + 64,), float("nan"), device="cuda")
+    args = lambda size: (qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E5), sa.data_ptr(), sb.data_ptr(), m, n, k, out.data_ptr(), _lib.code(out_dtype), parts,
+                         workspace.data_ptr(), size)
+    with pytest.raises(RuntimeError):
+        _lib.call("viola_group_gemm_in_parts", *args(floats - 1))
+    assert (out == 7.0).all()
+    _lib.call("viola_group_gemm_in_parts", *args(floats))
+    assert torch.equal(out, (_spell(a, sa, 1) @ _spell(b, sb, 1).T).to(out_dtype)) and torch.isnan(workspace[floats:]).all()
+
+
+def test_linear_weight_gradient_in_parts_against_float64():
+    """A shape the module runs in parts: no further from the float64 product of the very codes than the whole product is."""
+    from viola_amd.nn import _grouped_kernels as g
+    torch.manual_seed(1)
+    m, n, k = 768, 512, 8192
+    parts = _lib.library().viola_group_gemm_parts(m, n, k)
+    assert parts > 1
+    (qa, sa), (qb, sb) = (g.quantize(torch.randn(r, k, device="cuda").bfloat16(), E4, (1, 32)) for r in (m, n))
+    out, workspace = torch.empty(m, n, device="cuda"), torch.empty(parts * m * n, device="cuda")
+    _lib.call("viola_group_gemm_in_parts", qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E4), sa.data_ptr(), sb.data_ptr(), m, n, k, out.data_ptr(), 0, parts,
+              workspace.data_ptr(), workspace.numel())
+    whole = g.gemm(qa, qb, sa, sb, (1, 32), (1, 32), out_dtype=torch.float32)
+    exact = (qa.float() * sa.repeat_interleave(32, 1)).double() @ (qb.float() * sb.repeat_interleave(32, 1)).double().T
+    error = lambda t: ((t - exact).norm() / exact.norm()).item()
+    assert error(out) <= 1.05 * error(whole)

@@ -37,6 +37,7 @@ _SIGNATURES = {
     "viola_block_transpose": [_p, _p, _l, _l, _p, _p, _i, _i, _i, _p],
     "viola_skinny_linear": [_p, _i, _p, _l, _l, _p, _i, _p, _i, _l, _f, _i, _p, _l, _p, _p, _i, _p, _i, _p],
     "viola_group_gemm": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _i, _i, _i, _i, _p, _i, _p, _i, _p],
+    "viola_group_gemm_in_parts": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _p, _i, _i, _p, _l, _p],
     "viola_group_gemm_half": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _i, _i, _i, _i, _p, _i, _p, _i, _i, _i, _p],
     "viola_tensor_gemm_half": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _p, _i, _p, _i, _i, _i, _p],
     "viola_gated_gemm": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _i, _i, _i, _i, _p, _i, _p, _p, _i, _i, _i, _p],
@@ -79,7 +80,7 @@ _SIGNATURES = {
     "viola_selftest_fp8": [_p, _p],
     "viola_selftest_philox": [_p, _p, _l, _p],
 }
-EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan", "viola_tensor_encode_slices")
+EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan", "viola_tensor_encode_slices", "viola_group_gemm_parts")
 
 _lib = None
 
@@ -98,6 +99,7 @@ def library():
         lib.viola_abi_version.restype = ctypes.c_int
         lib.viola_error_string.argtypes, lib.viola_error_string.restype = [ctypes.c_int], ctypes.c_char_p
         lib.viola_tensor_encode_slices.argtypes, lib.viola_tensor_encode_slices.restype = [_i, _l, _l], ctypes.c_int64
+        lib.viola_group_gemm_parts.argtypes, lib.viola_group_gemm_parts.restype = [_l, _l, _l], ctypes.c_int
         lib.viola_ns_plan.argtypes, lib.viola_ns_plan.restype = [_l, _l, _l, _l, _i, _i, _i, ctypes.POINTER(ctypes.c_int)], ctypes.c_int
         assert lib.viola_abi_version() == 1
         _lib = lib

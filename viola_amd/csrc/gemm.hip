@@ -50,6 +50,36 @@ extern "C" int viola_group_gemm(const void* a, int a_dtype, const void* b, int b
     return launch_out<MODE_PLAIN>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, vec, dim3((unsigned)gx, (unsigned)gy), stream);
 }
 
+// (what the fast kernel asks of a product with a scale per row and 32 k on both sides, plus what 256 rows of a large tile do)
+static bool parts_take(const void* a, const void* b, int64_t m, int64_t n, int64_t k) {
+    const int64_t rows = m > n ? m : n;
+    return k % 16 == 0 && aligned16(a) && aligned16(b) && rows * k < (1ll << 31) && 256 * k < (1ll << 31) && rows * ((k + 31) / 32) * 4 < (1ll << 31) &&
+           m * n < (1ll << 31);
+}
+
+extern "C" int viola_group_gemm_parts(int64_t m, int64_t n, int64_t k) {
+    if (m <= 0 || n <= 0 || k <= 0 || m * n >= (1ll << 31)) return 1;
+    return plan_k_parts(m, n, k);
+}
+
+extern "C" int viola_group_gemm_in_parts(const void* a, int a_dtype, const void* b, int b_dtype, const float* sa, const float* sb, int64_t m, int64_t n,
+                                         int64_t k, void* out, int out_dtype, int parts, float* workspace, int64_t workspace_floats, viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG(viola_is_fp8(a_dtype) && viola_is_fp8(b_dtype) && viola_is_float(out_dtype));
+    VIOLA_CHECK_ARG(m >= 0 && n >= 0 && k > 0 && parts >= 2 && parts <= 64 && workspace && aligned16(workspace));
+    if (m == 0 || n == 0) return 0;
+    VIOLA_CHECK_ARG(a && b && sa && sb && out);
+    if (!parts_take(a, b, m, n, k)) return VIOLA_EUNSUPPORTED;
+    VIOLA_CHECK_ARG(workspace_floats >= parts * ((m * n + 3) / 4 * 4));
+    GemmArgs p = {};
+    p.a = static_cast<const uint8_t*>(a); p.b = static_cast<const uint8_t*>(b); p.sa = sa; p.sb = sb;
+    p.out = out; p.m = m; p.n = n; p.k = k; p.lda = k; p.ldb = k;
+    p.ldsa = (k + 31) / 32; p.ldsb = (k + 31) / 32; p.ldo = n;
+    p.sa_bytes = m * p.ldsa * 4; p.sb_bytes = n * p.ldsb * 4;
+    p.ar = 1; p.br = 1; p.ak_shift = 5; p.bk_shift = 5;
+    return launch_group_parts(p, parts, a_dtype, b_dtype, out_dtype, workspace, stream);
+}
+
 static int gcd_of(int a, int b) { while (b) { const int t = a % b; a = b; b = t; } return a; }
 
 extern "C" int viola_group_gemm_half(const void* a, int a_dtype, const void* b, int b_dtype, const float* sa, const float* sb,

@@ -22,6 +22,8 @@ struct GemmArgs {
     const int64_t* offsets; int groups; int64_t b_group_stride, sb_group_stride;
     // variable-group K ranges (grid.z = group): k range [koffsets[g], koffsets[g+1])
     const int64_t* koffsets; int64_t out_group_stride;
+    // the same with `parts` equal ranges of k_split (0: none; large tiles only), the parts' tiles one after the other in grid.x
+    int64_t k_split; int parts;
     // fast kernel only: 1-D grid of tiles_m * tiles_n output tiles (rounded up to a multiple of 8) walked in an
     // XCD-aware order; tiles_m == 0 keeps the plain (blockIdx.x, blockIdx.y) = (n tile, m tile) mapping
     int tiles_m, tiles_n;
@@ -52,6 +54,11 @@ int launch_group_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype
 // them), groups: k ranges. gemm_pingpong_grouped.hip.
 int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, unsigned groups,
                           hipStream_t stream);
+
+// How many parts of k a row-wise scaled product is computed in (1: whole), and the product in that many: FP32 partial products
+// [parts][m * n rounded up to 4] in workspace, then their sum in ascending order. gemm_fast.hip, gemm_pingpong_grouped.hip.
+int plan_k_parts(int64_t m, int64_t n, int64_t k);
+int launch_group_parts(const GemmArgs& p, int parts, int a_dtype, int b_dtype, int out_dtype, float* workspace, hipStream_t stream);
 
 // Per-tensor scales on the same fast kernel (one v_mfma_f32_32x32x64_f8f6f4 per sub-tile and 64 k); mode = MODE_PLAIN or a
 // gated mode (grid.x then counts the gated tile width). Defined in gemm_fast.hip.

@@ -78,6 +78,33 @@ static bool prefer_pingpong(const GemmArgs& p, bool rowscale, unsigned k_groups)
     return rounds * (chunks * busy + ends) + (rest > 0 ? chunks * (idle + (busy - idle) * rest) + ends : 0.0) < now;
 }
 
+// In how many parts of k a weight gradient runs, which has few tiles and a long k. Whole, 129 to 256 tiles of 128 x 128 leave CUs
+// without a tile, and fewer run as narrow tiles on a 16th of the data reuse; in parts, tiles of 256 x 128 fill the chip and a second
+// launch adds the partial products. The least of the estimates in microseconds (fitted to 24 shapes) decides, and only where it
+// saves a twentieth: 3072 x 768 x 9856 100 -> 65 us in three, 1024 x 1024 x 16384 90 -> 49 in eight, 1536 x 1536 x 8192 79 -> 56 in three,
+// 512 x 512 x 16384 89 -> 28 in 24; 4096 x 1024 x 8192 stays whole (88 us, 83 in two), so does 1024 x 1024 x 4096 (26.6 us, 28.0 in seven).
+int plan_k_parts(int64_t m, int64_t n, int64_t k) {
+    constexpr double CUS = 256.0;
+    if (k < 1024 || m < 64 || n < 64 || n % 4 != 0) return 1;               // (rows of the partial products in whole 16-byte pieces)
+    const double chunks = (double)k / 64.0, small = (double)((m + 127) / 128) * (double)((n + 127) / 128), large = (double)((m + 255) / 256) * (double)((n + 127) / 128);
+    // whole, as launch_group_gemm_fast runs it
+    const double pairs = floor(small / (2 * CUS)), left = small - pairs * 2 * CUS;
+    double least = small <= CUS / 2 ? chunks * (0.33 + 0.09 * small / 128.0) + 3.3 : small <= CUS ? chunks * 0.64 + 4.0
+                   : pairs * (chunks * 1.2 + 3.3) + (left > 0 ? chunks * 1.2 * (left <= CUS ? 0.52 : 1.0) + 3.3 : 0.0);
+    auto tiles_of = [&](double count, double length, double ends) {
+        const double rounds = floor(count / CUS), rest = count / CUS - rounds;
+        return rounds * (length * 1.04 + ends) + (rest > 0 ? length * (0.82 + 0.22 * rest) + ends : 0.0);
+    };
+    if (small > CUS) least = least < tiles_of(large, chunks, 6.0) ? least : tiles_of(large, chunks, 6.0);
+    int best = 1;
+    for (int parts = 2; parts <= 64 && chunks / parts >= 4.0; ++parts) {
+        const double sum = 5.0 + (double)m * n * (4.0 * parts + 2.0) / 4.3e6;
+        const double time = tiles_of(large * parts, ceil(chunks / parts), 7.5) + sum;
+        if (time < 0.95 * least) { least = time / 0.95; best = parts; }
+    }
+    return best;
+}
+
 int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale,
                            dim3 grid, hipStream_t stream) {
     GemmArgs p = args;

@@ -67,8 +67,9 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
         }
     }
     const int per_xcd = p.offsets ? (int)(((int64_t)tiles_m * p.tiles_n + 7) / 8) : (int)(gridDim.x / 8);
-    const int seq = blockIdx.x / 8, t = (blockIdx.x % 8) * per_xcd + seq;
-    if (seq >= per_xcd || t >= tiles_m * p.tiles_n) return;
+    const int seq = blockIdx.x / 8, place = (blockIdx.x % 8) * per_xcd + seq, tiles = tiles_m * p.tiles_n;
+    const int part = p.k_split ? place / tiles : 0, t = place - part * tiles;
+    if (seq >= per_xcd || (p.k_split ? part >= p.parts : t >= tiles)) return;
     const int walk = WALK * p.tiles_n, first_m = t / walk * WALK;
     const int rows_here = tiles_m - first_m < WALK ? tiles_m - first_m : WALK;
     const int tile_m = first_m + t % walk % rows_here;
@@ -99,6 +100,11 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
         k_begin = p.koffsets[blockIdx.z];
         k_end = p.koffsets[blockIdx.z + 1];
         out_shift = (int64_t)blockIdx.z * p.out_group_stride;
+    }
+    if (p.k_split) {
+        k_begin = part * p.k_split;
+        k_end = k_begin + p.k_split < p.k ? k_begin + p.k_split : p.k;
+        out_shift = part * p.out_group_stride;
     }
     const int64_t k_len = k_end - k_begin;
 

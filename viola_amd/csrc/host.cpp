@@ -556,9 +556,14 @@ Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const T
     const int64_t w_q = requantize ? temp.take(r.out * r.in) : -1;
     const int64_t w_s = requantize && r.grouped ? temp.take(ceil_div(r.out, 32) * ceil_div(r.in, 32) * r.scale_bytes()) : -1;
     if (needs_b) out.db = at::empty({r.out}, dx_options.dtype(kept.bias_grad));
+    int k_parts = 1;                                             // of the weight gradient's k range, and the partial products
+    int64_t k_parts_at = -1;
     if (r.grouped) {
         GroupSpace space;
         space.reserve(r, needs_x ? &temp : nullptr, needs_w ? &temp : nullptr, rows, r.out, pitch);
+        const int64_t size = r.out * r.in;
+        if (needs_w && !r.native) k_parts = viola_group_gemm_parts(r.out, r.in, space.pitch_t);
+        if (k_parts > 1) k_parts_at = temp.take(k_parts * ceil_to(size, 4) * 4);
         const bool rides = needs_b && needs_w;                   // the bias gradient's 32-row sums come from the quantizer's read of dy
         const int64_t partial_at = rides ? temp.take(parts * r.out * 4) : -1;
         temp.make(device);
@@ -630,7 +635,15 @@ Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const T
     }
     if (needs_w) {
         out.dw = at::empty({r.out, r.in}, dx_options.dtype(kept.weight_grad));
-        product(r, gt, r.bwd, t.input_t, r.fwd, r.out, r.in, 1, Tensor(), out.dw.mutable_data_ptr(), kept.weight_grad, device, stream);
+        int status = VIOLA_EUNSUPPORTED;
+        if (k_parts > 1) {
+            TORCH_INTERNAL_ASSERT(gt.pitch == t.input_t.pitch);
+            status = VIOLA_TRY(viola_group_gemm_in_parts, gt.q, r.bwd, t.input_t.q, r.fwd, static_cast<const float*>(gt.s), static_cast<const float*>(t.input_t.s),
+                               r.out, r.in, gt.pitch, out.dw.mutable_data_ptr(), code_of(kept.weight_grad), k_parts, temp.as<float>(k_parts_at),
+                               k_parts * ceil_to(r.out * r.in, 4), stream);
+            if (status != VIOLA_EUNSUPPORTED) check("viola_group_gemm_in_parts", status);
+        }
+        if (status != 0) product(r, gt, r.bwd, t.input_t, r.fwd, r.out, r.in, 1, Tensor(), out.dw.mutable_data_ptr(), kept.weight_grad, device, stream);
     }
     return out;
 }
