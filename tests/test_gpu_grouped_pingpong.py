@@ -98,6 +98,23 @@ def test_varlen_weight_gradient_on_large_tiles():
         start += length
 
 
+@pytest.mark.parametrize("m,n,k,out_dtype", [(4096, 1024, 8192, torch.bfloat16), (2000, 1028, 1536, torch.float32), (1921, 2047, 1552, torch.float16),
+                                             (1500, 1535, 1568, torch.bfloat16), (1536, 1536, 1808, torch.float32), (1536, 1536, 2064, torch.float32)])
+def test_row_scaled_products_whose_teams_share_the_k_range(m, n, k, out_dtype):
+    """129 to 256 tiles of 128 x 128: the teams' ranges of equal and different length, the second ending inside a block of scales (with
+    the next row's scale, a NaN, in the piece that holds its last ones), ragged rows and columns."""
+    from viola_amd.nn import _grouped_kernels as g
+    torch.manual_seed(m + n + k)
+    a, b, groups = _integers(m, k), _integers(n, k), -(-k // 32)
+    sa, sb = _scales(m, groups), _scales(n, groups)
+    bias = torch.randint(-8, 9, (n,), device="cuda").float()
+    want = _spell(a, sa, 1) @ _spell(b, sb, 1).T + bias
+    sa[7, 0], sb[n - 1, 0] = float("nan"), float("inf")
+    out = g.gemm(a.to(E4), b.to(E5), sa, sb, (1, 32), (1, 32), out_dtype=out_dtype, bias=bias)
+    rows = torch.arange(m, device="cuda") != 7
+    assert torch.equal(out[rows, :n - 1], want[rows, :n - 1].to(out_dtype)) and torch.isnan(out[7]).all()
+
+
 @pytest.mark.parametrize("m,n,k,parts,out_dtype", [(3072, 768, 9856, 3, torch.bfloat16), (512, 516, 2080, 8, torch.float32), (200, 100, 1040, 64, torch.float16),
                                                    (257, 333, 4112, 5, torch.bfloat16), (1024, 1024, 192, 2, torch.float32), (64, 40, 16, 2, torch.float32)])
 def test_product_in_parts_of_k(m, n, k, parts, out_dtype):

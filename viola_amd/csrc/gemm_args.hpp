@@ -55,6 +55,9 @@ int launch_group_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype
 int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, unsigned groups,
                           hipStream_t stream);
 
+// Row-wise b scales on tiles of 128 x 128, the k range split over two teams of waves that take turns. gemm_pingpong_grouped.hip.
+int launch_group_teams(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream);
+
 // How many parts of k a row-wise scaled product is computed in (1: whole), and the product in that many: FP32 partial products
 // [parts][m * n rounded up to 4] in workspace, then their sum in ascending order. gemm_fast.hip, gemm_pingpong_grouped.hip.
 int plan_k_parts(int64_t m, int64_t n, int64_t k);

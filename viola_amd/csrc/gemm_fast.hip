@@ -17,19 +17,14 @@ static void launch_formats(const GemmArgs& p, int a_dtype, int b_dtype, int bias
 }
 
 // plain mode, the k range of a tile split over two teams of waves
-template <int TN>
-static int launch_split(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, dim3 grid,
-                        hipStream_t stream) {
-#define VIOLA_SPLIT(TO)                                                                                         \
-    if (rowscale) launch_formats<MODE_PLAIN, true, TO, TN, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream); \
-    else launch_formats<MODE_PLAIN, false, TO, TN, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream);
+template <int TN, bool ROWSCALE>
+static int launch_split(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, dim3 grid, hipStream_t stream) {
     switch (out_dtype) {
-        case VIOLA_F32: VIOLA_SPLIT(float) break;
-        case VIOLA_BF16: VIOLA_SPLIT(bf16_t) break;
-        case VIOLA_F16: VIOLA_SPLIT(f16_t) break;
+        case VIOLA_F32: launch_formats<MODE_PLAIN, ROWSCALE, float, TN, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream); break;
+        case VIOLA_BF16: launch_formats<MODE_PLAIN, ROWSCALE, bf16_t, TN, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream); break;
+        case VIOLA_F16: launch_formats<MODE_PLAIN, ROWSCALE, f16_t, TN, true>(p, a_dtype, b_dtype, bias_dtype, grid, stream); break;
         default: return VIOLA_EINVAL;
     }
-#undef VIOLA_SPLIT
     return viola_launch_status();
 }
 
@@ -79,17 +74,17 @@ static bool prefer_pingpong(const GemmArgs& p, bool rowscale, unsigned k_groups)
 }
 
 // In how many parts of k a weight gradient runs, which has few tiles and a long k. Whole, 129 to 256 tiles of 128 x 128 leave CUs
-// without a tile, and fewer run as narrow tiles on a 16th of the data reuse; in parts, tiles of 256 x 128 fill the chip and a second
+// without a tile, and fewer run as narrow tiles, which read more per product; in parts, tiles of 256 x 128 fill the chip and a second
 // launch adds the partial products. The least of the estimates in microseconds (fitted to 24 shapes) decides, and only where it
-// saves a twentieth: 3072 x 768 x 9856 100 -> 65 us in three, 1024 x 1024 x 16384 90 -> 49 in eight, 1536 x 1536 x 8192 79 -> 56 in three,
-// 512 x 512 x 16384 89 -> 28 in 24; 4096 x 1024 x 8192 stays whole (88 us, 83 in two), so does 1024 x 1024 x 4096 (26.6 us, 28.0 in seven).
+// saves a twentieth: 3072 x 768 x 9856 82 -> 65 us in three, 1024 x 1024 x 16384 90 -> 49 in eight, 2048 x 1024 x 8192 56 -> 50 in four,
+// 512 x 512 x 16384 89 -> 28 in 24; 4096 x 1024 x 8192 stays whole (74 us, 83 in two), so does 1024 x 1024 x 4096 (26.6 us, 28.0 in seven).
 int plan_k_parts(int64_t m, int64_t n, int64_t k) {
     constexpr double CUS = 256.0;
     if (k < 1024 || m < 64 || n < 64 || n % 4 != 0) return 1;               // (rows of the partial products in whole 16-byte pieces)
     const double chunks = (double)k / 64.0, small = (double)((m + 127) / 128) * (double)((n + 127) / 128), large = (double)((m + 255) / 256) * (double)((n + 127) / 128);
     // whole, as launch_group_gemm_fast runs it
     const double pairs = floor(small / (2 * CUS)), left = small - pairs * 2 * CUS;
-    double least = small <= CUS / 2 ? chunks * (0.33 + 0.09 * small / 128.0) + 3.3 : small <= CUS ? chunks * 0.64 + 4.0
+    double least = small <= CUS / 2 ? chunks * (0.33 + 0.09 * small / 128.0) + 3.3 : small <= CUS ? chunks * (0.45 + 0.1 * small / CUS) + 4.0
                    : pairs * (chunks * 1.2 + 3.3) + (left > 0 ? chunks * 1.2 * (left <= CUS ? 0.52 : 1.0) + 3.3 : 0.0);
     auto tiles_of = [&](double count, double length, double ends) {
         const double rounds = floor(count / CUS), rest = count / CUS - rounds;
@@ -126,6 +121,9 @@ int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dt
     const bool few = mode == MODE_PLAIN && tiles <= 256;
     const bool fixed_k = !p.offsets && !p.koffsets;
     const bool split = few && tiles > 128 && fixed_k && p.k >= SPLIT_MIN_K;
+    // ... with row-wise b scales the teams take turns (4096 x 1024 x 8192 86 -> 74 us, 1536 x 1536 x 4096 43 -> 35; with uniform ones they do
+    // not gain by it, 68 against 77)
+    if (split && rowscale) return launch_group_teams(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
     const bool narrow = few && !split && p.n > 64;
     if (narrow) grid.x = (unsigned)((p.n + 63) / 64);
     if ((int64_t)grid.x * grid.y < (1 << 30)) {
@@ -133,8 +131,10 @@ int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dt
         p.tiles_m = (int)grid.y;
         grid = dim3((grid.x * grid.y + 7) / 8 * 8, 1, grid.z);
     }
-    if (split) return launch_split<2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
-    if (narrow && tiles <= 128 && fixed_k && p.k >= NARROW_SPLIT_MIN_K) return launch_split<1>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
+    if (split) return launch_split<2, false>(p, a_dtype, b_dtype, bias_dtype, out_dtype, grid, stream);
+    if (narrow && tiles <= 128 && fixed_k && p.k >= NARROW_SPLIT_MIN_K)
+        return rowscale ? launch_split<1, true>(p, a_dtype, b_dtype, bias_dtype, out_dtype, grid, stream)
+                        : launch_split<1, false>(p, a_dtype, b_dtype, bias_dtype, out_dtype, grid, stream);
     if (narrow) return launch_mode<MODE_PLAIN, 1>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
     if (mode == MODE_PLAIN) return launch_mode<MODE_PLAIN, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
     if (mode == MODE_GATED_FWD) return launch_mode<MODE_GATED_FWD, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);

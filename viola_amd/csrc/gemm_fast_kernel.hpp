@@ -125,15 +125,15 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // group 1), so lane (row, half) hands over the scale byte of K group `half` of its row. Scales travel in blocks of 16
 // K groups (one 16-byte piece per tile row and operand), double-buffered behind the ring; k must be a multiple of 128.
 constexpr int MX_GROUPS = 16, MX_CHUNKS = MX_GROUPS / FKG, MX_BLOCK = 2 * BM * MX_GROUPS;   // bytes of one block, a then b
-// KSPLIT (plain mode): for products with few tiles and a long k, such as a weight gradient (the launchers say how few: up to 256
-// tiles of 128 x 128 under grouped scales, fewer than 128 with tiles of 128 x 64 under the others). A block of 512 threads is two
+// KSPLIT (plain mode): for products with few tiles and a long k (the launchers say how few: up to 256 tiles of 128 x 128 under
+// grouped scales, with row-wise b scales and otherwise fewer than 128, with tiles of 128 x 64). A block of 512 threads is two
 // teams of 2 x 2 waves, each with a stage ring and scale buffers of its own, that compute the same tile over the two halves of the
 // k range (cut at a multiple of 256 k, one scale block); at the end team 1 hands its totals over in LDS and team 0 adds them to
 // its own (always in that order) and stores the tile. A CU with one block then holds eight waves; at 128 x 128 a wave also has the
 // 2 x 2 sub-tiles' better ratio of MFMAs to global loads and LDS reads.
 template <int MODE, bool A_BF8, bool B_BF8, bool B_ROWSCALE, typename TO, int TN, bool TENSOR = false, bool MX = false, bool KSPLIT = false>
 __global__ __launch_bounds__(KSPLIT ? 512 : FTHREADS, KSPLIT ? 1 : TENSOR ? 3 : 2) void group_gemm_fast(GemmArgs p, int bias_dtype) {
-    static_assert(!KSPLIT || (MODE == MODE_PLAIN && (TN == 1 || !(TENSOR || MX))), "the split exists for plain products, at 128 x 128 under grouped scales only");
+    static_assert(!KSPLIT || (MODE == MODE_PLAIN && (TN == 1 || !(TENSOR || MX || B_ROWSCALE))), "the split exists for plain products, at 128 x 128 under uniform grouped b scales only");
     static_assert(!TENSOR || !B_ROWSCALE, "per-tensor scaling has no row scales");
     static_assert(!MX || !TENSOR, "one scaling recipe per kernel");
     constexpr bool NOFOLD = TENSOR || MX;                                   // the products of a chunk go straight into the totals

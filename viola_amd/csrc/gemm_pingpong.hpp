@@ -18,10 +18,12 @@ namespace viola {
 template <int WM_, int WN_, int TM_, int TN_, int STAGES_>
 struct PingPongShape {
     static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, STAGES = STAGES_;
+    static constexpr int TEAMS = 8 / (WM * WN), THREADS = 512 / TEAMS;       // two teams of four waves: gemm_pingpong_grouped.hpp
     static constexpr int ROWS = WM * TM * 32, COLS = WN * TN * 32;
     static constexpr int A_BYTES = ROWS * FBK, B_BYTES = COLS * FBK, STAGE = A_BYTES + B_BYTES;
-    static constexpr int A_LOADS = ROWS / 128, B_LOADS = COLS / 128, LOADS = A_LOADS + B_LOADS;   // 512 threads x 16 bytes = 128 rows
-    static_assert(WM * WN == 8 && ROWS % 128 == 0 && COLS % 128 == 0);
+    static constexpr int LOAD_ROWS = THREADS / 4;                            // a load instruction of all threads: 16 bytes each
+    static constexpr int A_LOADS = ROWS / LOAD_ROWS, B_LOADS = COLS / LOAD_ROWS, LOADS = A_LOADS + B_LOADS;
+    static_assert(WM * WN * TEAMS == 8 && ROWS % LOAD_ROWS == 0 && COLS % LOAD_ROWS == 0);
 };
 
 // Epilogue. The tile's bias as fp32 in LDS (COLS floats), -0 where there is none: adding that changes nothing, not even a sign.
@@ -43,15 +45,16 @@ template <typename S, int SUBS, bool BIAS, typename TO>
 __device__ __forceinline__ void store_tile(const f32x16 (&total)[S::TN][S::TM], const GemmArgs& p, TO* out, int64_t m_begin, int64_t m_end,
                                            int64_t n_begin, uint8_t* ring, const float* bias_lds) {
     const int lane = threadIdx.x % WAVE, l32 = lane % 32, lhi = lane / 32;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE), wm = wave / S::WN, wn = wave % S::WN;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE), wm = wave % (S::WM * S::WN) / S::WN, wn = wave % S::WN;
     const bool pieces_out = (p.ldo * sizeof(TO)) % 16 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     constexpr int PER = 16 / (int)sizeof(TO), COLS_W = 32 * SUBS, PLD = COLS_W + PER, PIECES = COLS_W / PER;
-    static_assert(8 * 32 * PLD * (int)sizeof(TO) <= S::STAGES * S::STAGE);
+    static_assert(8 * 32 * PLD * (int)sizeof(TO) <= S::TEAMS * S::STAGES * S::STAGE);
     TO* park = reinterpret_cast<TO*>(ring) + wave * 32 * PLD;
     const int64_t ncol0 = n_begin + wn * COLS_W;
 #pragma unroll
-    for (int j = 0; j < S::TM; ++j) {
-        const int64_t row0 = m_begin + (wm * S::TM + j) * 32;
+    for (int j = 0; j < (S::TEAMS > 1 ? 1 : S::TM); ++j) {
+        // (two teams: either stores one row of sub-tiles, team t the t-th, which it holds in the first one's place)
+        const int64_t row0 = m_begin + (wm * S::TM + j + wave / (S::WM * S::WN)) * 32;
 #pragma unroll
         for (int i = 0; i < SUBS; ++i)
 #pragma unroll

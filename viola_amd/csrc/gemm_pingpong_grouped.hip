@@ -3,19 +3,18 @@
 
 namespace viola {
 
-template <bool ROWS>
+template <typename S, bool ROWS>
 static int launch(const GemmArgs& args, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, unsigned groups, hipStream_t stream) {
-    using S = std::conditional_t<ROWS, GroupedRows, GroupedWide>;
     GemmArgs p = args;
     p.tiles_m = row_tiles;
     p.tiles_n = (int)((p.n + S::COLS - 1) / S::COLS);
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * (p.k_split ? p.parts : 1);
     const dim3 grid((unsigned)((blocks + 7) / 8 * 8), 1, groups), block(512);
     const bool a5 = a_dtype == VIOLA_E5M2, b5 = b_dtype == VIOLA_E5M2;
-    if (!a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_grouped<false, false, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
-    else if (a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_grouped<true, false, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
-    else if (!a5 && b5) VIOLA_LAUNCH((gemm_pingpong_grouped<false, true, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
-    else VIOLA_LAUNCH((gemm_pingpong_grouped<true, true, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    if (!a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_grouped<false, false, S, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else if (a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_grouped<true, false, S, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else if (!a5 && b5) VIOLA_LAUNCH((gemm_pingpong_grouped<false, true, S, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else VIOLA_LAUNCH((gemm_pingpong_grouped<true, true, S, ROWS>), grid, block, 0, stream, p, bias_dtype, out_dtype);
     return viola_launch_status();
 }
 
@@ -57,7 +56,7 @@ int launch_group_parts(const GemmArgs& args, int parts, int a_dtype, int b_dtype
     p.k_split = (p.k + parts - 1) / parts;
     p.k_split = (p.k_split + FBK - 1) / FBK * FBK;                           // whole chunks; the last part may be shorter
     p.parts = parts = (int)((p.k + p.k_split - 1) / p.k_split);
-    const int status = launch<true>(p, (int)((p.m + GroupedRows::ROWS - 1) / GroupedRows::ROWS), a_dtype, b_dtype, VIOLA_F32, VIOLA_F32, 1, stream);
+    const int status = launch<GroupedRows, true>(p, (int)((p.m + GroupedRows::ROWS - 1) / GroupedRows::ROWS), a_dtype, b_dtype, VIOLA_F32, VIOLA_F32, 1, stream);
     if (status) return status;
     const dim3 grid((unsigned)((count + 2047) / 2048)), block(256);
     if (out_dtype == VIOLA_F32) VIOLA_LAUNCH(sum_parts<float>, grid, block, 0, stream, workspace, parts, p.out_group_stride, count, static_cast<float*>(args.out));
@@ -68,8 +67,12 @@ int launch_group_parts(const GemmArgs& args, int parts, int a_dtype, int b_dtype
 
 int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale,
                           unsigned groups, hipStream_t stream) {
-    return rowscale ? launch<true>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, groups, stream)
-                    : launch<false>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, groups, stream);
+    return rowscale ? launch<GroupedRows, true>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, groups, stream)
+                    : launch<GroupedWide, false>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, groups, stream);
+}
+
+int launch_group_teams(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+    return launch<GroupedTeams, true>(p, (int)((p.m + GroupedTeams::ROWS - 1) / GroupedTeams::ROWS), a_dtype, b_dtype, bias_dtype, out_dtype, 1, stream);
 }
 
 }  // namespace viola

@@ -15,6 +15,8 @@
 // Row-wise b scales (weight gradient; ROWS true, 256 x 128). The products sa * sb of a pair of units come from one
 // v_mfma_f32_32x32x1_2b (see group_gemm_fast), which occupies the FMA units for its 64 cycles as well; the pair of units before
 // is folded meanwhile, across chunks too, out of two sets of accumulators and products.
+// With few tiles (GroupedTeams, 128 x 128) the halves of the block are two teams with rings of their own that share the k range, as
+// in group_gemm_fast's split form: the same sums, added in the same order.   4096 x 1024 x 8192  86 -> 74 us
 //   22016 x 4096 x 16384  3450 -> 3070 us  4096 x 11008 x 16384   1660 -> 1545    4096 x 4096 x 4096   160 -> 142
 #pragma once
 #include "gemm_pingpong.hpp"
@@ -23,6 +25,8 @@ namespace viola {
 
 using GroupedWide = PingPongShape<2, 4, 4, 2, 4>;                            // uniform b scales: 64 x 128 outputs (a x b) per wave, transposed
 using GroupedRows = PingPongShape<4, 2, 2, 2, 4>;                            // row-wise b scales: 64 x 64
+
+using GroupedTeams = PingPongShape<2, 2, 2, 2, 4>;                           // row-wise, 128 x 128, two teams that share the k range
 
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 
@@ -39,18 +43,21 @@ __device__ __forceinline__ void group_row_tiles(const GemmArgs& p, int base, int
     }
 }
 
-template <bool A_BF8, bool B_BF8, bool ROWS>
+template <bool A_BF8, bool B_BF8, typename S, bool ROWS>
 __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int bias_dtype, int out_dtype) {
-    using S = std::conditional_t<ROWS, GroupedRows, GroupedWide>;
     constexpr int TM = S::TM, TN = S::TN, STAGES = S::STAGES, RING = STAGES * S::STAGE;
     // A scale block is 8 K groups in 16-byte pieces of 4: [half][row of a], then [half][row of b], or with uniform b scales
     // [half][sub-tile of b] (what 64 lanes of one load instruction bring)
     constexpr int B_ENTRIES = ROWS ? S::COLS : S::COLS / 32;
     constexpr int A_SCALES = 2 * S::ROWS * 16, B_SCALES = ROWS ? 2 * B_ENTRIES * 16 : 1024, SCALE_BLOCK = A_SCALES + B_SCALES;
-    static_assert(2 * S::ROWS == 512 && (ROWS || 2 * B_ENTRIES <= 64) && 2 * SCALE_BLOCK >= S::COLS * 4);
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[RING + 2 * SCALE_BLOCK];
-    const int tid = threadIdx.x, lane = tid % WAVE, l32 = lane % 32, lhi = lane / 32;
+    constexpr int TEAM_LDS = RING + 2 * SCALE_BLOCK;
+    static_assert(2 * S::ROWS == S::THREADS && (ROWS || 2 * B_ENTRIES <= 64) && 2 * SCALE_BLOCK >= S::COLS * 4);
+    __shared__ __attribute__((aligned(1024))) uint8_t lds_all[S::TEAMS * TEAM_LDS];
+    // tid, wave and lds are the team's own
+    const int team = S::TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / S::THREADS) : 0;
+    const int tid = threadIdx.x % S::THREADS, lane = tid % WAVE, l32 = lane % 32, lhi = lane / 32;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    uint8_t* const lds = lds_all + team * TEAM_LDS;
     const int wm = wave / S::WN, wn = wave % S::WN;
 
     // ---- tile: contiguous ranges per XCD, walked in groups of 4 m tiles, so that the 32 tiles at work on an XCD are 4 x 8
@@ -106,19 +113,28 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
         k_end = k_begin + p.k_split < p.k ? k_begin + p.k_split : p.k;
         out_shift = part * p.out_group_stride;
     }
+    int split_chunks = 0;                                                    // of the longer (first) half of two teams
+    if constexpr (S::TEAMS > 1) {
+        constexpr int64_t CUT = F_SGROUPS * 32;                              // a scale block belongs to one team
+        const int64_t len = k_end - k_begin, half = ((len + CUT - 1) / CUT + 1) / 2 * CUT, first = half < len ? half : len;
+        split_chunks = (int)((first + FBK - 1) / FBK);
+        if (team == 0) k_end = k_begin + first;
+        else k_begin += first;
+    }
     const int64_t k_len = k_end - k_begin;
 
     // ---- load plan: as in gemm_pingpong
     const i32x4 res_a = raw_resource(p.a + m_begin * p.lda + k_begin), res_b = raw_resource(bptr + k_begin);
     constexpr uint32_t OUTSIDE = 0x80000000u;
-    const int chunks = (int)((k_len + FBK - 1) / FBK), full_chunks = (int)(k_len / FBK), groups_total = (int)((k_len + 31) / 32);
+    // (both teams walk the first half's chunks, they share the barriers: past its own range a team loads zero codes)
+    const int chunks = S::TEAMS > 1 ? split_chunks : (int)((k_len + FBK - 1) / FBK), full_chunks = (int)(k_len / FBK), groups_total = (int)((k_len + 31) / 32);
     const int piece = (tid & 3) ^ ((tid >> 4) & 3);
     const bool inside_tail = (int64_t)full_chunks * FBK + piece * 16 < k_len;
     auto row_in = [](int64_t row, int64_t rows) -> uint32_t { return (uint32_t)(row < rows ? row : rows - 1); };
     uint32_t cur[S::LOADS];
 #pragma unroll
     for (int it = 0; it < S::LOADS; ++it) {
-        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * 128 + tid / 4;
+        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * S::LOAD_ROWS + tid / 4;
         if (it < S::A_LOADS) cur[it] = (uint32_t)(row_in(m_begin + r, m_end) - m_begin) * (uint32_t)p.lda;
         else cur[it] = row_in(n_begin + r, p.n) * (uint32_t)p.ldb;
         asm volatile("" : "+v"(cur[it]));                                    // (as one 64-bit multiply-add it would hold a register pair all along)
@@ -132,13 +148,13 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
 #pragma unroll
             for (int it = 0; it < S::LOADS; ++it) {
                 const uint32_t at = here ? cur[it] : OUTSIDE;
-                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, at, (uint32_t)c * FBK);
+                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * S::THREADS * 16 + (uint32_t)wave * 1024, at, (uint32_t)c * FBK);
             }
             return;
         }
 #pragma unroll
         for (int it = 0; it < S::LOADS; ++it)
-            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * FBK);
+            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * S::THREADS * 16 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * FBK);
     };
     // Scale block `block` -> buffer block & 1: every thread one piece of the a rows, the first waves one of b (lanes past b's last
     // entry read zero). Entries past the end of the k range, which hold whatever follows in memory (see group_gemm_fast), are
@@ -151,13 +167,15 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     if (b_half >= 2) sb_at = OUTSIDE;
     asm volatile("" : "+v"(sa_at), "+v"(sb_at));
     const int last_block = (groups_total - 1) / F_SGROUPS;
-    auto issue_scales = [&](int block) {                                     // (past the last block: that one again, to keep the load counts uniform)
+    // (past the last block: that one again, to keep the load counts uniform; a team that walks on past its own range reads zeros)
+    auto issue_scales = [&](int block) {
         const uint32_t to = lds_base + RING + (uint32_t)(block & 1) * SCALE_BLOCK + (uint32_t)wave * 1024;
         const uint32_t first = (uint32_t)(block < last_block ? block : last_block) * F_SGROUPS * 4;
-        if (wave < B_SCALES / 1024) load16_to_lds(res_sb, to + A_SCALES, sb_at, first);
-        load16_to_lds(res_sa, to, sa_at, first);
+        const bool past = S::TEAMS > 1 && block > last_block;
+        if (wave < B_SCALES / 1024) load16_to_lds(res_sb, to + A_SCALES, past ? OUTSIDE : sb_at, first);
+        load16_to_lds(res_sa, to, past ? OUTSIDE : sa_at, first);
     };
-    const bool straddles = groups_total % F_SGROUPS != 0;
+    const bool straddles = groups_total % F_SGROUPS != 0 || groups_total == 0;
     auto clear_past_the_end = [&] {
         const int left_a = groups_total - (last_block * F_SGROUPS + a_half * 4), left_b = groups_total - (last_block * F_SGROUPS + b_half * 4);
         float* mine = reinterpret_cast<float*>(lds + RING + (last_block & 1) * SCALE_BLOCK + tid * 16);
@@ -329,11 +347,14 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
     __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);                              // chunk 0 and scale block 0
     barrier();
-    if (last_block == 0 && straddles) {
+    if (S::TEAMS > 1) {                                                      // the condition differs between the teams, the barrier must not
+        if (last_block == 0 && straddles) clear_past_the_end();
+        __syncthreads();
+    } else if (last_block == 0 && straddles) {
         clear_past_the_end();
         __syncthreads();
     }
-    const bool late = wave >= 4;
+    const bool late = S::TEAMS > 1 ? team == 1 : wave >= 4;
     if (late) barrier();
     int stage = 0, fill = STAGES - 1;
     for (int c = 0; c < chunks; ++c) {
@@ -360,11 +381,42 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     drain();
     __builtin_amdgcn_s_waitcnt(0x0F70);                                      // the trailing loads must not land in what follows
     barrier();
-    float* bias_lds = reinterpret_cast<float*>(lds + RING);
+    if constexpr (S::TEAMS > 1) {
+        // team 0's sums of the second row of sub-tiles go to team 1, team 1's of the first to team 0 (the rings are idle now):
+        // [register quad][thread]. Either adds and stores half of the tile; x + y is y + x, so a launch is reproducible bit for bit.
+        static_assert(TM == 2);
+        float4* exchange = reinterpret_cast<float4*>(lds_all);
+        constexpr int QUADS = TN * 4;
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                auto give = [&](int e) -> float {
+                    const float first = total[i][0][4 * q + e], second = total[i][TM - 1][4 * q + e];
+                    return team == 0 ? second : first;
+                };
+                exchange[(team * QUADS + i * 4 + q) * S::THREADS + tid] = make_float4(give(0), give(1), give(2), give(3));
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 t = exchange[((1 - team) * QUADS + i * 4 + q) * S::THREADS + tid];
+                const float add[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {                                // (the half it stores goes to the first row of sub-tiles' place)
+                    const float first = total[i][0][4 * q + e], second = total[i][TM - 1][4 * q + e];
+                    total[i][0][4 * q + e] = (team == 0 ? first : second) + add[e];
+                }
+            }
+        __syncthreads();
+    }
+    float* bias_lds = reinterpret_cast<float*>(lds_all + S::TEAMS * TEAM_LDS - 2 * SCALE_BLOCK);
     stage_bias<S>(p, n_begin, bias_lds, bias_dtype);
     auto finish = [&](auto type) {
         using TO = decltype(type);
-        store_tile<S, TN, true>(total, p, static_cast<TO*>(p.out) + out_shift, m_begin, m_end, n_begin, lds, bias_lds);
+        store_tile<S, TN, true>(total, p, static_cast<TO*>(p.out) + out_shift, m_begin, m_end, n_begin, lds_all, bias_lds);
     };
     if (out_dtype == VIOLA_F32) finish(float{});
     else if (out_dtype == VIOLA_BF16) finish(bf16_t{});
