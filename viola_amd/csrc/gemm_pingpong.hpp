@@ -14,16 +14,18 @@
 
 namespace viola {
 
-// WM x WN waves of TM x TN sub-tiles of 32 x 32; STAGES chunks of 64 k in the ring
-template <int WM_, int WN_, int TM_, int TN_, int STAGES_>
+// WM x WN waves of TM x TN sub-tiles of 32 x 32; STAGES chunks of CHUNK k (bytes per operand row) in the ring
+template <int WM_, int WN_, int TM_, int TN_, int STAGES_, int CHUNK_ = FBK>
 struct PingPongShape {
+    static constexpr int CHUNK = CHUNK_, PIECES = CHUNK / 16, HALVES = CHUNK / 64;   // 16-byte pieces of a row; 64 k per MFMA
     static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, STAGES = STAGES_;
     static constexpr int TEAMS = 8 / (WM * WN), THREADS = 512 / TEAMS;       // two teams of four waves: gemm_pingpong_grouped.hpp
     static constexpr int ROWS = WM * TM * 32, COLS = WN * TN * 32;
-    static constexpr int A_BYTES = ROWS * FBK, B_BYTES = COLS * FBK, STAGE = A_BYTES + B_BYTES;
-    static constexpr int LOAD_ROWS = THREADS / 4;                            // a load instruction of all threads: 16 bytes each
-    static constexpr int A_LOADS = ROWS / LOAD_ROWS, B_LOADS = COLS / LOAD_ROWS, LOADS = A_LOADS + B_LOADS;
-    static_assert(WM * WN * TEAMS == 8 && ROWS % LOAD_ROWS == 0 && COLS % LOAD_ROWS == 0);
+    static constexpr int LOAD_ROWS = THREADS / PIECES;                       // a load instruction of all threads: 16 bytes each
+    static constexpr int A_LOADS = ROWS / LOAD_ROWS, B_LOADS = (COLS + LOAD_ROWS - 1) / LOAD_ROWS, LOADS = A_LOADS + B_LOADS;
+    static constexpr int B_ROWS = B_LOADS * LOAD_ROWS;                       // of b in a stage: past COLS nothing is fetched
+    static constexpr int A_BYTES = ROWS * CHUNK, B_BYTES = B_ROWS * CHUNK, STAGE = A_BYTES + B_BYTES;
+    static_assert(WM * WN * TEAMS == 8 && ROWS % LOAD_ROWS == 0);
 };
 
 // Epilogue. The tile's bias as fp32 in LDS (COLS floats), -0 where there is none: adding that changes nothing, not even a sign.
@@ -91,7 +93,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     static_assert(!GATED || TN == 2, "a gate and an up sub-tile per wave");
     constexpr int PANEL = GATED ? S::COLS / 2 : S::COLS;                     // columns of the output per tile
     constexpr int RING = STAGES * S::STAGE;
-    constexpr int SCALE_BLOCK = (S::ROWS + S::COLS) * MX_GROUPS;             // scale bytes of 16 K groups, a rows then b rows
+    constexpr int SCALE_BLOCK = (S::ROWS + S::B_ROWS) * MX_GROUPS;           // scale bytes of 16 K groups, a rows then b rows
     constexpr int TAIL = MX ? 2 * SCALE_BLOCK : S::COLS * 4;                 // behind the ring: scale blocks, later the bias row
     static_assert(TAIL >= S::COLS * 4);
     __shared__ __attribute__((aligned(1024))) uint8_t lds[RING + TAIL];
@@ -107,12 +109,14 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     const int rows_here = p.tiles_m - first_m < 8 ? p.tiles_m - first_m : 8;
     const int64_t m_begin = (int64_t)(first_m + t % group % rows_here) * S::ROWS, n_begin = (int64_t)(t % group / rows_here) * PANEL;
 
-    // ---- load plan: instruction `it` brings rows 128 it .. of an operand, unit U = 4 row + slot holds piece slot ^ ((row >> 2) & 3)
+    // ---- load plan: instruction `it` brings LOAD_ROWS rows of an operand, unit U = PIECES row + slot holds piece slot ^ swizzle(row)
     const i32x4 res_a = raw_resource(p.a + m_begin * p.lda), res_b = raw_resource(p.b);
     constexpr uint32_t OUTSIDE = 0x80000000u;
-    const int chunks = (int)((p.k + FBK - 1) / FBK), full_chunks = (int)(p.k / FBK), groups_total = (int)((p.k + 31) / 32);
-    const int piece = (tid & 3) ^ ((tid >> 4) & 3);
-    const bool inside_tail = (int64_t)full_chunks * FBK + piece * 16 < p.k;
+    const int chunks = (int)((p.k + S::CHUNK - 1) / S::CHUNK), full_chunks = (int)(p.k / S::CHUNK), groups_total = (int)((p.k + 31) / 32);
+    // 16 consecutive rows reading the same piece then cover all banks
+    auto swizzle = [](int row) -> int { return S::PIECES == 4 ? (row >> 2) & 3 : (row >> 1) & 7; };
+    const int piece = tid % S::PIECES ^ swizzle(tid / S::PIECES);
+    const bool inside_tail = (int64_t)full_chunks * S::CHUNK + piece * 16 < p.k;
     auto row_in = [](int64_t row, int64_t rows) -> uint32_t { return (uint32_t)(row < rows ? row : rows - 1); };
     auto b_row = [&](int r) -> uint32_t {                                    // tile-local b row -> row of b
         if constexpr (GATED) return (uint32_t)(r / PANEL) * (uint32_t)p.n + row_in(n_begin + r % PANEL, p.n);
@@ -121,9 +125,9 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     uint32_t cur[S::LOADS];
 #pragma unroll
     for (int it = 0; it < S::LOADS; ++it) {
-        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * 128 + tid / 4;
+        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * S::LOAD_ROWS + tid / S::PIECES;
         if (it < S::A_LOADS) cur[it] = (uint32_t)(row_in(m_begin + r, p.m) - m_begin) * (uint32_t)p.lda + piece * 16;
-        else cur[it] = b_row(r) * (uint32_t)p.ldb + piece * 16;
+        else cur[it] = r < S::COLS ? b_row(r) * (uint32_t)p.ldb + piece * 16 : OUTSIDE;
     }
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
     auto issue = [&](int c, int stage) {
@@ -133,13 +137,13 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
 #pragma unroll
             for (int it = 0; it < S::LOADS; ++it) {
                 const uint32_t at = here ? cur[it] : OUTSIDE;
-                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, at, (uint32_t)c * FBK);
+                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, at, (uint32_t)c * S::CHUNK);
             }
             return;
         }
 #pragma unroll
         for (int it = 0; it < S::LOADS; ++it)
-            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * FBK);
+            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * 8192 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * S::CHUNK);
     };
     // E8M0 scales: one 16-byte piece (16 K groups) per tile row, block `b` in buffer b & 1
     const i32x4 res_sa = raw_resource(p.sa, p.sa_bytes), res_sb = raw_resource(p.sb, p.sb_bytes);
@@ -148,14 +152,14 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
         scale_at = tid < S::ROWS ? row_in(m_begin + tid, p.m) / (uint32_t)p.ar * (uint32_t)p.ldsa : b_row(tid - S::ROWS) / (uint32_t)p.br * (uint32_t)p.ldsb;
     }
     auto issue_scales = [&](int block) {
-        if (wave * 64 >= S::ROWS + S::COLS) return;
+        if (wave * 64 >= S::ROWS + S::B_ROWS) return;
         const uint32_t to = lds_base + RING + (uint32_t)(block & 1) * SCALE_BLOCK + (uint32_t)wave * 1024;
         load16_to_lds(wave * 64 < S::ROWS ? res_sa : res_sb, to, block * MX_GROUPS < groups_total ? scale_at : OUTSIDE, (uint32_t)(block * MX_GROUPS));
     };
 
     // ---- operand reads
-    const int sw = (l32 >> 2) & 3;
-    const int rd_a = (wm * TM * 32 + l32) * FBK + ((lhi ^ sw) * 16), rd_b = S::A_BYTES + ((GATED ? wn : wn * TN) * 32 + l32) * FBK + ((lhi ^ sw) * 16);
+    const int sw = swizzle(l32);
+    const int rd_a = (wm * TM * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16), rd_b = S::A_BYTES + ((GATED ? wn : wn * TN) * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16);
     constexpr int NEXT_B = GATED ? PANEL : 32;                               // b rows from one sub-tile of a wave to the next
     f32x16 total[TN][TM];
 #pragma unroll
@@ -164,8 +168,9 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
         for (int j = 0; j < TM; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) total[i][j][r] = 0.0f;
-    i32x8 oa[TM], ob[TN];
-    // scale words of the chunk pair at hand: byte 0 = this lane's K group of the even chunk, byte 2 = of the odd chunk
+    constexpr int HALVES = S::HALVES;                                        // of a chunk: 64 k, one MFMA per sub-tile
+    i32x8 oa[HALVES][TM], ob[HALVES][TN];
+    // scale words of the 128 k at hand: byte 0 = this lane's K group of the first 64 k, byte 2 = of the second
     uint32_t wa[TM], wb[TN];
 #pragma unroll
     for (int j = 0; j < TM; ++j) wa[j] = 0;
@@ -173,17 +178,21 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     for (int i = 0; i < TN; ++i) wb[i] = 0;
     auto read = [&](int stage, int c) {
         const uint8_t* base = lds + stage * S::STAGE;
-        auto operand = [&](int offset) -> i32x8 {
-            const i32x4 lo = *reinterpret_cast<const i32x4*>(base + offset), hi = *reinterpret_cast<const i32x4*>(base + (offset ^ 32));
+        auto operand = [&](int offset, int half) -> i32x8 {                  // pieces 4 half + lhi and 4 half + lhi + 2
+            const i32x4 lo = *reinterpret_cast<const i32x4*>(base + (offset ^ (half * 64))), hi = *reinterpret_cast<const i32x4*>(base + (offset ^ (half * 64 + 32)));
             return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         };
 #pragma unroll
-        for (int i = 0; i < TN; ++i) ob[i] = operand(rd_b + i * NEXT_B * FBK);
+        for (int h = 0; h < HALVES; ++h) {
 #pragma unroll
-        for (int j = 0; j < TM; ++j) oa[j] = operand(rd_a + j * 32 * FBK);
+            for (int i = 0; i < TN; ++i) ob[h][i] = operand(rd_b + i * NEXT_B * S::CHUNK, h);
+#pragma unroll
+            for (int j = 0; j < TM; ++j) oa[h][j] = operand(rd_a + j * 32 * S::CHUNK, h);
+        }
         if constexpr (MX) {
-            if ((c & 1) == 0) {
-                const uint8_t* block = lds + RING + ((c / MX_CHUNKS) & 1) * SCALE_BLOCK + (c % MX_CHUNKS) * FKG;
+            if (HALVES == 2 || (c & 1) == 0) {
+                constexpr int CHUNKS = MX_CHUNKS / HALVES;               // per scale block
+                const uint8_t* block = lds + RING + ((c / CHUNKS) & 1) * SCALE_BLOCK + (c % CHUNKS) * FKG * HALVES;
 #pragma unroll
                 for (int j = 0; j < TM; ++j) wa[j] = *reinterpret_cast<const uint32_t*>(block + (wm * TM * 32 + j * 32 + l32) * MX_GROUPS) >> (8 * lhi);
 #pragma unroll
@@ -192,13 +201,21 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
         }
     };
     auto math = [&](auto odd) {
-        constexpr int FB = B_BF8 ? 1 : 0, FA = A_BF8 ? 1 : 0, BYTE = MX && decltype(odd)::value ? 2 : 0;
+        constexpr int FB = B_BF8 ? 1 : 0, FA = A_BF8 ? 1 : 0, BYTE = MX && HALVES == 1 && decltype(odd)::value ? 2 : 0;
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int i = 0; i < TN; ++i)
 #pragma unroll
             for (int j = 0; j < TM; ++j)
-                total[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ob[i], oa[j], total[i][j], FB, FA, BYTE, MX ? (int)wb[i] : 0, BYTE, MX ? (int)wa[j] : 0);
+                total[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ob[0][i], oa[0][j], total[i][j], FB, FA, BYTE, MX ? (int)wb[i] : 0, BYTE, MX ? (int)wa[j] : 0);
+        if constexpr (HALVES == 2) {
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j)
+                    total[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ob[HALVES - 1][i], oa[HALVES - 1][j], total[i][j], FB, FA, MX ? 2 : 0, MX ? (int)wb[i] : 0,
+                                                                                  MX ? 2 : 0, MX ? (int)wa[j] : 0);
+        }
         // (the compiler sinks MFMAs into the following read phase otherwise: intrinsics without side effects cross a barrier)
 #pragma unroll
         for (int i = 0; i < TN; ++i)
@@ -208,9 +225,12 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     };
     auto pin_operands = [&] {                                                // in registers before the barrier, scale bytes in place
 #pragma unroll
-        for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(oa[j]), "+v"(wa[j]));
+        for (int h = 0; h < HALVES; ++h) {
 #pragma unroll
-        for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(ob[i]), "+v"(wb[i]));
+            for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(oa[h][j]), "+v"(wa[j]));
+#pragma unroll
+            for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(ob[h][i]), "+v"(wb[i]));
+        }
     };
     auto barrier = [] {
         __builtin_amdgcn_sched_barrier(0);
@@ -236,7 +256,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     auto step = [&](int c, auto odd) {
         read(stage, c);
         if constexpr (MX) {
-            if (c % MX_CHUNKS == 0) issue_scales(c / MX_CHUNKS + 1);
+            if (c % (MX_CHUNKS / HALVES) == 0) issue_scales(c / (MX_CHUNKS / HALVES) + 1);
         }
         issue(c + STAGES - 1, fill);
         stage = stage == STAGES - 1 ? 0 : stage + 1;
@@ -300,10 +320,15 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     else finish(f16_t{});
 }
 
-// The three tiles: 256 x 256 and 256 x 128 with one block per CU, 128 x 128 with two.
+// The three tiles: 256 x 256 and 256 x 128 with one block per CU, 128 x 128 with one or two. A turn of the two halves costs some 200
+// cycles beside the math (barriers, the first LDS reads), which is a lot next to the 256 cycles of a wave's four MFMAs: where
+// registers and LDS allow it a chunk is 128 k (whole cache lines of the operands, too). 256 x 128: 4096 x 1152 x 9216 61 -> 47 us,
+// 8192 x 1024 x 4096 36 -> 30, 4096 x 1152 x 4608 33 -> 26 (E8M0 35 -> 30); 128 x 128 alone on its CU: 2048 x 1152 x 4608 22 -> 19.
+// (96- and 192-column tiles, which leave fewer CUs idle at widths like 1152, gain nothing: a smaller tile's turn takes as long.)
 using PingPongL = PingPongShape<2, 4, 4, 2, 4>;
-using PingPongM = PingPongShape<4, 2, 2, 2, 4>;
-using PingPongS = PingPongShape<2, 4, 2, 1, 4>;
+using PingPongM = PingPongShape<4, 2, 2, 2, 3, 128>;
+using PingPongS = PingPongShape<2, 4, 2, 1, 3, 128>;
+using PingPongPairs = PingPongShape<2, 4, 2, 1, 4>;
 
 template <bool MX, typename S, int WAVES_PER_SIMD, bool GATED = false>
 static int launch_pingpong(const GemmArgs& args, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
@@ -326,7 +351,8 @@ static int launch_pingpong_tile(const GemmArgs& p, ScaledTile tile, bool gated, 
     if (gated) return launch_pingpong<MX, PingPongL, 2, true>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
     if (tile == SCALED_TILE_L) return launch_pingpong<MX, PingPongL, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
     if (tile == SCALED_TILE_M) return launch_pingpong<MX, PingPongM, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
-    return launch_pingpong<MX, PingPongS, 4>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    if ((p.m + 127) / 128 * ((p.n + 127) / 128) <= 256) return launch_pingpong<MX, PingPongS, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    return launch_pingpong<MX, PingPongPairs, 4>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
 }
 
 }  // namespace viola
