@@ -1,5 +1,5 @@
-"""GPU parity: per-tensor and block-scaled products on the alternating-phase tiles whose chunks are 128 k (256 x 128, and 128 x 128
-alone on its CU). Integer operands and power-of-two scales, so every element must equal the integer product."""
+"""GPU parity: per-tensor and block-scaled products on the alternating-phase tiles whose chunks are 128 k (256 x 256, 256 x 128, and
+128 x 128 alone on its CU). Integer operands and power-of-two scales, so every element must equal the integer product."""
 
 import pytest
 import torch
@@ -12,7 +12,8 @@ E4, E5 = torch.float8_e4m3fn, torch.float8_e5m2
 # than stages; ragged rows and columns
 @pytest.mark.parametrize("scaling", ["tensor", "mx"])
 @pytest.mark.parametrize("m,n,k,formats", [(4096, 1152, 1296, (E4, E4)), (4090, 1150, 1360, (E5, E4)), (4096, 1152, 128, (E4, E5)), (4000, 1100, 256, (E4, E4)),
-                                           (2048, 1152, 4624, (E4, E4)), (2000, 1030, 2064, (E5, E5)), (1920, 1920, 640, (E4, E4)), (1921, 1919, 80, (E4, E4))])
+                                           (2048, 1152, 4624, (E4, E4)), (2000, 1030, 2064, (E5, E5)), (1920, 1920, 640, (E4, E4)), (1921, 1919, 80, (E4, E4)),
+                                           (4096, 4096, 1104, (E4, E5)), (4090, 4000, 2128, (E4, E4)), (4000, 4090, 4608, (E5, E5)), (4096, 4096, 384, (E4, E4))])
 def test_products_in_chunks_of_128(m, n, k, formats, scaling):
     from viola_amd.nn import _grouped_kernels as g, _linear_kernels as lk
     if scaling == "mx":

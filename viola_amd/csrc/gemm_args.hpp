@@ -82,10 +82,10 @@ bool launch_gated_pieces(const void* z, const void* dy, int64_t dy_stride, void*
 // The choice is the least of four estimates in microseconds, fitted to the measured times of 38 shapes (bf16 outputs, both recipes;
 // within 15 % of nearly all). A round of one tile per CU takes a fixed part (first loads, stores of the tile) and a time per chunk of 64 k
 // that grows with the share of CUs at work, because the clock falls as the matrix pipes fill (2.4 to 1.7 GHz):
-//   L 0.45 .. 0.75 + 7    M 0.22 .. 0.39 + 5.3    S 0.235 alone + 4; two blocks per CU 0.57 for the pair + 4
+//   L 0.40 .. 0.71 + 8.5    M 0.22 .. 0.39 + 5.3    S 0.235 alone + 4; two blocks per CU 0.57 for the pair + 4
 // group_gemm_fast has no rounds to speak of (three small blocks per CU, their stores under each other's math): 0.31 per tile
 // and chunk of a CU's share + 0.7 per tile. What that comes to: 8192 x 1024 x 4096 M (30 us), 4096 x 1152 x 4608 M (26),
-// 4096 x 4096 x 16384 L (195), 4096 x 4608 x 1152 stays (30), 2048 x 1152 x 4608 S (19).
+// 4096 x 4096 x 4096 L (55), 4096 x 4608 x 1152 stays (30), 2048 x 1152 x 4608 S (19).
 enum ScaledTile { SCALED_TILE_FAST = 0, SCALED_TILE_L, SCALED_TILE_M, SCALED_TILE_S };
 inline ScaledTile choose_scaled_tile(int64_t m, int64_t n, int64_t k) {
     constexpr int64_t CUS = 256;
@@ -97,7 +97,7 @@ inline ScaledTile choose_scaled_tile(int64_t m, int64_t n, int64_t k) {
         const double full = (double)(count / CUS), rest = (double)(count % CUS) / CUS;
         return full * (chunks * busy + fixed) + (rest > 0 ? chunks * (idle + (busy - idle) * rest) + fixed : 0.0);
     };
-    const double large = rounds(tiles(256, 256), 0.45, 0.75, 7.0), medium = rounds(tiles(256, 128), 0.22, 0.39, 5.3);
+    const double large = rounds(tiles(256, 256), 0.40, 0.71, 8.5), medium = rounds(tiles(256, 128), 0.22, 0.39, 5.3);
     const double pairs = small <= CUS ? chunks * 0.235 + 4.0 : (double)((small + 2 * CUS - 1) / (2 * CUS)) * (chunks * 0.57 + 4.0);
     const double fast = small >= 2 * CUS ? (double)small / CUS * (chunks * 0.31 + 0.7) + 4.0 : 1e30;
     ScaledTile best = SCALED_TILE_FAST;

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
 
     // ---- operand reads
     const int sw = swizzle(l32);
-    const int rd_a = (wm * TM * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16), rd_b = S::A_BYTES + ((GATED ? wn : wn * TN) * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16);
+    const int rd_a0 = (wm * TM * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16), rd_b0 = S::A_BYTES + ((GATED ? wn : wn * TN) * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16);
     constexpr int NEXT_B = GATED ? PANEL : 32;                               // b rows from one sub-tile of a wave to the next
     f32x16 total[TN][TM];
 #pragma unroll
@@ -169,6 +169,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
 #pragma unroll
             for (int r = 0; r < 16; ++r) total[i][j][r] = 0.0f;
     constexpr int HALVES = S::HALVES;                                        // of a chunk: 64 k, one MFMA per sub-tile
+    constexpr int SCALE_CHUNKS = MX_CHUNKS / HALVES;                         // chunks per scale block
     i32x8 oa[HALVES][TM], ob[HALVES][TN];
     // scale words of the 128 k at hand: byte 0 = this lane's K group of the first 64 k, byte 2 = of the second
     uint32_t wa[TM], wb[TN];
@@ -178,6 +179,8 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     for (int i = 0; i < TN; ++i) wb[i] = 0;
     auto read = [&](int stage, int c) {
         const uint8_t* base = lds + stage * S::STAGE;
+        int rd_a = rd_a0, rd_b = rd_b0;
+        asm volatile("" : "+v"(rd_a), "+v"(rd_b));                           // the addresses below: formed anew, 256 x 256 has no registers to keep them
         auto operand = [&](int offset, int half) -> i32x8 {                  // pieces 4 half + lhi and 4 half + lhi + 2
             const i32x4 lo = *reinterpret_cast<const i32x4*>(base + (offset ^ (half * 64))), hi = *reinterpret_cast<const i32x4*>(base + (offset ^ (half * 64 + 32)));
             return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -191,8 +194,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
         }
         if constexpr (MX) {
             if (HALVES == 2 || (c & 1) == 0) {
-                constexpr int CHUNKS = MX_CHUNKS / HALVES;               // per scale block
-                const uint8_t* block = lds + RING + ((c / CHUNKS) & 1) * SCALE_BLOCK + (c % CHUNKS) * FKG * HALVES;
+                const uint8_t* block = lds + RING + ((c / SCALE_CHUNKS) & 1) * SCALE_BLOCK + (c % SCALE_CHUNKS) * FKG * HALVES;
 #pragma unroll
                 for (int j = 0; j < TM; ++j) wa[j] = *reinterpret_cast<const uint32_t*>(block + (wm * TM * 32 + j * 32 + l32) * MX_GROUPS) >> (8 * lhi);
 #pragma unroll
@@ -243,29 +245,39 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     // 2c - 1) had their operands in registers before the barrier that ended that phase. Every wave ends its read phase of
     // chunk c with its own loads of chunk c + 1 landed (at most those of the STAGES - 2 chunks after it in flight; a scale
     // block among them only makes the wait stricter), and chunk c + 1 is first read two barriers later.
-    constexpr int AHEAD = (STAGES - 2) * S::LOADS;
-    static_assert((STAGES - 1) * S::LOADS < 16 && STAGES >= 3);
+    // Two stages: chunk c + 1 goes out in phase 2c, once waves 4-7 have read chunk c - 1 (waves 0-3 issue it in their read phase of
+    // chunk c, waves 4-7 in their math phase of chunk c - 1), and every wave waits for its part before the barrier that ends phase
+    // 2c + 1 (waves 0-3 behind their math, waves 4-7 behind their reads of chunk c).
+    constexpr bool TWO = STAGES == 2;
+    constexpr int AHEAD = TWO ? 0 : (STAGES - 2) * S::LOADS;
+    static_assert((STAGES - 1) * S::LOADS < 16);
     if constexpr (MX) issue_scales(0);
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
-    __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);                              // chunk 0 and scale block 0
+    for (int s = 0; s < (TWO ? 2 : STAGES - 1); ++s) issue(s, s);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (TWO ? S::LOADS : AHEAD));           // chunk 0 and scale block 0
     barrier();
     const bool late = wave >= 4;
     if (late) barrier();
-    int stage = 0, fill = STAGES - 1;
+    int stage = 0, fill = TWO && late ? 0 : STAGES - 1;
     auto step = [&](int c, auto odd) {
         read(stage, c);
-        if constexpr (MX) {
-            if (c % (MX_CHUNKS / HALVES) == 0) issue_scales(c / (MX_CHUNKS / HALVES) + 1);
-        }
-        issue(c + STAGES - 1, fill);
+        auto issue_next = [&](int next) {
+            if constexpr (MX) {
+                if (c % SCALE_CHUNKS == 0) issue_scales(c / SCALE_CHUNKS + 1);
+            }
+            if (!TWO || next > 1) issue(next, fill);                         // (two stages: chunk 1 went out with chunk 0)
+            fill = fill == STAGES - 1 ? 0 : fill + 1;
+        };
+        if (!TWO || !late) issue_next(c + STAGES - 1);
         stage = stage == STAGES - 1 ? 0 : stage + 1;
-        fill = fill == STAGES - 1 ? 0 : fill + 1;
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
+        if (!TWO || late) __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
+        else __builtin_amdgcn_s_waitcnt(0xC07F);                             // the LDS reads alone
         pin_operands();
         barrier();
+        if (TWO && late) issue_next(c + 2);
         math(odd);
+        if (TWO && !late) __builtin_amdgcn_s_waitcnt(0x0F70);
         barrier();
     };
     int c = 0;
@@ -321,11 +333,13 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
 }
 
 // The three tiles: 256 x 256 and 256 x 128 with one block per CU, 128 x 128 with one or two. A turn of the two halves costs some 200
-// cycles beside the math (barriers, the first LDS reads), which is a lot next to the 256 cycles of a wave's four MFMAs: where
-// registers and LDS allow it a chunk is 128 k (whole cache lines of the operands, too). 256 x 128: 4096 x 1152 x 9216 61 -> 47 us,
+// cycles beside the math (barriers, the first LDS reads), which is a lot next to the 256 or 512 cycles of a wave's four or eight
+// MFMAs: where registers and LDS allow it a chunk is 128 k (whole cache lines of the operands, too). 256 x 256, in two stages for
+// want of LDS: 4096 x 4096 x 4096 61 -> 55 us (E8M0 64 -> 57), 16384 x 4096 x 11008 547 -> 509, 8192 x 8192 x 8192 394 -> 387 (the
+// power limit), even up to k = 1024 and where CUs are idle. 256 x 128: 4096 x 1152 x 9216 61 -> 47 us,
 // 8192 x 1024 x 4096 36 -> 30, 4096 x 1152 x 4608 33 -> 26 (E8M0 35 -> 30); 128 x 128 alone on its CU: 2048 x 1152 x 4608 22 -> 19.
 // (96- and 192-column tiles, which leave fewer CUs idle at widths like 1152, gain nothing: a smaller tile's turn takes as long.)
-using PingPongL = PingPongShape<2, 4, 4, 2, 4>;
+using PingPongL = PingPongShape<2, 4, 4, 2, 2, 128>;
 using PingPongM = PingPongShape<4, 2, 2, 2, 3, 128>;
 using PingPongS = PingPongShape<2, 4, 2, 1, 3, 128>;
 using PingPongPairs = PingPongShape<2, 4, 2, 1, 4>;
