@@ -81,6 +81,39 @@ def test_varlen_products_on_large_tiles(counts):
         row += c
 
 
+# one round of 256 x 128 tiles in chunks of 128 k: k that ends with a chunk, in each quarter of one and inside a slot of 32; ragged rows and columns
+@pytest.mark.parametrize("m,n,k,out_dtype", [(8192, 1024, 2048, torch.bfloat16), (8000, 1000, 2064, torch.float32), (5000, 900, 2144, torch.float16),
+                                             (3000, 2304, 2208, torch.bfloat16), (2304, 2250, 1968, torch.float32), (16384, 512, 1792, torch.bfloat16)])
+def test_grouped_products_on_one_round_of_tall_tiles(m, n, k, out_dtype):
+    """(with a row's first scale a NaN, which the piece of the row before's last ones reaches into)"""
+    from viola_amd.nn import _grouped_kernels as g
+    torch.manual_seed(m + n + k)
+    a, b, groups = _integers(m, k), _integers(n, k), -(-k // 32)
+    sa, sb = _scales(m, groups), _scales(-(-n // 32), groups)
+    bias = torch.randint(-8, 9, (n,), device="cuda").float()
+    want = _spell(a, sa, 1) @ _spell(b, sb, 32).T + bias
+    sa[7, 0], sb[-1, 0] = float("nan"), float("inf")
+    out = g.gemm(a.to(E5), b.to(E4), sa, sb, (1, 32), (32, 32), out_dtype=out_dtype, bias=bias)
+    rows, columns = torch.arange(m, device="cuda") != 7, (n - 1) // 32 * 32
+    assert torch.equal(out[rows, :columns], want[rows, :columns].to(out_dtype)) and torch.isnan(out[7]).all()
+
+
+def test_varlen_products_on_one_round_of_tall_tiles():
+    torch.manual_seed(4)
+    counts = [2900, 0, 1, 3000, 256]
+    groups, n, k, total = len(counts), 1000, 2144, sum(counts)
+    a, b = _integers(total, k), _integers(groups, n, k)
+    offsets = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], device="cuda")
+    sa, sb = _scales(total, k // 32), _scales(groups, -(-n // 32), k // 32)
+    out, qa, qb = torch.full((total, n), 7.0, device="cuda"), a.to(E4), b.to(E4)
+    _lib.call("viola_varlen_group_gemm", qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E4), sa.data_ptr(), sb.data_ptr(), offsets.data_ptr(),
+              groups, total, n, k, 1, 32, 32, 32, n * k, sb[0].numel(), out.data_ptr(), 0)
+    row = 0
+    for g, c in enumerate(counts):
+        assert torch.equal(out[row:row + c], _spell(a[row:row + c], sa[row:row + c], 1) @ _spell(b[g], sb[g], 32).T)
+        row += c
+
+
 def test_varlen_weight_gradient_on_large_tiles():
     """k ranges per group: none, one slot of 32, ranges that end inside a chunk."""
     torch.manual_seed(3)

@@ -55,6 +55,9 @@ int launch_group_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype
 int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, unsigned groups,
                           hipStream_t stream);
 
+// Uniform b scales on one round of 256 x 128 tiles. gemm_pingpong_grouped.hip.
+int launch_group_tall(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream);
+
 // Row-wise b scales on tiles of 128 x 128, the k range split over two teams of waves that take turns. gemm_pingpong_grouped.hip.
 int launch_group_teams(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream);
 

@@ -73,6 +73,20 @@ static bool prefer_pingpong(const GemmArgs& p, bool rowscale, unsigned k_groups)
     return rounds * (chunks * busy + ends) + (rest > 0 ? chunks * (idle + (busy - idle) * rest) + ends : 0.0) < now;
 }
 
+// Whether a product with uniform b scales that is too small for 256 x 256 tiles runs on tiles of 256 x 128, one round of them: where two
+// blocks of 128 x 128 would share a CU. Measured over 129 to 256 such tiles (0 % to 20 % of them padding), both times are linear in the
+// share of the chip at work: 8192 x 1024 x 4096 70 -> 66 us, 9850 x 768 x 3072 51 -> 49, 16384 x 512 x 8192 136 -> 126, 5000 x 1024 x 4096
+// 58 -> 55; up to k = 1024 the small blocks, which cover each other's ends, are as fast (8192 x 1024 x 1024 20.7 us, x 512 12.6 against
+// 13.3). Two rounds always lose (12000 x 768 x 2048, 282 tiles, 48 -> 62).
+static bool prefer_tall(const GemmArgs& p) {
+    if (p.koffsets || 256 * p.lda >= (1ll << 31)) return false;
+    const int64_t columns = (p.n + 127) / 128, rows = p.offsets ? p.m / 256 + p.groups : (p.m + 255) / 256;
+    const double tall = (double)(rows * columns), small = (double)columns * (p.offsets ? (double)p.m / 128 + 0.5 * p.groups : (double)((p.m + 127) / 128));
+    if (small <= 256.0 || tall > 256.0) return false;
+    const double chunks = (double)p.k / 64.0;
+    return chunks * (0.45 + 0.5 * tall / 256.0) + 5.0 < chunks * (0.53 + 0.51 * small / 512.0) + 3.3;
+}
+
 // In how many parts of k a weight gradient runs, which has few tiles and a long k. Whole, 129 to 256 tiles of 128 x 128 leave CUs
 // without a tile, and fewer run as narrow tiles, which read more per product; in parts, tiles of 256 x 128 fill the chip and a second
 // launch adds the partial products. The least of the estimates in microseconds (fitted to 24 shapes) decides, and only where it
@@ -109,6 +123,10 @@ int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dt
     if (mode == MODE_PLAIN && prefer_pingpong(p, rowscale, grid.z)) {
         const int64_t row_tiles = p.offsets ? p.m / 256 + p.groups : (p.m + 255) / 256;
         return launch_group_pingpong(p, (int)row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid.z, stream);
+    }
+    if (mode == MODE_PLAIN && !rowscale && prefer_tall(p)) {
+        const int64_t row_tiles = p.offsets ? p.m / 256 + p.groups : (p.m + 255) / 256;
+        return launch_group_tall(p, (int)row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
     }
     // Two blocks of 128 x 128 fit a CU, so from 257 tiles up every CU has work and the full tile, which reads the least, is
     // the fastest form (4096 x 1152 x 4608: 75.6 -> 59.7 us against the split one, 6000 x 1000 x 1024: 27.0 -> 19.6 us against

@@ -71,6 +71,10 @@ int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_d
                     : launch<GroupedWide, false>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, groups, stream);
 }
 
+int launch_group_tall(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+    return launch<GroupedTall, false>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, 1, stream);
+}
+
 int launch_group_teams(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
     return launch<GroupedTeams, true>(p, (int)((p.m + GroupedTeams::ROWS - 1) / GroupedTeams::ROWS), a_dtype, b_dtype, bias_dtype, out_dtype, 1, stream);
 }

@@ -12,6 +12,9 @@
 // 432 us at 16384 x 4096 x 4096). The last two units of a chunk are folded in the wave's next read phase, under the other half's
 // MFMAs, so that the accumulators' numbering starts over with each chunk; all 256 registers are in use.
 //   16384 x 4096 x 4096   505 -> 445 us    16384 x 22016 x 4096   2700 -> 2400    8192 x 4096 x 1024   76 -> 67
+// Products too small for those take tiles of 256 x 128 (GroupedTall, 64 x 64 per wave) in chunks of 128 k, so that a turn has as much
+// math. Its registers allow more accumulators, but folding more units in the read phase gains nothing (lag of 3, 4, 5: 521, 529,
+// 532 us where 2 takes 515); nor does issuing the loads ahead of the LDS reads (521).   8192 x 1024 x 4096  70 -> 66 us
 // Row-wise b scales (weight gradient; ROWS true, 256 x 128). The products sa * sb of a pair of units come from one
 // v_mfma_f32_32x32x1_2b (see group_gemm_fast), which occupies the FMA units for its 64 cycles as well; the pair of units before
 // is folded meanwhile, across chunks too, out of two sets of accumulators and products.
@@ -25,6 +28,7 @@ namespace viola {
 
 using GroupedWide = PingPongShape<2, 4, 4, 2, 4>;                            // uniform b scales: 64 x 128 outputs (a x b) per wave, transposed
 using GroupedRows = PingPongShape<4, 2, 2, 2, 4>;                            // row-wise b scales: 64 x 64
+using GroupedTall = PingPongShape<4, 2, 2, 2, 3, 128>;                       // uniform b scales, half as wide: 64 x 64 per wave
 
 using GroupedTeams = PingPongShape<2, 2, 2, 2, 4>;                           // row-wise, 128 x 128, two teams that share the k range
 
@@ -48,10 +52,14 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     constexpr int TM = S::TM, TN = S::TN, STAGES = S::STAGES, RING = STAGES * S::STAGE;
     // A scale block is 8 K groups in 16-byte pieces of 4: [half][row of a], then [half][row of b], or with uniform b scales
     // [half][sub-tile of b] (what 64 lanes of one load instruction bring)
+    // Chunks of 128 k (OWN) bring their 4 K groups themselves: a block of [row of a], then [sub-tile of b] per stage.
+    constexpr int KG = S::CHUNK / 32;
+    constexpr bool OWN = KG == 4;
     constexpr int B_ENTRIES = ROWS ? S::COLS : S::COLS / 32;
-    constexpr int A_SCALES = 2 * S::ROWS * 16, B_SCALES = ROWS ? 2 * B_ENTRIES * 16 : 1024, SCALE_BLOCK = A_SCALES + B_SCALES;
-    constexpr int TEAM_LDS = RING + 2 * SCALE_BLOCK;
-    static_assert(2 * S::ROWS == S::THREADS && (ROWS || 2 * B_ENTRIES <= 64) && 2 * SCALE_BLOCK >= S::COLS * 4);
+    constexpr int A_SCALES = (OWN ? 1 : 2) * S::ROWS * 16, B_SCALES = ROWS ? 2 * B_ENTRIES * 16 : 1024, SCALE_BLOCK = A_SCALES + B_SCALES;
+    constexpr int SCALE_BUFFERS = OWN ? STAGES : 2, TEAM_LDS = RING + SCALE_BUFFERS * SCALE_BLOCK;
+    static_assert(2 * S::ROWS == S::THREADS && (ROWS || 2 * B_ENTRIES <= 64) && SCALE_BUFFERS * SCALE_BLOCK >= S::COLS * 4);
+    static_assert(KG == 2 || (OWN && !ROWS && S::TEAMS == 1));
     __shared__ __attribute__((aligned(1024))) uint8_t lds_all[S::TEAMS * TEAM_LDS];
     // tid, wave and lds are the team's own
     const int team = S::TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / S::THREADS) : 0;
@@ -117,7 +125,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     if constexpr (S::TEAMS > 1) {
         constexpr int64_t CUT = F_SGROUPS * 32;                              // a scale block belongs to one team
         const int64_t len = k_end - k_begin, half = ((len + CUT - 1) / CUT + 1) / 2 * CUT, first = half < len ? half : len;
-        split_chunks = (int)((first + FBK - 1) / FBK);
+        split_chunks = (int)((first + S::CHUNK - 1) / S::CHUNK);
         if (team == 0) k_end = k_begin + first;
         else k_begin += first;
     }
@@ -127,14 +135,15 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     const i32x4 res_a = raw_resource(p.a + m_begin * p.lda + k_begin), res_b = raw_resource(bptr + k_begin);
     constexpr uint32_t OUTSIDE = 0x80000000u;
     // (both teams walk the first half's chunks, they share the barriers: past its own range a team loads zero codes)
-    const int chunks = S::TEAMS > 1 ? split_chunks : (int)((k_len + FBK - 1) / FBK), full_chunks = (int)(k_len / FBK), groups_total = (int)((k_len + 31) / 32);
-    const int piece = (tid & 3) ^ ((tid >> 4) & 3);
-    const bool inside_tail = (int64_t)full_chunks * FBK + piece * 16 < k_len;
+    const int chunks = S::TEAMS > 1 ? split_chunks : (int)((k_len + S::CHUNK - 1) / S::CHUNK), full_chunks = (int)(k_len / S::CHUNK), groups_total = (int)((k_len + 31) / 32);
+    auto swizzle = [](int row) -> int { return S::PIECES == 4 ? (row >> 2) & 3 : (row >> 1) & 7; };
+    const int piece = tid % S::PIECES ^ swizzle(tid / S::PIECES);
+    const bool inside_tail = (int64_t)full_chunks * S::CHUNK + piece * 16 < k_len;
     auto row_in = [](int64_t row, int64_t rows) -> uint32_t { return (uint32_t)(row < rows ? row : rows - 1); };
     uint32_t cur[S::LOADS];
 #pragma unroll
     for (int it = 0; it < S::LOADS; ++it) {
-        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * S::LOAD_ROWS + tid / 4;
+        const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * S::LOAD_ROWS + tid / S::PIECES;
         if (it < S::A_LOADS) cur[it] = (uint32_t)(row_in(m_begin + r, m_end) - m_begin) * (uint32_t)p.lda;
         else cur[it] = row_in(n_begin + r, p.n) * (uint32_t)p.ldb;
         asm volatile("" : "+v"(cur[it]));                                    // (as one 64-bit multiply-add it would hold a register pair all along)
@@ -148,27 +157,34 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
 #pragma unroll
             for (int it = 0; it < S::LOADS; ++it) {
                 const uint32_t at = here ? cur[it] : OUTSIDE;
-                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * S::THREADS * 16 + (uint32_t)wave * 1024, at, (uint32_t)c * FBK);
+                load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * S::THREADS * 16 + (uint32_t)wave * 1024, at, (uint32_t)c * S::CHUNK);
             }
             return;
         }
 #pragma unroll
         for (int it = 0; it < S::LOADS; ++it)
-            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * S::THREADS * 16 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * FBK);
+            load16_to_lds(it < S::A_LOADS ? res_a : res_b, lds_base + (uint32_t)stage * S::STAGE + it * S::THREADS * 16 + (uint32_t)wave * 1024, cur[it], (uint32_t)c * S::CHUNK);
     };
     // Scale block `block` -> buffer block & 1: every thread one piece of the a rows, the first waves one of b (lanes past b's last
     // entry read zero). Entries past the end of the k range, which hold whatever follows in memory (see group_gemm_fast), are
     // cleared once in LDS.
     const i32x4 res_sa = raw_resource(p.sa, p.sa_bytes), res_sb = raw_resource(sbptr, p.sb_bytes);
-    const int a_half = wave * WAVE / S::ROWS, b_half = ROWS ? wave * WAVE / B_ENTRIES : lane / B_ENTRIES;
+    const int a_half = OWN ? 0 : wave * WAVE / S::ROWS, b_half = ROWS ? wave * WAVE / B_ENTRIES : lane / B_ENTRIES;
     const uint32_t group0 = (uint32_t)(k_begin >> 5) * 4;
     uint32_t sa_at = row_in(m_begin + tid % S::ROWS, m_end) / (uint32_t)p.ar * (uint32_t)p.ldsa * 4 + group0 + a_half * 16;
     uint32_t sb_at = row_in(n_begin + tid % B_ENTRIES * (ROWS ? 1 : 32), p.n) / (uint32_t)p.br * (uint32_t)p.ldsb * 4 + group0 + b_half * 16;
-    if (b_half >= 2) sb_at = OUTSIDE;
+    if (b_half >= (OWN ? 1 : 2)) sb_at = OUTSIDE;
     asm volatile("" : "+v"(sa_at), "+v"(sb_at));
     const int last_block = (groups_total - 1) / F_SGROUPS;
     // (past the last block: that one again, to keep the load counts uniform; a team that walks on past its own range reads zeros)
     auto issue_scales = [&](int block) {
+        if constexpr (OWN) {                                                 // waves 0-3: a; each of the others b, so that all have the same count
+            const bool first = wave * WAVE < S::ROWS;
+            const uint32_t to = lds_base + RING + (uint32_t)(block % STAGES) * SCALE_BLOCK + (first ? (uint32_t)wave * 1024 : A_SCALES);
+            const uint32_t at = first ? sa_at : sb_at;
+            load16_to_lds(first ? res_sa : res_sb, to, block < chunks ? at : OUTSIDE, (uint32_t)block * 16);
+            return;
+        }
         const uint32_t to = lds_base + RING + (uint32_t)(block & 1) * SCALE_BLOCK + (uint32_t)wave * 1024;
         const uint32_t first = (uint32_t)(block < last_block ? block : last_block) * F_SGROUPS * 4;
         const bool past = S::TEAMS > 1 && block > last_block;
@@ -187,8 +203,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     };
 
     // ---- operands: a lane's 16 bytes of K group kg of its row in every sub-tile, and the scales
-    const int sw = (l32 >> 2) & 3;
-    const int rd_a = (wm * TM * 32 + l32) * FBK + ((lhi ^ sw) * 16), rd_b = S::A_BYTES + (wn * TN * 32 + l32) * FBK + ((lhi ^ sw) * 16);
+    const int sw = swizzle(l32);
+    const int rd_a = (wm * TM * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16), rd_b = S::A_BYTES + (wn * TN * 32 + l32) * S::CHUNK + ((lhi ^ sw) * 16);
     f32x16 total[TN][TM];
 #pragma unroll
     for (int i = 0; i < TN; ++i)
@@ -196,22 +212,31 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
         for (int j = 0; j < TM; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) total[i][j][r] = 0.0f;
-    i32x4 oa[FKG][TM], ob[FKG][TN];
+    i32x4 oa[KG][TM], ob[KG][TN];
     // sa[j]: of the lane's row in sub-tile j; ROWS: sa[0] of row `lane` of the wave's 64, the operand of the scale products
     constexpr int SA = ROWS ? 1 : TM;
-    float sa[SA][FKG], sb[TN][FKG];
+    float sa[SA][KG], sb[TN][KG];
+    float4 va[SA], vb[TN];
     auto read = [&](int stage, int c) {
         // (addresses of K group 1 made here from those of K group 0: kept over the loop they would take two registers too many)
         int at_a = stage * S::STAGE + rd_a, at_b = stage * S::STAGE + rd_b;
         asm volatile("" : "+v"(at_a), "+v"(at_b));
 #pragma unroll
-        for (int kg = 0; kg < FKG; ++kg) {
+        for (int kg = 0; kg < KG; ++kg) {
 #pragma unroll
-            for (int i = 0; i < TN; ++i) ob[kg][i] = *reinterpret_cast<const i32x4*>(lds + (at_b ^ (kg * 32)) + i * 32 * FBK);
+            for (int i = 0; i < TN; ++i) ob[kg][i] = *reinterpret_cast<const i32x4*>(lds + (at_b ^ (kg * 32)) + i * 32 * S::CHUNK);
 #pragma unroll
-            for (int j = 0; j < TM; ++j) oa[kg][j] = *reinterpret_cast<const i32x4*>(lds + (at_a ^ (kg * 32)) + j * 32 * FBK);
+            for (int j = 0; j < TM; ++j) oa[kg][j] = *reinterpret_cast<const i32x4*>(lds + (at_a ^ (kg * 32)) + j * 32 * S::CHUNK);
         }
-        const int g8 = c % F_SCHUNKS * FKG;                                  // group of the block (even: both groups of the chunk in one read)
+        if constexpr (OWN) {
+            const float* block = reinterpret_cast<const float*>(lds + RING + stage * SCALE_BLOCK);
+#pragma unroll
+            for (int j = 0; j < SA; ++j) va[j] = *reinterpret_cast<const float4*>(&block[(wm * TM * 32 + j * 32 + l32) * 4]);
+#pragma unroll
+            for (int i = 0; i < TN; ++i) vb[i] = *reinterpret_cast<const float4*>(&block[A_SCALES / 4 + (wn * TN + i) * 4]);
+            return;
+        }
+        const int g8 = c % F_SCHUNKS * KG;                                  // group of the block (even: both groups of the chunk in one read)
         const float* block = reinterpret_cast<const float*>(lds + RING + ((c / F_SCHUNKS) & 1) * SCALE_BLOCK);
 #pragma unroll
         for (int j = 0; j < SA; ++j) {
@@ -227,9 +252,28 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
             sb[i][1] = ROWS ? v.y : __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v.y)));
         }
     };
+    // OWN: the scales of the chunk out of the pieces read. Past the end of k these hold whatever follows in memory, and the codes are zero.
+    auto take_scales = [&](int c) {
+        const int left = groups_total - c * KG;
+#pragma unroll
+        for (int j = 0; j < SA; ++j) asm volatile("" : "+v"(va[j].x), "+v"(va[j].y), "+v"(va[j].z), "+v"(va[j].w));
+#pragma unroll
+        for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(vb[i].x), "+v"(vb[i].y), "+v"(vb[i].z), "+v"(vb[i].w));
+#pragma unroll
+        for (int kg = 0; kg < KG; ++kg) {
+            const bool in = kg < left;
+#pragma unroll
+            for (int j = 0; j < SA; ++j) sa[j][kg] = in ? (&va[j].x)[kg] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const float v = in ? (&vb[i].x)[kg] : 0.0f;
+                sb[i][kg] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+            }
+        }
+    };
     auto pin_operands = [&] {                                                // in registers before the barrier
 #pragma unroll
-        for (int kg = 0; kg < FKG; ++kg) {
+        for (int kg = 0; kg < KG; ++kg) {
 #pragma unroll
             for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(oa[kg][j]));
 #pragma unroll
@@ -256,7 +300,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[x][r] = 0.0f;
     // uniform b scales: units in the order (kg, i, j), unit u in accumulator u % 3
-    constexpr int UNITS = FKG * TN * TM, LAG = 2;
+    constexpr int UNITS = KG * TN * TM, LAG = 2;
     float scale[ACCS] = {};
     auto fold_unit = [&](int u, int first, int count) {
         const int i = u / TM % TN, j = u % TM, x = u % ACCS;
@@ -264,7 +308,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
         for (int r = first; r < first + count; ++r) total[i][j][r] = fmaf(acc[x][r], scale[x], total[i][j][r]);
     };
     // row-wise: pairs of units (kg, i, j = 0 and 1), pair q in accumulators 2 (q & 1) + j, its scale products in prod[q & 1]
-    constexpr int PAIRS = FKG * TN;
+    constexpr int PAIRS = KG * TN;
     f32x32 prod[ROWS ? 2 : 1];
     if constexpr (ROWS) {
 #pragma unroll
@@ -340,17 +384,21 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     // buffer that block b - 1 left a chunk ago (its last readers, waves 4-7, had it in registers before the barrier that ended
     // their read phase); it has landed when the read phase of chunk 4 b + 1 ends and is first read in chunk 4 b + 4, with the
     // straddling piece cleared in chunk 4 b + 2.
-    constexpr int AHEAD = (STAGES - 2) * S::LOADS;
+    // (Chunks with scales of their own: these are one load more of the chunk.)
+    constexpr int AHEAD = (STAGES - 2) * (S::LOADS + (OWN ? 1 : 0));
     static_assert(AHEAD + 1 < 16 && STAGES >= 3);
-    issue_scales(0);
+    if (!OWN) issue_scales(0);
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
+    for (int s = 0; s < STAGES - 1; ++s) {
+        if (OWN) issue_scales(s);
+        issue(s, s);
+    }
     __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);                              // chunk 0 and scale block 0
     barrier();
     if (S::TEAMS > 1) {                                                      // the condition differs between the teams, the barrier must not
         if (last_block == 0 && straddles) clear_past_the_end();
         __syncthreads();
-    } else if (last_block == 0 && straddles) {
+    } else if (!OWN && last_block == 0 && straddles) {
         clear_past_the_end();
         __syncthreads();
     }
@@ -359,9 +407,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     int stage = 0, fill = STAGES - 1;
     for (int c = 0; c < chunks; ++c) {
         read(stage, c);
-        const bool scales_now = c % F_SCHUNKS == 0;
+        const bool scales_now = !OWN && c % F_SCHUNKS == 0;
         if (scales_now) issue_scales(c / F_SCHUNKS + 1);
-        if (c % F_SCHUNKS == 2 && c / F_SCHUNKS + 1 == last_block && straddles) clear_past_the_end();
+        if (!OWN && c % F_SCHUNKS == 2 && c / F_SCHUNKS + 1 == last_block && straddles) clear_past_the_end();
+        if (OWN) issue_scales(c + STAGES - 1);
         issue(c + STAGES - 1, fill);
         stage = stage == STAGES - 1 ? 0 : stage + 1;
         fill = fill == STAGES - 1 ? 0 : fill + 1;
@@ -369,6 +418,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
         if constexpr (!ROWS) {
             drain();
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (OWN) take_scales(c);
         }
         if (scales_now) __builtin_amdgcn_s_waitcnt(0x0070 | (AHEAD + 1));   // (the scale block just issued is among the newest)
         else __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
@@ -412,7 +462,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
             }
         __syncthreads();
     }
-    float* bias_lds = reinterpret_cast<float*>(lds_all + S::TEAMS * TEAM_LDS - 2 * SCALE_BLOCK);
+    float* bias_lds = reinterpret_cast<float*>(lds_all + S::TEAMS * TEAM_LDS - SCALE_BUFFERS * SCALE_BLOCK);
     stage_bias<S>(p, n_begin, bias_lds, bias_dtype);
     auto finish = [&](auto type) {
         using TO = decltype(type);
