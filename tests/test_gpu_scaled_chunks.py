@@ -13,7 +13,8 @@ E4, E5 = torch.float8_e4m3fn, torch.float8_e5m2
 @pytest.mark.parametrize("scaling", ["tensor", "mx"])
 @pytest.mark.parametrize("m,n,k,formats", [(4096, 1152, 1296, (E4, E4)), (4090, 1150, 1360, (E5, E4)), (4096, 1152, 128, (E4, E5)), (4000, 1100, 256, (E4, E4)),
                                            (2048, 1152, 4624, (E4, E4)), (2000, 1030, 2064, (E5, E5)), (1920, 1920, 640, (E4, E4)), (1921, 1919, 80, (E4, E4)),
-                                           (4096, 4096, 1104, (E4, E5)), (4090, 4000, 2128, (E4, E4)), (4000, 4090, 4608, (E5, E5)), (4096, 4096, 384, (E4, E4))])
+                                           (4096, 4096, 1104, (E4, E5)), (4090, 4000, 2128, (E4, E4)), (4000, 4090, 4608, (E5, E5)), (4096, 4096, 384, (E4, E4)),
+                                           (9200, 1150, 2064, (E4, E4)), (1152, 9216, 4160, (E5, E4))])
 def test_products_in_chunks_of_128(m, n, k, formats, scaling):
     from viola_amd.nn import _grouped_kernels as g, _linear_kernels as lk
     if scaling == "mx":

@@ -336,7 +336,9 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
 // cycles beside the math (barriers, the first LDS reads), which is a lot next to the 256 or 512 cycles of a wave's four or eight
 // MFMAs: where registers and LDS allow it a chunk is 128 k (whole cache lines of the operands, too). 256 x 256, in two stages for
 // want of LDS: 4096 x 4096 x 4096 61 -> 55 us (E8M0 64 -> 57), 16384 x 4096 x 11008 547 -> 509, 8192 x 8192 x 8192 394 -> 387 (the
-// power limit), even up to k = 1024 and where CUs are idle. 256 x 128: 4096 x 1152 x 9216 61 -> 47 us,
+// power limit), even up to k = 1024. (Four stages of
+// 64 k are on their way for longer, and faster at 180 tiles on warm operands, 9216 x 1152 x 4096 54 -> 48 us, but not behind the
+// quantizers of a step: 54.8 against 55.3.) 256 x 128: 4096 x 1152 x 9216 61 -> 47 us,
 // 8192 x 1024 x 4096 36 -> 30, 4096 x 1152 x 4608 33 -> 26 (E8M0 35 -> 30); 128 x 128 alone on its CU: 2048 x 1152 x 4608 22 -> 19.
 // (96- and 192-column tiles, which leave fewer CUs idle at widths like 1152, gain nothing: a smaller tile's turn takes as long.)
 using PingPongL = PingPongShape<2, 4, 4, 2, 2, 128>;
