@@ -151,8 +151,9 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     if constexpr (MX) {
         scale_at = tid < S::ROWS ? row_in(m_begin + tid, p.m) / (uint32_t)p.ar * (uint32_t)p.ldsa : b_row(tid - S::ROWS) / (uint32_t)p.br * (uint32_t)p.ldsb;
     }
+    const bool scale_wave = wave * 64 < S::ROWS + S::B_ROWS;
     auto issue_scales = [&](int block) {
-        if (wave * 64 >= S::ROWS + S::B_ROWS) return;
+        if (!scale_wave) return;
         const uint32_t to = lds_base + RING + (uint32_t)(block & 1) * SCALE_BLOCK + (uint32_t)wave * 1024;
         load16_to_lds(wave * 64 < S::ROWS ? res_sa : res_sb, to, block * MX_GROUPS < groups_total ? scale_at : OUTSIDE, (uint32_t)(block * MX_GROUPS));
     };
@@ -243,8 +244,9 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     // Phases. Waves 0-3 read chunk c in phase 2c and multiply in phase 2c + 1, waves 4-7 one phase later. The loads of chunk
     // c + STAGES - 1 go out in the read phase of chunk c, into the stage of chunk c - 1: its last readers (waves 4-7, phase
     // 2c - 1) had their operands in registers before the barrier that ended that phase. Every wave ends its read phase of
-    // chunk c with its own loads of chunk c + 1 landed (at most those of the STAGES - 2 chunks after it in flight; a scale
-    // block among them only makes the wait stricter), and chunk c + 1 is first read two barriers later.
+    // chunk c with its own loads of chunk c + 1 landed (at most those of the STAGES - 2 chunks after it in flight, and a
+    // scale block issued in this phase: waiting for that as well, 4096 x 1152 x 9216 and x 4608 took 105.9 us
+    // behind the quantizers of a step where they take 103.1), and chunk c + 1 is first read two barriers later.
     // Two stages: chunk c + 1 goes out in phase 2c, once waves 4-7 have read chunk c - 1 (waves 0-3 issue it in their read phase of
     // chunk c, waves 4-7 in their math phase of chunk c - 1), and every wave waits for its part before the barrier that ends phase
     // 2c + 1 (waves 0-3 behind their math, waves 4-7 behind their reads of chunk c).
@@ -271,7 +273,8 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
         if (!TWO || !late) issue_next(c + STAGES - 1);
         stage = stage == STAGES - 1 ? 0 : stage + 1;
         __builtin_amdgcn_sched_barrier(0);
-        if (!TWO || late) __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
+        if (MX && !TWO && c % SCALE_CHUNKS == 0 && scale_wave) __builtin_amdgcn_s_waitcnt(0x0070 | (AHEAD + 1));
+        else if (!TWO || late) __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
         else __builtin_amdgcn_s_waitcnt(0xC07F);                             // the LDS reads alone
         pin_operands();
         barrier();
