@@ -32,7 +32,7 @@ PEAK = {"fp8_tflops": 5000.0, "bf16_tflops": 2500.0, "hbm_gbs": 8000.0}
 # `rocprofv3 --pmc` runs of `bench.py --skip-cpu --skip-muon --steps 5 --warmup 3 --calibrate` (FETCH_SIZE, then WRITE_SIZE, KiB per
 # dispatch), each scaled by the same counter's reading for the 256 MiB copy_scaled_kernel launch (factors 2.00 and 1.00):
 # fetch (2 * 58.3 + 113.5) / 3 MB, write (2 * 41.9 + 8.4) / 3 MB. The algorithmic figure is 65 MB per launch.
-GEMM_TRAFFIC_BYTES = 76.7e6 + 30.8e6
+GEMM_TRAFFIC_BYTES = 76.6e6 + 30.8e6
 WARM_MS = 100.0
 
 
@@ -303,7 +303,7 @@ def main():
     breakdown = kernel_breakdown(step, args.steps)
     gemm = breakdown["viola_group_gemm"]
     gemm_tflops = 2 * M * K * N / (gemm["avg_ms"] * 1e-3) / 1e12
-    roofline = dict(bound="mfma", kernel="group_gemm_fast (viola_group_gemm: fwd, dgrad, wgrad)",
+    roofline = dict(bound="mfma", kernel="gemm_pingpong_grouped (viola_group_gemm: fwd, dgrad, wgrad)",
                     achieved=gemm_tflops, peak=PEAK["fp8_tflops"], unit="TFLOP/s", frac=gemm_tflops / PEAK["fp8_tflops"],
                     avg_launch_ms=gemm["avg_ms"], traffic=GEMM_TRAFFIC_BYTES,
                     traffic_source="stored calibration (two rocprofv3 --pmc runs, profiles/linear_step_8192x1024x4096_hbm_traffic.txt), not read in this run")
