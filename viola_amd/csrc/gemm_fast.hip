@@ -89,27 +89,38 @@ static bool prefer_tall(const GemmArgs& p) {
 
 // In how many parts of k a weight gradient runs, which has few tiles and a long k. Whole, 129 to 256 tiles of 128 x 128 leave CUs
 // without a tile, and fewer run as narrow tiles, which read more per product; in parts, tiles of 256 x 128 fill the chip and a second
-// launch adds the partial products. The least of the estimates in microseconds (fitted to 24 shapes) decides, and only where it
-// saves a twentieth: 3072 x 768 x 9856 82 -> 65 us in three, 1024 x 1024 x 16384 90 -> 49 in eight, 2048 x 1024 x 8192 56 -> 50 in four,
-// 512 x 512 x 16384 89 -> 28 in 24; 4096 x 1024 x 8192 stays whole (74 us, 83 in two), so does 1024 x 1024 x 4096 (26.6 us, 28.0 in seven).
+// launch adds the partial products, a few hundred cycles per part on top of their bytes. The least of the estimates in microseconds
+// decides, and only where it saves a twentieth. Fitted to 56 shapes, whole and in up to 20 counts of parts (whole within 7 %, the counts
+// that come near the best within 5 % on average); what it takes is within 8 % of the fastest count of each:
+//   3072 x 768 x 9856 82 -> 64 us in three    1024 x 1024 x 16384 89 -> 50 in eight    512 x 512 x 16384 88 -> 28 in 20
+//   256 x 256 x 16384 83 -> 24 in 32          1000 x 332 x 3200 22.5 -> 20.5 in ten    1152 x 1152 x 16384 90 -> 66 in five
+// It stays whole where parts gain nothing, 4096 x 1024 x 8192 (75 us, 84 in two) and 1024 x 1024 x 4096 (26.7 us, 28.6 in seven), and where
+// they gain less than the estimate can tell, 2048 x 1024 x 8192 (52.7 us, 50.3 in four).
 int plan_k_parts(int64_t m, int64_t n, int64_t k) {
     constexpr double CUS = 256.0;
     if (k < 1024 || m < 64 || n < 64 || n % 4 != 0) return 1;               // (rows of the partial products in whole 16-byte pieces)
-    const double chunks = (double)k / 64.0, small = (double)((m + 127) / 128) * (double)((n + 127) / 128), large = (double)((m + 255) / 256) * (double)((n + 127) / 128);
-    // whole, as launch_group_gemm_fast runs it
-    const double pairs = floor(small / (2 * CUS)), left = small - pairs * 2 * CUS;
-    double least = small <= CUS / 2 ? chunks * (0.33 + 0.09 * small / 128.0) + 3.3 : small <= CUS ? chunks * (0.45 + 0.1 * small / CUS) + 4.0
-                   : pairs * (chunks * 1.2 + 3.3) + (left > 0 ? chunks * 1.2 * (left <= CUS ? 0.52 : 1.0) + 3.3 : 0.0);
-    auto tiles_of = [&](double count, double length, double ends) {
+    const int64_t all = (k + FBK - 1) / FBK;
+    const double chunks = (double)all, small = (double)((m + 127) / 128) * (double)((n + 127) / 128), large = (double)((m + 255) / 256) * (double)((n + 127) / 128);
+    auto tiles_of = [&](double count, double length) {
         const double rounds = floor(count / CUS), rest = count / CUS - rounds;
-        return rounds * (length * 1.04 + ends) + (rest > 0 ? length * (0.82 + 0.22 * rest) + ends : 0.0);
+        return rounds * (length * 0.95 + 4.3) + (rest > 0 ? length * (0.77 + 0.18 * rest) + 4.3 : 0.0);
     };
-    if (small > CUS) least = least < tiles_of(large, chunks, 6.0) ? least : tiles_of(large, chunks, 6.0);
+    // whole, as launch_group_gemm_fast runs it
+    double least;
+    if (small <= CUS / 2) least = chunks * (0.32 + 0.05 * small / 128.0) + 4.5;
+    else if (small <= CUS) least = chunks * (0.35 + 0.18 * small / CUS) + 7.0;
+    else {
+        const double pairs = floor(small / (2 * CUS)), left = small - pairs * 2 * CUS, wide = tiles_of(large, chunks);
+        least = pairs * (chunks * 1.15 + 3.3) + (left > 0 ? chunks * 1.15 * (left <= CUS ? 0.52 : 1.0) + 3.3 : 0.0);
+        if (wide < least) least = wide;
+    }
+    least *= 0.95;
     int best = 1;
-    for (int parts = 2; parts <= 64 && chunks / parts >= 4.0; ++parts) {
-        const double sum = 5.0 + (double)m * n * (4.0 * parts + 2.0) / 4.3e6;
-        const double time = tiles_of(large * parts, ceil(chunks / parts), 7.5) + sum;
-        if (time < 0.95 * least) { least = time / 0.95; best = parts; }
+    for (int64_t parts = 2; parts <= 64 && all / parts >= 4; ++parts) {
+        const int64_t length = (all + parts - 1) / parts;
+        if ((all + length - 1) / length != parts) continue;                  // the last ones would be empty: the same as fewer
+        const double time = tiles_of(large * parts, (double)length) + 5.6 + 0.155 * parts + (double)m * n * (4.0 * parts + 2.0) / 4.1e6;
+        if (time < least) { least = time; best = (int)parts; }
     }
     return best;
 }
