@@ -218,8 +218,9 @@ int viola_group_gemm(const void* a, int a_dtype, const void* b, int b_dtype, con
 
 /* The same with a scale per row and 32 k on both sides (ar = br = 1, ak = bk = 32), no bias, the k range cut into `parts` (2 .. 64)
  * that are computed side by side: their FP32 products go to workspace (parts * (m * n rounded up to 4) floats, 16-byte aligned) and
- * are added in ascending order. viola_group_gemm_parts says how many are worth it (1: viola_group_gemm). VIOLA_EUNSUPPORTED, with
- * nothing launched, where k % 16 != 0, the operands are not 16-byte aligned or beyond 2 GiB. */
+ * are added in ascending order. viola_group_gemm_parts says how many are worth it (1: viola_group_gemm): never so many that the
+ * workspace would exceed 96 MiB, and 1 for sizes that are not taken. VIOLA_EUNSUPPORTED, with nothing launched, where k % 16 != 0,
+ * the operands are not 16-byte aligned or beyond 2 GiB. */
 int viola_group_gemm_parts(int64_t m, int64_t n, int64_t k);
 int viola_group_gemm_in_parts(const void* a, int a_dtype, const void* b, int b_dtype, const float* sa, const float* sb, int64_t m, int64_t n,
                               int64_t k, void* out, int out_dtype, int parts, float* workspace, int64_t workspace_floats, viola_stream_t stream);

@@ -30,3 +30,23 @@ def test_no_part_is_empty():
 def test_products_that_gain_nothing_stay_whole():
     for shape in ((1024, 1024, 1008), (63, 4096, 8192), (4096, 60, 8192), (512, 514, 8192), (0, 64, 8192), (64, 64, 0), (8192, 8192, 8192)):
         assert parts(*shape) == 1, shape
+
+
+def test_partial_products_stay_within_their_bound():
+    """At most 96 MiB of scratch, at most 34 MB up to 256 tiles of 128 x 128 and 16384 tokens."""
+    from itertools import product
+    widths = (64, 256, 512, 768, 1000, 1536, 2304, 3072, 3584, 4352, 5248, 7680, 8192)
+    largest = few = 0
+    for m, n, k in product(widths, widths, (1024, 3072, 8192, 9856, 15936, 16384, 65536)):
+        count = parts(m, n, k)
+        scratch = 0 if count == 1 else count * m * n * 4
+        largest = max(largest, scratch)
+        if -(-m // 128) * -(-n // 128) <= 256 and k <= 16384:
+            few = max(few, scratch)
+    assert 64 << 20 < largest <= 96 << 20 and few <= 34e6
+    assert parts(3072, 3072, 16384) == 2 and parts(4352, 4224, 16128) == parts(3584, 5248, 16384) == parts(7680, 2304, 15936) == 1
+
+
+def test_sizes_that_the_product_in_parts_refuses_are_whole():
+    for shape in ((512, 512, 1 << 23), (768, 512, 1 << 22), (1 << 40, 1 << 40, 8192), (512, 1 << 62, 8192), (512, 512, 1 << 62)):
+        assert parts(*shape) == 1, shape

@@ -51,14 +51,14 @@ extern "C" int viola_group_gemm(const void* a, int a_dtype, const void* b, int b
 }
 
 // (what the fast kernel asks of a product with a scale per row and 32 k on both sides, plus what 256 rows of a large tile do)
-static bool parts_take(const void* a, const void* b, int64_t m, int64_t n, int64_t k) {
+static bool parts_fit(int64_t m, int64_t n, int64_t k) {
     const int64_t rows = m > n ? m : n;
-    return k % 16 == 0 && aligned16(a) && aligned16(b) && rows * k < (1ll << 31) && 256 * k < (1ll << 31) && rows * ((k + 31) / 32) * 4 < (1ll << 31) &&
-           m * n < (1ll << 31);
+    return rows * k < (1ll << 31) && 256 * k < (1ll << 31) && rows * ((k + 31) / 32) * 4 < (1ll << 31) && m * n < (1ll << 31);
 }
 
 extern "C" int viola_group_gemm_parts(int64_t m, int64_t n, int64_t k) {
-    if (m <= 0 || n <= 0 || k <= 0 || m * n >= (1ll << 31)) return 1;
+    constexpr int64_t LARGEST = 1ll << 31;
+    if (m <= 0 || n <= 0 || k <= 0 || m >= LARGEST || n >= LARGEST || k >= LARGEST || !parts_fit(m, n, k)) return 1;
     return plan_k_parts(m, n, k);
 }
 
@@ -69,7 +69,7 @@ extern "C" int viola_group_gemm_in_parts(const void* a, int a_dtype, const void*
     VIOLA_CHECK_ARG(m >= 0 && n >= 0 && k > 0 && parts >= 2 && parts <= 64 && workspace && aligned16(workspace));
     if (m == 0 || n == 0) return 0;
     VIOLA_CHECK_ARG(a && b && sa && sb && out);
-    if (!parts_take(a, b, m, n, k)) return VIOLA_EUNSUPPORTED;
+    if (k % 16 != 0 || !aligned16(a) || !aligned16(b) || !parts_fit(m, n, k)) return VIOLA_EUNSUPPORTED;
     VIOLA_CHECK_ARG(workspace_floats >= parts * ((m * n + 3) / 4 * 4));
     GemmArgs p = {};
     p.a = static_cast<const uint8_t*>(a); p.b = static_cast<const uint8_t*>(b); p.sa = sa; p.sb = sb;

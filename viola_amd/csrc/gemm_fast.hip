@@ -96,6 +96,11 @@ static bool prefer_tall(const GemmArgs& p) {
 //   256 x 256 x 16384 83 -> 24 in 32          1000 x 332 x 3200 22.5 -> 20.5 in ten    1152 x 1152 x 16384 90 -> 66 in five
 // It stays whole where parts gain nothing, 4096 x 1024 x 8192 (75 us, 84 in two) and 1024 x 1024 x 4096 (26.7 us, 28.6 in seven), and where
 // they gain less than the estimate can tell, 2048 x 1024 x 8192 (52.7 us, 50.3 in four).
+// The partial products are scratch that a whole product does not need, in a pass that may be short of memory: at most PARTS_SCRATCH
+// bytes. Up to 256 tiles of 128 x 128 and 16384 tokens no count that is taken needs more than 34 MB. Beyond, whole products fill the
+// chip, and the 140 to 230 MB of larger ones, which gained 6 to 8 %, are not spent (4352 x 4224 x 16128 734 -> 681 us in two, 147 MB;
+// 3072 x 3072 x 16384 455 -> 375 in four, 151 MB, but 400 in two, 75 MB, which it takes).
+constexpr int64_t PARTS_SCRATCH = 96ll << 20;
 int plan_k_parts(int64_t m, int64_t n, int64_t k) {
     constexpr double CUS = 256.0;
     if (k < 1024 || m < 64 || n < 64 || n % 4 != 0) return 1;               // (rows of the partial products in whole 16-byte pieces)
@@ -116,7 +121,7 @@ int plan_k_parts(int64_t m, int64_t n, int64_t k) {
     }
     least *= 0.95;
     int best = 1;
-    for (int64_t parts = 2; parts <= 64 && all / parts >= 4; ++parts) {
+    for (int64_t parts = 2; parts <= 64 && all / parts >= 4 && parts * ((m * n + 3) / 4 * 16) <= PARTS_SCRATCH; ++parts) {
         const int64_t length = (all + parts - 1) / parts;
         if ((all + length - 1) / length != parts) continue;                  // the last ones would be empty: the same as fewer
         const double time = tiles_of(large * parts, (double)length) + 5.6 + 0.155 * parts + (double)m * n * (4.0 * parts + 2.0) / 4.1e6;
