@@ -169,7 +169,8 @@ def test_product_in_parts_of_k(m, n, k, parts, out_dtype):
 
 
 def test_linear_weight_gradient_in_parts_against_float64():
-    """A shape the module runs in parts: no further from the float64 product of the very codes than the whole product is."""
+    """The C entry point at a shape that the modules run in parts: no further from the float64 product of the very codes than the whole
+    product is."""
     from viola_amd.nn import _grouped_kernels as g
     torch.manual_seed(1)
     m, n, k = 768, 512, 8192
