@@ -140,3 +140,23 @@ def test_saved_codes_that_come_back_out_of_alignment():
     _, calls = _names(lambda: y.backward(dy))
     assert calls.index(IN_PARTS) == calls.index("viola_group_gemm", calls.index(IN_PARTS)) - 1
     assert not torch.equal(other.weight.grad, layer.weight.grad) and rel_l2(other.weight.grad, layer.weight.grad) < SUMS
+
+
+@pytest.mark.parametrize("tokens", [8192, 8208, 2064])
+def test_general_path_adds_in_the_same_order(tokens):
+    """A call that the native host path hands on (here for a weight with strided rows) cuts k at the same places and gives
+    the same bits where the token count is whole pieces of 16."""
+    x, dy = _values(tokens, 512, 768)
+    x.requires_grad_()
+    results = []
+    for strided in (False, True):
+        layer = _linear(512, 768)
+        if strided:
+            layer.weight.data = layer.weight.data.t().contiguous().t()
+        x.grad = None
+        _, calls = _names(lambda: layer(x).backward(dy))
+        results.append((layer.weight.grad, x.grad, layer.bias.grad, calls))
+    (dw, dx, db, native), (dw2, dx2, db2, general) = results
+    assert "viola_group_gemm" in general and ("viola_codes_transpose_pitched" in native) and ("viola_codes_transpose_pitched" not in general)
+    assert native.count(IN_PARTS) == general.count(IN_PARTS) == (tokens > 4096)
+    assert torch.equal(dw, dw2) and torch.equal(dx, dx2) and torch.equal(db, db2)

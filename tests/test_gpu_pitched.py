@@ -199,7 +199,8 @@ def test_variable_groups_on_sizes_that_are_multiples_of_nothing(bf16_gradients, 
 @pytest.mark.parametrize("tokens,n_in,n_out", [(500, 512, 512), (1001, 1024, 1024), (3001, 1024, 1024), (2049, 512, 512), (1533, 256, 300)])
 def test_step_behind_a_ragged_token_count_differs_by_the_order_of_the_sums(bf16_gradients, tokens, n_in, n_out):
     """A padded pitch takes the weight gradient off the guarded kernel, which adds the 32-k groups in ascending order, to kernels
-    that for few tiles and k >= 1024 add two halves of the k range separately. Below that nothing changes. Above it FP32 sums
+    that for few tiles and k >= 1024 add two halves of the k range separately (and longer ranges than these, several parts:
+    test_gpu_k_parts.py). Below that nothing changes. Above it FP32 sums
     differ by about sqrt(k / 32) 2^-24, a bf16 ulp is 2^-8 of the value: one gradient element in 10^4 rounds the other way
     (measured 0.7 to 2.3e-4), one momentum code in 10^5 (at most 2e-5 over 768 x 3072), by one step in the first step. The
     Newton-Schulz products spread that over the update: 1e-4 of the master's norm, and 0.2 to 0.5 % of the FP8 weights lie

@@ -20,7 +20,7 @@ def test_the_rule_answers_what_its_comment_says(m, n, k, says, fastest):
 
 def test_no_part_is_empty():
     for k in range(1024, 16385, 48):
-        chunks = -(-k // 64)
+        chunks = -(-k // 128) * 2                                             # of the padded rows that the modules give it
         for m, n in ((256, 256), (768, 512), (3072, 768), (1536, 1536), (3072, 3072)):
             count = parts(m, n, k)
             length = -(-chunks // count)

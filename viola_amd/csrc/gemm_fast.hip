@@ -104,7 +104,7 @@ constexpr int64_t PARTS_SCRATCH = 96ll << 20;
 int plan_k_parts(int64_t m, int64_t n, int64_t k) {
     constexpr double CUS = 256.0;
     if (k < 1024 || m < 64 || n < 64 || n % 4 != 0) return 1;               // (rows of the partial products in whole 16-byte pieces)
-    const int64_t all = (k + FBK - 1) / FBK;
+    const int64_t all = (k + 127) / 128 * (128 / FBK);                       // of the host path's pitch: see launch_group_parts
     const double chunks = (double)all, small = (double)((m + 127) / 128) * (double)((n + 127) / 128), large = (double)((m + 255) / 256) * (double)((n + 127) / 128);
     auto tiles_of = [&](double count, double length) {
         const double rounds = floor(count / CUS), rest = count / CUS - rounds;

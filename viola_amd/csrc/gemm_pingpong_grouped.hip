@@ -53,8 +53,10 @@ int launch_group_parts(const GemmArgs& args, int parts, int a_dtype, int b_dtype
     const int64_t count = p.m * p.n;
     p.out = workspace;
     p.out_group_stride = (count + 3) / 4 * 4;
-    p.k_split = (p.k + parts - 1) / parts;
-    p.k_split = (p.k_split + FBK - 1) / FBK * FBK;                           // whole chunks; the last part may be shorter
+    // Whole chunks; the last part may be shorter. Cut as the k range padded to whole 128 is, which the native host path gives its
+    // operands, so that the same values without the padding (the Python operators') are added in the same order.
+    p.k_split = ((p.k + 127) / 128 * 128 + parts - 1) / parts;
+    p.k_split = (p.k_split + FBK - 1) / FBK * FBK;
     p.parts = parts = (int)((p.k + p.k_split - 1) / p.k_split);
     const int status = launch<GroupedRows, true>(p, (int)((p.m + GroupedRows::ROWS - 1) / GroupedRows::ROWS), a_dtype, b_dtype, VIOLA_F32, VIOLA_F32, 1, stream);
     if (status) return status;

@@ -9,9 +9,10 @@
 // Row pitches: every GEMM operand made here has rows of a whole number of 128 k where its k axis is a token count (weight
 // gradient), and of 16 k (128 under E8M0 scales) otherwise, padded with zero codes, and the GEMM takes the pitch as its k.
 // Whatever the sizes, the kernels that load 16-byte pieces take the product. Their sums are the guarded kernel's but for the order
-// in which the k range is added: few tiles and a long k add two halves of it separately, so with a token count that is no whole
-// number of 16 one element in 10^4 of a weight gradient rounds the other way in 16 bits, and isolated momentum codes of an
-// optimizer step behind it (1 in 10^5) and FP8 weights (0.2 to 0.5 %) take the neighbouring code.
+// in which the k range of a weight gradient is added: few tiles and a long k add two halves of it separately, or two to 64 parts
+// (viola_group_gemm_parts). So with a token count that is no whole number of 16 one element in 10^4 of a weight gradient rounds the
+// other way in 16 bits, and isolated momentum codes of an optimizer step behind it (1 in 10^5) and FP8 weights (0.2 to 0.5 %) take
+// the neighbouring code.
 #include "host.hpp"
 
 #include <torch/csrc/autograd/functions/utils.h>

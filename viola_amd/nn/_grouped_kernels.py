@@ -126,13 +126,24 @@ def transpose(q, scale, group, *, native=False, limit=None):
     return quantize(q, q.dtype, group, native=native, limit=limit, transposed=True, source_scale=scale, source_group=group)
 
 
+def _in_parts(a, b, sa, sb, m, n, k, out):
+    """The product with a scale per row and 32 k on both sides in parts of k, where it has few tiles; False: not done."""
+    parts = _lib.library().viola_group_gemm_parts(m, n, k)
+    if parts == 1:
+        return False
+    workspace = torch.empty(parts * (-(-m * n // 4) * 4), device=a.device, dtype=torch.float32)
+    return _lib.call("viola_group_gemm_in_parts", _lib.ptr(a), _lib.code(a.dtype), _lib.ptr(b), _lib.code(b.dtype), _lib.ptr(sa), _lib.ptr(sb),
+                     m, n, k, _lib.ptr(out), _lib.code(out.dtype), parts, _lib.ptr(workspace), workspace.numel(), unsupported_ok=True) == 0
+
+
 def gemm(a, b, sa, sb, group_a, group_b, *, out_dtype, native=False, bias=None, autotune=False,
-         accum_dtype="fp32", accum_block_size=0, accum_reduce_dtype="fp32"):
+         accum_dtype="fp32", accum_block_size=0, accum_reduce_dtype="fp32", k_parts=False):
     """out[m, n] = sum over 32-wide K groups of (a_codes . b_codes^T) * sa * sb (+ bias); a [m, k], b [n, k].
 
     accum_dtype="fp16" (FP32 scales only) takes the FP16-accumulator model of the reference's kernel: FP16 partial sums
     per scale group, totals in accum_reduce_dtype. With FP32 accumulation the other two options change nothing (the
-    MFMA's sums are FP32 throughout)."""
+    MFMA's sums are FP32 throughout). k_parts (a weight gradient) lets a product of few tiles and a long k run in parts of
+    k, as the native host path does: FP32 sums in another order."""
     assert accum_dtype in ("fp32", "fp16") and accum_reduce_dtype in ("fp32", "bf16") and accum_block_size % 32 == 0
     assert a.is_cuda and b.is_cuda and a.shape[1] == b.shape[1]
     a, b, sa, sb = a.contiguous(), b.contiguous(), sa.contiguous(), sb.contiguous()
@@ -159,6 +170,8 @@ def gemm(a, b, sa, sb, group_a, group_b, *, out_dtype, native=False, bias=None, 
             return out
         # shapes the block-scaled MFMA kernel declines: the same products with the scales spelled out in FP32
         sa, sb = decode_scale(sa), decode_scale(sb)
+    if k_parts and not native and bias is None and tuple(group_a) == tuple(group_b) == (1, 32) and _in_parts(a, b, sa, sb, m, n, k, out):
+        return out
     _lib.call("viola_group_gemm", _lib.ptr(a), _lib.code(a.dtype), _lib.ptr(b), _lib.code(b.dtype), _lib.ptr(sa), _lib.ptr(sb),
               m, n, k, group_a[0], group_a[1], group_b[0], group_b[1],
               _lib.ptr(bias_c), _lib.code(bias_c.dtype) if bias_c is not None else 0, _lib.ptr(out), _lib.code(out_dtype))

@@ -6,6 +6,8 @@ Differences from the reference's schedule, none of which change a value:
     row-wise codes for the forward GEMM and the quantized transpose (the reference launches two
     quantize kernels, _grouped_linear.py:21 and :46-47);
   * likewise dY is read once for dgrad + wgrad when both are needed (:73 and :92).
+
+A weight gradient of few tiles is computed in parts of k, whose FP32 products are added in ascending order.
 """
 
 from types import SimpleNamespace
@@ -125,7 +127,7 @@ def backward_core(record, tensors, dy, needs, *, gated=None, aux=None):
                 xt, sxt = saved_x, saved_scale
             else:
                 xt, sxt = kernels.quantize(saved_x, fp8, gx, limit=record.input_limit, transposed=True, native=native)
-            dw = layer._group_gemm(gt, xt, sgt, sxt, gg, gx, out_dtype=record.weight_grad_dtype)
+            dw = layer._group_gemm(gt, xt, sgt, sxt, gg, gx, out_dtype=record.weight_grad_dtype, k_parts=True)
             gt = sgt = xt = sxt = None
     if needs[2] and db is None:
         db = dy.sum(0, dtype=record.bias_grad_dtype)

@@ -322,8 +322,8 @@ class Linear(nn.Module):
     def _accumulation(self):
         return dict(accum_dtype=self.accum_dtype, accum_block_size=self.accum_block_size, accum_reduce_dtype=self.accum_reduce_dtype)
 
-    def _group_gemm(self, a, b, sa, sb, ga, gb, *, out_dtype, bias=None):
-        return grouped.gemm(a, b, sa, sb, ga, gb, out_dtype=out_dtype, bias=bias, native=self._native_scaling, **self._accumulation())
+    def _group_gemm(self, a, b, sa, sb, ga, gb, *, out_dtype, bias=None, k_parts=False):
+        return grouped.gemm(a, b, sa, sb, ga, gb, out_dtype=out_dtype, bias=bias, native=self._native_scaling, k_parts=k_parts, **self._accumulation())
 
     def _tensor_gemm(self, a, b, sa, sb, *, out_dtype, bias=None):
         return kernels.gemm(a, b, sa, sb, out_dtype=out_dtype, bias=bias, **self._accumulation())
