@@ -22,10 +22,9 @@ struct PingPongShape {
     static constexpr int TEAMS = 8 / (WM * WN), THREADS = 512 / TEAMS;       // two teams of four waves: gemm_pingpong_grouped.hpp
     static constexpr int ROWS = WM * TM * 32, COLS = WN * TN * 32;
     static constexpr int LOAD_ROWS = THREADS / PIECES;                       // a load instruction of all threads: 16 bytes each
-    static constexpr int A_LOADS = ROWS / LOAD_ROWS, B_LOADS = (COLS + LOAD_ROWS - 1) / LOAD_ROWS, LOADS = A_LOADS + B_LOADS;
-    static constexpr int B_ROWS = B_LOADS * LOAD_ROWS;                       // of b in a stage: past COLS nothing is fetched
-    static constexpr int A_BYTES = ROWS * CHUNK, B_BYTES = B_ROWS * CHUNK, STAGE = A_BYTES + B_BYTES;
-    static_assert(WM * WN * TEAMS == 8 && ROWS % LOAD_ROWS == 0);
+    static constexpr int A_LOADS = ROWS / LOAD_ROWS, B_LOADS = COLS / LOAD_ROWS, LOADS = A_LOADS + B_LOADS;
+    static constexpr int A_BYTES = ROWS * CHUNK, B_BYTES = COLS * CHUNK, STAGE = A_BYTES + B_BYTES;
+    static_assert(WM * WN * TEAMS == 8 && ROWS % LOAD_ROWS == 0 && COLS % LOAD_ROWS == 0);
 };
 
 // Epilogue. The tile's bias as fp32 in LDS (COLS floats), -0 where there is none: adding that changes nothing, not even a sign.
@@ -93,7 +92,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     static_assert(!GATED || TN == 2, "a gate and an up sub-tile per wave");
     constexpr int PANEL = GATED ? S::COLS / 2 : S::COLS;                     // columns of the output per tile
     constexpr int RING = STAGES * S::STAGE;
-    constexpr int SCALE_BLOCK = (S::ROWS + S::B_ROWS) * MX_GROUPS;           // scale bytes of 16 K groups, a rows then b rows
+    constexpr int SCALE_BLOCK = (S::ROWS + S::COLS) * MX_GROUPS;             // scale bytes of 16 K groups, a rows then b rows
     constexpr int TAIL = MX ? 2 * SCALE_BLOCK : S::COLS * 4;                 // behind the ring: scale blocks, later the bias row
     static_assert(TAIL >= S::COLS * 4);
     __shared__ __attribute__((aligned(1024))) uint8_t lds[RING + TAIL];
@@ -127,7 +126,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     for (int it = 0; it < S::LOADS; ++it) {
         const int r = (it < S::A_LOADS ? it : it - S::A_LOADS) * S::LOAD_ROWS + tid / S::PIECES;
         if (it < S::A_LOADS) cur[it] = (uint32_t)(row_in(m_begin + r, p.m) - m_begin) * (uint32_t)p.lda + piece * 16;
-        else cur[it] = r < S::COLS ? b_row(r) * (uint32_t)p.ldb + piece * 16 : OUTSIDE;
+        else cur[it] = b_row(r) * (uint32_t)p.ldb + piece * 16;
     }
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
     auto issue = [&](int c, int stage) {
@@ -151,7 +150,7 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     if constexpr (MX) {
         scale_at = tid < S::ROWS ? row_in(m_begin + tid, p.m) / (uint32_t)p.ar * (uint32_t)p.ldsa : b_row(tid - S::ROWS) / (uint32_t)p.br * (uint32_t)p.ldsb;
     }
-    const bool scale_wave = wave * 64 < S::ROWS + S::B_ROWS;
+    const bool scale_wave = wave * 64 < S::ROWS + S::COLS;
     auto issue_scales = [&](int block) {
         if (!scale_wave) return;
         const uint32_t to = lds_base + RING + (uint32_t)(block & 1) * SCALE_BLOCK + (uint32_t)wave * 1024;
