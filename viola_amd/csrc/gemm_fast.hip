@@ -53,7 +53,7 @@ constexpr int64_t SPLIT_MIN_K = 1536, NARROW_SPLIT_MIN_K = 1024;
 // of 42 shapes (bf16 outputs, within 8 % of nearly all). Two blocks of 128 x 128 of group_gemm_fast share a CU and cover each
 // other's first loads and stores, so a round of 512 costs little beside its chunks of 64 k, and a last one of up to 256 goes
 // faster; the large tiles take a CU each, whole rounds of 256, with nothing to cover their ends. So they win from about k = 1024
-// (8192 x 4096 x 1024 74 -> 68 us, 16384 x 4096 x 256 55 -> 56) where they fill the chip (4096 x 4096 x 2048, 256 of them, 68 -> 61;
+// (8192 x 4096 x 1024 75 -> 67 us, 16384 x 4096 x 256 55 -> 56) where they fill the chip (4096 x 4096 x 2048, 256 of them, 68 -> 61;
 // 6000 x 4096 x 1024, 384, 55 -> 60; row-wise 4096 x 3072 x 8192, 384, 245 -> 251). At 256 tiles of 128 x 128 and fewer the split
 // forms have more of the chip at work (8192 x 4096 x 1024 transposed, 88 -> 115 us). Groups of rows fill half of their last tile
 // on average; groups of k have each the average length.

@@ -11,16 +11,17 @@
 // u - 2, whose sums are there without a wait (two accumulators, folding unit u - 1, cost nine wait states a unit: 500 against
 // 432 us at 16384 x 4096 x 4096). The last two units of a chunk are folded in the wave's next read phase, under the other half's
 // MFMAs, so that the accumulators' numbering starts over with each chunk; all 256 registers are in use.
-//   16384 x 4096 x 4096   505 -> 445 us    16384 x 22016 x 4096   2700 -> 2400    8192 x 4096 x 1024   76 -> 67
+//   16384 x 4096 x 4096   505 -> 440 us    16384 x 22016 x 4096   2700 -> 2380    8192 x 4096 x 1024   75 -> 67
 // Products too small for those take tiles of 256 x 128 (GroupedTall, 64 x 64 per wave) in chunks of 128 k, so that a turn has as much
-// math. Its registers allow more accumulators, but folding more units in the read phase gains nothing (lag of 3, 4, 5: 521, 529,
-// 532 us where 2 takes 515); nor does issuing the loads ahead of the LDS reads (521).   8192 x 1024 x 4096  70 -> 66 us
+// math. Its registers allow more accumulators, but folding more units in the read phase gains nothing (16384 x 4096 x 4096 on these
+// tiles: 487 us with a lag of two, 505, 505 and 506 with three, four and five; 8192 x 1024 x 4096 61.6, 64.8 to 65.3); nor does issuing
+// the loads ahead of the LDS reads (521 against 513, in an earlier form).   8192 x 1024 x 4096  70 -> 62 to 66 us
 // Row-wise b scales (weight gradient; ROWS true, 256 x 128). The products sa * sb of a pair of units come from one
 // v_mfma_f32_32x32x1_2b (see group_gemm_fast), which occupies the FMA units for its 64 cycles as well; the pair of units before
 // is folded meanwhile, across chunks too, out of two sets of accumulators and products.
+//   22016 x 4096 x 16384  3450 -> 3080 us    4096 x 11008 x 16384   1660 -> 1560    4096 x 4096 x 4096   160 -> 142 to 149
 // With few tiles (GroupedTeams, 128 x 128) the halves of the block are two teams with rings of their own that share the k range, as
-// in group_gemm_fast's split form: the same sums, added in the same order.   4096 x 1024 x 8192  86 -> 74 us
-//   22016 x 4096 x 16384  3450 -> 3070 us  4096 x 11008 x 16384   1660 -> 1545    4096 x 4096 x 4096   160 -> 142
+// in group_gemm_fast's split form: the same sums, added in the same order.   4096 x 1024 x 8192  86 -> 74 to 77 us
 #pragma once
 #include "gemm_pingpong.hpp"
 

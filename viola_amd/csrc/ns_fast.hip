@@ -246,7 +246,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void ns_gemm_fast(NsArgs
     // The residual pieces of the [m, n] placement are fetched one 32-row block ahead: the loads of block j + 1 leave
     // before block j is finished and stored, so that a wavefront waits for memory once per block and not once per piece.
     // A tile of one accumulator per wave has the registers to fetch its only block, and that of its mirrored copy, before the
-    // first chunk: nothing is waited for at the end (1 x 1024 x 1024 x 1024: r r^T 7.5 -> 7.0 us, z x 7.1 -> 6.8). (On the large tiles the
+    // first chunk: nothing is waited for at the end (1 x 1024 x 1024 x 1024, back to back: r r^T 7.2 -> 6.8 us, z x 6.6 -> 6.5). (On the large tiles the
     // same under the last chunk's math gives nothing.)
     constexpr bool EARLY = WM * WN == 1;
     constexpr int COL_ITERS = WCOLS * 4 / WAVE;
