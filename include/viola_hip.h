@@ -216,7 +216,14 @@ int viola_group_gemm(const void* a, int a_dtype, const void* b, int b_dtype, con
                      int64_t m, int64_t n, int64_t k, int ar, int ak, int br, int bk,
                      const void* bias, int bias_dtype, void* out, int out_dtype, viola_stream_t stream);
 
-/* The same with a scale per row and 32 k on both sides (ar = br = 1, ak = bk = 32), no bias, the k range cut into `parts` (2 .. 64)
+/* Which form viola_group_gemm (row_groups = k_groups = 0), viola_varlen_group_gemm (row_groups: its groups, m: its m_total) or
+ * viola_varlen_wgrad_gemm (k_groups: its groups, k: its t_total; m, n: its n, kout) runs a product in, for 16-byte aligned operands
+ * and scales per 32 k: 0..3 blocks of 128 x 128, with their k range split, of 128 x 64, with their k range split; 4 tiles of 256 x 256
+ * (row_scaled_b: 256 x 128), 5 one round of 256 x 128 tiles, 6 tiles of 128 x 128 whose teams take turns. Host arithmetic only,
+ * nothing is launched. VIOLA_EINVAL for sizes that the guarded kernel takes (k % 16 != 0, operands or scales beyond 2 GiB). */
+int viola_group_gemm_form(int64_t m, int64_t n, int64_t k, int row_scaled_b, int row_groups, int k_groups);
+
+/* viola_group_gemm with a scale per row and 32 k on both sides (ar = br = 1, ak = bk = 32), no bias, the k range cut into `parts` (2 .. 64)
  * that are computed side by side: their FP32 products go to workspace (parts * (m * n rounded up to 4) floats, 16-byte aligned) and
  * are added in ascending order. viola_group_gemm_parts says how many are worth it (1: viola_group_gemm): never so many that the
  * workspace would exceed 96 MiB, and 1 for sizes that are not taken. VIOLA_EUNSUPPORTED, with nothing launched, where k % 16 != 0,
@@ -274,7 +281,7 @@ int viola_mx_gated_gemm_encode(const void* a, int a_dtype, const void* b, int b_
  * (offsets: groups+1 int64 on the device, ascending) and operand b + g*b_group_stride (elements),
  * sb + g*sb_group_stride (floats). Same arithmetic per group as viola_group_gemm. The reference
  * has no such kernel (its "grouped" is group-scaled quantization); this serves the
- * variable-group linear named by the build's target workload. m_total bounds the grid. */
+ * variable-group linear (nn.GroupedExperts). m_total bounds the grid. */
 int viola_varlen_group_gemm(const void* a, int a_dtype, const void* b, int b_dtype, const float* sa, const float* sb,
                             const int64_t* offsets, int groups, int64_t m_total, int64_t n, int64_t k,
                             int ar, int ak, int br, int bk, int64_t b_group_stride, int64_t sb_group_stride,

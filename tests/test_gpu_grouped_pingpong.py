@@ -1,7 +1,7 @@
 """GPU parity: the large-tile form of the grouped-scale products (256 x 256, row-wise b scales 256 x 128) at its edges.
 
 Integer operands and power-of-two scales throughout, so that the sums are exact in FP32 and every element must equal the integer
-product, rounded once where the output is narrower."""
+product, rounded once where the output is narrower. test_group_form.py holds these shapes to the kernels they are here for."""
 
 import pytest
 import torch
@@ -26,9 +26,12 @@ def _spell(t, s, rows):
 
 # rows and columns short of the last tile, columns whose rows of the output are 16-byte aligned or not; k that ends inside a chunk
 # of 64, inside a piece of four scales and inside a block of eight
+LARGE = [(4090, 4070, 2064, (E4, E4), torch.float32), (4096, 4096, 1536, (E5, E4), torch.bfloat16),
+         (4001, 4072, 2272, (E4, E5), torch.float16), (8190, 8180, 2592, (E5, E5), torch.bfloat16)]
+
+
 @pytest.mark.parametrize("gb", [(32, 32), (1, 32)])
-@pytest.mark.parametrize("m,n,k,formats,out_dtype", [(4090, 4070, 2064, (E4, E4), torch.float32), (4096, 4096, 1536, (E5, E4), torch.bfloat16),
-                                                     (4001, 4072, 2272, (E4, E5), torch.float16), (8190, 8180, 2592, (E5, E5), torch.bfloat16)])
+@pytest.mark.parametrize("m,n,k,formats,out_dtype", LARGE)
 def test_grouped_products_on_large_tiles(m, n, k, formats, out_dtype, gb):
     from viola_amd.nn import _grouped_kernels as g
     torch.manual_seed(m + n + k)
@@ -39,8 +42,11 @@ def test_grouped_products_on_large_tiles(m, n, k, formats, out_dtype, gb):
     assert torch.equal(out, (_spell(a, sa, 1) @ _spell(b, sb, gb[0]).T + bias).to(out_dtype))
 
 
+LARGE_LEAK_K = [1568, 1824]                                                  # 49 and 57 groups: one scale in the last piece, and in the last block
+
+
 @pytest.mark.parametrize("gb", [(32, 32), (1, 32)])
-@pytest.mark.parametrize("k", [1568, 1824])                                  # 49 and 57 groups: one scale in the last piece, and in the last block
+@pytest.mark.parametrize("k", LARGE_LEAK_K)
 def test_scales_of_the_next_row_do_not_leak_on_large_tiles(gb, k):
     """The piece that holds a row's last scales reaches into the next row's: a NaN or an Inf there stays in its own row."""
     from viola_amd.nn import _grouped_kernels as g
@@ -64,14 +70,15 @@ def test_scales_of_the_next_row_do_not_leak_on_large_tiles(gb, k):
     assert torch.equal(out[:, ~inside], base[:, ~inside]) and torch.isnan(out[:, inside]).all()
 
 
-@pytest.mark.parametrize("counts", [[7500, 0, 1, 7400, 256, 15843, 0], [1000] * 66])
-def test_varlen_products_on_large_tiles(counts):
-    """Row ranges per group (more groups than a count of 64 covers in the second case), empty ones among them."""
-    torch.manual_seed(len(counts))
-    groups, n, k, total = len(counts), 1000, 2048, sum(counts)
+VARLEN_LARGE, VARLEN_LARGE_SIZE = [[7500, 0, 1, 7400, 256, 15843, 0], [1000] * 66], (1000, 2048)
+
+
+def _varlen_products(counts, n, k):
+    """viola_varlen_group_gemm on these groups of rows, every element against the exact product."""
+    groups, total = len(counts), sum(counts)
     a, b = _integers(total, k), _integers(groups, n, k)
     offsets = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], device="cuda")
-    sa, sb = _scales(total, k // 32), _scales(groups, -(-n // 32), k // 32)
+    sa, sb = _scales(total, -(-k // 32)), _scales(groups, -(-n // 32), -(-k // 32))
     out, qa, qb = torch.full((total, n), 7.0, device="cuda"), a.to(E4), b.to(E4)
     _lib.call("viola_varlen_group_gemm", qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E4), sa.data_ptr(), sb.data_ptr(), offsets.data_ptr(),
               groups, total, n, k, 1, 32, 32, 32, n * k, sb[0].numel(), out.data_ptr(), 0)
@@ -81,9 +88,19 @@ def test_varlen_products_on_large_tiles(counts):
         row += c
 
 
+@pytest.mark.parametrize("counts", VARLEN_LARGE)
+def test_varlen_products_on_large_tiles(counts):
+    """Row ranges per group (more groups than a count of 64 covers in the second case), empty ones among them."""
+    torch.manual_seed(len(counts))
+    _varlen_products(counts, *VARLEN_LARGE_SIZE)
+
+
 # one round of 256 x 128 tiles in chunks of 128 k: k that ends with a chunk, in each quarter of one and inside a slot of 32; ragged rows and columns
-@pytest.mark.parametrize("m,n,k,out_dtype", [(8192, 1024, 2048, torch.bfloat16), (8000, 1000, 2064, torch.float32), (5000, 900, 2144, torch.float16),
-                                             (3000, 2304, 2208, torch.bfloat16), (2304, 2250, 1968, torch.float32), (16384, 512, 1792, torch.bfloat16)])
+TALL = [(8192, 1024, 2048, torch.bfloat16), (8000, 1000, 2064, torch.float32), (5000, 900, 2144, torch.float16),
+        (3000, 2304, 2208, torch.bfloat16), (2304, 2250, 1968, torch.float32), (16384, 512, 1792, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("m,n,k,out_dtype", TALL)
 def test_grouped_products_on_one_round_of_tall_tiles(m, n, k, out_dtype):
     """(with a row's first scale a NaN, which the piece of the row before's last ones reaches into)"""
     from viola_amd.nn import _grouped_kernels as g
@@ -98,26 +115,23 @@ def test_grouped_products_on_one_round_of_tall_tiles(m, n, k, out_dtype):
     assert torch.equal(out[rows, :columns], want[rows, :columns].to(out_dtype)) and torch.isnan(out[7]).all()
 
 
-def test_varlen_products_on_one_round_of_tall_tiles():
-    torch.manual_seed(4)
-    counts = [2900, 0, 1, 3000, 256]
-    groups, n, k, total = len(counts), 1000, 2144, sum(counts)
-    a, b = _integers(total, k), _integers(groups, n, k)
-    offsets = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], device="cuda")
-    sa, sb = _scales(total, k // 32), _scales(groups, -(-n // 32), k // 32)
-    out, qa, qb = torch.full((total, n), 7.0, device="cuda"), a.to(E4), b.to(E4)
-    _lib.call("viola_varlen_group_gemm", qa.data_ptr(), _lib.code(E4), qb.data_ptr(), _lib.code(E4), sa.data_ptr(), sb.data_ptr(), offsets.data_ptr(),
-              groups, total, n, k, 1, 32, 32, 32, n * k, sb[0].numel(), out.data_ptr(), 0)
-    row = 0
-    for g, c in enumerate(counts):
-        assert torch.equal(out[row:row + c], _spell(a[row:row + c], sa[row:row + c], 1) @ _spell(b[g], sb[g], 32).T)
-        row += c
+# row ranges per group, empty ones among them; k that ends with a chunk, and in its first and third quarter
+VARLEN_TALL = [([2900, 0, 1, 3000, 256], 1000, 4192), ([2900, 0, 1, 3000, 256], 900, 4112), ([700, 0, 255, 257, 2884], 1024, 4224)]
+
+
+@pytest.mark.parametrize("counts,n,k", VARLEN_TALL)
+def test_varlen_products_on_one_round_of_tall_tiles(counts, n, k):
+    torch.manual_seed(k)
+    _varlen_products(counts, n, k)
+
+
+VARLEN_WGRAD = [0, 2080, 32, 4096, 1952, 0, 2176], 2040, 4000                # slots of the groups, rows and columns of the gradients
 
 
 def test_varlen_weight_gradient_on_large_tiles():
-    """k ranges per group: none, one slot of 32, ranges that end inside a chunk."""
+    """k ranges per group: none, one slot of 32, ranges that end inside a chunk; ragged rows and columns."""
     torch.manual_seed(3)
-    slots, n, kout = [0, 2080, 32, 4096, 1952, 0, 2176], 1024, 4000
+    slots, n, kout = VARLEN_WGRAD
     offsets = torch.tensor([0, *torch.tensor(slots).cumsum(0).tolist()], device="cuda")
     total = -(-sum(slots) // 128) * 128
     a, b = _integers(n, total), _integers(kout, total)
@@ -131,8 +145,11 @@ def test_varlen_weight_gradient_on_large_tiles():
         start += length
 
 
-@pytest.mark.parametrize("m,n,k,out_dtype", [(4096, 1024, 8192, torch.bfloat16), (2000, 1028, 1536, torch.float32), (1921, 2047, 1552, torch.float16),
-                                             (1500, 1535, 1568, torch.bfloat16), (1536, 1536, 1808, torch.float32), (1536, 1536, 2064, torch.float32)])
+TEAMS = [(4096, 1024, 8192, torch.bfloat16), (2000, 1028, 1536, torch.float32), (1921, 2047, 1552, torch.float16),
+         (1500, 1535, 1568, torch.bfloat16), (1536, 1536, 1808, torch.float32), (1536, 1536, 2064, torch.float32)]
+
+
+@pytest.mark.parametrize("m,n,k,out_dtype", TEAMS)
 def test_row_scaled_products_whose_teams_share_the_k_range(m, n, k, out_dtype):
     """129 to 256 tiles of 128 x 128: the teams' ranges of equal and different length, the second ending inside a block of scales (with
     the next row's scale, a NaN, in the piece that holds its last ones), ragged rows and columns."""

@@ -80,7 +80,8 @@ _SIGNATURES = {
     "viola_selftest_fp8": [_p, _p],
     "viola_selftest_philox": [_p, _p, _l, _p],
 }
-EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan", "viola_tensor_encode_slices", "viola_group_gemm_parts")
+EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan", "viola_tensor_encode_slices", "viola_group_gemm_parts",
+                                "viola_group_gemm_form")
 
 _lib = None
 
@@ -100,6 +101,7 @@ def library():
         lib.viola_error_string.argtypes, lib.viola_error_string.restype = [ctypes.c_int], ctypes.c_char_p
         lib.viola_tensor_encode_slices.argtypes, lib.viola_tensor_encode_slices.restype = [_i, _l, _l], ctypes.c_int64
         lib.viola_group_gemm_parts.argtypes, lib.viola_group_gemm_parts.restype = [_l, _l, _l], ctypes.c_int
+        lib.viola_group_gemm_form.argtypes, lib.viola_group_gemm_form.restype = [_l, _l, _l, _i, _i, _i], ctypes.c_int
         lib.viola_ns_plan.argtypes, lib.viola_ns_plan.restype = [_l, _l, _l, _l, _i, _i, _i, ctypes.POINTER(ctypes.c_int)], ctypes.c_int
         assert lib.viola_abi_version() == 1
         _lib = lib

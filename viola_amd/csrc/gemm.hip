@@ -9,15 +9,16 @@ static int shift_of(int v) {
     return s;
 }
 
+// the fast kernels address operands and scales with 31-bit byte offsets and stage the scales of 8 consecutive 32-wide K groups at once
+static bool fast_sizes(const GemmArgs& p, int64_t b_rows) {
+    return b_rows * p.ldb < (1ll << 31) && (int64_t)BM * p.lda < (1ll << 31) && (p.m + p.ar - 1) / p.ar * p.ldsa * 4 < (1ll << 31) &&
+           (b_rows + p.br - 1) / p.br * p.ldsb * 4 < (1ll << 31) && p.ak_shift == 5 && p.bk_shift == 5;
+}
+
 template <int MODE>
 static int launch_out(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, bool vec,
                       dim3 grid, hipStream_t stream) {
-    const int64_t b_rows = MODE == MODE_GATED_FWD ? 2 * p.n : p.n;
-    // the fast kernel addresses operands and scales with 31-bit byte offsets
-    const bool small = b_rows * p.ldb < (1ll << 31) && (int64_t)BM * p.lda < (1ll << 31) &&
-                       (p.m + p.ar - 1) / p.ar * p.ldsa * 4 < (1ll << 31) && (b_rows + p.br - 1) / p.br * p.ldsb * 4 < (1ll << 31) &&
-                       p.ak_shift == 5 && p.bk_shift == 5;         // and stages the scales of 8 consecutive 32-wide K groups at once
-    if (vec && small)
+    if (vec && fast_sizes(p, MODE == MODE_GATED_FWD ? 2 * p.n : p.n))
         return launch_group_gemm_fast(p, MODE, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
     return launch_group_gemm_generic(p, MODE, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
 }
@@ -48,6 +49,22 @@ extern "C" int viola_group_gemm(const void* a, int a_dtype, const void* b, int b
     const bool vec = k % 16 == 0 && aligned16(a) && aligned16(b);
     const bool rowscale = br % 32 != 0;
     return launch_out<MODE_PLAIN>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, vec, dim3((unsigned)gx, (unsigned)gy), stream);
+}
+
+extern "C" int viola_group_gemm_form(int64_t m, int64_t n, int64_t k, int row_scaled_b, int row_groups, int k_groups) {
+    constexpr int64_t LARGEST = 1ll << 31;
+    VIOLA_CHECK_ARG(m > 0 && n > 0 && k > 0 && m < LARGEST && n < LARGEST && k < LARGEST && k % 16 == 0);
+    VIOLA_CHECK_ARG(row_groups >= 0 && k_groups >= 0 && k_groups <= 65535 && (!k_groups || (row_scaled_b && !row_groups)));
+    const int64_t gy = (m + BM - 1) / BM + row_groups;
+    VIOLA_CHECK_ARG(gy <= 65535);
+    static const int64_t there = 0;                                          // (the rule asks only whether there are offsets)
+    GemmArgs p = {};
+    p.m = m; p.n = n; p.k = k; p.lda = k; p.ldb = k; p.groups = row_groups;
+    p.ar = 1; p.br = row_scaled_b ? 1 : 32; p.ldsa = p.ldsb = (k + 31) / 32; p.ak_shift = p.bk_shift = 5;
+    p.offsets = row_groups ? &there : nullptr;
+    p.koffsets = k_groups ? &there : nullptr;
+    VIOLA_CHECK_ARG(fast_sizes(p, n));
+    return group_form(p, row_scaled_b != 0, dim3((unsigned)((n + BN - 1) / BN), (unsigned)gy, k_groups ? (unsigned)k_groups : 1));
 }
 
 // (what the fast kernel asks of a product with a scale per row and 32 k on both sides, plus what 256 rows of a large tile do)

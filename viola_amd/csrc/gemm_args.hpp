@@ -50,6 +50,11 @@ int launch_group_gemm_half(const GemmArgs& p, bool per_tensor, int a_dtype, int 
 int launch_group_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype,
                            bool rowscale, dim3 grid, hipStream_t stream);
 
+// Which form a plain product under the grouped recipe runs in (the values are viola_group_gemm_form's): the blocks of group_gemm_fast
+// of 128 x 128 or 128 x 64, their k range split over two teams or not, or one of the three forms below. gemm_fast.hip.
+enum GroupForm { GROUP_BLOCKS = 0, GROUP_BLOCKS_SPLIT, GROUP_NARROW, GROUP_NARROW_SPLIT, GROUP_LARGE, GROUP_TALL, GROUP_TEAMS };
+GroupForm group_form(const GemmArgs& p, bool rowscale, dim3 grid);
+
 // The grouped recipe on tiles of 256 x 256 (row-wise b scales: 256 x 128); row_tiles: tiles of 256 rows (variable groups: a bound on
 // them), groups: k ranges. gemm_pingpong_grouped.hip.
 int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, unsigned groups,

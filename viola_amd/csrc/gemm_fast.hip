@@ -48,7 +48,6 @@ static int launch_mode(const GemmArgs& p, int a_dtype, int b_dtype, int bias_dty
 // on 128 x 64 tiles: k = 512 slower, k = 1024 9.8 -> 9.1 us, k = 1536 12.6 -> 11.1 us)
 constexpr int64_t SPLIT_MIN_K = 1536, NARROW_SPLIT_MIN_K = 1024;
 
-
 // Whether a plain product runs on gemm_pingpong_grouped: the lesser of two estimates in microseconds, fitted to the measured times
 // of 42 shapes (bf16 outputs, within 8 % of nearly all). Two blocks of 128 x 128 of group_gemm_fast share a CU and cover each
 // other's first loads and stores, so a round of 512 costs little beside its chunks of 64 k, and a last one of up to 256 goes
@@ -130,43 +129,46 @@ int plan_k_parts(int64_t m, int64_t n, int64_t k) {
     return best;
 }
 
+// The kernel of a product: plain ones on the large tiles where those win, else the blocks of group_gemm_fast. Two blocks of 128 x 128
+// fit a CU, so from 257 tiles up every CU has work and the full tile, which reads the least, is the fastest form (4096 x 1152 x 4608:
+// 75.6 -> 59.7 us against the split one, 6000 x 1000 x 1024: 27.0 -> 19.6 us against tiles halved in n). From 129 to 256 tiles a CU gets
+// one: over a long k keep the tile and split its k range over twice the waves inside the block (7-12 % faster at 256 tiles, k >= 2048;
+// with row-wise b scales the teams take turns, 4096 x 1024 x 8192 86 -> 74 us, 1536 x 1536 x 4096 43 -> 35, with uniform ones they do not
+// gain by it, 68 against 77), else halve the tile in n for a second block per CU. With 128 tiles or fewer the narrow tiles keep more
+// CUs busy and their k range is split: a CU then holds eight waves instead of four (1024 x 1024 x 16384: 98 -> 76 us, 512 x 512 x 4096:
+// 27.5 -> 22.3 us). Narrow split tiles are one per CU: past 256 of them the second round costs more than the split gives
+// (600 x 4096 x 1024: 17.2 us, unsplit 12.5 us).
+GroupForm group_form(const GemmArgs& p, bool rowscale, dim3 grid) {
+    if (prefer_pingpong(p, rowscale, grid.z)) return GROUP_LARGE;
+    if (!rowscale && prefer_tall(p)) return GROUP_TALL;
+    const int64_t tiles = (int64_t)grid.x * grid.y * grid.z;
+    if (tiles > 256) return GROUP_BLOCKS;
+    const bool fixed_k = !p.offsets && !p.koffsets;
+    if (tiles > 128 && fixed_k && p.k >= SPLIT_MIN_K) return rowscale ? GROUP_TEAMS : GROUP_BLOCKS_SPLIT;
+    if (p.n <= 64) return GROUP_BLOCKS;
+    return tiles <= 128 && fixed_k && p.k >= NARROW_SPLIT_MIN_K ? GROUP_NARROW_SPLIT : GROUP_NARROW;
+}
+
 int launch_group_gemm_fast(const GemmArgs& args, int mode, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale,
                            dim3 grid, hipStream_t stream) {
     GemmArgs p = args;
     const int64_t b_rows = mode == MODE_GATED_FWD ? 2 * p.n : p.n;
     p.sa_bytes = (p.m + p.ar - 1) / p.ar * p.ldsa * 4;
     p.sb_bytes = (b_rows + p.br - 1) / p.br * p.ldsb * 4;
-    if (mode == MODE_PLAIN && prefer_pingpong(p, rowscale, grid.z)) {
-        const int64_t row_tiles = p.offsets ? p.m / 256 + p.groups : (p.m + 255) / 256;
-        return launch_group_pingpong(p, (int)row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid.z, stream);
-    }
-    if (mode == MODE_PLAIN && !rowscale && prefer_tall(p)) {
-        const int64_t row_tiles = p.offsets ? p.m / 256 + p.groups : (p.m + 255) / 256;
-        return launch_group_tall(p, (int)row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
-    }
-    // Two blocks of 128 x 128 fit a CU, so from 257 tiles up every CU has work and the full tile, which reads the least, is
-    // the fastest form (4096 x 1152 x 4608: 75.6 -> 59.7 us against the split one, 6000 x 1000 x 1024: 27.0 -> 19.6 us against
-    // tiles halved in n). From 129 to 256 tiles a CU gets one: over a long k keep the tile and split its k range over twice the
-    // waves inside the block (7-12 % faster at 256 tiles, k >= 2048), else halve the tile in n for a second block per CU. With
-    // 128 tiles or fewer the narrow tiles keep more CUs busy and their k range is split: a CU then holds eight waves instead of
-    // four (1024 x 1024 x 16384: 98 -> 76 us, 512 x 512 x 4096: 27.5 -> 22.3 us). Narrow split tiles are one per CU: past 256 of
-    // them the second round costs more than the split gives (600 x 4096 x 1024: 17.2 us, unsplit 12.5 us).
-    const int64_t tiles = (int64_t)grid.x * grid.y * grid.z;
-    const bool few = mode == MODE_PLAIN && tiles <= 256;
-    const bool fixed_k = !p.offsets && !p.koffsets;
-    const bool split = few && tiles > 128 && fixed_k && p.k >= SPLIT_MIN_K;
-    // ... with row-wise b scales the teams take turns (4096 x 1024 x 8192 86 -> 74 us, 1536 x 1536 x 4096 43 -> 35; with uniform ones they do
-    // not gain by it, 68 against 77)
-    if (split && rowscale) return launch_group_teams(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
-    const bool narrow = few && !split && p.n > 64;
+    const GroupForm form = mode == MODE_PLAIN ? group_form(p, rowscale, grid) : GROUP_BLOCKS;
+    const int64_t row_tiles = p.offsets ? p.m / 256 + p.groups : (p.m + 255) / 256;
+    if (form == GROUP_LARGE) return launch_group_pingpong(p, (int)row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid.z, stream);
+    if (form == GROUP_TALL) return launch_group_tall(p, (int)row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    if (form == GROUP_TEAMS) return launch_group_teams(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    const bool narrow = form == GROUP_NARROW || form == GROUP_NARROW_SPLIT;
     if (narrow) grid.x = (unsigned)((p.n + 63) / 64);
     if ((int64_t)grid.x * grid.y < (1 << 30)) {
         p.tiles_n = (int)grid.x;
         p.tiles_m = (int)grid.y;
         grid = dim3((grid.x * grid.y + 7) / 8 * 8, 1, grid.z);
     }
-    if (split) return launch_split<2, false>(p, a_dtype, b_dtype, bias_dtype, out_dtype, grid, stream);
-    if (narrow && tiles <= 128 && fixed_k && p.k >= NARROW_SPLIT_MIN_K)
+    if (form == GROUP_BLOCKS_SPLIT) return launch_split<2, false>(p, a_dtype, b_dtype, bias_dtype, out_dtype, grid, stream);
+    if (form == GROUP_NARROW_SPLIT)
         return rowscale ? launch_split<1, true>(p, a_dtype, b_dtype, bias_dtype, out_dtype, grid, stream)
                         : launch_split<1, false>(p, a_dtype, b_dtype, bias_dtype, out_dtype, grid, stream);
     if (narrow) return launch_mode<MODE_PLAIN, 1>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, grid, stream);
