@@ -289,7 +289,7 @@ def main():
     def want(leg):
         return leg in only if only else not skipped[leg]
     if args.gpus != 1:
-        sys.exit("bench.py measures one GPU: this build has no multi-GPU path (run with --gpus 1)")
+        sys.exit("bench.py measures one GPU: viola_amd has no multi-GPU path (run with --gpus 1)")
     import torch
     from viola_amd import _lib
     assert torch.cuda.is_available(), "bench.py needs the GPU"

@@ -1,6 +1,6 @@
 """Base class for optimizers whose update needs a whole logical matrix
 (viola/optim/matrix.py:14-135, plain-tensor path). One GPU: DTensor parameters, owner
-gather/scatter and mesh all-reduces of the reference are not part of this build."""
+gather/scatter and mesh all-reduces of the reference are not part of this package."""
 
 import functools
 
