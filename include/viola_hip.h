@@ -338,10 +338,10 @@ int viola_adam_update(void* weight, int weight_dtype, const void* grad, int grad
                       int rounding, int64_t rounding_step, int64_t rounding_key, int64_t offset,
                       int adamw, int maximize, viola_stream_t stream);
 
-/* viola_momentum_update (1-D tiles of 256 / 512 / 1024, whole tiles only) for many tensors with the same number of
- * tiles, gradient dtype and hyper-parameters, in one launch (the reference launches once per matrix,
+/* viola_momentum_update (1-D tiles of 256 / 512 / 1024, whole tiles only) for many tensors of at most `tiles`
+ * tiles with the same gradient dtype and hyper-parameters, in one launch (the reference launches once per matrix,
  * viola/optim/muon.py:104-106). table: device array of `tensors` rows of eight int64: {grad, old_q, old_scale, new_q,
- * new_scale, update, rounding key, 0}; the gradient must be aligned to four elements, the codes to 4
+ * new_scale, update, rounding key, tiles}; a row's tiles may be fewer than `tiles` (0: the same); the gradient must be aligned to four elements, the codes to 4
  * bytes and the bf16 update to 8 bytes; old and new state may alias. */
 int viola_momentum_update_table(const int64_t* table, int64_t tensors, int64_t tiles, int grad_dtype, int tile_size,
                                 float beta, float inv_loss_scale, int nesterov, int rounding, int64_t rounding_step,
@@ -352,6 +352,11 @@ int viola_momentum_update_table(const int64_t* table, int64_t tensors, int64_t t
  * {weight (16-byte aligned), update (aligned to four elements of grad_dtype)}. */
 int viola_weight_update_table(const int64_t* table, int64_t tensors, int64_t count, int grad_dtype, float lr, float decay,
                               float update_scale, viola_stream_t stream);
+
+/* viola_weight_update_table for tensors of different sizes and update scales. table: rows of four int64: {weight, update, elements (a
+ * multiple of 4), the update scale's FP32 bits}; max_count: the largest number of elements. */
+int viola_weight_update_rows(const int64_t* table, int64_t tensors, int64_t max_count, int grad_dtype, float lr, float decay,
+                             viola_stream_t stream);
 
 /* The same update for many tensors that share dtypes, hyper-parameters and step count, in one launch (the reference
  * calls adam_update once per parameter, viola/optim/muon.py:137-140; vectors of a transformer are a few thousand
@@ -389,6 +394,18 @@ int viola_ns_gemm(const void* a, const void* bmat, const void* residual, void* o
                   int transpose_b, int epilogue, int64_t batch, int64_t m, int64_t n, int64_t k,
                   float add_diag, void* out_diag, int transpose_out, viola_stream_t stream);
 
+/* Up to eight products of viola_ns_gemm that do not depend on each other (the same step of the chains of several shapes), in one
+ * launch; the arguments and results of each are viola_ns_gemm's. VIOLA_EUNSUPPORTED, with nothing launched: more than eight, or one
+ * that viola_ns_plan gives the generic kernel; each then takes a call of its own. */
+typedef struct {
+    const void *a, *b, *residual;
+    void *out, *out_diag;
+    int64_t batch, m, n, k;
+    float add_diag;
+    int transpose_b, epilogue, transpose_out;
+} viola_ns_product;
+int viola_ns_gemm_many(const viola_ns_product* products, int count, int dtype, viola_stream_t stream);
+
 /* viola/optim/_orthogonalize_kernels.py:114-197 `plan` (the per-shape schedule the reference picks by timing its
  * candidates: bm, bn): which tile shape viola_ns_gemm runs a product on. Host arithmetic only, nothing is launched and
  * no GPU is needed. Operands are taken as 16-byte aligned; same_operand != 0 means a and bmat are one buffer.
@@ -406,6 +423,16 @@ int viola_ns_plan(int64_t batch, int64_t m, int64_t n, int64_t k, int transpose_
  * sums of squares; every slot is written before it is read, so it needs no clearing). */
 int viola_ns_prepare(const void* in, int in_dtype, void* out, int dtype, int64_t batch, int64_t rows, int64_t cols,
                      float* workspace, viola_stream_t stream);
+
+/* viola_ns_prepare of bf16 matrices of up to eight shapes, in one launch for each of its two stages. The workspace holds 256 floats
+ * per matrix of all of them. VIOLA_EUNSUPPORTED, with nothing launched: more than eight shapes or 65535 matrices, columns that are
+ * no multiple of 8, or operands off 16 bytes. */
+typedef struct {
+    const void* in;
+    void* out;
+    int64_t batch, rows, cols;
+} viola_ns_matrices;
+int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count, int dtype, float* workspace, viola_stream_t stream);
 
 /* No counterpart in the reference. viola_ns_prepare for callers that cannot allocate device memory (code under
  * HIP-graph capture, serving loops, harnesses that forbid hipMalloc): the same kernels and results, with the

@@ -2,7 +2,7 @@
 // momentum, Newton-Schulz chain, weight update; AdamW for vectors) and FP8Communication's round trip.
 //
 // Why it is native: the step of one 1024 x 1024 matrix is 20 kernels of 3-9 us (about 170 us) and took 300 us of Python to
-// enqueue; per parameter a step costs about 1 us here.
+// enqueue; per parameter a step costs about 1 us here, and the matrices of a step share their launches where they can.
 #include "host.hpp"
 
 #include <c10/core/Event.h>
@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <tuple>
 
@@ -21,49 +22,57 @@ namespace {
 // ---------------------------------------------------------------------------------------------------- Newton-Schulz
 constexpr float A_COEFFICIENT = 3.4445f;
 
-// orthogonalize [..., rows, cols] in `steps` steps; every product of the chain reads and writes one arena, the last one the result
-Tensor newton_schulz(const Tensor& matrix_, int64_t steps, bool gram) {
+// The products that orthogonalize [..., rows, cols] in `steps` steps, one after the other; each reads and writes the arena, the last one
+// the result.
+struct Chain {
+    Tensor matrix, result;
+    Arena arena;
+    int dtype = 0;
+    viola_ns_matrices start{};                                   // the scaled matrix, in front of the products
+    std::vector<viola_ns_product> products;
+};
+
+Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram) {
     TORCH_CHECK(matrix_.is_cuda(), "viola_amd kernels run on the GPU only");
     TORCH_CHECK(matrix_.dim() >= 2 && steps >= 0, "Newton-Schulz takes matrices and a number of steps, got ", matrix_.dim(), " dimensions and ", steps, " steps");
-    const Tensor matrix = matrix_.contiguous();
-    const int64_t rows = matrix.size(-2), cols = matrix.size(-1), m = std::min(rows, cols), n = std::max(rows, cols);
-    const int64_t batch = rows * cols ? matrix.numel() / (rows * cols) : 0;
+    Chain c;
+    c.matrix = matrix_.contiguous();
+    const int64_t rows = c.matrix.size(-2), cols = c.matrix.size(-1), m = std::min(rows, cols), n = std::max(rows, cols);
+    const int64_t batch = rows * cols ? c.matrix.numel() / (rows * cols) : 0;
     const bool tall = rows > cols;
     const at::ScalarType type = gram ? at::kHalf : at::kBFloat16;
-    const int dtype = code_of(type);
-    const viola_stream_t stream = stream_of(matrix);
-    const Tensor result = at::empty(matrix.sizes(), matrix.options().dtype(type));
-    if (matrix.numel() == 0) return result;
+    c.dtype = code_of(type);
+    c.result = at::empty(c.matrix.sizes(), c.matrix.options().dtype(type));
+    if (c.matrix.numel() == 0) return c;
     const bool quintic = !gram || m == n;                        // the plain iteration; else the recurrence on the Gram matrix
     const int64_t wide = 2 * batch * m * n, square = 2 * batch * m * m;
-    Arena arena;
-    const int64_t sums = arena.take(batch * 256 * 4);
     int64_t x_at[2], s_at[6];
     const int squares = quintic ? 2 : 6;
-    for (int64_t& at : x_at) at = arena.take(wide);
-    for (int i = 0; i < squares; ++i) s_at[i] = arena.take(square);
-    arena.make(matrix.device());
-    void *x = steps ? arena.at(x_at[0]) : result.mutable_data_ptr(), *spare = arena.at(x_at[1]);   // no steps: the scaled matrix
-    VIOLA_CALL(viola_ns_prepare, matrix.const_data_ptr(), code_of(matrix.scalar_type()), x, dtype, batch, rows, cols, arena.as<float>(sums), stream);
-    if (steps == 0) return result;
+    for (int64_t& at : x_at) at = c.arena.take(wide);
+    for (int i = 0; i < squares; ++i) s_at[i] = c.arena.take(square);
+    c.arena.make(c.matrix.device());
+    void *x = steps ? c.arena.at(x_at[0]) : c.result.mutable_data_ptr(), *spare = c.arena.at(x_at[1]);   // no steps: the scaled matrix
+    c.start = {c.matrix.const_data_ptr(), x, batch, rows, cols};
+    if (steps == 0) return c;
     auto gemm = [&](const void* a, const void* b, bool transpose_b, const void* residual, int epilogue, int64_t out_cols, int64_t k, void* out,
                     float add_diag, void* out_diag, bool transpose_out) {
-        VIOLA_CALL(viola_ns_gemm, a, b, residual, out, dtype, transpose_b, epilogue, batch, m, out_cols, k, add_diag, out_diag, transpose_out, stream);
+        c.products.push_back({a, b, residual, out, out_diag, batch, m, out_cols, k, add_diag, transpose_b, epilogue, transpose_out});
     };
     if (quintic) {
-        void *r = arena.at(s_at[0]), *z = arena.at(s_at[1]);
+        void *r = c.arena.at(s_at[0]), *z = c.arena.at(s_at[1]);
         for (int64_t step = 0; step < steps; ++step) {
             const bool last = step == steps - 1;
-            void* out = last ? result.mutable_data_ptr() : spare;
+            void* out = last ? c.result.mutable_data_ptr() : spare;
             gemm(x, x, true, nullptr, 0, m, n, r, 0, nullptr, false);
             gemm(r, r, true, r, 1, m, m, z, 0, nullptr, false);  // r = x x^T is symmetric bit for bit: r r = r r^T
             gemm(z, x, false, x, 2, n, m, out, 0, nullptr, tall && last);
             spare = x;
             x = out;
         }
-        return result;
+        return c;
     }
-    void *r = arena.at(s_at[0]), *z = arena.at(s_at[1]), *q = arena.at(s_at[2]), *q_next = arena.at(s_at[3]), *rz = arena.at(s_at[4]), *r_next = arena.at(s_at[5]);
+    void *r = c.arena.at(s_at[0]), *z = c.arena.at(s_at[1]), *q = c.arena.at(s_at[2]), *q_next = c.arena.at(s_at[3]), *rz = c.arena.at(s_at[4]),
+         *r_next = c.arena.at(s_at[5]);
     std::vector<int64_t> segments;
     for (const int64_t length : {std::min<int64_t>(steps, 2), std::max<int64_t>(steps - 2, 0)})
         if (length) segments.push_back(length);
@@ -84,12 +93,64 @@ Tensor newton_schulz(const Tensor& matrix_, int64_t steps, bool gram) {
                 std::swap(r, r_next);
             }
         }
-        void* out = last ? result.mutable_data_ptr() : spare;
+        void* out = last ? c.result.mutable_data_ptr() : spare;
         gemm(q, x, false, nullptr, 0, n, m, out, 0, nullptr, tall && last);
         spare = x;
         x = out;
     }
-    return result;
+    return c;
+}
+
+void prepare(const Chain& c, float* sums, viola_stream_t stream) {
+    VIOLA_CALL(viola_ns_prepare, c.start.in, code_of(c.matrix.scalar_type()), c.start.out, c.dtype, c.start.batch, c.start.rows, c.start.cols, sums, stream);
+}
+
+void multiply(const viola_ns_product& p, int dtype, viola_stream_t stream) {
+    VIOLA_CALL(viola_ns_gemm, p.a, p.b, p.residual, p.out, dtype, p.transpose_b, p.epilogue, p.batch, p.m, p.n, p.k, p.add_diag, p.out_diag, p.transpose_out, stream);
+}
+
+Arena sums_of(int64_t matrices, const at::Device& device) {
+    Arena sums;
+    sums.take(matrices * 256 * 4);
+    sums.make(device);
+    return sums;
+}
+
+Tensor newton_schulz(const Tensor& matrix, int64_t steps, bool gram) {
+    const Chain c = chain_of(matrix, steps, gram);
+    if (c.matrix.numel() == 0) return c.result;
+    const viola_stream_t stream = stream_of(c.matrix);
+    prepare(c, sums_of(c.start.batch, c.matrix.device()).as<float>(0), stream);
+    for (const viola_ns_product& p : c.products) multiply(p, c.dtype, stream);
+    return c.result;
+}
+
+// Chains of one type, step by step together: the products of a step are one launch where the tiled kernel takes them all.
+void run_together(const std::vector<Chain>& chains, viola_stream_t stream) {
+    const int dtype = chains[0].dtype;
+    std::vector<viola_ns_matrices> starts;
+    int64_t matrices = 0;
+    size_t steps = 0;
+    for (const Chain& c : chains) {
+        starts.push_back(c.start);
+        matrices += c.start.batch;
+        steps = std::max(steps, c.products.size());
+    }
+    const Arena sums = sums_of(matrices, chains[0].matrix.device());
+    int status = VIOLA_TRY(viola_ns_prepare_many, starts.data(), (int)starts.size(), dtype, sums.as<float>(0), stream);
+    if (status == VIOLA_EUNSUPPORTED) {
+        for (const Chain& c : chains) prepare(c, sums.as<float>(0), stream);      // (one after the other: each may overwrite the sums)
+    } else check("viola_ns_prepare_many", status);
+    std::vector<viola_ns_product> step;
+    for (size_t i = 0; i < steps; ++i) {
+        step.clear();
+        for (const Chain& c : chains)
+            if (i < c.products.size()) step.push_back(c.products[i]);
+        status = step.size() > 1 ? VIOLA_TRY(viola_ns_gemm_many, step.data(), (int)step.size(), dtype, stream) : VIOLA_EUNSUPPORTED;
+        if (status == VIOLA_EUNSUPPORTED) {
+            for (const viola_ns_product& p : step) multiply(p, dtype, stream);
+        } else check("viola_ns_gemm_many", status);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------- pointer tables
@@ -121,49 +182,66 @@ private:
 };
 enum { MOMENTUM_TABLE = 0, WEIGHT_TABLE = 1, ADAM_TABLE = 2 };
 
-// One launch for a list of tensors of equal size (AdamW: of any size) over a table of their pointers. False, with nothing done:
-// they do not fit the table kernel, and each takes a launch of its own.
+// One launch for a list of tensors over a table of their pointers. False, with nothing done: they do not fit the table kernel, and
+// each takes a launch of its own.
 struct MomentumRow {
     Tensor grad, q, scale;
     void* out;                                                   // bf16
-    int64_t key;
+    int64_t key, count;
 };
-bool momentum_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<MomentumRow>& rows, int64_t count, int64_t tile,
+bool momentum_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<MomentumRow>& rows, int64_t tile,
                        float beta, float inv_loss_scale, bool nesterov, int rounding, int64_t step, viola_stream_t stream) {
-    if (rows.empty() || rows.size() > 65535 || tile < 256 || count % tile != 0) return false;
+    if (rows.empty() || rows.size() > 65535 || tile < 256) return false;
     const at::ScalarType kind = rows[0].grad.scalar_type();
     std::vector<int64_t> words;
+    int64_t tiles = 0;
     for (const MomentumRow& r : rows) {
+        if (r.count % tile != 0) return false;
+        tiles = std::max(tiles, r.count / tile);
         const void *g = r.grad.const_data_ptr(), *q = r.q.const_data_ptr();
-        if (r.grad.scalar_type() != kind || r.grad.numel() != count || !r.grad.is_contiguous() || !aligned(g, 4 * r.grad.element_size()) || !aligned(q, 4) ||
+        if (r.grad.scalar_type() != kind || r.grad.numel() != r.count || !r.grad.is_contiguous() || !aligned(g, 4 * r.grad.element_size()) || !aligned(q, 4) ||
             !aligned(r.out, 8))
             return false;
-        const int64_t s = (int64_t)r.scale.const_data_ptr(), row[8] = {(int64_t)g, (int64_t)q, s, (int64_t)q, s, (int64_t)r.out, r.key, 0};
+        const int64_t s = (int64_t)r.scale.const_data_ptr(), row[8] = {(int64_t)g, (int64_t)q, s, (int64_t)q, s, (int64_t)r.out, r.key, r.count / tile};
         words.insert(words.end(), row, row + 8);
     }
     const int64_t* t = tables.get(MOMENTUM_TABLE, shape, (int64_t)rows.size(), ordinal, std::move(words), rows[0].q.device(), stream);
-    VIOLA_CALL(viola_momentum_update_table, t, (int64_t)rows.size(), count / tile, code_of(kind), (int)tile, beta, inv_loss_scale, nesterov, rounding, step, stream);
+    VIOLA_CALL(viola_momentum_update_table, t, (int64_t)rows.size(), tiles, code_of(kind), (int)tile, beta, inv_loss_scale, nesterov, rounding, step, stream);
     return true;
 }
 
 struct WeightRow {
     Tensor weight;
     const void* update;
+    int64_t count;
+    float scale;                                                 // of the update
 };
-bool weights_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<WeightRow>& rows, int64_t count,
-                      at::ScalarType update_type, float lr, float weight_decay, float update_scale, viola_stream_t stream) {
-    if (rows.empty() || rows.size() > 65535 || count % 4 != 0) return false;
+bool weights_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<WeightRow>& rows, at::ScalarType update_type,
+                      float lr, float weight_decay, viola_stream_t stream) {
+    if (rows.empty() || rows.size() > 65535) return false;
     const int64_t update_bytes = 4 * (int64_t)at::elementSize(update_type);
+    bool alike = true;
+    int64_t most = 0;
+    for (const WeightRow& r : rows) {
+        if (r.count % 4 != 0 || r.weight.scalar_type() != at::kFloat || r.weight.numel() != r.count || !r.weight.is_contiguous() ||
+            !aligned(r.weight.const_data_ptr(), 16) || !aligned(r.update, update_bytes))
+            return false;
+        alike = alike && r.count == rows[0].count && r.scale == rows[0].scale;
+        most = std::max(most, r.count);
+    }
     std::vector<int64_t> words;
     for (const WeightRow& r : rows) {
-        const void* w = r.weight.const_data_ptr();
-        if (r.weight.scalar_type() != at::kFloat || r.weight.numel() != count || !r.weight.is_contiguous() || !aligned(w, 16) || !aligned(r.update, update_bytes))
-            return false;
-        words.push_back((int64_t)w);
+        words.push_back((int64_t)r.weight.const_data_ptr());
         words.push_back((int64_t)r.update);
+        if (alike) continue;
+        uint32_t bits;
+        std::memcpy(&bits, &r.scale, 4);
+        words.push_back(r.count);
+        words.push_back(bits);
     }
     const int64_t* t = tables.get(WEIGHT_TABLE, shape, (int64_t)rows.size(), ordinal, std::move(words), rows[0].weight.device(), stream);
-    VIOLA_CALL(viola_weight_update_table, t, (int64_t)rows.size(), count, code_of(update_type), lr, weight_decay, update_scale, stream);
+    if (alike) VIOLA_CALL(viola_weight_update_table, t, (int64_t)rows.size(), most, code_of(update_type), lr, weight_decay, rows[0].scale, stream);
+    else VIOLA_CALL(viola_weight_update_rows, t, (int64_t)rows.size(), most, code_of(update_type), lr, weight_decay, stream);
     return true;
 }
 
@@ -370,8 +448,8 @@ private:
 
     // The chains of different buckets are independent, and a single chain leaves the GPU partly idle at every launch boundary
     // (a Newton-Schulz GEMM of 28 matrices is ~590 tiles for 512 tile slots: its second round is nearly empty). Buckets
-    // therefore go to up to `lanes` streams of default priority, so the blocks of one chain fill the tails of the others; the
-    // caller's stream waits for all of them at the end.
+    // that step_together does not take go to up to `lanes` streams of default priority, so the blocks of one chain fill the tails of the
+    // others; the caller's stream waits for all of them at the end.
     void step_buckets(std::vector<std::vector<Item>>& ready) {
         // buckets of one shape and size (a shape split because it exceeds batch_elements) each keep their own pointer tables
         std::map<std::pair<std::vector<int64_t>, size_t>, int64_t> seen;
@@ -381,6 +459,7 @@ private:
             ordinals.push_back(seen[{matrix_shape(bucket[0].param, *bucket[0].group), bucket.size()}]++);
             one_device = one_device && bucket[0].param.device() == ready[0][0].param.device();
         }
+        if (one_device && step_together(ready)) return;
         if (ready.size() < 2 || lanes < 2 || !one_device) {
             for (size_t i = 0; i < ready.size(); ++i) step_bucket(ready[i], ordinals[i]);
             return;
@@ -428,6 +507,64 @@ private:
         join.now();
     }
 
+    // The chains of all buckets step by step together, a product of each in one launch, and one launch each for the momentum, the two
+    // stages in front of the chains and the weights: 20 launches where buckets on lanes of their own take about 80 and the events that
+    // join them, which is all that a step of small matrices costs (one block of width 192: 253 -> 102 us, four of 256 316 -> 146, eight of
+    // 384 362 -> 349). Large sets gain by the mix of tile lengths (28 blocks of width 1152 12560 -> 12280 us, eight of 1280 5842 ->
+    // 5185). The recurrence on the Gram matrix gains less there: its launches are several rounds of short tiles with a tail each, which lanes
+    // fill (28 blocks of 384 805 us on lanes, 881 together; four of 512 373 and 331), so beyond TOGETHER_GRAM it keeps the lanes.
+    static constexpr double TOGETHER_GRAM = 1e10;                // sum of m m (m + n) over the matrices
+    static constexpr int64_t TOGETHER_ELEMENTS = 1ll << 29;      // all arenas are held at once: 12 GB
+    bool step_together(std::vector<std::vector<Item>>& ready) {
+        if (ready.size() < 2 || ready.size() > 8) return false;
+        const Item& head = ready[0][0];
+        const Group& g = *head.group;
+        const viola_stream_t stream = stream_of(head.param);
+        int64_t elements = 0;
+        double work = 0;
+        for (const auto& bucket : ready)
+            for (const Item& it : bucket) {
+                const Group& h = *it.group;
+                const std::vector<int64_t> shape = matrix_shape(it.param, h);
+                if (it.param.numel() == 0 || it.param.numel() % h.tile || h.granularity != 0 || it.step != head.step || h.tile != g.tile || h.momentum != g.momentum ||
+                    h.nesterov != g.nesterov || h.rounding != g.rounding || h.gram != g.gram || h.ns_steps != g.ns_steps || h.lr != g.lr ||
+                    h.weight_decay != g.weight_decay || h.match_rms != g.match_rms || shape.back() % 8 || shape[shape.size() - 2] % 8)
+                    return false;
+                if (it.param.scalar_type() != at::kFloat || !aligned(it.param.const_data_ptr(), 16)) return false;
+                elements += it.param.numel();
+                work += (double)it.param.numel() * (double)std::min(shape.back(), shape[shape.size() - 2]) *
+                        (1. + (double)std::min(shape.back(), shape[shape.size() - 2]) / (double)std::max(shape.back(), shape[shape.size() - 2]));
+            }
+        if (elements > TOGETHER_ELEMENTS || (g.gram && work > TOGETHER_GRAM)) return false;
+        std::vector<MomentumRow> momentum_rows;
+        std::vector<WeightRow> weight_rows;
+        std::vector<Tensor> inputs;
+        for (const auto& bucket : ready) {
+            const std::vector<int64_t> shape = matrix_shape(bucket[0].param, *bucket[0].group);
+            const int64_t count = bucket[0].param.numel(), rows = shape[shape.size() - 2], cols = shape.back();
+            inputs.push_back(at::empty({(int64_t)bucket.size(), count / (rows * cols), rows, cols}, at::TensorOptions().dtype(at::kBFloat16).device(head.param.device())));
+            char* out = static_cast<char*>(inputs.back().mutable_data_ptr());
+            for (const Item& it : bucket) {
+                momentum_rows.push_back({it.grad.contiguous(), it.q, it.scale, out, momentum_key(it), count});
+                out += 2 * count;
+            }
+        }
+        if (!momentum_together(tables_, {}, (int64_t)g.gram, momentum_rows, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step, stream)) return false;
+        std::vector<Chain> chains;
+        for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram));
+        run_together(chains, stream);
+        for (size_t i = 0; i < ready.size(); ++i) {
+            const int64_t count = ready[i][0].param.numel(), rows = chains[i].matrix.size(-2), cols = chains[i].matrix.size(-1);
+            const char* from = static_cast<const char*>(chains[i].result.const_data_ptr());
+            for (const Item& it : ready[i]) {
+                weight_rows.push_back({it.param, from, count, (float)update_scale(g, rows, cols)});
+                from += 2 * count;
+            }
+        }
+        TORCH_INTERNAL_ASSERT(weights_together(tables_, {}, (int64_t)g.gram, weight_rows, chains[0].result.scalar_type(), (float)g.lr, (float)g.weight_decay, stream));
+        return true;
+    }
+
     static double update_scale(const Group& g, int64_t rows, int64_t cols) {
         return g.match_rms ? .2 * std::pow((double)std::max(rows, cols), .5) : std::pow(std::max(1., (double)rows / (double)cols), .5);
     }
@@ -453,9 +590,9 @@ private:
             const Group& h = *it.group;
             together = it.step == head.step && h.granularity == g.granularity && h.tile == g.tile && h.momentum == g.momentum && h.nesterov == g.nesterov &&
                        h.rounding == g.rounding;
-            momentum_rows.push_back({grads[i], it.q, it.scale, out + 2 * count * i, momentum_key(it)});
+            momentum_rows.push_back({grads[i], it.q, it.scale, out + 2 * count * i, momentum_key(it), count});
         }
-        if (!together || !momentum_together(tables_, shape, ordinal, momentum_rows, count, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step, stream)) {
+        if (!together || !momentum_together(tables_, shape, ordinal, momentum_rows, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step, stream)) {
             for (size_t i = 0; i < bucket.size(); ++i) {
                 const Item& it = bucket[i];
                 const Group& h = *it.group;
@@ -478,11 +615,9 @@ private:
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Group& h = *bucket[i].group;
             together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms;
-            weight_rows.push_back({bucket[i].param, from + 2 * count * i});
+            weight_rows.push_back({bucket[i].param, from + 2 * count * i, count, (float)update_scale(g, rows, cols)});
         }
-        if (together && weights_together(tables_, shape, ordinal, weight_rows, count, updates.scalar_type(), (float)g.lr, (float)g.weight_decay,
-                                         (float)update_scale(g, rows, cols), stream))
-            return;
+        if (together && weights_together(tables_, shape, ordinal, weight_rows, updates.scalar_type(), (float)g.lr, (float)g.weight_decay, stream)) return;
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Item& it = bucket[i];
             const Group& h = *it.group;
@@ -553,9 +688,9 @@ void register_optimizer(py::module_& m) {
         for (size_t i = 0; i < grads.size(); ++i) {
             TORCH_CHECK(grads[i].is_cuda() && qs[i].is_cuda() && scales[i].is_cuda() && outs[i].is_cuda(), "viola_amd kernels run on the GPU only");
             if (outs[i].scalar_type() != at::kBFloat16 || outs[i].numel() < grads[i].numel()) return false;
-            rows.push_back({grads[i], qs[i], scales[i], outs[i].mutable_data_ptr(), keys[i]});
+            rows.push_back({grads[i], qs[i], scales[i], outs[i].mutable_data_ptr(), keys[i], grads[0].numel()});
         }
-        return momentum_together(tables, {}, 0, rows, grads[0].numel(), tile, (float)beta, (float)inv_loss_scale, nesterov, rounding, step, stream_of(grads[0]));
+        return momentum_together(tables, {}, 0, rows, tile, (float)beta, (float)inv_loss_scale, nesterov, rounding, step, stream_of(grads[0]));
     }));
     m.def("weight_update_many", torch::wrap_pybind_function([](Tables& tables, const std::vector<Tensor>& weights, const std::vector<Tensor>& updates, double lr,
                                                                double weight_decay, double update_scale) {
@@ -563,10 +698,9 @@ void register_optimizer(py::module_& m) {
         for (size_t i = 0; i < weights.size(); ++i) {
             TORCH_CHECK(weights[i].is_cuda() && updates[i].is_cuda(), "viola_amd kernels run on the GPU only");
             if (updates[i].scalar_type() != updates[0].scalar_type() || updates[i].numel() != weights[i].numel() || !updates[i].is_contiguous()) return false;
-            rows.push_back({weights[i], updates[i].const_data_ptr()});
+            rows.push_back({weights[i], updates[i].const_data_ptr(), weights[0].numel(), (float)update_scale});
         }
-        return weights_together(tables, {}, 0, rows, weights[0].numel(), updates[0].scalar_type(), (float)lr, (float)weight_decay, (float)update_scale,
-                                stream_of(weights[0]));
+        return weights_together(tables, {}, 0, rows, updates[0].scalar_type(), (float)lr, (float)weight_decay, stream_of(weights[0]));
     }));
     m.def("adam_update_many", torch::wrap_pybind_function([](Tables& tables, const std::vector<Tensor>& weights, const std::vector<Tensor>& grads,
                                                              const std::vector<Tensor>& firsts, const std::vector<Tensor>& seconds, const std::vector<int64_t>& keys,

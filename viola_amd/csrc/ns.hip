@@ -7,6 +7,7 @@
 // consecutive n. b may be given as [n, k] (transpose_b) or [k, n]; the latter is transposed on
 // its way into LDS.
 #include <type_traits>
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -280,8 +281,7 @@ template <typename TIn, bool IS_BF16> __device__ __forceinline__ float ns_workin
 }
 
 template <typename TIn, bool IS_BF16>
-__global__ __launch_bounds__(256) void ns_sumsq16_kernel(const TIn* __restrict__ in, float* __restrict__ workspace, int64_t count) {
-    const int64_t bz = blockIdx.y;
+__device__ __forceinline__ void ns_sumsq16(const TIn* __restrict__ in, float* __restrict__ workspace, int64_t count, int64_t bz) {
     const uint4* src = reinterpret_cast<const uint4*>(in + bz * count);
     const int64_t octets = count / 8;
     const int64_t per = (octets + PARTS - 1) / PARTS;
@@ -304,20 +304,25 @@ __global__ __launch_bounds__(256) void ns_sumsq16_kernel(const TIn* __restrict__
     if (threadIdx.x == 0) workspace[bz * PARTS + blockIdx.x] = (partial[0] + partial[1]) + (partial[2] + partial[3]);
 }
 
+template <typename TIn, bool IS_BF16>
+__global__ __launch_bounds__(256) void ns_sumsq16_kernel(const TIn* __restrict__ in, float* __restrict__ workspace, int64_t count) {
+    ns_sumsq16<TIn, IS_BF16>(in, workspace, count, blockIdx.y);
+}
+
 template <bool IS_BF16>
 __device__ __forceinline__ uint32_t ns_scaled(float v, float denom, const SharedDivisor& d) {
     return f32_to_half<IS_BF16>(d.fast ? d.quotient(v) : v / denom);
 }
 
+// Block `part` of `parts` of matrix bz.
 template <typename TIn, bool IS_BF16>
-__global__ __launch_bounds__(256) void ns_scale16_kernel(const TIn* __restrict__ in, uint16_t* __restrict__ out,
-                                                          const float* __restrict__ workspace, int64_t count) {
+__device__ __forceinline__ void ns_scale16(const TIn* __restrict__ in, uint16_t* __restrict__ out, const float* __restrict__ workspace, int64_t count,
+                                           int64_t bz, uint32_t part, uint32_t parts) {
     __shared__ float denom_s;
-    const int64_t bz = blockIdx.y;
     const uint4* src = reinterpret_cast<const uint4*>(in + bz * count);
     uint4* dst = reinterpret_cast<uint4*>(out + bz * count);
-    const int64_t octets = count / 8, step = (int64_t)gridDim.x * 256;
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t octets = count / 8, step = (int64_t)parts * 256;
+    int64_t i = (int64_t)part * 256 + threadIdx.x;
     uint4 next = i < octets ? src[i] : make_uint4(0, 0, 0, 0);               // under way while the denominator is formed
     const float denom = ns_denominator(workspace, bz, IS_BF16, &denom_s);
     const SharedDivisor divisor(denom, 0.0f);
@@ -336,6 +341,12 @@ __global__ __launch_bounds__(256) void ns_scale16_kernel(const TIn* __restrict__
         }
         dst[i] = make_uint4(o[0], o[1], o[2], o[3]);
     }
+}
+
+template <typename TIn, bool IS_BF16>
+__global__ __launch_bounds__(256) void ns_scale16_kernel(const TIn* __restrict__ in, uint16_t* __restrict__ out,
+                                                          const float* __restrict__ workspace, int64_t count) {
+    ns_scale16<TIn, IS_BF16>(in, out, workspace, count, blockIdx.y, blockIdx.x, gridDim.x);
 }
 
 // FP32 inputs (a gradient handed over as it is) in 16-byte accesses: four loads in flight per thread for the sum of
@@ -399,21 +410,19 @@ __global__ __launch_bounds__(256) void ns_scale32_kernel(const float* __restrict
 // Transposed: a wavefront parks 32 rows x 64 columns of raw 16-bit values in LDS and reads them back with
 // ds_read_b64_tr_b16, so each lane ends up with the 32 rows of one column = 64 contiguous bytes of the output.
 template <typename TIn, bool IS_BF16>
-__global__ __launch_bounds__(256) void ns_scale16_transposed_kernel(const TIn* __restrict__ in, uint16_t* __restrict__ out,
-                                                                     const float* __restrict__ workspace, int64_t rows,
-                                                                     int64_t cols) {
+__device__ __forceinline__ void ns_scale16_transposed(const TIn* __restrict__ in, uint16_t* __restrict__ out, const float* __restrict__ workspace,
+                                                      int64_t rows, int64_t cols, int64_t bz, uint32_t row_block, uint32_t col_block) {
     constexpr int LD = 64 + 32;
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
     __shared__ __attribute__((aligned(16))) uint16_t park[4][32 * LD];
     __shared__ float denom_s;
-    const int64_t bz = blockIdx.z;
     const float denom = ns_denominator(workspace, bz, IS_BF16, &denom_s);
     const SharedDivisor divisor(denom, 0.0f);
     const TIn* src = in + bz * rows * cols;
     uint16_t* dst = out + bz * rows * cols;
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    const int64_t r0 = (int64_t)blockIdx.y * 128 + wave * 32, c0 = (int64_t)blockIdx.x * 64;
+    const int64_t r0 = (int64_t)row_block * 128 + wave * 32, c0 = (int64_t)col_block * 64;
     if (r0 >= rows) return;
     uint16_t* mine = park[wave];
     const int lr = lane / 8, ch = lane % 8;
@@ -449,6 +458,61 @@ __global__ __launch_bounds__(256) void ns_scale16_transposed_kernel(const TIn* _
         } else {
             for (int e = 0; e < 32 && r0 + e < rows; ++e) row_out[e] = (uint16_t)(o[e / 2] >> (16 * (e % 2)));
         }
+    }
+}
+
+template <typename TIn, bool IS_BF16>
+__global__ __launch_bounds__(256) void ns_scale16_transposed_kernel(const TIn* __restrict__ in, uint16_t* __restrict__ out,
+                                                                     const float* __restrict__ workspace, int64_t rows,
+                                                                     int64_t cols) {
+    ns_scale16_transposed<TIn, IS_BF16>(in, out, workspace, rows, cols, blockIdx.z, blockIdx.y, blockIdx.x);
+}
+
+// Both stages for matrices of several shapes, one launch each: the values of the kernels above.
+struct NsPrepareMany {
+    struct Shape {
+        const bf16_t* in;
+        uint16_t* out;
+        int64_t rows, cols;
+        int batch, parts;                                                     // parts: blocks per matrix of the scaling pass
+    } shape[NS_MANY];
+    int count;
+};
+
+// the shape that block `rest` belongs to, with `each` blocks per matrix of a shape; rest becomes its number there
+template <typename Each>
+__device__ __forceinline__ int ns_shape_of(const NsPrepareMany& many, uint32_t& rest, int& first, Each each) {
+    int at = 0;
+    first = 0;                                                                // matrices before this shape's: their sums come first
+    while (at + 1 < many.count && rest >= (uint32_t)many.shape[at].batch * each(many.shape[at])) {
+        rest -= (uint32_t)many.shape[at].batch * each(many.shape[at]);
+        first += many.shape[at++].batch;
+    }
+    return at;
+}
+
+template <bool IS_BF16>
+__global__ __launch_bounds__(256) void ns_sumsq16_many(NsPrepareMany many, float* __restrict__ workspace) {
+    uint32_t matrix = blockIdx.y;
+    int first;
+    const int at = ns_shape_of(many, matrix, first, [](const NsPrepareMany::Shape&) { return 1u; });
+    const NsPrepareMany::Shape& shape = many.shape[at];
+    ns_sumsq16<bf16_t, IS_BF16>(shape.in, workspace + (int64_t)first * PARTS, shape.rows * shape.cols, matrix);
+}
+
+template <bool IS_BF16>
+__global__ __launch_bounds__(256) void ns_scale16_many(NsPrepareMany many, const float* __restrict__ workspace) {
+    uint32_t block = blockIdx.x;
+    int first;
+    const int at = ns_shape_of(many, block, first, [](const NsPrepareMany::Shape& shape) { return (uint32_t)shape.parts; });
+    const NsPrepareMany::Shape& shape = many.shape[at];
+    const uint32_t matrix = block / (uint32_t)shape.parts, part = block % (uint32_t)shape.parts;
+    workspace += (int64_t)first * PARTS;
+    if (shape.rows > shape.cols) {
+        const uint32_t across = (uint32_t)((shape.cols + 63) / 64);
+        ns_scale16_transposed<bf16_t, IS_BF16>(shape.in, shape.out, workspace, shape.rows, shape.cols, matrix, part / across, part % across);
+    } else {
+        ns_scale16<bf16_t, IS_BF16>(shape.in, shape.out, workspace, shape.rows * shape.cols, matrix, part, (uint32_t)shape.parts);
     }
 }
 
@@ -595,6 +659,55 @@ extern "C" int viola_ns_gemm(const void* a, const void* bmat, const void* residu
     if (vec) VIOLA_NS(false, false, true);
     VIOLA_NS(false, false, false);
 #undef VIOLA_NS
+}
+
+extern "C" int viola_ns_gemm_many(const viola_ns_product* products, int count, int dtype, viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG((dtype == VIOLA_BF16 || dtype == VIOLA_F16) && count >= 0 && (count == 0 || products));
+    if (count > NS_MANY) return VIOLA_EUNSUPPORTED;
+    NsMany many{};
+    for (int i = 0; i < count; ++i) {
+        const viola_ns_product& p = products[i];
+        VIOLA_CHECK_ARG(p.epilogue >= 0 && p.epilogue <= 2 && p.batch >= 0 && p.m >= 0 && p.n >= 0 && p.k >= 0);
+        if (p.batch == 0 || p.m == 0 || p.n == 0) continue;
+        VIOLA_CHECK_ARG(p.out && (p.k == 0 || (p.a && p.b)) && (p.epilogue == 0 || p.residual));
+        many.product[many.count++] = {static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), static_cast<const uint16_t*>(p.residual),
+                                      static_cast<uint16_t*>(p.out), static_cast<uint16_t*>(p.out_diag), p.batch, p.m, p.n, p.k, p.add_diag, p.transpose_out,
+                                      ns_is_mirrored(p.a, p.b, p.transpose_b, p.m, p.n, p.transpose_out), 0, 0, 0, 0, !p.transpose_b, p.epilogue};
+    }
+    if (many.count == 0) return 0;
+    // the longest k first: their tiles are not what the launch waits for at its end
+    std::stable_sort(many.product, many.product + many.count, [](const NsArgs& a, const NsArgs& b) { return a.k > b.k; });
+    if (!launch_ns_gemm_many(many, dtype == VIOLA_BF16, stream)) return VIOLA_EUNSUPPORTED;
+    return viola_launch_status();
+}
+
+extern "C" int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count, int dtype, float* workspace, viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG((dtype == VIOLA_BF16 || dtype == VIOLA_F16) && count >= 0 && (count == 0 || (shapes && workspace)));
+    if (count > NS_MANY) return VIOLA_EUNSUPPORTED;
+    NsPrepareMany many{};
+    int64_t matrices = 0, blocks = 0;
+    for (int i = 0; i < count; ++i) {
+        const viola_ns_matrices& s = shapes[i];
+        VIOLA_CHECK_ARG(s.batch >= 0 && s.rows >= 0 && s.cols >= 0);
+        if (s.batch == 0 || s.rows == 0 || s.cols == 0) continue;
+        VIOLA_CHECK_ARG(s.in && s.out);
+        const bool aligned = reinterpret_cast<uintptr_t>(s.in) % 16 == 0 && reinterpret_cast<uintptr_t>(s.out) % 16 == 0;
+        if (!aligned || s.cols % 8 || (matrices += s.batch) > 65535) return VIOLA_EUNSUPPORTED;
+        const int64_t parts = s.rows > s.cols ? ((s.cols + 63) / 64) * ((s.rows + 127) / 128) : ns_scale_blocks(s.rows * s.cols / 8, s.batch);
+        if (parts >= (1ll << 31) || (blocks += parts * s.batch) >= (1ll << 31)) return VIOLA_EUNSUPPORTED;
+        many.shape[many.count++] = {static_cast<const bf16_t*>(s.in), static_cast<uint16_t*>(s.out), s.rows, s.cols, (int)s.batch, (int)parts};
+    }
+    if (many.count == 0) return 0;
+    if (dtype == VIOLA_BF16) {
+        VIOLA_LAUNCH(ns_sumsq16_many<true>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
+        VIOLA_LAUNCH(ns_scale16_many<true>, dim3((unsigned)blocks), dim3(256), 0, stream, many, workspace);
+    } else {
+        VIOLA_LAUNCH(ns_sumsq16_many<false>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
+        VIOLA_LAUNCH(ns_scale16_many<false>, dim3((unsigned)blocks), dim3(256), 0, stream, many, workspace);
+    }
+    return viola_launch_status();
 }
 
 extern "C" int viola_ns_prepare(const void* in, int in_dtype, void* out, int dtype, int64_t batch, int64_t rows,

@@ -17,6 +17,15 @@ struct NsArgs {
     int tiles_m, tiles_n;
     int group_m;                // tile rows per band of the work order (ns_fast.hip)
     int64_t tiles;              // batch * tiles_m * tiles_n
+    int b_kn, epilogue;         // read where products of several kinds share a launch
+};
+
+// Products of one launch (by value in the kernel's arguments).
+constexpr int NS_MANY = 8;
+struct NsMany {
+    NsArgs product[NS_MANY];
+    int rounds[NS_MANY];        // blocks of a product per XCD
+    int count;
 };
 
 // Tile shapes of the tiled kernel (rows x columns of output per block); NS_TILE_GENERIC is the kernel in ns.hip that
@@ -26,7 +35,8 @@ NsTile ns_choose_tile(int64_t batch, int64_t m, int64_t n, bool symmetric);
 bool ns_fast_takes(const NsArgs& args);
 
 // Launches the tiled kernel when the shape qualifies (16-byte aligned rows, k and n multiples of 8,
-// one matrix below 2 GiB); returns false without launching otherwise.
+// one matrix below 2 GiB); returns false without launching otherwise. `many`: unless every product qualifies.
+bool launch_ns_gemm_many(const NsMany& many, bool is_bf16, hipStream_t stream);
 bool launch_ns_gemm_fast(const NsArgs& args, bool is_bf16, bool b_kn, int epilogue, hipStream_t stream);
 
 }  // namespace viola
