@@ -264,7 +264,7 @@ __device__ __forceinline__ void ns_tile(const NsArgs& p, int64_t work, uint16_t*
         }
     };
     uint4 mirrored[EARLY ? COL_ITERS : 1];
-    if (EARLY && EPILOGUE && !p.transpose_out) {
+    if (EARLY && EPILOGUE) {
         fetch_residual(0, ahead[0]);
         if (mirror) {
 #pragma unroll
@@ -402,7 +402,7 @@ __device__ __forceinline__ void ns_tile(const NsArgs& p, int64_t work, uint16_t*
             }
         return make_uint4(w[0], w[1], w[2], w[3]);
     };
-    if (!EARLY && EPILOGUE && !p.transpose_out) fetch_residual(0, ahead[0]);
+    if (!EARLY && EPILOGUE) fetch_residual(0, ahead[0]);
 #pragma unroll
     for (int j = 0; j < WM; ++j) {
 #pragma unroll
@@ -412,24 +412,28 @@ __device__ __forceinline__ void ns_tile(const NsArgs& p, int64_t work, uint16_t*
                 *reinterpret_cast<uint2*>(&park[l32 * PLD + i * 32 + r4 * 8 + lhi * 4]) =
                     make_uint2(ns_narrow2<IS_BF16>(acc[i][j][r4 * 4], acc[i][j][r4 * 4 + 1]), ns_narrow2<IS_BF16>(acc[i][j][r4 * 4 + 2], acc[i][j][r4 * 4 + 3]));
         const uint32_t row0 = tile_row + j * 32;                          // of the parked 32 x WCOLS block
-        if (!p.transpose_out) {
-            if (EPILOGUE && j + 1 < WM) fetch_residual(j + 1, ahead[(j + 1) & 1]);
+        if (EPILOGUE && j + 1 < WM) fetch_residual(j + 1, ahead[(j + 1) & 1]);
 #pragma unroll
-            for (int it = 0; it < ROW_ITERS; ++it) {
-                const int id = it * WAVE + lane, pr = id / PIECES, pc = id % PIECES;
-                const uint32_t row = row0 + pr, col = col0 + pc * 8;
-                const uint4 raw = *reinterpret_cast<const uint4*>(&park[pr * PLD + pc * 8]);
-                if (row >= um || col >= un) continue;                     // n is a multiple of 8: whole pieces
-                const uint4 res = EPILOGUE ? ahead[j & 1][it] : make_uint4(0, 0, 0, 0);
-                const uint4 o = make_uint4(finish(raw.x, res.x), finish(raw.y, res.y), finish(raw.z, res.z), finish(raw.w, res.w));
-                store_piece(out, row * un + col, o);
-                if (out_diag) store_piece(out_diag, row * un + col, row - col < 8u ? with_diagonal(o, row - col) : o);
+        for (int it = 0; it < ROW_ITERS; ++it) {
+            const int id = it * WAVE + lane, pr = id / PIECES, pc = id % PIECES;
+            const uint32_t row = row0 + pr, col = col0 + pc * 8;
+            uint4* at = reinterpret_cast<uint4*>(&park[pr * PLD + pc * 8]);
+            const uint4 raw = *at;
+            const uint4 res = EPILOGUE ? ahead[j & 1][it] : make_uint4(0, 0, 0, 0);
+            const uint4 o = make_uint4(finish(raw.x, res.x), finish(raw.y, res.y), finish(raw.z, res.z), finish(raw.w, res.w));
+            if (p.transpose_out) {                                        // stored below, from here
+                if (EPILOGUE) *at = o;
+                continue;
             }
+            if (row >= um || col >= un) continue;                         // n is a multiple of 8: whole pieces
+            store_piece(out, row * un + col, o);
+            if (out_diag) store_piece(out_diag, row * un + col, row - col < 8u ? with_diagonal(o, row - col) : o);
         }
         if (p.transpose_out || mirror) {
-            // element [n, m] of the placement has the product parked at [m][n]. A mirrored element takes the residual of
+            // element [n, m] of the placement has the product computed at [m][n]. A mirrored element takes the residual of
             // its own position (a . a^T is symmetric, its residual need not be; an off-diagonal tile holds no diagonal
-            // element), a transposed result the residual of the position it was computed for.
+            // element), a transposed result has taken that of the position it was computed for, along the rows. (Fetched here, element by
+            // element, 28 x 1152 x 4608 x 1152 transposed took 556 us instead of 388, one of 1024 x 4096 x 1024 23.3 instead of 17.)
             const bool whole = m % 8 == 0;
 #pragma unroll EARLY ? COL_ITERS : 1
             for (int it = 0; it < COL_ITERS; ++it) {                          // (not unrolled while the accumulators of later blocks are live)
@@ -439,16 +443,11 @@ __device__ __forceinline__ void ns_tile(const NsArgs& p, int64_t work, uint16_t*
 #pragma unroll
                 for (int e = 0; e < 8; e += 2) pw[e / 2] = (uint32_t)park[(lm + e) * PLD + ln] | ((uint32_t)park[(lm + e + 1) * PLD + ln] << 16);
                 if (orow >= un || ocol >= um) continue;
-                uint32_t rw[4] = {0, 0, 0, 0};
+                uint4 o = make_uint4(pw[0], pw[1], pw[2], pw[3]);
                 if (EPILOGUE && mirror) {                                 // m == n, a multiple of 8: a whole piece of residual row orow
                     const uint4 res = EARLY ? mirrored[EARLY ? it : 0] : load_piece(residual, orow * un + ocol);
-                    rw[0] = res.x; rw[1] = res.y; rw[2] = res.z; rw[3] = res.w;
-                } else if (EPILOGUE) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (ocol + e < um) rw[e / 2] |= (uint32_t)residual[(size_t)((ocol + e) * un + orow)] << (16 * (e % 2));
+                    o = make_uint4(finish(o.x, res.x), finish(o.y, res.y), finish(o.z, res.z), finish(o.w, res.w));
                 }
-                uint4 o = make_uint4(finish(pw[0], rw[0]), finish(pw[1], rw[1]), finish(pw[2], rw[2]), finish(pw[3], rw[3]));
                 const uint4 od = !mirror && orow - ocol < 8u ? with_diagonal(o, orow - ocol) : o;
                 if (whole) {
                     store_piece(out, orow * um + ocol, o);
