@@ -223,6 +223,11 @@ int viola_group_gemm(const void* a, int a_dtype, const void* b, int b_dtype, con
  * nothing is launched. VIOLA_EINVAL for sizes that the guarded kernel takes (k % 16 != 0, operands or scales beyond 2 GiB). */
 int viola_group_gemm_form(int64_t m, int64_t n, int64_t k, int row_scaled_b, int row_groups, int k_groups);
 
+/* Which form viola_tensor_gemm and viola_mx_gemm run a plain product in (operands that the fast kernels take, outputs beyond those of
+ * viola_skinny_linear): 0 blocks of 128 x 128 or less, several to a CU; 1 tiles of 256 x 256, 2 of 256 x 128, 3 of 128 x 128; 4 full rounds of
+ * 256 x 256 and a last round of 128 x 128. Host arithmetic only, nothing is launched. */
+int viola_scaled_gemm_form(int64_t m, int64_t n, int64_t k);
+
 /* viola_group_gemm with a scale per row and 32 k on both sides (ar = br = 1, ak = bk = 32), no bias, the k range cut into `parts` (2 .. 64)
  * that are computed side by side: their FP32 products go to workspace (parts * (m * n rounded up to 4) floats, 16-byte aligned) and
  * are added in ascending order. viola_group_gemm_parts says how many are worth it (1: viola_group_gemm): never so many that the

@@ -51,6 +51,12 @@ extern "C" int viola_group_gemm(const void* a, int a_dtype, const void* b, int b
     return launch_out<MODE_PLAIN>(p, a_dtype, b_dtype, bias_dtype, out_dtype, rowscale, vec, dim3((unsigned)gx, (unsigned)gy), stream);
 }
 
+extern "C" int viola_scaled_gemm_form(int64_t m, int64_t n, int64_t k) {
+    constexpr int64_t LARGEST = 1ll << 31;
+    VIOLA_CHECK_ARG(m > 0 && n > 0 && k > 0 && m < LARGEST && n < LARGEST && k < LARGEST);
+    return choose_scaled_tile(m, n, k);
+}
+
 extern "C" int viola_group_gemm_form(int64_t m, int64_t n, int64_t k, int row_scaled_b, int row_groups, int k_groups) {
     constexpr int64_t LARGEST = 1ll << 31;
     VIOLA_CHECK_ARG(m > 0 && n > 0 && k > 0 && m < LARGEST && n < LARGEST && k < LARGEST && k % 16 == 0);
@@ -155,7 +161,7 @@ static bool gated_in_two_passes(int64_t m, int64_t k, int64_t h, const void* aux
     const int64_t piece = out_dtype == VIOLA_F32 ? 4 : 8;
     if (!aux || h % piece != 0 || !aligned16(aux) || !aligned16(out) || m * (h / piece) / 256 >= 0x7fffffff) return false;   // the pass is one launch of 256-thread blocks
     if (backward) return m * h >= (1 << 17);
-    const ScaledTile tile = choose_scaled_tile(m, 2 * h, k);
+    const ScaledTile tile = choose_scaled_tile(m, 2 * h, k, false);
     return tile == SCALED_TILE_L || tile == SCALED_TILE_M;
 }
 
@@ -348,7 +354,7 @@ extern "C" int viola_mx_gated_gemm_encode(const void* a, int a_dtype, const void
         (br != 1 && br % 32 != 0) || h % br != 0 || h % 32 != 0 || m % 32 != 0 || !aligned16(aux) || !aligned16(enc) ||
         !aligned16(enc_t))
         return VIOLA_EUNSUPPORTED;
-    if (aux && enc_t && aux_dtype != VIOLA_F32 && choose_scaled_tile(m, 2 * h, k) != SCALED_TILE_FAST) {
+    if (aux && enc_t && aux_dtype != VIOLA_F32 && choose_scaled_tile(m, 2 * h, k, false) != SCALED_TILE_FAST) {
         // the plain GEMM on the tile that suits it writes [g | u], one pass over it writes the codes of h in both layouts
         // (the encoding epilogue does not fit the large tiles' registers; 2.0 ms against 2.5 ms at 16384 x 4096 -> 11008)
         const int status = mx_gemm(a, a_dtype, b, b_dtype, sa, sb, m, 2 * h, k, ar, br, bias, bias_dtype, aux, 2 * h, aux_dtype, stream);

@@ -94,8 +94,10 @@ bool launch_gated_pieces(const void* z, const void* dy, int64_t dy_stride, void*
 // group_gemm_fast has no rounds to speak of (three small blocks per CU, their stores under each other's math): 0.31 per tile
 // and chunk of a CU's share + 0.7 per tile. What that comes to: 8192 x 1024 x 4096 M (30 us), 4096 x 1152 x 4608 M (26),
 // 4096 x 4096 x 4096 L (55), 4096 x 4608 x 1152 stays (30), 2048 x 1152 x 4608 S (19).
-enum ScaledTile { SCALED_TILE_FAST = 0, SCALED_TILE_L, SCALED_TILE_M, SCALED_TILE_S };
-inline ScaledTile choose_scaled_tile(int64_t m, int64_t n, int64_t k) {
+enum ScaledTile { SCALED_TILE_FAST = 0, SCALED_TILE_L, SCALED_TILE_M, SCALED_TILE_S, SCALED_TILE_L_THEN_S };
+// L_THEN_S: full rounds of L, and the last up to 64 tiles as four S each (`last`; gated products do not run that way), which take
+// 0.22 .. 0.40 a chunk, as the share of CUs, + 4.
+inline ScaledTile choose_scaled_tile(int64_t m, int64_t n, int64_t k, bool last = true) {
     constexpr int64_t CUS = 256;
     auto tiles = [&](int64_t rows, int64_t cols) { return ((m + rows - 1) / rows) * ((n + cols - 1) / cols); };
     const int64_t small = tiles(128, 128);
@@ -113,6 +115,10 @@ inline ScaledTile choose_scaled_tile(int64_t m, int64_t n, int64_t k) {
     if (pairs < least) { least = pairs; best = SCALED_TILE_S; }
     if (medium < least) { least = medium; best = SCALED_TILE_M; }
     if (large < least) { least = large; best = SCALED_TILE_L; }
+    const int64_t whole = tiles(256, 256) / CUS, rest = tiles(256, 256) % CUS;
+    if (last && whole > 0 && rest > 0 && rest <= CUS / 4 &&
+        (double)whole * (chunks * 0.71 + 8.5) + chunks * (0.22 + 0.18 * (double)rest / (CUS / 4)) + 4.0 < least)
+        best = SCALED_TILE_L_THEN_S;
     return best;
 }
 

@@ -34,7 +34,7 @@ static int launch_scaled_gemm_fast(const GemmArgs& args, int mode, int a_dtype, 
     // a gated forward that keeps no [g | u] takes the large tile where the plain product would (with [g | u] kept it is that product
     // and a pass over it)
     const ScaledTile tile = mode == MODE_PLAIN ? choose_scaled_tile(p.m, p.n, p.k)
-                            : mode == MODE_GATED_FWD && !p.aux && !p.enc ? choose_scaled_tile(p.m, 2 * p.n, p.k) : SCALED_TILE_FAST;
+                            : mode == MODE_GATED_FWD && !p.aux && !p.enc ? choose_scaled_tile(p.m, 2 * p.n, p.k, false) : SCALED_TILE_FAST;
     if (mode == MODE_PLAIN ? tile != SCALED_TILE_FAST : tile == SCALED_TILE_L)
         return (MX ? launch_mx_pingpong : launch_tensor_pingpong)(p, tile, mode != MODE_PLAIN, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
     // fewer than 128 tiles of 128 x 128 (from 128 up choose_scaled_tile finds an alternating-phase tile): halve the tile in n to

@@ -84,29 +84,25 @@ __device__ __forceinline__ void store_tile(const f32x16 (&total)[S::TN][S::TM], 
     }
 }
 
-// GATED: the tile's b rows are COLS / 2 gate rows, then the up rows of the same columns of h (sub-tiles 0 and 1 of a wave);
+// Bytes of LDS a tile takes: the ring, and behind it two scale blocks of 16 K groups (a rows, then b rows), later the bias row.
+template <bool MX, typename S>
+constexpr int pingpong_lds() {
+    return S::STAGES * S::STAGE + (MX ? 2 * (S::ROWS + S::COLS) * MX_GROUPS : S::COLS * 4);
+}
+
+// One tile. GATED: the tile's b rows are COLS / 2 gate rows, then the up rows of the same columns of h (sub-tiles 0 and 1 of a wave);
 // out = act(g) * u, [g | u] itself is not kept.
-template <bool A_BF8, bool B_BF8, bool MX, typename S, int WAVES_PER_SIMD, bool GATED = false>
-__global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p, int bias_dtype, int out_dtype) {
+template <bool A_BF8, bool B_BF8, bool MX, typename S, bool GATED>
+__device__ __forceinline__ void pingpong_tile(const GemmArgs& p, int64_t m_begin, int64_t n_begin, uint8_t* lds, int bias_dtype, int out_dtype) {
     constexpr int TM = S::TM, TN = S::TN, STAGES = S::STAGES;
     static_assert(!GATED || TN == 2, "a gate and an up sub-tile per wave");
     constexpr int PANEL = GATED ? S::COLS / 2 : S::COLS;                     // columns of the output per tile
     constexpr int RING = STAGES * S::STAGE;
     constexpr int SCALE_BLOCK = (S::ROWS + S::COLS) * MX_GROUPS;             // scale bytes of 16 K groups, a rows then b rows
-    constexpr int TAIL = MX ? 2 * SCALE_BLOCK : S::COLS * 4;                 // behind the ring: scale blocks, later the bias row
-    static_assert(TAIL >= S::COLS * 4);
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[RING + TAIL];
+    static_assert(!MX || 2 * SCALE_BLOCK >= S::COLS * 4);
     const int tid = threadIdx.x, lane = tid % WAVE, l32 = lane % 32, lhi = lane / 32;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int wm = wave / S::WN, wn = wave % S::WN;
-
-    // ---- tile: contiguous ranges per XCD, walked in groups of 8 m tiles (see group_gemm_fast)
-    const int per_xcd = gridDim.x / 8;
-    const int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (t >= p.tiles_m * p.tiles_n) return;
-    const int group = 8 * p.tiles_n, first_m = t / group * 8;
-    const int rows_here = p.tiles_m - first_m < 8 ? p.tiles_m - first_m : 8;
-    const int64_t m_begin = (int64_t)(first_m + t % group % rows_here) * S::ROWS, n_begin = (int64_t)(t % group / rows_here) * PANEL;
 
     // ---- load plan: instruction `it` brings LOAD_ROWS rows of an operand, unit U = PIECES row + slot holds piece slot ^ swizzle(row)
     const i32x4 res_a = raw_resource(p.a + m_begin * p.lda), res_b = raw_resource(p.b);
@@ -334,6 +330,51 @@ __global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p,
     else finish(f16_t{});
 }
 
+// Tile `t` in the order of the walk: groups of 8 m tiles (see group_gemm_fast).
+__device__ __forceinline__ void pingpong_place(const GemmArgs& p, int t, int rows, int cols, int64_t& m_begin, int64_t& n_begin) {
+    const int group = 8 * p.tiles_n, first_m = t / group * 8;
+    const int rows_here = p.tiles_m - first_m < 8 ? p.tiles_m - first_m : 8;
+    m_begin = (int64_t)(first_m + t % group % rows_here) * rows;
+    n_begin = (int64_t)(t % group / rows_here) * cols;
+}
+
+template <bool A_BF8, bool B_BF8, bool MX, typename S, int WAVES_PER_SIMD, bool GATED = false>
+__global__ __launch_bounds__(512, WAVES_PER_SIMD) void gemm_pingpong(GemmArgs p, int bias_dtype, int out_dtype) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[pingpong_lds<MX, S>()];
+    const int t = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;       // contiguous ranges per XCD
+    if (t >= p.tiles_m * p.tiles_n) return;
+    int64_t m_begin, n_begin;
+    pingpong_place(p, t, S::ROWS, GATED ? S::COLS / 2 : S::COLS, m_begin, n_begin);
+    pingpong_tile<A_BF8, B_BF8, MX, S, GATED>(p, m_begin, n_begin, lds, bias_dtype, out_dtype);
+}
+
+// The first `whole` tiles (a multiple of 8) as they are, each of the others as tiles of the smaller shape T: a last round of few tiles, which
+// takes as long as a full one and leaves most CUs without a tile, is shared among four times as many. 256 x 256, then 128 x 128 (E8M0
+// scales, us): 4096 x 9216 x 1152 (two rounds and 64 tiles) 60.4 -> 53.8, 2891 x 5760 x 3072 (one and 20) 77 -> 60.5, 16384 x 1280 x 4096 (one and 64)
+// 100 -> 84, 4096 x 8704 x 8192 279 -> 247, 8192 x 8448 x 1024 (four and 32) 87.5 -> 81.8. (A last round on 256 x 128 takes 1 to 4 us
+// longer, rounds of 256 x 128 with a last one of 128 x 128 as long as 256 x 256 without: neither is built.)
+template <bool A_BF8, bool B_BF8, bool MX, typename S, typename T>
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_tail(GemmArgs p, int whole, int bias_dtype, int out_dtype) {
+    constexpr int ACROSS = S::COLS / T::COLS, EACH = S::ROWS / T::ROWS * ACROSS;
+    static_assert(S::ROWS % T::ROWS == 0 && S::COLS % T::COLS == 0);
+    constexpr int LDS_S = pingpong_lds<MX, S>(), LDS_T = pingpong_lds<MX, T>();
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_S > LDS_T ? LDS_S : LDS_T];
+    int64_t m_begin, n_begin;
+    const int block = blockIdx.x;
+    if (block < whole) {
+        pingpong_place(p, block % 8 * (whole / 8) + block / 8, S::ROWS, S::COLS, m_begin, n_begin);
+        pingpong_tile<A_BF8, B_BF8, MX, S, false>(p, m_begin, n_begin, lds, bias_dtype, out_dtype);
+        return;
+    }
+    const int rest = block - whole, u = rest % 8 * (((int)gridDim.x - whole) / 8) + rest / 8, t = whole + u / EACH, part = u % EACH;
+    if (t >= p.tiles_m * p.tiles_n) return;
+    pingpong_place(p, t, S::ROWS, S::COLS, m_begin, n_begin);
+    m_begin += part / ACROSS * T::ROWS;
+    n_begin += part % ACROSS * T::COLS;
+    if (m_begin >= p.m || n_begin >= p.n) return;                            // a tile across the edge: nothing of it here
+    pingpong_tile<A_BF8, B_BF8, MX, T, false>(p, m_begin, n_begin, lds, bias_dtype, out_dtype);
+}
+
 // The three tiles: 256 x 256 and 256 x 128 with one block per CU, 128 x 128 with one or two. A turn of the two halves costs some 200
 // cycles beside the math (barriers, the first LDS reads), which is a lot next to the 256 or 512 cycles of a wave's four or eight
 // MFMAs: where registers and LDS allow it a chunk is 128 k (whole cache lines of the operands, too). 256 x 256, in two stages for
@@ -364,11 +405,31 @@ static int launch_pingpong(const GemmArgs& args, int a_dtype, int b_dtype, int b
     return viola_launch_status();
 }
 
+template <bool MX, typename S, typename T>
+static int launch_pingpong_tail(const GemmArgs& args, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+    GemmArgs p = args;
+    p.tiles_m = (int)((p.m + S::ROWS - 1) / S::ROWS);
+    p.tiles_n = (int)((p.n + S::COLS - 1) / S::COLS);
+    if (!viola_is_float(out_dtype)) return VIOLA_EINVAL;
+    const bool a5 = a_dtype == VIOLA_E5M2, b5 = b_dtype == VIOLA_E5M2;
+    const int tiles = p.tiles_m * p.tiles_n, whole = tiles / 256 * 256, each = S::ROWS / T::ROWS * (S::COLS / T::COLS);
+    const dim3 grid((unsigned)(whole + ((int64_t)(tiles - whole) * each + 7) / 8 * 8)), block(512);
+    if (!a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_tail<false, false, MX, S, T>), grid, block, 0, stream, p, whole, bias_dtype, out_dtype);
+    else if (a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_tail<true, false, MX, S, T>), grid, block, 0, stream, p, whole, bias_dtype, out_dtype);
+    else if (!a5 && b5) VIOLA_LAUNCH((gemm_pingpong_tail<false, true, MX, S, T>), grid, block, 0, stream, p, whole, bias_dtype, out_dtype);
+    else VIOLA_LAUNCH((gemm_pingpong_tail<true, true, MX, S, T>), grid, block, 0, stream, p, whole, bias_dtype, out_dtype);
+    return viola_launch_status();
+}
+
 template <bool MX>
 static int launch_pingpong_tile(const GemmArgs& p, ScaledTile tile, bool gated, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
     if (gated) return launch_pingpong<MX, PingPongL, 2, true>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
-    if (tile == SCALED_TILE_L) return launch_pingpong<MX, PingPongL, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
-    if (tile == SCALED_TILE_M) return launch_pingpong<MX, PingPongM, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+    switch (tile) {
+        case SCALED_TILE_L: return launch_pingpong<MX, PingPongL, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+        case SCALED_TILE_L_THEN_S: return launch_pingpong_tail<MX, PingPongL, PingPongS>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+        case SCALED_TILE_M: return launch_pingpong<MX, PingPongM, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
+        default: break;
+    }
     if ((p.m + 127) / 128 * ((p.n + 127) / 128) <= 256) return launch_pingpong<MX, PingPongS, 2>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
     return launch_pingpong<MX, PingPongPairs, 4>(p, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
 }
