@@ -1,5 +1,5 @@
-"""GPU parity: per-tensor and block-scaled products whose last round of 256 x 256 tiles runs on tiles of 128 x 128. Integer operands and
-power-of-two scales, so every element must equal the integer product."""
+"""GPU parity: products whose last round of 256 x 256 tiles runs on smaller ones, per-tensor and block-scaled ones on tiles of 128 x 128, grouped
+ones on halves or quarters of 256 rows. Integer operands and power-of-two scales, so every element must equal the integer product."""
 
 import pytest
 import torch
@@ -33,3 +33,36 @@ def test_last_round_on_small_tiles(m, n, k, formats, out_dtype, scaling):
         out = g.gemm(qa, qb, sa, sb, (1, 32), (1, 32), out_dtype=out_dtype, bias=bias, native=True)
         want = spell(a, sa) @ spell(b, sb).T + bias
     assert torch.equal(out, want.to(out_dtype))
+
+
+# last rounds of 4, 52 and 64 tiles (quarters), 88, 96 and 128 (halves), 133 (whole); columns that end in a quarter, in front of one, with one;
+# k that ends in either half of a chunk
+GROUPED_LAST_ROUND = [(5000, 3300, 4112, (E4, E4), torch.bfloat16), (12000, 3072, 768, (E5, E4), torch.float32), (8192, 4608, 1056, (E4, E5), torch.float16),
+                      (6100, 6330, 2080, (E4, E4), torch.bfloat16), (8190, 4700, 1040, (E5, E5), torch.float32), (16384, 8704, 400, (E4, E4), torch.bfloat16),
+                      (11008, 3840, 2064, (E4, E4), torch.float32)]
+
+
+@pytest.mark.parametrize("m,n,k,formats,out_dtype", GROUPED_LAST_ROUND)
+def test_grouped_last_round(m, n, k, formats, out_dtype):
+    from viola_amd.nn import _grouped_kernels as g
+    torch.manual_seed(m + n + k)
+    a, b, groups = torch.randint(-2, 3, (m, k), device="cuda").float(), torch.randint(-2, 3, (n, k), device="cuda").float(), -(-k // 32)
+    scale = lambda rows: torch.exp2(torch.randint(-1, 2, (rows, groups), device="cuda").float())
+    sa, sb = scale(m), scale(-(-n // 32))
+    bias = torch.randint(-8, 9, (n,), device="cuda").float()
+    out = g.gemm(a.to(formats[0]), b.to(formats[1]), sa, sb, (1, 32), (32, 32), out_dtype=out_dtype, bias=bias)
+    spell = lambda t, s: t * s.repeat_interleave(32, 1)[:, :k]
+    want = spell(a, sa) @ spell(b, sb.repeat_interleave(32, 0)[:n]).T + bias
+    assert torch.equal(out, want.to(out_dtype))
+
+
+# rows of the groups, so that there are four rounds and 16 tiles, two and 96 (halves), five and 8 with empty groups and more of them than 64, one and 44
+VARLEN_LAST_ROUND = [([1800] * 14 + [2304, 2100], 2048, 1024), ([4096] * 4 + [1536, 1400], 2048, 2064), ([0, 1] * 33 + [16384, 16200, 0], 2048, 2048),
+                     ([5000, 500, 0, 257, 11], 3072, 4096)]
+
+
+@pytest.mark.parametrize("counts,n,k", VARLEN_LAST_ROUND)
+def test_varlen_last_round(counts, n, k):
+    import test_gpu_grouped_pingpong as cases
+    torch.manual_seed(n + k)
+    cases._varlen_products(counts, n, k)

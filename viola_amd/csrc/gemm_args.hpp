@@ -55,8 +55,8 @@ int launch_group_gemm_fast(const GemmArgs& p, int mode, int a_dtype, int b_dtype
 enum GroupForm { GROUP_BLOCKS = 0, GROUP_BLOCKS_SPLIT, GROUP_NARROW, GROUP_NARROW_SPLIT, GROUP_LARGE, GROUP_TALL, GROUP_TEAMS };
 GroupForm group_form(const GemmArgs& p, bool rowscale, dim3 grid);
 
-// The grouped recipe on tiles of 256 x 256 (row-wise b scales: 256 x 128); row_tiles: tiles of 256 rows (variable groups: a bound on
-// them), groups: k ranges. gemm_pingpong_grouped.hip.
+// The grouped recipe on tiles of 256 x 256, a last round of few on narrower ones (row-wise b scales: 256 x 128); row_tiles: tiles of 256 rows (variable groups: a bound on
+// them), groups: k ranges (row-wise b scales only). gemm_pingpong_grouped.hip.
 int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale, unsigned groups,
                           hipStream_t stream);
 

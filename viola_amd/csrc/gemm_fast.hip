@@ -55,7 +55,9 @@ constexpr int64_t SPLIT_MIN_K = 1536, NARROW_SPLIT_MIN_K = 1024;
 // (8192 x 4096 x 1024 75 -> 67 us, 16384 x 4096 x 256 55 -> 56) where they fill the chip (4096 x 4096 x 2048, 256 of them, 68 -> 61;
 // 6000 x 4096 x 1024, 384, 55 -> 60; row-wise 4096 x 3072 x 8192, 384, 245 -> 251). At 256 tiles of 128 x 128 and fewer the split
 // forms have more of the chip at work (8192 x 4096 x 1024 transposed, 88 -> 115 us). Groups of rows fill half of their last tile
-// on average; groups of k have each the average length.
+// on average; groups of k have each the average length. With uniform b scales a last round of up to 128 large tiles runs on halves or
+// quarters of them (gemm_pingpong_grouped_rounds), so that one round and a quarter pays too (4352 x 4096 x 4096, 272 tiles,
+// 154 -> 145; one and a half does not, 6000 x 4096 x 1024).
 static bool prefer_pingpong(const GemmArgs& p, bool rowscale, unsigned k_groups) {
     constexpr double CUS = 256.0;
     if (p.k < 256 || 256 * p.lda >= (1ll << 31)) return false;
@@ -69,7 +71,10 @@ static bool prefer_pingpong(const GemmArgs& p, bool rowscale, unsigned k_groups)
     const double pairs = floor(small / (2 * CUS)), left = small - pairs * 2 * CUS;
     const double now = pairs * (chunks * pair + 3.3) + (left > 0 ? chunks * pair * (left <= CUS ? 0.52 : 1.0) + 3.3 : 0.0);
     const double rounds = floor(large / CUS), rest = large / CUS - rounds;
-    return rounds * (chunks * busy + ends) + (rest > 0 ? chunks * (idle + (busy - idle) * rest) + ends : 0.0) < now;
+    double last = rest > 0 ? chunks * (idle + (busy - idle) * rest) + ends : 0.0;
+    if (!rowscale && rounds > 0 && rest > 0 && rest <= 0.25) last = chunks * (0.42 + 0.4 * rest) + 6.0;
+    else if (!rowscale && rounds > 1 && rest > 0 && rest <= 0.5) last = chunks * (0.45 + rest) + 5.0;
+    return rounds * (chunks * busy + ends) + last < now;
 }
 
 // Whether a product with uniform b scales that is too small for 256 x 256 tiles runs on tiles of 256 x 128, one round of them: where two

@@ -18,6 +18,21 @@ static int launch(const GemmArgs& args, int row_tiles, int a_dtype, int b_dtype,
     return viola_launch_status();
 }
 
+static int launch_rounds(const GemmArgs& args, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+    GemmArgs p = args;
+    p.tiles_m = row_tiles;
+    p.tiles_n = (int)((p.n + GroupedWide::COLS - 1) / GroupedWide::COLS);
+    // (variable groups: row_tiles is a bound; whatever the number of tiles turns out to be, their blocks are among these)
+    const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n + 256;
+    const dim3 grid((unsigned)((blocks + 7) / 8 * 8)), block(512);
+    const bool a5 = a_dtype == VIOLA_E5M2, b5 = b_dtype == VIOLA_E5M2;
+    if (!a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_grouped_rounds<false, false, GroupedWide, GroupedTall, GroupedQuarter>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else if (a5 && !b5) VIOLA_LAUNCH((gemm_pingpong_grouped_rounds<true, false, GroupedWide, GroupedTall, GroupedQuarter>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else if (!a5 && b5) VIOLA_LAUNCH((gemm_pingpong_grouped_rounds<false, true, GroupedWide, GroupedTall, GroupedQuarter>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    else VIOLA_LAUNCH((gemm_pingpong_grouped_rounds<true, true, GroupedWide, GroupedTall, GroupedQuarter>), grid, block, 0, stream, p, bias_dtype, out_dtype);
+    return viola_launch_status();
+}
+
 // out = sum of the parts, in ascending order. A thread owns eight consecutive values: 32 bytes of every part in flight at once.
 // Bound by the read of the partial products, which the kernel before has just written: most of them are still in the last-level
 // cache (3072 x 768 in three parts: 7.1 us for 33 MB).
@@ -70,7 +85,7 @@ int launch_group_parts(const GemmArgs& args, int parts, int a_dtype, int b_dtype
 int launch_group_pingpong(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, bool rowscale,
                           unsigned groups, hipStream_t stream) {
     return rowscale ? launch<GroupedRows, true>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, groups, stream)
-                    : launch<GroupedWide, false>(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, groups, stream);
+                    : launch_rounds(p, row_tiles, a_dtype, b_dtype, bias_dtype, out_dtype, stream);
 }
 
 int launch_group_tall(const GemmArgs& p, int row_tiles, int a_dtype, int b_dtype, int bias_dtype, int out_dtype, hipStream_t stream) {

@@ -31,6 +31,8 @@ using GroupedWide = PingPongShape<2, 4, 4, 2, 4>;                            // 
 using GroupedRows = PingPongShape<4, 2, 2, 2, 4>;                            // row-wise b scales: 64 x 64
 using GroupedTall = PingPongShape<4, 2, 2, 2, 3, 128>;                       // uniform b scales, half as wide: 64 x 64 per wave
 
+using GroupedQuarter = PingPongShape<4, 2, 2, 1, 3, 128>;                    // uniform b scales, 256 x 64: 64 x 32
+
 using GroupedTeams = PingPongShape<2, 2, 2, 2, 4>;                           // row-wise, 128 x 128, two teams that share the k range
 
 typedef float f32x32 __attribute__((ext_vector_type(32)));
@@ -48,20 +50,34 @@ __device__ __forceinline__ void group_row_tiles(const GemmArgs& p, int base, int
     }
 }
 
+// A scale block is 8 K groups in 16-byte pieces of 4: [half][row of a], then [half][row of b], or with uniform b scales
+// [half][sub-tile of b] (what 64 lanes of one load instruction bring); two buffers.
+// Chunks of 128 k (OWN) bring their 4 K groups themselves: a block of [row of a], then [sub-tile of b] per stage.
+template <typename S, bool ROWS>
+struct GroupedLds {
+    static constexpr bool OWN = S::CHUNK == 128;
+    static constexpr int B_ENTRIES = ROWS ? S::COLS : S::COLS / 32;
+    static constexpr int A_SCALES = (OWN ? 1 : 2) * S::ROWS * 16, B_SCALES = ROWS ? 2 * B_ENTRIES * 16 : 1024, SCALE_BLOCK = A_SCALES + B_SCALES;
+    static constexpr int RING = S::STAGES * S::STAGE, SCALE_BUFFERS = OWN ? S::STAGES : 2, TEAM = RING + SCALE_BUFFERS * SCALE_BLOCK;
+    static constexpr int BYTES = S::TEAMS * TEAM;
+};
+
+// Where a tile lies: its rows and first column, its k range, the b matrix of its group.
+struct GroupedPlace {
+    int64_t m_begin, m_end, n_begin, k_begin, k_end, out_shift;
+    const uint8_t* b;
+    const float* sb;
+};
+
 template <bool A_BF8, bool B_BF8, typename S, bool ROWS>
-__global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int bias_dtype, int out_dtype) {
+__device__ __forceinline__ void grouped_tile(const GemmArgs& p, const GroupedPlace& at, uint8_t* lds_all, int bias_dtype, int out_dtype) {
     constexpr int TM = S::TM, TN = S::TN, STAGES = S::STAGES, RING = STAGES * S::STAGE;
-    // A scale block is 8 K groups in 16-byte pieces of 4: [half][row of a], then [half][row of b], or with uniform b scales
-    // [half][sub-tile of b] (what 64 lanes of one load instruction bring)
-    // Chunks of 128 k (OWN) bring their 4 K groups themselves: a block of [row of a], then [sub-tile of b] per stage.
-    constexpr int KG = S::CHUNK / 32;
-    constexpr bool OWN = KG == 4;
-    constexpr int B_ENTRIES = ROWS ? S::COLS : S::COLS / 32;
-    constexpr int A_SCALES = (OWN ? 1 : 2) * S::ROWS * 16, B_SCALES = ROWS ? 2 * B_ENTRIES * 16 : 1024, SCALE_BLOCK = A_SCALES + B_SCALES;
-    constexpr int SCALE_BUFFERS = OWN ? STAGES : 2, TEAM_LDS = RING + SCALE_BUFFERS * SCALE_BLOCK;
+    using L = GroupedLds<S, ROWS>;
+    constexpr int KG = S::CHUNK / 32, B_ENTRIES = L::B_ENTRIES, A_SCALES = L::A_SCALES, B_SCALES = L::B_SCALES, SCALE_BLOCK = L::SCALE_BLOCK;
+    constexpr int SCALE_BUFFERS = L::SCALE_BUFFERS, TEAM_LDS = L::TEAM;
+    constexpr bool OWN = L::OWN;
     static_assert(2 * S::ROWS == S::THREADS && (ROWS || 2 * B_ENTRIES <= 64) && SCALE_BUFFERS * SCALE_BLOCK >= S::COLS * 4);
     static_assert(KG == 2 || (OWN && !ROWS && S::TEAMS == 1));
-    __shared__ __attribute__((aligned(1024))) uint8_t lds_all[S::TEAMS * TEAM_LDS];
     // tid, wave and lds are the team's own
     const int team = S::TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / S::THREADS) : 0;
     const int tid = threadIdx.x % S::THREADS, lane = tid % WAVE, l32 = lane % 32, lhi = lane / 32;
@@ -69,59 +85,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     uint8_t* const lds = lds_all + team * TEAM_LDS;
     const int wm = wave / S::WN, wn = wave % S::WN;
 
-    // ---- tile: contiguous ranges per XCD, walked in groups of 4 m tiles, so that the 32 tiles at work on an XCD are 4 x 8
-    // (8 x 4: 70 instead of 67 us at 8192 x 4096 x 1024). Variable groups: see group_gemm_fast.
-    constexpr int WALK = 4;
-    int tiles_m = p.tiles_m, group_tiles = 0, group_end = 0;
-    if (p.offsets) {
-        tiles_m = 0;
-        for (int base = 0; base < p.groups; base += WAVE) {
-            int count, end;
-            group_row_tiles<S::ROWS>(p, base, count, end);
-            if (base == 0) { group_tiles = count; group_end = end; }
-            tiles_m += __builtin_amdgcn_readlane(end, WAVE - 1);
-        }
-    }
-    const int per_xcd = p.offsets ? (int)(((int64_t)tiles_m * p.tiles_n + 7) / 8) : (int)(gridDim.x / 8);
-    const int seq = blockIdx.x / 8, place = (blockIdx.x % 8) * per_xcd + seq, tiles = tiles_m * p.tiles_n;
-    const int part = p.k_split ? place / tiles : 0, t = place - part * tiles;
-    if (seq >= per_xcd || (p.k_split ? part >= p.parts : t >= tiles)) return;
-    const int walk = WALK * p.tiles_n, first_m = t / walk * WALK;
-    const int rows_here = tiles_m - first_m < WALK ? tiles_m - first_m : WALK;
-    const int tile_m = first_m + t % walk % rows_here;
-    const int64_t n_begin = (int64_t)(t % walk / rows_here) * S::COLS;
-    int64_t m_begin = (int64_t)tile_m * S::ROWS, m_end = p.m, k_begin = 0, k_end = p.k;
-    const uint8_t* bptr = p.b;
-    const float* sbptr = p.sb;
-    int64_t out_shift = 0;
-    if (p.offsets) {
-        int tile = tile_m, g = 0;
-        for (int base = 0;; base += WAVE) {                                  // ends: tile_m is one of the tiles counted above
-            if (base) group_row_tiles<S::ROWS>(p, base, group_tiles, group_end);
-            const uint64_t past = __builtin_amdgcn_ballot_w64(tile < group_end);
-            if (past) {
-                const int at = __builtin_ctzll(past);
-                tile -= __builtin_amdgcn_readlane(group_end - group_tiles, at);
-                g = base + at;
-                break;
-            }
-            tile -= __builtin_amdgcn_readlane(group_end, WAVE - 1);
-        }
-        m_begin = p.offsets[g] + (int64_t)tile * S::ROWS;
-        m_end = p.offsets[g + 1];
-        bptr += (int64_t)g * p.b_group_stride;
-        sbptr += (int64_t)g * p.sb_group_stride;
-    }
-    if (p.koffsets) {
-        k_begin = p.koffsets[blockIdx.z];
-        k_end = p.koffsets[blockIdx.z + 1];
-        out_shift = (int64_t)blockIdx.z * p.out_group_stride;
-    }
-    if (p.k_split) {
-        k_begin = part * p.k_split;
-        k_end = k_begin + p.k_split < p.k ? k_begin + p.k_split : p.k;
-        out_shift = part * p.out_group_stride;
-    }
+    const int64_t m_begin = at.m_begin, m_end = at.m_end, n_begin = at.n_begin, out_shift = at.out_shift;
+    int64_t k_begin = at.k_begin, k_end = at.k_end;
+    const uint8_t* bptr = at.b;
+    const float* sbptr = at.sb;
     int split_chunks = 0;                                                    // of the longer (first) half of two teams
     if constexpr (S::TEAMS > 1) {
         constexpr int64_t CUT = F_SGROUPS * 32;                              // a scale block belongs to one team
@@ -472,6 +439,107 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int 
     if (out_dtype == VIOLA_F32) finish(float{});
     else if (out_dtype == VIOLA_BF16) finish(bf16_t{});
     else finish(f16_t{});
+}
+
+// Row tiles of all groups together; of the first 64 groups' those of each and up to it (see group_row_tiles).
+template <int ROWS>
+__device__ __forceinline__ int count_row_tiles(const GemmArgs& p, int& group_tiles, int& group_end) {
+    if (!p.offsets) return p.tiles_m;
+    int tiles_m = 0;
+    for (int base = 0; base < p.groups; base += WAVE) {
+        int count, end;
+        group_row_tiles<ROWS>(p, base, count, end);
+        if (base == 0) { group_tiles = count; group_end = end; }
+        tiles_m += __builtin_amdgcn_readlane(end, WAVE - 1);
+    }
+    return tiles_m;
+}
+
+// Tile t of tiles_m x p.tiles_n, walked in groups of 4 m tiles, so that the 32 tiles at work on an XCD are 4 x 8
+// (8 x 4: 70 instead of 67 us at 8192 x 4096 x 1024). Variable groups: see group_gemm_fast.
+template <typename S>
+__device__ __forceinline__ GroupedPlace grouped_place(const GemmArgs& p, int t, int tiles_m, int group_tiles, int group_end) {
+    constexpr int WALK = 4;
+    const int walk = WALK * p.tiles_n, first_m = t / walk * WALK;
+    const int rows_here = tiles_m - first_m < WALK ? tiles_m - first_m : WALK;
+    const int tile_m = first_m + t % walk % rows_here;
+    GroupedPlace at = {(int64_t)tile_m * S::ROWS, p.m, (int64_t)(t % walk / rows_here) * S::COLS, 0, p.k, 0, p.b, p.sb};
+    if (p.offsets) {
+        int tile = tile_m, g = 0;
+        for (int base = 0;; base += WAVE) {                                  // ends: tile_m is one of the tiles counted above
+            if (base) group_row_tiles<S::ROWS>(p, base, group_tiles, group_end);
+            const uint64_t past = __builtin_amdgcn_ballot_w64(tile < group_end);
+            if (past) {
+                const int lane = __builtin_ctzll(past);
+                tile -= __builtin_amdgcn_readlane(group_end - group_tiles, lane);
+                g = base + lane;
+                break;
+            }
+            tile -= __builtin_amdgcn_readlane(group_end, WAVE - 1);
+        }
+        at.m_begin = p.offsets[g] + (int64_t)tile * S::ROWS;
+        at.m_end = p.offsets[g + 1];
+        at.b += (int64_t)g * p.b_group_stride;
+        at.sb += (int64_t)g * p.sb_group_stride;
+    }
+    return at;
+}
+
+// Contiguous ranges of the tiles per XCD.
+template <bool A_BF8, bool B_BF8, typename S, bool ROWS>
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped(GemmArgs p, int bias_dtype, int out_dtype) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[GroupedLds<S, ROWS>::BYTES];
+    int group_tiles = 0, group_end = 0;
+    const int tiles_m = count_row_tiles<S::ROWS>(p, group_tiles, group_end), tiles = tiles_m * p.tiles_n;
+    const int per_xcd = p.offsets ? (int)(((int64_t)tiles + 7) / 8) : (int)(gridDim.x / 8);
+    const int seq = blockIdx.x / 8, place = (blockIdx.x % 8) * per_xcd + seq;
+    const int part = p.k_split ? place / tiles : 0, t = place - part * tiles;
+    if (seq >= per_xcd || (p.k_split ? part >= p.parts : t >= tiles)) return;
+    GroupedPlace at = grouped_place<S>(p, t, tiles_m, group_tiles, group_end);
+    if (p.koffsets) {
+        at.k_begin = p.koffsets[blockIdx.z];
+        at.k_end = p.koffsets[blockIdx.z + 1];
+        at.out_shift = (int64_t)blockIdx.z * p.out_group_stride;
+    }
+    if (p.k_split) {
+        at.k_begin = part * p.k_split;
+        at.k_end = at.k_begin + p.k_split < p.k ? at.k_begin + p.k_split : p.k;
+        at.out_shift = part * p.out_group_stride;
+    }
+    grouped_tile<A_BF8, B_BF8, S, ROWS>(p, at, lds, bias_dtype, out_dtype);
+}
+
+// Uniform b scales: rounds of S tiles, a CU each. A last round of few, which would take as long as a full one and leave CUs without a tile, runs
+// on tiles of the same rows and fewer columns: up to 128 tiles as two of HALF each, up to 64 as four of QUARTER. Here and not on the host,
+// because how many tiles variable groups make shows here only. Before, on blocks of 128 x 128 or tiles of 256 x 256 alone, and now (us):
+// 8192 x 4608 x 4096 (two rounds and 64) 286, 312 -> 264; 4352 x 4096 x 4096 (one and 16) 154, 200 -> 145; 16384 x 8704 x 1024 (eight and 128)
+// 326, 295 -> 275; 4096 x 10240 x 2048 (two and 128) 166, 169 -> 151; 4096 x 9216 x 1152 (two and 64) 95, 105 -> 87.5.
+template <bool A_BF8, bool B_BF8, typename S, typename HALF, typename QUARTER>
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_grouped_rounds(GemmArgs p, int bias_dtype, int out_dtype) {
+    constexpr int ROUND = 256;
+    static_assert(S::ROWS == HALF::ROWS && S::ROWS == QUARTER::ROWS && S::COLS == 2 * HALF::COLS && S::COLS == 4 * QUARTER::COLS);
+    constexpr int LDS_S = GroupedLds<S, false>::BYTES, LDS_H = GroupedLds<HALF, false>::BYTES;
+    static_assert(GroupedLds<QUARTER, false>::BYTES <= LDS_H);
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_S > LDS_H ? LDS_S : LDS_H];
+    int group_tiles = 0, group_end = 0;
+    const int tiles_m = count_row_tiles<S::ROWS>(p, group_tiles, group_end), tiles = tiles_m * p.tiles_n;
+    const int rest = tiles % ROUND, each = tiles < ROUND || rest * 2 > ROUND ? 1 : rest * 4 > ROUND ? 2 : 4;
+    const int whole = each > 1 ? tiles - rest : (tiles + 7) / 8 * 8;
+    const int block = blockIdx.x;
+    if (block < whole) {                                                     // contiguous ranges per XCD
+        const int t = block % 8 * (whole / 8) + block / 8;
+        if (t >= tiles) return;
+        grouped_tile<A_BF8, B_BF8, S, false>(p, grouped_place<S>(p, t, tiles_m, group_tiles, group_end), lds, bias_dtype, out_dtype);
+        return;
+    }
+    if (each == 1) return;
+    const int per_xcd = (rest * each + 7) / 8, seq = (block - whole) / 8, u = (block - whole) % 8 * per_xcd + seq, t = whole + u / each;
+    if (seq >= per_xcd || t >= tiles) return;
+    GroupedPlace at = grouped_place<S>(p, t, tiles_m, group_tiles, group_end);
+    at.n_begin += u % each * (S::COLS / each);
+    if (at.n_begin >= p.n) return;
+    if (each == 2) grouped_tile<A_BF8, B_BF8, HALF, false>(p, at, lds, bias_dtype, out_dtype);
+    else grouped_tile<A_BF8, B_BF8, QUARTER, false>(p, at, lds, bias_dtype, out_dtype);
 }
 
 }  // namespace viola
