@@ -352,6 +352,12 @@ int viola_momentum_update_table(const int64_t* table, int64_t tensors, int64_t t
                                 float beta, float inv_loss_scale, int nesterov, int rounding, int64_t rounding_step,
                                 viola_stream_t stream);
 
+/* viola_momentum_update_table that also leaves the sums of squares of the updates, read in working_dtype (bf16 or f16), in
+ * sums[tensor][256]: the first stage of viola_ns_prepare for one matrix per tensor (its partial sums in another order). */
+int viola_momentum_update_squares(const int64_t* table, int64_t tensors, int64_t tiles, int grad_dtype, int tile_size,
+                                  float beta, float inv_loss_scale, int nesterov, int rounding, int64_t rounding_step,
+                                  int working_dtype, float* sums, viola_stream_t stream);
+
 /* viola_weight_update with nearest rounding for many fp32 tensors of `count` elements each (a multiple of 4), one
  * launch (the reference: one launch per matrix, viola/optim/muon.py:131-132). table: rows of two int64:
  * {weight (16-byte aligned), update (aligned to four elements of grad_dtype)}. */
@@ -430,14 +436,14 @@ int viola_ns_prepare(const void* in, int in_dtype, void* out, int dtype, int64_t
                      float* workspace, viola_stream_t stream);
 
 /* viola_ns_prepare of bf16 matrices of up to eight shapes, in one launch for each of its two stages. The workspace holds 256 floats
- * per matrix of all of them. VIOLA_EUNSUPPORTED, with nothing launched: more than eight shapes or 65535 matrices, columns that are
+ * per matrix of all of them; with have_sums they are there already (viola_momentum_update_squares) and the second stage alone runs. VIOLA_EUNSUPPORTED, with nothing launched: more than eight shapes or 65535 matrices, columns that are
  * no multiple of 8, or operands off 16 bytes. */
 typedef struct {
     const void* in;
     void* out;
     int64_t batch, rows, cols;
 } viola_ns_matrices;
-int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count, int dtype, float* workspace, viola_stream_t stream);
+int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count, int dtype, float* workspace, int have_sums, viola_stream_t stream);
 
 /* No counterpart in the reference. viola_ns_prepare for callers that cannot allocate device memory (code under
  * HIP-graph capture, serving loops, harnesses that forbid hipMalloc): the same kernels and results, with the

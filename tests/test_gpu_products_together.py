@@ -64,11 +64,37 @@ def test_scaled_matrices_of_several_shapes_equal_one_shape_each(dtype):
     outs, rows = [torch.zeros(b, min(r, c), max(r, c), device="cuda", dtype=dtype) for b, r, c in shapes], (Matrices * len(shapes))()
     for i, ((b, r, c), x, out) in enumerate(zip(shapes, ins, outs)):
         rows[i] = Matrices(x.data_ptr(), out.data_ptr(), b, r, c)
-    _lib.call("viola_ns_prepare_many", ctypes.addressof(rows), len(shapes), _lib.code(dtype), _lib.ptr(sums))
+    _lib.call("viola_ns_prepare_many", ctypes.addressof(rows), len(shapes), _lib.code(dtype), _lib.ptr(sums), 0)
     for (b, r, c), x, out in zip(shapes, ins, outs):
         want = torch.empty_like(out)
         _lib.call("viola_ns_prepare", _lib.ptr(x), _lib.code(torch.bfloat16), _lib.ptr(want), _lib.code(dtype), b, r, c, _lib.ptr(sums))
         assert torch.equal(out.view(torch.int16), want.view(torch.int16)), (b, r, c)
+
+
+@pytest.mark.parametrize("working", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("grads,tile,rounding", [(torch.float32, 256, 0), (torch.bfloat16, 512, 1), (torch.float16, 1024, 0), (torch.float32, 1024, 1)])
+def test_momentum_with_sums_of_squares(grads, tile, rounding, working):
+    """State and updates are those of viola_momentum_update, one tensor at a time; the sums, whose order is not specified, those of the
+    updates in float64: at most 2^-24 for each of the some 40 additions on the way of a term."""
+    torch.manual_seed(tile)
+    tiles = [1, 5, 16, 300, 4099]
+    table, want, got, held = [], [], [], []
+    for i, n in enumerate(tiles):
+        g = (torch.randn(n * tile, device="cuda") * 1e-2).to(grads)
+        q, s = torch.randint(0, 120, (n * tile,), device="cuda", dtype=torch.uint8), torch.rand(n, device="cuda") * 1e-3
+        sides = [(q.clone(), s.clone(), torch.zeros(n * tile, device="cuda", dtype=torch.bfloat16)) for _ in range(2)]
+        (wq, ws, wu), (gq, gs, gu) = sides
+        _lib.call("viola_momentum_update", _lib.ptr(g), _lib.code(grads), _lib.ptr(wq), _lib.ptr(ws), _lib.ptr(wq), _lib.ptr(ws), _lib.ptr(wu), n * tile, .95, 1.0, 1, 0, tile,
+                  1, 1, 1, 1, 1, rounding, 3, 77 + i)
+        table.append([g.data_ptr(), gq.data_ptr(), gs.data_ptr(), gq.data_ptr(), gs.data_ptr(), gu.data_ptr(), 77 + i, n])
+        want.append((wq, ws, wu)); got.append((gq, gs, gu)); held.append(g)
+    rows, sums = torch.tensor(table, device="cuda"), torch.full((len(tiles), 256), float("nan"), device="cuda")
+    _lib.call("viola_momentum_update_squares", rows.data_ptr(), len(tiles), max(tiles), _lib.code(grads), tile, .95, 1.0, 1, rounding, 3, _lib.code(working), sums.data_ptr())
+    for a, b, row in zip(want, got, sums):
+        for x, y in zip(a, b):
+            assert torch.equal(x, y)
+        exact = a[2].to(working).double().square().sum().item()
+        assert abs(row.double().sum().item() - exact) <= 40 * 2.0 ** -24 * exact
 
 
 def test_calls_that_one_launch_does_not_take_are_refused_before_it():
@@ -80,7 +106,7 @@ def test_calls_that_one_launch_does_not_take_are_refused_before_it():
     for rows in ([good, odd], [good] * 9):
         assert _lib.call("viola_ns_gemm_many", ctypes.addressof((Product * len(rows))(*rows)), len(rows), _lib.code(torch.bfloat16), unsupported_ok=True) == -2
     for rows in ([Matrices(x.data_ptr(), out.data_ptr(), 1, 16, 15)], [Matrices(x.data_ptr() + 2, out.data_ptr(), 1, 8, 8)], [Matrices(x.data_ptr(), out.data_ptr(), 1, 16, 16)] * 9):
-        assert _lib.call("viola_ns_prepare_many", ctypes.addressof((Matrices * len(rows))(*rows)), len(rows), _lib.code(torch.bfloat16), _lib.ptr(sums), unsupported_ok=True) == -2
+        assert _lib.call("viola_ns_prepare_many", ctypes.addressof((Matrices * len(rows))(*rows)), len(rows), _lib.code(torch.bfloat16), _lib.ptr(sums), 0, unsupported_ok=True) == -2
     torch.cuda.synchronize()
     assert out.eq(7.0).all()
 

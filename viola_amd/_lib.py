@@ -64,6 +64,7 @@ _SIGNATURES = {
     "viola_mx_gated_gemm": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _i, _i, _p, _i, _p, _p, _i, _i, _i, _p],
     "viola_mx_gated_gemm_encode": [_p, _i, _p, _i, _p, _p, _l, _l, _l, _i, _i, _p, _i, _p, _i, _p, _p, _p, _p, _i, _f, _i, _p],
     "viola_momentum_update_table": [_p, _l, _l, _i, _i, _f, _f, _i, _i, _l, _p],
+    "viola_momentum_update_squares": [_p, _l, _l, _i, _i, _f, _f, _i, _i, _l, _i, _p, _p],
     "viola_weight_update_table": [_p, _l, _l, _i, _f, _f, _f, _p],
     "viola_weight_update_rows": [_p, _l, _l, _i, _f, _f, _p],
     "viola_adam_update_table": [_p, _l, _l, _i, _i, _i, _f, _f, _f, _f, _f, _f, _f, _i, _l, _i, _i, _p],
@@ -71,7 +72,7 @@ _SIGNATURES = {
     "viola_momentum_dequantize": [_p, _p, _p, _l, _i, _i, _l, _l, _l, _i, _i, _p],
     "viola_ns_gemm": [_p, _p, _p, _p, _i, _i, _i, _l, _l, _l, _l, _f, _p, _i, _p],
     "viola_ns_gemm_many": [_p, _i, _i, _p],
-    "viola_ns_prepare_many": [_p, _i, _i, _p, _p],
+    "viola_ns_prepare_many": [_p, _i, _i, _p, _i, _p],
     "viola_ns_prepare": [_p, _i, _p, _i, _l, _l, _l, _p, _p],
     "viola_ns_prepare_static": [_p, _i, _p, _i, _l, _l, _l, _p],
     "viola_comm_roundtrip": [_p, _l, _p, _l, _i, _i, _p],

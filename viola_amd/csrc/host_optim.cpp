@@ -125,19 +125,17 @@ Tensor newton_schulz(const Tensor& matrix, int64_t steps, bool gram) {
     return c.result;
 }
 
-// Chains of one type, step by step together: the products of a step are one launch where the tiled kernel takes them all.
-void run_together(const std::vector<Chain>& chains, viola_stream_t stream) {
+// Chains of one type, step by step together: the products of a step are one launch where the tiled kernel takes them all. `sums` holds the
+// matrices' sums of squares already, or (have_sums 0) has room for them.
+void run_together(const std::vector<Chain>& chains, const Arena& sums, int have_sums, viola_stream_t stream) {
     const int dtype = chains[0].dtype;
     std::vector<viola_ns_matrices> starts;
-    int64_t matrices = 0;
     size_t steps = 0;
     for (const Chain& c : chains) {
         starts.push_back(c.start);
-        matrices += c.start.batch;
         steps = std::max(steps, c.products.size());
     }
-    const Arena sums = sums_of(matrices, chains[0].matrix.device());
-    int status = VIOLA_TRY(viola_ns_prepare_many, starts.data(), (int)starts.size(), dtype, sums.as<float>(0), stream);
+    int status = VIOLA_TRY(viola_ns_prepare_many, starts.data(), (int)starts.size(), dtype, sums.as<float>(0), have_sums, stream);
     if (status == VIOLA_EUNSUPPORTED) {
         for (const Chain& c : chains) prepare(c, sums.as<float>(0), stream);      // (one after the other: each may overwrite the sums)
     } else check("viola_ns_prepare_many", status);
@@ -190,7 +188,7 @@ struct MomentumRow {
     int64_t key, count;
 };
 bool momentum_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<MomentumRow>& rows, int64_t tile,
-                       float beta, float inv_loss_scale, bool nesterov, int rounding, int64_t step, viola_stream_t stream) {
+                       float beta, float inv_loss_scale, bool nesterov, int rounding, int64_t step, viola_stream_t stream, float* sums = nullptr, int working = VIOLA_BF16) {
     if (rows.empty() || rows.size() > 65535 || tile < 256) return false;
     const at::ScalarType kind = rows[0].grad.scalar_type();
     std::vector<int64_t> words;
@@ -206,7 +204,8 @@ bool momentum_together(Tables& tables, const std::vector<int64_t>& shape, int64_
         words.insert(words.end(), row, row + 8);
     }
     const int64_t* t = tables.get(MOMENTUM_TABLE, shape, (int64_t)rows.size(), ordinal, std::move(words), rows[0].q.device(), stream);
-    VIOLA_CALL(viola_momentum_update_table, t, (int64_t)rows.size(), tiles, code_of(kind), (int)tile, beta, inv_loss_scale, nesterov, rounding, step, stream);
+    if (sums) VIOLA_CALL(viola_momentum_update_squares, t, (int64_t)rows.size(), tiles, code_of(kind), (int)tile, beta, inv_loss_scale, nesterov, rounding, step, working, sums, stream);
+    else VIOLA_CALL(viola_momentum_update_table, t, (int64_t)rows.size(), tiles, code_of(kind), (int)tile, beta, inv_loss_scale, nesterov, rounding, step, stream);
     return true;
 }
 
@@ -507,8 +506,8 @@ private:
         join.now();
     }
 
-    // The chains of all buckets step by step together, a product of each in one launch, and one launch each for the momentum, the two
-    // stages in front of the chains and the weights: 20 launches where buckets on lanes of their own take about 80 and the events that
+    // The chains of all buckets step by step together, a product of each in one launch, and one launch each for the momentum with the sums
+    // of squares, the scaling in front of the chains and the weights: 20 launches where buckets on lanes of their own take about 80 and the events that
     // join them, which is all that a step of small matrices costs (one block of width 192: 253 -> 102 us, four of 256 316 -> 146, eight of
     // 384 362 -> 349). Large sets gain by the mix of tile lengths (28 blocks of width 1152 12560 -> 12280 us, eight of 1280 5842 ->
     // 5185). The recurrence on the Gram matrix gains less there: its launches are several rounds of short tiles with a tail each, which lanes
@@ -516,7 +515,7 @@ private:
     static constexpr double TOGETHER_GRAM = 1e10;                // sum of m m (m + n) over the matrices
     static constexpr int64_t TOGETHER_ELEMENTS = 1ll << 29;      // all arenas are held at once: 12 GB
     bool step_together(std::vector<std::vector<Item>>& ready) {
-        if (ready.size() < 2 || ready.size() > 8) return false;
+        if (ready.empty() || ready.size() > 8) return false;
         const Item& head = ready[0][0];
         const Group& g = *head.group;
         const viola_stream_t stream = stream_of(head.param);
@@ -549,10 +548,17 @@ private:
                 out += 2 * count;
             }
         }
-        if (!momentum_together(tables_, {}, (int64_t)g.gram, momentum_rows, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step, stream)) return false;
+        // a parameter that is one matrix (not a batch of them): its sum of squares comes with its momentum
+        int64_t matrices = 0;
+        for (const Tensor& input : inputs) matrices += input.size(0) * input.size(1);
+        const bool single = matrices == (int64_t)momentum_rows.size();
+        const Arena sums = sums_of(matrices, head.param.device());
+        if (!momentum_together(tables_, {}, (int64_t)g.gram, momentum_rows, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step, stream,
+                               single ? sums.as<float>(0) : nullptr, g.gram ? VIOLA_F16 : VIOLA_BF16))
+            return false;
         std::vector<Chain> chains;
         for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram));
-        run_together(chains, stream);
+        run_together(chains, sums, single, stream);
         for (size_t i = 0; i < ready.size(); ++i) {
             const int64_t count = ready[i][0].param.numel(), rows = chains[i].matrix.size(-2), cols = chains[i].matrix.size(-1);
             const char* from = static_cast<const char*>(chains[i].result.const_data_ptr());

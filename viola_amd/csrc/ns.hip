@@ -682,7 +682,7 @@ extern "C" int viola_ns_gemm_many(const viola_ns_product* products, int count, i
     return viola_launch_status();
 }
 
-extern "C" int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count, int dtype, float* workspace, viola_stream_t stream_) {
+extern "C" int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count, int dtype, float* workspace, int have_sums, viola_stream_t stream_) {
     hipStream_t stream = viola_enter(stream_);
     VIOLA_CHECK_ARG((dtype == VIOLA_BF16 || dtype == VIOLA_F16) && count >= 0 && (count == 0 || (shapes && workspace)));
     if (count > NS_MANY) return VIOLA_EUNSUPPORTED;
@@ -701,10 +701,10 @@ extern "C" int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count,
     }
     if (many.count == 0) return 0;
     if (dtype == VIOLA_BF16) {
-        VIOLA_LAUNCH(ns_sumsq16_many<true>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
+        if (!have_sums) VIOLA_LAUNCH(ns_sumsq16_many<true>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
         VIOLA_LAUNCH(ns_scale16_many<true>, dim3((unsigned)blocks), dim3(256), 0, stream, many, workspace);
     } else {
-        VIOLA_LAUNCH(ns_sumsq16_many<false>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
+        if (!have_sums) VIOLA_LAUNCH(ns_sumsq16_many<false>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
         VIOLA_LAUNCH(ns_scale16_many<false>, dim3((unsigned)blocks), dim3(256), 0, stream, many, workspace);
     }
     return viola_launch_status();
