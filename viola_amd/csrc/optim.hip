@@ -202,9 +202,10 @@ __global__ __launch_bounds__(256) void momentum_table_quads(const int64_t* __res
                                              inv_loss_scale, nesterov, step, (uint64_t)row[6]);
 }
 
-// The same with what Newton-Schulz starts from, the sums of squares of the updates: 256 blocks per tensor, each with every 256th sixteen tiles of
-// it, leave their sums in sums[tensor][block], which is what a pass over the updates would write (viola_ns_prepare), so that this pass, 2
+// The same with what Newton-Schulz starts from, the sums of squares of the updates: up to 256 blocks per tensor, each with a share of its tiles
+// sixteen at a time, leave their sums in sums[tensor][block] (zeros in the rest of the 256), which is what a pass over the updates would write (viola_ns_prepare), so that this pass, 2
 // bytes per element, is not needed: 28 blocks of width 1152 625 + 181 -> 688 us (with blocks of 256 threads 738), one of 1024 x 1024 5.3 + 3.3 -> 5.7.
+constexpr int SQUARES_PARTS = 256;
 template <typename TG, int EPL, bool STOCHASTIC, int SQUARES>
 __global__ __launch_bounds__(1024) void momentum_squares_quads(const int64_t* __restrict__ table, int64_t blocks, float beta,
                                                                float inv_loss_scale, int nesterov, uint64_t step, float* __restrict__ sums) {
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(1024) void momentum_squares_quads(const int64_t* __
     if (threadIdx.x == 0) {
         sum = 0.0f;
         for (int w = 0; w < WAVES; ++w) sum += partial[w];
-        sums[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = sum;
+        for (unsigned slot = blockIdx.x; slot < SQUARES_PARTS; slot += gridDim.x) sums[(int64_t)blockIdx.y * SQUARES_PARTS + slot] = slot == blockIdx.x ? sum : 0.0f;
     }
 }
 
@@ -519,7 +520,8 @@ extern "C" int viola_momentum_update_squares(const int64_t* table, int64_t tenso
     VIOLA_CHECK_ARG(working_dtype == VIOLA_BF16 || working_dtype == VIOLA_F16);
     if (tensors == 0) return 0;
     VIOLA_CHECK_ARG(table && sums);
-    const dim3 grid(256, (unsigned)tensors);                                 // the parts that viola_ns_prepare's second stage adds
+    const int64_t blocks = (tiles + 15) / 16;                                // SQUARES_PARTS: what viola_ns_prepare's second stage adds
+    const dim3 grid((unsigned)(blocks < 1 ? 1 : blocks > SQUARES_PARTS ? SQUARES_PARTS : blocks), (unsigned)tensors);
     auto launch = [&](auto type, auto quads, auto stochastic, auto squares) {
         VIOLA_LAUNCH((momentum_squares_quads<decltype(type), decltype(quads)::value, decltype(stochastic)::value, decltype(squares)::value>), grid, dim3(1024), 0, stream,
                      table, tiles, beta, inv_loss_scale, nesterov, (uint64_t)rounding_step, sums);
