@@ -407,13 +407,18 @@ int viola_ns_gemm(const void* a, const void* bmat, const void* residual, void* o
 
 /* Up to eight products of viola_ns_gemm that do not depend on each other (the same step of the chains of several shapes), in one
  * launch; the arguments and results of each are viola_ns_gemm's. VIOLA_EUNSUPPORTED, with nothing launched: more than eight, or one
- * that viola_ns_plan gives the generic kernel; each then takes a call of its own. */
+ * that viola_ns_plan gives the generic kernel; each then takes a call of its own.
+ * weights, if not null: a device array of `batch` addresses of FP32 matrices, 16-byte aligned and laid out as the result would be, which
+ * become weight * keep - rate * result (viola_weight_update); out is not written. With epilogue 0 or 2, transpose_b 0, no out_diag, and m and n
+ * multiples of 8 (VIOLA_EUNSUPPORTED else). */
 typedef struct {
     const void *a, *b, *residual;
     void *out, *out_diag;
     int64_t batch, m, n, k;
     float add_diag;
     int transpose_b, epilogue, transpose_out;
+    const int64_t* weights;
+    float keep, rate;
 } viola_ns_product;
 int viola_ns_gemm_many(const viola_ns_product* products, int count, int dtype, viola_stream_t stream);
 

@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 class Product(ctypes.Structure):
     _fields_ = [(name, ctypes.c_void_p) for name in ("a", "b", "residual", "out", "out_diag")] + [(name, ctypes.c_int64) for name in ("batch", "m", "n", "k")] + \
-               [("add_diag", ctypes.c_float)] + [(name, ctypes.c_int) for name in ("transpose_b", "epilogue", "transpose_out")]
+               [("add_diag", ctypes.c_float)] + [(name, ctypes.c_int) for name in ("transpose_b", "epilogue", "transpose_out")] + \
+               [("weights", ctypes.c_void_p), ("keep", ctypes.c_float), ("rate", ctypes.c_float)]
 
 
 class Matrices(ctypes.Structure):
@@ -50,6 +51,44 @@ def test_products_in_one_launch_equal_one_launch_each(case, dtype):
     _lib.call("viola_ns_gemm_many", ctypes.addressof(rows), len(case), _lib.code(dtype))
     for i, (got, want) in enumerate(zip(outs, wants)):
         assert torch.isfinite(want).all() and torch.equal(got, want), i
+
+
+# (batch, m, n, k, epilogue, transposed weight): edges and remainders of each tile, with a product that is stored in the same launch
+INTO_WEIGHTS = [[(1, 8, 8, 8, 0, 0), (2, 64, 136, 72, 2, 0), (1, 72, 136, 64, 2, 1), (3, 40, 200, 40, 0, 1)], [(20, 256, 384, 256, 2, 1), (24, 264, 136, 40, 0, 0)],
+                [(40, 192, 576, 192, 2, 1), (40, 384, 384, 72, 2, 0), (24, 192, 200, 72, 0, 1)], [(100, 384, 1152, 384, 2, 1), (128, 384, 384, 72, 0, 0), (100, 768, 200, 40, 2, 0)]]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", INTO_WEIGHTS)
+def test_products_into_weights_equal_product_and_update(case, dtype):
+    torch.manual_seed(len(case))
+    lr, decay, scale = .02, .1, 1.7
+    f32 = lambda v: torch.tensor(v, dtype=torch.float32)
+    keep, rate = (1.0 - f32(lr) * f32(decay)).item(), (f32(lr) * f32(scale)).item()
+    rows, pairs, held = (Product * len(case))(), [], []
+    for i, (batch, m, n, k, epilogue, transposed) in enumerate(case):
+        a, b = (torch.randn(batch, m, k, device="cuda") / k ** .5).to(dtype), torch.randn(batch, k, n, device="cuda").to(dtype)
+        residual = torch.randn(batch, m, n, device="cuda").to(dtype) if epilogue else None
+        shape = (n, m) if transposed else (m, n)
+        weights = [torch.randn(*shape, device="cuda") for _ in range(batch)]
+        update = torch.empty(batch, *shape, device="cuda", dtype=dtype)
+        _lib.call("viola_ns_gemm", _lib.ptr(a), _lib.ptr(b), _lib.ptr(residual), _lib.ptr(update), _lib.code(dtype), 0, epilogue, batch, m, n, k, 0.0, None, transposed)
+        for w, u in zip(weights, update):
+            want = w.clone()
+            _lib.call("viola_weight_update", _lib.ptr(want), 0, _lib.ptr(u), _lib.code(dtype), w.numel(), lr, decay, scale, 0, 0, 0, 0)
+            pairs.append((w, want))
+        addresses = torch.tensor([w.data_ptr() for w in weights], device="cuda")
+        rows[i] = Product(_lib.ptr(a), _lib.ptr(b), _lib.ptr(residual), None, None, batch, m, n, k, 0.0, 0, epilogue, transposed, addresses.data_ptr(), keep, rate)
+        held += [a, b, residual, addresses]
+    stored = torch.full((1, 384, 192), float("nan"), device="cuda", dtype=dtype)
+    x, y = torch.randn(1, 384, 64, device="cuda").to(dtype), torch.randn(1, 64, 192, device="cuda").to(dtype)
+    more = (Product * (len(case) + 1))(*rows, Product(_lib.ptr(x), _lib.ptr(y), None, _lib.ptr(stored), None, 1, 384, 192, 64, 0.0, 0, 0, 0, None, 0, 0))
+    _lib.call("viola_ns_gemm_many", ctypes.addressof(more), len(case) + 1, _lib.code(dtype))
+    for got, want in pairs:
+        assert torch.equal(got, want)
+    want = torch.empty_like(stored)
+    _lib.call("viola_ns_gemm", _lib.ptr(x), _lib.ptr(y), None, _lib.ptr(want), _lib.code(dtype), 0, 0, 1, 384, 192, 64, 0.0, None, 0)
+    assert torch.equal(stored, want)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -103,7 +142,10 @@ def test_calls_that_one_launch_does_not_take_are_refused_before_it():
     sums = torch.zeros(256 * 16, device="cuda")
     good = Product(x.data_ptr(), x.data_ptr(), None, out.data_ptr(), None, 1, 16, 16, 16, 0.0, 1, 0, 0)
     odd = Product(x.data_ptr(), x.data_ptr(), None, out.data_ptr(), None, 1, 15, 15, 15, 0.0, 1, 0, 0)          # rows that are no 16-byte pieces
-    for rows in ([good, odd], [good] * 9):
+    address = torch.tensor([out.data_ptr()], device="cuda")
+    into = lambda *kinds, m=16: Product(x.data_ptr(), x.data_ptr(), x.data_ptr(), None, kinds[3], 1, m, 16, 16, 0.0, *kinds[:3], address.data_ptr(), 1.0, 1.0)
+    refused = [into(1, 0, 0, None), into(0, 1, 0, None), into(0, 2, 0, out.data_ptr()), into(0, 2, 1, None, m=12)]
+    for rows in ([good, odd], [good] * 9, *([p] for p in refused)):
         assert _lib.call("viola_ns_gemm_many", ctypes.addressof((Product * len(rows))(*rows)), len(rows), _lib.code(torch.bfloat16), unsupported_ok=True) == -2
     for rows in ([Matrices(x.data_ptr(), out.data_ptr(), 1, 16, 15)], [Matrices(x.data_ptr() + 2, out.data_ptr(), 1, 8, 8)], [Matrices(x.data_ptr(), out.data_ptr(), 1, 16, 16)] * 9):
         assert _lib.call("viola_ns_prepare_many", ctypes.addressof((Matrices * len(rows))(*rows)), len(rows), _lib.code(torch.bfloat16), _lib.ptr(sums), 0, unsupported_ok=True) == -2

@@ -30,6 +30,7 @@ struct Chain {
     int dtype = 0;
     viola_ns_matrices start{};                                   // the scaled matrix, in front of the products
     std::vector<viola_ns_product> products;
+    bool applied = false;                                        // the last product went into the weights
 };
 
 Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram) {
@@ -56,7 +57,7 @@ Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram) {
     if (steps == 0) return c;
     auto gemm = [&](const void* a, const void* b, bool transpose_b, const void* residual, int epilogue, int64_t out_cols, int64_t k, void* out,
                     float add_diag, void* out_diag, bool transpose_out) {
-        c.products.push_back({a, b, residual, out, out_diag, batch, m, out_cols, k, add_diag, transpose_b, epilogue, transpose_out});
+        c.products.push_back({a, b, residual, out, out_diag, batch, m, out_cols, k, add_diag, transpose_b, epilogue, transpose_out, nullptr, 0, 0});
     };
     if (quintic) {
         void *r = c.arena.at(s_at[0]), *z = c.arena.at(s_at[1]);
@@ -127,7 +128,7 @@ Tensor newton_schulz(const Tensor& matrix, int64_t steps, bool gram) {
 
 // Chains of one type, step by step together: the products of a step are one launch where the tiled kernel takes them all. `sums` holds the
 // matrices' sums of squares already, or (have_sums 0) has room for them.
-void run_together(const std::vector<Chain>& chains, const Arena& sums, int have_sums, viola_stream_t stream) {
+void run_together(std::vector<Chain>& chains, const Arena& sums, int have_sums, viola_stream_t stream) {
     const int dtype = chains[0].dtype;
     std::vector<viola_ns_matrices> starts;
     size_t steps = 0;
@@ -142,12 +143,19 @@ void run_together(const std::vector<Chain>& chains, const Arena& sums, int have_
     std::vector<viola_ns_product> step;
     for (size_t i = 0; i < steps; ++i) {
         step.clear();
+        bool into_weights = false;
         for (const Chain& c : chains)
-            if (i < c.products.size()) step.push_back(c.products[i]);
-        status = step.size() > 1 ? VIOLA_TRY(viola_ns_gemm_many, step.data(), (int)step.size(), dtype, stream) : VIOLA_EUNSUPPORTED;
+            if (i < c.products.size()) {
+                step.push_back(c.products[i]);
+                into_weights = into_weights || step.back().weights;
+            }
+        status = step.size() > 1 || into_weights ? VIOLA_TRY(viola_ns_gemm_many, step.data(), (int)step.size(), dtype, stream) : VIOLA_EUNSUPPORTED;
         if (status == VIOLA_EUNSUPPORTED) {
-            for (const viola_ns_product& p : step) multiply(p, dtype, stream);
-        } else check("viola_ns_gemm_many", status);
+            for (const viola_ns_product& p : step) multiply(p, dtype, stream);        // (results: the weights are the caller's then)
+            continue;
+        }
+        check("viola_ns_gemm_many", status);
+        for (Chain& c : chains) c.applied = c.applied || (i + 1 == c.products.size() && c.products[i].weights);
     }
 }
 
@@ -178,7 +186,7 @@ private:
     };
     std::map<std::tuple<viola_stream_t, int, std::vector<int64_t>, int64_t, int64_t>, Table> tables_;
 };
-enum { MOMENTUM_TABLE = 0, WEIGHT_TABLE = 1, ADAM_TABLE = 2 };
+enum { MOMENTUM_TABLE = 0, WEIGHT_TABLE = 1, ADAM_TABLE = 2, ADDRESS_TABLE = 3 };
 
 // One launch for a list of tensors over a table of their pointers. False, with nothing done: they do not fit the table kernel, and
 // each takes a launch of its own.
@@ -507,9 +515,9 @@ private:
     }
 
     // The chains of all buckets step by step together, a product of each in one launch, and one launch each for the momentum with the sums
-    // of squares, the scaling in front of the chains and the weights: 20 launches where buckets on lanes of their own take about 80 and the events that
-    // join them, which is all that a step of small matrices costs (one block of width 192: 253 -> 102 us, four of 256 316 -> 146, eight of
-    // 384 362 -> 349). Large sets gain by the mix of tile lengths (28 blocks of width 1152 12560 -> 12280 us, eight of 1280 5842 ->
+    // of squares and for the scaling in front of the chains: 18 launches where buckets on lanes of their own took about 80 and the events that
+    // join them, which is all that a step of small matrices costs (one block of width 192: 253 -> 99 us, four of 256 316 -> 140, eight of
+    // 384 362 -> 325). Large sets gain by the mix of tile lengths (by that alone 28 blocks of width 1152 12560 -> 12280 us, eight of 1280 5842 ->
     // 5185). The recurrence on the Gram matrix gains less there: its launches are several rounds of short tiles with a tail each, which lanes
     // fill (28 blocks of 384 805 us on lanes, 881 together; four of 512 373 and 331), so beyond TOGETHER_GRAM it keeps the lanes.
     static constexpr double TOGETHER_GRAM = 1e10;                // sum of m m (m + n) over the matrices
@@ -558,8 +566,20 @@ private:
             return false;
         std::vector<Chain> chains;
         for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram));
+        // the last products of the chains go into the weights
+        std::vector<int64_t> addresses;
+        for (size_t i = 0; i < ready.size(); ++i)
+            for (const Item& it : ready[i])
+                for (int64_t plane = 0; plane < chains[i].matrix.size(1); ++plane)
+                    addresses.push_back((int64_t)it.param.const_data_ptr() + plane * chains[i].matrix.size(-2) * chains[i].matrix.size(-1) * 4);
+        const int64_t* at = tables_.get(ADDRESS_TABLE, {}, (int64_t)addresses.size(), (int64_t)g.gram, std::move(addresses), head.param.device(), stream);
+        for (Chain& c : chains) {
+            if (!c.products.empty()) into_weights(c.products.back(), at, g, c.matrix.size(-2), c.matrix.size(-1));
+            at += c.start.batch;
+        }
         run_together(chains, sums, single, stream);
         for (size_t i = 0; i < ready.size(); ++i) {
+            if (chains[i].applied) continue;
             const int64_t count = ready[i][0].param.numel(), rows = chains[i].matrix.size(-2), cols = chains[i].matrix.size(-1);
             const char* from = static_cast<const char*>(chains[i].result.const_data_ptr());
             for (const Item& it : ready[i]) {
@@ -567,12 +587,21 @@ private:
                 from += 2 * count;
             }
         }
-        TORCH_INTERNAL_ASSERT(weights_together(tables_, {}, (int64_t)g.gram, weight_rows, chains[0].result.scalar_type(), (float)g.lr, (float)g.weight_decay, stream));
+        if (!weight_rows.empty())
+            TORCH_INTERNAL_ASSERT(weights_together(tables_, {}, (int64_t)g.gram, weight_rows, chains[0].result.scalar_type(), (float)g.lr, (float)g.weight_decay, stream));
         return true;
     }
 
     static double update_scale(const Group& g, int64_t rows, int64_t cols) {
         return g.match_rms ? .2 * std::pow((double)std::max(rows, cols), .5) : std::pow(std::max(1., (double)rows / (double)cols), .5);
+    }
+
+    // weight = weight * (1 - lr decay) - lr scale update, with the FP32 roundings of viola_weight_update
+    static void into_weights(viola_ns_product& last, const int64_t* weights, const Group& g, int64_t rows, int64_t cols) {
+        const float lr = (float)g.lr, decayed = lr * (float)g.weight_decay;
+        last.weights = weights;
+        last.keep = 1.0f - decayed;
+        last.rate = lr * (float)update_scale(g, rows, cols);
     }
 
     void step_bucket(std::vector<Item>& bucket, int64_t ordinal) {
@@ -611,17 +640,35 @@ private:
             }
         }
 
-        const Tensor updates = newton_schulz(updates_in, g.ns_steps, g.gram);
+        Chain chain = chain_of(updates_in, g.ns_steps, g.gram);
+        prepare(chain, sums_of(chain.start.batch, device).as<float>(0), stream);
+        for (size_t i = 0; i + 1 < chain.products.size(); ++i) multiply(chain.products[i], chain.dtype, stream);
+        const Tensor updates = chain.result;
         const char* from = static_cast<const char*>(updates.const_data_ptr());
         const int update_code = code_of(updates.scalar_type());
 
         // ---- weights
         together = true;
+        bool in_place = true;
         std::vector<WeightRow> weight_rows;
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Group& h = *bucket[i].group;
             together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms;
             weight_rows.push_back({bucket[i].param, from + 2 * count * i, count, (float)update_scale(g, rows, cols)});
+            in_place = in_place && bucket[i].param.scalar_type() == at::kFloat && aligned(bucket[i].param.const_data_ptr(), 16);
+        }
+        if (!chain.products.empty()) {                           // the last product: into the weights where they allow it
+            viola_ns_product& last = chain.products.back();
+            if (together && in_place && rows * cols % 4 == 0) {
+                std::vector<int64_t> addresses;
+                for (const Item& it : bucket)
+                    for (int64_t plane = 0; plane < updates.size(1); ++plane) addresses.push_back((int64_t)it.param.const_data_ptr() + plane * rows * cols * 4);
+                into_weights(last, tables_.get(ADDRESS_TABLE, shape, (int64_t)addresses.size(), ordinal, std::move(addresses), device, stream), g, rows, cols);
+                const int status = VIOLA_TRY(viola_ns_gemm_many, &last, 1, chain.dtype, stream);
+                if (status == 0) return;
+                if (status != VIOLA_EUNSUPPORTED) check("viola_ns_gemm_many", status);
+            }
+            multiply(last, chain.dtype, stream);
         }
         if (together && weights_together(tables_, shape, ordinal, weight_rows, updates.scalar_type(), (float)g.lr, (float)g.weight_decay, stream)) return;
         for (size_t i = 0; i < bucket.size(); ++i) {

@@ -670,10 +670,12 @@ extern "C" int viola_ns_gemm_many(const viola_ns_product* products, int count, i
         const viola_ns_product& p = products[i];
         VIOLA_CHECK_ARG(p.epilogue >= 0 && p.epilogue <= 2 && p.batch >= 0 && p.m >= 0 && p.n >= 0 && p.k >= 0);
         if (p.batch == 0 || p.m == 0 || p.n == 0) continue;
-        VIOLA_CHECK_ARG(p.out && (p.k == 0 || (p.a && p.b)) && (p.epilogue == 0 || p.residual));
+        VIOLA_CHECK_ARG((p.out || p.weights) && (p.k == 0 || (p.a && p.b)) && (p.epilogue == 0 || p.residual));
+        if (p.weights && (p.transpose_b || p.epilogue == 1 || p.out_diag || p.m % 8 || p.n % 8)) return VIOLA_EUNSUPPORTED;
         many.product[many.count++] = {static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), static_cast<const uint16_t*>(p.residual),
                                       static_cast<uint16_t*>(p.out), static_cast<uint16_t*>(p.out_diag), p.batch, p.m, p.n, p.k, p.add_diag, p.transpose_out,
-                                      ns_is_mirrored(p.a, p.b, p.transpose_b, p.m, p.n, p.transpose_out), 0, 0, 0, 0, !p.transpose_b, p.epilogue};
+                                      ns_is_mirrored(p.a, p.b, p.transpose_b, p.m, p.n, p.transpose_out), 0, 0, 0, 0, !p.transpose_b, p.epilogue,
+                                      p.weights, p.keep, p.rate};
     }
     if (many.count == 0) return 0;
     // the longest k first: their tiles are not what the launch waits for at its end

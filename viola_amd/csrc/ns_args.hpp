@@ -18,6 +18,8 @@ struct NsArgs {
     int group_m;                // tile rows per band of the work order (ns_fast.hip)
     int64_t tiles;              // batch * tiles_m * tiles_n
     int b_kn, epilogue;         // read where products of several kinds share a launch
+    const int64_t* weights;     // such launches: not null, weights[batch] -> FP32 [m, n] (transpose_out: [n, m]) = weight * keep - rate * result,
+    float keep, rate;           // and the result itself is not stored
 };
 
 // Products of one launch (by value in the kernel's arguments).
