@@ -53,9 +53,9 @@ def test_products_in_one_launch_equal_one_launch_each(case, dtype):
         assert torch.isfinite(want).all() and torch.equal(got, want), i
 
 
-# (batch, m, n, k, epilogue, transposed weight): edges and remainders of each tile, with a product that is stored in the same launch
+# (batch, m, n, k, epilogue, transposed weight): edges and remainders of each tile, with a product that is stored in the same launch; 128 x 64 alone
 INTO_WEIGHTS = [[(1, 8, 8, 8, 0, 0), (2, 64, 136, 72, 2, 0), (1, 72, 136, 64, 2, 1), (3, 40, 200, 40, 0, 1)], [(20, 256, 384, 256, 2, 1), (24, 264, 136, 40, 0, 0)],
-                [(40, 192, 576, 192, 2, 1), (40, 384, 384, 72, 2, 0), (24, 192, 200, 72, 0, 1)], [(100, 384, 1152, 384, 2, 1), (128, 384, 384, 72, 0, 0), (100, 768, 200, 40, 2, 0)]]
+                [(40, 192, 576, 192, 2, 1), (40, 384, 384, 72, 2, 0), (24, 192, 200, 72, 0, 1)], [(100, 384, 1152, 384, 2, 1), (128, 384, 384, 72, 0, 0), (100, 768, 200, 40, 2, 0)], [(1, 1016, 3080, 1016, 2, 1)]]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -82,13 +82,16 @@ def test_products_into_weights_equal_product_and_update(case, dtype):
         held += [a, b, residual, addresses]
     stored = torch.full((1, 384, 192), float("nan"), device="cuda", dtype=dtype)
     x, y = torch.randn(1, 384, 64, device="cuda").to(dtype), torch.randn(1, 64, 192, device="cuda").to(dtype)
-    more = (Product * (len(case) + 1))(*rows, Product(_lib.ptr(x), _lib.ptr(y), None, _lib.ptr(stored), None, 1, 384, 192, 64, 0.0, 0, 0, 0, None, 0, 0))
-    _lib.call("viola_ns_gemm_many", ctypes.addressof(more), len(case) + 1, _lib.code(dtype))
+    if len(case) > 1:
+        more = (Product * (len(case) + 1))(*rows, Product(_lib.ptr(x), _lib.ptr(y), None, _lib.ptr(stored), None, 1, 384, 192, 64, 0.0, 0, 0, 0, None, 0, 0))
+    else:
+        more = rows
+    _lib.call("viola_ns_gemm_many", ctypes.addressof(more), len(more), _lib.code(dtype))
     for got, want in pairs:
         assert torch.equal(got, want)
     want = torch.empty_like(stored)
     _lib.call("viola_ns_gemm", _lib.ptr(x), _lib.ptr(y), None, _lib.ptr(want), _lib.code(dtype), 0, 0, 1, 384, 192, 64, 0.0, None, 0)
-    assert torch.equal(stored, want)
+    assert len(case) == 1 or torch.equal(stored, want)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -28,12 +28,13 @@ struct Chain {
     Tensor matrix, result;
     Arena arena;
     int dtype = 0;
+    float* sums = nullptr;                                       // of squares, where the chain has room for its own
     viola_ns_matrices start{};                                   // the scaled matrix, in front of the products
     std::vector<viola_ns_product> products;
     bool applied = false;                                        // the last product went into the weights
 };
 
-Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram) {
+Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram, bool own_sums = true) {
     TORCH_CHECK(matrix_.is_cuda(), "viola_amd kernels run on the GPU only");
     TORCH_CHECK(matrix_.dim() >= 2 && steps >= 0, "Newton-Schulz takes matrices and a number of steps, got ", matrix_.dim(), " dimensions and ", steps, " steps");
     Chain c;
@@ -48,10 +49,12 @@ Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram) {
     const bool quintic = !gram || m == n;                        // the plain iteration; else the recurrence on the Gram matrix
     const int64_t wide = 2 * batch * m * n, square = 2 * batch * m * m;
     int64_t x_at[2], s_at[6];
+    const int64_t sums_at = own_sums ? c.arena.take(batch * 256 * 4) : -1;
     const int squares = quintic ? 2 : 6;
     for (int64_t& at : x_at) at = c.arena.take(wide);
     for (int i = 0; i < squares; ++i) s_at[i] = c.arena.take(square);
     c.arena.make(c.matrix.device());
+    if (own_sums) c.sums = c.arena.as<float>(sums_at);
     void *x = steps ? c.arena.at(x_at[0]) : c.result.mutable_data_ptr(), *spare = c.arena.at(x_at[1]);   // no steps: the scaled matrix
     c.start = {c.matrix.const_data_ptr(), x, batch, rows, cols};
     if (steps == 0) return c;
@@ -121,7 +124,7 @@ Tensor newton_schulz(const Tensor& matrix, int64_t steps, bool gram) {
     const Chain c = chain_of(matrix, steps, gram);
     if (c.matrix.numel() == 0) return c.result;
     const viola_stream_t stream = stream_of(c.matrix);
-    prepare(c, sums_of(c.start.batch, c.matrix.device()).as<float>(0), stream);
+    prepare(c, c.sums, stream);
     for (const viola_ns_product& p : c.products) multiply(p, c.dtype, stream);
     return c.result;
 }
@@ -565,7 +568,7 @@ private:
                                single ? sums.as<float>(0) : nullptr, g.gram ? VIOLA_F16 : VIOLA_BF16))
             return false;
         std::vector<Chain> chains;
-        for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram));
+        for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram, false));
         // the last products of the chains go into the weights
         std::vector<int64_t> addresses;
         for (size_t i = 0; i < ready.size(); ++i)
@@ -596,6 +599,7 @@ private:
         return g.match_rms ? .2 * std::pow((double)std::max(rows, cols), .5) : std::pow(std::max(1., (double)rows / (double)cols), .5);
     }
 
+    static constexpr int64_t INTO_WEIGHTS = 6 << 20;             // elements of a bucket on a lane
     // weight = weight * (1 - lr decay) - lr scale update, with the FP32 roundings of viola_weight_update
     static void into_weights(viola_ns_product& last, const int64_t* weights, const Group& g, int64_t rows, int64_t cols) {
         const float lr = (float)g.lr, decayed = lr * (float)g.weight_decay;
@@ -641,7 +645,7 @@ private:
         }
 
         Chain chain = chain_of(updates_in, g.ns_steps, g.gram);
-        prepare(chain, sums_of(chain.start.batch, device).as<float>(0), stream);
+        prepare(chain, chain.sums, stream);
         for (size_t i = 0; i + 1 < chain.products.size(); ++i) multiply(chain.products[i], chain.dtype, stream);
         const Tensor updates = chain.result;
         const char* from = static_cast<const char*>(updates.const_data_ptr());
@@ -657,9 +661,11 @@ private:
             weight_rows.push_back({bucket[i].param, from + 2 * count * i, count, (float)update_scale(g, rows, cols)});
             in_place = in_place && bucket[i].param.scalar_type() == at::kFloat && aligned(bucket[i].param.const_data_ptr(), 16);
         }
-        if (!chain.products.empty()) {                           // the last product: into the weights where they allow it
+        if (!chain.products.empty()) {
+            // the last product: into the weights where they allow it, and are enough for several rounds of tiles (below that other lanes
+            // hide the weights' launch better than a tile hides their loads: two blocks of 768, recurrence, 400 us, 420 so)
             viola_ns_product& last = chain.products.back();
-            if (together && in_place && rows * cols % 4 == 0) {
+            if (together && in_place && rows * cols % 4 == 0 && size * count >= INTO_WEIGHTS) {
                 std::vector<int64_t> addresses;
                 for (const Item& it : bucket)
                     for (int64_t plane = 0; plane < updates.size(1); ++plane) addresses.push_back((int64_t)it.param.const_data_ptr() + plane * rows * cols * 4);

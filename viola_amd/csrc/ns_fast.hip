@@ -635,7 +635,9 @@ NsTile ns_choose_tile_many(const NsMany& many) {
     if (!symmetric && area[0] <= area[1] && blocks[0] >= 3 * 256) return NS_TILE_384x192;
     if (area[1] * 20 <= area[2] * 21 && blocks[1] >= NS_FILL) return NS_TILE_192x192;
     if (area[1] * 25 <= area[2] * 27 && blocks[1] >= 1024) return NS_TILE_192x192;
-    return blocks[2] >= NS_FILL ? NS_TILE_128x128 : NS_TILE_64x64;
+    if (blocks[2] >= NS_FILL) return NS_TILE_128x128;
+    // a product alone, as in a launch of its own
+    return many.count == 1 ? ns_choose_tile(many.product[0].batch, many.product[0].m, many.product[0].n, symmetric) : NS_TILE_64x64;
 }
 
 template <bool IS_BF16, int WM, int WN, int WAVES_M, int WAVES_N, int SBK, int STAGES>
@@ -655,6 +657,7 @@ static void launch_shape_many(const NsMany& many, hipStream_t stream) {
         case NS_TILE_384x192: launch_tiles_many<IS_BF16, 3, 3, 4, 2, 64, 2>(many, stream); break;
         case NS_TILE_192x192: launch_tiles_many<IS_BF16, 3, 3, 2, 2, 32, 3>(many, stream); break;
         case NS_TILE_128x128: launch_tiles_many<IS_BF16, 2, 2, 2, 2, 32, 3>(many, stream); break;
+        case NS_TILE_128x64: launch_tiles_many<IS_BF16, 2, 1, 2, 2, 32, 3>(many, stream); break;
         default: launch_tiles_many<IS_BF16, 1, 1, 2, 2, NS_SMALL_SBK, NS_SMALL_STAGES>(many, stream); break;
     }
 }
