@@ -323,8 +323,8 @@ def main():
             if args.muon_streams:
                 opt._LANES = args.muon_streams
             step_ms, step_wall = timed(opt.step, 5, 3)
-            # the step runs its shape buckets on several streams; for per-launch durations that do not overlap each
-            # other the instrumented pass (and one timing next to it) keeps them on one
+            # a step whose matrices do not share their launches runs its shape buckets on several streams; for per-launch
+            # durations that do not overlap each other the instrumented pass (and one timing next to it) keeps them on one
             lanes, opt._LANES = opt._LANES, 1
             serial_ms, _ = timed(opt.step, 3, 1)
             b = kernel_breakdown(opt.step, 2)
@@ -336,15 +336,18 @@ def main():
                         ns_flops += 5 * (4 * m_ * m_ * n_ + 2 * m_ ** 3)
                     else:
                         ns_flops += 5 * 6 * m_ ** 3 if m_ == n_ else 8 * m_ * m_ * n_ + 28 * m_ ** 3
-            ns_ms = b["viola_ns_gemm"]["avg_ms"] * b["viola_ns_gemm"]["launches_per_step"]
-            mom = b.get("viola_momentum_update_table") or b["viola_momentum_update"]
-            upd = b.get("viola_weight_update_table") or b["viola_weight_update"]
-            extra[f"muon_{method}"] = dict(step_ms=step_ms, step_wall_ms=step_wall, streams=lanes, step_one_stream_ms=serial_ms,
+            def spent(prefix):
+                return sum(v["avg_ms"] * v["launches_per_step"] for name, v in b.items() if name.startswith(prefix))
+
+            ns_ms, momentum_ms, weight_ms = spent("viola_ns_gemm"), spent("viola_momentum_update"), spent("viola_weight_update")
+            shared = b.get("viola_ns_prepare_many", {}).get("launches_per_step") == 1
+            extra[f"muon_{method}"] = dict(step_ms=step_ms, step_wall_ms=step_wall, streams=1 if shared else lanes, step_one_stream_ms=serial_ms,
                                            muon_elements=elements,
                                            ns_gemm_ms=ns_ms, ns_tflops=ns_flops / (ns_ms * 1e-3) / 1e12,
                                            ns_frac_bf16_peak=ns_flops / (ns_ms * 1e-3) / 1e12 / PEAK["bf16_tflops"],
-                                           momentum_gbs=8.03 * elements / (mom["avg_ms"] * mom["launches_per_step"] * 1e-3) / 1e9,
-                                           weight_update_gbs=10 * elements / (upd["avg_ms"] * upd["launches_per_step"] * 1e-3) / 1e9,
+                                           momentum_gbs=8.03 * elements / (momentum_ms * 1e-3) / 1e9,
+                                           # none where the last product of a chain goes into the weights (its time is in ns_gemm_ms)
+                                           weight_update_gbs=10 * elements / (weight_ms * 1e-3) / 1e9 if weight_ms else None,
                                            launches_per_step=sum(v["launches_per_step"] for v in b.values()))
             del opt, params
             torch.cuda.empty_cache()

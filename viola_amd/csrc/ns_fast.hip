@@ -245,7 +245,7 @@ __device__ __forceinline__ void ns_tile(const NsArgs& p, int64_t work, uint16_t*
     };
     // WEIGHTS: a piece of the result goes into the weight, whose piece at the same place is fetched beforehand (all of a 32-row block's: a
     // store to the weight holds back the loads behind it; before the first chunk where the registers allow it). In place of a pass of
-    // 10 bytes per element over results that are 2 bytes each to store: 28 blocks of width 1152 1110 + 816 -> 1380 us of a step, 11.9 -> 11.2
+    // 10 bytes per element over results that are 2 bytes each to store: 28 blocks of width 1152 1100 + 816 -> 1440 us of a step, 11.9 -> 11.2
     // ms; eight of 768 1337 -> 1222 us, four of 512 310 -> 292.
     float* const weight = WEIGHTS ? reinterpret_cast<float*>(p.weights[bz]) : nullptr;
     struct Piece8 { float4 a, b; };
