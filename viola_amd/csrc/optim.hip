@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void momentum_table_quads(const int64_t* __res
 
 // The same with what Newton-Schulz starts from, the sums of squares of the updates: up to 256 blocks per tensor, each with a share of its tiles
 // sixteen at a time, leave their sums in sums[tensor][block] (zeros in the rest of the 256), which is what a pass over the updates would write (viola_ns_prepare), so that this pass, 2
-// bytes per element, is not needed: 28 blocks of width 1152 625 + 181 -> 688 us (with blocks of 256 threads 738), one of 1024 x 1024 5.3 + 3.3 -> 5.7.
+// bytes per element, is not needed: 28 blocks of width 1152 625 + 181 -> 660 us (with blocks of 256 threads 40 more), one of 1024 x 1024 5.3 + 3.3 -> 5.7.
 constexpr int SQUARES_PARTS = 256;
 template <typename TG, int EPL, bool STOCHASTIC, int SQUARES>
 __global__ __launch_bounds__(1024) void momentum_squares_quads(const int64_t* __restrict__ table, int64_t blocks, float beta,

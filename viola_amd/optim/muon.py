@@ -110,8 +110,8 @@ class FP8Muon(MatrixOptimizer):
             self.observer.momentum(param, grad, *before, q, scale, matrix, group, 1., quant)
         return matrix
 
-    # Streams the shape buckets of one step are spread over, and the most elements one bucket's chain takes
-    # (csrc/host_optim.cpp: step_buckets, batch_elements).
+    # Streams the shape buckets of one step are spread over where they do not share their launches, and the most elements one bucket's chain takes
+    # (csrc/host_optim.cpp: step_together, step_buckets, batch_elements).
     _LANES, _BATCH_ELEMENTS = 4, 1 << 28
 
     @property
