@@ -166,6 +166,14 @@ int viola_tensor_encode(const void* x, int x_dtype, int64_t rows, int64_t cols, 
                         float* history, int history_len, int64_t index, int delayed, float limit, float* scale, void* q,
                         int64_t q_pitch, void* qt, int64_t qt_pitch, int q_dtype, void* column_sum, int sum_dtype,
                         viola_stream_t stream);
+/* The same, and in the quantizer's launch codes_t [code_cols, code_pitch] = codes [code_rows, code_cols] transposed, zeros past the rows (the one-matrix,
+ * scale-less viola_codes_transpose_pitched). codes may be NULL. VIOLA_EUNSUPPORTED, with nothing launched, also for code_rows, code_cols,
+ * code_pitch or addresses that are no multiples of 4, and without q and qt. */
+int viola_tensor_encode_beside(const void* x, int x_dtype, int64_t rows, int64_t cols, float* workspace, int64_t workspace_floats,
+                               float* history, int history_len, int64_t index, int delayed, float limit, float* scale, void* q,
+                               int64_t q_pitch, void* qt, int64_t qt_pitch, int q_dtype, void* column_sum, int sum_dtype,
+                               const void* codes, void* codes_t, int64_t code_rows, int64_t code_cols, int64_t code_pitch,
+                               viola_stream_t stream);
 int64_t viola_tensor_encode_slices(int x_dtype, int64_t rows, int64_t cols);
 
 /* ---------------------------------------------------------------- Hadamard-64 rotation (`rotation_size=64`)

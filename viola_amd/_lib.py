@@ -28,6 +28,7 @@ _SIGNATURES = {
     "viola_codes_transpose_pitched": [_p, _p, _l, _l, _l, _l, _p, _p, _i, _i, _i, _p, _l, _l, _p, _i, _p],
     "viola_codes_repack": [_p, _p, _l, _l, _l, _l, _p, _p, _i, _i, _i, _p],
     "viola_tensor_encode": [_p, _i, _l, _l, _p, _l, _p, _i, _l, _i, _f, _p, _p, _l, _p, _l, _i, _p, _i, _p],
+    "viola_tensor_encode_beside": [_p, _i, _l, _l, _p, _l, _p, _i, _l, _i, _f, _p, _p, _l, _p, _l, _i, _p, _i, _p, _p, _l, _l, _l, _p],
     "viola_gated_quantize_dual": [_p, _i, _l, _l, _i, _p, _p, _p, _p, _i, _i, _f, _i, _p],
     "viola_gated_quantize_dual_pitched": [_p, _i, _l, _l, _i, _p, _l, _p, _p, _l, _p, _i, _f, _i, _p],
     "viola_gated_backward_quantize_dual": [_p, _p, _i, _l, _l, _i, _p, _p, _p, _l, _p, _i, _f, _p, _i, _p],

@@ -556,6 +556,8 @@ Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const T
     const bool requantize = make_wt && !cached && !r.fp8_weight; // memory mode with 16-bit storage: this forward's codes again
     const int64_t w_q = requantize ? temp.take(r.out * r.in) : -1;
     const int64_t w_s = requantize && r.grouped ? temp.take(ceil_div(r.out, 32) * ceil_div(r.in, 32) * r.scale_bytes()) : -1;
+    // per-tensor codes as stored: the quantizer of dy turns them in its own launch where they are whole words
+    const bool beside = make_wt && !cached && !requantize && !r.grouped && r.out % 4 == 0 && r.in % 4 == 0 && pitch % 4 == 0 && reinterpret_cast<uintptr_t>(ptr(w)) % 4 == 0;
     if (needs_b) out.db = at::empty({r.out}, dx_options.dtype(kept.bias_grad));
     int k_parts = 1;                                             // of the weight gradient's k range, and the partial products
     int64_t k_parts_at = -1;
@@ -587,17 +589,18 @@ Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const T
         float* scale = temp.as<float>(scale_at);
         const Tensor& history = l.history[GRAD];
         auto encode = [&](bool with_sum) {
-            return VIOLA_TRY(viola_tensor_encode, ptr(dy), dtype, rows, r.out, temp.as<float>(work_at), floats, static_cast<float*>(history.mutable_data_ptr()),
+            return VIOLA_TRY(viola_tensor_encode_beside, ptr(dy), dtype, rows, r.out, temp.as<float>(work_at), floats, static_cast<float*>(history.mutable_data_ptr()),
                              (int)history.numel(), l.counter[GRAD]->value, l.counter[GRAD]->delayed, r.bwd_limit, scale, needs_x ? temp.at(q) : nullptr, pitch,
                              needs_w ? temp.at(qt) : nullptr, pitch_t, r.bwd, with_sum ? out.db.mutable_data_ptr() : nullptr,
-                             with_sum ? code_of(kept.bias_grad) : VIOLA_F32, stream);
+                             with_sum ? code_of(kept.bias_grad) : VIOLA_F32, beside ? ptr(w) : nullptr, beside ? temp.at(wt_q) : nullptr, r.out, r.in, pitch,
+                             stream);
         };
         int status = encode(rides);
         if (status == VIOLA_EUNSUPPORTED && rides) {             // columns that are not whole 16-byte pieces: the sum as a pass of its own
             out.db = at::sum(dy, at::IntArrayRef{0}, false, kept.bias_grad);
             status = encode(false);
         }
-        check("viola_tensor_encode", status);
+        check("viola_tensor_encode_beside", status);
         ++l.counter[GRAD]->value;
         if (needs_x) g = {temp.at(q), scale, pitch};
         if (needs_w) gt = {temp.at(qt), scale, pitch_t};
@@ -608,7 +611,7 @@ Gradients unproject(const Layer& l, const Kept& kept, const Restored& t, const T
         if (make_wt && cached) {
             VIOLA_CALL(viola_codes_repack, ptr(t.weight_t), temp.at(wt_q), 1, r.in, r.out, pitch, r.grouped ? ptr(t.weight_t_scale) : nullptr,
                        r.grouped ? temp.at(wt_s) : nullptr, 32, 32, r.scale_format(), stream);
-        } else if (make_wt) {
+        } else if (make_wt && !beside) {
             const void* codes = ptr(w);
             if (requantize) {
                 codes = temp.at(w_q);

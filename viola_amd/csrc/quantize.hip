@@ -12,6 +12,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "transpose_words.hpp"
 
 namespace viola {
 
@@ -669,9 +670,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const TQ* __restrict__ 
 }
 
 // ------------------------------------------------------------------ byte transpose, 64 x 64 tile
-// WORDS: rows and cols multiples of 4 and both pointers 4-byte aligned. A thread then owns a 4 x 4 byte block: four
-// 4-byte loads (16 lanes cover 64 contiguous bytes of a row), a 4 x 4 transpose with byte permutes, the four words
-// handed over through LDS so that the stores are again 64 contiguous bytes per 16 lanes.
+// WORDS: rows, cols and pitch multiples of 4 and both pointers 4-byte aligned (transpose_words).
 // With a scale grid (one entry of scale_bytes bytes per block of codes, [srows, scols]), the grid is transposed in the
 // same launch: the blocks share out its entries, thread 0 .. moving one each. Rows of the output are out_pitch codes
 // (scale_pitch entries) apart; what lies past the matrix is zero codes and zero scales.
@@ -712,26 +711,7 @@ __global__ __launch_bounds__(256) void transpose_bytes(const uint8_t* __restrict
     out += (int64_t)blockIdx.z * out_pitch * cols;
     if constexpr (WORDS) {
         __shared__ uint32_t tile[64][17];
-        const int b = threadIdx.x % 16, a = threadIdx.x / 16;               // block of rows 4a.., cols 4b..
-        uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (r0 + 4 * a + i < rows && c0 + 4 * b < cols) w[i] = *reinterpret_cast<const uint32_t*>(x + (r0 + 4 * a + i) * cols + c0 + 4 * b);
-        // t[j] = byte j of w[0..3]
-        const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);   // w0.b0 w1.b0 w0.b1 w1.b1
-        const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);   // w0.b2 w1.b2 w0.b3 w1.b3
-        const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-        const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-        tile[4 * b + 0][a] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);    // bytes 0,1 of lo01 then of lo23
-        tile[4 * b + 1][a] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-        tile[4 * b + 2][a] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-        tile[4 * b + 3][a] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = threadIdx.x / 16 + 16 * i, ra = threadIdx.x % 16;
-            if (c0 + c < cols && r0 + 4 * ra < out_pitch) *reinterpret_cast<uint32_t*>(out + (c0 + c) * out_pitch + r0 + 4 * ra) = tile[c][ra];
-        }
+        transpose_words(x, out, rows, cols, out_pitch, r0, c0, tile);
     } else {
         __shared__ uint8_t tile[64][64 + 4];
         for (int id = threadIdx.x; id < 64 * 64; id += 256) {
