@@ -361,7 +361,7 @@ int viola_momentum_update_table(const int64_t* table, int64_t tensors, int64_t t
                                 viola_stream_t stream);
 
 /* viola_momentum_update_table that also leaves the sums of squares of the updates, read in working_dtype (bf16 or f16), in
- * sums[tensor][256]: the first stage of viola_ns_prepare for one matrix per tensor (its partial sums in another order). */
+ * sums[tensor][256]: the first stage of viola_ns_prepare for one matrix per tensor, bit for bit where its columns are a multiple of 8. */
 int viola_momentum_update_squares(const int64_t* table, int64_t tensors, int64_t tiles, int grad_dtype, int tile_size,
                                   float beta, float inv_loss_scale, int nesterov, int rounding, int64_t rounding_step,
                                   int working_dtype, float* sums, viola_stream_t stream);

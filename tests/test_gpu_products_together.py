@@ -116,8 +116,7 @@ def test_scaled_matrices_of_several_shapes_equal_one_shape_each(dtype):
 @pytest.mark.parametrize("working", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("grads,tile,rounding", [(torch.float32, 256, 0), (torch.bfloat16, 512, 1), (torch.float16, 1024, 0), (torch.float32, 1024, 1)])
 def test_momentum_with_sums_of_squares(grads, tile, rounding, working):
-    """State and updates are those of viola_momentum_update, one tensor at a time; the sums, whose order is not specified, those of the
-    updates in float64: at most 2^-24 for each of the some 40 additions on the way of a term."""
+    """State and updates are those of viola_momentum_update, one tensor at a time; the sums those of the updates in float64: at most 2^-24 for each of the some 40 additions on the way of a term."""
     torch.manual_seed(tile)
     tiles = [1, 5, 16, 300, 4099]
     table, want, got, held = [], [], [], []

@@ -12,6 +12,7 @@
 #include <mutex>
 
 #include "ns_args.hpp"
+#include "ns_sums.hpp"
 
 namespace viola {
 
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(256, 2) void ns_gemm_kernel(const uint16_t* __restr
 
 // ------------------------------------------------------------------ normalisation
 // Stage 1: partial sums of squares of dtype(in) per (batch, slice) -> workspace[batch][PARTS].
-constexpr int PARTS = 256;
+constexpr int PARTS = NS_PARTS;
 
 template <typename TIn, bool IS_BF16>
 __global__ __launch_bounds__(256) void ns_sumsq_kernel(const TIn* __restrict__ in, float* __restrict__ workspace, int64_t count) {
@@ -280,28 +281,42 @@ template <typename TIn, bool IS_BF16> __device__ __forceinline__ float ns_workin
     return half_to_f32<IS_BF16>(f32_to_half<IS_BF16>(v));
 }
 
+// Partial sums of matrix bz, a slot per block of four wavefronts with four chunks each (ns_sums.hpp), four units in flight. Before (256 contiguous
+// ranges in 16-byte loads) and now, us: 56 x 1152 x 4608 128, 127; 28 x 3456 x 1152 45.6, 46.0; one of 4096 x 4096 12.7, 7.5; 28 x 384 x 384 5.4, 3.6; one of
+// 1024 x 1024 2.7, 3.0.
 template <typename TIn, bool IS_BF16>
 __device__ __forceinline__ void ns_sumsq16(const TIn* __restrict__ in, float* __restrict__ workspace, int64_t count, int64_t bz) {
-    const uint4* src = reinterpret_cast<const uint4*>(in + bz * count);
-    const int64_t octets = count / 8;
-    const int64_t per = (octets + PARTS - 1) / PARTS;
-    const int64_t begin = (int64_t)blockIdx.x * per;
-    const int64_t end = begin + per < octets ? begin + per : octets;
-    float sum = 0.0f;
-    for (int64_t i = begin + threadIdx.x; i < end; i += 256) {
-        const uint4 raw = src[i];
-        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+    constexpr int KEPT = 4, TURNS = 4;
+    const TIn* src = in + bz * count;
+    float sums[KEPT] = {};
+    auto add = [&](float& sum, const uint2& raw) {
+        const float v[4] = {ns_working<TIn, IS_BF16>(raw.x & 0xffffu), ns_working<TIn, IS_BF16>(raw.x >> 16), ns_working<TIn, IS_BF16>(raw.y & 0xffffu),
+                            ns_working<TIn, IS_BF16>(raw.y >> 16)};
+        ns_add_squares(sum, v);
+    };
+    const int64_t turn = (int64_t)gridDim.x * NS_UNIT;
+    int64_t unit = (int64_t)blockIdx.x * NS_UNIT;
+    const int lane = threadIdx.x / WAVE * (KEPT * NS_CHUNK) + threadIdx.x % WAVE * 4;   // first of the thread's elements in a unit
+    for (; unit + (TURNS - 1) * turn + NS_UNIT <= count; unit += TURNS * turn) {
+        uint2 raw[TURNS][KEPT];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float v = ns_working<TIn, IS_BF16>(e % 2 ? w[e / 2] >> 16 : w[e / 2] & 0xffffu);
-            sum += v * v;
-        }
+        for (int t = 0; t < TURNS; ++t)
+#pragma unroll
+            for (int k = 0; k < KEPT; ++k) raw[t][k] = *reinterpret_cast<const uint2*>(src + unit + t * turn + lane + k * NS_CHUNK);
+#pragma unroll
+        for (int t = 0; t < TURNS; ++t)
+#pragma unroll
+            for (int k = 0; k < KEPT; ++k) add(sums[k], raw[t][k]);
     }
-    __shared__ float partial[4];
-    sum = wave_sum(sum);
-    if (threadIdx.x % WAVE == 0) partial[threadIdx.x / WAVE] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) workspace[bz * PARTS + blockIdx.x] = (partial[0] + partial[1]) + (partial[2] + partial[3]);
+    for (int64_t at = unit + lane; at < count; at += turn) {
+        uint2 raw[KEPT];
+#pragma unroll
+        for (int k = 0; k < KEPT; ++k) raw[k] = *reinterpret_cast<const uint2*>(src + (at + k * NS_CHUNK < count ? at + k * NS_CHUNK : at));
+#pragma unroll
+        for (int k = 0; k < KEPT; ++k)
+            if (at + k * NS_CHUNK < count) add(sums[k], raw[k]);
+    }
+    ns_store_slot(sums, workspace + bz * NS_PARTS);
 }
 
 template <typename TIn, bool IS_BF16>
@@ -544,7 +559,7 @@ static int launch_prepare(const void* in, void* out, int64_t batch, int64_t rows
     if constexpr (sizeof(TIn) == 2) {
         const bool aligned = reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
         if (aligned && cols % 8 == 0 && (rows * cols) % 8 == 0 && (rows + 127) / 128 <= 65535) {
-            VIOLA_LAUNCH((ns_sumsq16_kernel<TIn, IS_BF16>), dim3(PARTS, (unsigned)batch), dim3(256), 0, stream, src, workspace, rows * cols);
+            VIOLA_LAUNCH((ns_sumsq16_kernel<TIn, IS_BF16>), ns_sum_blocks(rows * cols, batch), dim3(256), 0, stream, src, workspace, rows * cols);
             if (rows > cols) {
                 const dim3 tgrid((unsigned)((cols + 63) / 64), (unsigned)((rows + 127) / 128), (unsigned)batch);
                 VIOLA_LAUNCH((ns_scale16_transposed_kernel<TIn, IS_BF16>), tgrid, dim3(256), 0, stream, src, static_cast<uint16_t*>(out), workspace, rows, cols);
@@ -689,7 +704,7 @@ extern "C" int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count,
     VIOLA_CHECK_ARG((dtype == VIOLA_BF16 || dtype == VIOLA_F16) && count >= 0 && (count == 0 || (shapes && workspace)));
     if (count > NS_MANY) return VIOLA_EUNSUPPORTED;
     NsPrepareMany many{};
-    int64_t matrices = 0, blocks = 0;
+    int64_t matrices = 0, blocks = 0, largest = 0;
     for (int i = 0; i < count; ++i) {
         const viola_ns_matrices& s = shapes[i];
         VIOLA_CHECK_ARG(s.batch >= 0 && s.rows >= 0 && s.cols >= 0);
@@ -699,14 +714,15 @@ extern "C" int viola_ns_prepare_many(const viola_ns_matrices* shapes, int count,
         if (!aligned || s.cols % 8 || (matrices += s.batch) > 65535) return VIOLA_EUNSUPPORTED;
         const int64_t parts = s.rows > s.cols ? ((s.cols + 63) / 64) * ((s.rows + 127) / 128) : ns_scale_blocks(s.rows * s.cols / 8, s.batch);
         if (parts >= (1ll << 31) || (blocks += parts * s.batch) >= (1ll << 31)) return VIOLA_EUNSUPPORTED;
+        largest = std::max(largest, s.rows * s.cols);
         many.shape[many.count++] = {static_cast<const bf16_t*>(s.in), static_cast<uint16_t*>(s.out), s.rows, s.cols, (int)s.batch, (int)parts};
     }
     if (many.count == 0) return 0;
     if (dtype == VIOLA_BF16) {
-        if (!have_sums) VIOLA_LAUNCH(ns_sumsq16_many<true>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
+        if (!have_sums) VIOLA_LAUNCH(ns_sumsq16_many<true>, ns_sum_blocks(largest, matrices), dim3(256), 0, stream, many, workspace);
         VIOLA_LAUNCH(ns_scale16_many<true>, dim3((unsigned)blocks), dim3(256), 0, stream, many, workspace);
     } else {
-        if (!have_sums) VIOLA_LAUNCH(ns_sumsq16_many<false>, dim3(PARTS, (unsigned)matrices), dim3(256), 0, stream, many, workspace);
+        if (!have_sums) VIOLA_LAUNCH(ns_sumsq16_many<false>, ns_sum_blocks(largest, matrices), dim3(256), 0, stream, many, workspace);
         VIOLA_LAUNCH(ns_scale16_many<false>, dim3((unsigned)blocks), dim3(256), 0, stream, many, workspace);
     }
     return viola_launch_status();

@@ -4,6 +4,7 @@
 // reference kernels write it. Pointers need only element alignment: accesses are per element,
 // lane-contiguous, so a wavefront still reads and writes whole cache lines.
 #include "common.hpp"
+#include "ns_sums.hpp"
 
 namespace viola {
 
@@ -102,16 +103,16 @@ template <> __device__ __forceinline__ void load_quad<f16_t>(const f16_t* p, flo
     v[0] = (float)t[0]; v[1] = (float)t[1]; v[2] = (float)t[2]; v[3] = (float)t[3];
 }
 
-// SQUARES: also the lane's sum of squares of its update as Newton-Schulz reads it, in bf16 (1) or rounded to FP16 once more (2).
+// SQUARES: adds the squares of the lane's update as Newton-Schulz reads it, in bf16 (1) or rounded to FP16 once more (2), to squares[its chunk of 256].
 template <typename TG, int EPL, bool STOCHASTIC, int SQUARES = 0>
-__device__ __forceinline__ float momentum_quads_tile(const TG* __restrict__ grad, const uint8_t* old_q, const float* old_scale,
-                                                     uint8_t* new_q, float* new_scale, uint16_t* __restrict__ update, int64_t b,
-                                                     float beta, float inv_loss_scale, int nesterov, uint64_t step, uint64_t key) {
+__device__ __forceinline__ void momentum_quads_tile(const TG* __restrict__ grad, const uint8_t* old_q, const float* old_scale,
+                                                    uint8_t* new_q, float* new_scale, uint16_t* __restrict__ update, int64_t b,
+                                                    float beta, float inv_loss_scale, int nesterov, uint64_t step, uint64_t key,
+                                                    float* squares = nullptr) {
     constexpr int TILE = EPL * WAVE, QUADS = EPL / 4;
     const int lane = threadIdx.x % WAVE;
     const float scale_old = old_scale[b];
     const float one_minus = 1.0f - beta;
-    float squares = 0.0f;
     float g[QUADS][4], m[QUADS][4];
     float amax = 0.0f, poison = 0.0f;
 #pragma unroll
@@ -169,13 +170,11 @@ __device__ __forceinline__ float momentum_quads_tile(const TG* __restrict__ grad
         if constexpr (SQUARES != 0) {
             float v[4] = {__uint_as_float(stored.x << 16), __uint_as_float(stored.x & 0xffff0000u), __uint_as_float(stored.y << 16), __uint_as_float(stored.y & 0xffff0000u)};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < 4; ++e)
                 if (SQUARES == 2) v[e] = (float)(_Float16)v[e];
-                squares += v[e] * v[e];
-            }
+            ns_add_squares(squares[c], v);
         }
     }
-    return squares;
 }
 
 template <typename TG, int EPL, bool STOCHASTIC>
@@ -202,32 +201,24 @@ __global__ __launch_bounds__(256) void momentum_table_quads(const int64_t* __res
                                              inv_loss_scale, nesterov, step, (uint64_t)row[6]);
 }
 
-// The same with what Newton-Schulz starts from, the sums of squares of the updates: up to 256 blocks per tensor, each with a share of its tiles
-// sixteen at a time, leave their sums in sums[tensor][block] (zeros in the rest of the 256), which is what a pass over the updates would write (viola_ns_prepare), so that this pass, 2
-// bytes per element, is not needed: 28 blocks of width 1152 625 + 181 -> 660 us (with blocks of 256 threads 40 more), one of 1024 x 1024 5.3 + 3.3 -> 5.7.
-constexpr int SQUARES_PARTS = 256;
+// The same with what Newton-Schulz starts from, the sums of squares of the updates in sums[tensor][256], so that the pass over the updates that
+// would form them (viola_ns_prepare's first), 2 bytes per element, is not needed. In that pass's order, whatever the tile (ns_sums.hpp): a block
+// takes a unit of a tensor at a time, each wavefront a tile of it. 28 blocks of width 1152 625 + 181 -> 660 us. Blocks of 16 tiles, whose order
+// depended on the tile, and now, us: 56 x 1152 x 4608 in tiles of 256 427, 430, of 1024 459, 458; one of 1024 x 1024 4.1, 4.2 and 7.8, 5.6;
+// 4096 x 4096 23.3, 23.4 and 22.6, 27.9 (blocks of four wavefronts, and no other matrix to fill the chip).
 template <typename TG, int EPL, bool STOCHASTIC, int SQUARES>
-__global__ __launch_bounds__(1024) void momentum_squares_quads(const int64_t* __restrict__ table, int64_t blocks, float beta,
-                                                               float inv_loss_scale, int nesterov, uint64_t step, float* __restrict__ sums) {
-    constexpr int WAVES = 1024 / WAVE;
+__global__ __launch_bounds__(4096 / EPL) void momentum_squares_quads(const int64_t* __restrict__ table, int64_t blocks, float beta,
+                                                                     float inv_loss_scale, int nesterov, uint64_t step, float* __restrict__ sums) {
+    constexpr int TILES = NS_UNIT / (EPL * WAVE);
     const int64_t* row = table + (int64_t)blockIdx.y * 8;
     const int64_t tiles = row[7] ? row[7] : blocks;
-    const int wave = threadIdx.x / WAVE;
-    float sum = 0.0f;
-    for (int64_t b = (int64_t)blockIdx.x * WAVES + wave; b < tiles; b += (int64_t)gridDim.x * WAVES)
-        sum += momentum_quads_tile<TG, EPL, STOCHASTIC, SQUARES>(reinterpret_cast<const TG*>(row[0]), reinterpret_cast<const uint8_t*>(row[1]),
-                                                                 reinterpret_cast<const float*>(row[2]), reinterpret_cast<uint8_t*>(row[3]),
-                                                                 reinterpret_cast<float*>(row[4]), reinterpret_cast<uint16_t*>(row[5]), b, beta,
-                                                                 inv_loss_scale, nesterov, step, (uint64_t)row[6]);
-    __shared__ float partial[WAVES];
-    sum = wave_sum(sum);
-    if (threadIdx.x % WAVE == 0) partial[wave] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        sum = 0.0f;
-        for (int w = 0; w < WAVES; ++w) sum += partial[w];
-        for (unsigned slot = blockIdx.x; slot < SQUARES_PARTS; slot += gridDim.x) sums[(int64_t)blockIdx.y * SQUARES_PARTS + slot] = slot == blockIdx.x ? sum : 0.0f;
-    }
+    float squares[EPL / 4] = {};
+    for (int64_t b = (int64_t)blockIdx.x * TILES + threadIdx.x / WAVE; b < tiles; b += (int64_t)gridDim.x * TILES)
+        momentum_quads_tile<TG, EPL, STOCHASTIC, SQUARES>(reinterpret_cast<const TG*>(row[0]), reinterpret_cast<const uint8_t*>(row[1]),
+                                                          reinterpret_cast<const float*>(row[2]), reinterpret_cast<uint8_t*>(row[3]),
+                                                          reinterpret_cast<float*>(row[4]), reinterpret_cast<uint16_t*>(row[5]), b, beta,
+                                                          inv_loss_scale, nesterov, step, (uint64_t)row[6], squares);
+    ns_store_slot(squares, sums + (int64_t)blockIdx.y * NS_PARTS);
 }
 
 // ------------------------------------------------------------------ 2-D blocks: one wavefront per block
@@ -520,11 +511,10 @@ extern "C" int viola_momentum_update_squares(const int64_t* table, int64_t tenso
     VIOLA_CHECK_ARG(working_dtype == VIOLA_BF16 || working_dtype == VIOLA_F16);
     if (tensors == 0) return 0;
     VIOLA_CHECK_ARG(table && sums);
-    const int64_t blocks = (tiles + 15) / 16;                                // SQUARES_PARTS: what viola_ns_prepare's second stage adds
-    const dim3 grid((unsigned)(blocks < 1 ? 1 : blocks > SQUARES_PARTS ? SQUARES_PARTS : blocks), (unsigned)tensors);
+    const dim3 grid = ns_sum_blocks(tiles * tile_size, tensors);
     auto launch = [&](auto type, auto quads, auto stochastic, auto squares) {
-        VIOLA_LAUNCH((momentum_squares_quads<decltype(type), decltype(quads)::value, decltype(stochastic)::value, decltype(squares)::value>), grid, dim3(1024), 0, stream,
-                     table, tiles, beta, inv_loss_scale, nesterov, (uint64_t)rounding_step, sums);
+        VIOLA_LAUNCH((momentum_squares_quads<decltype(type), decltype(quads)::value, decltype(stochastic)::value, decltype(squares)::value>), grid,
+                     dim3(NS_UNIT / tile_size * WAVE), 0, stream, table, tiles, beta, inv_loss_scale, nesterov, (uint64_t)rounding_step, sums);
     };
     auto with_squares = [&](auto type, auto quads, auto stochastic) {
         if (working_dtype == VIOLA_BF16) launch(type, quads, stochastic, std::integral_constant<int, 1>{});
