@@ -1,0 +1,42 @@
+"""What an optimizer step holds and allocates on the way."""
+
+import pytest
+import torch
+
+import viola_amd
+
+pytestmark = pytest.mark.gpu
+
+
+def _optimizer(shapes, **options):
+    torch.manual_seed(0)
+    params = [torch.nn.Parameter(torch.randn(*s, device="cuda") * .05) for s in shapes]
+    opt = viola_amd.optim.FP8Muon(params, lr=2e-3, **options)
+    for p in params:
+        p.grad = torch.randn_like(p) * 1e-2
+    opt.step()                                                                # state and pointer tables
+    torch.cuda.synchronize()
+    return params, opt
+
+
+def _peak(opt):
+    """Bytes that a step holds at once beyond what is there before it."""
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    opt.step()
+    torch.cuda.synchronize()
+    return torch.cuda.max_memory_allocated() - before
+
+
+@pytest.mark.parametrize("method", ["standard", "gram"])
+def test_a_step_holds_no_more_than_its_lanes_may(method):
+    """Buckets of one matrix, one at a time: what one of them needs, not four. Per element 2 bytes of updates, 2 of the result, 4 for the two sides of
+    the chain and 1 for each of its two squares of 512 x 512 (six in the Gram recurrence); 256 KB of sums and tables."""
+    shapes, elements = [(512, 1024)] * 4, 512 * 1024
+    params, opt = _optimizer(shapes, ns_method=method)
+    together = _peak(opt)
+    opt._LANES, opt._BATCH_ELEMENTS = 1, elements
+    opt.step()
+    one = _peak(opt)
+    assert one <= (10 if method == "standard" else 14) * elements + (1 << 18) and together > 2 * one

@@ -524,7 +524,8 @@ private:
     // 5185). The recurrence on the Gram matrix gains less there: its launches are several rounds of short tiles with a tail each, which lanes
     // fill (28 blocks of 384 805 us on lanes, 881 together; four of 512 373 and 331), so beyond TOGETHER_GRAM it keeps the lanes.
     static constexpr double TOGETHER_GRAM = 1e10;                // sum of m m (m + n) over the matrices
-    static constexpr int64_t TOGETHER_ELEMENTS = 1ll << 29;      // all arenas are held at once: 12 GB
+    // All arenas are held at once, 12 bytes per element at most (6.4 GB); and no more elements than the buckets on lanes may hold.
+    static constexpr int64_t TOGETHER_ELEMENTS = 1ll << 29;
     bool step_together(std::vector<std::vector<Item>>& ready) {
         if (ready.empty() || ready.size() > 8) return false;
         const Item& head = ready[0][0];
@@ -545,7 +546,7 @@ private:
                 work += (double)it.param.numel() * (double)std::min(shape.back(), shape[shape.size() - 2]) *
                         (1. + (double)std::min(shape.back(), shape[shape.size() - 2]) / (double)std::max(shape.back(), shape[shape.size() - 2]));
             }
-        if (elements > TOGETHER_ELEMENTS || (g.gram && work > TOGETHER_GRAM)) return false;
+        if (elements > TOGETHER_ELEMENTS || elements / std::max<int64_t>(lanes, 1) > batch_elements || (g.gram && work > TOGETHER_GRAM)) return false;
         std::vector<MomentumRow> momentum_rows;
         std::vector<WeightRow> weight_rows;
         std::vector<Tensor> inputs;

@@ -110,7 +110,8 @@ class FP8Muon(MatrixOptimizer):
             self.observer.momentum(param, grad, *before, q, scale, matrix, group, 1., quant)
         return matrix
 
-    # Streams the shape buckets of one step are spread over where they do not share their launches, and the most elements one bucket's chain takes
+    # Streams the shape buckets of one step are spread over where they do not share their launches, and the most elements one bucket's chain takes.
+    # Buckets share launches up to the product of the two: what a step holds at once follows these
     # (csrc/host_optim.cpp: step_together, step_buckets, batch_elements).
     _LANES, _BATCH_ELEMENTS = 4, 1 << 28
 
