@@ -41,3 +41,22 @@ def test_a_step_holds_no_more_than_its_lanes_may(method):
     opt.step()
     one = _peak(opt)
     assert one <= (10 if method == "standard" else 14) * elements + (2 << 20) and together > 2 * one
+
+
+def _allocated(opt):
+    """Bytes that a step asks the allocator for, freed on the way or not."""
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_stats()["allocated_bytes.all.allocated"]
+    opt.step()
+    torch.cuda.synchronize()
+    return torch.cuda.memory_stats()["allocated_bytes.all.allocated"] - before
+
+
+@pytest.mark.parametrize("options", [dict(tile_size=128), dict(tile_size=64), dict(granularity="block")])
+def test_what_cannot_go_together_is_refused_before_it_is_prepared(options):
+    """A gradient that is no row-major matrix is copied once: per element 4 bytes of it, 2 of updates, 2 of the result, 4 for the two sides of the
+    chain, 4 for its two squares."""
+    params, opt = _optimizer([(1024, 1024)], **options)
+    params[0].grad = (torch.randn(1024, 1024, device="cuda") * 1e-2).t()
+    opt.step()
+    assert _allocated(opt) <= 16 * (1 << 20) + (1 << 18)

@@ -531,7 +531,9 @@ private:
         const Item& head = ready[0][0];
         const Group& g = *head.group;
         const viola_stream_t stream = stream_of(head.param);
-        int64_t elements = 0;
+        // what momentum_together would refuse, before anything is allocated or copied for it
+        if (g.tile < 256) return false;
+        int64_t elements = 0, parameters = 0;
         double work = 0;
         for (const auto& bucket : ready)
             for (const Item& it : bucket) {
@@ -542,6 +544,9 @@ private:
                     h.weight_decay != g.weight_decay || h.match_rms != g.match_rms || shape.back() % 8 || shape[shape.size() - 2] % 8)
                     return false;
                 if (it.param.scalar_type() != at::kFloat || !aligned(it.param.const_data_ptr(), 16)) return false;
+                if (it.grad.scalar_type() != head.grad.scalar_type() || it.grad.numel() != it.param.numel() || !aligned(it.q.const_data_ptr(), 4) ||
+                    (it.grad.is_contiguous() && !aligned(it.grad.const_data_ptr(), 4 * it.grad.element_size())) || ++parameters > 65535)
+                    return false;
                 elements += it.param.numel();
                 work += (double)it.param.numel() * (double)std::min(shape.back(), shape[shape.size() - 2]) *
                         (1. + (double)std::min(shape.back(), shape[shape.size() - 2]) / (double)std::max(shape.back(), shape[shape.size() - 2]));
@@ -565,9 +570,8 @@ private:
         for (const Tensor& input : inputs) matrices += input.size(0) * input.size(1);
         const bool single = matrices == (int64_t)momentum_rows.size();
         const Arena sums = sums_of(matrices, head.param.device());
-        if (!momentum_together(tables_, {}, (int64_t)g.gram, momentum_rows, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step, stream,
-                               single ? sums.as<float>(0) : nullptr, g.gram ? VIOLA_F16 : VIOLA_BF16))
-            return false;
+        TORCH_INTERNAL_ASSERT(momentum_together(tables_, {}, (int64_t)g.gram, momentum_rows, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step,
+                                                stream, single ? sums.as<float>(0) : nullptr, g.gram ? VIOLA_F16 : VIOLA_BF16));
         std::vector<Chain> chains;
         for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram, false));
         // the last products of the chains go into the weights
