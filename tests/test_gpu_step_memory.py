@@ -52,6 +52,13 @@ def _allocated(opt):
     return torch.cuda.memory_stats()["allocated_bytes.all.allocated"] - before
 
 
+@pytest.mark.parametrize("shapes", [[(1024, 1024), (1024, 3072), (2048, 1024)], [(1024, 1024)]])
+def test_a_chain_that_ends_in_the_weights_has_no_result(shapes):
+    """Per element 2 bytes of updates and 4 for the two sides of the chain, and two squares of the smaller extent; sums, tables, rounding."""
+    params, opt = _optimizer(shapes)
+    assert _allocated(opt) <= sum(6 * p.numel() + 4 * min(p.shape) ** 2 for p in params) + (2 << 20)
+
+
 @pytest.mark.parametrize("options", [dict(tile_size=128), dict(tile_size=64), dict(granularity="block")])
 def test_what_cannot_go_together_is_refused_before_it_is_prepared(options):
     """A gradient that is no row-major matrix is copied once: per element 4 bytes of it, 2 of updates, 2 of the result, 4 for the two sides of the

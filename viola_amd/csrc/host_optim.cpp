@@ -25,16 +25,16 @@ constexpr float A_COEFFICIENT = 3.4445f;
 // The products that orthogonalize [..., rows, cols] in `steps` steps, one after the other; each reads and writes the arena, the last one
 // the result.
 struct Chain {
-    Tensor matrix, result;
+    Tensor matrix, result;                                       // (none where the last product goes into the weights)
     Arena arena;
     int dtype = 0;
     float* sums = nullptr;                                       // of squares, where the chain has room for its own
     viola_ns_matrices start{};                                   // the scaled matrix, in front of the products
     std::vector<viola_ns_product> products;
-    bool applied = false;                                        // the last product went into the weights
 };
 
-Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram, bool own_sums = true) {
+// own_sums: with room for its sums of squares. stored: with room for the result; else its last product has nowhere to go yet.
+Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram, bool own_sums = true, bool stored = true) {
     TORCH_CHECK(matrix_.is_cuda(), "viola_amd kernels run on the GPU only");
     TORCH_CHECK(matrix_.dim() >= 2 && steps >= 0, "Newton-Schulz takes matrices and a number of steps, got ", matrix_.dim(), " dimensions and ", steps, " steps");
     Chain c;
@@ -44,7 +44,7 @@ Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram, bool own_sums = 
     const bool tall = rows > cols;
     const at::ScalarType type = gram ? at::kHalf : at::kBFloat16;
     c.dtype = code_of(type);
-    c.result = at::empty(c.matrix.sizes(), c.matrix.options().dtype(type));
+    if (stored || steps == 0) c.result = at::empty(c.matrix.sizes(), c.matrix.options().dtype(type));
     if (c.matrix.numel() == 0) return c;
     const bool quintic = !gram || m == n;                        // the plain iteration; else the recurrence on the Gram matrix
     const int64_t wide = 2 * batch * m * n, square = 2 * batch * m * m;
@@ -55,7 +55,8 @@ Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram, bool own_sums = 
     for (int i = 0; i < squares; ++i) s_at[i] = c.arena.take(square);
     c.arena.make(c.matrix.device());
     if (own_sums) c.sums = c.arena.as<float>(sums_at);
-    void *x = steps ? c.arena.at(x_at[0]) : c.result.mutable_data_ptr(), *spare = c.arena.at(x_at[1]);   // no steps: the scaled matrix
+    void *const into = c.result.defined() ? c.result.mutable_data_ptr() : nullptr;
+    void *x = steps ? c.arena.at(x_at[0]) : into, *spare = c.arena.at(x_at[1]);   // no steps: the scaled matrix
     c.start = {c.matrix.const_data_ptr(), x, batch, rows, cols};
     if (steps == 0) return c;
     auto gemm = [&](const void* a, const void* b, bool transpose_b, const void* residual, int epilogue, int64_t out_cols, int64_t k, void* out,
@@ -66,7 +67,7 @@ Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram, bool own_sums = 
         void *r = c.arena.at(s_at[0]), *z = c.arena.at(s_at[1]);
         for (int64_t step = 0; step < steps; ++step) {
             const bool last = step == steps - 1;
-            void* out = last ? c.result.mutable_data_ptr() : spare;
+            void* out = last ? into : spare;
             gemm(x, x, true, nullptr, 0, m, n, r, 0, nullptr, false);
             gemm(r, r, true, r, 1, m, m, z, 0, nullptr, false);  // r = x x^T is symmetric bit for bit: r r = r r^T
             gemm(z, x, false, x, 2, n, m, out, 0, nullptr, tall && last);
@@ -97,12 +98,19 @@ Chain chain_of(const Tensor& matrix_, int64_t steps, bool gram, bool own_sums = 
                 std::swap(r, r_next);
             }
         }
-        void* out = last ? c.result.mutable_data_ptr() : spare;
+        void* out = last ? into : spare;
         gemm(q, x, false, nullptr, 0, n, m, out, 0, nullptr, tall && last);
         spare = x;
         x = out;
     }
     return c;
+}
+
+// A last product that could not go into the weights is stored after all.
+void store_result(Chain& c) {
+    c.result = at::empty(c.matrix.sizes(), c.matrix.options().dtype(c.dtype == VIOLA_F16 ? at::kHalf : at::kBFloat16));
+    c.products.back().out = c.result.mutable_data_ptr();
+    c.products.back().weights = nullptr;
 }
 
 void prepare(const Chain& c, float* sums, viola_stream_t stream) {
@@ -129,9 +137,9 @@ Tensor newton_schulz(const Tensor& matrix, int64_t steps, bool gram) {
     return c.result;
 }
 
-// Chains of one type, step by step together: the products of a step are one launch where the tiled kernel takes them all. `sums` holds the
+// Chains of one type that the tiled kernel takes, at most eight, step by step together: the products of a step are one launch. `sums` holds the
 // matrices' sums of squares already, or (have_sums 0) has room for them.
-void run_together(std::vector<Chain>& chains, const Arena& sums, int have_sums, viola_stream_t stream) {
+void run_together(const std::vector<Chain>& chains, const Arena& sums, int have_sums, viola_stream_t stream) {
     const int dtype = chains[0].dtype;
     std::vector<viola_ns_matrices> starts;
     size_t steps = 0;
@@ -152,13 +160,8 @@ void run_together(std::vector<Chain>& chains, const Arena& sums, int have_sums, 
                 step.push_back(c.products[i]);
                 into_weights = into_weights || step.back().weights;
             }
-        status = step.size() > 1 || into_weights ? VIOLA_TRY(viola_ns_gemm_many, step.data(), (int)step.size(), dtype, stream) : VIOLA_EUNSUPPORTED;
-        if (status == VIOLA_EUNSUPPORTED) {
-            for (const viola_ns_product& p : step) multiply(p, dtype, stream);        // (results: the weights are the caller's then)
-            continue;
-        }
-        check("viola_ns_gemm_many", status);
-        for (Chain& c : chains) c.applied = c.applied || (i + 1 == c.products.size() && c.products[i].weights);
+        if (step.size() > 1 || into_weights) VIOLA_CALL(viola_ns_gemm_many, step.data(), (int)step.size(), dtype, stream);
+        else multiply(step[0], dtype, stream);
     }
 }
 
@@ -524,15 +527,15 @@ private:
     // 5185). The recurrence on the Gram matrix gains less there: its launches are several rounds of short tiles with a tail each, which lanes
     // fill (28 blocks of 384 805 us on lanes, 881 together; four of 512 373 and 331), so beyond TOGETHER_GRAM it keeps the lanes.
     static constexpr double TOGETHER_GRAM = 1e10;                // sum of m m (m + n) over the matrices
-    // All arenas are held at once, 12 bytes per element at most (6.4 GB); and no more elements than the buckets on lanes may hold.
+    // All arenas are held at once, 10 bytes per element at most (5.4 GB); and no more elements than the buckets on lanes may hold.
     static constexpr int64_t TOGETHER_ELEMENTS = 1ll << 29;
     bool step_together(std::vector<std::vector<Item>>& ready) {
         if (ready.empty() || ready.size() > 8) return false;
         const Item& head = ready[0][0];
         const Group& g = *head.group;
         const viola_stream_t stream = stream_of(head.param);
-        // what momentum_together would refuse, before anything is allocated or copied for it
-        if (g.tile < 256) return false;
+        // what momentum_together would refuse, before anything is allocated or copied for it; and a chain of no product leaves none for the weights
+        if (g.tile < 256 || g.ns_steps < 1) return false;
         int64_t elements = 0, parameters = 0;
         double work = 0;
         for (const auto& bucket : ready)
@@ -553,7 +556,6 @@ private:
             }
         if (elements > TOGETHER_ELEMENTS || elements / std::max<int64_t>(lanes, 1) > batch_elements || (g.gram && work > TOGETHER_GRAM)) return false;
         std::vector<MomentumRow> momentum_rows;
-        std::vector<WeightRow> weight_rows;
         std::vector<Tensor> inputs;
         for (const auto& bucket : ready) {
             const std::vector<int64_t> shape = matrix_shape(bucket[0].param, *bucket[0].group);
@@ -573,7 +575,7 @@ private:
         TORCH_INTERNAL_ASSERT(momentum_together(tables_, {}, (int64_t)g.gram, momentum_rows, g.tile, (float)g.momentum, 1.0f, g.nesterov, g.rounding, head.step,
                                                 stream, single ? sums.as<float>(0) : nullptr, g.gram ? VIOLA_F16 : VIOLA_BF16));
         std::vector<Chain> chains;
-        for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram, false));
+        for (const Tensor& input : inputs) chains.push_back(chain_of(input, g.ns_steps, g.gram, false, false));
         // the last products of the chains go into the weights
         std::vector<int64_t> addresses;
         for (size_t i = 0; i < ready.size(); ++i)
@@ -582,21 +584,10 @@ private:
                     addresses.push_back((int64_t)it.param.const_data_ptr() + plane * chains[i].matrix.size(-2) * chains[i].matrix.size(-1) * 4);
         const int64_t* at = tables_.get(ADDRESS_TABLE, {}, (int64_t)addresses.size(), (int64_t)g.gram, std::move(addresses), head.param.device(), stream);
         for (Chain& c : chains) {
-            if (!c.products.empty()) into_weights(c.products.back(), at, g, c.matrix.size(-2), c.matrix.size(-1));
+            into_weights(c.products.back(), at, g, c.matrix.size(-2), c.matrix.size(-1));
             at += c.start.batch;
         }
         run_together(chains, sums, single, stream);
-        for (size_t i = 0; i < ready.size(); ++i) {
-            if (chains[i].applied) continue;
-            const int64_t count = ready[i][0].param.numel(), rows = chains[i].matrix.size(-2), cols = chains[i].matrix.size(-1);
-            const char* from = static_cast<const char*>(chains[i].result.const_data_ptr());
-            for (const Item& it : ready[i]) {
-                weight_rows.push_back({it.param, from, count, (float)update_scale(g, rows, cols)});
-                from += 2 * count;
-            }
-        }
-        if (!weight_rows.empty())
-            TORCH_INTERNAL_ASSERT(weights_together(tables_, {}, (int64_t)g.gram, weight_rows, chains[0].result.scalar_type(), (float)g.lr, (float)g.weight_decay, stream));
         return true;
     }
 
@@ -649,38 +640,39 @@ private:
             }
         }
 
-        Chain chain = chain_of(updates_in, g.ns_steps, g.gram);
+        // ---- the chain, its last product into the weights where they allow it
+        together = true;
+        bool in_place = rows % 8 == 0 && cols % 8 == 0 && g.ns_steps > 0;
+        for (const Item& it : bucket) {
+            const Group& h = *it.group;
+            together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms;
+            in_place = in_place && it.param.scalar_type() == at::kFloat && aligned(it.param.const_data_ptr(), 16);
+        }
+        // and where they are enough for several rounds of tiles (below that other lanes hide the weights' launch better than a tile hides their
+        // loads: two blocks of 768, recurrence, 400 us, 420 so)
+        in_place = in_place && together && size * count >= INTO_WEIGHTS;
+        Chain chain = chain_of(updates_in, g.ns_steps, g.gram, true, !in_place);
         prepare(chain, chain.sums, stream);
         for (size_t i = 0; i + 1 < chain.products.size(); ++i) multiply(chain.products[i], chain.dtype, stream);
+        if (in_place) {
+            std::vector<int64_t> addresses;
+            for (const Item& it : bucket)
+                for (int64_t plane = 0; plane < chain.matrix.size(1); ++plane) addresses.push_back((int64_t)it.param.const_data_ptr() + plane * rows * cols * 4);
+            viola_ns_product& last = chain.products.back();
+            into_weights(last, tables_.get(ADDRESS_TABLE, shape, (int64_t)addresses.size(), ordinal, std::move(addresses), device, stream), g, rows, cols);
+            const int status = VIOLA_TRY(viola_ns_gemm_many, &last, 1, chain.dtype, stream);
+            if (status == 0) return;
+            if (status != VIOLA_EUNSUPPORTED) check("viola_ns_gemm_many", status);
+            store_result(chain);                                 // a matrix of 2 GB and more
+        }
+        if (!chain.products.empty()) multiply(chain.products.back(), chain.dtype, stream);
+
+        // ---- weights
         const Tensor updates = chain.result;
         const char* from = static_cast<const char*>(updates.const_data_ptr());
         const int update_code = code_of(updates.scalar_type());
-
-        // ---- weights
-        together = true;
-        bool in_place = true;
         std::vector<WeightRow> weight_rows;
-        for (size_t i = 0; i < bucket.size(); ++i) {
-            const Group& h = *bucket[i].group;
-            together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms;
-            weight_rows.push_back({bucket[i].param, from + 2 * count * i, count, (float)update_scale(g, rows, cols)});
-            in_place = in_place && bucket[i].param.scalar_type() == at::kFloat && aligned(bucket[i].param.const_data_ptr(), 16);
-        }
-        if (!chain.products.empty()) {
-            // the last product: into the weights where they allow it, and are enough for several rounds of tiles (below that other lanes
-            // hide the weights' launch better than a tile hides their loads: two blocks of 768, recurrence, 400 us, 420 so)
-            viola_ns_product& last = chain.products.back();
-            if (together && in_place && rows * cols % 4 == 0 && size * count >= INTO_WEIGHTS) {
-                std::vector<int64_t> addresses;
-                for (const Item& it : bucket)
-                    for (int64_t plane = 0; plane < updates.size(1); ++plane) addresses.push_back((int64_t)it.param.const_data_ptr() + plane * rows * cols * 4);
-                into_weights(last, tables_.get(ADDRESS_TABLE, shape, (int64_t)addresses.size(), ordinal, std::move(addresses), device, stream), g, rows, cols);
-                const int status = VIOLA_TRY(viola_ns_gemm_many, &last, 1, chain.dtype, stream);
-                if (status == 0) return;
-                if (status != VIOLA_EUNSUPPORTED) check("viola_ns_gemm_many", status);
-            }
-            multiply(last, chain.dtype, stream);
-        }
+        for (size_t i = 0; i < bucket.size(); ++i) weight_rows.push_back({bucket[i].param, from + 2 * count * i, count, (float)update_scale(g, rows, cols)});
         if (together && weights_together(tables_, shape, ordinal, weight_rows, updates.scalar_type(), (float)g.lr, (float)g.weight_decay, stream)) return;
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Item& it = bucket[i];
