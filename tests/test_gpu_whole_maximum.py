@@ -9,14 +9,14 @@ import oracle.tensor as ot
 pytestmark = pytest.mark.gpu
 
 
-def _encode(x, limit, index=0, delayed=0):
+def _encode(x, limit, index=0, delayed=0, work=None):
     from viola_amd import _lib
     rows, cols = x.shape
     pitch_t = -(-rows // 128) * 128
     history, scale = torch.zeros(4, device="cuda"), torch.empty(1, device="cuda")
     q, qt = torch.empty(rows, cols, dtype=torch.uint8, device="cuda"), torch.empty(cols, pitch_t, dtype=torch.uint8, device="cuda")
     code = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}[x.dtype]
-    work = torch.full((1024,), float("nan"), device="cuda")
+    work = torch.full((1024,), float("nan"), device="cuda") if work is None else work
     _lib.call("viola_tensor_encode", _lib.ptr(x), code, rows, cols, _lib.ptr(work), 1024, _lib.ptr(history), 4, index, delayed, limit, _lib.ptr(scale), _lib.ptr(q),
               cols, _lib.ptr(qt), pitch_t, _lib.E4M3, None, _lib.F32)
     return history.cpu(), scale.cpu(), q.cpu(), qt.cpu()
@@ -58,3 +58,14 @@ def test_nan_is_no_maximum(dtype, place):
     x.view(-1)[place] = -float("inf")
     history, scale, _, _ = _encode(x.cuda(), 448.0)
     assert history[0] == float("inf") and scale[0] == float("inf")
+
+
+@pytest.mark.parametrize("dtype,kilobytes,whole", [(torch.bfloat16, 128, True), (torch.float32, 128, True), (torch.bfloat16, 132, False), (torch.float16, 256, False),
+                                                    (torch.float32, 132, False)])
+def test_beyond_128_kb_the_maximum_is_a_pass_of_its_own(dtype, kilobytes, whole):
+    """There the blocks' serial walks over the whole tensor take longer than the pass that they save, most of all over an x that no cache holds. Only the
+    pass leaves maxima in the workspace."""
+    x = torch.randn((kilobytes << 10) // torch.finfo(dtype).bits * 8).to(dtype).view(-1, 256)
+    work = torch.full((1024,), float("nan"), device="cuda")
+    _check(x, *_encode(x.cuda(), 448.0, work=work))
+    assert torch.isnan(work).all().item() == whole

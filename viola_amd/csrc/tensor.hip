@@ -558,10 +558,12 @@ extern "C" int viola_tensor_encode_beside(const void* x, int x_dtype, int64_t ro
     hipStream_t stream = viola_enter(stream_);
     VIOLA_CHECK_ARG(viola_is_float(x_dtype) && viola_is_fp8(q_dtype) && rows > 0 && cols > 0 && x && workspace && history && history_len > 0);
     VIOLA_CHECK_ARG(index >= 0 && limit > 0.0f && scale && (!column_sum || viola_is_float(sum_dtype)));
-    // Small tensors, a tile or less to a CU: every block of the quantizer takes the maximum of the whole by itself, 0.8 us per 64 KB, in place of a
-    // launch of 3 us on the host and 3 on the device. Kernels (us): 8 KB 6.3 -> 4.7, 64 KB 6.6 -> 4.7, 128 KB 7.1 -> 5.6, 256 KB 7.0 -> 7.2 and
-    // a launch's gap less, 384 KB 7.2 -> 9.3. Forward and backward of 256 x 512 -> 2048 78.9 -> 73.6.
-    constexpr int64_t FEW = 512, WHOLE_BYTES = 256 << 10, WHOLE_TILES = 256;
+    // Small tensors, a tile or less to a CU: every block of the quantizer takes the maximum of the whole by itself, in turns of 64 KB, in place of a
+    // launch of 3 us on the host and 1.5 on the device. Up to where that is the shorter also for an x that no cache holds, which each XCD then fetches
+    // for itself. Two launches and one, BF16 with both layouts, x in the caches and (not), us: 8 KB 5.4 (6.7), 4.0 (4.6); 64 KB 5.6 (6.5), 4.0 (4.9); 128 KB
+    // 5.6 (6.7), 4.6 (6.1); 160 KB 5.6 (6.8), 5.4 (7.2); 256 KB 5.7 (6.7), 6.1 (8.5). FP32: 128 KB 5.6 (7.0), 4.5 (6.2); 160 KB 5.6 (7.2), 5.1 (7.2);
+    // 256 KB 5.8 (7.2), 5.7 (8.8).
+    constexpr int64_t FEW = 512, WHOLE_BYTES = 128 << 10, WHOLE_TILES = 256;
     TensorQuantizeSide side = {};
     if (codes) {
         VIOLA_CHECK_ARG(codes_t && code_rows > 0 && code_cols > 0 && code_pitch >= code_rows);
