@@ -46,6 +46,26 @@ def test_sums_beside_the_momentum_are_those_of_a_pass(shapes, tile, working):
         assert torch.equal(sums[i], _prepared(update, working)[0]), shapes[i]
 
 
+# in more than 512 blocks each takes half as many wavefronts, with two tiles each: the last of them has one, or none
+@pytest.mark.parametrize("grads", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("working", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tiles", [(1, 2, 15, 16, 17, 301, 4098, 4099), (4096, 4096), (3,) * 171, (4096,)])
+def test_stochastic_momentum_and_sums_are_those_of_a_tensor_alone(tiles, working, grads):
+    torch.manual_seed(len(tiles))
+    table, pairs = [], []
+    for i, n in enumerate(tiles):
+        g, q, s = (torch.randn(256 * n, device="cuda") * 1e-2).to(grads), torch.randint(0, 120, (256 * n,), device="cuda", dtype=torch.uint8), torch.rand(n, device="cuda") * 1e-3
+        want, got = [(q.clone(), s.clone(), torch.zeros(1, 32 * n, 8, device="cuda", dtype=torch.bfloat16)) for _ in range(2)]
+        _lib.call("viola_momentum_update", _lib.ptr(g), _lib.code(grads), *map(_lib.ptr, (*want[:2], *want)), 256 * n, .95, 1.0, 1, 0, 256, 1, 1, 1, 1, 1, 1, 3, 77 + i)
+        table.append([t.data_ptr() for t in (g, *got[:2], *got)] + [77 + i, n])
+        pairs.append((want, got, g))
+    rows, sums = torch.tensor(table, device="cuda"), torch.full((len(tiles), 256), float("nan"), device="cuda")
+    _lib.call("viola_momentum_update_squares", rows.data_ptr(), len(tiles), max(tiles), _lib.code(grads), 256, .95, 1.0, 1, 1, 3, _lib.code(working), sums.data_ptr())
+    for i, (want, got, _) in enumerate(pairs):
+        assert all(torch.equal(a, b) for a, b in zip(want, got)), tiles[i]
+        assert torch.equal(sums[i], _prepared(got[2], working)[0]), tiles[i]
+
+
 @pytest.mark.parametrize("working", [torch.bfloat16, torch.float16])
 def test_sums_of_several_shapes_are_those_of_each_matrix_alone(working):
     """Extents that end within a unit, a chunk and a wavefront; of several matrices one holds infinities and NaN."""

@@ -203,21 +203,25 @@ __global__ __launch_bounds__(256) void momentum_table_quads(const int64_t* __res
 
 // The same with what Newton-Schulz starts from, the sums of squares of the updates in sums[tensor][256], so that the pass over the updates that
 // would form them (viola_ns_prepare's first), 2 bytes per element, is not needed. In that pass's order, whatever the tile (ns_sums.hpp): a block
-// takes a unit of a tensor at a time, each wavefront a tile of it. 28 blocks of width 1152 625 + 181 -> 660 us. Blocks of 16 tiles, whose order
+// takes a unit of a tensor at a time, each wavefront KEPT chunks of it. 28 blocks of width 1152 625 + 181 -> 660 us. Blocks of 16 tiles, whose order
 // depended on the tile, and now, us: 56 x 1152 x 4608 in tiles of 256 427, 430, of 1024 459, 458; one of 1024 x 1024 4.1, 4.2 and 7.8, 5.6;
 // 4096 x 4096 23.3, 23.4 and 22.6, 27.9 (blocks of four wavefronts, and no other matrix to fill the chip).
-template <typename TG, int EPL, bool STOCHASTIC, int SQUARES>
-__global__ __launch_bounds__(4096 / EPL) void momentum_squares_quads(const int64_t* __restrict__ table, int64_t blocks, float beta,
-                                                                     float inv_loss_scale, int nesterov, uint64_t step, float* __restrict__ sums) {
-    constexpr int TILES = NS_UNIT / (EPL * WAVE);
+template <typename TG, int EPL, bool STOCHASTIC, int SQUARES, int KEPT>
+__global__ __launch_bounds__(1024 / KEPT) void momentum_squares_quads(const int64_t* __restrict__ table, int64_t blocks, float beta,
+                                                                      float inv_loss_scale, int nesterov, uint64_t step, float* __restrict__ sums) {
+    constexpr int TILES = NS_UNIT / (EPL * WAVE), QUADS = EPL / 4, EACH = KEPT / QUADS;
+    static_assert(KEPT % QUADS == 0);
     const int64_t* row = table + (int64_t)blockIdx.y * 8;
     const int64_t tiles = row[7] ? row[7] : blocks;
-    float squares[EPL / 4] = {};
-    for (int64_t b = (int64_t)blockIdx.x * TILES + threadIdx.x / WAVE; b < tiles; b += (int64_t)gridDim.x * TILES)
-        momentum_quads_tile<TG, EPL, STOCHASTIC, SQUARES>(reinterpret_cast<const TG*>(row[0]), reinterpret_cast<const uint8_t*>(row[1]),
-                                                          reinterpret_cast<const float*>(row[2]), reinterpret_cast<uint8_t*>(row[3]),
-                                                          reinterpret_cast<float*>(row[4]), reinterpret_cast<uint16_t*>(row[5]), b, beta,
-                                                          inv_loss_scale, nesterov, step, (uint64_t)row[6], squares);
+    float squares[KEPT] = {};
+    for (int64_t first = (int64_t)blockIdx.x * TILES + threadIdx.x / WAVE * EACH; first < tiles; first += (int64_t)gridDim.x * TILES)
+#pragma unroll
+        for (int each = 0; each < EACH; ++each)
+            if (first + each < tiles)
+                momentum_quads_tile<TG, EPL, STOCHASTIC, SQUARES>(reinterpret_cast<const TG*>(row[0]), reinterpret_cast<const uint8_t*>(row[1]),
+                                                                  reinterpret_cast<const float*>(row[2]), reinterpret_cast<uint8_t*>(row[3]),
+                                                                  reinterpret_cast<float*>(row[4]), reinterpret_cast<uint16_t*>(row[5]), first + each, beta,
+                                                                  inv_loss_scale, nesterov, step, (uint64_t)row[6], squares + each * QUADS);
     ns_store_slot(squares, sums + (int64_t)blockIdx.y * NS_PARTS);
 }
 
@@ -513,8 +517,18 @@ extern "C" int viola_momentum_update_squares(const int64_t* table, int64_t tenso
     VIOLA_CHECK_ARG(table && sums);
     const dim3 grid = ns_sum_blocks(tiles * tile_size, tensors);
     auto launch = [&](auto type, auto quads, auto stochastic, auto squares) {
-        VIOLA_LAUNCH((momentum_squares_quads<decltype(type), decltype(quads)::value, decltype(stochastic)::value, decltype(squares)::value>), grid,
-                     dim3(NS_UNIT / tile_size * WAVE), 0, stream, table, tiles, beta, inv_loss_scale, nesterov, (uint64_t)rounding_step, sums);
+        constexpr int QUADS = decltype(quads)::value / 4;
+        auto go = [&](auto kept) {
+            VIOLA_LAUNCH((momentum_squares_quads<decltype(type), decltype(quads)::value, decltype(stochastic)::value, decltype(squares)::value, decltype(kept)::value>), grid,
+                         dim3(1024 / decltype(kept)::value), 0, stream, table, tiles, beta, inv_loss_scale, nesterov, (uint64_t)rounding_step, sums);
+        };
+        // Random bits are the most of the work, and a block of 1024 threads, whose place is free only when its last wavefront is done, leaves too few of them
+        // at it: with more than the two such blocks that a CU holds, halves of them. us, tiles of 256, 1024 threads and 512 (the update without sums): 76 x
+        // 1108992 390, 284 (249); 92 x 248832 100, 74 (72); 12 x 196608 15.2, 13.7 (10.0); up to 512 blocks 1 x 16777216 62, 73 (56), 4 x 110592 5.9, 6.8.
+        // Rounded to nearest, 1024: 112 x 3981312 648, 668.
+        if constexpr (QUADS == 1 && decltype(stochastic)::value)
+            if ((int64_t)grid.x * grid.y > 512) return go(std::integral_constant<int, 2>{});
+        go(std::integral_constant<int, QUADS>{});
     };
     auto with_squares = [&](auto type, auto quads, auto stochastic) {
         if (working_dtype == VIOLA_BF16) launch(type, quads, stochastic, std::integral_constant<int, 1>{});
