@@ -429,6 +429,8 @@ typedef struct {
     float keep, rate;
 } viola_ns_product;
 int viola_ns_gemm_many(const viola_ns_product* products, int count, int dtype, viola_stream_t stream);
+/* The tile that viola_ns_gemm_many runs these on, numbered as in viola_ns_plan's plan[3] (0: it refuses them). Host arithmetic only. */
+int viola_ns_plan_many(const viola_ns_product* products, int count, int* tile);
 
 /* viola/optim/_orthogonalize_kernels.py:114-197 `plan` (the per-shape schedule the reference picks by timing its
  * candidates: bm, bn): which tile shape viola_ns_gemm runs a product on. Host arithmetic only, nothing is launched and

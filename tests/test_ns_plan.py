@@ -3,6 +3,7 @@ viola/optim/_orthogonalize_kernels.py:114 `plan`), so it can be replayed here wi
 parity tests use, and over every product of the optimizer benchmark's DiT-XL step. A tile shape of the kernel, or a
 product of that step, that no GPU test reaches fails this file."""
 
+import ctypes
 import itertools
 
 import pytest
@@ -87,3 +88,28 @@ def test_plan_of_known_shapes():
     assert not plan(28, 1152, 1152, 3456, transpose_b=True, same_operand=True, transpose_out=True)["mirrored"]
     assert plan(2, 33, 47, 65)["kernel"] == "generic"                        # k, n not multiples of 8
     assert plan(0, 64, 64, 64)["kernel"] == "generic"
+
+
+def together(blocks, width, symmetric):
+    """The tile of a launch that `blocks` transformer blocks' chains share: their Gram products or the products with their squares."""
+    from test_gpu_products_together import Product
+    from viola_amd import _lib
+    rows = []
+    for columns, each in ((width, 1), (3 * width, 1), (4 * width, 2)):
+        a, b, n, k = (4096, 4096, width, columns) if symmetric else (4096, 8192, columns, width)   # stand-ins: aligned, equal or not
+        rows.append(Product(a, b, None, 12288, None, blocks * each, width, n, k, 0.0, int(symmetric), 0, 0))
+    tile = ctypes.c_int(-1)
+    assert _lib.library().viola_ns_plan_many((Product * len(rows))(*rows), len(rows), ctypes.byref(tile)) == 0
+    return ("generic", *KERNELS)[tile.value]
+
+
+@pytest.mark.parametrize("blocks,width,tile", [(28, 1152, "384x192"), (10, 704, "384x192"), (10, 608, "128x128"), (12, 608, "128x128"), (10, 640, "128x128"),
+                                               (14, 608, "192x192"), (28, 608, "192x192"), (28, 640, "192x192"), (12, 1024, "192x192"), (6, 800, "128x128"), (16, 480, "128x128"),
+                                               (5, 608, "128x128"), (1, 192, "64x64")])
+def test_products_together_take_a_wide_tile_where_they_pay_for_its_padding(blocks, width, tile):
+    assert together(blocks, width, False) == tile
+
+
+@pytest.mark.parametrize("blocks,width,tile", [(28, 1152, "192x192"), (28, 768, "192x192"), (8, 768, "128x128"), (28, 640, "128x128"), (4, 384, "64x64")])
+def test_gram_products_together(blocks, width, tile):
+    assert together(blocks, width, True) == tile

@@ -85,7 +85,7 @@ _SIGNATURES = {
     "viola_selftest_fp8": [_p, _p],
     "viola_selftest_philox": [_p, _p, _l, _p],
 }
-EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan", "viola_tensor_encode_slices", "viola_group_gemm_parts",
+EXPORTS = tuple(_SIGNATURES) + ("viola_abi_version", "viola_error_string", "viola_ns_plan", "viola_ns_plan_many", "viola_tensor_encode_slices", "viola_group_gemm_parts",
                                 "viola_group_gemm_form", "viola_scaled_gemm_form")
 
 _lib = None
@@ -109,6 +109,7 @@ def library():
         lib.viola_group_gemm_form.argtypes, lib.viola_group_gemm_form.restype = [_l, _l, _l, _i, _i, _i], ctypes.c_int
         lib.viola_scaled_gemm_form.argtypes, lib.viola_scaled_gemm_form.restype = [_l, _l, _l], ctypes.c_int
         lib.viola_ns_plan.argtypes, lib.viola_ns_plan.restype = [_l, _l, _l, _l, _i, _i, _i, ctypes.POINTER(ctypes.c_int)], ctypes.c_int
+        lib.viola_ns_plan_many.argtypes, lib.viola_ns_plan_many.restype = [_p, _i, ctypes.POINTER(ctypes.c_int)], ctypes.c_int
         assert lib.viola_abi_version() == 1
         _lib = lib
     return _lib

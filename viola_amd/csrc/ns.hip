@@ -676,11 +676,10 @@ extern "C" int viola_ns_gemm(const void* a, const void* bmat, const void* residu
 #undef VIOLA_NS
 }
 
-extern "C" int viola_ns_gemm_many(const viola_ns_product* products, int count, int dtype, viola_stream_t stream_) {
-    hipStream_t stream = viola_enter(stream_);
-    VIOLA_CHECK_ARG((dtype == VIOLA_BF16 || dtype == VIOLA_F16) && count >= 0 && (count == 0 || products));
+// The products that have a result, as the tiled kernel's arguments.
+static int gather_products(const viola_ns_product* products, int count, NsMany& many) {
+    VIOLA_CHECK_ARG(count >= 0 && (count == 0 || products));
     if (count > NS_MANY) return VIOLA_EUNSUPPORTED;
-    NsMany many{};
     for (int i = 0; i < count; ++i) {
         const viola_ns_product& p = products[i];
         VIOLA_CHECK_ARG(p.epilogue >= 0 && p.epilogue <= 2 && p.batch >= 0 && p.m >= 0 && p.n >= 0 && p.k >= 0);
@@ -692,6 +691,24 @@ extern "C" int viola_ns_gemm_many(const viola_ns_product* products, int count, i
                                       ns_is_mirrored(p.a, p.b, p.transpose_b, p.m, p.n, p.transpose_out), 0, 0, 0, 0, !p.transpose_b, p.epilogue,
                                       p.weights, p.keep, p.rate};
     }
+    return 0;
+}
+
+extern "C" int viola_ns_plan_many(const viola_ns_product* products, int count, int* tile) {
+    VIOLA_CHECK_ARG(tile);
+    NsMany many{};
+    const int status = gather_products(products, count, many);
+    if (status) return status;
+    *tile = many.count && ns_many_takes(many) ? (int)ns_choose_tile_many(many) : (int)NS_TILE_GENERIC;
+    return 0;
+}
+
+extern "C" int viola_ns_gemm_many(const viola_ns_product* products, int count, int dtype, viola_stream_t stream_) {
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG(dtype == VIOLA_BF16 || dtype == VIOLA_F16);
+    NsMany many{};
+    const int status = gather_products(products, count, many);
+    if (status) return status;
     if (many.count == 0) return 0;
     // the longest k first: their tiles are not what the launch waits for at its end
     std::stable_sort(many.product, many.product + many.count, [](const NsArgs& a, const NsArgs& b) { return a.k > b.k; });

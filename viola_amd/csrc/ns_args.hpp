@@ -35,6 +35,8 @@ struct NsMany {
 enum NsTile { NS_TILE_GENERIC = 0, NS_TILE_64x64 = 1, NS_TILE_128x64 = 2, NS_TILE_128x128 = 3, NS_TILE_192x192 = 4, NS_TILE_384x192 = 5 };
 NsTile ns_choose_tile(int64_t batch, int64_t m, int64_t n, bool symmetric);
 bool ns_fast_takes(const NsArgs& args);
+NsTile ns_choose_tile_many(const NsMany& many);
+bool ns_many_takes(const NsMany& many);
 
 // Launches the tiled kernel when the shape qualifies (16-byte aligned rows, k and n multiples of 8,
 // one matrix below 2 GiB); returns false without launching otherwise. `many`: unless every product qualifies.

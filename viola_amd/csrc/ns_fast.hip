@@ -616,7 +616,11 @@ bool launch_ns_gemm_fast(const NsArgs& p, bool is_bf16, bool b_kn, int epilogue,
 
 // The tile shape for a launch of several products: one for all, by the same criteria, over the blocks of all, and a little more
 // padding where the launch is several rounds of wide tiles: 28 blocks of width 768 whose Gram products, 7 % larger on them, run on
-// 192 x 192 take 4.63 ms a step, on 128 x 128 4.77 (five: 1031 and 1009 us).
+// 192 x 192 take 4.63 ms a step, on 128 x 128 4.77 (five: 1031 and 1009 us). Where 384 x 192 pads no more than 192 x 192, but both more than that, the
+// many tiles of a large set still gain by the smaller traffic, 8192 of them for twice the area. The third launch of a step, us on 384 x 192, 192 x 192
+// and 128 x 128: width 608 (24 % more) 1600 tiles of 192 x 192 97, 82, 72, 1920 103, 99, 93, 2240 126, 108, 122, 4480 248, 234, 266; width 640 (26 %) 1680
+// 97, 89, 79, 2352 134, 133, 142; width 1024 (16 %) 1584 133, 121, 124, 4752 371, 377, 434; width 992 (15 %) 1536 115, 107, 120, 10752 843, 817, 967. Steps
+// of 10, 14 and 28 blocks of width 608, on 384 x 192 alone before, 1130 -> 976, 1509 -> 1407, 2831 -> 2754 us; four of 992 1488 -> 1327.
 NsTile ns_choose_tile_many(const NsMany& many) {
     constexpr int SHAPES = 4;
     static const int rows_of[SHAPES] = {384, 192, 128, 64}, cols_of[SHAPES] = {192, 192, 128, 64};
@@ -632,8 +636,10 @@ NsTile ns_choose_tile_many(const NsMany& many) {
             area[i] += tiles * rows_of[i] * cols_of[i] * p.k;
         }
     }
-    if (!symmetric && area[0] <= area[1] && blocks[0] >= 3 * 256) return NS_TILE_384x192;
-    if (area[1] * 20 <= area[2] * 21 && blocks[1] >= NS_FILL) return NS_TILE_192x192;
+    const bool wide = area[1] * 20 <= area[2] * 21, big = !symmetric && area[0] <= area[1] && blocks[0] >= 3 * 256;
+    if (big && wide) return NS_TILE_384x192;
+    if (big) return (double)(area[1] - area[2]) * 8192 <= (double)area[2] * (double)blocks[1] ? NS_TILE_192x192 : NS_TILE_128x128;
+    if (wide && blocks[1] >= NS_FILL) return NS_TILE_192x192;
     if (area[1] * 25 <= area[2] * 27 && blocks[1] >= 1024) return NS_TILE_192x192;
     if (blocks[2] >= NS_FILL) return NS_TILE_128x128;
     // a product alone, as in a launch of its own
@@ -662,14 +668,18 @@ static void launch_shape_many(const NsMany& many, hipStream_t stream) {
     }
 }
 
-bool launch_ns_gemm_many(const NsMany& many, bool is_bf16, hipStream_t stream) {
+bool ns_many_takes(const NsMany& many) {
     int64_t blocks = 0;
     for (int at = 0; at < many.count; ++at) {
         const NsArgs& p = many.product[at];
         if (!ns_fast_takes(p)) return false;
         blocks += p.batch * ((p.m + 63) / 64) * ((p.n + 63) / 64) + 8;
     }
-    if (blocks >= (1ll << 31)) return false;
+    return blocks < (1ll << 31);
+}
+
+bool launch_ns_gemm_many(const NsMany& many, bool is_bf16, hipStream_t stream) {
+    if (!ns_many_takes(many)) return false;
     if (is_bf16) launch_shape_many<true>(many, stream);
     else launch_shape_many<false>(many, stream);
     return true;
