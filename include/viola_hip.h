@@ -372,11 +372,6 @@ int viola_momentum_update_squares(const int64_t* table, int64_t tensors, int64_t
 int viola_weight_update_table(const int64_t* table, int64_t tensors, int64_t count, int grad_dtype, float lr, float decay,
                               float update_scale, viola_stream_t stream);
 
-/* viola_weight_update_table for tensors of different sizes and update scales. table: rows of four int64: {weight, update, elements (a
- * multiple of 4), the update scale's FP32 bits}; max_count: the largest number of elements. */
-int viola_weight_update_rows(const int64_t* table, int64_t tensors, int64_t max_count, int grad_dtype, float lr, float decay,
-                             viola_stream_t stream);
-
 /* The same update for many tensors that share dtypes, hyper-parameters and step count, in one launch (the reference
  * calls adam_update once per parameter, viola/optim/muon.py:137-140; vectors of a transformer are a few thousand
  * elements each, so their launches dominate). table: device array of `tensors` rows of seven int64:

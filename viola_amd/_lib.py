@@ -67,7 +67,6 @@ _SIGNATURES = {
     "viola_momentum_update_table": [_p, _l, _l, _i, _i, _f, _f, _i, _i, _l, _p],
     "viola_momentum_update_squares": [_p, _l, _l, _i, _i, _f, _f, _i, _i, _l, _i, _p, _p],
     "viola_weight_update_table": [_p, _l, _l, _i, _f, _f, _f, _p],
-    "viola_weight_update_rows": [_p, _l, _l, _i, _f, _f, _p],
     "viola_adam_update_table": [_p, _l, _l, _i, _i, _i, _f, _f, _f, _f, _f, _f, _f, _i, _l, _i, _i, _p],
     "viola_copy_scaled": [_p, _i, _p, _i, _l, _l, _l, _f, _p],
     "viola_momentum_dequantize": [_p, _p, _p, _l, _i, _i, _l, _l, _l, _i, _i, _p],

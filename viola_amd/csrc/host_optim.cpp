@@ -11,7 +11,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <cstring>
 #include <map>
 #include <tuple>
 
@@ -226,35 +225,21 @@ bool momentum_together(Tables& tables, const std::vector<int64_t>& shape, int64_
 struct WeightRow {
     Tensor weight;
     const void* update;
-    int64_t count;
-    float scale;                                                 // of the update
 };
-bool weights_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<WeightRow>& rows, at::ScalarType update_type,
-                      float lr, float weight_decay, viola_stream_t stream) {
-    if (rows.empty() || rows.size() > 65535) return false;
+bool weights_together(Tables& tables, const std::vector<int64_t>& shape, int64_t ordinal, const std::vector<WeightRow>& rows, int64_t count,
+                      at::ScalarType update_type, float lr, float weight_decay, float update_scale, viola_stream_t stream) {
+    if (rows.empty() || rows.size() > 65535 || count % 4 != 0) return false;
     const int64_t update_bytes = 4 * (int64_t)at::elementSize(update_type);
-    bool alike = true;
-    int64_t most = 0;
-    for (const WeightRow& r : rows) {
-        if (r.count % 4 != 0 || r.weight.scalar_type() != at::kFloat || r.weight.numel() != r.count || !r.weight.is_contiguous() ||
-            !aligned(r.weight.const_data_ptr(), 16) || !aligned(r.update, update_bytes))
-            return false;
-        alike = alike && r.count == rows[0].count && r.scale == rows[0].scale;
-        most = std::max(most, r.count);
-    }
     std::vector<int64_t> words;
     for (const WeightRow& r : rows) {
-        words.push_back((int64_t)r.weight.const_data_ptr());
+        const void* w = r.weight.const_data_ptr();
+        if (r.weight.scalar_type() != at::kFloat || r.weight.numel() != count || !r.weight.is_contiguous() || !aligned(w, 16) || !aligned(r.update, update_bytes))
+            return false;
+        words.push_back((int64_t)w);
         words.push_back((int64_t)r.update);
-        if (alike) continue;
-        uint32_t bits;
-        std::memcpy(&bits, &r.scale, 4);
-        words.push_back(r.count);
-        words.push_back(bits);
     }
     const int64_t* t = tables.get(WEIGHT_TABLE, shape, (int64_t)rows.size(), ordinal, std::move(words), rows[0].weight.device(), stream);
-    if (alike) VIOLA_CALL(viola_weight_update_table, t, (int64_t)rows.size(), most, code_of(update_type), lr, weight_decay, rows[0].scale, stream);
-    else VIOLA_CALL(viola_weight_update_rows, t, (int64_t)rows.size(), most, code_of(update_type), lr, weight_decay, stream);
+    VIOLA_CALL(viola_weight_update_table, t, (int64_t)rows.size(), count, code_of(update_type), lr, weight_decay, update_scale, stream);
     return true;
 }
 
@@ -672,8 +657,10 @@ private:
         const char* from = static_cast<const char*>(updates.const_data_ptr());
         const int update_code = code_of(updates.scalar_type());
         std::vector<WeightRow> weight_rows;
-        for (size_t i = 0; i < bucket.size(); ++i) weight_rows.push_back({bucket[i].param, from + 2 * count * i, count, (float)update_scale(g, rows, cols)});
-        if (together && weights_together(tables_, shape, ordinal, weight_rows, updates.scalar_type(), (float)g.lr, (float)g.weight_decay, stream)) return;
+        for (size_t i = 0; i < bucket.size(); ++i) weight_rows.push_back({bucket[i].param, from + 2 * count * i});
+        if (together && weights_together(tables_, shape, ordinal, weight_rows, count, updates.scalar_type(), (float)g.lr, (float)g.weight_decay,
+                                         (float)update_scale(g, rows, cols), stream))
+            return;
         for (size_t i = 0; i < bucket.size(); ++i) {
             const Item& it = bucket[i];
             const Group& h = *it.group;
@@ -754,9 +741,10 @@ void register_optimizer(py::module_& m) {
         for (size_t i = 0; i < weights.size(); ++i) {
             TORCH_CHECK(weights[i].is_cuda() && updates[i].is_cuda(), "viola_amd kernels run on the GPU only");
             if (updates[i].scalar_type() != updates[0].scalar_type() || updates[i].numel() != weights[i].numel() || !updates[i].is_contiguous()) return false;
-            rows.push_back({weights[i], updates[i].const_data_ptr(), weights[0].numel(), (float)update_scale});
+            rows.push_back({weights[i], updates[i].const_data_ptr()});
         }
-        return weights_together(tables, {}, 0, rows, updates[0].scalar_type(), (float)lr, (float)weight_decay, stream_of(weights[0]));
+        return weights_together(tables, {}, 0, rows, weights[0].numel(), updates[0].scalar_type(), (float)lr, (float)weight_decay, (float)update_scale,
+                                stream_of(weights[0]));
     }));
     m.def("adam_update_many", torch::wrap_pybind_function([](Tables& tables, const std::vector<Tensor>& weights, const std::vector<Tensor>& grads,
                                                              const std::vector<Tensor>& firsts, const std::vector<Tensor>& seconds, const std::vector<int64_t>& keys,

@@ -305,17 +305,14 @@ __global__ __launch_bounds__(256) void weight_quads_kernel(float* weight, const 
     }
 }
 
-// Many fp32 tensors of whole quads: row t of `table` holds {weight, update}, and with ROWS {.., elements, bits of the update scale};
-// blockIdx.y walks the tensors.
-template <typename TG, bool ROWS>
+// Many fp32 tensors of `quads` whole quads each: row t of `table` holds {weight, update}; blockIdx.y walks the tensors.
+template <typename TG>
 __global__ __launch_bounds__(256) void weight_table_quads_kernel(const int64_t* __restrict__ table, int64_t quads, float lr,
                                                                   float decay, float update_scale) {
-    const int64_t* row = table + (int64_t)blockIdx.y * (ROWS ? 4 : 2);
     const float keep = 1.0f - lr * decay;
-    const float rate = lr * (ROWS ? __uint_as_float((uint32_t)row[3]) : update_scale);
-    float* weight = reinterpret_cast<float*>(row[0]);
-    const TG* grad = reinterpret_cast<const TG*>(row[1]);
-    if (ROWS) quads = row[2] / 4;
+    const float rate = lr * update_scale;
+    float* weight = reinterpret_cast<float*>(table[(int64_t)blockIdx.y * 2]);
+    const TG* grad = reinterpret_cast<const TG*>(table[(int64_t)blockIdx.y * 2 + 1]);
     for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < quads; j += (int64_t)gridDim.x * blockDim.x) {
         float4 w = reinterpret_cast<const float4*>(weight)[j];
         float g[4];
@@ -491,20 +488,6 @@ extern "C" int viola_momentum_update_table(const int64_t* table, int64_t tensors
     return viola_launch_status();
 }
 
-template <bool ROWS>
-static int weight_table(const int64_t* table, int64_t tensors, int64_t count, int grad_dtype, float lr, float decay, float update_scale, hipStream_t stream) {
-    VIOLA_CHECK_ARG(viola_is_float(grad_dtype) && tensors >= 0 && tensors <= 65535 && count >= 0 && count % 4 == 0);
-    if (tensors == 0 || count == 0) return 0;
-    VIOLA_CHECK_ARG(table);
-    const int64_t quads = count / 4;
-    const int64_t blocks = (quads + 255) / 256;
-    const dim3 grid((unsigned)(blocks > 4096 ? 4096 : blocks), (unsigned)tensors);
-    if (grad_dtype == VIOLA_F32) VIOLA_LAUNCH((weight_table_quads_kernel<float, ROWS>), grid, dim3(256), 0, stream, table, quads, lr, decay, update_scale);
-    else if (grad_dtype == VIOLA_BF16) VIOLA_LAUNCH((weight_table_quads_kernel<bf16_t, ROWS>), grid, dim3(256), 0, stream, table, quads, lr, decay, update_scale);
-    else VIOLA_LAUNCH((weight_table_quads_kernel<f16_t, ROWS>), grid, dim3(256), 0, stream, table, quads, lr, decay, update_scale);
-    return viola_launch_status();
-}
-
 extern "C" int viola_momentum_update_squares(const int64_t* table, int64_t tensors, int64_t tiles, int grad_dtype, int tile_size,
                                              float beta, float inv_loss_scale, int nesterov, int rounding, int64_t rounding_step,
                                              int working_dtype, float* sums, viola_stream_t stream_) {
@@ -551,12 +534,17 @@ extern "C" int viola_momentum_update_squares(const int64_t* table, int64_t tenso
 
 extern "C" int viola_weight_update_table(const int64_t* table, int64_t tensors, int64_t count, int grad_dtype, float lr,
                                          float decay, float update_scale, viola_stream_t stream_) {
-    return weight_table<false>(table, tensors, count, grad_dtype, lr, decay, update_scale, viola_enter(stream_));
-}
-
-extern "C" int viola_weight_update_rows(const int64_t* table, int64_t tensors, int64_t max_count, int grad_dtype, float lr,
-                                        float decay, viola_stream_t stream_) {
-    return weight_table<true>(table, tensors, max_count, grad_dtype, lr, decay, 0.0f, viola_enter(stream_));
+    hipStream_t stream = viola_enter(stream_);
+    VIOLA_CHECK_ARG(viola_is_float(grad_dtype) && tensors >= 0 && tensors <= 65535 && count >= 0 && count % 4 == 0);
+    if (tensors == 0 || count == 0) return 0;
+    VIOLA_CHECK_ARG(table);
+    const int64_t quads = count / 4;
+    const int64_t blocks = (quads + 255) / 256;
+    const dim3 grid((unsigned)(blocks > 4096 ? 4096 : blocks), (unsigned)tensors);
+    if (grad_dtype == VIOLA_F32) VIOLA_LAUNCH(weight_table_quads_kernel<float>, grid, dim3(256), 0, stream, table, quads, lr, decay, update_scale);
+    else if (grad_dtype == VIOLA_BF16) VIOLA_LAUNCH(weight_table_quads_kernel<bf16_t>, grid, dim3(256), 0, stream, table, quads, lr, decay, update_scale);
+    else VIOLA_LAUNCH(weight_table_quads_kernel<f16_t>, grid, dim3(256), 0, stream, table, quads, lr, decay, update_scale);
+    return viola_launch_status();
 }
 
 extern "C" int viola_weight_update(void* weight, int weight_dtype, const void* grad, int grad_dtype, int64_t n, float lr,
