@@ -1,5 +1,7 @@
 """What an optimizer step holds and allocates on the way."""
 
+import gc
+
 import pytest
 import torch
 
@@ -20,7 +22,8 @@ def _optimizer(shapes, **options):
 
 
 def _peak(opt):
-    """Bytes that a step holds at once beyond what is there before it."""
+    """Bytes that a step holds at once beyond what is there before it (optimizers that are no longer in use are not: they would go on the way)."""
+    gc.collect()
     torch.cuda.synchronize()
     before = torch.cuda.memory_allocated()
     torch.cuda.reset_peak_memory_stats()
