@@ -116,7 +116,8 @@ def test_scaled_matrices_of_several_shapes_equal_one_shape_each(dtype):
 @pytest.mark.parametrize("working", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("grads,tile,rounding", [(torch.float32, 256, 0), (torch.bfloat16, 512, 1), (torch.float16, 1024, 0), (torch.float32, 1024, 1)])
 def test_momentum_with_sums_of_squares(grads, tile, rounding, working):
-    """State and updates are those of viola_momentum_update, one tensor at a time; the sums those of the updates in float64: at most 2^-24 for each of the some 40 additions on the way of a term."""
+    """State and updates are those of viola_momentum_update, one tensor at a time; the sums those of the updates in float64: at most 2^-24 for each of
+    the some 40 additions on the way of a term."""
     torch.manual_seed(tile)
     tiles = [1, 5, 16, 300, 4099]
     table, want, got, held = [], [], [], []
@@ -157,14 +158,19 @@ def test_calls_that_one_launch_does_not_take_are_refused_before_it():
 
 @pytest.mark.parametrize("method", ["standard", "gram"])
 @pytest.mark.parametrize("options", [dict(), dict(tile_size=512, nesterov=False, adjust_lr_fn="match_rms_adamw"), dict(rounding="stochastic", rounding_seed=9, ns_steps=3)])
-def test_step_of_several_shapes_equals_stepping_each_parameter_alone(method, options):
-    """Sets of shapes that step together, wide, tall, square and batched ones, for three steps; a bf16 gradient dtype as well."""
+@pytest.mark.parametrize("batched,dtype", [(True, torch.float32), (False, torch.float32), (False, torch.bfloat16)])
+def test_step_of_several_shapes_equals_stepping_each_parameter_alone(method, options, batched, dtype):
+    """Sets of shapes that step together, wide, tall and square ones, for three steps: with a parameter of two matrices, whose sums of squares are a pass of
+    their own, and without, where they come with the momentum, of FP32 and BF16 gradients."""
     import viola_amd
     shapes = [(192, 64), (64, 192), (64, 64), (192, 64), (2, 32, 64), (256, 64), (96, 128), (64, 64)]
+    shapes = [s for s in shapes if batched or len(s) == 2]
 
     def build(one_each):
         torch.manual_seed(3)
         params = [torch.nn.Parameter(torch.randn(*s, device="cuda") * .05) for s in shapes]
+        for p in params:
+            p.grad_dtype = dtype
         groups = [dict(params=[p], batched=p.dim() == 3) for p in params]
         make = lambda gs: viola_amd.optim.FP8Muon(gs, lr=2e-3, weight_decay=.01, ns_method=method, **options)
         if not one_each:
@@ -177,7 +183,7 @@ def test_step_of_several_shapes_equals_stepping_each_parameter_alone(method, opt
     (together, one), (apart, each) = build(False), build(True)
     for step in range(3):
         torch.manual_seed(50 + step)
-        grads = [torch.randn(*s, device="cuda") * 1e-2 for s in shapes]
+        grads = [(torch.randn(*s, device="cuda") * 1e-2).to(dtype) for s in shapes]
         for params, optimizers in ((together, one), (apart, each)):
             for p, g in zip(params, grads):
                 p.grad = g.clone()
