@@ -60,12 +60,15 @@ def test_nan_is_no_maximum(dtype, place):
     assert history[0] == float("inf") and scale[0] == float("inf")
 
 
-@pytest.mark.parametrize("dtype,kilobytes,whole", [(torch.bfloat16, 128, True), (torch.float32, 128, True), (torch.bfloat16, 132, False), (torch.float16, 256, False),
-                                                    (torch.float32, 132, False)])
-def test_beyond_128_kb_the_maximum_is_a_pass_of_its_own(dtype, kilobytes, whole):
-    """There the blocks' serial walks over the whole tensor take longer than the pass that they save, most of all over an x that no cache holds. Only the
-    pass leaves maxima in the workspace."""
-    x = torch.randn((kilobytes << 10) // torch.finfo(dtype).bits * 8).to(dtype).view(-1, 256)
-    work = torch.full((1024,), float("nan"), device="cuda")
-    _check(x, *_encode(x.cuda(), 448.0, work=work))
-    assert torch.isnan(work).all().item() == whole
+@pytest.mark.parametrize("dtype,kilobytes,whole", [(torch.bfloat16, 256, True), (torch.float16, 256, True), (torch.float32, 192, True), (torch.bfloat16, 260, False),
+                                                    (torch.float16, 260, False), (torch.float32, 196, False)])
+def test_beyond_its_limit_the_maximum_is_a_pass_of_its_own(dtype, kilobytes, whole):
+    """There the blocks' walks over the whole tensor take longer than the launch that they save, over an x that no cache holds most of all. Only the pass
+    leaves maxima in the workspace. The largest value lies in each of a walk's turns of 64 KB, wherever a block begins."""
+    n = (kilobytes << 10) // torch.finfo(dtype).bits * 8
+    for place in range(n // 8, n, n // 4):
+        x = torch.randn(n).to(dtype).view(-1, 256)
+        x.view(-1)[place] = 30.0
+        work = torch.full((1024,), float("nan"), device="cuda")
+        _check(x, *_encode(x.cuda(), 448.0, work=work))
+        assert torch.isnan(work).all().item() == whole

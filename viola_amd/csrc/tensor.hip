@@ -70,7 +70,8 @@ __global__ __launch_bounds__(256) void tensor_amax_kernel(const TIn* __restrict_
 }
 
 // A thread's part of the maximum of a whole small tensor, for a block of 256 that needs it by itself: 64 KB of loads at a time, those past the
-// end repeating the last.
+// end repeating the last. Neighbours on an XCD start with different 64 KB, so that what no cache holds is fetched once for all of them and not turn by turn:
+// cold tensors of BF16 192 KB 7.3 -> 6.5 us, 256 KB 8.5 -> 7.2 (in the caches 6.1 either way); 128 KB of loads at a time 7.3.
 template <typename TIn>
 __device__ __forceinline__ float absmax_whole(const TIn* __restrict__ x, int n) {
     constexpr int N = Vec16<TIn>::N, LOADS = 16;
@@ -78,7 +79,11 @@ __device__ __forceinline__ float absmax_whole(const TIn* __restrict__ x, int n) 
     if (head > n) head = n;
     const int vectors = (n - head) / N;
     auto walk = [&](auto fold) {
-        for (int v = threadIdx.x; v < vectors; v += LOADS * 256) {
+        const int turns = (vectors + LOADS * 256 - 1) / (LOADS * 256);
+        int turn = turns > 1 ? (int)(blockIdx.x / 8) % turns : 0;
+        for (int done = 0; done < turns; ++done) {
+            const int v = turn * (LOADS * 256) + (int)threadIdx.x;
+            if (++turn == turns) turn = 0;
             uint4 raw[LOADS];
 #pragma unroll
             for (int i = 0; i < LOADS; ++i) raw[i] = reinterpret_cast<const uint4*>(x + head)[min(v + i * 256, vectors - 1)];
@@ -558,12 +563,13 @@ extern "C" int viola_tensor_encode_beside(const void* x, int x_dtype, int64_t ro
     hipStream_t stream = viola_enter(stream_);
     VIOLA_CHECK_ARG(viola_is_float(x_dtype) && viola_is_fp8(q_dtype) && rows > 0 && cols > 0 && x && workspace && history && history_len > 0);
     VIOLA_CHECK_ARG(index >= 0 && limit > 0.0f && scale && (!column_sum || viola_is_float(sum_dtype)));
-    // Small tensors, a tile or less to a CU: every block of the quantizer takes the maximum of the whole by itself, in turns of 64 KB, in place of a
-    // launch of 3 us on the host and 1.5 on the device. Up to where that is the shorter also for an x that no cache holds, which each XCD then fetches
-    // for itself. Two launches and one, BF16 with both layouts, x in the caches and (not), us: 8 KB 5.4 (6.7), 4.0 (4.6); 64 KB 5.6 (6.5), 4.0 (4.9); 128 KB
-    // 5.6 (6.7), 4.6 (6.1); 160 KB 5.6 (6.8), 5.4 (7.2); 256 KB 5.7 (6.7), 6.1 (8.5). FP32: 128 KB 5.6 (7.0), 4.5 (6.2); 160 KB 5.6 (7.2), 5.1 (7.2);
-    // 256 KB 5.8 (7.2), 5.7 (8.8).
-    constexpr int64_t FEW = 512, WHOLE_BYTES = 128 << 10, WHOLE_TILES = 256;
+    // Small tensors, a tile or less to a CU: every block of the quantizer takes the maximum of the whole by itself, in place of a launch of 3 us on the
+    // host and 1.5 on the device. Two launches and one, both layouts, x in the caches and (not), us, BF16: 8 KB 5.4 (6.7), 4.1 (4.7); 64 KB 5.7 (6.5),
+    // 4.0 (5.0); 128 KB 5.6 (6.7), 4.6 (5.6); 192 KB 5.7 (6.8), 5.4 (6.5); 256 KB 5.6 (6.8), 6.1 (7.2); 384 KB 5.7 (6.9), 7.6 (8.7). FP32: 128 KB 5.7
+    // (7.0), 4.5 (5.6); 192 KB 5.7 (7.2), 5.1 (6.9); 256 KB 5.7 (7.1), 5.7 (8.2). 16-bit tensors of up to 256 KB, as a layer whose tensors are so small
+    // waits for the host: 256 x 512 -> 2048, forward and backward, 79.7 us in two launches, 75.
+    constexpr int64_t FEW = 512, WHOLE_TILES = 256;
+    const int64_t whole_bytes = (x_dtype == VIOLA_F32 ? 192 : 256) << 10;
     TensorQuantizeSide side = {};
     if (codes) {
         VIOLA_CHECK_ARG(codes_t && code_rows > 0 && code_cols > 0 && code_pitch >= code_rows);
@@ -598,7 +604,7 @@ extern "C" int viola_tensor_encode_beside(const void* x, int x_dtype, int64_t ro
         parts = wanted <= 2048 ? (wanted < 256 ? wanted : 256) : 1024;
         VIOLA_CHECK_ARG(workspace_floats >= parts);
         const int64_t across = (max64(cols, q ? q_pitch : 0) + 63) / 64, down = (max64(rows, qt ? qt_pitch : 0) + 63) / 64;
-        side.whole = n * viola_dtype_size(x_dtype) <= WHOLE_BYTES && across * down <= WHOLE_TILES && (q || qt) && !(delayed && index != 0);
+        side.whole = n * viola_dtype_size(x_dtype) <= whole_bytes && across * down <= WHOLE_TILES && (q || qt) && !(delayed && index != 0);
         status = side.whole ? 0 : viola_tensor_amax(x, x_dtype, n, workspace, parts, stream_);
     }
     if (status) return status;
