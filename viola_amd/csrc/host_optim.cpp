@@ -506,11 +506,13 @@ private:
     }
 
     // The chains of all buckets step by step together, a product of each in one launch, and one launch each for the momentum with the sums
-    // of squares and for the scaling in front of the chains: 18 launches where buckets on lanes of their own took about 80 and the events that
+    // of squares and for the scaling in front of the chains: 17 launches where buckets on lanes of their own took about 80 and the events that
     // join them, which is all that a step of small matrices costs (one block of width 192: 253 -> 99 us, four of 256 316 -> 140, eight of
     // 384 362 -> 325). Large sets gain by the mix of tile lengths (by that alone 28 blocks of width 1152 12560 -> 12280 us, eight of 1280 5842 ->
     // 5185). The recurrence on the Gram matrix gains less there: its launches are several rounds of short tiles with a tail each, which lanes
-    // fill (28 blocks of 384 805 us on lanes, 881 together; four of 512 373 and 331), so beyond TOGETHER_GRAM it keeps the lanes.
+    // fill, so beyond TOGETHER_GRAM it keeps the lanes. On lanes and together, us, by the sum of m m (m + n): 28 blocks of 256 (7.5e9) 571, 400; two of 640
+    // (8.4e9) 386, 314; four of 512 (8.6e9) 400, 316; 23 of 288 (8.8e9) 532, 515; 20 of 320 (1.05e10) 517, 524; four of 640 (1.7e10) 480, 471; ten of 512
+    // (2.1e10) 593, 589; 28 of 384 (2.5e10) 803, 835; two of 1024 (3.4e10) 719, 653; 19 of 608 (6.8e10) 1666, 1706.
     static constexpr double TOGETHER_GRAM = 1e10;                // sum of m m (m + n) over the matrices
     // All arenas are held at once, 10 bytes per element at most (5.4 GB); and no more elements than the buckets on lanes may hold.
     static constexpr int64_t TOGETHER_ELEMENTS = 1ll << 29;
@@ -580,7 +582,6 @@ private:
         return g.match_rms ? .2 * std::pow((double)std::max(rows, cols), .5) : std::pow(std::max(1., (double)rows / (double)cols), .5);
     }
 
-    static constexpr int64_t INTO_WEIGHTS = 6 << 20;             // elements of a bucket on a lane
     // weight = weight * (1 - lr decay) - lr scale update, with the FP32 roundings of viola_weight_update
     static void into_weights(viola_ns_product& last, const int64_t* weights, const Group& g, int64_t rows, int64_t cols) {
         const float lr = (float)g.lr, decayed = lr * (float)g.weight_decay;
@@ -633,9 +634,9 @@ private:
             together = together && h.lr == g.lr && h.weight_decay == g.weight_decay && h.match_rms == g.match_rms;
             in_place = in_place && it.param.scalar_type() == at::kFloat && aligned(it.param.const_data_ptr(), 16);
         }
-        // and where they are enough for several rounds of tiles (below that other lanes hide the weights' launch better than a tile hides their
-        // loads: two blocks of 768, recurrence, 400 us, 420 so)
-        in_place = in_place && together && size * count >= INTO_WEIGHTS;
+        // (of any size: a launch less, and 8 bytes per element. us, with a launch for the weights and without: one block of 192 335, 324; eight of 384 379,
+        // 364; two of 768 418, 403; eight of 1024 2453, 2361)
+        in_place = in_place && together;
         Chain chain = chain_of(updates_in, g.ns_steps, g.gram, true, !in_place);
         prepare(chain, chain.sums, stream);
         for (size_t i = 0; i + 1 < chain.products.size(); ++i) multiply(chain.products[i], chain.dtype, stream);
