@@ -74,6 +74,12 @@ def timed(fn, steps, warmup, warm=True):
     return max(start.elapsed_time(end), 0.0) / steps, wall / steps
 
 
+def set_streams(opt, streams):
+    """Gives FP8Muon so many streams and returns how many it had. What a step may hold at once stays the same, and with it which matrices share their launches."""
+    had, opt._BATCH_ELEMENTS, opt._LANES = opt._LANES, opt._BATCH_ELEMENTS * opt._LANES // streams, streams
+    return had
+
+
 def kernel_breakdown(fn, steps):
     """Second, instrumented pass: HIP events around every C-ABI call on the stream it is launched on."""
     import torch
@@ -321,11 +327,11 @@ def main():
             log(f"FP8Muon step, {method}")
             opt, params, elements = muon_case(method)
             if args.muon_streams:
-                opt._LANES = args.muon_streams
+                set_streams(opt, args.muon_streams)
             step_ms, step_wall = timed(opt.step, 5, 3)
             # a step whose matrices do not share their launches runs its shape buckets on several streams; for per-launch
             # durations that do not overlap each other the instrumented pass (and one timing next to it) keeps them on one
-            lanes, opt._LANES = opt._LANES, 1
+            lanes = set_streams(opt, 1)
             serial_ms, _ = timed(opt.step, 3, 1)
             b = kernel_breakdown(opt.step, 2)
             ns_flops = 0.0
